@@ -66,7 +66,7 @@ extern "C" {
  * backward entry point take `int operand_type` before `tuning` / `stream`; a caller built against an older header
  * would pass its tuning selector there).  The Python binding checks for an exact match when it loads the library.
  */
-#define PROTEUS_VERSION 301
+#define PROTEUS_VERSION 302
 int proteus_version(void);
 
 /* Human-readable text for a return code of any entry point. */
@@ -114,6 +114,22 @@ int proteus_we_fwd_check(const float* coords, int coords_layout,
                          const float* wavenumbers, const uint8_t* mask,
                          const float* out, const float* cos_sums, const float* sin_sums,
                          int Z, int N, int K, int tuning);
+
+/*
+ * proteus_we_fwd with a caller-provided workspace: with tuning = 0 and a workspace of at least
+ * proteus_we_fwd_workspace_bytes(Z, N, K, 0) bytes the distances of an observer are spread onto a uniform grid and the grid
+ * is evaluated at the wavenumbers (we_grid.hip), instead of one sine and cosine per (pair of tokens, wavenumber).  Same
+ * result as proteus_we_fwd to single-precision rounding, deterministic.
+ *   workspace    device memory, 256-byte aligned; not initialised by the caller, nothing kept in it between calls; calls
+ *                that share one workspace must not overlap.  NULL, too small, or tuning != 0: the call is proteus_we_fwd.
+ *   proteus_we_fwd_workspace_bytes returns 0 where the direct kernels are the better choice (few wavenumbers or tokens)
+ *   and for tuning != 0.
+ */
+size_t proteus_we_fwd_workspace_bytes(int Z, int N, int K, int tuning);
+int proteus_we_fwd_ws(const float* coords, int coords_layout,
+                      const float* wavenumbers, const uint8_t* mask,
+                      float* out, float* cos_sums, float* sin_sums, void* workspace, size_t workspace_bytes,
+                      int Z, int N, int K, int tuning, void* stream);
 
 int         proteus_we_num_variants(void);
 const char* proteus_we_variant_name(int tuning);

@@ -12,14 +12,14 @@ LIB_PATH = os.path.join(HERE, "libproteus_hip.so")
 
 COORDS_SOA = 0
 COORDS_AOS = 1
-ABI_VERSION = 301                    # PROTEUS_VERSION of the include/proteus_hip.h these argument lists were written from
+ABI_VERSION = 302                    # PROTEUS_VERSION of the include/proteus_hip.h these argument lists were written from
 OPERAND_BF16, OPERAND_F16 = 0, 1     # PROTEUS_OPERAND_* of include/proteus_hip.h
 DTYPE_F32, DTYPE_BF16, DTYPE_F16 = 0, 1, 2   # PROTEUS_DTYPE_*
 
 # every symbol include/proteus_hip.h declares
 SYMBOLS = [
     "proteus_version", "proteus_strerror",
-    "proteus_we_fwd", "proteus_we_fwd_check", "proteus_we_legacy_fwd", "proteus_we_dropout_fwd", "proteus_we_dropout_fwd_check",
+    "proteus_we_fwd", "proteus_we_fwd_check", "proteus_we_fwd_workspace_bytes", "proteus_we_fwd_ws", "proteus_we_legacy_fwd", "proteus_we_dropout_fwd", "proteus_we_dropout_fwd_check",
     "proteus_we_dropout_threshold", "proteus_we_num_variants", "proteus_we_variant_name",
     "proteus_we_aniso_fwd", "proteus_we_aniso_fwd_check", "proteus_we_aniso_num_variants", "proteus_we_aniso_variant_name",
     "proteus_we_bwd_workspace_bytes", "proteus_we_bwd", "proteus_we_bwd_check", "proteus_we_bwd_static", "proteus_we_aniso_bwd", "proteus_we_aniso_bwd_check",
@@ -79,6 +79,10 @@ def load():
     lib.proteus_we_aniso_variant_name.restype = ctypes.c_char_p
     lib.proteus_we_aniso_variant_name.argtypes = [ci]
     sz = ctypes.c_size_t
+    lib.proteus_we_fwd_workspace_bytes.restype = sz
+    lib.proteus_we_fwd_workspace_bytes.argtypes = [ci, ci, ci, ci]
+    lib.proteus_we_fwd_ws.restype = ci
+    lib.proteus_we_fwd_ws.argtypes = [vp, ci, vp, vp, vp, vp, vp, vp, sz, ci, ci, ci, ci, vp]
     lib.proteus_we_bwd_workspace_bytes.restype = sz
     lib.proteus_we_bwd_workspace_bytes.argtypes = [ci, ci, ci]
     lib.proteus_we_bwd.restype = ci

@@ -68,11 +68,15 @@ def we_forward(coords, wavenumbers, mask=None, tuning: int = 0, magnitude_type: 
                                             out.data_ptr(), cos_sums.data_ptr(), sin_sums.data_ptr(),
                                             Z, N, K, int(magnitude_type), dropout_p, int(rng_seed) & 0xffffffff, stream)
         elif magnitude_type == 1:
-            rc = lib.proteus_we_fwd(c.data_ptr(), _lib.COORDS_AOS, w.data_ptr(),
-                                    None if m is None else m.data_ptr(),
-                                    out.data_ptr(), cos_sums.data_ptr() if need_sums else None,
-                                    sin_sums.data_ptr() if need_sums else None,
-                                    Z, N, K, int(tuning), stream)
+            # with a workspace the library may go through grids of the distances (its size is 0 where that is of no use)
+            ws_bytes = lib.proteus_we_fwd_workspace_bytes(Z, N, K, int(tuning))
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
+            rc = lib.proteus_we_fwd_ws(c.data_ptr(), _lib.COORDS_AOS, w.data_ptr(),
+                                       None if m is None else m.data_ptr(),
+                                       out.data_ptr(), cos_sums.data_ptr() if need_sums else None,
+                                       sin_sums.data_ptr() if need_sums else None,
+                                       None if ws is None else ws.data_ptr(), ws_bytes,
+                                       Z, N, K, int(tuning), stream)
         else:
             rc = lib.proteus_we_legacy_fwd(c.data_ptr(), _lib.COORDS_AOS, w.data_ptr(),
                                            None if m is None else m.data_ptr(),

@@ -1,0 +1,101 @@
+"""The embedding forward through distance grids (proteus_we_fwd_ws with a workspace) against the float64 oracle, at the
+sizes where it can go wrong: tiles of 16 observers, flushes after 1024 sources, octave and window borders of the grid,
+pairs closer than half a cell, coordinates that are not finite."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import c_oracle
+from proteusai_amd import _lib, synth
+
+pytestmark = pytest.mark.gpu
+
+
+def run_grid(gpu, coords, wn, mask=None, sums=True, layout=_lib.COORDS_AOS):
+    lib = _lib.load()
+    Z, N, K = coords.shape[0], coords.shape[1] if layout == _lib.COORDS_AOS else coords.shape[2], wn.numel()
+    c, w = coords.to(gpu), wn.to(gpu)
+    m = None if mask is None else mask.to(gpu).view(torch.uint8)
+    bufs = [torch.full(s, float("nan"), device=gpu) for s in ((Z, N, 2 * K), (Z, N, K), (Z, N, K))]
+    nbytes = lib.proteus_we_fwd_workspace_bytes(Z, max(N, 1024), max(K, 64), 0)      # (the size grows with N and K)
+    ws = torch.full((nbytes,), 0xA5, dtype=torch.uint8, device=gpu)
+    rc = lib.proteus_we_fwd_ws(c.data_ptr(), layout, w.data_ptr(), None if m is None else m.data_ptr(), bufs[0].data_ptr(),
+                               bufs[1].data_ptr() if sums else None, bufs[2].data_ptr() if sums else None, ws.data_ptr(), nbytes,
+                               Z, N, K, 0, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, lib.proteus_strerror(rc)
+    torch.cuda.synchronize()
+    return [b.cpu().numpy() for b in bufs[:3 if sums else 1]]
+
+
+def rel_l2(a, b):
+    a, b = np.asarray(a, np.float64), np.asarray(b, np.float64)
+    nb = np.linalg.norm(b)
+    return float(np.linalg.norm(a - b) / nb) if nb > 0 else float(np.linalg.norm(a - b))
+
+
+CASES = {                       # N, Z, K, scale of the chain, mask
+    "one tile": (16, 1, 16, 1.0, None),
+    "tile and a bit, odd K": (17, 3, 37, 1.0, None),
+    "two tokens": (2, 2, 5, 1.0, None),
+    "one flush exactly": (1024, 1, 64, 1.0, None),
+    "one source more than a flush": (1025, 1, 64, 1.0, None),
+    "flushes, scattered mask": (2100, 2, 20, 1.0, "scattered"),
+    "tail masks, empty item, lone survivor": (333, 4, 48, 1.0, "tail"),
+    "large K": (70, 1, 300, 1.0, None),
+    "many pairs closer than half a cell": (200, 1, 64, 0.05, None),
+    "all pairs closer than half a cell": (60, 2, 40, 0.005, None),
+    "several windows of the grid": (700, 2, 33, 30.0, None),
+    "several windows and flushes": (1500, 1, 16, 20.0, "scattered"),
+    "beyond the windows": (90, 1, 33, 3000.0, None),
+}
+
+
+@pytest.mark.parametrize("name", CASES)
+def test_grid_matches_the_oracle(gpu, name):
+    N, Z, K, scale, kind = CASES[name]
+    coords, _ = synth.we_inputs(N, seed=N + K, batch=Z)
+    coords = coords * scale
+    if N > 50:
+        coords[0, 40] = coords[0, 12]                          # a coincident pair is dropped like the observer itself
+        coords[0, 20] = coords[0, 30] + torch.tensor([0.01, -0.02, 0.015])      # and one that is merely very close is not
+    g = torch.Generator().manual_seed(K)
+    wn = synth.wavenumbers(2 * K) * torch.where(torch.rand(K, generator=g) < 0.3, -1.0, 1.0)
+    mask = None
+    if kind == "scattered":
+        mask = torch.rand(Z, N, generator=g) < 0.35
+    elif kind == "tail":
+        mask = torch.arange(N)[None, :] >= torch.tensor([N, 100, 0, 1])[:, None]
+    junk = coords.clone()
+    if mask is not None:
+        junk[mask] = float("nan")                              # what padded positions hold reaches nothing
+    got = run_grid(gpu, junk, wn, mask)
+    ref = c_oracle.we(coords.numpy(), wn.numpy(), None if mask is None else mask.numpy(), precision="f64")
+    # Bar: 4 x the aliasing error of the grid (2.2e-7) and of its fixed-point sums (2e-7), plus what single precision makes of a
+    # phase k r: the distance and (in the direct sums) the phase are each rounded to 2^-24 of themselves, at most k_max times
+    # the largest distance.
+    c = coords if mask is None else coords.masked_fill(mask[..., None], 0.0)
+    far = float((c.amax(1) - c.amin(1)).norm(dim=-1).max())
+    bar = 1.7e-6 + 2 * 2.0 ** -24 * float(wn.abs().max()) * far
+    for a, r, what in zip(got, ref, ("out", "cos_sums", "sin_sums")):
+        assert np.isfinite(a).all(), f"{name}: {what}"
+        if mask is not None:
+            assert (a[mask.numpy()] == 0).all(), f"{name}: {what} of padded rows"
+        assert rel_l2(a, r) <= bar, f"{name}: {what} {rel_l2(a, r):.3e} (bar {bar:.1e})"
+    again = run_grid(gpu, junk, wn, mask)
+    lean = run_grid(gpu, junk, wn, mask, sums=False)
+    assert all(np.array_equal(a, b) for a, b in zip(got, again)) and np.array_equal(got[0], lean[0])
+    soa = run_grid(gpu, junk.transpose(1, 2).contiguous(), wn, mask, layout=_lib.COORDS_SOA)
+    assert all(np.array_equal(a, b) for a, b in zip(got, soa))
+
+
+def test_values_that_are_not_finite_come_through(gpu):
+    # as in the direct kernels: an unpadded token at NaN makes every sum of its batch item NaN and touches no other item
+    coords, wn = synth.we_inputs(200, seed=5, batch=2, d_model=128)
+    coords[1, 77, 1] = float("nan")
+    got = run_grid(gpu, coords, wn)
+    ref = c_oracle.we(coords[:1].numpy(), wn.numpy(), precision="f64")
+    for a, r in zip(got, ref):
+        assert np.isnan(a[1]).all() and rel_l2(a[0], r[0]) <= 1e-5
+    bad = wn.clone()
+    bad[3] = float("nan")
+    assert np.isnan(run_grid(gpu, coords[:1], bad)[0][:, :, 6:8]).all()
