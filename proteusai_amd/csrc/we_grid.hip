@@ -31,23 +31,21 @@
 namespace {
 
 constexpr int WG_OBS     = 16;                    // observers per workgroup (one tile of the 16x16x4 product)
-constexpr int WG_WAVES   = 8;
-constexpr int WG_THREADS = WG_WAVES * 64;
-constexpr int WG_STEP    = WG_WAVES * 4;          // sources per iteration: a wave takes 16 observers x 4 sources
-constexpr int WG_FLUSH   = 1024;                  // sources between two flushes
-constexpr int WG_ROWS    = 1216;                  // rows of 16 cells in LDS: 77 824 bytes, two workgroups per compute unit
+constexpr int WG_FLUSH   = 2048;                  // sources between two flushes
+constexpr int WG_ROWS    = 1216;                  // rows of 16 cells in LDS: 77 824 bytes, two workgroups of 8 waves per compute unit
 constexpr int WG_R0      = 8;                     // rows in front of the first node (zeros, read by the product)
-constexpr int WG_OCT     = 5;                     // extra rows per octave: six nodes reach five rows into the next one
-constexpr int WG_CELLS   = WG_ROWS - 2 * WG_R0 - WG_OCT * 11;      // cells per window (n < 2^11)
+constexpr int WG_OCT     = 8;                     // extra rows per octave: six nodes reach five rows into the next one (8: a shift in the address)
+constexpr int WG_TRASH   = WG_ROWS - 6;           // the rows of sources that belong to no cell
+constexpr int WG_CELLS   = WG_TRASH - WG_R0 - 5 - WG_OCT * 10;     // cells per window (n < 2^11)
 constexpr int WG_MAX_WINDOWS = 16;
 constexpr int WG_GROUPS  = (WG_CELLS + 5 + 1) / 2 / 8 + 1;         // groups of 8 rows of the tables
-constexpr int WG_CHUNKS  = (WG_ROWS * WG_OBS / 4 + WG_THREADS - 1) / WG_THREADS;   // float4 pieces of the grid per thread
 
 constexpr float WG_OVERSAMPLING = 3.5f;
-constexpr float WG_SCALE = 2097000.0f;            // 1024 x 2 x WG_SCALE < 2^32
+constexpr float WG_UNIT  = 4096.0f;               // coordinates are scaled by this power of two (see the spread)
 constexpr float WG_MAGIC = 12582912.0f;           // 1.5 x 2^23: t + WG_MAGIC holds rint(t) in its low bits
+constexpr uint32_t WG_MAGIC_BITS = 0x4B400000u;
 
-static_assert(WG_R0 + WG_CELLS - 1 + WG_OCT * 10 + 6 + WG_R0 <= WG_ROWS, "rows of the spread");
+static_assert(WG_R0 + WG_CELLS - 1 + WG_OCT * 10 + 6 <= WG_TRASH, "rows of the spread");
 static_assert(WG_R0 + 8 * WG_GROUPS * 2 + 8 <= WG_ROWS, "rows of the product");
 
 struct WgParams {                 // head of the workspace, written by the preparation
@@ -60,18 +58,22 @@ struct WgWave { double rev; float q, dq; };      // k h / 2 pi; 1/phihat and its
 __device__ const double kQ[8] = {0.5144796916399992, 0.1467794687271181, 0.022356478641989086, 0.0024221529567290006,
                                  0.00020978467048036778, 1.54869506429115e-05, 9.95433626001851e-07, 7.199788952850109e-08};
 
-struct WgLayout { size_t counts, waves, table, sources, bytes; int npad, nkt; };
+struct WgBox { float lo[3], hi[3], bad, pad; };  // of 64 tokens, unpadded ones only; bad: one of them is not finite
+
+struct WgLayout { size_t counts, waves, table, boxes, sources, bytes; int npad, nkt, nbox; };
 
 __host__ __device__ inline WgLayout wg_layout(int Z, int N, int K)
 {
     WgLayout l;
     l.nkt  = (K + 15) / 16;
-    l.npad = (N + 63) / 64 * 64 + 128;            // the stream reads up to two iterations past the end
+    l.npad = (N + 63) / 64 * 64 + 512;            // the stream reads up to an iteration (256 sources) past the end
+    l.nbox = (N + 63) / 64;
     auto up = [](size_t v) { return (v + 255) / 256 * 256; };
     l.counts  = sizeof(WgParams);
     l.waves   = l.counts + up((size_t)Z * 4);
     l.table   = l.waves + up((size_t)l.nkt * 16 * sizeof(WgWave));
-    l.sources = l.table + (size_t)WG_GROUPS * l.nkt * 64 * 16;
+    l.boxes   = l.table + (size_t)WG_GROUPS * l.nkt * 64 * 16;
+    l.sources = l.boxes + up((size_t)Z * l.nbox * sizeof(WgBox));
     l.bytes   = l.sources + up((size_t)Z * l.npad * 16);
     return l;
 }
@@ -128,15 +130,28 @@ void we_grid_prepare_kernel(const float* __restrict__ coords, const int layout, 
         const int before = min(b * 256, N) - below + base + __builtin_popcountll(bal & ((1ull << lane) - 1ull));   // unpadded tokens in front of j
         if (b == 0 && tid == 0) reinterpret_cast<int*>(ws + L.counts)[z] = n;
         const float inf = __builtin_inff();
-        if (in) {
-            float4 v = make_float4(inf, inf, inf, __builtin_bit_cast(float, j));
-            if (valid) {
-                if (layout == PROTEUS_COORDS_SOA) { v.x = cz[j]; v.y = cz[(size_t)N + j]; v.z = cz[2 * (size_t)N + j]; }
-                else { v.x = cz[3 * (size_t)j]; v.y = cz[3 * (size_t)j + 1]; v.z = cz[3 * (size_t)j + 2]; }
+        float4 v = make_float4(inf, inf, inf, __builtin_bit_cast(float, in ? j : -1));
+        if (valid) {
+            if (layout == PROTEUS_COORDS_SOA) { v.x = cz[j]; v.y = cz[(size_t)N + j]; v.z = cz[2 * (size_t)N + j]; }
+            else { v.x = cz[3 * (size_t)j]; v.y = cz[3 * (size_t)j + 1]; v.z = cz[3 * (size_t)j + 2]; }
+            v.x *= WG_UNIT; v.y *= WG_UNIT; v.z *= WG_UNIT;
+        }
+        if (b * 4 + wave < L.nbox) {
+            float lo[3] = {v.x, v.y, v.z}, hi[3] = {valid ? v.x : -inf, valid ? v.y : -inf, valid ? v.z : -inf};
+            const bool bad = valid && !(fabsf(v.x) + fabsf(v.y) + fabsf(v.z) < 3.0e38f);
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+                for (int o = 32; o > 0; o >>= 1) { lo[c] = fminf(lo[c], __shfl_xor(lo[c], o)); hi[c] = fmaxf(hi[c], __shfl_xor(hi[c], o)); }
+            const bool any_bad = __builtin_amdgcn_ballot_w64(bad) != 0;
+            if (lane == 0) {
+                WgBox* box = reinterpret_cast<WgBox*>(ws + L.boxes) + (size_t)z * L.nbox + b * 4 + wave;
+                *box = WgBox{{lo[0], lo[1], lo[2]}, {hi[0], hi[1], hi[2]}, any_bad ? inf : 0.f, 0.f};
             }
+        }
+        if (in) {
             src[valid ? before : n + (j - before)] = v;
         } else if (j < L.npad) {
-            src[j] = make_float4(inf, inf, inf, __builtin_bit_cast(float, -1));
+            src[j] = v;
         }
         return;
     }
@@ -195,7 +210,7 @@ __device__ __forceinline__ float wg_vgpr(float v)
     return v;
 }
 
-// distance of a pair: 1/r (0 for r = 0) and r within 1 ulp
+// distance of a pair: 1/r (a hardware reciprocal square root) and r, with one Newton step, to half an ulp
 __device__ __forceinline__ void wg_distance(const float dx, const float dy, const float dz, float& r2, float& inv, float& r)
 {
     r2  = dx * dx + dy * dy + dz * dz;
@@ -204,6 +219,9 @@ __device__ __forceinline__ void wg_distance(const float dx, const float dy, cons
     r = __builtin_fmaf(__builtin_fmaf(-r0, r0, r2), 0.5f * inv, r0);
 }
 
+typedef __attribute__((address_space(3))) uint32_t wg_lds_u32;
+struct wg_true { static constexpr bool value = true; };
+struct wg_false { static constexpr bool value = false; };
 typedef float wg_f4 __attribute__((ext_vector_type(4)));
 
 // The sources of `near` pairs of one observer (all of them if `all`), summed directly by one wave, a lane per wavenumber.
@@ -216,7 +234,7 @@ __device__ void wg_direct(const float4* __restrict__ src, const int n, const flo
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int k = kb + 64 * u + lane;
-            kr[u] = (float)((k < K ? (double)wavenumbers[k] : 0.0) * 0.15915494309189533577);
+            kr[u] = (float)((k < K ? (double)wavenumbers[k] : 0.0) * 0.15915494309189533577) * (1.0f / WG_UNIT);
             oc[u] = os[u] = c[u] = s[u] = 0.f;
         }
         for (int j0 = 0; j0 < n; j0 += 64) {
@@ -243,6 +261,7 @@ __device__ void wg_direct(const float4* __restrict__ src, const int n, const flo
         for (int u = 0; u < 4; ++u) {
             const int k = kb + 64 * u + lane;
             if (k >= K) continue;
+            oc[u] *= WG_UNIT; os[u] *= WG_UNIT;
             if (!all) { oc[u] += o[2 * k]; os[u] += o[2 * k + 1]; }
             o[2 * k] = oc[u]; o[2 * k + 1] = os[u];
             if (SUMS) {
@@ -253,14 +272,21 @@ __device__ void wg_direct(const float4* __restrict__ src, const int n, const flo
     }
 }
 
-template <bool SUMS>
-__global__ __launch_bounds__(WG_THREADS, 4)
+// WAVES  8: two workgroups share a compute unit, one's product under the other's spread; 16: twice the waves on the same
+//        observers, for launches of at most one workgroup per compute unit
+template <bool SUMS, int WAVES>
+__global__ __launch_bounds__(WAVES * 64, 4)
 void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ wavenumbers,
                     float* __restrict__ out, float* __restrict__ cos_sums, float* __restrict__ sin_sums,
                     const int Z, const int N, const int K)
 {
+    constexpr int THREADS = WAVES * 64;
+    constexpr int STEP    = WAVES * 16;           // sources per iteration: a wave takes 16 observers x 4 sources, four times
+    constexpr int CHUNKS  = (WG_ROWS * WG_OBS / 4 + THREADS - 1) / THREADS;    // float4 pieces of the grid per thread
+    constexpr int KT      = 16 / WAVES;           // tiles of 16 wavenumbers a wave takes at a time
+    constexpr int AHEAD   = WAVES == 16 ? 4 : 2;  // groups of the tables in flight: a lone workgroup has nothing else to cover their latency
     extern __shared__ __align__(16) uint32_t s_grid[];          // [WG_ROWS][WG_OBS]
-    __shared__ float s_red[WG_WAVES];
+    __shared__ float s_red[WAVES];
     __shared__ int   s_near[WG_OBS];
     __shared__ int   s_tok[WG_OBS];
 
@@ -273,7 +299,7 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
     const float4* __restrict__ src = reinterpret_cast<const float4*>(ws + L.sources) + (size_t)z * L.npad;
     const WgWave* __restrict__ waves = reinterpret_cast<const WgWave*>(ws + L.waves);
     const float4* __restrict__ table = reinterpret_cast<const float4*>(ws + L.table);
-    const float inv_h = reinterpret_cast<const WgParams*>(ws)->inv_h, h = reinterpret_cast<const WgParams*>(ws)->h;
+    const float inv_h = reinterpret_cast<const WgParams*>(ws)->inv_h * (1.0f / WG_UNIT), h = reinterpret_cast<const WgParams*>(ws)->h;
 
     // ---- the workgroup's slots: unpadded observers first, then padded tokens (zero rows), then nothing ----
     const int slot0 = blockIdx.x * WG_OBS;
@@ -288,8 +314,8 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
             const int t = s_tok[q];
             if (t < 0) continue;
             const size_t row = zN + t;
-            for (int k = tid; k < 2 * K; k += WG_THREADS) out[row * 2 * K + k] = 0.f;
-            if (SUMS) for (int k = tid; k < K; k += WG_THREADS) { cos_sums[row * K + k] = 0.f; sin_sums[row * K + k] = 0.f; }
+            for (int k = tid; k < 2 * K; k += THREADS) out[row * 2 * K + k] = 0.f;
+            if (SUMS) for (int k = tid; k < K; k += THREADS) { cos_sums[row * K + k] = 0.f; sin_sums[row * K + k] = 0.f; }
         }
         return;
     }
@@ -305,18 +331,20 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
             for (int o = 8; o > 0; o >>= 1) { lo[c] = fminf(lo[c], __shfl_xor(lo[c], o)); hi[c] = fmaxf(hi[c], __shfl_xor(hi[c], o)); }
         const float mx = 0.5f * (lo[0] + hi[0]), my = 0.5f * (lo[1] + hi[1]), mz = 0.5f * (lo[2] + hi[2]);
         const float ex = hi[0] - mx, ey = hi[1] - my, ez = hi[2] - mz;
+        // the corners of the boxes around every 64 tokens bound the distances (a thread has one box up to N = 64 THREADS)
+        const WgBox* __restrict__ boxes = reinterpret_cast<const WgBox*>(ws + L.boxes) + (size_t)z * L.nbox;
         float far2 = 0.f;
-        for (int j = tid; j < n; j += WG_THREADS) {
-            const float4 q = src[j];
-            const float dx = q.x - mx, dy = q.y - my, dz = q.z - mz;
-            const float d2 = dx * dx + dy * dy + dz * dz;
-            far2 = d2 < 3.0e38f ? fmaxf(far2, d2) : __builtin_inff();       // (NaN counts as infinity and stays)
+        for (int b = tid; b < L.nbox; b += THREADS) {
+            const WgBox q = boxes[b];
+            const float dx = fmaxf(q.hi[0] - mx, mx - q.lo[0]), dy = fmaxf(q.hi[1] - my, my - q.lo[1]), dz = fmaxf(q.hi[2] - mz, mz - q.lo[2]);
+            const float d2 = dx * dx + dy * dy + dz * dz + q.bad;
+            if (q.lo[0] <= q.hi[0] || q.bad != 0.f) far2 = d2 < 3.0e38f ? fmaxf(far2, d2) : __builtin_inff();       // (NaN counts as infinity and stays)
         }
         for (int o = 32; o > 0; o >>= 1) far2 = fmaxf(far2, __shfl_xor(far2, o));
         if (lane == 0) s_red[wave] = far2;
         __syncthreads();
 #pragma unroll
-        for (int w = 0; w < WG_WAVES; ++w) far2 = fmaxf(far2, s_red[w]);
+        for (int w = 0; w < WAVES; ++w) far2 = fmaxf(far2, s_red[w]);
         const float reach = (__builtin_sqrtf(far2) + __builtin_sqrtf(ex * ex + ey * ey + ez * ez)) * 1.00001f;
         const float cells = reach * inv_h + 2.0f;
         direct = !(cells < (float)(WG_CELLS * WG_MAX_WINDOWS));
@@ -326,83 +354,103 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
     }
 
     if (!direct) {
-        // ---- the spreading kernel's coefficients ----
-        const float e00 = wg_vgpr(0.8198235f),    e01 = wg_vgpr(-0.41093102f), e02 = wg_vgpr(0.08094943f);
-        const float o00 = wg_vgpr(0.65685374f),   o01 = wg_vgpr(-0.43981674f), o02 = wg_vgpr(0.14080364f);
-        const float e10 = wg_vgpr(0.15015647f),   e11 = wg_vgpr(0.37342498f),  e12 = wg_vgpr(-0.1214422f);
-        const float o10 = wg_vgpr(0.40670425f),   o11 = wg_vgpr(0.057586372f), o12 = wg_vgpr(-0.069855906f);
-        const float e20 = wg_vgpr(0.0018756188f), e21 = wg_vgpr(0.037506126f), e22 = wg_vgpr(0.04049774f);
-        const float o20 = wg_vgpr(0.013345578f),  o21 = wg_vgpr(0.05343353f),  o22 = wg_vgpr(0.01371953f);
-        const float half = wg_vgpr(0.5f), magic = wg_vgpr(WG_MAGIC), inv_hv = wg_vgpr(inv_h), sch = wg_vgpr(WG_SCALE * h);
+        // ---- the spreading kernel's coefficients, in fixed point ----
+        // A weight is made as a single-precision denormal: its bit pattern is the rounded integer, and no conversion is needed
+        // (4.7 clocks each).  Of the 2^-149 that takes 2^-12 comes with 1/r (WG_UNIT) and the rest with the coefficients, so that
+        // every factor is a normal number.  One unit is `scale` of a full weight: 2 scale (the largest weight) times the
+        // sources between two flushes stays below 2^32.
+        const int nit = (n + STEP - 1) / STEP, quarter = nit * (STEP / 4);
+        const bool flushes = nit * STEP > WG_FLUSH;
+        const float scale = flushes ? 1048000.0f : fminf(4190000.0f, 2147000000.0f / (float)(nit * STEP));
+        const float fix = scale * h * 0x1p-137f;
+        const float e00 = wg_vgpr(fix * 0.8198235f),    e01 = wg_vgpr(fix * -0.41093102f), e02 = wg_vgpr(fix * 0.08094943f);
+        const float o00 = wg_vgpr(fix * 0.65685374f),   o01 = wg_vgpr(fix * -0.43981674f), o02 = wg_vgpr(fix * 0.14080364f);
+        const float e10 = wg_vgpr(fix * 0.15015647f),   e11 = wg_vgpr(fix * 0.37342498f),  e12 = wg_vgpr(fix * -0.1214422f);
+        const float o10 = wg_vgpr(fix * 0.40670425f),   o11 = wg_vgpr(fix * 0.057586372f), o12 = wg_vgpr(fix * -0.069855906f);
+        const float e20 = wg_vgpr(fix * 0.0018756188f), e21 = wg_vgpr(fix * 0.037506126f), e22 = wg_vgpr(fix * 0.04049774f);
+        const float o20 = wg_vgpr(fix * 0.013345578f),  o21 = wg_vgpr(fix * 0.05343353f),  o22 = wg_vgpr(fix * 0.01371953f);
+        const float magic = wg_vgpr(WG_MAGIC), inv_hv = wg_vgpr(inv_h);
+        uint32_t emask = 0xff800000u;
+        asm volatile("" : "+v"(emask));
 
-        const int nit = (n + WG_STEP - 1) / WG_STEP;
-        const bool flushes = n > WG_FLUSH;
+        float lowest = 3.0e38f;                    // smallest n of any source, as magic + n
 
         for (int n_lo = 1; n_lo <= ncell; n_lo += WG_CELLS) {
             const int cells = min(WG_CELLS, ncell + 1 - n_lo);           // source cells n_lo .. n_lo + cells - 1
             const int e_lo  = 31 - __builtin_clz(n_lo);
             const int e_hi  = 31 - __builtin_clz(n_lo + cells - 1);
             const int used  = WG_R0 + cells + 5 + WG_OCT * (e_hi - e_lo);      // rows that hold anything
-            wg_f4 facc[WG_CHUNKS];
+            wg_f4 facc[CHUNKS];
 #pragma unroll
-            for (int i = 0; i < WG_CHUNKS; ++i) facc[i] = wg_f4{0.f, 0.f, 0.f, 0.f};
+            for (int i = 0; i < CHUNKS; ++i) facc[i] = wg_f4{0.f, 0.f, 0.f, 0.f};
 
             uint4* g4 = reinterpret_cast<uint4*>(s_grid);
+            auto me_again = [&]() { int v = tid; asm volatile("" : "+v"(v)); return v; };     // (keeps the addresses of these passes out of registers between them)
             __syncthreads();                                             // the previous window's product is done
-            for (int i = tid; i < WG_ROWS * WG_OBS / 4; i += WG_THREADS) g4[i] = make_uint4(0, 0, 0, 0);
+            for (int i = tid; i < used * (WG_OBS / 4); i += THREADS) g4[i] = make_uint4(0, 0, 0, 0);
             __syncthreads();
 
-            // byte address of a source's first node: row (n - n_lo) + 5 (e - e_lo), with n and e taken from float bits
-            const uint32_t base = (uint32_t)((WG_R0 - n_lo - WG_OCT * e_lo) * WG_OBS + obs) * 4u
-                                  - (0x4B400000u << 6) - 127u * (WG_OCT * WG_OBS * 4u);
-            const uint32_t first = 0x4B400000u + (uint32_t)n_lo;
-            char* lds = reinterpret_cast<char*>(s_grid);
+            // LDS address of a source's first node: row (n - n_lo) + 8 (e - e_lo), with n and e taken from float bits.  Sources
+            // that belong to no cell of this window go to the trash rows: with one window those are the observer itself and slots
+            // past the end (n is NaN) and pairs closer than h / 2 (n = 0, whose exponent takes the address below zero), all of
+            // which one unsigned minimum catches.
+            uint32_t base = (uint32_t)(uintptr_t)(wg_lds_u32*)s_grid + (uint32_t)((WG_R0 - n_lo - WG_OCT * e_lo) * WG_OBS + obs) * 4u
+                            - (WG_MAGIC_BITS << 6) - 127u * (WG_OCT * WG_OBS * 4u);
+            uint32_t trash = (uint32_t)(uintptr_t)(wg_lds_u32*)s_grid + (uint32_t)(WG_TRASH * WG_OBS + obs) * 4u;
+            asm volatile("" : "+v"(base), "+v"(trash));
+            const uint32_t first = WG_MAGIC_BITS + (uint32_t)n_lo;
 
-            const float4* p = src + wave * 4 + (lane >> 4);
-            float4 q0 = p[0];
-            int until = flushes ? WG_FLUSH / WG_STEP : nit;
+            // The four sources of a wave instruction come from four quarters of the sequence: neighbours in the chain lie in the
+            // same cells, and additions to one address take turns.
+            const float4* p = src + (lane >> 4) * quarter + wave * 2;
+            auto spread = [&](const float4& q, auto multi) {
+                float r2, inv, r;
+                wg_distance(me.x - q.x, me.y - q.y, me.z - q.z, r2, inv, r);
+                const float u  = __builtin_fmaf(r, inv_hv, magic);
+                const float nf = u - magic;
+                const float x  = __builtin_fmaf(r, inv_hv, -nf);
+                const uint32_t ub = __builtin_bit_cast(uint32_t, u);
+                const uint32_t eb = __builtin_bit_cast(uint32_t, nf) & emask;
+                const float c  = inv * __builtin_bit_cast(float, eb);                      // 2^e / r
+                const float x2 = x * x, xc = x * c;
+                const float E0 = __builtin_fmaf(__builtin_fmaf(e02, x2, e01), x2, e00), O0 = __builtin_fmaf(__builtin_fmaf(o02, x2, o01), x2, o00);
+                const float E1 = __builtin_fmaf(__builtin_fmaf(e12, x2, e11), x2, e10), O1 = __builtin_fmaf(__builtin_fmaf(o12, x2, o11), x2, o10);
+                const float E2 = __builtin_fmaf(__builtin_fmaf(e22, x2, e21), x2, e20), O2 = __builtin_fmaf(__builtin_fmaf(o22, x2, o21), x2, o20);
+                const float t0 = E0 * c, t1 = E1 * c, t2 = E2 * c;
+                uint32_t at = (ub << 6) + base + (eb >> 14);
+                if (decltype(multi)::value) at = ub - first < (uint32_t)cells ? at : trash;
+                else                        at = min(at, trash);
+                wg_lds_u32* a = (wg_lds_u32*)(uintptr_t)at;
+                auto add = [&](const int l, const float w) {
+                    __hip_atomic_fetch_add(a + l * WG_OBS, __builtin_bit_cast(uint32_t, w), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                };
+                add(0, __builtin_fmaf(-O2, xc, t2));
+                add(1, __builtin_fmaf(-O1, xc, t1));
+                add(2, __builtin_fmaf(-O0, xc, t0));
+                add(3, __builtin_fmaf(O0, xc, t0));
+                add(4, __builtin_fmaf(O1, xc, t1));
+                add(5, __builtin_fmaf(O2, xc, t2));
+                lowest = __builtin_fminf(lowest, u);
+            };
+            float4 q0 = p[0], q1 = p[1], q2 = p[STEP / 8], q3 = p[STEP / 8 + 1];
+            int until = flushes ? WG_FLUSH / STEP : nit;
             for (int it = 0;;) {
-#pragma unroll 2
-                for (; it < until; ++it) {
-                    const float4 q = q0;
-                    q0 = p[(size_t)(it + 1) * WG_STEP];
-                    float r2, inv, r;
-                    wg_distance(me.x - q.x, me.y - q.y, me.z - q.z, r2, inv, r);
-                    const float u  = __builtin_fmaf(r, inv_hv, magic);
-                    const uint32_t ub = __builtin_bit_cast(uint32_t, u);
-                    const float nf = u - magic;
-                    const float x  = __builtin_fmaf(r, inv_hv, -nf);
-                    const uint32_t nb = __builtin_bit_cast(uint32_t, nf);
-                    const float p2 = __builtin_bit_cast(float, nb & 0xff800000u);          // 2^e
-                    const float c  = (inv * sch) * p2;                                     // 2^e h / r, scaled
-                    const float x2 = x * x, xc = x * c;
-                    const float E0 = __builtin_fmaf(__builtin_fmaf(e02, x2, e01), x2, e00), O0 = __builtin_fmaf(__builtin_fmaf(o02, x2, o01), x2, o00);
-                    const float E1 = __builtin_fmaf(__builtin_fmaf(e12, x2, e11), x2, e10), O1 = __builtin_fmaf(__builtin_fmaf(o12, x2, o11), x2, o10);
-                    const float E2 = __builtin_fmaf(__builtin_fmaf(e22, x2, e21), x2, e20), O2 = __builtin_fmaf(__builtin_fmaf(o22, x2, o21), x2, o20);
-                    const float t0 = __builtin_fmaf(E0, c, half), t1 = __builtin_fmaf(E1, c, half), t2 = __builtin_fmaf(E2, c, half);
-                    const bool on = ub - first < (uint32_t)cells;
-                    if (on) {
-                        uint32_t* a = reinterpret_cast<uint32_t*>(lds + (base + (ub << 6) + (nb >> 23) * (uint32_t)(WG_OCT * WG_OBS * 4)));
-                        auto add = [&](const int row, const float w) {
-                            __hip_atomic_fetch_add(a + row * WG_OBS, (uint32_t)w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                        };
-                        add(0, __builtin_fmaf(-O2, xc, t2));
-                        add(1, __builtin_fmaf(-O1, xc, t1));
-                        add(2, __builtin_fmaf(-O0, xc, t0));
-                        add(3, __builtin_fmaf(O0, xc, t0));
-                        add(4, __builtin_fmaf(O1, xc, t1));
-                        add(5, __builtin_fmaf(O2, xc, t2));
+                auto stream = [&](auto multi) {
+                    for (; it < until; ++it) {
+                        p += STEP / 4;
+                        spread(q0, multi); spread(q1, multi);
+                        q0 = p[0]; q1 = p[1];
+                        spread(q2, multi); spread(q3, multi);
+                        q2 = p[STEP / 8]; q3 = p[STEP / 8 + 1];
                     }
-                    if (__builtin_amdgcn_ballot_w64(on) != ~0ull) {
-                        // (rare while there is one window: the observer itself, sources past the end, pairs closer than h / 2)
-                        if (!on && ub == 0x4B400000u && r2 != 0.0f && ok) s_near[obs] = 1;
-                    }
-                }
+                };
+                if (ncell > WG_CELLS) stream(wg_true{}); else stream(wg_false{});
                 if (!flushes) break;
                 __syncthreads();
+                const int tf = me_again();
 #pragma unroll
-                for (int i = 0; i < WG_CHUNKS; ++i) {
-                    const int q = tid + i * WG_THREADS;
+                for (int i = 0; i < CHUNKS; ++i) {
+                    const int q = tf + i * THREADS;
                     if (q < used * (WG_OBS / 4)) {
                         const uint4 v = g4[q];
                         facc[i] += wg_f4{(float)v.x, (float)v.y, (float)v.z, (float)v.w};
@@ -412,15 +460,16 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
                 }
                 __syncthreads();
                 if (it >= nit) break;
-                until = min(it + WG_FLUSH / WG_STEP, nit);
+                until = min(it + WG_FLUSH / STEP, nit);
             }
             if (!flushes) __syncthreads();
 
             // ---- bring the octaves together: node v = n_lo - 3 + p to row WG_R0 + p, zeros behind the last ----
             const int nodes = cells + 5;
+            const int tc = me_again();
 #pragma unroll
-            for (int i = 0; i < WG_CHUNKS; ++i) {
-                const int q = tid + i * WG_THREADS;
+            for (int i = 0; i < CHUNKS; ++i) {
+                const int q = tc + i * THREADS;
                 const int pn = (q >> 2) - WG_R0;
                 wg_f4 v = {0.f, 0.f, 0.f, 0.f};
                 if (pn >= 0 && pn < nodes) {
@@ -438,14 +487,16 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
                 facc[i] = v;
             }
             __syncthreads();
+            const int tw = me_again();
 #pragma unroll
-            for (int i = 0; i < WG_CHUNKS; ++i) {
-                const int q = tid + i * WG_THREADS;
-                if (q < WG_ROWS * (WG_OBS / 4)) reinterpret_cast<wg_f4*>(s_grid)[q] = facc[i];
+            for (int i = 0; i < CHUNKS; ++i) {
+                const int q = tw + i * THREADS;
+                if (q < (WG_R0 + nodes + 8) * (WG_OBS / 4)) reinterpret_cast<wg_f4*>(s_grid)[q] = facc[i];
             }
             __syncthreads();
 
             // ---- the grid at the wavenumbers: rows j = 0 .. on both sides of the middle ----
+            // A wave's tiles share the grid values; the tables come from L2, AHEAD groups of rows ahead.
             const float* g = reinterpret_cast<const float*>(s_grid);
             const int mid    = (nodes + 1) / 2;
             const int groups = (mid + 7) / 8;
@@ -453,52 +504,71 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
             const int mm     = lane >> 4;
             const float* gp  = g + (WG_R0 + mid + mm) * WG_OBS + obs;
             const float* gm  = g + (WG_R0 + mid - 1 - mm) * WG_OBS + obs;
-            for (int kt = wave; kt < L.nkt; kt += WG_WAVES) {
-                wg_f4 ec = {0.f, 0.f, 0.f, 0.f}, os = ec, oc = ec, es = ec;
-                const float4* tb = table + (size_t)kt * 64 + lane;
-                const size_t  ts = (size_t)L.nkt * 64;
-                float4 b0 = tb[0];
-                float y = (float)mm + 0.5f;
-#pragma unroll 2
-                for (int gr = 0; gr < groups; ++gr) {
-                    const float4 b = b0;
-                    b0 = tb[(size_t)min(gr + 1, WG_GROUPS - 1) * ts];
+            for (int kp = KT * wave; kp < L.nkt; kp += KT * WAVES) {
+                wg_f4 ec[KT], os[KT], oc[KT], es[KT];
 #pragma unroll
-                    for (int s = 0; s < 2; ++s) {
-                        const int off = (8 * gr + 4 * s) * WG_OBS;
-                        const float a = gp[off], m = gm[-off];
-                        const float E = a + m, O = a - m;
-                        const float bc = s ? b.z : b.x, bs = s ? b.w : b.y;
-                        ec = __builtin_amdgcn_mfma_f32_16x16x4f32(E, bc, ec, 0, 0, 0);
-                        os = __builtin_amdgcn_mfma_f32_16x16x4f32(O, bs, os, 0, 0, 0);
-                        if (SUMS) {
-                            oc = __builtin_amdgcn_mfma_f32_16x16x4f32(O * y, bc, oc, 0, 0, 0);
-                            es = __builtin_amdgcn_mfma_f32_16x16x4f32(E * y, bs, es, 0, 0, 0);
+                for (int t = 0; t < KT; ++t) ec[t] = os[t] = oc[t] = es[t] = wg_f4{0.f, 0.f, 0.f, 0.f};
+                const float4* tb = table + (size_t)kp * 64 + lane;
+                const size_t  ts = (size_t)L.nkt * 64;
+                const int     k2 = kp + 1 < L.nkt ? 64 : 0;                 // (an odd number of tiles: the last one twice, written once)
+                float4 b[AHEAD][KT];
+                auto fetch = [&](const int gr, float4 (&bb)[KT]) {
+                    const float4* at = tb + (size_t)min(gr, WG_GROUPS - 1) * ts;
+#pragma unroll
+                    for (int t = 0; t < KT; ++t) bb[t] = at[t * k2];
+                };
+#pragma unroll
+                for (int i = 0; i < AHEAD; ++i) fetch(i, b[i]);
+                float y = (float)mm + 0.5f;
+                for (int g0 = 0; g0 < groups; g0 += AHEAD) {
+#pragma unroll
+                    for (int i = 0; i < AHEAD; ++i) {
+                        const int gr = g0 + i;
+                        if (gr >= groups) break;
+#pragma unroll
+                        for (int s = 0; s < 2; ++s) {
+                            const int off = (8 * gr + 4 * s) * WG_OBS;
+                            const float a = gp[off], m = gm[-off];
+                            const float E = a + m, O = a - m;
+                            const float Oy = O * y, Ey = E * y;
+#pragma unroll
+                            for (int t = 0; t < KT; ++t) {
+                                const float bc = s ? b[i][t].z : b[i][t].x, bs = s ? b[i][t].w : b[i][t].y;
+                                ec[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(E, bc, ec[t], 0, 0, 0);
+                                os[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(O, bs, os[t], 0, 0, 0);
+                                if (SUMS) {
+                                    oc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(Oy, bc, oc[t], 0, 0, 0);
+                                    es[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(Ey, bs, es[t], 0, 0, 0);
+                                }
+                            }
+                            y += 4.0f;
                         }
-                        y += 4.0f;
+                        fetch(gr + AHEAD, b[i]);
                     }
                 }
-                const int k = kt * 16 + obs;
-                if (k < K) {
+#pragma unroll
+                for (int t = 0; t < KT; ++t) {
+                    const int k = (kp + t) * 16 + obs;
+                    if (k >= K) continue;
                     const WgWave w = waves[k];
                     const double ph = w.rev * (double)vc;
                     const float f  = (float)(ph - __builtin_floor(ph));
                     const float rc = __builtin_amdgcn_cosf(f), rs = __builtin_amdgcn_sinf(f);
-                    const float q1 = w.q / (WG_SCALE * h), q0s = w.q / WG_SCALE, dq = w.dq / WG_SCALE;
+                    const float q1 = w.q / (scale * h), q0s = w.q / scale, dq = w.dq / scale;
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        const int  t    = s_tok[mm * 4 + i];
-                        if (t < 0) continue;
+                        const int  tok  = s_tok[mm * 4 + i];
+                        if (tok < 0) continue;
                         const bool keep = slot0 + mm * 4 + i < n;
-                        const size_t row = zN + t;
-                        float2 v = make_float2(q1 * (ec[i] * rc - os[i] * rs), q1 * (ec[i] * rs + os[i] * rc));
+                        const size_t row = zN + tok;
+                        float2 v = make_float2(q1 * (ec[t][i] * rc - os[t][i] * rs), q1 * (ec[t][i] * rs + os[t][i] * rc));
                         float2* po = reinterpret_cast<float2*>(out + row * 2 * K) + k;
-                        if (n_lo > 1) { const float2 b = *po; v.x += b.x; v.y += b.y; }
+                        if (n_lo > 1) { const float2 o = *po; v.x += o.x; v.y += o.y; }
                         *po = keep ? v : make_float2(0.f, 0.f);
                         if (SUMS) {
                             // F0 = rot [ q h (vc G + Gy) - i q' h G ] with G = ec + i os, Gy = oc + i es
-                            const float gr_ = q0s * ((float)vc * ec[i] + oc[i]) + dq * os[i];
-                            const float gi_ = q0s * ((float)vc * os[i] + es[i]) - dq * ec[i];
+                            const float gr_ = q0s * ((float)vc * ec[t][i] + oc[t][i]) + dq * os[t][i];
+                            const float gi_ = q0s * ((float)vc * os[t][i] + es[t][i]) - dq * ec[t][i];
                             float c0 = gr_ * rc - gi_ * rs, s0 = gr_ * rs + gi_ * rc;
                             float* pc = cos_sums + row * K + k;
                             float* ps = sin_sums + row * K + k;
@@ -510,11 +580,12 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
                 }
             }
         }
+        if (lowest == WG_MAGIC && ok) s_near[obs] = 1;
     }
 
     // ---- pairs closer than h / 2, and everything where the grid is of no use ----
     __syncthreads();
-    for (int q = wave; q < WG_OBS; q += WG_WAVES) {
+    for (int q = wave; q < WG_OBS; q += WAVES) {
         const int t = s_tok[q];
         if (t < 0) continue;
         const size_t row = zN + t;
@@ -565,9 +636,10 @@ extern "C" int proteus_we_fwd_ws(const float* coords, int coords_layout,
     hipLaunchKernelGGL(we_grid_prepare_kernel, dim3(prep), dim3(256), 0, st, coords, coords_layout, wavenumbers, mask, (char*)workspace, Z, N, K);
     const dim3 grid((N + WG_OBS - 1) / WG_OBS, Z);
     const size_t lds = (size_t)WG_ROWS * WG_OBS * 4;
-    if (cos_sums)
-        hipLaunchKernelGGL((we_grid_kernel<true>), grid, dim3(WG_THREADS), lds, st, (const char*)workspace, wavenumbers, out, cos_sums, sin_sums, Z, N, K);
-    else
-        hipLaunchKernelGGL((we_grid_kernel<false>), grid, dim3(WG_THREADS), lds, st, (const char*)workspace, wavenumbers, out, cos_sums, sin_sums, Z, N, K);
+    const bool few = (long)grid.x * Z <= 256;
+#define WG_GO(S_, W_) hipLaunchKernelGGL((we_grid_kernel<S_, W_>), grid, dim3(W_ * 64), lds, st, (const char*)workspace, wavenumbers, out, cos_sums, sin_sums, Z, N, K)
+    if (cos_sums) { if (few) WG_GO(true, 16); else WG_GO(true, 8); }
+    else          { if (few) WG_GO(false, 16); else WG_GO(false, 8); }
+#undef WG_GO
     return (int)hipGetLastError();
 }
