@@ -211,6 +211,18 @@ int proteus_we_aniso_fwd_check(const float* coordsA, const float* coordsB, int c
                                const float* out, const float* d_cb, const float* d_k,
                                int Z, int N, int K, int tuning);
 
+/*
+ * proteus_we_aniso_fwd with a caller-provided workspace (as proteus_we_fwd_ws): through grids of the distances
+ * (we_aniso_grid.hip), one where all C-beta scales are equal and no derivative is wanted, otherwise one per term of an
+ * expansion of the phase in the C-beta projection; where those would be too many, the direct kernel does the work.
+ * partials: whether d_cb and d_k will be wanted, padded: whether there will be a mask (the size is the same, but not where it is 0).
+ */
+size_t proteus_we_aniso_fwd_workspace_bytes(int Z, int N, int K, int partials, int padded, int tuning);
+int proteus_we_aniso_fwd_ws(const float* coordsA, const float* coordsB, int coords_layout,
+                            const float* cb_magnitudes, const float* wavenumbers, const uint8_t* mask,
+                            float* out, float* d_cb, float* d_k, void* workspace, size_t workspace_bytes,
+                            int Z, int N, int K, int tuning, void* stream);
+
 int         proteus_we_aniso_num_variants(void);
 const char* proteus_we_aniso_variant_name(int tuning);
 

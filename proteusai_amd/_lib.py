@@ -21,7 +21,7 @@ SYMBOLS = [
     "proteus_version", "proteus_strerror",
     "proteus_we_fwd", "proteus_we_fwd_check", "proteus_we_fwd_workspace_bytes", "proteus_we_fwd_ws", "proteus_we_legacy_fwd", "proteus_we_dropout_fwd", "proteus_we_dropout_fwd_check",
     "proteus_we_dropout_threshold", "proteus_we_num_variants", "proteus_we_variant_name",
-    "proteus_we_aniso_fwd", "proteus_we_aniso_fwd_check", "proteus_we_aniso_num_variants", "proteus_we_aniso_variant_name",
+    "proteus_we_aniso_fwd", "proteus_we_aniso_fwd_check", "proteus_we_aniso_fwd_workspace_bytes", "proteus_we_aniso_fwd_ws", "proteus_we_aniso_num_variants", "proteus_we_aniso_variant_name",
     "proteus_we_bwd_workspace_bytes", "proteus_we_bwd", "proteus_we_bwd_check", "proteus_we_bwd_static", "proteus_we_aniso_bwd", "proteus_we_aniso_bwd_check",
     "proteus_geo_attn_fwd", "proteus_geo_attn_fwd_check", "proteus_geo_attn_legacy_fwd", "proteus_geo_attn_bwd",
     "proteus_geo_attn_fwd_workspace_bytes", "proteus_geo_attn_fwd_ws", "proteus_geo_attn_fwd_ws_check",
@@ -81,6 +81,10 @@ def load():
     sz = ctypes.c_size_t
     lib.proteus_we_fwd_workspace_bytes.restype = sz
     lib.proteus_we_fwd_workspace_bytes.argtypes = [ci, ci, ci, ci]
+    lib.proteus_we_aniso_fwd_workspace_bytes.restype = sz
+    lib.proteus_we_aniso_fwd_workspace_bytes.argtypes = [ci, ci, ci, ci, ci, ci]
+    lib.proteus_we_aniso_fwd_ws.restype = ci
+    lib.proteus_we_aniso_fwd_ws.argtypes = [vp, vp, ci, vp, vp, vp, vp, vp, vp, vp, sz, ci, ci, ci, ci, vp]
     lib.proteus_we_fwd_ws.restype = ci
     lib.proteus_we_fwd_ws.argtypes = [vp, ci, vp, vp, vp, vp, vp, vp, sz, ci, ci, ci, ci, vp]
     lib.proteus_we_bwd_workspace_bytes.restype = sz

@@ -25,6 +25,7 @@
 #include <type_traits>
 #include "proteus_hip.h"
 #include "we_ranked.h"
+#include "we_aniso_direct.h"
 
 namespace {
 
@@ -48,8 +49,9 @@ void we_aniso_fwd_kernel(const float* __restrict__ coordsA, const float* __restr
                          const float* __restrict__ cb_magnitudes, const float* __restrict__ wavenumbers,
                          const uint8_t* __restrict__ mask,
                          float* __restrict__ out, float* __restrict__ d_cb, float* __restrict__ d_k,
-                         const int N, const int K)
+                         const int N, const int K, const int* __restrict__ taken)
 {
+    if (taken && *taken != 0) return;
     __shared__ float4 s_ka[WA_JB + WA_WAVES];    // source positions   (padding: the loop reads one step ahead)
     __shared__ float4 s_kb[WA_JB + WA_WAVES];    // source C-beta vectors
     __shared__ int    s_wcount[WA_WAVES];
@@ -342,13 +344,13 @@ constexpr int kNumVariants = (int)(sizeof(kVariants) / sizeof(kVariants[0]));
 
 template <int KT, bool SPLIT, bool GRADS>
 int launch(const float* ca, const float* cbv, int layout, const float* cbm, const float* wn, const uint8_t* mask,
-           float* out, float* d_cb, float* d_k, int Z, int N, int K, hipStream_t st)
+           float* out, float* d_cb, float* d_k, int Z, int N, int K, const int* taken, hipStream_t st)
 {
     const int iblocks = (N + 63) / 64;
     const int ktiles  = SPLIT ? (K + KT - 1) / KT : (K + KT * WA_WAVES - 1) / (KT * WA_WAVES);
     dim3 grid(iblocks, ktiles, Z);
     hipLaunchKernelGGL((we_aniso_fwd_kernel<KT, SPLIT, GRADS>), grid, dim3(WA_THREADS), 0, st,
-                       ca, cbv, layout, cbm, wn, mask, out, d_cb, d_k, N, K);
+                       ca, cbv, layout, cbm, wn, mask, out, d_cb, d_k, N, K, taken);
     return (int)hipGetLastError();
 }
 
@@ -384,6 +386,13 @@ extern "C" int proteus_we_aniso_fwd(const float* coordsA, const float* coordsB, 
     const int rc = proteus_we_aniso_fwd_check(coordsA, coordsB, coords_layout, cb_magnitudes, wavenumbers, mask,
                                               out, d_cb, d_k, Z, N, K, tuning);
     if (rc != PROTEUS_OK) return rc;
+    return proteus_we_aniso_direct(coordsA, coordsB, coords_layout, cb_magnitudes, wavenumbers, mask, out, d_cb, d_k, Z, N, K, tuning, nullptr, stream);
+}
+
+int proteus_we_aniso_direct(const float* coordsA, const float* coordsB, int coords_layout,
+                            const float* cb_magnitudes, const float* wavenumbers, const uint8_t* mask,
+                            float* out, float* d_cb, float* d_k, int Z, int N, int K, int tuning, const int* taken, void* stream)
+{
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
 
     int kt = kVariants[tuning].kt;
@@ -409,8 +418,8 @@ extern "C" int proteus_we_aniso_fwd(const float* coordsA, const float* coordsB, 
         }
         if (!d_cb && N >= 4 * 64) split = true;
     }
-#define WA_GO(KT_, GR_) (split ? launch<KT_, true, GR_>(coordsA, coordsB, coords_layout, cb_magnitudes, wavenumbers, mask, out, d_cb, d_k, Z, N, K, st) \
-                               : launch<KT_, false, GR_>(coordsA, coordsB, coords_layout, cb_magnitudes, wavenumbers, mask, out, d_cb, d_k, Z, N, K, st))
+#define WA_GO(KT_, GR_) (split ? launch<KT_, true, GR_>(coordsA, coordsB, coords_layout, cb_magnitudes, wavenumbers, mask, out, d_cb, d_k, Z, N, K, taken, st) \
+                               : launch<KT_, false, GR_>(coordsA, coordsB, coords_layout, cb_magnitudes, wavenumbers, mask, out, d_cb, d_k, Z, N, K, taken, st))
     if (d_cb) {
         if (kt == 16) return WA_GO(16, true);
         return WA_GO(8, true);

@@ -1,0 +1,470 @@
+// Anisotropic (C-beta scaled) Wavefunction Embedding forward through distance grids, for gfx950 (MI355X).
+//
+// What it computes: the sums of we_aniso_fwd.hip, with R = a_i - a_j, r = |R|, A = (b_j . R)/r and phase k (r - cb_k A):
+//     F(k, cb) = sum_j e^(i k (r_j - cb A_j)) / r_j (out: cos at even, sin at odd features), d_k = dF/dk, d_cb = dF/dcb.
+// The grids are those of we_grid.hip (spreading kernel, octaves, fixed point, product), with two changes:
+//   - Position: with c the middle of the scales, r_j - cb_k A_j = (r_j - c A_j) - (cb_k - c) A_j, and it is r - c A that is spread.
+//     If all scales are equal, as the module constructs them, that is all there is to it: one grid, as in the isotropic case.
+//   - Otherwise the rest of the phase is expanded in Chebyshev polynomials of A/b, b the longest C-beta vector:
+//     e^(-i z t) = sum_p (2 - delta_p0) (-i)^p J_p(z) T_p(t),  z = k (cb_k - c) b,  t = A/b     (Jacobi-Anger)
+//     with one grid per term, of the weights T_p(A_j/b) / r_j.  The terms come two at a time (two grids share the LDS and a pass
+//     over the sources); (z/2)^P / P! < 1e-7 sets their number P: 2 with partial derivatives and equal scales, about 10 for
+//     scales 1 +- 0.5 and wavelengths down to 3.7 A.
+//   d_cb needs J_p' in place of J_p times k b, d_k that times (cb_k - c) b plus the k-derivative of the grids (we_grid.hip's F0).
+// Per pair of tokens and pair of terms: about 40 vector instructions and twelve integer LDS additions, against 10 instructions per
+// wavenumber in the direct kernel.
+// Pairs that no cell takes (r - c A below h/2, or r so small against r - c A that the weight leaves its fixed-point range) are summed
+// directly, as are all pairs of a workgroup whose distances need too many windows.  Where the expansion needs so many terms that the
+// direct kernel is the faster one, which only the device can tell, that kernel does the work and this one returns at once.
+#include "we_grid.h"
+#include "we_aniso_direct.h"
+
+namespace {
+
+using namespace proteus_we_grid;
+
+constexpr int WA_FLUSH = 1024;           // sources between two flushes: 1024 x 2 x 2^20 is what a signed cell holds
+
+// ---- preparation: one launch for the lists of sources, one for the tables, which need the longest C-beta vector ----
+
+__global__ __launch_bounds__(256)
+void we_aniso_grid_sources_kernel(const float* __restrict__ coordsA, const float* __restrict__ coordsB, const int layout,
+                                  const uint8_t* __restrict__ mask, char* __restrict__ ws, const int Z, const int N, const int K)
+{
+    const WgLayout L = wg_layout(Z, N, K, true);
+    const int z = blockIdx.x / L.blocks, j = (blockIdx.x % L.blocks) * 256 + threadIdx.x;
+    const int slot = wg_compact(coordsA, layout, mask, ws, L, N, blockIdx.x);
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (j < N && !(mask && mask[(size_t)z * N + j])) {
+        const float* b = coordsB + (size_t)z * N * 3;
+        if (layout == PROTEUS_COORDS_SOA) v = make_float4(b[j], b[(size_t)N + j], b[2 * (size_t)N + j], 0.f);
+        else                              v = make_float4(b[3 * (size_t)j], b[3 * (size_t)j + 1], b[3 * (size_t)j + 2], 0.f);
+    }
+    if (slot < L.npad) reinterpret_cast<float4*>(ws + L.sources_b)[(size_t)z * L.npad + slot] = v;
+    const float b2 = wg_block_max(v.x * v.x + v.y * v.y + v.z * v.z);
+    if (threadIdx.x == 0) reinterpret_cast<float*>(ws + L.lengths)[blockIdx.x] = b2;
+}
+
+__global__ __launch_bounds__(256)
+void we_aniso_grid_tables_kernel(const float* __restrict__ cb_magnitudes, const float* __restrict__ wavenumbers,
+                                 char* __restrict__ ws, const int Z, const int N, const int K, const int partials)
+{
+    const WgLayout L = wg_layout(Z, N, K, true);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const float inv_h = wg_cells_per_length(wavenumbers, K);
+    const double h = 1.0 / (double)inv_h;
+
+    float b2 = 0.f, hi = -3.0e38f, lo = -3.0e38f;                       // lo: largest of -cb
+    for (int i = tid; i < Z * L.blocks; i += 256) b2 = fmaxf(b2, reinterpret_cast<const float*>(ws + L.lengths)[i]);
+    bool bad = false;
+    for (int k = tid; k < K; k += 256) { const float c = cb_magnitudes[k]; bad |= !(fabsf(c) < 1.0e18f); hi = fmaxf(hi, c); lo = fmaxf(lo, -c); }
+    b2 = wg_block_max(bad ? __builtin_inff() : b2);
+    hi = wg_block_max(hi); lo = wg_block_max(lo);
+    const float mid = 0.5f * (hi - lo), b = __builtin_sqrtf(b2) * 1.0001f;
+    float z = 0.f;
+    for (int k = tid; k < K; k += 256) z = fmaxf(z, fabsf(wavenumbers[k] * (cb_magnitudes[k] - mid)));
+    z = wg_block_max(z) * b;
+    // number of terms: the tail of the series starts with 2 J_P(z) <= 2 (z/2)^P / P! (at the one wavenumber where z is largest), that of
+    // its derivative with J_(P-1)(z)
+    int terms = 0;
+    if (b < 1.0e18f && z < 20.0f) {
+        float t = 1.0f;
+        for (terms = 1; terms <= WG_MAX_TERMS; ++terms) { t *= 0.5f * z / (float)terms; if (2.0f * t < 3.0e-7f) break; }
+        terms += partials;
+        if (terms > WG_MAX_TERMS) terms = 0;
+    }
+    if (terms > 1) {
+        // The direct kernel or the grids?  Estimated microseconds (measured at K = 256, 1 x 1000 ... 8 x 2000 tokens, 4 to 12 terms): the direct
+        // kernel takes 0.34 ps per pair and wavenumber with partial derivatives and 0.24 without; a pass over the sources takes a round of
+        // workgroups (two per compute unit) 22 us for its grids and products and 0.059 us per source, down to 0.026 for few workgroups.
+        float pairs = 0.f, nmax = 0.f, groups = 0.f, ext = 0.f;
+        for (int i = tid; i < Z; i += 256) {
+            const float n = (float)reinterpret_cast<const int*>(ws + L.counts)[i];
+            pairs += n * n; nmax = fmaxf(nmax, n); groups += __builtin_ceilf(n / WG_OBS);
+        }
+        float far[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};           // extent of the batch, from its first token
+        const float4 at = reinterpret_cast<const float4*>(ws + L.sources)[0];
+        for (int i = tid; i < Z * L.nbox; i += 256) {
+            const WgBox q = reinterpret_cast<const WgBox*>(ws + L.boxes)[i];
+            if (!(q.lo[0] <= q.hi[0])) continue;
+            far[0] = fmaxf(far[0], q.hi[0] - at.x); far[1] = fmaxf(far[1], q.hi[1] - at.y); far[2] = fmaxf(far[2], q.hi[2] - at.z);
+            far[3] = fmaxf(far[3], at.x - q.lo[0]); far[4] = fmaxf(far[4], at.y - q.lo[1]); far[5] = fmaxf(far[5], at.z - q.lo[2]);
+        }
+        for (int c = 0; c < 3; ++c) { const float e = wg_block_max(far[c]) + wg_block_max(far[3 + c]); ext += e * e; }
+        pairs = wg_block_sum(pairs); groups = wg_block_sum(groups); nmax = wg_block_max(nmax);
+        const float cells   = 0.7f * __builtin_sqrtf(ext) * (1.0f / WG_UNIT) * inv_h;
+        const float windows = __builtin_ceilf(fmaxf(1.0f, cells / (float)WgGrid<2>::CELLS));
+        const float grid    = (float)((terms + 1) / 2) * windows * (22.0f + (0.026f + 0.033f * fminf(1.0f, groups / 512.0f)) * nmax) * fmaxf(1.0f, groups / 512.0f);
+        const float direct  = pairs * (float)K * (partials ? 3.4e-7f : 2.4e-7f);
+        if (!(grid < direct)) terms = 0;
+    }
+    const int unit = (int)blockIdx.x * 4 + (tid >> 6);
+    if (unit == 0 && lane == 0) {
+        WgParams* p = reinterpret_cast<WgParams*>(ws);
+        p->inv_h = inv_h; p->h = (float)h; p->cb_mid = mid; p->b_max = b; p->terms = terms;
+    }
+    const int rows = WG_GROUPS * L.nkt;
+    if (unit < rows) { wg_fill_tables(wavenumbers, ws, L, K, h, unit); return; }
+    // (2 - delta_p0) J_p and its derivative: four orders of 16 wavenumbers per wave, by the power series in double precision (|z| <= 10)
+    const int kt = (unit - rows) % L.nkt, p = (unit - rows) / L.nkt * 4 + (lane >> 4), k = kt * 16 + (lane & 15);
+    if (p >= terms) return;
+    const double x = k < K ? 0.5 * (double)(wavenumbers[k] * (cb_magnitudes[k] - mid)) * (double)b : 0.0;
+    auto bessel = [&](const int n) {
+        double term = 1.0;
+        for (int i = 1; i <= n; ++i) term *= x / (double)i;
+        double s = term;
+        for (int m = 1; m <= 40; ++m) { term *= -x * x / ((double)m * (double)(m + n)); s += term; }
+        return s;
+    };
+    const double j = bessel(p), jd = p ? 0.5 * (bessel(p - 1) - bessel(p + 1)) : -bessel(1);
+    const double f = p ? 2.0 : 1.0;
+    reinterpret_cast<float2*>(ws + L.terms)[(size_t)p * L.nkt * 16 + k] = make_float2((float)(f * j), (float)(f * jd));
+}
+
+// ---- main kernel ----
+
+// What decides whether a pair has a cell: n = rint((r - c A)/h) >= 1 and 2^floor(log2 n) h / r <= 2.
+struct Place { float A, r, inv, u, nf, x, c; uint32_t eb; };
+
+__device__ __forceinline__ Place wa_place(const float dx, const float dy, const float dz, const float4& b, const float mid, const float inv_h, const float magic, const uint32_t emask, float& r2)
+{
+    Place p;
+    wg_distance(dx, dy, dz, r2, p.inv, p.r);
+    p.A = (b.x * dx + b.y * dy + b.z * dz) * p.inv;
+    const float s = __builtin_fmaf(-mid, p.A, p.r);
+    p.u  = __builtin_fmaf(s, inv_h, magic);
+    p.nf = __builtin_fmaxf(p.u, magic) - magic;               // (a value that is not a number becomes 0)
+    p.x  = __builtin_fmaf(s, inv_h, -p.nf);
+    p.eb = __builtin_bit_cast(uint32_t, p.nf) & emask;
+    p.c  = p.inv * __builtin_bit_cast(float, p.eb);           // 2^e / r; 0 for n = 0
+    return p;
+}
+
+template <bool GRADS>
+__device__ void wa_direct(const float4* __restrict__ src, const float4* __restrict__ srcb, const int n, const float xi, const float yi, const float zi,
+                          const float mid, const float inv_h, const float climit, const bool all,
+                          const float* __restrict__ cb_magnitudes, const float* __restrict__ wavenumbers,
+                          float* __restrict__ o, float* __restrict__ ob, float* __restrict__ ok, const int K, const int lane)
+{
+    for (int kb = 0; kb < K; kb += 128) {
+        float kr[2], cb[2], s[2][GRADS ? 6 : 2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int k = kb + 64 * u + lane;
+            kr[u] = (float)((k < K ? (double)wavenumbers[k] : 0.0) * 0.15915494309189533577);
+            cb[u] = k < K ? cb_magnitudes[k] : 0.f;
+#pragma unroll
+            for (int i = 0; i < (GRADS ? 6 : 2); ++i) s[u][i] = 0.f;
+        }
+        for (int j0 = 0; j0 < n; j0 += 64) {
+            const float4 q = src[j0 + lane];
+            float r2;
+            const Place p = wa_place(xi - q.x, yi - q.y, zi - q.z, srcb[j0 + lane], mid * WG_UNIT, inv_h, WG_MAGIC, 0xff800000u, r2);
+            const bool near = !(p.u > WG_MAGIC) || p.c > climit;
+            uint64_t todo = __builtin_amdgcn_ballot_w64(j0 + lane < n && r2 != 0.0f && (all || near));
+            const float r = p.r * (1.0f / WG_UNIT), m = p.inv * WG_UNIT;
+            while (todo) {
+                const int b = __builtin_ctzll(todo);
+                todo &= todo - 1;
+                const float rb = wg_lane(r, b), mb = wg_lane(m, b), Ab = wg_lane(p.A, b);
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const float ph = __builtin_amdgcn_fractf(__builtin_fmaf(-cb[u], Ab, rb) * kr[u]);
+                    const float cs = __builtin_amdgcn_cosf(ph), sn = __builtin_amdgcn_sinf(ph);
+                    s[u][0] = __builtin_fmaf(cs, mb, s[u][0]);
+                    s[u][1] = __builtin_fmaf(sn, mb, s[u][1]);
+                    if constexpr (GRADS) {
+                        s[u][2] += cs; s[u][3] += sn;
+                        s[u][4] = __builtin_fmaf(cs, mb * Ab, s[u][4]);
+                        s[u][5] = __builtin_fmaf(sn, mb * Ab, s[u][5]);
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int k = kb + 64 * u + lane;
+            if (k >= K) continue;
+            auto put = [&](float* to, float re, float im) {
+                if (!all) { re += to[2 * k]; im += to[2 * k + 1]; }
+                to[2 * k] = re; to[2 * k + 1] = im;
+            };
+            put(o, s[u][0], s[u][1]);
+            if constexpr (GRADS) {
+                put(ok, -s[u][3] + cb[u] * s[u][5], s[u][2] - cb[u] * s[u][4]);
+                put(ob, wavenumbers[k] * s[u][5], -wavenumbers[k] * s[u][4]);
+            }
+        }
+    }
+}
+
+// GP  grids per pass over the sources: 1 where the expansion has a single term (then its weights are those of the isotropic kernel,
+//     unsigned denormals), 2 otherwise (signed weights, through the low bits of a magic sum)
+template <bool GRADS, int GP>
+__device__ __forceinline__ void wa_grids(uint32_t* s_grid, int* s_near, const int* s_tok, const char* __restrict__ ws, const WgLayout& L,
+                                         const float* __restrict__ cb_magnitudes, const float* __restrict__ wavenumbers,
+                                         float* __restrict__ out, float* __restrict__ d_cb, float* __restrict__ d_k,
+                                         const float4* __restrict__ src, const float4* __restrict__ srcb, const float4& me, const bool ok,
+                                         const int n, const int slot0, const int ncell, const size_t zN, const int K)
+{
+    constexpr int THREADS = 512, WAVES = 8;
+    constexpr int STEP   = WAVES * 8;                     // sources per iteration: a wave takes 16 observers x 4 sources, twice
+    constexpr int CHUNKS = (WG_ROWS * WG_OBS / 4 + THREADS - 1) / THREADS;
+    constexpr int CELLS  = WgGrid<GP>::CELLS;
+    constexpr int FLUSH  = GP == 1 ? WG_FLUSH : WA_FLUSH;
+    constexpr bool SIGNED = GP == 2;
+    const int tid = threadIdx.x, lane = tid & 63, obs = lane & 15, mm = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const WgParams* __restrict__ params = reinterpret_cast<const WgParams*>(ws);
+    const float inv_h = params->inv_h * (1.0f / WG_UNIT), h = params->h, mid_cb = params->cb_mid, bmax = params->b_max;
+    const int terms = params->terms;
+    const float4* __restrict__ table = reinterpret_cast<const float4*>(ws + L.table);
+    const WgWave* __restrict__ waves = reinterpret_cast<const WgWave*>(ws + L.waves);
+    const float2* __restrict__ coef = reinterpret_cast<const float2*>(ws + L.terms);
+
+    const int nit = (n + STEP - 1) / STEP, quarter = nit * (STEP / 4);
+    const bool flushes = nit * STEP > FLUSH;
+    const float scale = GP == 1 ? (flushes ? 1048000.0f : fminf(4190000.0f, 2147000000.0f / (float)(nit * STEP)))
+                                : (flushes ? 1048000.0f : fminf(2090000.0f, 1073000000.0f / (float)(nit * STEP)));
+    const WgKernel kernel(GP == 1 ? scale * h * 0x1p-137f : scale * h * WG_UNIT);
+    const float magic = wg_vgpr(WG_MAGIC), inv_hv = wg_vgpr(inv_h), midv = wg_vgpr(mid_cb * WG_UNIT), climit = wg_vgpr(2.0f * inv_h);
+    const float inv_b = wg_vgpr(bmax > 0.f ? 1.0f / bmax : 0.f);
+    uint32_t emask = 0xff800000u, mbits = WG_MAGIC_BITS;
+    asm volatile("" : "+v"(emask), "+v"(mbits));
+    float lowest = 3.0e38f, largest = 0.f;
+
+    for (int p0 = 0; p0 < terms; p0 += GP) {
+        for (int n_lo = 1; n_lo <= ncell; n_lo += CELLS) {
+            const int cells = min(CELLS, ncell + 1 - n_lo);
+            const int e_lo  = 31 - __builtin_clz(n_lo), e_hi = 31 - __builtin_clz(n_lo + cells - 1);
+            const int used  = WG_R0 + cells + 5 + WG_OCT * (e_hi - e_lo);
+            wg_f4 facc[CHUNKS];
+#pragma unroll
+            for (int i = 0; i < CHUNKS; ++i) facc[i] = wg_f4{0.f, 0.f, 0.f, 0.f};
+            __syncthreads();
+            wg_clear<GP, THREADS>(s_grid, used);
+            __syncthreads();
+
+            uint32_t base = (uint32_t)(uintptr_t)(wg_lds_u32*)s_grid + (uint32_t)((WG_R0 - n_lo - WG_OCT * e_lo) * WG_OBS + obs) * 4u
+                            - (WG_MAGIC_BITS << 6) - 127u * (WG_OCT * WG_OBS * 4u);
+            uint32_t trash = (uint32_t)(uintptr_t)(wg_lds_u32*)s_grid + (uint32_t)(WgGrid<GP>::TRASH * WG_OBS + obs) * 4u;
+            asm volatile("" : "+v"(base), "+v"(trash));
+            const uint32_t first = WG_MAGIC_BITS + (uint32_t)n_lo;
+
+            const int from = (lane >> 4) * quarter + wave * 2;
+            const float4* p = src + from;
+            const float4* pb = srcb + from;
+            auto spread = [&](const float4& q, const float4& qb) {
+                float r2;
+                const Place w = wa_place(me.x - q.x, me.y - q.y, me.z - q.z, qb, midv, inv_hv, magic, emask, r2);
+                float wt[6];
+                kernel(w.x, w.c, wt);
+                const uint32_t ub = __builtin_bit_cast(uint32_t, w.nf + magic);
+                uint32_t at = (ub << 6) + base + (w.eb >> 14);
+                at = ub - first < (uint32_t)cells && !(w.c > climit) ? at : trash;
+                lowest  = __builtin_fminf(lowest, w.u);
+                largest = __builtin_fmaxf(largest, w.c);
+                wg_lds_u32* a = (wg_lds_u32*)(uintptr_t)at;
+                auto add = [&](const int row, const uint32_t v) { __hip_atomic_fetch_add(a + row * WG_OBS, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
+                if (GP == 1) {
+#pragma unroll
+                    for (int l = 0; l < 6; ++l) add(l, __builtin_bit_cast(uint32_t, wt[l]));
+                } else {
+                    // T_p0 and T_(p0+1) of t = A/b by their recurrence, two orders at a time
+                    const float t = w.A * inv_b, t2 = t + t;
+                    float Ta = 1.0f, Tb = t;
+                    for (int i = 0; i < p0; i += 2) { Ta = __builtin_fmaf(t2, Tb, -Ta); Tb = __builtin_fmaf(t2, Ta, -Tb); }
+#pragma unroll
+                    for (int l = 0; l < 6; ++l) {
+                        add(l, __builtin_bit_cast(uint32_t, __builtin_fmaf(wt[l], Ta, magic)) - mbits);
+                        add(l + WgGrid<GP>::ROWS, __builtin_bit_cast(uint32_t, __builtin_fmaf(wt[l], Tb, magic)) - mbits);
+                    }
+                }
+            };
+            float4 qa = p[0], qb = p[1], ba = pb[0], bb = pb[1];
+            int until = flushes ? FLUSH / STEP : nit;
+            for (int it = 0;;) {
+                for (; it < until; ++it) {
+                    p += STEP / 4; pb += STEP / 4;
+                    spread(qa, ba);
+                    qa = p[0]; ba = pb[0];
+                    spread(qb, bb);
+                    qb = p[1]; bb = pb[1];
+                }
+                if (!flushes) break;
+                __syncthreads();
+                wg_flush<GP, THREADS, CHUNKS, SIGNED>(s_grid, facc, used, it >= nit);
+                __syncthreads();
+                if (it >= nit) break;
+                until = min(it + FLUSH / STEP, nit);
+            }
+            if (!flushes) __syncthreads();
+            wg_combine<GP, THREADS, CHUNKS, SIGNED>(s_grid, facc, n_lo, cells, flushes);
+            __syncthreads();
+
+            const int mid    = (cells + 6) / 2;
+            const int groups = (mid + 7) / 8;
+            const int vc     = n_lo - 3 + mid;
+            const bool more  = n_lo > 1 || p0 > 0;
+            for (int kp = wave; kp < L.nkt; kp += WAVES) {
+                const int k = kp * 16 + obs;
+                float2 o[4], ob[4], okk[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[i] = ob[i] = okk[i] = make_float2(0.f, 0.f);
+                const WgWave w = waves[k];
+                const double ph = w.rev * (double)vc;
+                const float f  = (float)(ph - __builtin_floor(ph));
+                const float rc = __builtin_amdgcn_cosf(f), rs = __builtin_amdgcn_sinf(f);
+                const float q1 = w.q / (scale * h), q0s = w.q / scale, dq = w.dq / scale;
+                const float wn = k < K ? wavenumbers[k] : 0.f, kb = wn * bmax, db = k < K ? (cb_magnitudes[k] - mid_cb) * bmax : 0.f;
+#pragma unroll
+                for (int g = 0; g < GP; ++g) {
+                    if (p0 + g >= terms) break;
+                    wg_f4 ec[1], os[1], oc[1], es[1];
+                    wg_product<1, 2, GRADS>(reinterpret_cast<const float*>(s_grid) + g * WgGrid<GP>::ROWS * WG_OBS, mid, groups,
+                                            table + (size_t)kp * 64 + lane, (size_t)L.nkt * 64, 0, ec, os, oc, es);
+                    const float2 J = coef[(size_t)(p0 + g) * L.nkt * 16 + k];
+                    const int turn = (p0 + g) & 3;                                 // (-i)^p
+                    auto turned = [&](const float x, const float y) {
+                        return turn == 0 ? make_float2(x, y) : turn == 1 ? make_float2(y, -x) : turn == 2 ? make_float2(-x, -y) : make_float2(-y, x);
+                    };
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float2 F = turned(q1 * (ec[0][i] * rc - os[0][i] * rs), q1 * (ec[0][i] * rs + os[0][i] * rc));
+                        o[i].x += J.x * F.x; o[i].y += J.x * F.y;
+                        if (GRADS) {
+                            const float gr = q0s * ((float)vc * ec[0][i] + oc[0][i]) + dq * os[0][i];
+                            const float gi = q0s * ((float)vc * os[0][i] + es[0][i]) - dq * ec[0][i];
+                            const float2 D = turned(-(gr * rs + gi * rc), gr * rc - gi * rs);          // dF/dk = i F0
+                            ob[i].x  += kb * J.y * F.x;                 ob[i].y  += kb * J.y * F.y;
+                            okk[i].x += db * J.y * F.x + J.x * D.x;     okk[i].y += db * J.y * F.y + J.x * D.y;
+                        }
+                    }
+                }
+                if (k >= K) continue;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int tok = s_tok[mm * 4 + i];
+                    if (tok < 0) continue;
+                    const bool keep = slot0 + mm * 4 + i < n;
+                    auto put = [&](float* to, float2 v) {
+                        float2* at = reinterpret_cast<float2*>(to + (zN + tok) * 2 * K) + k;
+                        if (more) { const float2 was = *at; v.x += was.x; v.y += was.y; }
+                        *at = keep ? v : make_float2(0.f, 0.f);
+                    };
+                    put(out, o[i]);
+                    if (GRADS) { put(d_cb, ob[i]); put(d_k, okk[i]); }
+                }
+            }
+        }
+    }
+    if (ok && (!(lowest > WG_MAGIC) || largest > climit)) s_near[obs] = 1;
+}
+
+template <bool GRADS>
+__global__ __launch_bounds__(512, 4)
+void we_aniso_grid_kernel(const char* __restrict__ ws, const float* __restrict__ cb_magnitudes, const float* __restrict__ wavenumbers,
+                          float* __restrict__ out, float* __restrict__ d_cb, float* __restrict__ d_k, const int Z, const int N, const int K)
+{
+    constexpr int THREADS = 512, WAVES = 8;
+    extern __shared__ __align__(16) uint32_t s_grid[];
+    __shared__ float s_red[WAVES];
+    __shared__ int   s_near[WG_OBS];
+    __shared__ int   s_tok[WG_OBS];
+
+    const WgLayout L = wg_layout(Z, N, K, true);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int z = blockIdx.y;
+    const size_t zN = (size_t)z * N;
+    const int n = reinterpret_cast<const int*>(ws + L.counts)[z];
+    const float4* __restrict__ src  = reinterpret_cast<const float4*>(ws + L.sources) + (size_t)z * L.npad;
+    const float4* __restrict__ srcb = reinterpret_cast<const float4*>(ws + L.sources_b) + (size_t)z * L.npad;
+    const WgParams* __restrict__ params = reinterpret_cast<const WgParams*>(ws);
+    const float inv_h = params->inv_h * (1.0f / WG_UNIT), mid_cb = params->cb_mid;
+    const int terms = params->terms;
+    if (terms == 0) return;                                    // the direct kernel's
+
+    const int slot0 = blockIdx.x * WG_OBS;
+    const int obs   = lane & 15;
+    const float4 me = src[slot0 + obs];
+    const bool ok   = slot0 + obs < n;
+    if (tid < WG_OBS) { s_tok[tid] = slot0 + tid < N ? __builtin_bit_cast(int, me.w) : -1; s_near[tid] = 0; }
+    if (slot0 >= n) {
+        __syncthreads();
+        for (int q = 0; q < WG_OBS; ++q) {
+            const int t = s_tok[q];
+            if (t < 0) continue;
+            const size_t row = (zN + t) * 2 * K;
+            for (int k = tid; k < 2 * K; k += THREADS) { out[row + k] = 0.f; if (GRADS) { d_cb[row + k] = 0.f; d_k[row + k] = 0.f; } }
+        }
+        return;
+    }
+
+    const float reach = (wg_reach<WAVES>(me, ok, reinterpret_cast<const WgBox*>(ws + L.boxes) + (size_t)z * L.nbox, L.nbox, s_red)
+                         + fabsf(mid_cb) * params->b_max * WG_UNIT) * inv_h + 2.0f;
+    const bool one    = !GRADS && terms == 1;
+    const bool direct = __builtin_amdgcn_readfirstlane(!(reach < (float)((one ? WgGrid<1>::CELLS : WgGrid<2>::CELLS) * WG_MAX_WINDOWS))) != 0;
+    const int  ncell  = __builtin_amdgcn_readfirstlane(direct ? 0 : (int)reach);
+    if (!direct) {
+        if (!GRADS && one) wa_grids<GRADS, 1>(s_grid, s_near, s_tok, ws, L, cb_magnitudes, wavenumbers, out, d_cb, d_k, src, srcb, me, ok, n, slot0, ncell, zN, K);
+        else               wa_grids<GRADS, 2>(s_grid, s_near, s_tok, ws, L, cb_magnitudes, wavenumbers, out, d_cb, d_k, src, srcb, me, ok, n, slot0, ncell, zN, K);
+    }
+
+    __syncthreads();
+    for (int q = wave; q < WG_OBS; q += WAVES) {
+        const int t = s_tok[q];
+        if (t < 0) continue;
+        const size_t row = (zN + t) * 2 * K;
+        if (slot0 + q >= n) {
+            if (direct) for (int k = lane; k < 2 * K; k += 64) { out[row + k] = 0.f; if (GRADS) { d_cb[row + k] = 0.f; d_k[row + k] = 0.f; } }
+            continue;
+        }
+        if (!direct && !s_near[q]) continue;
+        wa_direct<GRADS>(src, srcb, n, wg_lane(me.x, q), wg_lane(me.y, q), wg_lane(me.z, q), mid_cb, inv_h, 2.0f * inv_h, direct,
+                         cb_magnitudes, wavenumbers, out + row, GRADS ? d_cb + row : nullptr, GRADS ? d_k + row : nullptr, K, lane);
+    }
+}
+
+// What the grids need beside the direct kernel, two launches of preparation and one that finds nothing to do, costs 13 us.  Without
+// partial derivatives the scales are likely to be equal, where the grid wins from about 1 x 512 tokens on (K = 256: 1 x 512 41 / 49 us,
+// 1 x 2000 79 / 272, 8 x 1000 67 / 486); with them they are likely to differ, and the grids win where the direct kernel takes 400 us or more
+// (8 x 1000 484 / 701, 8 x 2000 1.6 / 2.7 ms, compact 1 x 8192 1.25 / 5.5 ms).  A batch with a padding mask is taken to hold 0.4 of its pairs.
+bool we_aniso_grid_wanted(int Z, int N, int K, bool partials, bool padded, int tuning)
+{
+    return tuning == 0 && K >= 64 && (padded ? 0.4 : 1.0) * Z * N * N * K >= (partials ? 1.0e9 : 2.0e8);
+}
+
+}  // namespace
+
+extern "C" size_t proteus_we_aniso_fwd_workspace_bytes(int Z, int N, int K, int partials, int padded, int tuning)
+{
+    if (Z <= 0 || N <= 0 || K <= 0 || N > PROTEUS_WE_MAX_N || K > PROTEUS_WE_MAX_K || Z > 65535) return 0;
+    return we_aniso_grid_wanted(Z, N, K, partials != 0, padded != 0, tuning) ? wg_layout(Z, N, K, true).bytes : 0;
+}
+
+extern "C" int proteus_we_aniso_fwd_ws(const float* coordsA, const float* coordsB, int coords_layout,
+                                       const float* cb_magnitudes, const float* wavenumbers, const uint8_t* mask,
+                                       float* out, float* d_cb, float* d_k, void* workspace, size_t workspace_bytes,
+                                       int Z, int N, int K, int tuning, void* stream)
+{
+    const int rc = proteus_we_aniso_fwd_check(coordsA, coordsB, coords_layout, cb_magnitudes, wavenumbers, mask, out, d_cb, d_k, Z, N, K, tuning);
+    if (rc != PROTEUS_OK) return rc;
+    const WgLayout L = wg_layout(Z, N, K, true);
+    if (!workspace || tuning != 0 || workspace_bytes < L.bytes)
+        return proteus_we_aniso_fwd(coordsA, coordsB, coords_layout, cb_magnitudes, wavenumbers, mask, out, d_cb, d_k, Z, N, K, tuning, stream);
+    if ((uintptr_t)workspace & 255) return PROTEUS_ERR_BAD_ALIGNMENT;
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    char* ws = (char*)workspace;
+    hipLaunchKernelGGL(we_aniso_grid_sources_kernel, dim3((unsigned)Z * (unsigned)L.blocks), dim3(256), 0, st, coordsA, coordsB, coords_layout, mask, ws, Z, N, K);
+    const unsigned units = (unsigned)((WG_GROUPS + (WG_MAX_TERMS + 3) / 4) * L.nkt);
+    hipLaunchKernelGGL(we_aniso_grid_tables_kernel, dim3((units + 3) / 4), dim3(256), 0, st, cb_magnitudes, wavenumbers, ws, Z, N, K, d_cb ? 1 : 0);
+    const dim3 grid((N + WG_OBS - 1) / WG_OBS, Z);
+    const size_t lds = (size_t)WG_ROWS * WG_OBS * 4;
+    if (d_cb) hipLaunchKernelGGL((we_aniso_grid_kernel<true>), grid, dim3(512), lds, st, (const char*)ws, cb_magnitudes, wavenumbers, out, d_cb, d_k, Z, N, K);
+    else      hipLaunchKernelGGL((we_aniso_grid_kernel<false>), grid, dim3(512), lds, st, (const char*)ws, cb_magnitudes, wavenumbers, out, d_cb, d_k, Z, N, K);
+    const int rl = (int)hipGetLastError();
+    if (rl) return rl;
+    return proteus_we_aniso_direct(coordsA, coordsB, coords_layout, cb_magnitudes, wavenumbers, mask, out, d_cb, d_k, Z, N, K, 0,
+                                   &reinterpret_cast<const WgParams*>(ws)->terms, stream);
+}

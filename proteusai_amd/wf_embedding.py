@@ -207,10 +207,14 @@ def we_aniso_forward(coordsA, coordsB, cb_magnitudes, wavenumbers, mask=None, tu
         return out, d_cb, d_k
     with _lib.on_device(dev):
         stream = _lib.raw_stream(dev)
-        rc = lib.proteus_we_aniso_fwd(a.data_ptr(), b.data_ptr(), _lib.COORDS_AOS, cb.data_ptr(), w.data_ptr(),
-                                      None if m is None else m.data_ptr(),
-                                      out.data_ptr(), d_cb.data_ptr() if partials else None, d_k.data_ptr() if partials else None,
-                                      Z, N, K, int(tuning), stream)
+        # with a workspace the library may go through grids of the distances (its size is 0 where that is of no use)
+        ws_bytes = lib.proteus_we_aniso_fwd_workspace_bytes(Z, N, K, int(partials), int(m is not None), int(tuning))
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
+        rc = lib.proteus_we_aniso_fwd_ws(a.data_ptr(), b.data_ptr(), _lib.COORDS_AOS, cb.data_ptr(), w.data_ptr(),
+                                         None if m is None else m.data_ptr(),
+                                         out.data_ptr(), d_cb.data_ptr() if partials else None, d_k.data_ptr() if partials else None,
+                                         None if ws is None else ws.data_ptr(), ws_bytes,
+                                         Z, N, K, int(tuning), stream)
     _lib.check(rc, "proteus_we_aniso_fwd")
     return out, d_cb, d_k
 

@@ -99,3 +99,68 @@ def test_values_that_are_not_finite_come_through(gpu):
     bad = wn.clone()
     bad[3] = float("nan")
     assert np.isnan(run_grid(gpu, coords[:1], bad)[0][:, :, 6:8]).all()
+
+
+def run_aniso(gpu, a, b, cb, wn, mask=None, partials=True):
+    lib = _lib.load()
+    Z, N, K = a.shape[0], a.shape[1], wn.numel()
+    a, b, cb, w = a.to(gpu), b.to(gpu), cb.to(gpu), wn.to(gpu)
+    m = None if mask is None else mask.to(gpu).view(torch.uint8)
+    bufs = [torch.full((Z, N, 2 * K), float("nan"), device=gpu) for _ in range(3)]
+    nbytes = lib.proteus_we_aniso_fwd_workspace_bytes(Z, max(N, 4096), max(K, 64), 1, 0, 0)
+    ws = torch.full((nbytes,), 0xA5, dtype=torch.uint8, device=gpu)
+    rc = lib.proteus_we_aniso_fwd_ws(a.data_ptr(), b.data_ptr(), _lib.COORDS_AOS, cb.data_ptr(), w.data_ptr(), None if m is None else m.data_ptr(),
+                                     bufs[0].data_ptr(), bufs[1].data_ptr() if partials else None, bufs[2].data_ptr() if partials else None,
+                                     ws.data_ptr(), nbytes, Z, N, K, 0, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, lib.proteus_strerror(rc)
+    torch.cuda.synchronize()
+    return [t.cpu().numpy() for t in bufs[:3 if partials else 1]]
+
+
+ANISO = {                       # N, Z, K, scale of the chain, spread of the C-beta scales around 1, mask
+    "equal scales": (700, 1, 64, 1.0, 0.0, None),
+    "equal scales, flushes, scattered mask": (2100, 2, 20, 1.0, 0.0, "scattered"),
+    "equal scales, several windows": (300, 2, 20, 60.0, 0.0, None),
+    "four terms, an empty item, a lone survivor": (1100, 4, 256, 1.0, 0.01, "tail"),
+    "ten terms and flushes": (2100, 2, 256, 1.0, 0.2, None),
+    "two grids in several windows": (2100, 2, 256, 3.0, 0.02, "scattered"),
+    "many pairs too close for a cell": (1300, 3, 256, 0.3, 0.02, None),
+    "more terms than pay": (200, 2, 64, 1.0, 1.5, None),
+}
+
+
+@pytest.mark.parametrize("name", ANISO)
+def test_anisotropic_grids_match_the_oracle(gpu, name):
+    N, Z, K, scale, spread, kind = ANISO[name]
+    a, _ = synth.we_inputs(N, seed=N + K, batch=Z)
+    a = a * scale
+    a[0, 40] = a[0, 12]
+    g = torch.Generator().manual_seed(K + N)
+    b = torch.randn(Z, N, 3, generator=g)
+    b = 1.5 * b / b.norm(dim=-1, keepdim=True)
+    b[:, 0] = 0.0
+    cb = 1.0 + spread * torch.randn(K, generator=g)
+    wn = synth.wavenumbers(2 * K) * torch.where(torch.rand(K, generator=g) < 0.3, -1.0, 1.0)
+    mask = None
+    if kind == "scattered":
+        mask = torch.rand(Z, N, generator=g) < 0.35
+    elif kind == "tail":
+        mask = torch.arange(N)[None, :] >= torch.tensor([N, 500, 0, 1])[:, None]
+    rows = None if N <= 512 else np.unique(np.concatenate([np.arange(0, N, 41), [15, 16, 1023, 1024, N - 1]]))
+    rows = None if rows is None else rows[rows < N].astype(np.int32)
+    got = run_aniso(gpu, a, b, cb, wn, mask)
+    ref = c_oracle.we_aniso(a.numpy(), b.numpy(), cb.numpy(), wn.numpy(), None if mask is None else mask.numpy(), rows=rows)
+    sel = slice(None) if rows is None else rows
+    # the bar of the isotropic grids, plus 3e-7 for the terms left out of the expansion
+    c = a if mask is None else a.masked_fill(mask[..., None], 0.0)
+    far = float((c.amax(1) - c.amin(1)).norm(dim=-1).max())
+    bar = 2e-6 + 2 * 2.0 ** -24 * float(wn.abs().max()) * far
+    for x, r, what in zip(got, ref, ("out", "d_cb", "d_k")):
+        assert np.isfinite(x).all(), f"{name}: {what}"
+        if mask is not None:
+            assert (x[mask.numpy()] == 0).all(), f"{name}: {what} of padded rows"
+        assert rel_l2(x[:, sel], r) <= bar, f"{name}: {what} {rel_l2(x[:, sel], r):.3e} (bar {bar:.1e})"
+    again = run_aniso(gpu, a, b, cb, wn, mask)
+    assert all(np.array_equal(x, y) for x, y in zip(got, again))
+    lean = run_aniso(gpu, a, b, cb, wn, mask, partials=False)[0]
+    assert np.isfinite(lean).all() and rel_l2(lean[:, sel], ref[0]) <= bar
