@@ -258,7 +258,7 @@ __device__ __forceinline__ void wa_grids(uint32_t* s_grid, int* s_near, const in
                 float r2;
                 const Place w = wa_place(me.x - q.x, me.y - q.y, me.z - q.z, qb, midv, inv_hv, magic, emask, r2);
                 float wt[6];
-                kernel(w.x, w.c, wt);
+                kernel.template weights<GP == 1>(w.x, w.c, wt);
                 const uint32_t ub = __builtin_bit_cast(uint32_t, w.nf + magic);
                 uint32_t at = (ub << 6) + base + (w.eb >> 14);
                 at = ub - first < (uint32_t)cells && !(w.c > climit) ? at : trash;

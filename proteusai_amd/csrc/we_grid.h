@@ -160,15 +160,17 @@ __device__ __forceinline__ float wg_block_sum(float v)
     return s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
 }
 
-// Cells per unit of length, rounded to float once: h is its exact inverse from here on (a wavenumber beyond any use gives an
-// infinite value, which sends every workgroup to the direct sums).
+// Cells per unit of length, rounded to float once: h is its exact inverse from here on.  Wavenumbers beyond any use (wavelengths
+// below 0.11, where the coefficients of the spreading kernel would lose bits as denormals) give an infinite value, which sends
+// every workgroup to the direct sums.
 __device__ __forceinline__ float wg_cells_per_length(const float* __restrict__ wavenumbers, const int K)
 {
     float km = 0.f;
     bool bad = false;
     for (int k = threadIdx.x; k < K; k += 256) { const float w = fabsf(wavenumbers[k]); bad |= !(w < 3.0e38f); km = fmaxf(km, w); }
     km = wg_block_max(bad ? __builtin_inff() : km);
-    return fmaxf(km * (WG_OVERSAMPLING / 3.14159265f) * 1.000001f, 1.0e-6f);
+    const float inv_h = fmaxf(km * (WG_OVERSAMPLING / 3.14159265f) * 1.000001f, 1.0e-6f);
+    return inv_h < 64.0f ? inv_h : __builtin_inff();
 }
 
 // Wave `unit` fills 8 rows of the tables for 16 wavenumbers: cosine and sine of k h (row + 1/2), two rows of four per lane.
@@ -241,13 +243,22 @@ struct WgKernel {
 #pragma unroll
             for (int j = 0; j < 3; ++j) { e[i][j] = wg_vgpr(f * E[i][j]); o[i][j] = wg_vgpr(f * O[i][j]); }
     }
-    // weights of the six nodes, first to last, times c
-    __device__ __forceinline__ void operator()(const float x, const float c, float (&w)[6]) const
+    // Weights of the six nodes, first to last, times c.  Where they are denormals none may come out as -0, whose bit pattern is
+    // 2^31: the outermost weight falls to 2.54e-6 of a full one at the edge of the cell, 2.66 units at the smallest `scale`
+    // (1.048e6), and E c is rounded to a whole unit.  With c > 1/2 (the isotropic 2^e h / r) at least 0.8 units are left.
+    // SMALL_C: c may be anything above zero, and the outermost pair takes c last: E - x O is a normal number above zero.
+    template <bool SMALL_C = false>
+    __device__ __forceinline__ void weights(const float x, const float c, float (&w)[6]) const
     {
         const float x2 = x * x, xc = x * c;
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
             const float E = __builtin_fmaf(__builtin_fmaf(e[i][2], x2, e[i][1]), x2, e[i][0]), O = __builtin_fmaf(__builtin_fmaf(o[i][2], x2, o[i][1]), x2, o[i][0]);
+            if (SMALL_C && i == 2) {
+                w[0] = __builtin_fmaf(-O, x, E) * c;
+                w[5] = __builtin_fmaf(O, x, E) * c;
+                continue;
+            }
             const float t = E * c;
             w[2 - i] = __builtin_fmaf(-O, xc, t);
             w[3 + i] = __builtin_fmaf(O, xc, t);

@@ -201,7 +201,7 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
                 const uint32_t eb = __builtin_bit_cast(uint32_t, nf) & emask;
                 const float c  = inv * __builtin_bit_cast(float, eb);                      // 2^e / r
                 float w[6];
-                kernel(x, c, w);
+                kernel.weights(x, c, w);
                 uint32_t at = (ub << 6) + base + (eb >> 14);
                 if (decltype(multi)::value) at = ub - first < (uint32_t)cells ? at : trash;
                 else                        at = min(at, trash);

@@ -164,3 +164,20 @@ def test_anisotropic_grids_match_the_oracle(gpu, name):
     assert all(np.array_equal(x, y) for x, y in zip(got, again))
     lean = run_aniso(gpu, a, b, cb, wn, mask, partials=False)[0]
     assert np.isfinite(lean).all() and rel_l2(lean[:, sel], ref[0]) <= bar
+
+
+def test_weights_that_fall_below_half_a_unit(gpu):
+    # equal C-beta scales: r - cb A may be a small part of r, and with it every fixed-point weight of the pair.  In a ball of three
+    # angstrom some hundred thousand pairs lie near the outer edge of the first cell with r four to five times that.
+    N, K = 2100, 64
+    g = torch.Generator().manual_seed(11)
+    a = torch.randn(1, N, 3, generator=g)
+    a = 3.0 * a / a.norm(dim=-1, keepdim=True) * torch.rand(1, N, 1, generator=g) ** (1 / 3)
+    b = torch.randn(1, N, 3, generator=g)
+    b = 1.8154 * b / b.norm(dim=-1, keepdim=True)
+    cb, wn = torch.ones(K), synth.wavenumbers(2 * K)
+    got = run_aniso(gpu, a, b, cb, wn, partials=False)[0]
+    ref = c_oracle.we_aniso(a.numpy(), b.numpy(), cb.numpy(), wn.numpy(), None, rows=np.arange(N, dtype=np.int32))[0]
+    # the bar of the anisotropic grids, row by row: one pair's cell that is off by 2^31 units changes a row by 100 times its norm
+    err = np.linalg.norm(got - ref, axis=-1) / np.linalg.norm(ref, axis=-1)
+    assert err.max() <= 4 * (2e-6 + 2 * 2.0 ** -24 * float(wn.max()) * 6.0), err.max()
