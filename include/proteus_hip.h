@@ -66,7 +66,7 @@ extern "C" {
  * backward entry point take `int operand_type` before `tuning` / `stream`; a caller built against an older header
  * would pass its tuning selector there).  The Python binding checks for an exact match when it loads the library.
  */
-#define PROTEUS_VERSION 302
+#define PROTEUS_VERSION 303
 int proteus_version(void);
 
 /* Human-readable text for a return code of any entry point. */
@@ -462,6 +462,42 @@ int proteus_geo_attn_delta(const float* O, const void* dO, const int64_t* stride
                            int Z, int H, int N, int d_head, int dO_dtype, void* stream);
 int proteus_geo_attn_delta_check(const float* O, const void* dO, const int64_t* strides, const float* D,
                                  int Z, int H, int N, int d_head, int dO_dtype);
+
+/*
+ * proteus_geo_attn_delta, and with it what else the backward wants before it runs, in the same launch:
+ *   dO_cast   NULL, or where dO goes in the operand type (operand_type = PROTEUS_OPERAND_BF16 / _F16, round to nearest
+ *             even); 16-byte aligned
+ *   d_sigma, d_beta   NULL, or f32 [H] arrays to clear
+ *   strides   NULL: everything contiguous; else 9 element strides, of O, dO and dO_cast (the last three multiples of 8; not
+ *             looked at without dO_cast)
+ */
+int proteus_geo_attn_prepare_bwd(const float* O, const void* dO, const int64_t* strides, float* D, uint16_t* dO_cast,
+                                 float* d_sigma, float* d_beta,
+                                 int Z, int H, int N, int d_head, int dO_dtype, int operand_type, void* stream);
+int proteus_geo_attn_prepare_bwd_check(const float* O, const void* dO, const int64_t* strides, const float* D, const uint16_t* dO_cast,
+                                       const float* d_sigma, const float* d_beta,
+                                       int Z, int H, int N, int d_head, int dO_dtype, int operand_type);
+
+/*
+ * proteus_geo_attn_bwd (strides = NULL) or _bwd_strided with a choice of the gradients' type: grad_type = PROTEUS_GRAD_F32, or
+ * PROTEUS_GRAD_OPERAND for dQ, dK, dV in the operands' 16-bit type (the fp32 sums rounded to nearest even; their strides
+ * are then multiples of 8 elements).
+ */
+#define PROTEUS_GRAD_F32     0
+#define PROTEUS_GRAD_OPERAND 1
+int proteus_geo_attn_bwd_typed(const uint16_t* Q, const uint16_t* K, const uint16_t* V, const uint16_t* dO,
+                               const int64_t* strides,
+                               const float* coords, const float* sigma, const float* beta,
+                               const uint8_t* key_pad_mask, const float* L, const float* D,
+                               void* dQ, void* dK, void* dV, float* d_sigma, float* d_beta,
+                               int Z, int H, int N, int d_head, float min_rbf, float max_rbf, int operand_type, int grad_type, void* stream);
+int proteus_geo_attn_bwd_typed_check(const uint16_t* Q, const uint16_t* K, const uint16_t* V, const uint16_t* dO,
+                                     const int64_t* strides,
+                                     const float* coords, const float* sigma, const float* beta,
+                                     const uint8_t* key_pad_mask, const float* L, const float* D,
+                                     const void* dQ, const void* dK, const void* dV,
+                                     const float* d_sigma, const float* d_beta,
+                                     int Z, int H, int N, int d_head, float min_rbf, float max_rbf, int operand_type, int grad_type);
 
 int         proteus_geo_attn_num_variants(void);
 const char* proteus_geo_attn_variant_name(int tuning);

@@ -12,8 +12,9 @@ LIB_PATH = os.path.join(HERE, "libproteus_hip.so")
 
 COORDS_SOA = 0
 COORDS_AOS = 1
-ABI_VERSION = 302                    # PROTEUS_VERSION of the include/proteus_hip.h these argument lists were written from
+ABI_VERSION = 303                    # PROTEUS_VERSION of the include/proteus_hip.h these argument lists were written from
 OPERAND_BF16, OPERAND_F16 = 0, 1     # PROTEUS_OPERAND_* of include/proteus_hip.h
+GRAD_F32, GRAD_OPERAND = 0, 1        # PROTEUS_GRAD_*
 DTYPE_F32, DTYPE_BF16, DTYPE_F16 = 0, 1, 2   # PROTEUS_DTYPE_*
 
 # every symbol include/proteus_hip.h declares
@@ -23,7 +24,8 @@ SYMBOLS = [
     "proteus_we_dropout_threshold", "proteus_we_num_variants", "proteus_we_variant_name",
     "proteus_we_aniso_fwd", "proteus_we_aniso_fwd_check", "proteus_we_aniso_fwd_workspace_bytes", "proteus_we_aniso_fwd_ws", "proteus_we_aniso_num_variants", "proteus_we_aniso_variant_name",
     "proteus_we_bwd_workspace_bytes", "proteus_we_bwd", "proteus_we_bwd_check", "proteus_we_bwd_static", "proteus_we_aniso_bwd", "proteus_we_aniso_bwd_check",
-    "proteus_geo_attn_fwd", "proteus_geo_attn_fwd_check", "proteus_geo_attn_legacy_fwd", "proteus_geo_attn_bwd",
+    "proteus_geo_attn_fwd", "proteus_geo_attn_fwd_check", "proteus_geo_attn_legacy_fwd", "proteus_geo_attn_bwd", "proteus_geo_attn_bwd_typed", "proteus_geo_attn_bwd_typed_check",
+    "proteus_geo_attn_prepare_bwd", "proteus_geo_attn_prepare_bwd_check",
     "proteus_geo_attn_fwd_workspace_bytes", "proteus_geo_attn_fwd_ws", "proteus_geo_attn_fwd_ws_check",
     "proteus_geo_attn_bwd_check", "proteus_geo_attn_fwd_strided", "proteus_geo_attn_fwd_strided_check",
     "proteus_geo_attn_legacy_fwd_strided",
@@ -138,6 +140,14 @@ def load():
     lib.proteus_add_layernorm_fwd_check.argtypes = [vp, vp, vp, vp, vp, ctypes.c_long, ci, cf, ci]
     lib.proteus_geo_attn_delta.restype = ci
     lib.proteus_geo_attn_delta.argtypes = [vp, vp, i64p, vp, ci, ci, ci, ci, ci, vp]
+    lib.proteus_geo_attn_prepare_bwd.restype = ci
+    lib.proteus_geo_attn_prepare_bwd.argtypes = [vp, vp, i64p, vp, vp, vp, vp, ci, ci, ci, ci, ci, ci, vp]
+    lib.proteus_geo_attn_prepare_bwd_check.restype = ci
+    lib.proteus_geo_attn_prepare_bwd_check.argtypes = [vp, vp, i64p, vp, vp, vp, vp, ci, ci, ci, ci, ci, ci]
+    lib.proteus_geo_attn_bwd_typed.restype = ci
+    lib.proteus_geo_attn_bwd_typed.argtypes = [vp] * 4 + [i64p] + [vp] * 11 + [ci, ci, ci, ci, cf, cf, ci, ci, vp]
+    lib.proteus_geo_attn_bwd_typed_check.restype = ci
+    lib.proteus_geo_attn_bwd_typed_check.argtypes = [vp] * 4 + [i64p] + [vp] * 11 + [ci, ci, ci, ci, cf, cf, ci, ci]
     lib.proteus_geo_attn_delta_check.restype = ci
     lib.proteus_geo_attn_delta_check.argtypes = [vp, vp, i64p, vp, ci, ci, ci, ci, ci]
     _lib = lib

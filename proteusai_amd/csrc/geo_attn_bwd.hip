@@ -56,17 +56,19 @@ GbStrides contiguous_strides(int H, int N, int d) {
     const long t[3] = {(long)H * N * d, (long)N * d, (long)d};
     long* all[7] = {gs.q, gs.k, gs.v, gs.g, gs.dq, gs.dk, gs.dv};
     for (int a = 0; a < 7; ++a) for (int i = 0; i < 3; ++i) all[a][i] = t[i];
+    gs.grads16 = 0;
     return gs;
 }
 
 // strides[21]: (batch, head, token) element strides of Q, K, V, dO, dQ, dK, dV in this order
-int strides_from(const int64_t* strides, int Z, int H, int N, int d, GbStrides& gs) {
+int strides_from(const int64_t* strides, int Z, int H, int N, int d, GbStrides& gs, bool grads16 = false) {
     if (!strides) return PROTEUS_ERR_NULL_POINTER;
+    gs.grads16 = grads16;
     long* dst[7] = {gs.q, gs.k, gs.v, gs.g, gs.dq, gs.dk, gs.dv};
     for (int t = 0; t < 7; ++t) {
         const int64_t sz = strides[3 * t], sh = strides[3 * t + 1], sn = strides[3 * t + 2];
         if (sz < 0 || sh < 0 || sn < d) return PROTEUS_ERR_BAD_LAYOUT;
-        const int align = (t >= 4) ? 4 : 8;            // 16-byte rows: f32 outputs, bf16 inputs
+        const int align = (t >= 4 && !grads16) ? 4 : 8;            // 16-byte rows: f32 gradients, 16-bit everything else
         if ((sz % align) || (sh % align) || (sn % align)) return PROTEUS_ERR_BAD_ALIGNMENT;
         if ((Z > 1 && sz == 0) || (H > 1 && sh == 0)) return PROTEUS_ERR_BAD_LAYOUT;
         if ((long)N * sn >= (1L << 30)) return PROTEUS_ERR_BAD_SHAPE;
@@ -141,4 +143,37 @@ extern "C" int proteus_geo_attn_bwd_strided(const uint16_t* Q, const uint16_t* K
     if (rc != PROTEUS_OK) return rc;
     return launch_bwd_any(beta != nullptr, operand_type == PROTEUS_OPERAND_F16, d_head, Q, K, V, dO, coords, sigma, beta, key_pad_mask,
                           L, D, dQ, dK, dV, d_sigma, d_beta, Z, H, N, min_rbf, max_rbf, gs, reinterpret_cast<hipStream_t>(stream));
+}
+
+extern "C" int proteus_geo_attn_bwd_typed_check(const uint16_t* Q, const uint16_t* K, const uint16_t* V, const uint16_t* dO,
+                                                const int64_t* strides,
+                                                const float* coords, const float* sigma, const float* beta,
+                                                const uint8_t* key_pad_mask, const float* L, const float* D,
+                                                const void* dQ, const void* dK, const void* dV,
+                                                const float* d_sigma, const float* d_beta,
+                                                int Z, int H, int N, int d_head, float min_rbf, float max_rbf, int operand_type, int grad_type)
+{
+    if (grad_type != PROTEUS_GRAD_F32 && grad_type != PROTEUS_GRAD_OPERAND) return PROTEUS_ERR_BAD_OPERAND_TYPE;
+    const int rc = proteus_geo_attn_bwd_check(Q, K, V, dO, coords, sigma, beta, key_pad_mask, L, D, (const float*)dQ, (const float*)dK, (const float*)dV,
+                                              d_sigma, d_beta, Z, H, N, d_head, min_rbf, max_rbf, operand_type);
+    if (rc != PROTEUS_OK || !strides) return rc;
+    GbStrides gs;
+    return strides_from(strides, Z, H, N, d_head, gs, grad_type == PROTEUS_GRAD_OPERAND);
+}
+
+extern "C" int proteus_geo_attn_bwd_typed(const uint16_t* Q, const uint16_t* K, const uint16_t* V, const uint16_t* dO,
+                                          const int64_t* strides,
+                                          const float* coords, const float* sigma, const float* beta,
+                                          const uint8_t* key_pad_mask, const float* L, const float* D,
+                                          void* dQ, void* dK, void* dV, float* d_sigma, float* d_beta,
+                                          int Z, int H, int N, int d_head, float min_rbf, float max_rbf, int operand_type, int grad_type, void* stream)
+{
+    const int rc = proteus_geo_attn_bwd_typed_check(Q, K, V, dO, strides, coords, sigma, beta, key_pad_mask, L, D, dQ, dK, dV,
+                                                    d_sigma, d_beta, Z, H, N, d_head, min_rbf, max_rbf, operand_type, grad_type);
+    if (rc != PROTEUS_OK) return rc;
+    GbStrides gs = contiguous_strides(H, N, d_head);
+    if (strides) strides_from(strides, Z, H, N, d_head, gs);
+    gs.grads16 = grad_type == PROTEUS_GRAD_OPERAND;
+    return launch_bwd_any(beta != nullptr, operand_type == PROTEUS_OPERAND_F16, d_head, Q, K, V, dO, coords, sigma, beta, key_pad_mask,
+                          L, D, (float*)dQ, (float*)dK, (float*)dV, d_sigma, d_beta, Z, H, N, min_rbf, max_rbf, gs, reinterpret_cast<hipStream_t>(stream));
 }

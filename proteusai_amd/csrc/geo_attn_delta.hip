@@ -5,16 +5,22 @@
 // bf16 or fp16, as autograd hands it over), products and sum in fp32, D [Z,H,N] fp32.  HBM-bound streaming work:
 // (4 + sizeof(dO element)) bytes per element read, 4 bytes per row written.  d / 4 lanes share a row, every lane
 // loads 4 consecutive elements of both tensors (16 / 8 bytes), the lanes of a row meet by shuffles.
+//
+// The backward also needs dO in the operands' 16-bit type and its per-head sums cleared.  Both are done here on request
+// (proteus_geo_attn_prepare_bwd): dO is in registers anyway, so its cast costs the 2 bytes that are written instead of a
+// launch that reads 4 and writes 2.
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include "proteus_hip.h"
+#include "geo_attn_ops.h"
 
 namespace {
 
 constexpr int GD_THREADS = 256;
 
-struct GdStrides { long o[3], g[3]; };      // (batch, head, token) element strides of O and dO
+struct GdStrides { long o[3], g[3], c[3]; };      // (batch, head, token) element strides of O, dO and the cast of dO
+struct GdExtra { uint16_t* cast; float* zero_a; float* zero_b; };      // any of them may be NULL
 
 template <int DTYPE> struct Grad;
 template <> struct Grad<PROTEUS_DTYPE_F32> {
@@ -42,12 +48,17 @@ template <> struct Grad<PROTEUS_DTYPE_F16> {
     }
 };
 
-// LPR = d / 4 lanes per row (8, 16, 32)
-template <int DTYPE, int LPR>
+// LPR = d / 4 lanes per row (8, 16, 32); F16: the cast is to fp16, otherwise to bf16
+template <int DTYPE, int LPR, bool F16>
 __global__ __launch_bounds__(GD_THREADS)
 void geo_attn_delta_kernel(const float* __restrict__ O, const typename Grad<DTYPE>::T* __restrict__ dO, float* __restrict__ D,
-                           const long rows, const int H, const int N, const GdStrides st)
+                           const long rows, const int H, const int N, const GdStrides st, const GdExtra ex)
 {
+    if (blockIdx.x == 0)
+        for (int i = threadIdx.x; i < H; i += GD_THREADS) {
+            if (ex.zero_a) ex.zero_a[i] = 0.f;
+            if (ex.zero_b) ex.zero_b[i] = 0.f;
+        }
     constexpr int RPW = GD_THREADS / LPR;                    // rows per workgroup
     const int  sub = threadIdx.x % LPR;
     const long row = (long)blockIdx.x * RPW + threadIdx.x / LPR;
@@ -62,6 +73,8 @@ void geo_attn_delta_kernel(const float* __restrict__ O, const typename Grad<DTYP
         a[0] = t.x; a[1] = t.y; a[2] = t.z; a[3] = t.w;
 #pragma unroll
         for (int e = 0; e < 4; ++e) s = __builtin_fmaf(a[e], b[e], s);
+        typedef proteus_ops::Operand<F16> Op;
+        if (ex.cast) *reinterpret_cast<uint2*>(ex.cast + z * st.c[0] + h * st.c[1] + n * st.c[2] + 4 * sub) = make_uint2(Op::pack(b[0], b[1]), Op::pack(b[2], b[3]));
     }
     // (rows of a wave all take part: a row past the end adds zeros among its own lanes)
 #pragma unroll
@@ -69,16 +82,16 @@ void geo_attn_delta_kernel(const float* __restrict__ O, const typename Grad<DTYP
     if (row < rows && sub == 0) D[row] = s;
 }
 
-template <int DTYPE>
-int launch(const float* O, const void* dO, float* D, int Z, int H, int N, int d, const GdStrides& st, hipStream_t stream)
+template <int DTYPE, bool F16>
+int launch(const float* O, const void* dO, float* D, int Z, int H, int N, int d, const GdStrides& st, const GdExtra& ex, hipStream_t stream)
 {
     typedef typename Grad<DTYPE>::T T;
     const long rows = (long)Z * H * N;
     const int  lpr = d / 4;
     const dim3 grid((unsigned)((rows + GD_THREADS / lpr - 1) / (GD_THREADS / lpr)));
-    if (lpr == 8)       hipLaunchKernelGGL((geo_attn_delta_kernel<DTYPE, 8>), grid, dim3(GD_THREADS), 0, stream, O, (const T*)dO, D, rows, H, N, st);
-    else if (lpr == 16) hipLaunchKernelGGL((geo_attn_delta_kernel<DTYPE, 16>), grid, dim3(GD_THREADS), 0, stream, O, (const T*)dO, D, rows, H, N, st);
-    else                hipLaunchKernelGGL((geo_attn_delta_kernel<DTYPE, 32>), grid, dim3(GD_THREADS), 0, stream, O, (const T*)dO, D, rows, H, N, st);
+    if (lpr == 8)       hipLaunchKernelGGL((geo_attn_delta_kernel<DTYPE, 8, F16>), grid, dim3(GD_THREADS), 0, stream, O, (const T*)dO, D, rows, H, N, st, ex);
+    else if (lpr == 16) hipLaunchKernelGGL((geo_attn_delta_kernel<DTYPE, 16, F16>), grid, dim3(GD_THREADS), 0, stream, O, (const T*)dO, D, rows, H, N, st, ex);
+    else                hipLaunchKernelGGL((geo_attn_delta_kernel<DTYPE, 32, F16>), grid, dim3(GD_THREADS), 0, stream, O, (const T*)dO, D, rows, H, N, st, ex);
     return (int)hipGetLastError();
 }
 
@@ -105,6 +118,34 @@ int check(const float* O, const void* dO, const int64_t* strides, const float* D
     return PROTEUS_OK;
 }
 
+// strides[9]: of O, dO and the cast of dO, whose rows start on multiples of 16 bytes as the backward wants its operands
+int check_prepare(const float* O, const void* dO, const int64_t* strides, const float* D, const uint16_t* cast,
+                  int Z, int H, int N, int d_head, int dtype, int operand_type, GdStrides& st)
+{
+    const int rc = check(O, dO, strides, D, Z, H, N, d_head, dtype, st);
+    if (rc != PROTEUS_OK) return rc;
+    if (operand_type != PROTEUS_OPERAND_BF16 && operand_type != PROTEUS_OPERAND_F16) return PROTEUS_ERR_BAD_OPERAND_TYPE;
+    if ((uintptr_t)cast & 15) return PROTEUS_ERR_BAD_ALIGNMENT;
+    for (int i = 0; i < 3; ++i) st.c[i] = strides && cast ? (long)strides[6 + i] : st.o[i];
+    if (strides && cast) {
+        for (int i = 0; i < 3; ++i) {
+            if (st.c[i] < 0) return PROTEUS_ERR_BAD_LAYOUT;
+            if (st.c[i] & 7) return PROTEUS_ERR_BAD_ALIGNMENT;
+        }
+        if (st.c[2] < d_head || (Z > 1 && st.c[0] == 0) || (H > 1 && st.c[1] == 0)) return PROTEUS_ERR_BAD_LAYOUT;
+    }
+    return PROTEUS_OK;
+}
+
+int launch_any(bool f16, const float* O, const void* dO, float* D, int Z, int H, int N, int d, int dtype, const GdStrides& st, const GdExtra& ex, hipStream_t s)
+{
+#define GD_GO(T_) (f16 ? launch<T_, true>(O, dO, D, Z, H, N, d, st, ex, s) : launch<T_, false>(O, dO, D, Z, H, N, d, st, ex, s))
+    if (dtype == PROTEUS_DTYPE_F32)  return GD_GO(PROTEUS_DTYPE_F32);
+    if (dtype == PROTEUS_DTYPE_BF16) return GD_GO(PROTEUS_DTYPE_BF16);
+    return GD_GO(PROTEUS_DTYPE_F16);
+#undef GD_GO
+}
+
 }  // namespace
 
 extern "C" int proteus_geo_attn_delta_check(const float* O, const void* dO, const int64_t* strides, const float* D,
@@ -121,7 +162,23 @@ extern "C" int proteus_geo_attn_delta(const float* O, const void* dO, const int6
     const int rc = check(O, dO, strides, D, Z, H, N, d_head, dO_dtype, st);
     if (rc != PROTEUS_OK) return rc;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    if (dO_dtype == PROTEUS_DTYPE_F32)  return launch<PROTEUS_DTYPE_F32>(O, dO, D, Z, H, N, d_head, st, s);
-    if (dO_dtype == PROTEUS_DTYPE_BF16) return launch<PROTEUS_DTYPE_BF16>(O, dO, D, Z, H, N, d_head, st, s);
-    return launch<PROTEUS_DTYPE_F16>(O, dO, D, Z, H, N, d_head, st, s);
+    return launch_any(false, O, dO, D, Z, H, N, d_head, dO_dtype, st, GdExtra{nullptr, nullptr, nullptr}, s);
+}
+
+extern "C" int proteus_geo_attn_prepare_bwd_check(const float* O, const void* dO, const int64_t* strides, const float* D, const uint16_t* dO_cast,
+                                                  const float* d_sigma, const float* d_beta, int Z, int H, int N, int d_head, int dO_dtype, int operand_type)
+{
+    (void)d_sigma; (void)d_beta;
+    GdStrides st;
+    return check_prepare(O, dO, strides, D, dO_cast, Z, H, N, d_head, dO_dtype, operand_type, st);
+}
+
+extern "C" int proteus_geo_attn_prepare_bwd(const float* O, const void* dO, const int64_t* strides, float* D, uint16_t* dO_cast,
+                                            float* d_sigma, float* d_beta, int Z, int H, int N, int d_head, int dO_dtype, int operand_type, void* stream)
+{
+    GdStrides st;
+    const int rc = check_prepare(O, dO, strides, D, dO_cast, Z, H, N, d_head, dO_dtype, operand_type, st);
+    if (rc != PROTEUS_OK) return rc;
+    return launch_any(operand_type == PROTEUS_OPERAND_F16, O, dO, D, Z, H, N, d_head, dO_dtype, st, GdExtra{dO_cast, d_sigma, d_beta},
+                      reinterpret_cast<hipStream_t>(stream));
 }

@@ -8,8 +8,9 @@ namespace proteus_internal {
 
 // Element strides (batch, head, token) of Q, K, V (16-bit) and O (f32); the head dimension is contiguous.
 struct GaStrides { long q[3], k[3], v[3], o[3]; };
-// ... of Q, K, V, dO (16-bit) and dQ, dK, dV (f32)
-struct GbStrides { long q[3], k[3], v[3], g[3], dq[3], dk[3], dv[3]; };
+// ... of Q, K, V, dO (16-bit) and dQ, dK, dV (f32, or of the operand type where grads16 is set: then the gradients' pointers,
+// float* in the argument lists, point to 16-bit elements)
+struct GbStrides { long q[3], k[3], v[3], g[3], dq[3], dk[3], dv[3]; int grads16; };
 
 #define PROTEUS_HIDDEN __attribute__((visibility("hidden")))
 

@@ -165,16 +165,57 @@ def geo_attn(Q, K, V, coords, sigma, key_padding_mask=None, return_lse: bool = F
 _DELTA_DTYPES = {torch.float32: _lib.DTYPE_F32, torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_F16}
 
 
+def _delta_in_place(O, dO):
+    """Can the kernel read these two [Z,H,N,d] tensors where they lie?"""
+    if not (O.is_cuda and O.dtype == torch.float32 and dO.dtype in _DELTA_DTYPES and dO.shape == O.shape
+            and O.data_ptr() % 16 == 0 and dO.data_ptr() % (4 * dO.element_size()) == 0):
+        return False
+    Z, H, N, d = O.shape
+    if not (d in (32, 64, 128) and Z * H * N > 0 and Z * H <= 65535):
+        return False
+    if O.is_contiguous() and dO.is_contiguous():
+        return True
+    return (O.stride(3) == 1 and dO.stride(3) == 1 and O.stride(2) >= d and dO.stride(2) >= d
+            and all(s % 4 == 0 for s in O.stride()[:3] + dO.stride()[:3]))
+
+
+def _prepare_backward(O, dO, op_dtype, op_type, betas):
+    """D = rowsum(O * dO), dO in the operand type and cleared d_sigma [H] (and d_betas [H] where there are betas): one
+    launch where the layouts allow, the separate operations otherwise."""
+    Z, H, N, d = O.shape
+    dev = O.device
+    cast = None
+    if _delta_in_place(O, dO):
+        if dO.dtype != op_dtype:
+            cast = torch.empty_like(dO, dtype=op_dtype)             # (the memory order of dO where that is dense)
+            ok = _rows_ok(cast, 2)
+        else:
+            ok = _rows_ok(dO, 2)
+        if ok:
+            D = torch.empty(Z, H, N, dtype=torch.float32, device=dev)
+            d_sigma = torch.empty(H, dtype=torch.float32, device=dev)
+            d_beta = None if betas is None else torch.empty(H, dtype=torch.float32, device=dev)
+            if _is_plain(O, dO) and (cast is None or cast.is_contiguous()):
+                strides = None
+            else:
+                strides = _lib.stride_array(O, dO, dO if cast is None else cast)
+            with _lib.on_device(dev):
+                rc = _lib.load().proteus_geo_attn_prepare_bwd(O.data_ptr(), dO.data_ptr(), strides, D.data_ptr(),
+                                                              None if cast is None else cast.data_ptr(), d_sigma.data_ptr(),
+                                                              None if d_beta is None else d_beta.data_ptr(),
+                                                              Z, H, N, d, _DELTA_DTYPES[dO.dtype], op_type, _lib.raw_stream(dev))
+            _lib.check(rc, "proteus_geo_attn_prepare_bwd")
+            return D, dO if cast is None else cast, d_sigma, d_beta
+    D = _delta(O, dO)
+    return (D, _operand(dO, op_dtype), torch.zeros(H, dtype=torch.float32, device=dev),
+            None if betas is None else torch.zeros(H, dtype=torch.float32, device=dev))
+
+
 def _delta(O, dO):
     """D = rowsum(O * dO) [Z,H,N] fp32 (old/old_scripts/attn/geometric_attn.py:618), in one pass over both tensors
     where their layout allows (rows of d contiguous, strides multiples of 4 elements); the torch expression otherwise."""
     Z, H, N, d = O.shape
-    plain = (O.is_cuda and O.dtype == torch.float32 and dO.dtype in _DELTA_DTYPES and dO.shape == O.shape and d in (32, 64, 128)
-             and Z * H * N > 0 and Z * H <= 65535
-             and O.stride(3) == 1 and dO.stride(3) == 1 and O.stride(2) >= d and dO.stride(2) >= d
-             and all(s % 4 == 0 for s in O.stride()[:3] + dO.stride()[:3])
-             and O.data_ptr() % 16 == 0 and dO.data_ptr() % (4 * dO.element_size()) == 0)
-    if not plain:
+    if not _delta_in_place(O, dO):
         return torch.sum(O.float() * dO, dim=3).contiguous()       # fp32 by type promotion
     D = torch.empty(Z, H, N, dtype=torch.float32, device=O.device)
     strides = None if (O.is_contiguous() and dO.is_contiguous()) else _lib.stride_array(O, dO)
@@ -186,14 +227,15 @@ def _delta(O, dO):
 
 
 def geo_attn_backward(Q, K, V, O, L, dO, coords, sigma, key_padding_mask=None, betas=None,
-                      min_rbf: float = 0.0, max_rbf: float = 1.0, operand_dtype=None, grads=None):
+                      min_rbf: float = 0.0, max_rbf: float = 1.0, operand_dtype=None, grads=None, grad_dtype=None):
     """dQ, dK, dV [Z,H,N,d] f32, d_sigma [H] f32, d_betas [H] f32 | None from the forward's O and logsumexp L.
 
     What the reference's wrapper does around its backward kernel (geometric_attn.py:609-660):
     D = rowsum(O*dO), dO cast to the operand type (bf16, or fp16 with operand_dtype=torch.float16 and betas), zeroed
     accumulators for the per-head scalars.
-    grads: optional (dQ, dK, dV) fp32 [Z,H,N,d] tensors to write into (rows of d contiguous, e.g. views of one
-    [Z,N,3,H,d] buffer); allocated here otherwise.
+    grads: optional (dQ, dK, dV) [Z,H,N,d] tensors of the gradients' type to write into (rows of d contiguous, e.g. views
+    of one [Z,N,3,H,d] buffer); allocated here otherwise.
+    grad_dtype: None (fp32) or the operand type, in which dQ, dK, dV are then returned: the same sums, rounded once.
     """
     Z, H, N, d = Q.shape
     if not Q.is_cuda:
@@ -202,8 +244,11 @@ def geo_attn_backward(Q, K, V, O, L, dO, coords, sigma, key_padding_mask=None, b
     dev = Q.device
     op_dtype, op_type = _operand_type(operand_dtype, betas is not None)
     q, k, v = _operand(Q, op_dtype), _operand(K, op_dtype), _operand(V, op_dtype)
-    D = _delta(O.detach(), dO.detach())
-    do = _operand(dO, op_dtype)
+    if grad_dtype not in (None, torch.float32, op_dtype):
+        raise AssertionError(f"grad_dtype must be torch.float32 or the operand type {op_dtype}, not {grad_dtype}")
+    grad_dtype = grad_dtype or torch.float32
+    gbytes = grad_dtype.itemsize
+    D, do, d_sigma, d_beta = _prepare_backward(O.detach(), dO.detach(), op_dtype, op_type, betas)
     c = _f32(coords, dev)
     s = _f32(sigma, dev)
     lse = _f32(L, dev)
@@ -211,30 +256,28 @@ def geo_attn_backward(Q, K, V, O, L, dO, coords, sigma, key_padding_mask=None, b
     bt = None if betas is None else _f32(betas, dev)
     # gradients in the memory order of their operands (dense), so that what consumes them needs no reshuffle
     def like(t):
-        g = torch.empty_like(t, dtype=torch.float32)
-        return g if _rows_ok(g, 4) else torch.empty(Z, H, N, d, dtype=torch.float32, device=dev)
+        g = torch.empty_like(t, dtype=grad_dtype)
+        return g if _rows_ok(g, gbytes) else torch.empty(Z, H, N, d, dtype=grad_dtype, device=dev)
     if grads is None:
         dQ, dK, dV = like(Q), like(K), like(V)
     else:
         dQ, dK, dV = grads
         for g_ in grads:
-            if g_.dtype != torch.float32 or tuple(g_.shape) != (Z, H, N, d) or not _rows_ok(g_, 4):
-                raise AssertionError("grads must be fp32 [Z,H,N,d] tensors with contiguous, 16-byte aligned rows")
-    d_sigma = torch.zeros(H, dtype=torch.float32, device=dev)
-    d_beta = None if bt is None else torch.zeros(H, dtype=torch.float32, device=dev)
+            if g_.dtype != grad_dtype or tuple(g_.shape) != (Z, H, N, d) or not _rows_ok(g_, gbytes):
+                raise AssertionError(f"grads must be {grad_dtype} [Z,H,N,d] tensors with contiguous, 16-byte aligned rows")
     if Z == 0 or H == 0 or N == 0:
         return dQ, dK, dV, d_sigma, d_beta
     with _lib.on_device(dev):
         stream = _lib.raw_stream(dev)
-        tail = (c.data_ptr(), s.data_ptr(), None if bt is None else bt.data_ptr(), None if m is None else m.data_ptr(),
-                lse.data_ptr(), D.data_ptr(), dQ.data_ptr(), dK.data_ptr(), dV.data_ptr(),
-                d_sigma.data_ptr(), None if d_beta is None else d_beta.data_ptr(),
-                Z, H, N, d, float(min_rbf), float(max_rbf), op_type, stream)
-        if _is_plain(q, k, v, do, dQ, dK, dV):
-            rc = lib.proteus_geo_attn_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), do.data_ptr(), *tail)
-        else:
-            rc = lib.proteus_geo_attn_bwd_strided(q.data_ptr(), k.data_ptr(), v.data_ptr(), do.data_ptr(),
-                                                  _lib.stride_array(q, k, v, do, dQ, dK, dV), *tail)
+        plain = _is_plain(q, k, v, do, dQ, dK, dV)
+        rc = lib.proteus_geo_attn_bwd_typed(q.data_ptr(), k.data_ptr(), v.data_ptr(), do.data_ptr(),
+                                            None if plain else _lib.stride_array(q, k, v, do, dQ, dK, dV),
+                                            c.data_ptr(), s.data_ptr(), None if bt is None else bt.data_ptr(),
+                                            None if m is None else m.data_ptr(),
+                                            lse.data_ptr(), D.data_ptr(), dQ.data_ptr(), dK.data_ptr(), dV.data_ptr(),
+                                            d_sigma.data_ptr(), None if d_beta is None else d_beta.data_ptr(),
+                                            Z, H, N, d, float(min_rbf), float(max_rbf), op_type,
+                                            _lib.GRAD_F32 if grad_dtype == torch.float32 else _lib.GRAD_OPERAND, stream)
     _lib.check(rc, "proteus_geo_attn_bwd")
     return dQ, dK, dV, d_sigma, d_beta
 
@@ -257,15 +300,17 @@ class _geometric_attn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dO):
         Q, K, V, O, L, coords, spreads, betas, mask = ctx.saved_tensors
+        op_dtype = ctx.operand_dtype or torch.bfloat16
         dQ, dK, dV, d_sigma, d_beta = geo_attn_backward(Q, K, V, O, L, dO, coords, spreads, mask, betas,
-                                                        ctx.min_rbf, ctx.max_rbf, ctx.operand_dtype)
+                                                        ctx.min_rbf, ctx.max_rbf, ctx.operand_dtype,
+                                                        grad_dtype=op_dtype if Q.dtype == K.dtype == V.dtype == op_dtype else None)
         return (dQ.to(Q.dtype), dK.to(K.dtype), dV.to(V.dtype), None, d_sigma.to(spreads.dtype),
                 None if betas is None else d_beta.to(betas.dtype), None, None, None, None, None, None, None)
 
 
 def _fused_grad_views_ok(grads):
-    """Can the backward kernels write dQ, dK, dV straight into these views of one fused [Z,N,3,H,d] fp32 buffer?"""
-    return all(_rows_ok(g_, 4) for g_ in grads)
+    """Can the backward kernels write dQ, dK, dV straight into these views of one fused [Z,N,3,H,d] buffer?"""
+    return all(_rows_ok(g_, g_.element_size()) for g_ in grads)
 
 
 class _geometric_attn_qkv(torch.autograd.Function):
@@ -287,11 +332,13 @@ class _geometric_attn_qkv(torch.autograd.Function):
     def backward(ctx, dO):
         qkv, O, L, coords, spreads, betas, mask = ctx.saved_tensors
         Q, K, V = (qkv[:, :, i].permute(0, 2, 1, 3) for i in range(3))
-        g = torch.empty(qkv.shape, dtype=torch.float32, device=qkv.device)
+        op_dtype = ctx.operand_dtype or torch.bfloat16
+        grad_dtype = op_dtype if qkv.dtype == op_dtype else torch.float32
+        g = torch.empty(qkv.shape, dtype=grad_dtype, device=qkv.device)
         grads = tuple(g[:, :, i].permute(0, 2, 1, 3) for i in range(3))
         if _fused_grad_views_ok(grads):
             _, _, _, d_sigma, d_beta = geo_attn_backward(Q, K, V, O, L, dO, coords, spreads, mask, betas,
-                                                         ctx.min_rbf, ctx.max_rbf, ctx.operand_dtype, grads=grads)
+                                                         ctx.min_rbf, ctx.max_rbf, ctx.operand_dtype, grads=grads, grad_dtype=grad_dtype)
         else:
             # a sequence of the fused buffer spans 2 GiB or more: the kernels cannot address it in place, so the
             # gradients go to buffers of their own (as the sliced operator does) and are copied in
