@@ -818,7 +818,7 @@ extern "C" int proteus_geo_attn_legacy_fwd(const uint16_t* Q, const uint16_t* K,
     rc = legacy_args_check(beta, min_rbf, max_rbf, operand_type);
     if (rc != PROTEUS_OK) return rc;
     // a pair mask makes the result sensitive to the last bits of the rbf: use direct distances then
-    if ((tuning == 0 || tuning >= 3) && (min_rbf > 0.f || max_rbf < 1.f)) tuning = 2;
+    if ((tuning == 0 || tuning >= 3) && (min_rbf > 0.f || max_rbf < 1.f)) tuning = tuning == 0 ? GA_AUTO_DIRECT : 2;
     return launch_attn(true, operand_type == PROTEUS_OPERAND_F16, d_head, Q, K, V, coords, sigma, key_pad_mask, O, L, Z, H, N, tuning,
                        beta, min_rbf, max_rbf, contiguous_strides(H, N, d_head), reinterpret_cast<hipStream_t>(stream));
 }
@@ -838,7 +838,7 @@ extern "C" int proteus_geo_attn_legacy_fwd_strided(const uint16_t* Q, const uint
     GaStrides gs;
     rc = strides_from(strides, Z, H, N, d_head, gs);
     if (rc != PROTEUS_OK) return rc;
-    if ((tuning == 0 || tuning >= 3) && (min_rbf > 0.f || max_rbf < 1.f)) tuning = 2;
+    if ((tuning == 0 || tuning >= 3) && (min_rbf > 0.f || max_rbf < 1.f)) tuning = tuning == 0 ? GA_AUTO_DIRECT : 2;
     return launch_attn(true, operand_type == PROTEUS_OPERAND_F16, d_head, Q, K, V, coords, sigma, key_pad_mask, O, L, Z, H, N, tuning,
                        beta, min_rbf, max_rbf, gs, reinterpret_cast<hipStream_t>(stream));
 }

@@ -101,7 +101,8 @@ def geo_attn(Q, K, V, coords, sigma, key_padding_mask=None, return_lse: bool = F
     if not Q.is_cuda:
         raise _lib.ProteusError("geo_attn needs tensors on the GPU (there is no CPU path)")
     # (reading the answer back synchronises with the device: callers whose sigma is positive by construction skip it)
-    if check_sigma and not bool(torch.all(sigma > 0)):
+    # (one copy of the H floats instead of a comparison, a reduction and the copy of its result)
+    if check_sigma and not all(x > 0 for x in sigma.tolist()):
         raise AssertionError(f"spreads must be a tensor of positive, non-zero floats, not {sigma}")
     lib = _lib.load()
     dev = Q.device
