@@ -66,7 +66,7 @@ extern "C" {
  * backward entry point take `int operand_type` before `tuning` / `stream`; a caller built against an older header
  * would pass its tuning selector there).  The Python binding checks for an exact match when it loads the library.
  */
-#define PROTEUS_VERSION 303
+#define PROTEUS_VERSION 304
 int proteus_version(void);
 
 /* Human-readable text for a return code of any entry point. */
@@ -519,6 +519,34 @@ int proteus_add_layernorm_fwd(const void* x, const void* res, const void* gamma,
                               long rows, int D, float eps, int dtype, void* stream);
 int proteus_add_layernorm_fwd_check(const void* x, const void* res, const void* gamma, const void* beta, const void* out,
                                     long rows, int D, float eps, int dtype);
+
+/*
+ * The encoder's training step between its matrix products (fp32; sums over rows in a fixed order, the same bits on every call).
+ *
+ * proteus_add_layernorm_train_fwd   ysum = x + res, out = LayerNorm(ysum) * gamma + beta, stat [rows][2] = (mean, 1 / sqrt(var + eps)).
+ *                                   D a multiple of 4, at most 2048; all pointers 16-byte aligned.
+ * proteus_layernorm_bwd             dx [rows][D] (the gradient of x and of res) and dgamma_dbeta [2][D] from what the forward kept.
+ * proteus_colsum                    sums [C] = column sums of a [rows][C]; with h: of dh = a * gelu'(h) (exact GELU), written too.
+ *                                   C a multiple of 4; dh is a buffer of its own.  Workspace: proteus_train_workspace_bytes (may be 0).
+ * proteus_heads_layout              tensors = {q, k, v projections [H][d_model][d_head], their biases [H][d_head], NULL or the spread
+ *                                   weights' gradient [H], output projection [d_model][d_head][H]} and
+ *                                   W [d_model][3][H][d_head], b [3][H][d_head], Wo [d_model][H][d_head], sigma [H]:
+ *                                   forward fills the latter from the former, sigma = min_spread + exp(spread_w); backward fills the
+ *                                   former (those that are not NULL) from the latter's gradients, spread = sigma * exp(spread_w).
+ *                                   d_model = H * d_head.  `tensors` is read on the host before the call returns.
+ * proteus_embedding_bwd             dW [V][D] = sums of the rows of dout [T][D] per index; V at most 64, D a multiple of 4.
+ */
+size_t proteus_train_workspace_bytes(long rows, int C);
+size_t proteus_layernorm_bwd_workspace_bytes(long rows, int D);
+size_t proteus_embedding_bwd_workspace_bytes(long T, int V, int D);
+int proteus_add_layernorm_train_fwd(const float* x, const float* res, const float* gamma, const float* beta, float* out,
+                                    float* ysum, float* stat, long rows, int D, float eps, void* stream);
+int proteus_layernorm_bwd(const float* dout, const float* ysum, const float* stat, const float* gamma, float* dx,
+                          float* dgamma_dbeta, void* ws, size_t ws_bytes, long rows, int D, void* stream);
+int proteus_colsum(const float* a, const float* h, float* dh, float* sums, void* ws, size_t ws_bytes, long rows, int C, void* stream);
+int proteus_heads_layout(float* const* tensors, float* W, float* b, float* Wo, float* sigma, const float* spread_w,
+                         int d_model, int H, int d_head, float min_spread, int backward, void* stream);
+int proteus_embedding_bwd(const float* dout, const int64_t* tokens, float* dW, void* ws, size_t ws_bytes, long T, int V, int D, void* stream);
 
 #ifdef __cplusplus
 }

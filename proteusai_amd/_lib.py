@@ -12,7 +12,7 @@ LIB_PATH = os.path.join(HERE, "libproteus_hip.so")
 
 COORDS_SOA = 0
 COORDS_AOS = 1
-ABI_VERSION = 303                    # PROTEUS_VERSION of the include/proteus_hip.h these argument lists were written from
+ABI_VERSION = 304                    # PROTEUS_VERSION of the include/proteus_hip.h these argument lists were written from
 OPERAND_BF16, OPERAND_F16 = 0, 1     # PROTEUS_OPERAND_* of include/proteus_hip.h
 GRAD_F32, GRAD_OPERAND = 0, 1        # PROTEUS_GRAD_*
 DTYPE_F32, DTYPE_BF16, DTYPE_F16 = 0, 1, 2   # PROTEUS_DTYPE_*
@@ -32,6 +32,8 @@ SYMBOLS = [
     "proteus_geo_attn_bwd_strided", "proteus_geo_attn_bwd_strided_check", "proteus_geo_attn_num_variants",
     "proteus_geo_attn_variant_name",
     "proteus_add_layernorm_fwd", "proteus_add_layernorm_fwd_check", "proteus_geo_attn_delta", "proteus_geo_attn_delta_check",
+    "proteus_train_workspace_bytes", "proteus_layernorm_bwd_workspace_bytes", "proteus_embedding_bwd_workspace_bytes",
+    "proteus_add_layernorm_train_fwd", "proteus_layernorm_bwd", "proteus_colsum", "proteus_heads_layout", "proteus_embedding_bwd",
 ]
 
 _lib = None
@@ -150,6 +152,21 @@ def load():
     lib.proteus_geo_attn_bwd_typed_check.argtypes = [vp] * 4 + [i64p] + [vp] * 11 + [ci, ci, ci, ci, cf, cf, ci, ci]
     lib.proteus_geo_attn_delta_check.restype = ci
     lib.proteus_geo_attn_delta_check.argtypes = [vp, vp, i64p, vp, ci, ci, ci, ci, ci]
+    cl = ctypes.c_long
+    lib.proteus_train_workspace_bytes.restype = lib.proteus_layernorm_bwd_workspace_bytes.restype = sz
+    lib.proteus_train_workspace_bytes.argtypes = lib.proteus_layernorm_bwd_workspace_bytes.argtypes = [cl, ci]
+    lib.proteus_embedding_bwd_workspace_bytes.restype = sz
+    lib.proteus_embedding_bwd_workspace_bytes.argtypes = [cl, ci, ci]
+    lib.proteus_add_layernorm_train_fwd.restype = ci
+    lib.proteus_add_layernorm_train_fwd.argtypes = [vp] * 7 + [cl, ci, cf, vp]
+    lib.proteus_layernorm_bwd.restype = ci
+    lib.proteus_layernorm_bwd.argtypes = [vp] * 7 + [sz, cl, ci, vp]
+    lib.proteus_colsum.restype = ci
+    lib.proteus_colsum.argtypes = [vp] * 5 + [sz, cl, ci, vp]
+    lib.proteus_heads_layout.restype = ci
+    lib.proteus_heads_layout.argtypes = [ctypes.POINTER(vp)] + [vp] * 5 + [ci, ci, ci, cf, ci, vp]
+    lib.proteus_embedding_bwd.restype = ci
+    lib.proteus_embedding_bwd.argtypes = [vp] * 4 + [sz, cl, ci, ci, vp]
     _lib = lib
     return lib
 

@@ -13,7 +13,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from . import _lib
+from . import _lib, train_ops
 from .geometric_attn import GeoAttention
 from .wf_embedding import WaveFunctionEmbedding
 
@@ -69,6 +69,10 @@ class MLP(nn.Module):
         nn.init.zeros_(self.out_proj.bias)
 
     def forward(self, x):
+        if torch.is_grad_enabled() and self.act is F.gelu and not self.hidden_proj and train_ops.inactive_dropout(self.in_dropout):
+            out = train_ops.gelu_mlp(x, self.in_proj, self.out_proj)
+            if out is not None:
+                return out
         x = self.in_dropout(self.act(self.in_proj(x)))
         for hidden, dropout in zip(self.hidden_proj, self.hidden_dropout):
             x = dropout(self.act(hidden(x)))
@@ -88,9 +92,14 @@ class Encoder(nn.Module):
         self.dropout = nn.Dropout(dropout)
 
     def forward(self, q, k, v, coords, mask=None):
-        q = add_layer_norm(q, self.dropout(self.attn(q, k, v, coords, mask=mask)), self.attn_norm)
-        q = add_layer_norm(q, self.dropout(self.ffn(q)), self.ffn_norm)
+        q = self._residual_norm(q, self.dropout(self.attn(q, k, v, coords, mask=mask)), self.attn_norm)
+        q = self._residual_norm(q, self.dropout(self.ffn(q)), self.ffn_norm)
         return q
+
+    @staticmethod
+    def _residual_norm(q, branch, norm):
+        out = train_ops.add_layer_norm(q, branch, norm)
+        return add_layer_norm(q, branch, norm) if out is None else out
 
 
 class ProteusEncoder(nn.Module):
@@ -121,7 +130,8 @@ class ProteusEncoder(nn.Module):
 
     def forward(self, coords, tokens, key_padding_mask=None):
         wf = self.wf_embedding(coords, None, key_padding_mask=key_padding_mask)           # fp32 [Z,N,d_model]
-        x = wf + self.aa_embedding(tokens).to(wf.dtype)
+        aa = train_ops.embedding(tokens, self.aa_embedding)
+        x = wf + (self.aa_embedding(tokens) if aa is None else aa).to(wf.dtype)
         x = x.to(self.head.weight.dtype)
         for layer in self.layers:
             x = layer(x, x, x, coords, mask=key_padding_mask)

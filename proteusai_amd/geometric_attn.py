@@ -452,6 +452,10 @@ class GeoAttention(nn.Module):
         # where the GEMM left them ([Z,N,(3,)H,d_k], as strided [Z,H,N,d_k] views) and write O token-major, so
         # no head split or merge is ever copied.
         H, dk = self.heads, self.d_k
+        if q is k and k is v:
+            out = train_ops.self_attention(q, coords, mask, self)       # fp32 training
+            if out is not None:
+                return out
 
         def heads_first(x):                # [Z, N, H*d_k] -> [Z, H, N, d_k] view
             return x.view(batch, N, H, dk).permute(0, 2, 1, 3)
@@ -547,3 +551,6 @@ class GeoAttention(nn.Module):
         b = torch.stack((self.q_bias, self.k_bias, self.v_bias)).reshape(-1)
         self._qkv_cache = (key, w.detach(), b.detach()) if keep else None
         return w, b
+
+
+from . import train_ops  # noqa: E402  (it uses the operators above)

@@ -1,0 +1,295 @@
+"""The encoder's training step between its matrix products, as autograd functions on the HIP kernels of encoder_train.hip.
+
+Each function stands for a torch expression that the modules keep as their general path (fp32 tensors on the GPU take
+these; anything else, e.g. other types, autocast, functional transforms, forward-mode differentiation, tracing, tensor
+subclasses, modules with hooks, takes the expression).  A backward that is itself recorded (create_graph) differentiates
+the expression.
+"""
+import ctypes
+
+import torch
+import torch.nn as nn
+import torch.nn.functional as F
+
+from . import _lib
+from . import geometric_attn as ga
+
+_PLAIN_TYPES = (torch.Tensor, nn.Parameter)
+
+
+def recording(*tensors):
+    """Does plain reverse-mode autograd record an operator on these tensors, all of them ordinary fp32 tensors on one GPU?"""
+    if not torch.is_grad_enabled() or torch.is_autocast_enabled("cuda"):
+        return False
+    needed = False
+    dev = tensors[0].device
+    for t in tensors:
+        if type(t) not in _PLAIN_TYPES or t.dtype != torch.float32 or not t.is_cuda or t.device != dev or t.layout != torch.strided:
+            return False
+        needed = needed or t.requires_grad
+    return (needed and torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
+            and not torch.jit.is_tracing() and not torch.compiler.is_compiling())
+
+
+def plain_module(m, cls):
+    """Is `m` exactly a `cls` whose call is its forward: no hooks, no replaced forward?"""
+    g = nn.modules.module
+    return (type(m) is cls and "forward" not in m.__dict__
+            and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+                     or g._global_forward_hooks or g._global_forward_pre_hooks or g._global_backward_hooks or g._global_backward_pre_hooks))
+
+
+def inactive_dropout(m):
+    return plain_module(m, nn.Dropout) and (m.p == 0.0 or not m.training)
+
+
+def aligned(*tensors):
+    return all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in tensors)
+
+
+def _call(fn, dev, *args):
+    """One entry point on torch's current stream; tensors stand for their addresses."""
+    with _lib.on_device(dev):
+        rc = getattr(_lib.load(), fn)(*[a.data_ptr() if isinstance(a, torch.Tensor) else a for a in args], _lib.raw_stream(dev))
+    _lib.check(rc, fn)
+
+
+def _workspace(nbytes, dev):
+    return torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
+
+
+def _dense(t):
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
+def _recorded(expr, inputs, needs, grad):
+    """Gradients of expr(*inputs) as a graph of their own, for the inputs that need one."""
+    with torch.enable_grad():
+        wanted = [t for t, n in zip(inputs, needs) if n]
+        got = iter(torch.autograd.grad(expr(*inputs), wanted, grad, create_graph=True, allow_unused=True))
+    return tuple(next(got) if n else None for n in needs)
+
+
+def column_sums(a, h=None):
+    """Column sums of a [rows, C]; with h (dh, its column sums) of dh = a * gelu'(h)."""
+    rows, C = a.shape
+    sums = torch.empty(C, dtype=torch.float32, device=a.device)
+    dh = None if h is None else torch.empty_like(h)
+    n = _lib.load().proteus_train_workspace_bytes(rows, C)
+    _call("proteus_colsum", a.device, a, h, dh, sums, _workspace(n, a.device), n, rows, C)
+    return sums if h is None else (dh, sums)
+
+
+# ---------------------------------------------------------------------------------------------------- add + LayerNorm
+
+class _AddLayerNorm(torch.autograd.Function):
+    """(LayerNorm(x + res), x + res): the sum is an output so that a recorded backward stays connected to x and res without
+    keeping either."""
+
+    @staticmethod
+    def forward(ctx, x, res, w, b, eps):
+        D = x.shape[-1]
+        rows = x.numel() // D
+        xc, rc_ = _dense(x), _dense(res)
+        out, ysum = torch.empty_like(xc), torch.empty_like(xc)
+        stat = torch.empty(rows, 2, dtype=torch.float32, device=x.device)
+        _call("proteus_add_layernorm_train_fwd", x.device, xc, rc_, w, b, out, ysum, stat, rows, D, eps)
+        ctx.save_for_backward(ysum, stat, w, b)
+        ctx.eps = eps
+        ctx.set_materialize_grads(False)
+        return out, ysum
+
+    @staticmethod
+    def backward(ctx, d, dy):
+        ysum, stat, w, b = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        if d is None:
+            return dy if need[0] else None, dy if need[1] else None, None, None, None
+        if torch.is_grad_enabled():
+            dx, dw, db = _recorded(lambda y_, w_, b_: F.layer_norm(y_, (w.numel(),), w_, b_, ctx.eps), (ysum, w, b), (True, need[2], need[3]), d)
+        else:
+            D = w.numel()
+            rows = ysum.numel() // D
+            d = _dense(d)
+            dx = torch.empty_like(ysum)
+            dwb = torch.empty(2, D, dtype=torch.float32, device=d.device)
+            n = _lib.load().proteus_layernorm_bwd_workspace_bytes(rows, D)
+            _call("proteus_layernorm_bwd", d.device, d, ysum, stat, w, dx, dwb, _workspace(n, d.device), n, rows, D)
+            dw, db = dwb[0] if need[2] else None, dwb[1] if need[3] else None
+        if dy is not None:
+            dx = dx + dy
+        return dx if need[0] else None, dx if need[1] else None, dw, db, None
+
+
+def add_layer_norm(x, res, norm):
+    """norm(x + res), or None where the kernels do not take it."""
+    if not torch.is_grad_enabled():
+        return None
+    w, b = norm.weight, norm.bias
+    if (w is None or b is None or not plain_module(norm, nn.LayerNorm) or x.shape != res.shape or x.dim() < 1 or w.dim() != 1
+            or w.numel() != x.shape[-1] or x.numel() == 0 or w.numel() % 4 or w.numel() > 2048
+            or not recording(x, res, w, b) or not aligned(w, b)):
+        return None
+    return _AddLayerNorm.apply(x, res, w, b, float(norm.eps))[0]
+
+
+# ---------------------------------------------------------------------------------------------------- feed-forward
+
+class _GeluMLP(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, w1, b1, w2, b2):
+        x2 = _dense(x).view(-1, x.shape[-1])
+        h = torch.addmm(b1, x2, w1.t())
+        a = F.gelu(h)
+        ctx.save_for_backward(x, w1, b1, w2, b2, h, a)
+        return torch.addmm(b2, a, w2.t()).view(*x.shape[:-1], w2.shape[0])
+
+    @staticmethod
+    def backward(ctx, d):
+        x, w1, b1, w2, b2, h, a = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        if torch.is_grad_enabled():
+            return _recorded(lambda x_, w1_, b1_, w2_, b2_: F.linear(F.gelu(F.linear(x_, w1_, b1_)), w2_, b2_), (x, w1, b1, w2, b2), need, d)
+        d2 = _dense(d).view(-1, w2.shape[0])
+        x2 = _dense(x).view(-1, w1.shape[1])
+        dw2 = d2.t().mm(a) if need[3] else None
+        db2 = column_sums(d2) if need[4] else None
+        dx = dw1 = db1 = None
+        if need[0] or need[1] or need[2]:
+            dh, db1 = column_sums(d2.mm(w2), h)
+            dw1 = dh.t().mm(x2) if need[1] else None
+            dx = dh.mm(w1).view(x.shape) if need[0] else None
+        return dx, dw1, db1 if need[2] else None, dw2, db2
+
+
+def gelu_mlp(x, lin1, lin2):
+    """lin2(gelu(lin1(x))), or None where the kernels do not take it."""
+    if not torch.is_grad_enabled():
+        return None
+    if not (plain_module(lin1, nn.Linear) and plain_module(lin2, nn.Linear)) or lin1.bias is None or lin2.bias is None:
+        return None
+    w1, b1, w2, b2 = lin1.weight, lin1.bias, lin2.weight, lin2.bias
+    if (x.dim() < 2 or x.shape[-1] != w1.shape[1] or w1.shape[0] != w2.shape[1] or x.numel() == 0 or w1.shape[0] % 4 or w2.shape[0] % 4
+            or not recording(x, w1, b1, w2, b2)):
+        return None
+    return _GeluMLP.apply(x, w1, b1, w2, b2)
+
+
+# ---------------------------------------------------------------------------------------------------- self-attention
+
+def _self_attention_expression(x, coords, mask, qw, kw, vw, qb, kb, vb, spread_w, wo, min_spread, operand_dtype):
+    H, dm, dk = qw.shape
+    Z, N, _ = x.shape
+    w = torch.stack((qw, kw, vw)).permute(2, 0, 1, 3).reshape(dm, 3 * H * dk)
+    b = torch.stack((qb, kb, vb)).reshape(-1)
+    qkv = torch.addmm(b, x.reshape(Z * N, dm), w).view(Z, N, 3, H, dk)
+    O = ga.geometric_attn_qkv(qkv, coords, min_spread + torch.exp(spread_w), None, mask=mask, check_spreads=False, out_dtype=x.dtype,
+                              operand_dtype=operand_dtype)
+    return F.linear(O.permute(0, 2, 1, 3).reshape(Z, N, dm), wo.view(dm, dk, H).permute(0, 2, 1).reshape(dm, dm))
+
+
+def _layout(tensors, W, b, Wo, sigma, spread_w, dm, H, dk, min_spread, backward):
+    ptrs = (ctypes.c_void_p * 8)(*[None if t is None else t.data_ptr() for t in tensors])
+    _call("proteus_heads_layout", W.device, ptrs, W, b, Wo, sigma, spread_w, dm, H, dk, float(min_spread), backward)
+
+
+def _heads(qkv):
+    return tuple(qkv[:, :, i].permute(0, 2, 1, 3) for i in range(3))
+
+
+class _SelfAttention(torch.autograd.Function):
+    """Projections, attention and output projection of one self-attention layer.  The heads' weights are laid side by side
+    by one launch, the fused projection is cast to the operand type once (kept for the backward in that type), and the
+    gradients of the heads' weights and biases leave through one launch."""
+
+    @staticmethod
+    def forward(ctx, x, coords, mask, qw, kw, vw, qb, kb, vb, spread_w, wo, min_spread, operand_dtype):
+        H, dm, dk = qw.shape
+        Z, N, _ = x.shape
+        dev = x.device
+        W = torch.empty(dm, 3 * dm, dtype=torch.float32, device=dev)
+        Wo = torch.empty(dm, dm, dtype=torch.float32, device=dev)
+        b = torch.empty(3 * dm, dtype=torch.float32, device=dev)
+        sigma = torch.empty(H, dtype=torch.float32, device=dev)
+        _layout((qw, kw, vw, qb, kb, vb, None, wo), W, b, Wo, sigma, spread_w, dm, H, dk, min_spread, 0)
+        qkv = torch.addmm(b, _dense(x).view(Z * N, dm), W).to(operand_dtype or torch.bfloat16).view(Z, N, 3, H, dk)
+        O, L = ga.geo_attn(*_heads(qkv), coords, sigma, mask, return_lse=True, check_sigma=False, token_major_out=True,
+                           operand_dtype=operand_dtype)
+        ctx.save_for_backward(x, coords, mask, qw, kw, vw, qb, kb, vb, spread_w, wo, W, Wo, sigma, qkv, O, L)
+        ctx.min_spread, ctx.operand_dtype = min_spread, operand_dtype
+        return O.permute(0, 2, 1, 3).reshape(Z * N, dm).mm(Wo.t()).view(Z, N, dm)
+
+    @staticmethod
+    def backward(ctx, d):
+        x, coords, mask, *params, W, Wo, sigma, qkv, O, L = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        if torch.is_grad_enabled():
+            gx, *gp = _recorded(lambda x_, *p: _self_attention_expression(x_, coords, mask, *p, ctx.min_spread, ctx.operand_dtype),
+                                (x, *params), (need[0], *need[3:11]), d)
+            return (gx, None, None, *gp, None, None)
+        Z, N, _, H, dk = qkv.shape
+        dm = H * dk
+        d2 = _dense(d).view(Z * N, dm)
+        dO = d2.mm(Wo).view(Z, N, H, dk).permute(0, 2, 1, 3)
+        dWo = d2.t().mm(O.permute(0, 2, 1, 3).reshape(Z * N, dm)) if need[10] else Wo      # (Wo: not looked at)
+        g = torch.empty(qkv.shape, dtype=torch.float32, device=d.device)
+        _, _, _, d_sigma, _ = ga.geo_attn_backward(*_heads(qkv), O, L, dO, coords, sigma, mask, None, operand_dtype=ctx.operand_dtype,
+                                                   grads=_heads(g))
+        g2 = g.view(Z * N, 3 * dm)
+        dx = g2.mm(W.t()).view(x.shape) if need[0] else None
+        grads = [torch.empty_like(p, memory_format=torch.contiguous_format) if n else None for p, n in zip(params, need[3:11])]
+        dW = _dense(x).view(Z * N, dm).t().mm(g2) if any(need[3:6]) else W
+        db = column_sums(g2) if any(need[6:9]) else W
+        # (what a gradient is not asked of is not looked at: its place in the list is None)
+        _layout(grads, dW, db, dWo, d_sigma, params[6], dm, H, dk, ctx.min_spread, 1)
+        return (dx, None, None, *grads, None, None)
+
+
+def self_attention(x, coords, mask, m):
+    """The output of the GeoAttention module `m` (README logits) on x, x, x, or None where the kernels do not take it."""
+    if not torch.is_grad_enabled():
+        return None
+    H, dk, dm = m.heads, m.d_k, m.d_model
+    params = (m.q_proj, m.k_proj, m.v_proj, m.q_bias, m.k_bias, m.v_bias, m.spread_weights, m.out_proj.weight)
+    if (m.legacy_logits or dk not in (32, 64, 128) or x.numel() == 0 or not coords.is_cuda or coords.requires_grad or type(coords) not in _PLAIN_TYPES
+            or (mask is not None and type(mask) is not torch.Tensor)
+            or x.shape[1] * 3 * dm * 4 >= 2 ** 31 or m.operand_dtype not in (None, torch.bfloat16)
+            or type(m).get_spreads is not ga.GeoAttention.get_spreads
+            or not recording(x, *params) or not aligned(*params)):
+        return None
+    return _SelfAttention.apply(x, coords, mask, *params, m.min_spread, m.operand_dtype)
+
+
+# ---------------------------------------------------------------------------------------------------- token embedding
+
+class _SmallEmbedding(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, weight, tokens):
+        ctx.save_for_backward(weight, tokens)
+        return F.embedding(tokens, weight)
+
+    @staticmethod
+    def backward(ctx, d):
+        weight, tokens = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return (*_recorded(lambda w: F.embedding(tokens, w), (weight,), (True,), d), None)
+        V, D = weight.shape
+        d, t = _dense(d), tokens.contiguous()
+        dW = torch.empty(V, D, dtype=torch.float32, device=d.device)
+        n = _lib.load().proteus_embedding_bwd_workspace_bytes(t.numel(), V, D)
+        _call("proteus_embedding_bwd", d.device, d, t, dW, _workspace(n, d.device), n, t.numel(), V, D)
+        return dW, None
+
+
+def embedding(tokens, m):
+    """m(tokens) for an nn.Embedding of few rows, or None where the kernel does not take its gradient."""
+    if not torch.is_grad_enabled():
+        return None
+    if not (plain_module(m, nn.Embedding) and m.padding_idx is None and m.max_norm is None and not m.scale_grad_by_freq and not m.sparse):
+        return None
+    V, D = m.weight.shape
+    if (V > 64 or D % 4 or D > 16384 or type(tokens) is not torch.Tensor or tokens.dtype != torch.int64 or tokens.device != m.weight.device
+            or tokens.numel() == 0 or tokens.numel() > 65535 * 128 or not recording(m.weight)):
+        return None
+    return _SmallEmbedding.apply(m.weight, tokens)

@@ -1,0 +1,141 @@
+"""GPU tests of the training step's own kernels (proteusai_amd/train_ops.py) against the torch expressions they stand for,
+evaluated in float64 on the CPU from the same inputs.
+
+Bars: results are fp32 with at most a few thousand terms per sum, taken as short chains of partial sums; 2^-24 per operation over
+chains of some 50 additions of random sign gives rel-L2 below 1e-6, and products (MLP) of K <= 2048 terms below 3e-6."""
+import pytest
+import torch
+import torch.nn as nn
+import torch.nn.functional as F
+
+import proteusai_amd as pa
+from proteusai_amd import synth, train_ops
+
+pytestmark = pytest.mark.gpu
+
+
+def rel(a, b):
+    return float((a.double().cpu() - b).norm() / b.norm().clamp_min(1e-30))
+
+
+def double_copy(m):
+    import copy
+    return copy.deepcopy(m).double().cpu()
+
+
+@pytest.mark.parametrize("shape", [(1, 4), (3, 64), (2, 5, 260), (130, 512), (1027, 1000), (2049, 2048)])
+def test_add_layer_norm(gpu, shape):
+    torch.manual_seed(shape[-1])
+    norm = nn.LayerNorm(shape[-1])
+    with torch.no_grad():
+        norm.weight.add_(0.3 * torch.randn(shape[-1]))
+        norm.bias.add_(torch.randn(shape[-1]))
+    x, r, d = (torch.randn(shape) + 0.5 for _ in range(3))
+    x64, r64 = x.double().requires_grad_(), r.double().requires_grad_()
+    n64 = double_copy(norm)
+    ref = n64(x64 + r64)
+    want = torch.autograd.grad(ref, [x64, r64, n64.weight, n64.bias], d.double())
+    norm = norm.to(gpu)
+    xg, rg = x.to(gpu).requires_grad_(), r.to(gpu).requires_grad_()
+    out = train_ops.add_layer_norm(xg, rg, norm)
+    got = torch.autograd.grad(out, [xg, rg, norm.weight, norm.bias], d.to(gpu))
+    assert rel(out.detach(), ref.detach()) <= 1e-6
+    for g, w, name in zip(got, want, ("x", "res", "gamma", "beta")):
+        assert rel(g, w) <= 2e-6, (name, rel(g, w))
+
+
+@pytest.mark.parametrize("rows,d,hidden", [(1, 4, 8), (2, 12, 20), (129, 64, 100), (2048, 128, 256), (4100, 64, 132)])
+def test_mlp(gpu, rows, d, hidden):
+    torch.manual_seed(rows)
+    mlp = pa.MLP(d_in=d, d_out=d, d_hidden=hidden, dropout=0.0)
+    x, dout = torch.randn(1, rows, d), torch.randn(1, rows, d)
+    m64, x64 = double_copy(mlp), x.double().requires_grad_()
+    ref = m64(x64)
+    want = torch.autograd.grad(ref, [x64, *m64.parameters()], dout.double())
+    mlp, xg = mlp.to(gpu), x.to(gpu).requires_grad_()
+    assert train_ops.gelu_mlp(xg, mlp.in_proj, mlp.out_proj) is not None
+    out = mlp(xg)
+    got = torch.autograd.grad(out, [xg, *mlp.parameters()], dout.to(gpu))
+    assert rel(out.detach(), ref.detach()) <= 3e-6
+    for g, w in zip(got, want):
+        assert rel(g, w) <= 3e-6, (tuple(w.shape), rel(g, w))
+
+
+@pytest.mark.parametrize("T,V,D", [(1, 1, 4), (127, 33, 64), (129, 64, 100), (2048, 33, 512), (8201, 21, 260)])
+def test_embedding_gradient(gpu, T, V, D):
+    torch.manual_seed(T)
+    emb = nn.Embedding(V, D)
+    tokens, d = torch.randint(0, V, (T,)), torch.randn(T, D)
+    want = torch.zeros(V, D, dtype=torch.float64).index_add_(0, tokens, d.double())
+    emb = emb.to(gpu)
+    out = train_ops.embedding(tokens.to(gpu), emb)
+    assert torch.equal(out, emb(tokens.to(gpu)))
+    got, = torch.autograd.grad(out, [emb.weight], d.to(gpu))
+    assert rel(got, want) <= 1e-6
+
+
+@pytest.mark.parametrize("Z,N,H,dk,frozen", [(1, 1, 1, 32, False), (2, 70, 4, 64, False), (2, 129, 2, 128, True)])
+def test_self_attention_module_equals_its_expression(gpu, Z, N, H, dk, frozen, monkeypatch):
+    # the same kernels and products on the same bf16 operands: what differs is the order of the bias sums, one rounding in sigma
+    # and the products' own choice of order (a flipped bf16 rounding of an operand: 2^-9 of single elements)
+    torch.manual_seed(N)
+    m = pa.GeoAttention(d_model=H * dk, heads=H).to(gpu)
+    with torch.no_grad():
+        for p in m.parameters():
+            p.add_(0.1 * torch.randn_like(p))
+    if frozen:
+        m.k_proj.requires_grad_(False)
+        m.q_bias.requires_grad_(False)
+        m.out_proj.weight.requires_grad_(False)
+        m.spread_weights.requires_grad_(False)
+    coords = torch.stack([synth.random_walk_chain(N, torch.Generator().manual_seed(i)) for i in range(Z)]).to(gpu)
+    mask = torch.arange(N, device=gpu)[None, :] >= torch.tensor([N, max(1, N - 9)][:Z], device=gpu)[:, None]
+    x = torch.randn(Z, N, H * dk, device=gpu, requires_grad=True)
+    d = torch.randn(Z, N, H * dk, device=gpu)
+    leaves = [x] + [p for n, p in m.named_parameters() if p.requires_grad and n != "beta_weights"]
+    assert train_ops.self_attention(x, coords, mask, m) is not None
+    out = m(x, x, x, coords, mask)
+    got = torch.autograd.grad(out, leaves, d)
+    monkeypatch.setattr(train_ops, "self_attention", lambda *a: None)
+    ref = m(x, x, x, coords, mask)
+    want = torch.autograd.grad(ref, leaves, d)
+    assert float((out - ref).norm() / ref.norm()) <= 1e-4
+    for g, w in zip(got, want):
+        # (one token: every softmax is 1, and the gradients of q, k and sigma are rounding errors about zero)
+        assert float((g - w).norm()) <= 1e-3 * float(w.norm()) + 1e-4, tuple(w.shape)
+
+
+def test_recorded_backward_differentiates_the_expression(gpu):
+    torch.manual_seed(0)
+    mlp, norm = pa.MLP(d_in=16, d_out=16, d_hidden=24, dropout=0.0), nn.LayerNorm(16)
+    x = torch.randn(1, 9, 16)
+
+    def second(mlp, norm, x, fused):
+        h = mlp(x)
+        out = train_ops.add_layer_norm(x, h, norm) if fused else norm(x + h)
+        g, = torch.autograd.grad((out ** 3).sum(), [x], create_graph=True)
+        return torch.autograd.grad((g ** 2).sum(), [x, norm.weight, mlp.in_proj.weight])
+    want = second(double_copy(mlp), double_copy(norm), x.double().requires_grad_(), False)
+    got = second(mlp.to(gpu), norm.to(gpu), x.to(gpu).requires_grad_(), True)
+    for g, w in zip(got, want):
+        assert rel(g, w) <= 1e-5
+
+
+def test_what_the_general_path_keeps(gpu):
+    mlp, norm = pa.MLP(d_in=16, d_out=16, d_hidden=24, dropout=0.0).to(gpu), nn.LayerNorm(16).to(gpu)
+    x = torch.randn(1, 9, 16, device=gpu, requires_grad=True)
+    lin = (mlp.in_proj, mlp.out_proj)
+    assert train_ops.gelu_mlp(x, *lin) is not None
+    with torch.no_grad():
+        assert train_ops.gelu_mlp(x, *lin) is None
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert train_ops.gelu_mlp(x, *lin) is None and train_ops.add_layer_norm(x, x, norm) is None
+    assert train_ops.gelu_mlp(x.bfloat16(), *lin) is None
+    seen = []
+    handle = mlp.in_proj.register_forward_hook(lambda *a: seen.append(1))
+    mlp(x)
+    handle.remove()
+    assert seen == [1]
+    tangent = torch.func.jvp(lambda t: norm(t + mlp(t)), (x.detach(),), (torch.ones_like(x),))[1]
+    assert torch.isfinite(tangent).all()
+    assert torch.func.vmap(mlp)(x.detach()).shape == x.shape
