@@ -25,6 +25,14 @@ using namespace proteus_we_grid;
 
 constexpr int WA_FLUSH = 1024;           // sources between two flushes: 1024 x 2 x 2^20 is what a signed cell holds
 
+// Few enough workgroups of 16 observers for 16 waves each?  (A batch with a padding mask is taken to hold 0.6 of its tokens.)  With
+// 8 and 16 waves, partial derivatives of 10 terms at K = 256: 252 workgroups 267 / 240 us, 250 with 4000 sources 549 / 449, 226 of
+// 376 unpadded 389 / 349, 304 of 504 unpadded 337 / 356, 454 of 752 472 / 540.
+__host__ __device__ inline bool wa_few(const int Z, const int N, const bool padded)
+{
+    return (padded ? 0.6f : 1.0f) * (float)Z * (float)((N + WG_OBS - 1) / WG_OBS) <= 256.0f;
+}
+
 // ---- preparation: one launch for the lists of sources, one for the tables, which need the longest C-beta vector ----
 
 __global__ __launch_bounds__(256)
@@ -45,9 +53,18 @@ void we_aniso_grid_sources_kernel(const float* __restrict__ coordsA, const float
     if (threadIdx.x == 0) reinterpret_cast<float*>(ws + L.lengths)[blockIdx.x] = b2;
 }
 
+// Terms after which the series at z has a tail below `tail`; more than WG_MAX_TERMS if there is no such number.
+__device__ __forceinline__ int wa_terms(const float z, const float tail)
+{
+    float t = 1.0f;
+    int n = 1;
+    for (; n <= WG_MAX_TERMS; ++n) { t *= 0.5f * z / (float)n; if (2.0f * t < tail) break; }
+    return n;
+}
+
 __global__ __launch_bounds__(256)
 void we_aniso_grid_tables_kernel(const float* __restrict__ cb_magnitudes, const float* __restrict__ wavenumbers,
-                                 char* __restrict__ ws, const int Z, const int N, const int K, const int partials)
+                                 char* __restrict__ ws, const int Z, const int N, const int K, const int partials, const int few)
 {
     const WgLayout L = wg_layout(Z, N, K, true);
     const int tid = threadIdx.x, lane = tid & 63;
@@ -68,15 +85,13 @@ void we_aniso_grid_tables_kernel(const float* __restrict__ cb_magnitudes, const 
     // its derivative with J_(P-1)(z)
     int terms = 0;
     if (b < 1.0e18f && z < 20.0f) {
-        float t = 1.0f;
-        for (terms = 1; terms <= WG_MAX_TERMS; ++terms) { t *= 0.5f * z / (float)terms; if (2.0f * t < 3.0e-7f) break; }
-        terms += partials;
+        terms = wa_terms(z, 3.0e-7f) + partials;
         if (terms > WG_MAX_TERMS) terms = 0;
     }
     if (terms > 1) {
-        // The direct kernel or the grids?  Estimated microseconds (measured at K = 256, 1 x 1000 ... 8 x 2000 tokens, 4 to 12 terms): the direct
-        // kernel takes 0.34 ps per pair and wavenumber with partial derivatives and 0.24 without; a pass over the sources takes a round of
-        // workgroups (two per compute unit) 22 us for its grids and products and 0.059 us per source, down to 0.026 for few workgroups.
+        // The direct kernel or the grids?  Estimated microseconds: the direct kernel takes 0.34 ps per pair and wavenumber with partial
+        // derivatives (0.36 to 0.40 where it has few workgroups) and 0.24 without.  A pass over the sources (8 waves, K = 256, 1 x 1000 ... 8 x 2000 tokens, 4 to 12 terms) takes a round
+        // of workgroups (two per compute unit) 22 us for its grids and products and 0.059 us per source, down to 0.026 for few workgroups.
         float pairs = 0.f, nmax = 0.f, groups = 0.f, ext = 0.f;
         for (int i = tid; i < Z; i += 256) {
             const float n = (float)reinterpret_cast<const int*>(ws + L.counts)[i];
@@ -94,8 +109,13 @@ void we_aniso_grid_tables_kernel(const float* __restrict__ cb_magnitudes, const 
         pairs = wg_block_sum(pairs); groups = wg_block_sum(groups); nmax = wg_block_max(nmax);
         const float cells   = 0.7f * __builtin_sqrtf(ext) * (1.0f / WG_UNIT) * inv_h;
         const float windows = __builtin_ceilf(fmaxf(1.0f, cells / (float)WgGrid<2>::CELLS));
-        const float grid    = (float)((terms + 1) / 2) * windows * (22.0f + (0.026f + 0.033f * fminf(1.0f, groups / 512.0f)) * nmax) * fmaxf(1.0f, groups / 512.0f);
-        const float direct  = pairs * (float)K * (partials ? 3.4e-7f : 2.4e-7f);
+        // (16 waves, 28 batches of 1 x 500 ... 2 x 2000 tokens, K = 128 and 256: a preparation of 37 to 53 us, and per pass 0.0128 us per source,
+        // 0.3 ns per cell and wavenumber, half of that without partial derivatives, and 10 us for the flushes of more than 1024 sources.)
+        const float passes  = (float)((terms + 1) / 2) * windows;
+        const float grid    = few ? (partials ? 53.0f : 37.0f) + passes * (0.0128f * nmax + (partials ? 3.0e-4f : 1.4e-4f) * (float)K * cells / windows
+                                                                          + (nmax > (float)WA_FLUSH ? 10.0f : 0.0f))
+                                  : passes * (22.0f + (0.026f + 0.033f * fminf(1.0f, groups / 512.0f)) * nmax) * fmaxf(1.0f, groups / 512.0f);
+        const float direct  = pairs * (float)K * (partials ? (few ? 3.7e-7f : 3.4e-7f) : 2.4e-7f);
         if (!(grid < direct)) terms = 0;
     }
     const int unit = (int)blockIdx.x * 4 + (tid >> 6);
@@ -103,6 +123,14 @@ void we_aniso_grid_tables_kernel(const float* __restrict__ cb_magnitudes, const 
         WgParams* p = reinterpret_cast<WgParams*>(ws);
         p->inv_h = inv_h; p->h = (float)h; p->cb_mid = mid; p->b_max = b; p->terms = terms;
     }
+    // A tile of 16 wavenumbers takes part in the terms that its own z asks for (at a tenth of the tail above, which only the worst
+    // wavenumber of all comes near): 267 -> 251 us at 4 x 1000 tokens, 10 terms, partial derivatives.
+    if (blockIdx.x == 0)
+        for (int t = tid; t < L.nkt; t += 256) {
+            float zt = 0.f;
+            for (int k = t * 16; k < min(t * 16 + 16, K); ++k) zt = fmaxf(zt, fabsf(wavenumbers[k] * (cb_magnitudes[k] - mid)));
+            reinterpret_cast<int*>(ws + L.tiles)[t] = min(terms, wa_terms(zt * b, 3.0e-8f) + partials);
+        }
     const int rows = WG_GROUPS * L.nkt;
     if (unit < rows) { wg_fill_tables(wavenumbers, ws, L, K, h, unit); return; }
     // (2 - delta_p0) J_p and its derivative: four orders of 16 wavenumbers per wave, by the power series in double precision (|z| <= 10)
@@ -113,7 +141,7 @@ void we_aniso_grid_tables_kernel(const float* __restrict__ cb_magnitudes, const 
         double term = 1.0;
         for (int i = 1; i <= n; ++i) term *= x / (double)i;
         double s = term;
-        for (int m = 1; m <= 40; ++m) { term *= -x * x / ((double)m * (double)(m + n)); s += term; }
+        for (int m = 1; m <= 40; ++m) { term *= -x * x / ((double)m * (double)(m + n)); s += term; if (fabs(term) <= 1.0e-17 * fabs(s)) break; }
         return s;
     };
     const double j = bessel(p), jd = p ? 0.5 * (bessel(p - 1) - bessel(p + 1)) : -bessel(1);
@@ -200,14 +228,14 @@ __device__ void wa_direct(const float4* __restrict__ src, const float4* __restri
 
 // GP  grids per pass over the sources: 1 where the expansion has a single term (then its weights are those of the isotropic kernel,
 //     unsigned denormals), 2 otherwise (signed weights, through the low bits of a magic sum)
-template <bool GRADS, int GP>
+template <bool GRADS, int GP, int WAVES>
 __device__ __forceinline__ void wa_grids(uint32_t* s_grid, int* s_near, const int* s_tok, const char* __restrict__ ws, const WgLayout& L,
                                          const float* __restrict__ cb_magnitudes, const float* __restrict__ wavenumbers,
                                          float* __restrict__ out, float* __restrict__ d_cb, float* __restrict__ d_k,
                                          const float4* __restrict__ src, const float4* __restrict__ srcb, const float4& me, const bool ok,
                                          const int n, const int slot0, const int ncell, const size_t zN, const int K)
 {
-    constexpr int THREADS = 512, WAVES = 8;
+    constexpr int THREADS = WAVES * 64;
     constexpr int STEP   = WAVES * 8;                     // sources per iteration: a wave takes 16 observers x 4 sources, twice
     constexpr int CHUNKS = (WG_ROWS * WG_OBS / 4 + THREADS - 1) / THREADS;
     constexpr int CELLS  = WgGrid<GP>::CELLS;
@@ -307,10 +335,27 @@ __device__ __forceinline__ void wa_grids(uint32_t* s_grid, int* s_near, const in
             const int vc     = n_lo - 3 + mid;
             const bool more  = n_lo > 1 || p0 > 0;
             for (int kp = wave; kp < L.nkt; kp += WAVES) {
+                const int mine = GP == 1 ? 1 : __builtin_amdgcn_readfirstlane(reinterpret_cast<const int*>(ws + L.tiles)[kp]);
+                if (p0 >= mine) continue;
                 const int k = kp * 16 + obs;
+                // (a tile that takes part in the first of two terms only runs the product of the second for nothing, every other pass)
+                wg_f4 ec[GP][1], os[GP][1], oc[GP][1], es[GP][1];
+                wg_product<1, WAVES == 16 ? 4 : 2, GRADS, GP>(reinterpret_cast<const float*>(s_grid), WgGrid<GP>::ROWS * WG_OBS, mid, groups,
+                                                              table + (size_t)kp * 64 + lane, (size_t)L.nkt * 64, 0, ec, os, oc, es);
+                // (what earlier terms and windows left, all loads in flight at once; with the two grids sharing the reads of the tables 251 -> 240 us
+                // at 4 x 1000 tokens, 10 terms, partial derivatives)
+                int tok[4];
                 float2 o[4], ob[4], okk[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) o[i] = ob[i] = okk[i] = make_float2(0.f, 0.f);
+                for (int i = 0; i < 4; ++i) {
+                    tok[i] = k < K ? s_tok[mm * 4 + i] : -1;
+                    o[i] = ob[i] = okk[i] = make_float2(0.f, 0.f);
+                    if (more && tok[i] >= 0) {
+                        const size_t at = (zN + tok[i]) * K + k;
+                        o[i] = reinterpret_cast<const float2*>(out)[at];
+                        if (GRADS) { ob[i] = reinterpret_cast<const float2*>(d_cb)[at]; okk[i] = reinterpret_cast<const float2*>(d_k)[at]; }
+                    }
+                }
                 const WgWave w = waves[k];
                 const double ph = w.rev * (double)vc;
                 const float f  = (float)(ph - __builtin_floor(ph));
@@ -319,10 +364,7 @@ __device__ __forceinline__ void wa_grids(uint32_t* s_grid, int* s_near, const in
                 const float wn = k < K ? wavenumbers[k] : 0.f, kb = wn * bmax, db = k < K ? (cb_magnitudes[k] - mid_cb) * bmax : 0.f;
 #pragma unroll
                 for (int g = 0; g < GP; ++g) {
-                    if (p0 + g >= terms) break;
-                    wg_f4 ec[1], os[1], oc[1], es[1];
-                    wg_product<1, 2, GRADS>(reinterpret_cast<const float*>(s_grid) + g * WgGrid<GP>::ROWS * WG_OBS, mid, groups,
-                                            table + (size_t)kp * 64 + lane, (size_t)L.nkt * 64, 0, ec, os, oc, es);
+                    if (p0 + g >= mine) break;
                     const float2 J = coef[(size_t)(p0 + g) * L.nkt * 16 + k];
                     const int turn = (p0 + g) & 3;                                 // (-i)^p
                     auto turned = [&](const float x, const float y) {
@@ -330,30 +372,26 @@ __device__ __forceinline__ void wa_grids(uint32_t* s_grid, int* s_near, const in
                     };
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        const float2 F = turned(q1 * (ec[0][i] * rc - os[0][i] * rs), q1 * (ec[0][i] * rs + os[0][i] * rc));
+                        const float e = ec[g][0][i], s = os[g][0][i];
+                        const float2 F = turned(q1 * (e * rc - s * rs), q1 * (e * rs + s * rc));
                         o[i].x += J.x * F.x; o[i].y += J.x * F.y;
                         if (GRADS) {
-                            const float gr = q0s * ((float)vc * ec[0][i] + oc[0][i]) + dq * os[0][i];
-                            const float gi = q0s * ((float)vc * os[0][i] + es[0][i]) - dq * ec[0][i];
+                            const float gr = q0s * ((float)vc * e + oc[g][0][i]) + dq * s;
+                            const float gi = q0s * ((float)vc * s + es[g][0][i]) - dq * e;
                             const float2 D = turned(-(gr * rs + gi * rc), gr * rc - gi * rs);          // dF/dk = i F0
                             ob[i].x  += kb * J.y * F.x;                 ob[i].y  += kb * J.y * F.y;
                             okk[i].x += db * J.y * F.x + J.x * D.x;     okk[i].y += db * J.y * F.y + J.x * D.y;
                         }
                     }
                 }
-                if (k >= K) continue;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const int tok = s_tok[mm * 4 + i];
-                    if (tok < 0) continue;
+                    if (tok[i] < 0) continue;
                     const bool keep = slot0 + mm * 4 + i < n;
-                    auto put = [&](float* to, float2 v) {
-                        float2* at = reinterpret_cast<float2*>(to + (zN + tok) * 2 * K) + k;
-                        if (more) { const float2 was = *at; v.x += was.x; v.y += was.y; }
-                        *at = keep ? v : make_float2(0.f, 0.f);
-                    };
-                    put(out, o[i]);
-                    if (GRADS) { put(d_cb, ob[i]); put(d_k, okk[i]); }
+                    const size_t at = (zN + tok[i]) * K + k;
+                    const float2 zero = make_float2(0.f, 0.f);
+                    reinterpret_cast<float2*>(out)[at] = keep ? o[i] : zero;
+                    if (GRADS) { reinterpret_cast<float2*>(d_cb)[at] = keep ? ob[i] : zero; reinterpret_cast<float2*>(d_k)[at] = keep ? okk[i] : zero; }
                 }
             }
         }
@@ -361,12 +399,14 @@ __device__ __forceinline__ void wa_grids(uint32_t* s_grid, int* s_near, const in
     if (ok && (!(lowest > WG_MAGIC) || largest > climit)) s_near[obs] = 1;
 }
 
-template <bool GRADS>
-__global__ __launch_bounds__(512, 4)
+// WAVES  8: two workgroups share a compute unit; 16: twice the waves on the same observers, for launches whose workgroups with
+//        unpadded observers have a compute unit to themselves
+template <bool GRADS, int WAVES>
+__global__ __launch_bounds__(WAVES * 64, 4)
 void we_aniso_grid_kernel(const char* __restrict__ ws, const float* __restrict__ cb_magnitudes, const float* __restrict__ wavenumbers,
                           float* __restrict__ out, float* __restrict__ d_cb, float* __restrict__ d_k, const int Z, const int N, const int K)
 {
-    constexpr int THREADS = 512, WAVES = 8;
+    constexpr int THREADS = WAVES * 64;
     extern __shared__ __align__(16) uint32_t s_grid[];
     __shared__ float s_red[WAVES];
     __shared__ int   s_near[WG_OBS];
@@ -407,8 +447,8 @@ void we_aniso_grid_kernel(const char* __restrict__ ws, const float* __restrict__
     const bool direct = __builtin_amdgcn_readfirstlane(!(reach < (float)((one ? WgGrid<1>::CELLS : WgGrid<2>::CELLS) * WG_MAX_WINDOWS))) != 0;
     const int  ncell  = __builtin_amdgcn_readfirstlane(direct ? 0 : (int)reach);
     if (!direct) {
-        if (!GRADS && one) wa_grids<GRADS, 1>(s_grid, s_near, s_tok, ws, L, cb_magnitudes, wavenumbers, out, d_cb, d_k, src, srcb, me, ok, n, slot0, ncell, zN, K);
-        else               wa_grids<GRADS, 2>(s_grid, s_near, s_tok, ws, L, cb_magnitudes, wavenumbers, out, d_cb, d_k, src, srcb, me, ok, n, slot0, ncell, zN, K);
+        if (!GRADS && one) wa_grids<GRADS, 1, WAVES>(s_grid, s_near, s_tok, ws, L, cb_magnitudes, wavenumbers, out, d_cb, d_k, src, srcb, me, ok, n, slot0, ncell, zN, K);
+        else               wa_grids<GRADS, 2, WAVES>(s_grid, s_near, s_tok, ws, L, cb_magnitudes, wavenumbers, out, d_cb, d_k, src, srcb, me, ok, n, slot0, ncell, zN, K);
     }
 
     __syncthreads();
@@ -429,7 +469,7 @@ void we_aniso_grid_kernel(const char* __restrict__ ws, const float* __restrict__
 // What the grids need beside the direct kernel, two launches of preparation and one that finds nothing to do, costs 13 us.  Without
 // partial derivatives the scales are likely to be equal, where the grid wins from about 1 x 512 tokens on (K = 256: 1 x 512 41 / 49 us,
 // 1 x 2000 79 / 272, 8 x 1000 67 / 486); with them they are likely to differ, and the grids win where the direct kernel takes 400 us or more
-// (8 x 1000 484 / 701, 8 x 2000 1.6 / 2.7 ms, compact 1 x 8192 1.25 / 5.5 ms).  A batch with a padding mask is taken to hold 0.4 of its pairs.
+// (4 x 1000 240 / 365, 1 x 2000 315 / 400, 8 x 1000 484 / 701, compact 1 x 8192 1.25 / 5.5 ms; below, 1 x 1500 305 / 238).  A batch with a padding mask is taken to hold 0.4 of its pairs.
 bool we_aniso_grid_wanted(int Z, int N, int K, bool partials, bool padded, int tuning)
 {
     return tuning == 0 && K >= 64 && (padded ? 0.4 : 1.0) * Z * N * N * K >= (partials ? 1.0e9 : 2.0e8);
@@ -457,12 +497,15 @@ extern "C" int proteus_we_aniso_fwd_ws(const float* coordsA, const float* coords
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     char* ws = (char*)workspace;
     hipLaunchKernelGGL(we_aniso_grid_sources_kernel, dim3((unsigned)Z * (unsigned)L.blocks), dim3(256), 0, st, coordsA, coordsB, coords_layout, mask, ws, Z, N, K);
+    const bool few = wa_few(Z, N, mask != nullptr);
     const unsigned units = (unsigned)((WG_GROUPS + (WG_MAX_TERMS + 3) / 4) * L.nkt);
-    hipLaunchKernelGGL(we_aniso_grid_tables_kernel, dim3((units + 3) / 4), dim3(256), 0, st, cb_magnitudes, wavenumbers, ws, Z, N, K, d_cb ? 1 : 0);
+    hipLaunchKernelGGL(we_aniso_grid_tables_kernel, dim3((units + 3) / 4), dim3(256), 0, st, cb_magnitudes, wavenumbers, ws, Z, N, K, d_cb ? 1 : 0, few ? 1 : 0);
     const dim3 grid((N + WG_OBS - 1) / WG_OBS, Z);
     const size_t lds = (size_t)WG_ROWS * WG_OBS * 4;
-    if (d_cb) hipLaunchKernelGGL((we_aniso_grid_kernel<true>), grid, dim3(512), lds, st, (const char*)ws, cb_magnitudes, wavenumbers, out, d_cb, d_k, Z, N, K);
-    else      hipLaunchKernelGGL((we_aniso_grid_kernel<false>), grid, dim3(512), lds, st, (const char*)ws, cb_magnitudes, wavenumbers, out, d_cb, d_k, Z, N, K);
+#define WA_GO(G_, W_) hipLaunchKernelGGL((we_aniso_grid_kernel<G_, W_>), grid, dim3(W_ * 64), lds, st, (const char*)ws, cb_magnitudes, wavenumbers, out, d_cb, d_k, Z, N, K)
+    if (d_cb) { if (few) WA_GO(true, 16); else WA_GO(true, 8); }
+    else      { if (few) WA_GO(false, 16); else WA_GO(false, 8); }
+#undef WA_GO
     const int rl = (int)hipGetLastError();
     if (rl) return rl;
     return proteus_we_aniso_direct(coordsA, coordsB, coords_layout, cb_magnitudes, wavenumbers, mask, out, d_cb, d_k, Z, N, K, 0,

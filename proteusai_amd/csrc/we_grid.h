@@ -45,7 +45,7 @@ __device__ const double WG_Q[8] = {0.5144796916399992, 0.1467794687271181, 0.022
 
 struct WgBox { float lo[3], hi[3], bad, pad; };  // of 64 tokens, unpadded ones only; bad: one of them is not finite
 
-struct WgLayout { size_t counts, waves, table, boxes, sources, sources_b, lengths, terms, bytes; int npad, nkt, nbox, blocks; };
+struct WgLayout { size_t counts, waves, table, boxes, sources, sources_b, lengths, terms, tiles, bytes; int npad, nkt, nbox, blocks; };
 
 __host__ __device__ inline WgLayout wg_layout(int Z, int N, int K, bool aniso)
 {
@@ -63,7 +63,8 @@ __host__ __device__ inline WgLayout wg_layout(int Z, int N, int K, bool aniso)
     l.sources_b = l.sources + up((size_t)Z * l.npad * 16);
     l.lengths   = l.sources_b + (aniso ? up((size_t)Z * l.npad * 16) : 0);
     l.terms     = l.lengths + (aniso ? up((size_t)Z * l.blocks * 4) : 0);
-    l.bytes     = l.terms + (aniso ? (size_t)WG_MAX_TERMS * l.nkt * 16 * 8 : 0);
+    l.tiles     = l.terms + (aniso ? (size_t)WG_MAX_TERMS * l.nkt * 16 * 8 : 0);
+    l.bytes     = l.tiles + (aniso ? up((size_t)l.nkt * 4) : 0);
     return l;
 }
 
@@ -364,18 +365,20 @@ __device__ __forceinline__ void wg_combine(uint32_t* s_grid, wg_f4 (&acc)[CHUNKS
     }
 }
 
-// One grid at KT tiles of 16 wavenumbers: rows j = 0 .. groups * 8 on both sides of the middle, E and O the sum and difference
-// of the two sides: ec += E cos, os += O sin and (MOMENT) oc += y O cos, es += y E sin with y = j + 1/2.  The tiles share the
-// grid values; the tables come from L2, AHEAD groups of 8 rows ahead.
-template <int KT, int AHEAD, bool MOMENT>
-__device__ __forceinline__ void wg_product(const float* g, const int mid, const int groups, const float4* __restrict__ tb, const size_t ts, const int k2,
-                                           wg_f4 (&ec)[KT], wg_f4 (&os)[KT], wg_f4 (&oc)[KT], wg_f4 (&es)[KT])
+// GR grids (`gs` floats apart) at KT tiles of 16 wavenumbers: rows j = 0 .. groups * 8 on both sides of the middle, E and O the sum
+// and difference of the two sides: ec += E cos, os += O sin and (MOMENT) oc += y O cos, es += y E sin with y = j + 1/2.  The tiles
+// share the grid values, the grids the tables, which come from L2, AHEAD groups of 8 rows ahead.
+template <int KT, int AHEAD, bool MOMENT, int GR>
+__device__ __forceinline__ void wg_product(const float* g, const int gs, const int mid, const int groups, const float4* __restrict__ tb, const size_t ts, const int k2,
+                                           wg_f4 (&ec)[GR][KT], wg_f4 (&os)[GR][KT], wg_f4 (&oc)[GR][KT], wg_f4 (&es)[GR][KT])
 {
     const int lane = threadIdx.x & 63, obs = lane & 15, mm = lane >> 4;
     const float* gp = g + (WG_R0 + mid + mm) * WG_OBS + obs;
     const float* gm = g + (WG_R0 + mid - 1 - mm) * WG_OBS + obs;
 #pragma unroll
-    for (int t = 0; t < KT; ++t) ec[t] = os[t] = oc[t] = es[t] = wg_f4{0.f, 0.f, 0.f, 0.f};
+    for (int r = 0; r < GR; ++r)
+#pragma unroll
+        for (int t = 0; t < KT; ++t) ec[r][t] = os[r][t] = oc[r][t] = es[r][t] = wg_f4{0.f, 0.f, 0.f, 0.f};
     float4 b[AHEAD][KT];
     auto fetch = [&](const int gr, float4 (&bb)[KT]) {
         const float4* at = tb + (size_t)min(gr, WG_GROUPS - 1) * ts;
@@ -393,17 +396,20 @@ __device__ __forceinline__ void wg_product(const float* g, const int mid, const 
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
                 const int off = (8 * gr + 4 * s) * WG_OBS;
-                const float a = gp[off], m = gm[-off];
-                const float E = a + m, O = a - m;
-                const float Oy = O * y, Ey = E * y;
 #pragma unroll
-                for (int t = 0; t < KT; ++t) {
-                    const float bc = s ? b[i][t].z : b[i][t].x, bs = s ? b[i][t].w : b[i][t].y;
-                    ec[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(E, bc, ec[t], 0, 0, 0);
-                    os[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(O, bs, os[t], 0, 0, 0);
-                    if (MOMENT) {
-                        oc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(Oy, bc, oc[t], 0, 0, 0);
-                        es[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(Ey, bs, es[t], 0, 0, 0);
+                for (int r = 0; r < GR; ++r) {
+                    const float a = gp[r * gs + off], m = gm[r * gs - off];
+                    const float E = a + m, O = a - m;
+                    const float Oy = O * y, Ey = E * y;
+#pragma unroll
+                    for (int t = 0; t < KT; ++t) {
+                        const float bc = s ? b[i][t].z : b[i][t].x, bs = s ? b[i][t].w : b[i][t].y;
+                        ec[r][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(E, bc, ec[r][t], 0, 0, 0);
+                        os[r][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(O, bs, os[r][t], 0, 0, 0);
+                        if (MOMENT) {
+                            oc[r][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(Oy, bc, oc[r][t], 0, 0, 0);
+                            es[r][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(Ey, bs, es[r][t], 0, 0, 0);
+                        }
                     }
                 }
                 y += 4.0f;

@@ -242,10 +242,11 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
             const int vc     = n_lo - 3 + mid;                              // the middle lies at vc h
             const int mm     = lane >> 4;
             for (int kp = KT * wave; kp < L.nkt; kp += KT * WAVES) {
-                wg_f4 ec[KT], os[KT], oc[KT], es[KT];
+                wg_f4 ec_[1][KT], os_[1][KT], oc_[1][KT], es_[1][KT];
                 // (an odd number of tiles: the last one twice, written once)
-                wg_product<KT, AHEAD, SUMS>(reinterpret_cast<const float*>(s_grid), mid, groups, table + (size_t)kp * 64 + lane, (size_t)L.nkt * 64,
-                                            kp + 1 < L.nkt ? 64 : 0, ec, os, oc, es);
+                wg_product<KT, AHEAD, SUMS, 1>(reinterpret_cast<const float*>(s_grid), 0, mid, groups, table + (size_t)kp * 64 + lane, (size_t)L.nkt * 64,
+                                               kp + 1 < L.nkt ? 64 : 0, ec_, os_, oc_, es_);
+                const auto &ec = ec_[0], &os = os_[0], &oc = oc_[0], &es = es_[0];
 #pragma unroll
                 for (int t = 0; t < KT; ++t) {
                     const int k = (kp + t) * 16 + obs;
