@@ -139,3 +139,12 @@ def test_what_the_general_path_keeps(gpu):
     tangent = torch.func.jvp(lambda t: norm(t + mlp(t)), (x.detach(),), (torch.ones_like(x),))[1]
     assert torch.isfinite(tangent).all()
     assert torch.func.vmap(mlp)(x.detach()).shape == x.shape
+
+
+def test_replaced_spreads_keep_the_general_path(gpu):
+    m = pa.GeoAttention(d_model=64, heads=2).to(gpu)
+    x = torch.randn(1, 9, 64, device=gpu, requires_grad=True)
+    coords = synth.random_walk_chain(9, torch.Generator().manual_seed(0)).unsqueeze(0).to(gpu)
+    assert train_ops.self_attention(x, coords, None, m) is not None
+    m.get_spreads = lambda: torch.full((2,), 5.0, device=gpu)
+    assert train_ops.self_attention(x, coords, None, m) is None
