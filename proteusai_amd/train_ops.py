@@ -63,11 +63,20 @@ def _dense(t):
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
+def _by_expression(d):
+    """Does a backward that is handed the gradient `d` differentiate the expression?  Where it is itself recorded, and where `d` has
+    no memory of its own for a kernel to read: batched gradients (is_grads_batched, jacobians by vmap)."""
+    return (torch.is_grad_enabled() or type(d) not in _PLAIN_TYPES or not torch._C._has_storage(d)
+            or torch._C._functorch.peek_interpreter_stack() is not None)
+
+
 def _recorded(expr, inputs, needs, grad):
-    """Gradients of expr(*inputs) as a graph of their own, for the inputs that need one."""
+    """Gradients of expr(*inputs) for the inputs that need one, as a graph of their own where gradients are recorded."""
+    create_graph = torch.is_grad_enabled()
     with torch.enable_grad():
         wanted = [t for t, n in zip(inputs, needs) if n]
-        got = iter(torch.autograd.grad(expr(*inputs), wanted, grad, create_graph=True, allow_unused=True))
+        # (retain_graph: the inputs may be outputs of the very node whose backward this is)
+        got = iter(torch.autograd.grad(expr(*inputs), wanted, grad, create_graph=create_graph, retain_graph=True, allow_unused=True))
     return tuple(next(got) if n else None for n in needs)
 
 
@@ -106,7 +115,7 @@ class _AddLayerNorm(torch.autograd.Function):
         need = ctx.needs_input_grad
         if d is None:
             return dy if need[0] else None, dy if need[1] else None, None, None, None
-        if torch.is_grad_enabled():
+        if _by_expression(d):
             dx, dw, db = _recorded(lambda y_, w_, b_: F.layer_norm(y_, (w.numel(),), w_, b_, ctx.eps), (ysum, w, b), (True, need[2], need[3]), d)
         else:
             D = w.numel()
@@ -149,7 +158,7 @@ class _GeluMLP(torch.autograd.Function):
     def backward(ctx, d):
         x, w1, b1, w2, b2, h, a = ctx.saved_tensors
         need = ctx.needs_input_grad
-        if torch.is_grad_enabled():
+        if _by_expression(d):
             return _recorded(lambda x_, w1_, b1_, w2_, b2_: F.linear(F.gelu(F.linear(x_, w1_, b1_)), w2_, b2_), (x, w1, b1, w2, b2), need, d)
         d2 = _dense(d).view(-1, w2.shape[0])
         x2 = _dense(x).view(-1, w1.shape[1])
@@ -224,7 +233,7 @@ class _SelfAttention(torch.autograd.Function):
     def backward(ctx, d):
         x, coords, mask, *params, W, Wo, sigma, qkv, O, L = ctx.saved_tensors
         need = ctx.needs_input_grad
-        if torch.is_grad_enabled():
+        if _by_expression(d):
             gx, *gp = _recorded(lambda x_, *p: _self_attention_expression(x_, coords, mask, *p, ctx.min_spread, ctx.operand_dtype),
                                 (x, *params), (need[0], *need[3:11]), d)
             return (gx, None, None, *gp, None, None)
@@ -272,7 +281,7 @@ class _SmallEmbedding(torch.autograd.Function):
     @staticmethod
     def backward(ctx, d):
         weight, tokens = ctx.saved_tensors
-        if torch.is_grad_enabled():
+        if _by_expression(d):
             return (*_recorded(lambda w: F.embedding(tokens, w), (weight,), (True,), d), None)
         V, D = weight.shape
         d, t = _dense(d), tokens.contiguous()

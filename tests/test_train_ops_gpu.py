@@ -148,3 +148,21 @@ def test_replaced_spreads_keep_the_general_path(gpu):
     assert train_ops.self_attention(x, coords, None, m) is not None
     m.get_spreads = lambda: torch.full((2,), 5.0, device=gpu)
     assert train_ops.self_attention(x, coords, None, m) is None
+
+
+def test_batched_gradients_differentiate_the_expressions(gpu):
+    # is_grads_batched hands every backward a batch of gradients under vmap: no memory that a kernel could read
+    torch.manual_seed(1)
+    mlp, norm, emb = pa.MLP(d_in=16, d_out=16, d_hidden=24, dropout=0.0).to(gpu), nn.LayerNorm(16).to(gpu), nn.Embedding(7, 16).to(gpu)
+    x = torch.randn(1, 9, 16, device=gpu, requires_grad=True)
+    tokens = torch.randint(0, 7, (1, 9), device=gpu)
+    out = train_ops.add_layer_norm(train_ops.embedding(tokens, emb), mlp(x), norm)
+    leaves = [x, emb.weight, *norm.parameters(), *mlp.parameters()]
+    d = torch.randn(3, *out.shape, device=gpu)
+    got = torch.autograd.grad(out, leaves, d, is_grads_batched=True, retain_graph=True)
+    for i in range(3):
+        want = torch.autograd.grad(out, leaves, d[i], retain_graph=True)
+        for g, w in zip(got, want):
+            assert rel(g[i], w.double().cpu()) <= 6e-6, tuple(w.shape)        # twice the bar of the kernels: two fp32 results
+    jac = torch.autograd.functional.jacobian(lambda t: mlp(t), x.detach()[:, :2], vectorize=True)
+    assert jac.shape == (1, 2, 16, 1, 2, 16) and torch.isfinite(jac).all()
