@@ -1,8 +1,8 @@
 """The encoder's training step between its matrix products, as autograd functions on the HIP kernels of encoder_train.hip.
 
 Each function stands for a torch expression that the modules keep as their general path (fp32 tensors on the GPU take
-these; anything else, e.g. other types, autocast, functional transforms, forward-mode differentiation, tracing, tensor
-subclasses, modules with hooks, takes the expression).  A backward that is itself recorded (create_graph) differentiates
+these; anything else, e.g. other types, autocast, functional transforms, forward-mode differentiation, tracing, dispatch
+modes, tensor subclasses, modules with hooks, takes the expression).  A backward that is itself recorded (create_graph) differentiates
 the expression.
 """
 import ctypes
@@ -27,8 +27,9 @@ def recording(*tensors):
         if type(t) not in _PLAIN_TYPES or t.dtype != torch.float32 or not t.is_cuda or t.device != dev or t.layout != torch.strided:
             return False
         needed = needed or t.requires_grad
+    # (a dispatch mode, e.g. make_fx's, sees the torch operators only: a graph traced past a kernel would not hold what it writes)
     return (needed and torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
-            and not torch.jit.is_tracing() and not torch.compiler.is_compiling())
+            and torch._C._len_torch_dispatch_stack() == 0 and not torch.jit.is_tracing() and not torch.compiler.is_compiling())
 
 
 def plain_module(m, cls):
@@ -64,10 +65,10 @@ def _dense(t):
 
 
 def _by_expression(d):
-    """Does a backward that is handed the gradient `d` differentiate the expression?  Where it is itself recorded, and where `d` has
-    no memory of its own for a kernel to read: batched gradients (is_grads_batched, jacobians by vmap)."""
+    """Does a backward that is handed the gradient `d` differentiate the expression?  Where it is itself recorded, where `d` has
+    no memory of its own for a kernel to read (batched gradients: is_grads_batched, jacobians by vmap), and under a dispatch mode."""
     return (torch.is_grad_enabled() or type(d) not in _PLAIN_TYPES or not torch._C._has_storage(d)
-            or torch._C._functorch.peek_interpreter_stack() is not None)
+            or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() > 0)
 
 
 def _recorded(expr, inputs, needs, grad):

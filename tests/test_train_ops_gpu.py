@@ -166,3 +166,22 @@ def test_batched_gradients_differentiate_the_expressions(gpu):
             assert rel(g[i], w.double().cpu()) <= 6e-6, tuple(w.shape)        # twice the bar of the kernels: two fp32 results
     jac = torch.autograd.functional.jacobian(lambda t: mlp(t), x.detach()[:, :2], vectorize=True)
     assert jac.shape == (1, 2, 16, 1, 2, 16) and torch.isfinite(jac).all()
+
+
+def test_traced_graphs_hold_the_expressions(gpu):
+    # make_fx records torch operators: a graph recorded past a kernel would replay with whatever its output buffer held
+    from torch.fx.experimental.proxy_tensor import make_fx
+    torch.manual_seed(2)
+    layer = pa.Encoder(d_model=64, heads=2, d_hidden=96, dropout=0.0).to(gpu)
+
+    def forward(a, b):
+        return layer._residual_norm(a, layer.ffn(b), layer.attn_norm)
+
+    def gradient(a, b):
+        # (cubes: the sum of squares of a normalised row is constant, its gradient a rounding error)
+        return torch.autograd.grad((forward(a, b) ** 3).sum(), [layer.ffn.in_proj.bias, layer.attn_norm.weight])
+    for f in (lambda a, b: (forward(a, b),), gradient):
+        graph = make_fx(f)(*(torch.randn(1, 9, 64, device=gpu) for _ in range(2)))
+        args = [torch.randn(1, 9, 64, device=gpu) for _ in range(2)]
+        for g, w in zip(graph(*args), f(*args)):
+            assert rel(g.detach(), w.detach().double().cpu()) <= 6e-6          # twice the bar of the kernels: two fp32 results
