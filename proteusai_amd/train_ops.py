@@ -66,8 +66,9 @@ def _dense(t):
 
 def _by_expression(d):
     """Does a backward that is handed the gradient `d` differentiate the expression?  Where it is itself recorded, where `d` has
-    no memory of its own for a kernel to read (batched gradients: is_grads_batched, jacobians by vmap), and under a dispatch mode."""
-    return (torch.is_grad_enabled() or type(d) not in _PLAIN_TYPES or not torch._C._has_storage(d)
+    no memory of its own for a kernel to read (batched gradients: is_grads_batched, jacobians by vmap), where it may carry a tangent
+    (forward-mode differentiation), and under a dispatch mode."""
+    return (torch.is_grad_enabled() or type(d) not in _PLAIN_TYPES or not torch._C._has_storage(d) or torch.autograd.forward_ad._current_level >= 0
             or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() > 0)
 
 

@@ -185,3 +185,20 @@ def test_traced_graphs_hold_the_expressions(gpu):
         args = [torch.randn(1, 9, 64, device=gpu) for _ in range(2)]
         for g, w in zip(graph(*args), f(*args)):
             assert rel(g.detach(), w.detach().double().cpu()) <= 6e-6          # twice the bar of the kernels: two fp32 results
+
+
+def test_tangents_of_gradients_come_through(gpu):
+    # a graph recorded outside dual_level, differentiated inside it with a dual gradient: gradients are linear in it
+    import torch.autograd.forward_ad as fwad
+    torch.manual_seed(3)
+    mlp, norm, emb = pa.MLP(d_in=16, d_out=16, d_hidden=24, dropout=0.0).to(gpu), nn.LayerNorm(16).to(gpu), nn.Embedding(7, 16).to(gpu)
+    x = torch.randn(1, 9, 16, device=gpu, requires_grad=True)
+    out = train_ops.add_layer_norm(train_ops.embedding(torch.randint(0, 7, (1, 9), device=gpu), emb), mlp(x), norm)
+    leaves = [x, emb.weight, *norm.parameters(), *mlp.parameters()]
+    d, t = torch.randn_like(out), torch.randn_like(out)
+    with fwad.dual_level():
+        got = [fwad.unpack_dual(g) for g in torch.autograd.grad(out, leaves, fwad.make_dual(d, t), retain_graph=True)]
+        got = [(g.primal, g.tangent) for g in got]
+    want = [torch.autograd.grad(out, leaves, v, retain_graph=True) for v in (d, t)]
+    for (p, q), wp, wt in zip(got, *want):
+        assert rel(p, wp.double().cpu()) <= 6e-6 and q is not None and rel(q, wt.double().cpu()) <= 6e-6      # two fp32 results
