@@ -263,7 +263,7 @@ def self_attention(x, coords, mask, m):
         return None
     H, dk, dm = m.heads, m.d_k, m.d_model
     params = (m.q_proj, m.k_proj, m.v_proj, m.q_bias, m.k_bias, m.v_bias, m.spread_weights, m.out_proj.weight)
-    if (m.legacy_logits or dk not in (32, 64, 128) or x.numel() == 0 or not coords.is_cuda or coords.requires_grad or type(coords) not in _PLAIN_TYPES
+    if (m.legacy_logits or dk not in (32, 64, 128) or dm > 16384 or x.numel() == 0 or not coords.is_cuda or coords.requires_grad or type(coords) not in _PLAIN_TYPES
             or (mask is not None and type(mask) is not torch.Tensor)
             or x.shape[1] * 3 * dm * 4 >= 2 ** 31 or m.operand_dtype not in (None, torch.bfloat16)
             or type(m).get_spreads is not ga.GeoAttention.get_spreads or "get_spreads" in m.__dict__

@@ -202,3 +202,14 @@ def test_tangents_of_gradients_come_through(gpu):
     want = [torch.autograd.grad(out, leaves, v, retain_graph=True) for v in (d, t)]
     for (p, q), wp, wt in zip(got, *want):
         assert rel(p, wp.double().cpu()) <= 6e-6 and q is not None and rel(q, wt.double().cpu()) <= 6e-6      # two fp32 results
+
+
+def test_more_features_than_the_layout_kernel_takes(gpu):
+    # proteus_heads_layout takes up to 16384: beyond, the module trains through its expression
+    with torch.device(gpu):
+        m = pa.GeoAttention(d_model=129 * 128, heads=129)
+    x = torch.randn(1, 3, 129 * 128, device=gpu)
+    coords = synth.random_walk_chain(3, torch.Generator().manual_seed(0)).unsqueeze(0).to(gpu)
+    assert train_ops.self_attention(x, coords, None, m) is None
+    g, = torch.autograd.grad(m(x, x, x, coords).sum(), [m.v_bias])
+    assert g.shape == m.v_bias.shape and torch.isfinite(g).all()
