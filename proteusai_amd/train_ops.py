@@ -139,7 +139,7 @@ def add_layer_norm(x, res, norm):
         return None
     w, b = norm.weight, norm.bias
     if (w is None or b is None or not plain_module(norm, nn.LayerNorm) or x.shape != res.shape or x.dim() < 1 or w.dim() != 1
-            or w.numel() != x.shape[-1] or x.numel() == 0 or w.numel() % 4 or w.numel() > 2048
+            or w.numel() != x.shape[-1] or x.numel() == 0 or w.numel() % 4 or w.numel() > 2048 or not norm.eps >= 0.0
             or not recording(x, res, w, b) or not aligned(w, b)):
         return None
     return _AddLayerNorm.apply(x, res, w, b, float(norm.eps))[0]
@@ -182,6 +182,7 @@ def gelu_mlp(x, lin1, lin2):
         return None
     w1, b1, w2, b2 = lin1.weight, lin1.bias, lin2.weight, lin2.bias
     if (x.dim() < 2 or x.shape[-1] != w1.shape[1] or w1.shape[0] != w2.shape[1] or x.numel() == 0 or w1.shape[0] % 4 or w2.shape[0] % 4
+            or x.numel() // x.shape[-1] > 65535 * 2048        # (rows of a column sum)
             or not recording(x, w1, b1, w2, b2)):
         return None
     return _GeluMLP.apply(x, w1, b1, w2, b2)

@@ -61,7 +61,7 @@ def test_mlp(gpu, rows, d, hidden):
         assert rel(g, w) <= 3e-6, (tuple(w.shape), rel(g, w))
 
 
-@pytest.mark.parametrize("T,V,D", [(1, 1, 4), (127, 33, 64), (129, 64, 100), (2048, 33, 512), (8201, 21, 260)])
+@pytest.mark.parametrize("T,V,D", [(1, 1, 4), (127, 33, 64), (129, 64, 100), (2048, 33, 512), (8201, 21, 260), (300, 64, 100)])
 def test_embedding_gradient(gpu, T, V, D):
     torch.manual_seed(T)
     emb = nn.Embedding(V, D)
@@ -213,3 +213,16 @@ def test_more_features_than_the_layout_kernel_takes(gpu):
     assert train_ops.self_attention(x, coords, None, m) is None
     g, = torch.autograd.grad(m(x, x, x, coords).sum(), [m.v_bias])
     assert g.shape == m.v_bias.shape and torch.isfinite(g).all()
+
+
+def test_what_the_kernels_refuse_the_expressions_take(gpu):
+    norm = nn.LayerNorm(16, eps=-1e-6).to(gpu)
+    x = torch.randn(1, 9, 16, device=gpu, requires_grad=True)
+    assert train_ops.add_layer_norm(x, x, norm) is None and torch.isfinite(pa.Encoder._residual_norm(x, x, norm)).all()
+    mlp = pa.MLP(d_in=4, d_out=4, d_hidden=4, dropout=0.0).to(gpu)
+    rows = torch.zeros(1, 1, 4, device=gpu).expand(1, 65535 * 2048 + 1, 4)
+    assert train_ops.gelu_mlp(rows, mlp.in_proj, mlp.out_proj) is None
+    # the embedding's gradient keeps a table of all rows in LDS: 64 of them
+    tokens = torch.randint(0, 64, (5,), device=gpu)
+    assert train_ops.embedding(tokens, nn.Embedding(64, 12).to(gpu)) is not None
+    assert train_ops.embedding(tokens, nn.Embedding(65, 12).to(gpu)) is None
