@@ -48,10 +48,10 @@ void we_grid_prepare_kernel(const float* __restrict__ coords, const int layout, 
     if (unit < WG_GROUPS * L.nkt) wg_fill_tables(wavenumbers, ws, L, K, h, unit);
 }
 
-// The sources of `near` pairs of one observer (all of them if `all`), summed directly by one wave, a lane per wavenumber.
+// The sources of `near` pairs of one observer, summed directly by one wave, a lane per wavenumber.
 template <bool SUMS>
-__device__ void wg_direct(const float4* __restrict__ src, const int n, const float xi, const float yi, const float zi, const float inv_h, const bool all,
-                          const float* __restrict__ wavenumbers, float* __restrict__ o, float* __restrict__ pc, float* __restrict__ ps, const int K, const int lane)
+__device__ void wg_near(const float4* __restrict__ src, const int n, const float xi, const float yi, const float zi, const float inv_h,
+                        const float* __restrict__ wavenumbers, float* __restrict__ o, float* __restrict__ pc, float* __restrict__ ps, const int K, const int lane)
 {
     for (int kb = 0; kb < K; kb += 256) {
         float kr[4], oc[4], os[4], c[4], s[4];
@@ -66,13 +66,14 @@ __device__ void wg_direct(const float4* __restrict__ src, const int n, const flo
             float r2, inv, r;
             wg_distance(xi - q.x, yi - q.y, zi - q.z, r2, inv, r);
             const bool near = __builtin_bit_cast(int, __builtin_fmaf(r, inv_h, WG_MAGIC)) == __builtin_bit_cast(int, WG_MAGIC);
-            uint64_t todo = __builtin_amdgcn_ballot_w64(j0 + lane < n && r2 != 0.0f && (all || near));
+            uint64_t todo = __builtin_amdgcn_ballot_w64(j0 + lane < n && r2 != 0.0f && near);
             while (todo) {
                 const int b = __builtin_ctzll(todo);
                 todo &= todo - 1;
                 const float rb = wg_lane(r, b), mb = wg_lane(inv, b);
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
+                    if (kb + 64 * u >= K) break;
                     const float ph = __builtin_amdgcn_fractf(rb * kr[u]);
                     const float cs = __builtin_amdgcn_cosf(ph), sn = __builtin_amdgcn_sinf(ph);
                     oc[u] = __builtin_fmaf(cs, mb, oc[u]);
@@ -85,12 +86,102 @@ __device__ void wg_direct(const float4* __restrict__ src, const int n, const flo
         for (int u = 0; u < 4; ++u) {
             const int k = kb + 64 * u + lane;
             if (k >= K) continue;
-            oc[u] *= WG_UNIT; os[u] *= WG_UNIT;
-            if (!all) { oc[u] += o[2 * k]; os[u] += o[2 * k + 1]; }
-            o[2 * k] = oc[u]; o[2 * k + 1] = os[u];
-            if (SUMS) {
-                if (!all) { c[u] += pc[k]; s[u] += ps[k]; }
-                pc[k] = c[u]; ps[k] = s[u];
+            o[2 * k] += oc[u] * WG_UNIT; o[2 * k + 1] += os[u] * WG_UNIT;
+            if (SUMS) { pc[k] += c[u]; ps[k] += s[u]; }
+        }
+    }
+}
+
+// Sums of four values over the four rows of 16 lanes: row i gets that of v_i.
+__device__ __forceinline__ float wg_rows(const float v0, const float v1, const float v2, const float v3)
+{
+    typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+    auto bits = [](const float v) { return __builtin_bit_cast(uint32_t, v); };
+    auto sum  = [](const u2 v) { const uint32_t x = v.x, y = v.y; return __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y); };
+    const float a = sum(__builtin_bit_cast(u2, __builtin_amdgcn_permlane32_swap(bits(v0), bits(v2), false, false)));      // rows 0 + 2, 1 + 3 of v0 | of v2
+    const float b = sum(__builtin_bit_cast(u2, __builtin_amdgcn_permlane32_swap(bits(v1), bits(v3), false, false)));
+    return sum(__builtin_bit_cast(u2, __builtin_amdgcn_permlane16_swap(bits(a), bits(b), false, false)));
+}
+
+// All pairs of the workgroup's 16 observers summed directly, about as fast as the direct kernel does it (vector issue: a multiplication,
+// fract, sine, cosine and two or four accumulations per pair and wavenumber; 1 x 4096, K = 256 1137 us bounded and 1305 unbounded against
+// 1097 and 1188, K = 64 293 and 334 against 321 and 353; a wave per observer, its sources one by one, took 1225 at either K).  A lane holds an observer and a quarter of the
+// wave's sources, 16 wavenumbers sit in scalar registers.  Tiles of 16 wavenumbers `first`, `first` + `step`, ...: as many waves as
+// divide their number evenly take a tile each, the others of a tile share the sources and meet in LDS.
+// BOUNDED: no phase leaves the +-256 revolutions that sine and cosine accept.
+template <bool SUMS, int WAVES, bool BOUNDED>
+__device__ __forceinline__ void wg_direct(uint32_t* s_grid, const int* s_tok, const float4* __restrict__ src, const int n, const int slot0, const float4& me,
+                                          const float* __restrict__ wavenumbers, float* __restrict__ out, float* __restrict__ cos_sums,
+                                          float* __restrict__ sin_sums, const size_t zN, const int K, const int first, const int step)
+{
+    constexpr int KT = 16, V = SUMS ? 4 : 2, BATCH = 8;       // V sums per observer and wavenumber
+    static_assert(WAVES * WG_OBS * KT * V <= WG_ROWS * WG_OBS, "sums of the waves in LDS");
+    const int tid = threadIdx.x, lane = tid & 63, obs = lane & 15, row = lane >> 4;
+    const int wave  = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tiles = ((K + KT - 1) / KT - first + step - 1) / step;
+    const int kw = min(WAVES, tiles & -tiles), sw = WAVES / kw;          // tiles at a time, waves per tile
+    const int kg = wave / sw, sg = wave % sw;
+    typedef float Sums __attribute__((ext_vector_type(V)));
+    Sums* red = reinterpret_cast<Sums*>(s_grid);              // [WAVES][WG_OBS][KT]
+#pragma unroll 1
+    for (int tile = 0; tile < tiles; tile += kw) {
+        const int kl = (first + (tile + kg) * step) * KT + obs;
+        const float krl = (float)((kl < K ? (double)wavenumbers[kl] : 0.0) * 0.15915494309189533577) * (1.0f / WG_UNIT);
+        float kr[KT], acc[V][KT];
+#pragma unroll
+        for (int t = 0; t < KT; ++t) {
+            kr[t] = wg_lane(krl, t);
+#pragma unroll
+            for (int v = 0; v < V; ++v) acc[v][t] = 0.f;
+        }
+        float4 q = src[sg * 4 + row];                          // (reads past the end stay inside the list's padding)
+#pragma unroll 1
+        for (int j0 = sg * 4; j0 < n; j0 += sw * 4) {
+            const float4 p = q;
+            q = src[j0 + sw * 4 + row];
+            float r2, inv, r;
+            wg_distance(me.x - p.x, me.y - p.y, me.z - p.z, r2, inv, r);
+            const bool use = j0 + row < n && r2 != 0.0f;
+            inv = use ? inv : 0.f; r = use ? r : 0.f;
+            const float one = use ? 1.f : 0.f;
+            // phases, then sines and cosines, then accumulations, as in the direct kernel
+#pragma unroll
+            for (int t0 = 0; t0 < KT; t0 += BATCH) {
+                float cs[BATCH], sn[BATCH];
+#pragma unroll
+                for (int t = 0; t < BATCH; ++t) sn[t] = BOUNDED ? r * kr[t0 + t] : __builtin_amdgcn_fractf(r * kr[t0 + t]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int t = 0; t < BATCH; ++t) { cs[t] = __builtin_amdgcn_cosf(sn[t]); sn[t] = __builtin_amdgcn_sinf(sn[t]); }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int t = 0; t < BATCH; ++t) {
+                    acc[0][t0 + t] = __builtin_fmaf(cs[t], inv, acc[0][t0 + t]);
+                    acc[1][t0 + t] = __builtin_fmaf(sn[t], inv, acc[1][t0 + t]);
+                    if constexpr (SUMS) { acc[2][t0 + t] = __builtin_fmaf(cs[t], one, acc[2][t0 + t]); acc[3][t0 + t] = __builtin_fmaf(sn[t], one, acc[3][t0 + t]); }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        __syncthreads();                                       // the previous tiles' sums are read
+#pragma unroll
+        for (int t = 0; t < KT; t += 4) {
+            Sums v;
+#pragma unroll
+            for (int i = 0; i < V; ++i) v[i] = wg_rows(acc[i][t], acc[i][t + 1], acc[i][t + 2], acc[i][t + 3]);
+            red[(wave * WG_OBS + obs) * KT + t + row] = v;
+        }
+        __syncthreads();
+        for (int i = tid; i < kw * WG_OBS * KT; i += WAVES * 64) {
+            const int g = i / (WG_OBS * KT), e = i % (WG_OBS * KT);
+            const int tok = s_tok[e / KT], k = (first + (tile + g) * step) * KT + e % KT;
+            Sums v = red[g * sw * WG_OBS * KT + e];
+            for (int w = 1; w < sw; ++w) v += red[(g * sw + w) * WG_OBS * KT + e];
+            if (tok >= 0 && k < K) {
+                const bool keep = slot0 + e / KT < n;
+                const size_t at = (zN + tok) * K + k;
+                reinterpret_cast<float2*>(out)[at] = keep ? make_float2(v[0] * WG_UNIT, v[1] * WG_UNIT) : make_float2(0.f, 0.f);
+                if constexpr (SUMS) { cos_sums[at] = keep ? v[2] : 0.f; sin_sums[at] = keep ? v[3] : 0.f; }
             }
         }
     }
@@ -126,7 +217,8 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
     const float4* __restrict__ table = reinterpret_cast<const float4*>(ws + L.table);
     const float inv_h = reinterpret_cast<const WgParams*>(ws)->inv_h * (1.0f / WG_UNIT), h = reinterpret_cast<const WgParams*>(ws)->h;
 
-    // ---- the workgroup's slots: unpadded observers first, then padded tokens (zero rows), then nothing ----
+    // ---- the workgroup's slots: unpadded observers first, then padded tokens (zero rows), then nothing.  (Workgroups of a further
+    //      blockIdx.z have the same slots: they only take part in direct sums.) ----
     const int slot0 = blockIdx.x * WG_OBS;
     const int obs   = lane & 15;
     const float4 me = src[slot0 + obs];
@@ -134,6 +226,7 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
     if (tid < WG_OBS) { s_tok[tid] = slot0 + tid < N ? __builtin_bit_cast(int, me.w) : -1; s_near[tid] = 0; }
     if (slot0 >= n) {
         // padded tokens only
+        if (blockIdx.z) return;
         __syncthreads();
         for (int q = 0; q < WG_OBS; ++q) {
             const int t = s_tok[q];
@@ -146,10 +239,28 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
     }
 
     const float reach = wg_reach<WAVES>(me, ok, reinterpret_cast<const WgBox*>(ws + L.boxes) + (size_t)z * L.nbox, L.nbox, s_red) * inv_h + 2.0f;
-    const bool direct = __builtin_amdgcn_readfirstlane(!(reach < (float)(CELLS * WG_MAX_WINDOWS))) != 0;
-    const int  ncell  = __builtin_amdgcn_readfirstlane(direct ? 0 : (int)reach);
+    // Sums without the grid: where there is nothing to spread onto (values that are not finite, wavelengths below 0.11, more than 16
+    // windows), where everything lies in a few cells and most pairs in none, and where the windows, each of which streams all sources
+    // again, cost more.  Per window 8 + 0.006 n us (16 waves; 8 waves, of which two workgroups share a compute unit, 16.6 + 0.0033 n per
+    // workgroup), its product 0.095 K, without the sums 0.055 K; all pairs directly 1.2e-3 n K and 1.0e-3 n K.  (Between the two, so that the
+    // choice and with it `out` do not depend on whether the sums are wanted.)  The direct kernel, the grid alone and this choice, us:
+    // K = 64, a structure 20 times as large 1 x 1024 40 / 168 / 31, 1 x 4096 352 / 499 / 342, 40 times 353 / 1225 / 334; 1 x 4096 at wavelengths from
+    // 1000 on, K = 64 321 / 1116 / 293, K = 256 1097 / 1122 / 1138; a token that is not finite, K = 64 339 / 1223 / 335, K = 256 1125 / 1225 / 1303.
+    const bool far = !(reach < (float)(CELLS * WG_MAX_WINDOWS));
+    const float windows = __builtin_ceilf(reach * (1.0f / (float)CELLS));
+    const float by_grid = windows * ((WAVES == 16 ? 8.0f + 6.0e-3f * (float)n : 16.6f + 3.3e-3f * (float)n) + 0.075f * (float)K);
+    const float by_pair = 1.1e-3f * (float)n * (float)K / (float)gridDim.z;
+    const bool direct = __builtin_amdgcn_readfirstlane(far || reach < 4.0f || (windows > 1.0f && by_grid > by_pair)) != 0;
+    if (direct) {
+        // (a cell is at most pi / 3.5 of phase: 1750 of them are 250 revolutions)
+        if (reach < 1750.0f) wg_direct<SUMS, WAVES, true>(s_grid, s_tok, src, n, slot0, me, wavenumbers, out, cos_sums, sin_sums, zN, K, blockIdx.z, gridDim.z);
+        else                 wg_direct<SUMS, WAVES, false>(s_grid, s_tok, src, n, slot0, me, wavenumbers, out, cos_sums, sin_sums, zN, K, blockIdx.z, gridDim.z);
+        return;
+    }
+    if (blockIdx.z) return;
+    const int ncell = __builtin_amdgcn_readfirstlane((int)reach);
 
-    if (!direct) {
+    {
         // ---- the spreading kernel's coefficients, in fixed point ----
         // A weight is made as a single-precision denormal: its bit pattern is the rounded integer, and no conversion is needed
         // (4.7 clocks each).  Of the 2^-149 that takes 2^-12 comes with 1/r (WG_UNIT) and the rest with the coefficients, so that
@@ -284,24 +395,13 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
         if (lowest == WG_MAGIC && ok) s_near[obs] = 1;
     }
 
-    // ---- pairs closer than h / 2, and everything where the grid is of no use ----
+    // ---- pairs closer than h / 2 ----
     __syncthreads();
     for (int q = wave; q < WG_OBS; q += WAVES) {
-        const int t = s_tok[q];
-        if (t < 0) continue;
-        const size_t row = zN + t;
-        float* o  = out + row * 2 * K;
-        float* pc = SUMS ? cos_sums + row * K : nullptr;
-        float* ps = SUMS ? sin_sums + row * K : nullptr;
-        if (slot0 + q >= n) {
-            if (direct) {
-                for (int k = lane; k < 2 * K; k += 64) o[k] = 0.f;
-                if (SUMS) for (int k = lane; k < K; k += 64) { pc[k] = 0.f; ps[k] = 0.f; }
-            }
-            continue;
-        }
-        if (!direct && !s_near[q]) continue;
-        wg_direct<SUMS>(src, n, wg_lane(me.x, q), wg_lane(me.y, q), wg_lane(me.z, q), inv_h, direct, wavenumbers, o, pc, ps, K, lane);
+        if (slot0 + q >= n || !s_near[q]) continue;
+        const size_t row = zN + s_tok[q];
+        wg_near<SUMS>(src, n, wg_lane(me.x, q), wg_lane(me.y, q), wg_lane(me.z, q), inv_h, wavenumbers, out + row * 2 * K,
+                      SUMS ? cos_sums + row * K : nullptr, SUMS ? sin_sums + row * K : nullptr, K, lane);
     }
 }
 
@@ -335,9 +435,10 @@ extern "C" int proteus_we_fwd_ws(const float* coords, int coords_layout,
     const WgLayout L = wg_layout(Z, N, K, false);
     const unsigned prep = (unsigned)Z * (unsigned)L.blocks + (unsigned)((WG_GROUPS * L.nkt + 3) / 4);
     hipLaunchKernelGGL(we_grid_prepare_kernel, dim3(prep), dim3(256), 0, st, coords, coords_layout, wavenumbers, mask, (char*)workspace, Z, N, K);
-    const dim3 grid((N + WG_OBS - 1) / WG_OBS, Z);
+    dim3 grid((N + WG_OBS - 1) / WG_OBS, Z);
     const size_t lds = (size_t)WG_ROWS * WG_OBS * 4;
     const bool few = (long)grid.x * Z <= 256;
+    if (few) grid.z = min(L.nkt, 256 / (int)(grid.x * grid.y));        // (direct sums share the wavenumbers out over the idle compute units)
 #define WG_GO(S_, W_) hipLaunchKernelGGL((we_grid_kernel<S_, W_>), grid, dim3(W_ * 64), lds, st, (const char*)workspace, wavenumbers, out, cos_sums, sin_sums, Z, N, K)
     if (cos_sums) { if (few) WG_GO(true, 16); else WG_GO(true, 8); }
     else          { if (few) WG_GO(false, 16); else WG_GO(false, 8); }

@@ -47,6 +47,13 @@ CASES = {                       # N, Z, K, scale of the chain, mask
     "several windows of the grid": (700, 2, 33, 30.0, None),
     "several windows and flushes": (1500, 1, 16, 20.0, "scattered"),
     "beyond the windows": (90, 1, 33, 3000.0, None),
+    # sums without the grid: tiles of wavenumbers shared out over workgroups and over the waves of one
+    "beyond the windows, 250 wavenumbers, an empty item": (333, 4, 250, 900.0, "tail"),
+    "beyond the windows, more than 256 workgroups": (130, 32, 72, 3000.0, "scattered"),
+    "windows that cost more than the pairs": (1100, 1, 64, 25.0, "scattered"),
+    "windows that cost more than the pairs, more than 256 workgroups": (1100, 4, 112, 25.0, None),
+    "everything in a cell or two": (500, 2, 64, 0.002, "scattered"),
+    "everything in a cell or two, more than 256 workgroups": (300, 16, 16, 0.002, None),
 }
 
 
