@@ -6,6 +6,7 @@ modes, tensor subclasses, modules with hooks, takes the expression).  A backward
 the expression.
 """
 import ctypes
+import functools
 
 import torch
 import torch.nn as nn
@@ -72,6 +73,18 @@ def _by_expression(d):
             or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() > 0)
 
 
+def _without_autocast(backward):
+    """A backward whose products stay in fp32 as its forward's are (`recording`): under autocast, which holds for products of a
+    backward called inside its region, they would come out in 16 bits, and the kernels would read past their ends."""
+    @functools.wraps(backward)
+    def run(ctx, *grads):
+        if not torch.is_autocast_enabled("cuda"):
+            return backward(ctx, *grads)
+        with torch.autocast("cuda", enabled=False):
+            return backward(ctx, *grads)
+    return run
+
+
 def _recorded(expr, inputs, needs, grad):
     """Gradients of expr(*inputs) for the inputs that need one, as a graph of their own where gradients are recorded."""
     create_graph = torch.is_grad_enabled()
@@ -112,6 +125,7 @@ class _AddLayerNorm(torch.autograd.Function):
         return out, ysum
 
     @staticmethod
+    @_without_autocast
     def backward(ctx, d, dy):
         ysum, stat, w, b = ctx.saved_tensors
         need = ctx.needs_input_grad
@@ -157,6 +171,7 @@ class _GeluMLP(torch.autograd.Function):
         return torch.addmm(b2, a, w2.t()).view(*x.shape[:-1], w2.shape[0])
 
     @staticmethod
+    @_without_autocast
     def backward(ctx, d):
         x, w1, b1, w2, b2, h, a = ctx.saved_tensors
         need = ctx.needs_input_grad
@@ -233,6 +248,7 @@ class _SelfAttention(torch.autograd.Function):
         return O.permute(0, 2, 1, 3).reshape(Z * N, dm).mm(Wo.t()).view(Z, N, dm)
 
     @staticmethod
+    @_without_autocast
     def backward(ctx, d):
         x, coords, mask, *params, W, Wo, sigma, qkv, O, L = ctx.saved_tensors
         need = ctx.needs_input_grad
@@ -282,6 +298,7 @@ class _SmallEmbedding(torch.autograd.Function):
         return F.embedding(tokens, weight)
 
     @staticmethod
+    @_without_autocast
     def backward(ctx, d):
         weight, tokens = ctx.saved_tensors
         if _by_expression(d):

@@ -226,3 +226,23 @@ def test_what_the_kernels_refuse_the_expressions_take(gpu):
     tokens = torch.randint(0, 64, (5,), device=gpu)
     assert train_ops.embedding(tokens, nn.Embedding(64, 12).to(gpu)) is not None
     assert train_ops.embedding(tokens, nn.Embedding(65, 12).to(gpu)) is None
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_backward_inside_an_autocast_region(gpu, dtype):
+    # a forward outside autocast (or in a region that disables it), differentiated inside: products in 16 bits would be handed
+    # to kernels that read fp32
+    torch.manual_seed(4)
+    layer = pa.Encoder(d_model=128, heads=2, d_hidden=192, dropout=0.0).to(gpu)
+    emb = nn.Embedding(7, 128).to(gpu)
+    coords = synth.random_walk_chain(65, torch.Generator().manual_seed(0)).unsqueeze(0).to(gpu)
+    x = train_ops.embedding(torch.randint(0, 7, (1, 65), device=gpu), emb)
+    out = layer(x, x, x, coords)
+    leaves = [emb.weight] + [p for n, p in layer.named_parameters() if not n.endswith("beta_weights")]
+    d = torch.randn_like(out)
+    want = torch.autograd.grad(out, leaves, d, retain_graph=True)
+    with torch.autocast("cuda", dtype=dtype):
+        got = torch.autograd.grad(out, leaves, d)
+    for g, w in zip(got, want):
+        # twice the bar of the kernels: two fp32 results (the spreads' gradient: sums in the order of atomics)
+        assert rel(g, w.double().cpu()) <= (1e-4 if w.shape == layer.attn.spread_weights.shape else 6e-6), tuple(w.shape)
