@@ -73,6 +73,14 @@ def _by_expression(d):
             or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() > 0)
 
 
+def _saved(t, shape, dtype=torch.float32):
+    """A saved tensor as a kernel may read it.  What saved-tensor hooks give back may lie differently (strides, alignment); another
+    type or shape is an error, as it would be in a torch operator."""
+    if t.dtype != dtype or tuple(t.shape) != tuple(shape):
+        raise RuntimeError(f"a tensor saved as {dtype} {tuple(shape)} came back as {t.dtype} {tuple(t.shape)}")
+    return _dense(t)
+
+
 def _without_autocast(backward):
     """A backward whose products stay in fp32 as its forward's are (`recording`): under autocast, which holds for products of a
     backward called inside its region, they would come out in 16 bits, and the kernels would read past their ends."""
@@ -134,9 +142,10 @@ class _AddLayerNorm(torch.autograd.Function):
         if _by_expression(d):
             dx, dw, db = _recorded(lambda y_, w_, b_: F.layer_norm(y_, (w.numel(),), w_, b_, ctx.eps), (ysum, w, b), (True, need[2], need[3]), d)
         else:
-            D = w.numel()
-            rows = ysum.numel() // D
-            d = _dense(d)
+            D = d.shape[-1]
+            rows = d.numel() // D
+            d, w = _dense(d), _saved(w, (D,))
+            ysum, stat = _saved(ysum, d.shape), _saved(stat, (rows, 2))
             dx = torch.empty_like(ysum)
             dwb = torch.empty(2, D, dtype=torch.float32, device=d.device)
             n = _lib.load().proteus_layernorm_bwd_workspace_bytes(rows, D)
@@ -183,7 +192,8 @@ class _GeluMLP(torch.autograd.Function):
         db2 = column_sums(d2) if need[4] else None
         dx = dw1 = db1 = None
         if need[0] or need[1] or need[2]:
-            dh, db1 = column_sums(d2.mm(w2), h)
+            da = d2.mm(w2)
+            dh, db1 = column_sums(da, _saved(h, da.shape))
             dw1 = dh.t().mm(x2) if need[1] else None
             dx = dh.mm(w1).view(x.shape) if need[0] else None
         return dx, dw1, db1 if need[2] else None, dw2, db2
@@ -260,17 +270,17 @@ class _SelfAttention(torch.autograd.Function):
         dm = H * dk
         d2 = _dense(d).view(Z * N, dm)
         dO = d2.mm(Wo).view(Z, N, H, dk).permute(0, 2, 1, 3)
-        dWo = d2.t().mm(O.permute(0, 2, 1, 3).reshape(Z * N, dm)) if need[10] else Wo      # (Wo: not looked at)
         g = torch.empty(qkv.shape, dtype=torch.float32, device=d.device)
         _, _, _, d_sigma, _ = ga.geo_attn_backward(*_heads(qkv), O, L, dO, coords, sigma, mask, None, operand_dtype=ctx.operand_dtype,
                                                    grads=_heads(g))
         g2 = g.view(Z * N, 3 * dm)
         dx = g2.mm(W.t()).view(x.shape) if need[0] else None
         grads = [torch.empty_like(p, memory_format=torch.contiguous_format) if n else None for p, n in zip(params, need[3:11])]
-        dW = _dense(x).view(Z * N, dm).t().mm(g2) if any(need[3:6]) else W
-        db = column_sums(g2) if any(need[6:9]) else W
         # (what a gradient is not asked of is not looked at: its place in the list is None)
-        _layout(grads, dW, db, dWo, d_sigma, params[6], dm, H, dk, ctx.min_spread, 1)
+        dW = _dense(x).view(Z * N, dm).t().mm(g2) if any(need[3:6]) else g2
+        db = column_sums(g2) if any(need[6:9]) else g2
+        dWo = d2.t().mm(O.permute(0, 2, 1, 3).reshape(Z * N, dm)) if need[10] else g2
+        _layout(grads, dW, db, dWo, d_sigma, _saved(params[6], (H,)), dm, H, dk, ctx.min_spread, 1)
         return (dx, None, None, *grads, None, None)
 
 
@@ -304,7 +314,7 @@ class _SmallEmbedding(torch.autograd.Function):
         if _by_expression(d):
             return (*_recorded(lambda w: F.embedding(tokens, w), (weight,), (True,), d), None)
         V, D = weight.shape
-        d, t = _dense(d), tokens.contiguous()
+        d, t = _dense(d), _saved(tokens, d.shape[:-1], torch.int64)
         dW = torch.empty(V, D, dtype=torch.float32, device=d.device)
         n = _lib.load().proteus_embedding_bwd_workspace_bytes(t.numel(), V, D)
         _call("proteus_embedding_bwd", d.device, d, t, dW, _workspace(n, d.device), n, t.numel(), V, D)

@@ -246,3 +246,43 @@ def test_backward_inside_an_autocast_region(gpu, dtype):
     for g, w in zip(got, want):
         # twice the bar of the kernels: two fp32 results (the spreads' gradient: sums in the order of atomics)
         assert rel(g, w.double().cpu()) <= (1e-4 if w.shape == layer.attn.spread_weights.shape else 6e-6), tuple(w.shape)
+
+
+def _layer_and_inputs(gpu):
+    torch.manual_seed(5)
+    layer = pa.Encoder(d_model=64, heads=2, d_hidden=96, dropout=0.0).to(gpu)
+    coords = synth.random_walk_chain(33, torch.Generator().manual_seed(0)).unsqueeze(0).to(gpu)
+    return layer, nn.Embedding(7, 64).to(gpu), torch.randint(0, 7, (1, 33), device=gpu), coords
+
+
+def test_saved_tensors_that_come_back_lying_differently(gpu):
+    # saved-tensor hooks may give back tensors with other strides, at addresses that are multiples of 4 bytes only
+    layer, emb, tokens, coords = _layer_and_inputs(gpu)
+    leaves = [emb.weight] + [p for n, p in layer.named_parameters() if not n.endswith("beta_weights")]
+
+    def gradients(unpack):
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+            x = train_ops.embedding(tokens, emb)
+            out = layer(x, x, x, coords)
+        return torch.autograd.grad(out, leaves, torch.ones_like(out).tril())
+
+    def shifted(t):
+        return torch.cat((t.new_zeros(1), t.reshape(-1)))[1:].view(t.shape)
+
+    def strided(t):
+        return torch.stack((t, t), -1)[..., 0]
+    want = gradients(lambda t: t)
+    for unpack in (shifted, strided):
+        for g, w in zip(gradients(unpack), want):
+            # twice the bar of the kernels: two fp32 results (the spreads' gradient: sums in the order of atomics)
+            assert rel(g, w.double().cpu()) <= (1e-4 if w.shape == layer.attn.spread_weights.shape else 6e-6), tuple(w.shape)
+
+
+def test_saved_tensors_of_another_type_are_refused(gpu):
+    layer, emb, tokens, coords = _layer_and_inputs(gpu)
+    x = torch.randn(1, 33, 64, device=gpu, requires_grad=True)
+    for f in (lambda: train_ops.embedding(tokens, emb), lambda: layer.ffn(x), lambda: train_ops.add_layer_norm(x, x, layer.ffn_norm)):
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t.to(torch.int32 if t.dtype == torch.int64 else torch.bfloat16)):
+            out = f()
+        with pytest.raises(RuntimeError):
+            out.sum().backward()
