@@ -177,7 +177,8 @@ class _GeluMLP(torch.autograd.Function):
         h = torch.addmm(b1, x2, w1.t())
         a = F.gelu(h)
         ctx.save_for_backward(x, w1, b1, w2, b2, h, a)
-        return torch.addmm(b2, a, w2.t()).view(*x.shape[:-1], w2.shape[0])
+        # (not a view: what is changed in place behind the feed-forward must not be one)
+        return torch.ops.aten._unsafe_view(torch.addmm(b2, a, w2.t()), (*x.shape[:-1], w2.shape[0]))
 
     @staticmethod
     @_without_autocast
@@ -255,7 +256,7 @@ class _SelfAttention(torch.autograd.Function):
                            operand_dtype=operand_dtype)
         ctx.save_for_backward(x, coords, mask, qw, kw, vw, qb, kb, vb, spread_w, wo, W, Wo, sigma, qkv, O, L)
         ctx.min_spread, ctx.operand_dtype = min_spread, operand_dtype
-        return O.permute(0, 2, 1, 3).reshape(Z * N, dm).mm(Wo.t()).view(Z, N, dm)
+        return torch.ops.aten._unsafe_view(O.permute(0, 2, 1, 3).reshape(Z * N, dm).mm(Wo.t()), (Z, N, dm))      # (not a view, as in the feed-forward)
 
     @staticmethod
     @_without_autocast

@@ -286,3 +286,14 @@ def test_saved_tensors_of_another_type_are_refused(gpu):
             out = f()
         with pytest.raises(RuntimeError):
             out.sum().backward()
+
+
+def test_outputs_may_be_changed_in_place(gpu):
+    layer, emb, tokens, coords = _layer_and_inputs(gpu)
+    x = torch.randn(1, 33, 64, device=gpu, requires_grad=True)
+    for f in (lambda: train_ops.embedding(tokens, emb), lambda: layer.ffn(x), lambda: layer.attn(x, x, x, coords),
+              lambda: train_ops.add_layer_norm(x, x, layer.ffn_norm)):
+        out = f()
+        assert out is not None and not out._is_view()
+        out += 1.0
+        out.sum().backward()
