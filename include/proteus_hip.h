@@ -66,7 +66,7 @@ extern "C" {
  * backward entry point take `int operand_type` before `tuning` / `stream`; a caller built against an older header
  * would pass its tuning selector there).  The Python binding checks for an exact match when it loads the library.
  */
-#define PROTEUS_VERSION 304
+#define PROTEUS_VERSION 305
 int proteus_version(void);
 
 /* Human-readable text for a return code of any entry point. */
@@ -528,8 +528,8 @@ int proteus_add_layernorm_fwd_check(const void* x, const void* res, const void* 
  * proteus_layernorm_bwd             dx [rows][D] (the gradient of x and of res) and dgamma_dbeta [2][D] from what the forward kept.
  * proteus_colsum                    sums [C] = column sums of a [rows][C]; with h: of dh = a * gelu'(h) (exact GELU), written too.
  *                                   C a multiple of 4; dh is a buffer of its own.  Workspace: proteus_train_workspace_bytes (may be 0).
- * proteus_heads_layout              tensors = {q, k, v projections [H][d_model][d_head], their biases [H][d_head], NULL or the spread
- *                                   weights' gradient [H], output projection [d_model][d_head][H]} and
+ * proteus_heads_layout              tensors = {q, k, v projections [H][d_model][d_head], their biases [H][d_head], NULL or [H] (forward: a
+ *                                   copy of spread_w; backward: its gradient), output projection [d_model][d_head][H]} and
  *                                   W [d_model][3][H][d_head], b [3][H][d_head], Wo [d_model][H][d_head], sigma [H]:
  *                                   forward fills the latter from the former, sigma = min_spread + exp(spread_w); backward fills the
  *                                   former (those that are not NULL) from the latter's gradients, spread = sigma * exp(spread_w).

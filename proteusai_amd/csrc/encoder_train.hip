@@ -215,7 +215,7 @@ int colsum(const float* a, const float* h, float* dh, float* out, float* ws, lon
 }
 
 // Per-head projections [H][dm][dk] (three of them) <-> one matrix W [dm][3][H][dk]; output projection [dm][dk][H] <->
-// Wo [dm][H][dk]; biases; sigma = min_spread + exp(w).  torch: two cat, two copies, two elementwise launches forward;
+// Wo [dm][H][dk]; biases; sigma = min_spread + exp(w), with a copy of w.  torch: two cat, two copies, two elementwise launches forward;
 // copies and additions of views backward (some 12).  One launch each way, 5 us.
 struct HeadTensors {
     float *q_w, *k_w, *v_w, *q_b, *k_b, *v_b, *spread, *out_w;
@@ -252,8 +252,11 @@ void heads_layout_kernel(const HeadTensors t, float* __restrict__ W, float* __re
             if (s) { if (BACK) s[e] = b[c]; else b[c] = s[e]; }
         } else {
             const int h = (int)(i - nW - nO - nB);
-            if (!BACK) sigma[h] = min_spread + expf(spread_w[h]);
-            else if (t.spread) t.spread[h] = sigma[h] * expf(spread_w[h]);        // sigma: its gradient
+            if (!BACK) {
+                const float w = spread_w[h];
+                sigma[h] = min_spread + expf(w);
+                if (t.spread) t.spread[h] = w;
+            } else if (t.spread) t.spread[h] = sigma[h] * expf(spread_w[h]);        // sigma: its gradient
         }
     }
 }

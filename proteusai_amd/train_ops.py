@@ -207,7 +207,8 @@ def gelu_mlp(x, lin1, lin2):
     if not (plain_module(lin1, nn.Linear) and plain_module(lin2, nn.Linear)) or lin1.bias is None or lin2.bias is None:
         return None
     w1, b1, w2, b2 = lin1.weight, lin1.bias, lin2.weight, lin2.bias
-    if (x.dim() < 2 or x.shape[-1] != w1.shape[1] or w1.shape[0] != w2.shape[1] or x.numel() == 0 or w1.shape[0] % 4 or w2.shape[0] % 4
+    # (a frozen first layer keeps the expression, which does not keep x: x may be changed in place behind it)
+    if (not w1.requires_grad or x.dim() < 2 or x.shape[-1] != w1.shape[1] or w1.shape[0] != w2.shape[1] or x.numel() == 0 or w1.shape[0] % 4 or w2.shape[0] % 4
             or x.numel() // x.shape[-1] > 65535 * 2048        # (rows of a column sum)
             or not recording(x, w1, b1, w2, b2)):
         return None
@@ -249,21 +250,27 @@ class _SelfAttention(torch.autograd.Function):
         W = torch.empty(dm, 3 * dm, dtype=torch.float32, device=dev)
         Wo = torch.empty(dm, dm, dtype=torch.float32, device=dev)
         b = torch.empty(3 * dm, dtype=torch.float32, device=dev)
-        sigma = torch.empty(H, dtype=torch.float32, device=dev)
-        _layout((qw, kw, vw, qb, kb, vb, None, wo), W, b, Wo, sigma, spread_w, dm, H, dk, min_spread, 0)
+        sigma, spread = torch.empty(2, H, dtype=torch.float32, device=dev)
+        _layout((qw, kw, vw, qb, kb, vb, spread, wo), W, b, Wo, sigma, spread_w, dm, H, dk, min_spread, 0)
         qkv = torch.addmm(b, _dense(x).view(Z * N, dm), W).to(operand_dtype or torch.bfloat16).view(Z, N, 3, H, dk)
         O, L = ga.geo_attn(*_heads(qkv), coords, sigma, mask, return_lse=True, check_sigma=False, token_major_out=True,
                            operand_dtype=operand_dtype)
-        ctx.save_for_backward(x, coords, mask, qw, kw, vw, qb, kb, vb, spread_w, wo, W, Wo, sigma, qkv, O, L)
+        ctx.save_for_backward(x, coords, mask, W, Wo, sigma, spread, qkv, O, L)
+        # The parameters themselves are wanted by the expression only: what a backward reads of them it has as copies, so that they
+        # may be changed (an optimizer's step) between forward and backward.
+        ctx.params = (qw, kw, vw, qb, kb, vb, spread_w, wo)
+        ctx.versions = [p._version for p in ctx.params]
         ctx.min_spread, ctx.operand_dtype = min_spread, operand_dtype
         return torch.ops.aten._unsafe_view(O.permute(0, 2, 1, 3).reshape(Z * N, dm).mm(Wo.t()), (Z, N, dm))      # (not a view, as in the feed-forward)
 
     @staticmethod
     @_without_autocast
     def backward(ctx, d):
-        x, coords, mask, *params, W, Wo, sigma, qkv, O, L = ctx.saved_tensors
-        need = ctx.needs_input_grad
+        x, coords, mask, W, Wo, sigma, spread, qkv, O, L = ctx.saved_tensors
+        need, params = ctx.needs_input_grad, ctx.params
         if _by_expression(d):
+            if any(p._version != v for p, v in zip(params, ctx.versions)):
+                raise RuntimeError("a parameter of the self-attention was changed in place after the forward pass whose gradient is recorded")
             gx, *gp = _recorded(lambda x_, *p: _self_attention_expression(x_, coords, mask, *p, ctx.min_spread, ctx.operand_dtype),
                                 (x, *params), (need[0], *need[3:11]), d)
             return (gx, None, None, *gp, None, None)
@@ -281,7 +288,7 @@ class _SelfAttention(torch.autograd.Function):
         dW = _dense(x).view(Z * N, dm).t().mm(g2) if any(need[3:6]) else g2
         db = column_sums(g2) if any(need[6:9]) else g2
         dWo = d2.t().mm(O.permute(0, 2, 1, 3).reshape(Z * N, dm)) if need[10] else g2
-        _layout(grads, dW, db, dWo, d_sigma, _saved(params[6], (H,)), dm, H, dk, ctx.min_spread, 1)
+        _layout(grads, dW, db, dWo, d_sigma, _saved(spread, (H,)), dm, H, dk, ctx.min_spread, 1)
         return (dx, None, None, *grads, None, None)
 
 
@@ -291,7 +298,8 @@ def self_attention(x, coords, mask, m):
         return None
     H, dk, dm = m.heads, m.d_k, m.d_model
     params = (m.q_proj, m.k_proj, m.v_proj, m.q_bias, m.k_bias, m.v_bias, m.spread_weights, m.out_proj.weight)
-    if (m.legacy_logits or dk not in (32, 64, 128) or dm > 16384 or x.numel() == 0 or not coords.is_cuda or coords.requires_grad or type(coords) not in _PLAIN_TYPES
+    # (frozen projections keep the expression, which does not keep x: x may be changed in place behind it)
+    if (not any(p.requires_grad for p in params[:3]) or m.legacy_logits or dk not in (32, 64, 128) or dm > 16384 or x.numel() == 0 or not coords.is_cuda or coords.requires_grad or type(coords) not in _PLAIN_TYPES
             or (mask is not None and type(mask) is not torch.Tensor)
             or x.shape[1] * 3 * dm * 4 >= 2 ** 31 or m.operand_dtype not in (None, torch.bfloat16)
             or type(m).get_spreads is not ga.GeoAttention.get_spreads or "get_spreads" in m.__dict__

@@ -297,3 +297,33 @@ def test_outputs_may_be_changed_in_place(gpu):
         assert out is not None and not out._is_view()
         out += 1.0
         out.sum().backward()
+
+
+def test_parameters_may_change_between_forward_and_backward(gpu):
+    # the attention's gradients are those of the parameters that the forward pass used
+    layer, _, _, coords = _layer_and_inputs(gpu)
+    x, params = torch.randn(1, 33, 64, device=gpu, requires_grad=True), [p for n, p in layer.attn.named_parameters() if n != "beta_weights"]
+    out = layer.attn(x, x, x, coords)
+    d = torch.randn_like(out)
+    want = torch.autograd.grad(out, [x, *params], d, retain_graph=True)
+    with torch.no_grad():
+        for p in params:
+            p.add_(0.1)
+    for g, w in zip(torch.autograd.grad(out, [x, *params], d, retain_graph=True), want):
+        assert rel(g, w.double().cpu()) <= (1e-4 if w.shape == layer.attn.spread_weights.shape else 6e-6), tuple(w.shape)
+    with pytest.raises(RuntimeError, match="changed in place"):
+        torch.autograd.grad(out, [x], d, create_graph=True)
+
+
+def test_frozen_weights_leave_the_input_free(gpu):
+    # as with torch's products, whose gradient of the input needs the weights alone
+    layer, _, _, coords = _layer_and_inputs(gpu)
+    for p in layer.parameters():
+        p.requires_grad_(False)
+    leaf = torch.randn(1, 33, 64, device=gpu, requires_grad=True)
+    for f in (layer.ffn, lambda t: layer.attn(t, t, t, coords)):
+        x = leaf * 2.0
+        out = f(x)
+        x += out
+        g, = torch.autograd.grad(x.sum(), [leaf])
+        assert torch.isfinite(g).all()
