@@ -62,6 +62,36 @@ __device__ __forceinline__ int wa_terms(const float z, const float tail)
     return n;
 }
 
+// Length of the longest diagonal of the batch items' boxes (infinite if one of them holds a token that is not finite), by one
+// block: as many lanes share an item as have boxes to read.
+__device__ __forceinline__ float wa_extent(const WgBox* __restrict__ boxes, const int Z, const int nbox)
+{
+    const int tid = threadIdx.x;
+    int lanes = 1;
+    while (lanes < 64 && lanes < nbox) lanes *= 2;
+    float longest = 0.f;
+    for (int z = tid / lanes; z - tid / lanes < Z; z += 256 / lanes) {         // (all lanes of a wave meet in the exchanges)
+        float lo[3] = {3.0e38f, 3.0e38f, 3.0e38f}, hi[3] = {-3.0e38f, -3.0e38f, -3.0e38f}, bad = 0.f;
+        if (z < Z)
+            for (int i = tid % lanes; i < nbox; i += lanes) {
+                const WgBox q = boxes[(size_t)z * nbox + i];
+                bad = fmaxf(bad, q.bad);
+                if (!(q.lo[0] <= q.hi[0])) continue;                            // padded tokens only
+#pragma unroll
+                for (int c = 0; c < 3; ++c) { lo[c] = fminf(lo[c], q.lo[c]); hi[c] = fmaxf(hi[c], q.hi[c]); }
+            }
+        for (int o = 1; o < lanes; o *= 2) {
+            bad = fmaxf(bad, __shfl_xor(bad, o));
+#pragma unroll
+            for (int c = 0; c < 3; ++c) { lo[c] = fminf(lo[c], __shfl_xor(lo[c], o)); hi[c] = fmaxf(hi[c], __shfl_xor(hi[c], o)); }
+        }
+        const float dx = hi[0] - lo[0], dy = hi[1] - lo[1], dz = hi[2] - lo[2];
+        if (lo[0] <= hi[0]) longest = fmaxf(longest, __builtin_sqrtf(dx * dx + dy * dy + dz * dz));
+        longest += bad;
+    }
+    return wg_block_max(longest);
+}
+
 __global__ __launch_bounds__(256)
 void we_aniso_grid_tables_kernel(const float* __restrict__ cb_magnitudes, const float* __restrict__ wavenumbers,
                                  char* __restrict__ ws, const int Z, const int N, const int K, const int partials, const int few)
@@ -92,22 +122,14 @@ void we_aniso_grid_tables_kernel(const float* __restrict__ cb_magnitudes, const 
         // The direct kernel or the grids?  Estimated microseconds: the direct kernel takes 0.34 ps per pair and wavenumber with partial
         // derivatives (0.36 to 0.40 where it has few workgroups) and 0.24 without.  A pass over the sources (8 waves, K = 256, 1 x 1000 ... 8 x 2000 tokens, 4 to 12 terms) takes a round
         // of workgroups (two per compute unit) 22 us for its grids and products and 0.059 us per source, down to 0.026 for few workgroups.
-        float pairs = 0.f, nmax = 0.f, groups = 0.f, ext = 0.f;
+        float pairs = 0.f, nmax = 0.f, groups = 0.f;
         for (int i = tid; i < Z; i += 256) {
             const float n = (float)reinterpret_cast<const int*>(ws + L.counts)[i];
             pairs += n * n; nmax = fmaxf(nmax, n); groups += __builtin_ceilf(n / WG_OBS);
         }
-        float far[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};           // extent of the batch, from its first token
-        const float4 at = reinterpret_cast<const float4*>(ws + L.sources)[0];
-        for (int i = tid; i < Z * L.nbox; i += 256) {
-            const WgBox q = reinterpret_cast<const WgBox*>(ws + L.boxes)[i];
-            if (!(q.lo[0] <= q.hi[0])) continue;
-            far[0] = fmaxf(far[0], q.hi[0] - at.x); far[1] = fmaxf(far[1], q.hi[1] - at.y); far[2] = fmaxf(far[2], q.hi[2] - at.z);
-            far[3] = fmaxf(far[3], at.x - q.lo[0]); far[4] = fmaxf(far[4], at.y - q.lo[1]); far[5] = fmaxf(far[5], at.z - q.lo[2]);
-        }
-        for (int c = 0; c < 3; ++c) { const float e = wg_block_max(far[c]) + wg_block_max(far[3 + c]); ext += e * e; }
         pairs = wg_block_sum(pairs); groups = wg_block_sum(groups); nmax = wg_block_max(nmax);
-        const float cells   = 0.7f * __builtin_sqrtf(ext) * (1.0f / WG_UNIT) * inv_h;
+        const float extent  = wa_extent(reinterpret_cast<const WgBox*>(ws + L.boxes), Z, L.nbox) * (1.0f / WG_UNIT);
+        const float cells   = 0.7f * extent * inv_h;
         const float windows = __builtin_ceilf(fmaxf(1.0f, cells / (float)WgGrid<2>::CELLS));
         // (16 waves, 28 batches of 1 x 500 ... 2 x 2000 tokens, K = 128 and 256: a preparation of 37 to 53 us, and per pass 0.0128 us per source,
         // 0.3 ns per cell and wavenumber, half of that without partial derivatives, and 10 us for the flushes of more than 1024 sources.)

@@ -190,3 +190,57 @@ def test_weights_that_fall_below_half_a_unit(gpu):
     # the bar of the anisotropic grids, row by row: one pair's cell that is off by 2^31 units changes a row by 100 times its norm
     err = np.linalg.norm(got - ref, axis=-1) / np.linalg.norm(ref, axis=-1)
     assert err.max() <= 4 * (2e-6 + 2 * 2.0 ** -24 * float(wn.max()) * 6.0), err.max()
+
+
+def run_aniso_route(gpu, a, b, cb, wn, mask=None, partials=True):
+    """The results, and the terms of the expansion that the device chose (0: the direct kernel did the work)."""
+    lib = _lib.load()
+    Z, N, K = a.shape[0], a.shape[1], wn.numel()
+    a, b, cb, w = a.to(gpu), b.to(gpu), cb.to(gpu), wn.to(gpu)
+    m = None if mask is None else mask.to(gpu).view(torch.uint8)
+    bufs = [torch.full((Z, N, 2 * K), float("nan"), device=gpu) for _ in range(3 if partials else 1)]
+    nbytes = lib.proteus_we_aniso_fwd_workspace_bytes(Z, N, K, int(partials), int(mask is not None), 0)
+    assert nbytes > 0
+    ws = torch.full((nbytes,), 0xA5, dtype=torch.uint8, device=gpu)
+    rc = lib.proteus_we_aniso_fwd_ws(a.data_ptr(), b.data_ptr(), _lib.COORDS_AOS, cb.data_ptr(), w.data_ptr(), None if m is None else m.data_ptr(),
+                                     bufs[0].data_ptr(), *([t.data_ptr() for t in bufs[1:]] if partials else [None, None]),
+                                     ws.data_ptr(), nbytes, Z, N, K, 0, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, lib.proteus_strerror(rc)
+    return [t.cpu().numpy() for t in bufs], int(ws[16:20].view(torch.int32).item())
+
+
+ROUTES = {                      # N, Z, K, scale of the chain, spread of the C-beta scales, partial derivatives, kind, through grids?
+    "items in frames of their own": (2000, 2, 256, 1.0, 0.02, True, "frames", True),
+    "the first item empty": (2000, 3, 256, 1.0, 0.02, True, "first empty", True),
+}
+
+
+@pytest.mark.parametrize("name", ROUTES)
+def test_anisotropic_grids_where_they_pay(gpu, name):
+    N, Z, K, scale, spread, partials, kind, grids = ROUTES[name]
+    a, _ = synth.we_inputs(N, seed=N + K, batch=Z)
+    a = a * scale
+    g = torch.Generator().manual_seed(K + N)
+    b = torch.randn(Z, N, 3, generator=g)
+    b = 1.5 * b / b.norm(dim=-1, keepdim=True)
+    cb, wn = 1.0 + spread * torch.randn(K, generator=g), synth.wavenumbers(2 * K)
+    mask = None
+    if kind == "frames":
+        a[1] += torch.tensor([8192.0, -4096.0, 4096.0])
+    elif kind == "first empty":
+        mask = (torch.arange(Z) == 0)[:, None].expand(Z, N)
+    elif kind == "scattered":
+        mask = torch.rand(Z, N, generator=g) < 0.2
+    elif kind == "nan":
+        a[1, 77, 1] = float("nan")
+    got, terms = run_aniso_route(gpu, a, b, cb, wn, mask, partials)
+    assert (terms > 0) == grids, terms
+    if kind == "nan":           # an unpadded token at NaN makes every sum of its batch item NaN and touches no other item
+        assert np.isnan(got[0][1]).all()
+        a, b, got = a[:1], b[:1], [x[:1] for x in got]
+    rows = np.unique(np.concatenate([np.arange(0, N, 41), [15, 16, N - 1]])).astype(np.int32)
+    ref = c_oracle.we_aniso(a.numpy(), b.numpy(), cb.numpy(), wn.numpy(), None if mask is None else mask.numpy(), rows=rows)
+    far = float((a.amax(1) - a.amin(1)).norm(dim=-1).max())         # the bar of the tests above
+    bar = 2e-6 + 2 * 2.0 ** -24 * float(wn.abs().max()) * far
+    for x, r in zip(got, ref):
+        assert np.isfinite(x).all() and rel_l2(x[:, rows], r) <= bar, (name, rel_l2(x[:, rows], r), bar)
