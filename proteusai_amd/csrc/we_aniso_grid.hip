@@ -14,8 +14,8 @@
 // Per pair of tokens and pair of terms: about 40 vector instructions and twelve integer LDS additions, against 10 instructions per
 // wavenumber in the direct kernel.
 // Pairs that no cell takes (r - c A below h/2, or r so small against r - c A that the weight leaves its fixed-point range) are summed
-// directly, as are all pairs of a workgroup whose distances need too many windows.  Where the expansion needs so many terms that the
-// direct kernel is the faster one, which only the device can tell, that kernel does the work and this one returns at once.
+// directly.  Where the expansion needs so many terms, or the distances so many windows of the grids, that the direct kernel is the faster
+// one, and where something is not finite, which only the device can tell, that kernel does the work and this one returns at once.
 #include "we_grid.h"
 #include "we_aniso_direct.h"
 
@@ -118,7 +118,7 @@ void we_aniso_grid_tables_kernel(const float* __restrict__ cb_magnitudes, const 
         terms = wa_terms(z, 3.0e-7f) + partials;
         if (terms > WG_MAX_TERMS) terms = 0;
     }
-    if (terms > 1) {
+    if (terms > 0) {
         // The direct kernel or the grids?  Estimated microseconds: the direct kernel takes 0.34 ps per pair and wavenumber with partial
         // derivatives (0.36 to 0.40 where it has few workgroups) and 0.24 without.  A pass over the sources (8 waves, K = 256, 1 x 1000 ... 8 x 2000 tokens, 4 to 12 terms) takes a round
         // of workgroups (two per compute unit) 22 us for its grids and products and 0.059 us per source, down to 0.026 for few workgroups.
@@ -128,17 +128,28 @@ void we_aniso_grid_tables_kernel(const float* __restrict__ cb_magnitudes, const 
             pairs += n * n; nmax = fmaxf(nmax, n); groups += __builtin_ceilf(n / WG_OBS);
         }
         pairs = wg_block_sum(pairs); groups = wg_block_sum(groups); nmax = wg_block_max(nmax);
-        const float extent  = wa_extent(reinterpret_cast<const WgBox*>(ws + L.boxes), Z, L.nbox) * (1.0f / WG_UNIT);
+        const float extent = wa_extent(reinterpret_cast<const WgBox*>(ws + L.boxes), Z, L.nbox) * (1.0f / WG_UNIT);
+        const bool  one     = terms == 1;                                // (a single grid: no partial derivatives)
+        const int   most    = one ? WgGrid<1>::CELLS : WgGrid<2>::CELLS;
         const float cells   = 0.7f * extent * inv_h;
-        const float windows = __builtin_ceilf(fmaxf(1.0f, cells / (float)WgGrid<2>::CELLS));
+        const float windows = __builtin_ceilf(fmaxf(1.0f, cells / (float)most));
+        const float rounds  = groups * (1.0f / 512.0f), share = fminf(1.0f, rounds);
         // (16 waves, 28 batches of 1 x 500 ... 2 x 2000 tokens, K = 128 and 256: a preparation of 37 to 53 us, and per pass 0.0128 us per source,
         // 0.3 ns per cell and wavenumber, half of that without partial derivatives, and 10 us for the flushes of more than 1024 sources.)
         const float passes  = (float)((terms + 1) / 2) * windows;
-        const float grid    = few ? (partials ? 53.0f : 37.0f) + passes * (0.0128f * nmax + (partials ? 3.0e-4f : 1.4e-4f) * (float)K * cells / windows
-                                                                          + (nmax > (float)WA_FLUSH ? 10.0f : 0.0f))
-                                  : passes * (22.0f + (0.026f + 0.033f * fminf(1.0f, groups / 512.0f)) * nmax) * fmaxf(1.0f, groups / 512.0f);
-        const float direct  = pairs * (float)K * (partials ? (few ? 3.7e-7f : 3.4e-7f) : 2.4e-7f);
-        if (!(grid < direct)) terms = 0;
+        float grid   = few ? (partials ? 53.0f : 37.0f) + passes * (0.0128f * nmax + (partials ? 3.0e-4f : 1.4e-4f) * (float)K * cells / windows
+                                                                    + (nmax > (float)WA_FLUSH ? 10.0f : 0.0f))
+                           : passes * (22.0f + (0.026f + 0.033f * share) * nmax) * fmaxf(1.0f, rounds);
+        float direct = pairs * (float)K * (partials ? (few ? 3.7e-7f : 3.4e-7f) : 2.4e-7f);
+        if (one) {
+            // A single grid, 60 batches of 1 x 1000 ... 32 x 500 tokens, K = 64 to 256, extents of up to 16 windows.  Grids / direct, us:
+            // 1 x 2000 K = 64 1 window 45 / 172, 4 116 / 180, 7 212 / 179, 13 402 / 179; 1 x 4000 K = 64 5 234 / 350, 9 430 / 353; 1 x 4000 K = 256
+            // 10 598 / 1074; 8 x 1000 K = 256 6 387 / 527, 11 742 / 529.  The direct kernel takes 0.086 us per source where its workgroups do not fill the chip.
+            grid   = 12.0f + windows * (few ? 10.0f + 0.008f * nmax + 0.05f * (float)K
+                                            : (6.0f + (0.5f + 0.5f * share) * (0.0118f * nmax + 0.18f * (float)K)) * fmaxf(1.0f, rounds));
+            direct = fmaxf(direct, 0.086f * nmax);
+        }
+        if (!(grid < direct) || !(cells + fabsf(mid) * b * inv_h < (float)(most * WG_MAX_WINDOWS))) terms = 0;
     }
     const int unit = (int)blockIdx.x * 4 + (tid >> 6);
     if (unit == 0 && lane == 0) {
@@ -190,11 +201,12 @@ __device__ __forceinline__ Place wa_place(const float dx, const float dy, const 
     return p;
 }
 
+// The pairs of one observer that have no cell, summed directly by one wave, a lane per wavenumber.
 template <bool GRADS>
-__device__ void wa_direct(const float4* __restrict__ src, const float4* __restrict__ srcb, const int n, const float xi, const float yi, const float zi,
-                          const float mid, const float inv_h, const float climit, const bool all,
-                          const float* __restrict__ cb_magnitudes, const float* __restrict__ wavenumbers,
-                          float* __restrict__ o, float* __restrict__ ob, float* __restrict__ ok, const int K, const int lane)
+__device__ void wa_near(const float4* __restrict__ src, const float4* __restrict__ srcb, const int n, const float xi, const float yi, const float zi,
+                        const float mid, const float inv_h, const float climit,
+                        const float* __restrict__ cb_magnitudes, const float* __restrict__ wavenumbers,
+                        float* __restrict__ o, float* __restrict__ ob, float* __restrict__ ok, const int K, const int lane)
 {
     for (int kb = 0; kb < K; kb += 128) {
         float kr[2], cb[2], s[2][GRADS ? 6 : 2];
@@ -211,7 +223,7 @@ __device__ void wa_direct(const float4* __restrict__ src, const float4* __restri
             float r2;
             const Place p = wa_place(xi - q.x, yi - q.y, zi - q.z, srcb[j0 + lane], mid * WG_UNIT, inv_h, WG_MAGIC, 0xff800000u, r2);
             const bool near = !(p.u > WG_MAGIC) || p.c > climit;
-            uint64_t todo = __builtin_amdgcn_ballot_w64(j0 + lane < n && r2 != 0.0f && (all || near));
+            uint64_t todo = __builtin_amdgcn_ballot_w64(j0 + lane < n && r2 != 0.0f && near);
             const float r = p.r * (1.0f / WG_UNIT), m = p.inv * WG_UNIT;
             while (todo) {
                 const int b = __builtin_ctzll(todo);
@@ -236,8 +248,7 @@ __device__ void wa_direct(const float4* __restrict__ src, const float4* __restri
             const int k = kb + 64 * u + lane;
             if (k >= K) continue;
             auto put = [&](float* to, float re, float im) {
-                if (!all) { re += to[2 * k]; im += to[2 * k + 1]; }
-                to[2 * k] = re; to[2 * k + 1] = im;
+                to[2 * k] += re; to[2 * k + 1] += im;
             };
             put(o, s[u][0], s[u][1]);
             if constexpr (GRADS) {
@@ -463,28 +474,19 @@ void we_aniso_grid_kernel(const char* __restrict__ ws, const float* __restrict__
         return;
     }
 
-    const float reach = (wg_reach<WAVES>(me, ok, reinterpret_cast<const WgBox*>(ws + L.boxes) + (size_t)z * L.nbox, L.nbox, s_red)
-                         + fabsf(mid_cb) * params->b_max * WG_UNIT) * inv_h + 2.0f;
-    const bool one    = !GRADS && terms == 1;
-    const bool direct = __builtin_amdgcn_readfirstlane(!(reach < (float)((one ? WgGrid<1>::CELLS : WgGrid<2>::CELLS) * WG_MAX_WINDOWS))) != 0;
-    const int  ncell  = __builtin_amdgcn_readfirstlane(direct ? 0 : (int)reach);
-    if (!direct) {
-        if (!GRADS && one) wa_grids<GRADS, 1, WAVES>(s_grid, s_near, s_tok, ws, L, cb_magnitudes, wavenumbers, out, d_cb, d_k, src, srcb, me, ok, n, slot0, ncell, zN, K);
-        else               wa_grids<GRADS, 2, WAVES>(s_grid, s_near, s_tok, ws, L, cb_magnitudes, wavenumbers, out, d_cb, d_k, src, srcb, me, ok, n, slot0, ncell, zN, K);
-    }
+    // (The tables' launch has seen to it that 0.7 of an item's extent, and b, stay within WG_MAX_WINDOWS windows; the far corner and
+    // the observers' own radius are at most twice that.)
+    const int ncell = __builtin_amdgcn_readfirstlane((int)((wg_reach<WAVES>(me, ok, reinterpret_cast<const WgBox*>(ws + L.boxes) + (size_t)z * L.nbox, L.nbox, s_red)
+                                                            + fabsf(mid_cb) * params->b_max * WG_UNIT) * inv_h + 2.0f));
+    if (!GRADS && terms == 1) wa_grids<GRADS, 1, WAVES>(s_grid, s_near, s_tok, ws, L, cb_magnitudes, wavenumbers, out, d_cb, d_k, src, srcb, me, ok, n, slot0, ncell, zN, K);
+    else                      wa_grids<GRADS, 2, WAVES>(s_grid, s_near, s_tok, ws, L, cb_magnitudes, wavenumbers, out, d_cb, d_k, src, srcb, me, ok, n, slot0, ncell, zN, K);
 
     __syncthreads();
     for (int q = wave; q < WG_OBS; q += WAVES) {
-        const int t = s_tok[q];
-        if (t < 0) continue;
-        const size_t row = (zN + t) * 2 * K;
-        if (slot0 + q >= n) {
-            if (direct) for (int k = lane; k < 2 * K; k += 64) { out[row + k] = 0.f; if (GRADS) { d_cb[row + k] = 0.f; d_k[row + k] = 0.f; } }
-            continue;
-        }
-        if (!direct && !s_near[q]) continue;
-        wa_direct<GRADS>(src, srcb, n, wg_lane(me.x, q), wg_lane(me.y, q), wg_lane(me.z, q), mid_cb, inv_h, 2.0f * inv_h, direct,
-                         cb_magnitudes, wavenumbers, out + row, GRADS ? d_cb + row : nullptr, GRADS ? d_k + row : nullptr, K, lane);
+        if (slot0 + q >= n || !s_near[q]) continue;
+        const size_t row = (zN + s_tok[q]) * 2 * K;
+        wa_near<GRADS>(src, srcb, n, wg_lane(me.x, q), wg_lane(me.y, q), wg_lane(me.z, q), mid_cb, inv_h, 2.0f * inv_h,
+                       cb_magnitudes, wavenumbers, out + row, GRADS ? d_cb + row : nullptr, GRADS ? d_k + row : nullptr, K, lane);
     }
 }
 

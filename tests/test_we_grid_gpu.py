@@ -210,8 +210,14 @@ def run_aniso_route(gpu, a, b, cb, wn, mask=None, partials=True):
 
 
 ROUTES = {                      # N, Z, K, scale of the chain, spread of the C-beta scales, partial derivatives, kind, through grids?
+    "one grid in several windows": (2000, 1, 64, 10.0, 0.0, False, None, True),
+    "one grid in more windows than pay": (2000, 1, 64, 40.0, 0.0, False, None, False),
+    "one grid in more windows than pay, more than 256 workgroups": (1000, 8, 64, 40.0, 0.0, False, None, False),
+    "more windows than there are": (1000, 1, 256, 3000.0, 0.0, False, None, False),
     "items in frames of their own": (2000, 2, 256, 1.0, 0.02, True, "frames", True),
     "the first item empty": (2000, 3, 256, 1.0, 0.02, True, "first empty", True),
+    "a token that is not finite": (1000, 2, 256, 1.0, 0.0, False, "nan", False),
+    "more items than lanes of a block share": (300, 40, 256, 1.0, 0.0, False, "scattered", True),
 }
 
 
