@@ -126,7 +126,7 @@ __device__ __forceinline__ void wg_direct(uint32_t* s_grid, const int* s_tok, co
 #pragma unroll 1
     for (int tile = 0; tile < tiles; tile += kw) {
         const int kl = (first + (tile + kg) * step) * KT + obs;
-        const float krl = (float)((kl < K ? (double)wavenumbers[kl] : 0.0) * 0.15915494309189533577) * (1.0f / WG_UNIT);
+        const float krl = (float)((kl < K ? (double)wavenumbers[kl] : 0.0) * 0.15915494309189533577);
         float kr[KT], acc[V][KT];
 #pragma unroll
         for (int t = 0; t < KT; ++t) {
@@ -140,7 +140,8 @@ __device__ __forceinline__ void wg_direct(uint32_t* s_grid, const int* s_tok, co
             const float4 p = q;
             q = src[j0 + sw * 4 + row];
             float r2, inv, r;
-            wg_distance(me.x - p.x, me.y - p.y, me.z - p.z, r2, inv, r);
+            // (in units of length: the square of a scaled distance overflows from 4.5e15 on)
+            wg_distance((me.x - p.x) * (1.0f / WG_UNIT), (me.y - p.y) * (1.0f / WG_UNIT), (me.z - p.z) * (1.0f / WG_UNIT), r2, inv, r);
             const bool use = j0 + row < n && r2 != 0.0f;
             inv = use ? inv : 0.f; r = use ? r : 0.f;
             const float one = use ? 1.f : 0.f;
@@ -180,7 +181,7 @@ __device__ __forceinline__ void wg_direct(uint32_t* s_grid, const int* s_tok, co
             if (tok >= 0 && k < K) {
                 const bool keep = slot0 + e / KT < n;
                 const size_t at = (zN + tok) * K + k;
-                reinterpret_cast<float2*>(out)[at] = keep ? make_float2(v[0] * WG_UNIT, v[1] * WG_UNIT) : make_float2(0.f, 0.f);
+                reinterpret_cast<float2*>(out)[at] = keep ? make_float2(v[0], v[1]) : make_float2(0.f, 0.f);
                 if constexpr (SUMS) { cos_sums[at] = keep ? v[2] : 0.f; sin_sums[at] = keep ? v[3] : 0.f; }
             }
         }

@@ -108,6 +108,19 @@ def test_values_that_are_not_finite_come_through(gpu):
     assert np.isnan(run_grid(gpu, coords[:1], bad)[0][:, :, 6:8]).all()
 
 
+def test_distances_whose_scaled_squares_overflow(gpu):
+    # a token 1e17 away (its square fits in fp32, that of 4096 times it does not) adds next to nothing, as in the direct kernels
+    coords, wn = synth.we_inputs(200, seed=5, batch=2, d_model=128)
+    near = coords[1:].clone()
+    coords[1, 77, 1] = 1e17
+    got = run_grid(gpu, coords, wn)
+    keep = np.arange(200) != 77
+    ref = c_oracle.we(near[:, keep].numpy(), wn.numpy(), precision="f64")[0]
+    assert all(np.isfinite(a).all() for a in got) and np.abs(got[0][1, 77]).max() <= 200 * 1.001e-17
+    # the bar of the values that are not finite: single-precision phases of a short chain
+    assert rel_l2(got[0][1:, keep], ref) <= 1e-5
+
+
 def run_aniso(gpu, a, b, cb, wn, mask=None, partials=True):
     lib = _lib.load()
     Z, N, K = a.shape[0], a.shape[1], wn.numel()
