@@ -21,7 +21,7 @@
 //     the waves of a workgroup share the grids and the result is the same from run to run.  A cell's octave e = floor(log2 n)
 //     sets its scale: what is added is phi 2^e h / r < 2, so near and far sources keep the same relative precision (the
 //     rounding of one addition is 2^-22 of the largest term); octaves have their own rows where they overlap.  After
-//     1024 sources (what 32 bits hold at that scale) the integers are moved on to float accumulators.
+//     2048 sources (what 32 bits hold at that scale) the integers are moved on to float accumulators.
 //   - Pairs closer than h/2 (never the case for real structures) are summed directly, as are all pairs of a workgroup
 //     whose distances would need too many windows of the grid or are not finite.
 #include "we_grid.h"
@@ -409,8 +409,10 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
 }  // namespace
 
 // The grid pays from about 6e7 (pair, wavenumber) units on, below which two launches and the latency of one workgroup's
-// phases are what a call costs (measured, grid against direct kernel: 1 x 512 and K = 256 27 / 26 us, 16 x 128 and K = 256
-// 20 / 23 us, 1 x 128 17.6 / 8.2 us, 1 x 256 and K = 64 14.7 / 11.4 us, 32 x 64 and K = 64 12.2 / 7.9 us), and from 64 wavenumbers on.
+// phases are what a call costs, and from 64 wavenumbers on.  Measured, us, grid / direct kernel, with the sums and without: at 6.7e7 units
+// 1 x 512 and K = 256 24.2 / 29.9 and 19.0 / 25.6, 16 x 128 and K = 256 21.3 / 26.8 and 17.0 / 22.1, 1 x 1000 and K = 64 23.3 / 36.6 and 21.1 / 31.6;
+// at 3.4e7 4 x 256 and K = 128 18.2 / 18.0 and 15.2 / 15.4, 32 x 64 and K = 256 18.7 / 18.1 and 15.4 / 15.0, 1 x 512 and K = 128 19.2 / 21.2 and
+// 17.1 / 18.3; 1 x 256 and K = 256 (1.7e7) 19.7 / 12.9 and 15.6 / 11.3.
 static bool we_grid_wanted(int Z, int N, int K, int tuning)
 {
     return tuning == 0 && K >= 64 && (double)Z * N * N * K >= 6.0e7;

@@ -447,3 +447,22 @@ def test_other_source_weights(gpu, mag_type, N, Z, K):
                                         torch.from_numpy(ref[1]), torch.from_numpy(ref[2]))
     if rows is None:
         assert rel_l2(w.grad.cpu().numpy(), dk.numpy()) <= REL_L2_TOL
+
+
+@pytest.mark.parametrize("N,K,lens", [(520, 64, None), (1024, 256, [1024, 130, 777, 512])])      # byte-wise scan of the mask; several rows of the snake
+def test_ranked_direct_kernel_against_the_oracle(gpu, N, K, lens):
+    # the kernel without a workspace (the operator takes the grids at these sizes), into buffers full of NaN
+    g = torch.Generator().manual_seed(N)
+    lens = torch.randint(1, N + 1, (5,), generator=g) if lens is None else torch.tensor(lens)
+    mask = torch.arange(N)[None, :] >= lens[:, None]
+    Z = len(lens)
+    coords, _ = synth.we_inputs(N, seed=N, batch=Z)
+    wn = synth.wavenumbers(2 * K)
+    c, w, m = coords.to(gpu), wn.to(gpu), mask.to(gpu).view(torch.uint8)
+    bufs = [torch.full(s, float("nan"), device=gpu) for s in ((Z, N, 2 * K), (Z, N, K), (Z, N, K))]
+    rc = _lib.load().proteus_we_fwd(c.data_ptr(), _lib.COORDS_AOS, w.data_ptr(), m.data_ptr(), *[b.data_ptr() for b in bufs], Z, N, K, 0,
+                                    torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    got = [b.cpu().numpy() for b in bufs]
+    assert all((a[mask.numpy()] == 0).all() for a in got)
+    check(got, coords, wn, mask)

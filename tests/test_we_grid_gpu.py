@@ -1,5 +1,5 @@
 """The embedding forward through distance grids (proteus_we_fwd_ws with a workspace) against the float64 oracle, at the
-sizes where it can go wrong: tiles of 16 observers, flushes after 1024 sources, octave and window borders of the grid,
+sizes where it can go wrong: tiles of 16 observers, flushes after 2048 sources, octave and window borders of the grid,
 pairs closer than half a cell, coordinates that are not finite."""
 import numpy as np
 import pytest
@@ -37,15 +37,21 @@ CASES = {                       # N, Z, K, scale of the chain, mask
     "one tile": (16, 1, 16, 1.0, None),
     "tile and a bit, odd K": (17, 3, 37, 1.0, None),
     "two tokens": (2, 2, 5, 1.0, None),
-    "one flush exactly": (1024, 1, 64, 1.0, None),
-    "one source more than a flush": (1025, 1, 64, 1.0, None),
-    "flushes, scattered mask": (2100, 2, 20, 1.0, "scattered"),
+    "half a flush": (1024, 1, 64, 1.0, None),
+    "half a flush and a source": (1025, 1, 64, 1.0, None),
+    "as many sources as need no flush": (2048, 1, 64, 1.0, None),
+    "flushes, one source": (2049, 1, 64, 1.0, None),
+    "scattered mask, more than 256 workgroups": (2100, 2, 20, 1.0, "scattered"),
+    "flushes, scattered mask": (3600, 1, 20, 1.0, "scattered"),
+    "flushes, more than 256 workgroups, an odd number of tiles": (3600, 2, 37, 1.0, "scattered"),
     "tail masks, empty item, lone survivor": (333, 4, 48, 1.0, "tail"),
     "large K": (70, 1, 300, 1.0, None),
     "many pairs closer than half a cell": (200, 1, 64, 0.05, None),
     "all pairs closer than half a cell": (60, 2, 40, 0.005, None),
     "several windows of the grid": (700, 2, 33, 30.0, None),
-    "several windows and flushes": (1500, 1, 16, 20.0, "scattered"),
+    "several windows, scattered mask": (1500, 1, 16, 20.0, "scattered"),
+    "flushes, windows": (3600, 1, 64, 5.0, None),
+    "flushes, windows, more than 256 workgroups": (2500, 2, 64, 5.0, None),
     "beyond the windows": (90, 1, 33, 3000.0, None),
     # sums without the grid: tiles of wavenumbers shared out over workgroups and over the waves of one
     "beyond the windows, 250 wavenumbers, an empty item": (333, 4, 250, 900.0, "tail"),
@@ -83,6 +89,10 @@ def test_grid_matches_the_oracle(gpu, name):
     c = coords if mask is None else coords.masked_fill(mask[..., None], 0.0)
     far = float((c.amax(1) - c.amin(1)).norm(dim=-1).max())
     bar = 1.7e-6 + 2 * 2.0 ** -24 * float(wn.abs().max()) * far
+    sources = N if mask is None else int((~mask).sum(1).max())
+    assert ("flushes" in name) == (sources > 2048), sources
+    if "flushes, windows" in name:        # 1117 cells of pi / (3.5 k_max) are a window; up to five, which cost less than the pairs
+        assert 1117 < 0.5 * far * float(wn.abs().max()) * 3.5 / np.pi and far * float(wn.abs().max()) * 3.5 / np.pi < 5 * 1117, far
     for a, r, what in zip(got, ref, ("out", "cos_sums", "sin_sums")):
         assert np.isfinite(a).all(), f"{name}: {what}"
         if mask is not None:
@@ -139,7 +149,8 @@ def run_aniso(gpu, a, b, cb, wn, mask=None, partials=True):
 
 ANISO = {                       # N, Z, K, scale of the chain, spread of the C-beta scales around 1, mask
     "equal scales": (700, 1, 64, 1.0, 0.0, None),
-    "equal scales, flushes, scattered mask": (2100, 2, 20, 1.0, 0.0, "scattered"),
+    "equal scales, scattered mask": (2100, 2, 20, 1.0, 0.0, "scattered"),
+    "equal scales, flushes, scattered mask": (3600, 1, 20, 1.0, 0.0, "scattered"),
     "equal scales, several windows": (300, 2, 20, 60.0, 0.0, None),
     "four terms, an empty item, a lone survivor": (1100, 4, 256, 1.0, 0.01, "tail"),
     "ten terms and flushes": (2100, 2, 256, 1.0, 0.2, None),
@@ -182,6 +193,8 @@ def test_anisotropic_grids_match_the_oracle(gpu, name):
         if mask is not None:
             assert (x[mask.numpy()] == 0).all(), f"{name}: {what} of padded rows"
         assert rel_l2(x[:, sel], r) <= bar, f"{name}: {what} {rel_l2(x[:, sel], r):.3e} (bar {bar:.1e})"
+    if "equal scales, flushes" in name:                     # (a single grid is flushed after 2048 sources, two after 1024)
+        assert int((~mask).sum(1).max()) > 2048
     again = run_aniso(gpu, a, b, cb, wn, mask)
     assert all(np.array_equal(x, y) for x, y in zip(got, again))
     lean = run_aniso(gpu, a, b, cb, wn, mask, partials=False)[0]
