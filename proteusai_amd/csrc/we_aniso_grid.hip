@@ -62,8 +62,8 @@ __device__ __forceinline__ int wa_terms(const float z, const float tail)
     return n;
 }
 
-// Length of the longest diagonal of the batch items' boxes (infinite if one of them holds a token that is not finite), by one
-// block: as many lanes share an item as have boxes to read.
+// Length of the longest diagonal of a thread's share of the batch items' boxes (infinite if one of them holds a token that is not
+// finite), for the 256 threads of a block: as many lanes share an item as have boxes to read.
 __device__ __forceinline__ float wa_extent(const WgBox* __restrict__ boxes, const int Z, const int nbox)
 {
     const int tid = threadIdx.x;
@@ -89,7 +89,7 @@ __device__ __forceinline__ float wa_extent(const WgBox* __restrict__ boxes, cons
         if (lo[0] <= hi[0]) longest = fmaxf(longest, __builtin_sqrtf(dx * dx + dy * dy + dz * dz));
         longest += bad;
     }
-    return wg_block_max(longest);
+    return longest;
 }
 
 __global__ __launch_bounds__(256)
@@ -105,9 +105,9 @@ void we_aniso_grid_tables_kernel(const float* __restrict__ cb_magnitudes, const 
     for (int i = tid; i < Z * L.blocks; i += 256) b2 = fmaxf(b2, reinterpret_cast<const float*>(ws + L.lengths)[i]);
     bool bad = false;
     for (int k = tid; k < K; k += 256) { const float c = cb_magnitudes[k]; bad |= !(fabsf(c) < 1.0e18f); hi = fmaxf(hi, c); lo = fmaxf(lo, -c); }
-    b2 = wg_block_max(bad ? __builtin_inff() : b2);
-    hi = wg_block_max(hi); lo = wg_block_max(lo);
-    const float mid = 0.5f * (hi - lo), b = __builtin_sqrtf(b2) * 1.0001f;
+    float most_of[3] = {bad ? __builtin_inff() : b2, hi, lo};
+    wg_block_reduce<0>(most_of);
+    const float mid = 0.5f * (most_of[1] - most_of[2]), b = __builtin_sqrtf(most_of[0]) * 1.0001f;
     float z = 0.f;
     for (int k = tid; k < K; k += 256) z = fmaxf(z, fabsf(wavenumbers[k] * (cb_magnitudes[k] - mid)));
     z = wg_block_max(z) * b;
@@ -118,7 +118,8 @@ void we_aniso_grid_tables_kernel(const float* __restrict__ cb_magnitudes, const 
         terms = wa_terms(z, 3.0e-7f) + partials;
         if (terms > WG_MAX_TERMS) terms = 0;
     }
-    if (terms > 0) {
+    // (The first block's answer is the one that counts: the others only fill tables.)
+    if (terms > 0 && blockIdx.x == 0) {
         // The direct kernel or the grids?  Estimated microseconds: the direct kernel takes 0.34 ps per pair and wavenumber with partial
         // derivatives (0.36 to 0.40 where it has few workgroups) and 0.24 without.  A pass over the sources (8 waves, K = 256, 1 x 1000 ... 8 x 2000 tokens, 4 to 12 terms) takes a round
         // of workgroups (two per compute unit) 22 us for its grids and products and 0.059 us per source, down to 0.026 for few workgroups.
@@ -127,8 +128,10 @@ void we_aniso_grid_tables_kernel(const float* __restrict__ cb_magnitudes, const 
             const float n = (float)reinterpret_cast<const int*>(ws + L.counts)[i];
             pairs += n * n; nmax = fmaxf(nmax, n); groups += __builtin_ceilf(n / WG_OBS);
         }
-        pairs = wg_block_sum(pairs); groups = wg_block_sum(groups); nmax = wg_block_max(nmax);
-        const float extent = wa_extent(reinterpret_cast<const WgBox*>(ws + L.boxes), Z, L.nbox) * (1.0f / WG_UNIT);
+        float all[4] = {pairs, groups, nmax, wa_extent(reinterpret_cast<const WgBox*>(ws + L.boxes), Z, L.nbox)};
+        wg_block_reduce<2>(all);
+        pairs = all[0]; groups = all[1]; nmax = all[2];
+        const float extent = all[3] * (1.0f / WG_UNIT);
         const bool  one     = terms == 1;                                // (a single grid: no partial derivatives)
         const int   most    = one ? WgGrid<1>::CELLS : WgGrid<2>::CELLS;
         const float cells   = 0.7f * extent * inv_h;

@@ -151,14 +151,24 @@ __device__ __forceinline__ float wg_block_max(float v)
     return fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
 }
 
-__device__ __forceinline__ float wg_block_sum(float v)
+// Several at once: sums of the first SUMS values, largest of the others.  (Its LDS is not guarded against a second call in one kernel.)
+template <int SUMS, int COUNT>
+__device__ __forceinline__ void wg_block_reduce(float (&v)[COUNT])
 {
-    __shared__ float s_sum[4];
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    __shared__ float s_red[COUNT][4];
+    const float inf = __builtin_inff();
+#pragma unroll
+    for (int i = 0; i < COUNT; ++i) {
+        if (i >= SUMS) v[i] = v[i] < 3.0e38f ? v[i] : inf;
+        for (int o = 32; o > 0; o >>= 1) { const float w = __shfl_xor(v[i], o); v[i] = i < SUMS ? v[i] + w : fmaxf(v[i], w); }
+        if ((threadIdx.x & 63) == 0) s_red[i][threadIdx.x >> 6] = v[i];
+    }
     __syncthreads();
-    if ((threadIdx.x & 63) == 0) s_sum[threadIdx.x >> 6] = v;
-    __syncthreads();
-    return s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
+#pragma unroll
+    for (int i = 0; i < COUNT; ++i) {
+        const float x = s_red[i][0], y = s_red[i][1], z = s_red[i][2], w = s_red[i][3];
+        v[i] = i < SUMS ? x + y + z + w : fmaxf(fmaxf(x, y), fmaxf(z, w));
+    }
 }
 
 // Cells per unit of length, rounded to float once: h is its exact inverse from here on.  Wavenumbers beyond any use (wavelengths
