@@ -161,7 +161,7 @@ def add_layer_norm(x, res, norm):
     if not torch.is_grad_enabled():
         return None
     w, b = norm.weight, norm.bias
-    if (w is None or b is None or not plain_module(norm, nn.LayerNorm) or x.shape != res.shape or x.dim() < 1 or w.dim() != 1
+    if (w is None or b is None or not plain_module(norm, nn.LayerNorm) or x.shape != res.shape or x.dim() < 1 or w.dim() != 1 or b.shape != w.shape
             or w.numel() != x.shape[-1] or x.numel() == 0 or w.numel() % 4 or w.numel() > 2048 or not norm.eps >= 0.0
             or not recording(x, res, w, b) or not aligned(w, b)):
         return None
@@ -298,6 +298,10 @@ def self_attention(x, coords, mask, m):
         return None
     H, dk, dm = m.heads, m.d_k, m.d_model
     params = (m.q_proj, m.k_proj, m.v_proj, m.q_bias, m.k_bias, m.v_bias, m.spread_weights, m.out_proj.weight)
+    # (whatever does not have the shape it was constructed with is the expression's to judge)
+    if not (params[0].shape == params[1].shape == params[2].shape == (H, dm, dk) and params[3].shape == params[4].shape == params[5].shape == (H, dk)
+            and params[6].shape == (H,) and params[7].shape == (dm, dm)):
+        return None
     # (frozen projections keep the expression, which does not keep x: x may be changed in place behind it)
     if (not any(p.requires_grad for p in params[:3]) or m.legacy_logits or dk not in (32, 64, 128) or dm > 16384 or x.numel() == 0 or not coords.is_cuda or coords.requires_grad or type(coords) not in _PLAIN_TYPES
             or (mask is not None and type(mask) is not torch.Tensor)

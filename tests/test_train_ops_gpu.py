@@ -327,3 +327,15 @@ def test_frozen_weights_leave_the_input_free(gpu):
         x += out
         g, = torch.autograd.grad(x.sum(), [leaf])
         assert torch.isfinite(g).all()
+
+
+def test_parameters_of_other_shapes_are_the_expressions_to_refuse(gpu):
+    # the kernels would read past the end of a smaller parameter; the expressions raise
+    layer, _, _, coords = _layer_and_inputs(gpu)
+    x = torch.randn(1, 33, 64, device=gpu, requires_grad=True)
+    layer.attn.spread_weights = nn.Parameter(torch.zeros(1, device=gpu))
+    with pytest.raises(AssertionError):
+        layer.attn(x, x, x, coords)
+    layer.ffn_norm.bias = nn.Parameter(torch.zeros(4, device=gpu))
+    with pytest.raises(RuntimeError):
+        layer._residual_norm(x, x, layer.ffn_norm)
