@@ -306,7 +306,7 @@ def self_attention(x, coords, mask, m):
     if (not any(p.requires_grad for p in params[:3]) or m.legacy_logits or dk not in (32, 64, 128) or dm > 16384 or x.numel() == 0 or not coords.is_cuda or coords.requires_grad or type(coords) not in _PLAIN_TYPES
             or (mask is not None and type(mask) is not torch.Tensor)
             or x.shape[1] * 3 * dm * 4 >= 2 ** 31 or m.operand_dtype not in (None, torch.bfloat16)
-            or type(m).get_spreads is not ga.GeoAttention.get_spreads or "get_spreads" in m.__dict__
+            or type(m).get_spreads is not ga.GeoAttention.get_spreads or "get_spreads" in m.__dict__ or not isinstance(m.min_spread, (int, float))
             or not recording(x, *params) or not aligned(*params)):
         return None
     return _SelfAttention.apply(x, coords, mask, *params, m.min_spread, m.operand_dtype)

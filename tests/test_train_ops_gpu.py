@@ -339,3 +339,11 @@ def test_parameters_of_other_shapes_are_the_expressions_to_refuse(gpu):
     layer.ffn_norm.bias = nn.Parameter(torch.zeros(4, device=gpu))
     with pytest.raises(RuntimeError):
         layer._residual_norm(x, x, layer.ffn_norm)
+
+
+def test_minimal_spreads_in_a_tensor_keep_the_general_path(gpu):
+    layer, _, _, coords = _layer_and_inputs(gpu)
+    x = torch.randn(1, 33, 64, device=gpu, requires_grad=True)
+    layer.attn.min_spread = torch.tensor([2.0, 3.0], device=gpu, requires_grad=True)
+    g, = torch.autograd.grad(layer.attn(x, x, x, coords).square().sum(), [layer.attn.min_spread])
+    assert torch.isfinite(g).all() and g.any()
