@@ -98,8 +98,8 @@ def geo_attn(Q, K, V, coords, sigma, key_padding_mask=None, return_lse: bool = F
         raise AssertionError(f"coordinates must be of shape (batch, N, 3), not {tuple(coords.shape)}")
     if sigma.dim() != 1 or sigma.size(0) != H:
         raise AssertionError(f"number of spreads must be equal to nheads, not {tuple(sigma.shape)} and {H=}")
-    if not Q.is_cuda:
-        raise _lib.ProteusError("geo_attn needs tensors on the GPU (there is no CPU path)")
+    if not Q.is_cuda or not (Q.device == K.device == V.device):
+        raise _lib.ProteusError("geo_attn needs tensors on the GPU, all on one (there is no CPU path)")
     # (reading the answer back synchronises with the device: callers whose sigma is positive by construction skip it)
     # (one copy of the H floats instead of a comparison, a reduction and the copy of its result)
     if check_sigma and not all(x > 0 for x in sigma.tolist()):
@@ -239,8 +239,11 @@ def geo_attn_backward(Q, K, V, O, L, dO, coords, sigma, key_padding_mask=None, b
     grad_dtype: None (fp32) or the operand type, in which dQ, dK, dV are then returned: the same sums, rounded once.
     """
     Z, H, N, d = Q.shape
-    if not Q.is_cuda:
-        raise _lib.ProteusError("geo_attn_backward needs tensors on the GPU (there is no CPU path)")
+    if not Q.is_cuda or not (Q.device == K.device == V.device == O.device == dO.device):
+        raise _lib.ProteusError("geo_attn_backward needs tensors on the GPU, all on one (there is no CPU path)")
+    if not (Q.shape == K.shape == V.shape == O.shape == dO.shape) or L.numel() != Z * H * N:
+        raise AssertionError(f"Q, K, V, O and dO must have one shape and L an element per row, but got {Q.shape=}, {K.shape=}, {V.shape=}, "
+                             f"{O.shape=}, {dO.shape=}, {L.shape=}")
     lib = _lib.load()
     dev = Q.device
     op_dtype, op_type = _operand_type(operand_dtype, betas is not None)

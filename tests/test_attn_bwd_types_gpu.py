@@ -4,7 +4,7 @@ import pytest
 import torch
 
 import proteusai_amd as pa
-from proteusai_amd import synth
+from proteusai_amd import _lib, synth
 from proteusai_amd.geometric_attn import _delta, _prepare_backward
 
 pytestmark = pytest.mark.gpu
@@ -65,3 +65,18 @@ def ds_like(H, gpu):
     junk = [torch.full((H,), 7.0, device=gpu) for _ in range(4)]
     del junk
     return torch.ones(H, device=gpu)
+
+
+def test_tensors_that_do_not_go_together_are_refused(gpu):
+    # before anything is launched: their addresses or sizes are not what the kernels take them for
+    q, k, v, coords, sigma, mask, dO = _inputs(gpu, 2, 3, 40, 32, torch.bfloat16, 1)
+    for t in ((q, k.cpu(), v), (q, k, v.cpu())):
+        with pytest.raises(_lib.ProteusError, match="all on one"):
+            pa.geo_attn(*t, coords, sigma, mask)
+    O, L = pa.geo_attn(q, k, v, coords, sigma, mask, return_lse=True)
+    for t in ((q, k.cpu(), v, O, L, dO), (q, k, v, O.cpu(), L, dO), (q, k, v, O, L, dO.cpu())):
+        with pytest.raises(_lib.ProteusError, match="all on one"):
+            pa.geo_attn_backward(*t, coords, sigma, mask)
+    for t in ((q, k[:, :, :39], v, O, L, dO), (q, k, v, O[:, :2], L, dO), (q, k, v, O, L[:1], dO), (q, k, v, O, L, dO[..., :1])):
+        with pytest.raises(AssertionError, match="one shape"):
+            pa.geo_attn_backward(*t, coords, sigma, mask)
