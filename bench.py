@@ -1,7 +1,6 @@
 """Headline benchmark: Wavefunction Embedding forward at B=1, N=16384, d_model=512
-(BASELINE.json configs[1]) on one MI355X.  Beside it, one timed leg per other configuration
-(configs[0] WE N=512; configs[2] padded attention B=4 N=4096; configs[3] encoder forward;
-configs[4] WE N=65536 and attention N=16384), roofline fractions for every kernel and the
+on one MI355X.  Beside it, one timed leg per other configuration
+(WE N=512; padded attention B=4 N=4096; encoder forward; WE N=65536 and attention N=16384), roofline fractions for every kernel and the
 CPU PyTorch path timed on the host cores as a baseline for each.
 
   python bench.py [--gpus 1] [--steps K] [--warmup W] [--legs a,b,...] [--no-cpu] [--full-cpu]
@@ -314,7 +313,7 @@ def main():
         "baseline_note": "reference README.md:34: 386 ms (178 Gpair*wavenumber/s) for this shape on an H100",
         "dtype": "f32", "data": "synthetic",
         "config": {"workload": "WE forward B=1 N=16384 d_model=512 (256 wavenumbers), compacted random-walk C-alpha chain, "
-                               "lambda 3.7-20 A base 20, no mask (BASELINE.json configs[1])",
+                               "lambda 3.7-20 A base 20, no mask",
                    "Z": Z, "N": N, "K": K, "we_variant": _lib.we_variants()[args.we_tuning]},
         "roofline": roofline,
     }
@@ -391,14 +390,14 @@ def main():
         result["we_aniso"]["ms_embedding_only"] = xl_ms           # d_cb = d_k = NULL: two running sums per wavenumber instead of six
         del ao
 
-    # ---------------- configs[0]: WE forward B=1, N=512 (the reference's CPU-runnable case) ----------------
+    # ---------------- WE forward B=1, N=512 (the reference's CPU-runnable case) ----------------
     if "cfg1" in legs:
         c1, _ = synth.we_inputs(512, seed=1, batch=1, d_model=d_model, compact=False)
         c1d = c1.to(dev).contiguous()
         o1, cs1, ss1 = (torch.empty(1, 512, n, device=dev) for n in (2 * K, K, K))
         _, ms1 = time_launches(torch, lambda: we_forward_into(c1d, w, None, o1, cs1, ss1), 200)
         W1 = 512.0 * 512 * K
-        leg = {"workload": "WE forward B=1 N=512 d_model=512, random-walk chain, no mask (BASELINE.json configs[0]); "
+        leg = {"workload": "WE forward B=1 N=512 d_model=512, random-walk chain, no mask; "
                            "8 observer blocks of 64 rows x 64 tiles of 4 wavenumbers: 512 short workgroups, a launch-latency-sized kernel",
                "ms": ms1, "gpair_wavenumber_per_s": W1 / (ms1 * 1e-3) / 1e9, "dtype": "f32",
                "roofline": {"kernel": "we_fwd_kernel", "bound": "valu", "achieved": 9.0 * W1 / (ms1 * 1e-3) / 1e12,
@@ -411,14 +410,14 @@ def main():
                                    "sample": f"the full workload, median of {runs} runs, tiled CPU PyTorch fp32, {dt * 1e3:.1f} ms"}
         result["cfg1_we_n512"] = leg
 
-    # ---------------- configs[4], WE half: B=1, N=65536, same compacted-chain generator ----------------
+    # ---------------- WE forward B=1, N=65536, same compacted-chain generator ----------------
     if "cfg5_we" in legs:
         c5, _ = synth.we_inputs(65536, seed=5, compact=True)
         c5d = c5.to(dev).contiguous()
         o5, cs5, ss5 = (torch.empty(1, 65536, n, device=dev) for n in (2 * K, K, K))
         ms5, _ = time_launches(torch, lambda: we_forward_into(c5d, w, None, o5, cs5, ss5), 3, 0.0)
         W5 = 65536.0 * 65536 * K
-        leg = {"workload": "WE forward B=1 N=65536 d_model=512, compacted random-walk chain, no mask (BASELINE.json configs[4])",
+        leg = {"workload": "WE forward B=1 N=65536 d_model=512, compacted random-walk chain, no mask",
                "ms": ms5, "gpair_wavenumber_per_s": W5 / (ms5 * 1e-3) / 1e9, "dtype": "f32",
                "roofline": {"kernel": "we_fwd_kernel", "bound": "valu", "achieved": 9.0 * W5 / (ms5 * 1e-3) / 1e12,
                             "peak": PEAK_FP32_VECTOR_TFLOPS, "unit": "TFLOP/s",
@@ -443,7 +442,7 @@ def main():
         if rc != 0:
             _lib.check(rc, "proteus_geo_attn_fwd")
 
-    # ---------------- configs[2]: geometric attention B=4, N=4096, H=8, d=64, lengths in [2048, 4096] ----------------
+    # ---------------- geometric attention B=4, N=4096, H=8, d=64, lengths in [2048, 4096] ----------------
     if "cfg3" in legs:
         Q3, K3, V3, c3, sg3, m3 = synth.attn_inputs(4, 8, 4096, 64, seed=3, min_len=2048)
         q3, k3, v3, c3d, s3d, m3d = (t.to(dev) for t in (Q3, K3, V3, c3, sg3, m3))
@@ -475,7 +474,7 @@ def main():
         useful = 4.0 * 8 * 64 * float((lens * lens).sum())
         dense = 4.0 * 4 * 8 * 64 * 4096 * 4096
         leg = {"workload": "geometric attention forward B=4 H=8 N=4096 d_head=64 bf16, random-walk chains, sigma 3-25 A, "
-                           "valid lengths uniform in [2048, 4096], the rest padded (BASELINE.json configs[2])",
+                           "valid lengths uniform in [2048, 4096], the rest padded",
                "ms": ms3, "lengths": [int(x) for x in lens], "dtype": "bf16",
                "tflops_useful": useful / (ms3 * 1e-3) / 1e12, "tflops_dense_equivalent": dense / (ms3 * 1e-3) / 1e12,
                "entry_point": "proteus_geo_attn_fwd_ws (plan kernel + split-items grid: two launches)",
@@ -513,7 +512,7 @@ def main():
         result["cfg3_attn_b4_n4096_padded"] = leg
         del q3, k3, v3, O3, L3, ws3
 
-    # ---------------- one unpadded sequence that does not fill the chip: Z=1, H=8, N=8192 (not a BASELINE configuration) ----------------
+    # ---------------- one unpadded sequence that does not fill the chip: Z=1, H=8, N=8192 ----------------
     if "attn" in legs:
         Q1, K1, V1, c1, sg1, _ = synth.attn_inputs(1, 8, 8192, 64, seed=8)
         q1, k1, v1, c1d, s1d = (t.to(dev) for t in (Q1, K1, V1, c1, sg1))
@@ -538,7 +537,7 @@ def main():
             "frac_plain_grid": flop1 / (ms1_plain * 1e-3) / 1e12 / PEAK_BF16_MFMA_TFLOPS}
         del q1, k1, v1, O1, L1, ws1
 
-    # ---------------- geometric attention forward, N=16384, H=8, d=64 (configs[4]) ----------------
+    # ---------------- geometric attention forward, N=16384, H=8, d=64 ----------------
     if "attn" in legs or "attn_bwd" in legs:
         wc, _ = synth.we_inputs(65536, seed=5, compact=True)
         Q, Kt, V, ac, sigma, _ = synth.attn_inputs(1, 8, 16384, 64, seed=5, coords=wc[:, :16384].contiguous())
@@ -550,7 +549,7 @@ def main():
         a_tflops = flops / (a_ms * 1e-3) / 1e12
         a_traffic, a_traffic_src = traffic_from(PROFILE_ATTN)
         leg = {
-            "workload": "geometric attention forward Z=1 H=8 N=16384 d_head=64 bf16, compacted chain, sigma 3-25 A (BASELINE.json configs[4])",
+            "workload": "geometric attention forward Z=1 H=8 N=16384 d_head=64 bf16, compacted chain, sigma 3-25 A",
             "ms": a_ms, "tflops": a_tflops, "dtype": "bf16",
             "roofline": {"kernel": "geo_attn_fwd_pipe_kernel", "bound": "mfma", "achieved": a_tflops, "peak": PEAK_BF16_MFMA_TFLOPS,
                          "unit": "TFLOP/s", "frac": a_tflops / PEAK_BF16_MFMA_TFLOPS,
@@ -657,7 +656,7 @@ def main():
             del dOb, Dv, dQ_, dK_, dV_, bet, dbt
         del q, k, v, O, L
 
-    # ---------------- encoder forward, B=8, N=1024, 4 layers, bf16 weights, fp32 WE (configs[3]) ----------------
+    # ---------------- encoder forward, B=8, N=1024, 4 layers, bf16 weights, fp32 WE ----------------
     if "encoder" in legs:
         import proteusai_amd as pa
         torch.manual_seed(4)
@@ -684,7 +683,7 @@ def main():
             torch.cuda.synchronize()
         result["encoder_forward"] = {
             "workload": "WE + 33x512 embedding, 4 x (geometric MHA H=8 + LN + FFN 512-2048-512 GELU + LN), head to 20; "
-                        "B=8 N=1024 lengths 128-1024, bf16 weights, fp32 WE (BASELINE.json configs[3])",
+                        "B=8 N=1024 lengths 128-1024, bf16 weights, fp32 WE",
             "ms": e0.elapsed_time(e1) / 10, "valid_tokens": int(lens.sum()),
             "tokens_per_s": float(lens.sum()) / (e0.elapsed_time(e1) / 10 * 1e-3),
         }

@@ -77,7 +77,7 @@ def tail_mask(Z, N, g, lo):
 
 def test_library_takes_the_balanced_schedule_where_these_tests_expect_it():
     lib = _lib.load()
-    assert lib.proteus_geo_attn_fwd_workspace_bytes(4, 8, 4096, 64, 0) > 0        # automatic
+    assert lib.proteus_geo_attn_fwd_workspace_bytes(4, 8, 4096, 64, 0) > 0        # the benchmark's padded batch: automatic
     assert lib.proteus_geo_attn_fwd_workspace_bytes(8, 8, 1024, 64, 0) == 0       # the encoder's batch: plain grid
     assert lib.proteus_geo_attn_fwd_workspace_bytes(8, 8, 1024, 64, BALANCED) > 0
     assert lib.proteus_geo_attn_fwd_workspace_bytes(3, 2, 700, 32, BALANCED) == 0     # d_head = 64 only
@@ -139,7 +139,7 @@ def test_scattered_padding_empty_sequence_and_padded_query_tiles(gpu, sched):
 
 
 def test_cfg3_shape_takes_the_split_items_schedule_automatically(gpu):
-    # B=4, H=8, N=4096, lengths in [2048, 4096]; tuning 0 through the operator
+    # the benchmark's padded batch: B=4, H=8, N=4096, lengths in [2048, 4096]; tuning 0 through the operator
     Q, K, V, coords, sigma, mask = synth.attn_inputs(4, 8, 4096, 64, seed=3, min_len=2048)
     auto = run(gpu, Q, K, V, coords, sigma, mask, 0)
     forced = run(gpu, Q, K, V, coords, sigma, mask, SPLIT)

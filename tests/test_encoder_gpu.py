@@ -1,4 +1,4 @@
-"""GPU tests of the encoder stack built around the two kernels (BASELINE configuration 4)."""
+"""GPU tests of the encoder stack built around the two kernels."""
 import numpy as np
 import pytest
 import torch
@@ -175,7 +175,7 @@ def _cfg4_batch():
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32_weights", "bf16_weights"])
 def test_cfg4_shape_logits_match_the_cpu_statement_of_the_whole_stack(gpu, dtype):
-    """The whole encoder at BASELINE.json configs[3] (B=8, N=1024, d_model=512, H=8, 4 layers, FFN 2048, head to 20
+    """The whole encoder at its benchmark configuration (B=8, N=1024, d_model=512, H=8, 4 layers, FFN 2048, head to 20
     logits, lengths in [128, 1024]) against the fp32 CPU statement of the same stack with the same weights
     (torch_oracle.encoder_forward_torch: dense torch attention and embedding oracles, pinned in
     tests/test_oracle_encoder.py), on every valid token.
@@ -184,7 +184,7 @@ def test_cfg4_shape_logits_match_the_cpu_statement_of_the_whole_stack(gpu, dtype
     bf16 weights 9.2e-3, 4.6e-2, 1.1 %).  fp32 weights: the only low-precision steps are the attention's bf16 operands
     and probabilities (four layers): rel-L2 over all valid logits <= 8e-3, per token <= 5e-2, max-abs <= 2 % of the
     logits' range.  bf16 weights (the
-    configuration BASELINE names): every activation between two layers is rounded to bf16 (2^-9 relative, some 30
+    benchmark's configuration): every activation between two layers is rounded to bf16 (2^-9 relative, some 30
     roundings from the embedding to the head, which LayerNorm renormalises rather than damps): rel-L2 <= 2e-2, per
     token rel-L2 <= 8e-2 on every token, max-abs <= 4 % of the logits' range, and the arg-max amino acid agrees where
     the reference's top two logits are further apart than that."""
@@ -204,7 +204,7 @@ def test_cfg4_shape_logits_match_the_cpu_statement_of_the_whole_stack(gpu, dtype
     per_token = ((got - want).norm(dim=1) / want.norm(dim=1))
     span = float(want.max() - want.min())
     max_abs = float((got - want).abs().max())
-    print(f"encoder at configs[3], {dtype}: rel-L2 {rel:.3e}, worst token {float(per_token.max()):.3e}, "
+    print(f"encoder at B=8 N=1024, {dtype}: rel-L2 {rel:.3e}, worst token {float(per_token.max()):.3e}, "
           f"max abs {max_abs:.3e} of a logit range of {span:.2f}", flush=True)
     bars = {torch.float32: (8e-3, 5e-2, 0.02), torch.bfloat16: (2e-2, 8e-2, 0.04)}[dtype]
     assert rel <= bars[0], f"rel-L2 {rel:.3e}"
