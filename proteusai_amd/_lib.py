@@ -211,6 +211,18 @@ def stride_array(*tensors):
     return _stride_array_of(vals)
 
 
+@functools.lru_cache(maxsize=1024)
+def we_workspace_bytes(Z, N, K, tuning):
+    """proteus_we_fwd_workspace_bytes, kept per shape: asking the library costs a small call 2 % of its time."""
+    return load().proteus_we_fwd_workspace_bytes(Z, N, K, tuning)
+
+
+@functools.lru_cache(maxsize=1024)
+def we_aniso_workspace_bytes(Z, N, K, partials, padded, tuning):
+    """proteus_we_aniso_fwd_workspace_bytes, kept per shape."""
+    return load().proteus_we_aniso_fwd_workspace_bytes(Z, N, K, partials, padded, tuning)
+
+
 def raw_stream(dev):
     """Handle of torch's current stream on `dev` for the `stream` argument of the entry points."""
     import torch

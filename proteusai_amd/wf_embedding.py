@@ -69,14 +69,14 @@ def we_forward(coords, wavenumbers, mask=None, tuning: int = 0, magnitude_type: 
                                             Z, N, K, int(magnitude_type), dropout_p, int(rng_seed) & 0xffffffff, stream)
         elif magnitude_type == 1:
             # with a workspace the library may go through grids of the distances (its size is 0 where that is of no use)
-            ws_bytes = lib.proteus_we_fwd_workspace_bytes(Z, N, K, int(tuning))
-            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
-            rc = lib.proteus_we_fwd_ws(c.data_ptr(), _lib.COORDS_AOS, w.data_ptr(),
-                                       None if m is None else m.data_ptr(),
-                                       out.data_ptr(), cos_sums.data_ptr() if need_sums else None,
-                                       sin_sums.data_ptr() if need_sums else None,
-                                       None if ws is None else ws.data_ptr(), ws_bytes,
-                                       Z, N, K, int(tuning), stream)
+            args = (c.data_ptr(), _lib.COORDS_AOS, w.data_ptr(), None if m is None else m.data_ptr(),
+                    out.data_ptr(), cos_sums.data_ptr() if need_sums else None, sin_sums.data_ptr() if need_sums else None)
+            ws_bytes = _lib.we_workspace_bytes(Z, N, K, int(tuning))
+            if ws_bytes:
+                ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+                rc = lib.proteus_we_fwd_ws(*args, ws.data_ptr(), ws_bytes, Z, N, K, int(tuning), stream)
+            else:
+                rc = lib.proteus_we_fwd(*args, Z, N, K, int(tuning), stream)
         else:
             rc = lib.proteus_we_legacy_fwd(c.data_ptr(), _lib.COORDS_AOS, w.data_ptr(),
                                            None if m is None else m.data_ptr(),
@@ -208,13 +208,14 @@ def we_aniso_forward(coordsA, coordsB, cb_magnitudes, wavenumbers, mask=None, tu
     with _lib.on_device(dev):
         stream = _lib.raw_stream(dev)
         # with a workspace the library may go through grids of the distances (its size is 0 where that is of no use)
-        ws_bytes = lib.proteus_we_aniso_fwd_workspace_bytes(Z, N, K, int(partials), int(m is not None), int(tuning))
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
-        rc = lib.proteus_we_aniso_fwd_ws(a.data_ptr(), b.data_ptr(), _lib.COORDS_AOS, cb.data_ptr(), w.data_ptr(),
-                                         None if m is None else m.data_ptr(),
-                                         out.data_ptr(), d_cb.data_ptr() if partials else None, d_k.data_ptr() if partials else None,
-                                         None if ws is None else ws.data_ptr(), ws_bytes,
-                                         Z, N, K, int(tuning), stream)
+        args = (a.data_ptr(), b.data_ptr(), _lib.COORDS_AOS, cb.data_ptr(), w.data_ptr(), None if m is None else m.data_ptr(),
+                out.data_ptr(), d_cb.data_ptr() if partials else None, d_k.data_ptr() if partials else None)
+        ws_bytes = _lib.we_aniso_workspace_bytes(Z, N, K, int(partials), int(m is not None), int(tuning))
+        if ws_bytes:
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+            rc = lib.proteus_we_aniso_fwd_ws(*args, ws.data_ptr(), ws_bytes, Z, N, K, int(tuning), stream)
+        else:
+            rc = lib.proteus_we_aniso_fwd(*args, Z, N, K, int(tuning), stream)
     _lib.check(rc, "proteus_we_aniso_fwd")
     return out, d_cb, d_k
 
