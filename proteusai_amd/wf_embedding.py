@@ -14,6 +14,20 @@ from . import _lib
 from .cb_utils import get_coords
 
 
+def _f32(t, dev):
+    """fp32, contiguous, on `dev`: the tensor itself where it already is all that (only its address is used)."""
+    if t.dtype == torch.float32 and t.device == dev and t.is_contiguous():
+        return t
+    return t.detach().to(device=dev, dtype=torch.float32).contiguous()
+
+
+def _mask_bytes(mask, dev):
+    """One byte per token, not 0 = padded."""
+    if mask.dtype == torch.bool and mask.device == dev and mask.is_contiguous():
+        return mask
+    return mask.to(device=dev, dtype=torch.bool).contiguous()
+
+
 def we_forward(coords, wavenumbers, mask=None, tuning: int = 0, magnitude_type: int = 1, need_sums: bool = True,
                dropout_p: float = 0.0, rng_seed=None):
     """out, cos_sums, sin_sums = we_forward(coords [Z,N,3], wavenumbers [K], mask [Z,N] bool | None).
@@ -43,15 +57,14 @@ def we_forward(coords, wavenumbers, mask=None, tuning: int = 0, magnitude_type: 
     lib = _lib.load()
     dev = coords.device
     # everything in fp32, as isotropic/cuda/wf_embedding.py:32-35
-    c = coords.detach().to(torch.float32).contiguous()
-    w = wavenumbers.detach().to(device=dev, dtype=torch.float32).contiguous()
+    c, w = _f32(coords, dev), _f32(wavenumbers, dev)
     Z, N, _ = c.shape
     K = w.shape[0]
     m = None
     if mask is not None:
         if tuple(mask.shape) != (Z, N):
             raise ValueError(f"mask must be of shape ({Z}, {N}), not {tuple(mask.shape)}")
-        m = mask.to(device=dev, dtype=torch.bool).contiguous().view(torch.uint8)
+        m = _mask_bytes(mask, dev)
     out = torch.empty(Z, N, 2 * K, dtype=torch.float32, device=dev)
     need_sums = need_sums or magnitude_type != 1 or dropout_p != 0.0
     cos_sums = torch.empty(Z, N, K, dtype=torch.float32, device=dev) if need_sums else None
@@ -90,7 +103,7 @@ def _bwd_prepare(dO, *saved):
     if not dO.is_cuda:
         raise RuntimeError("the WE backward runs on the HIP kernels only: tensors must be on the GPU")
     Z, N, K2 = dO.shape
-    ts = [dO.contiguous().float()] + [None if t is None else t.contiguous().float() for t in saved]
+    ts = [None if t is None else _f32(t, dO.device) for t in (dO, *saved)]
     lib = _lib.load()
     ws = torch.empty(max(1, lib.proteus_we_bwd_workspace_bytes(Z, N, K2 // 2) // 4), dtype=torch.float32, device=dO.device)
     return lib, ts, ws, Z, N, K2 // 2, _lib.raw_stream(dO.device)
@@ -189,17 +202,14 @@ def we_aniso_forward(coordsA, coordsB, cb_magnitudes, wavenumbers, mask=None, tu
         raise _lib.ProteusError("we_aniso_forward needs tensors on the GPU (there is no CPU path)")
     lib = _lib.load()
     dev = coordsA.device
-    a = coordsA.detach().to(torch.float32).contiguous()
-    b = coordsB.detach().to(device=dev, dtype=torch.float32).contiguous()
-    w = wavenumbers.detach().to(device=dev, dtype=torch.float32).contiguous()
-    cb = cb_magnitudes.detach().to(device=dev, dtype=torch.float32).contiguous()
+    a, b, w, cb = (_f32(t, dev) for t in (coordsA, coordsB, wavenumbers, cb_magnitudes))
     Z, N, _ = a.shape
     K = w.shape[0]
     m = None
     if mask is not None:
         if tuple(mask.shape) != (Z, N):
             raise ValueError(f"mask must be of shape ({Z}, {N}), not {tuple(mask.shape)}")
-        m = mask.to(device=dev, dtype=torch.bool).contiguous().view(torch.uint8)
+        m = _mask_bytes(mask, dev)
     out = torch.empty(Z, N, 2 * K, dtype=torch.float32, device=dev)
     d_cb = torch.empty_like(out) if partials else None
     d_k = torch.empty_like(out) if partials else None
