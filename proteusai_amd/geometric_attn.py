@@ -98,7 +98,7 @@ def geo_attn(Q, K, V, coords, sigma, key_padding_mask=None, return_lse: bool = F
         raise AssertionError(f"coordinates must be of shape (batch, N, 3), not {tuple(coords.shape)}")
     if sigma.dim() != 1 or sigma.size(0) != H:
         raise AssertionError(f"number of spreads must be equal to nheads, not {tuple(sigma.shape)} and {H=}")
-    if not Q.is_cuda or not (Q.device == K.device == V.device):
+    if not Q.is_cuda or not (Q.get_device() == K.get_device() == V.get_device()):
         raise _lib.ProteusError("geo_attn needs tensors on the GPU, all on one (there is no CPU path)")
     # (reading the answer back synchronises with the device: callers whose sigma is positive by construction skip it)
     # (one copy of the H floats instead of a comparison, a reduction and the copy of its result)
@@ -238,12 +238,18 @@ def geo_attn_backward(Q, K, V, O, L, dO, coords, sigma, key_padding_mask=None, b
     of one [Z,N,3,H,d] buffer); allocated here otherwise.
     grad_dtype: None (fp32) or the operand type, in which dQ, dK, dV are then returned: the same sums, rounded once.
     """
-    Z, H, N, d = Q.shape
-    if not Q.is_cuda or not (Q.device == K.device == V.device == O.device == dO.device):
+    Z, H, N, _ = Q.shape
+    if not Q.is_cuda or not (Q.get_device() == K.get_device() == V.get_device() == O.get_device() == dO.get_device()):
         raise _lib.ProteusError("geo_attn_backward needs tensors on the GPU, all on one (there is no CPU path)")
     if not (Q.shape == K.shape == V.shape == O.shape == dO.shape) or L.numel() != Z * H * N:
         raise AssertionError(f"Q, K, V, O and dO must have one shape and L an element per row, but got {Q.shape=}, {K.shape=}, {V.shape=}, "
                              f"{O.shape=}, {dO.shape=}, {L.shape=}")
+    return _backward(Q, K, V, O, L, dO, coords, sigma, key_padding_mask, betas, min_rbf, max_rbf, operand_dtype, grads, grad_dtype)
+
+
+def _backward(Q, K, V, O, L, dO, coords, sigma, key_padding_mask, betas, min_rbf, max_rbf, operand_dtype, grads=None, grad_dtype=None):
+    """geo_attn_backward on tensors that are known to go together (the forward's own, and a gradient from autograd)."""
+    Z, H, N, d = Q.shape
     lib = _lib.load()
     dev = Q.device
     op_dtype, op_type = _operand_type(operand_dtype, betas is not None)
@@ -305,9 +311,9 @@ class _geometric_attn(torch.autograd.Function):
     def backward(ctx, dO):
         Q, K, V, O, L, coords, spreads, betas, mask = ctx.saved_tensors
         op_dtype = ctx.operand_dtype or torch.bfloat16
-        dQ, dK, dV, d_sigma, d_beta = geo_attn_backward(Q, K, V, O, L, dO, coords, spreads, mask, betas,
-                                                        ctx.min_rbf, ctx.max_rbf, ctx.operand_dtype,
-                                                        grad_dtype=op_dtype if Q.dtype == K.dtype == V.dtype == op_dtype else None)
+        dQ, dK, dV, d_sigma, d_beta = _backward(Q, K, V, O, L, dO, coords, spreads, mask, betas,
+                                                ctx.min_rbf, ctx.max_rbf, ctx.operand_dtype,
+                                                grad_dtype=op_dtype if Q.dtype == K.dtype == V.dtype == op_dtype else None)
         return (dQ.to(Q.dtype), dK.to(K.dtype), dV.to(V.dtype), None, d_sigma.to(spreads.dtype),
                 None if betas is None else d_beta.to(betas.dtype), None, None, None, None, None, None, None)
 
@@ -341,13 +347,13 @@ class _geometric_attn_qkv(torch.autograd.Function):
         g = torch.empty(qkv.shape, dtype=grad_dtype, device=qkv.device)
         grads = tuple(g[:, :, i].permute(0, 2, 1, 3) for i in range(3))
         if _fused_grad_views_ok(grads):
-            _, _, _, d_sigma, d_beta = geo_attn_backward(Q, K, V, O, L, dO, coords, spreads, mask, betas,
-                                                         ctx.min_rbf, ctx.max_rbf, ctx.operand_dtype, grads=grads, grad_dtype=grad_dtype)
+            _, _, _, d_sigma, d_beta = _backward(Q, K, V, O, L, dO, coords, spreads, mask, betas,
+                                                 ctx.min_rbf, ctx.max_rbf, ctx.operand_dtype, grads=grads, grad_dtype=grad_dtype)
         else:
             # a sequence of the fused buffer spans 2 GiB or more: the kernels cannot address it in place, so the
             # gradients go to buffers of their own (as the sliced operator does) and are copied in
-            dQ, dK, dV, d_sigma, d_beta = geo_attn_backward(Q, K, V, O, L, dO, coords, spreads, mask, betas,
-                                                            ctx.min_rbf, ctx.max_rbf, ctx.operand_dtype)
+            dQ, dK, dV, d_sigma, d_beta = _backward(Q, K, V, O, L, dO, coords, spreads, mask, betas,
+                                                    ctx.min_rbf, ctx.max_rbf, ctx.operand_dtype)
             for dst, src in zip(grads, (dQ, dK, dV)):
                 dst.copy_(src)
         return (g.to(qkv.dtype), None, d_sigma.to(spreads.dtype), None if betas is None else d_beta.to(betas.dtype),

@@ -279,8 +279,7 @@ class _SelfAttention(torch.autograd.Function):
         d2 = _dense(d).view(Z * N, dm)
         dO = d2.mm(Wo).view(Z, N, H, dk).permute(0, 2, 1, 3)
         g = torch.empty(qkv.shape, dtype=torch.float32, device=d.device)
-        _, _, _, d_sigma, _ = ga.geo_attn_backward(*_heads(qkv), O, L, dO, coords, sigma, mask, None, operand_dtype=ctx.operand_dtype,
-                                                   grads=_heads(g))
+        _, _, _, d_sigma, _ = ga._backward(*_heads(qkv), O, L, dO, coords, sigma, mask, None, 0.0, 1.0, ctx.operand_dtype, grads=_heads(g))
         g2 = g.view(Z * N, 3 * dm)
         dx = g2.mm(W.t()).view(x.shape) if need[0] else None
         grads = [torch.empty_like(p, memory_format=torch.contiguous_format) if n else None for p, n in zip(params, need[3:11])]
