@@ -62,35 +62,53 @@ __device__ __forceinline__ int wa_terms(const float z, const float tail)
     return n;
 }
 
-// Length of the longest diagonal of a thread's share of the batch items' boxes (infinite if one of them holds a token that is not
-// finite), for the 256 threads of a block: as many lanes share an item as have boxes to read.
-__device__ __forceinline__ float wa_extent(const WgBox* __restrict__ boxes, const int Z, const int nbox)
-{
-    const int tid = threadIdx.x;
-    int lanes = 1;
-    while (lanes < 64 && lanes < nbox) lanes *= 2;
-    float longest = 0.f;
-    for (int z = tid / lanes; z - tid / lanes < Z; z += 256 / lanes) {         // (all lanes of a wave meet in the exchanges)
-        float lo[3] = {3.0e38f, 3.0e38f, 3.0e38f}, hi[3] = {-3.0e38f, -3.0e38f, -3.0e38f}, bad = 0.f;
-        if (z < Z)
-            for (int i = tid % lanes; i < nbox; i += lanes) {
-                const WgBox q = boxes[(size_t)z * nbox + i];
-                bad = fmaxf(bad, q.bad);
-                if (!(q.lo[0] <= q.hi[0])) continue;                            // padded tokens only
+// The batch items' boxes, read by a block of 256 threads: as many lanes share an item as it has boxes.  `fetch` sends off a thread's
+// first two, `longest` returns the length of the longest diagonal of its items (infinite if one holds a token that is not finite).
+struct WaBoxes {
+    const WgBox* __restrict__ boxes;
+    int Z, nbox, lanes, z, i;
+    WgBox q[2];
+    __device__ __forceinline__ void fetch(const WgBox* __restrict__ from, const int Z_, const int nbox_)
+    {
+        boxes = from; Z = Z_; nbox = nbox_;
+        lanes = nbox > 32 ? 64 : nbox > 16 ? 32 : nbox > 8 ? 16 : nbox > 4 ? 8 : nbox > 2 ? 4 : nbox;
+        z = (int)threadIdx.x / lanes; i = (int)threadIdx.x % lanes;
+        const float inf = __builtin_inff();
 #pragma unroll
-                for (int c = 0; c < 3; ++c) { lo[c] = fminf(lo[c], q.lo[c]); hi[c] = fmaxf(hi[c], q.hi[c]); }
-            }
-        for (int o = 1; o < lanes; o *= 2) {
-            bad = fmaxf(bad, __shfl_xor(bad, o));
-#pragma unroll
-            for (int c = 0; c < 3; ++c) { lo[c] = fminf(lo[c], __shfl_xor(lo[c], o)); hi[c] = fmaxf(hi[c], __shfl_xor(hi[c], o)); }
+        for (int u = 0; u < 2; ++u) {
+            q[u] = WgBox{{inf, inf, inf}, {-inf, -inf, -inf}, 0.f, 0.f};                // (as of padded tokens only)
+            if (z < Z && i + u * lanes < nbox) q[u] = boxes[(size_t)z * nbox + i + u * lanes];
         }
-        const float dx = hi[0] - lo[0], dy = hi[1] - lo[1], dz = hi[2] - lo[2];
-        if (lo[0] <= hi[0]) longest = fmaxf(longest, __builtin_sqrtf(dx * dx + dy * dy + dz * dz));
-        longest += bad;
     }
-    return longest;
-}
+    __device__ __forceinline__ float longest()
+    {
+        float far = 0.f;
+        const int step = 256 / lanes;
+        for (int item = z; item - z < Z; item += step) {                                // (all lanes of a wave meet in the exchanges)
+            float lo[3], hi[3], bad = 0.f;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) { lo[c] = 3.0e38f; hi[c] = -3.0e38f; }
+            auto add = [&](const WgBox& w) {
+                bad = fmaxf(bad, w.bad);
+#pragma unroll
+                for (int c = 0; c < 3; ++c) { lo[c] = fminf(lo[c], w.lo[c]); hi[c] = fmaxf(hi[c], w.hi[c]); }
+            };
+            if (item == z) { add(q[0]); add(q[1]); }
+            for (int j = item == z ? i + 2 * lanes : i; item < Z && j < nbox; j += lanes) add(boxes[(size_t)item * nbox + j]);
+#pragma unroll
+            for (int o = 1; o < 64; o *= 2) {
+                if (o >= lanes) break;
+                bad = fmaxf(bad, __shfl_xor(bad, o));
+#pragma unroll
+                for (int c = 0; c < 3; ++c) { lo[c] = fminf(lo[c], __shfl_xor(lo[c], o)); hi[c] = fmaxf(hi[c], __shfl_xor(hi[c], o)); }
+            }
+            const float dx = hi[0] - lo[0], dy = hi[1] - lo[1], dz = hi[2] - lo[2];
+            if (lo[0] <= hi[0]) far = fmaxf(far, __builtin_sqrtf(dx * dx + dy * dy + dz * dz));
+            far += bad;
+        }
+        return far;
+    }
+};
 
 __global__ __launch_bounds__(256)
 void we_aniso_grid_tables_kernel(const float* __restrict__ cb_magnitudes, const float* __restrict__ wavenumbers,
@@ -98,18 +116,42 @@ void we_aniso_grid_tables_kernel(const float* __restrict__ cb_magnitudes, const 
 {
     const WgLayout L = wg_layout(Z, N, K, true);
     const int tid = threadIdx.x, lane = tid & 63;
-    const float inv_h = wg_cells_per_length(wavenumbers, K);
-    const double h = 1.0 / (double)inv_h;
-
-    float b2 = 0.f, hi = -3.0e38f, lo = -3.0e38f;                       // lo: largest of -cb
-    for (int i = tid; i < Z * L.blocks; i += 256) b2 = fmaxf(b2, reinterpret_cast<const float*>(ws + L.lengths)[i]);
+    // Everything that needs no other answer meets in one reduction, the first values of every list loaded before any of them is
+    // looked at: a list after the other cost a trip to memory each (8192 tokens with equal scales: this launch 5.8 us, 8.3 so and with
+    // the tiles below for a single grid, which has no use for them).
+    const float* lengths = reinterpret_cast<const float*>(ws + L.lengths);
+    const int* counts = reinterpret_cast<const int*>(ws + L.counts);
+    const bool first = blockIdx.x == 0;                                 // the block that estimates
+    WaBoxes boxes;
+    if (first) boxes.fetch(reinterpret_cast<const WgBox*>(ws + L.boxes), Z, L.nbox);
+    int n0 = first && tid < Z ? counts[tid] : 0;
+    float b2 = tid < Z * L.blocks ? lengths[tid] : 0.f;
+    float hi = -3.0e38f, lo = -3.0e38f, km = 0.f;                       // lo: largest of -cb
     bool bad = false;
-    for (int k = tid; k < K; k += 256) { const float c = cb_magnitudes[k]; bad |= !(fabsf(c) < 1.0e18f); hi = fmaxf(hi, c); lo = fmaxf(lo, -c); }
-    float most_of[3] = {bad ? __builtin_inff() : b2, hi, lo};
-    wg_block_reduce<0>(most_of);
-    const float mid = 0.5f * (most_of[1] - most_of[2]), b = __builtin_sqrtf(most_of[0]) * 1.0001f;
-    float z = 0.f;
-    for (int k = tid; k < K; k += 256) z = fmaxf(z, fabsf(wavenumbers[k] * (cb_magnitudes[k] - mid)));
+    const float c0 = tid < K ? cb_magnitudes[tid] : 0.f, w0 = tid < K ? wavenumbers[tid] : 0.f;
+    for (int k = tid; k < K; k += 256) {
+        const float c = k == tid ? c0 : cb_magnitudes[k], w = fabsf(k == tid ? w0 : wavenumbers[k]);
+        bad |= !(fabsf(c) < 1.0e18f);
+        hi = fmaxf(hi, c); lo = fmaxf(lo, -c); km = fmaxf(km, w < 3.0e38f ? w : __builtin_inff());
+    }
+    for (int i = tid + 256; i < Z * L.blocks; i += 256) b2 = fmaxf(b2, lengths[i]);
+    float pairs = 0.f, nmax = 0.f, groups = 0.f, extent = 0.f;
+    if (first) {
+        for (int i = tid; i < Z; i += 256) {
+            if (i > tid) n0 = counts[i];
+            const float n = (float)n0;
+            pairs += n * n; nmax = fmaxf(nmax, n); groups += __builtin_ceilf(n / WG_OBS);
+        }
+        extent = boxes.longest() * (1.0f / WG_UNIT);
+    }
+    float all[8] = {pairs, groups, km, bad ? __builtin_inff() : b2, hi, lo, nmax, extent};
+    wg_block_reduce<2>(all);
+    pairs = all[0]; groups = all[1]; nmax = all[6]; extent = all[7];
+    const float inv_h = wg_cells_per_length(all[2]);
+    const double h = 1.0 / (double)inv_h;
+    const float mid = 0.5f * (all[4] - all[5]), b = __builtin_sqrtf(all[3]) * 1.0001f;
+    float z = tid < K ? fabsf(w0 * (c0 - mid)) : 0.f;
+    for (int k = tid + 256; k < K; k += 256) z = fmaxf(z, fabsf(wavenumbers[k] * (cb_magnitudes[k] - mid)));
     z = wg_block_max(z) * b;
     // number of terms: the tail of the series starts with 2 J_P(z) <= 2 (z/2)^P / P! (at the one wavenumber where z is largest), that of
     // its derivative with J_(P-1)(z)
@@ -118,20 +160,11 @@ void we_aniso_grid_tables_kernel(const float* __restrict__ cb_magnitudes, const 
         terms = wa_terms(z, 3.0e-7f) + partials;
         if (terms > WG_MAX_TERMS) terms = 0;
     }
-    // (The first block's answer is the one that counts: the others only fill tables.)
-    if (terms > 0 && blockIdx.x == 0) {
+    // (The first block answers, the others fill the tables.)
+    if (terms > 0 && first) {
         // The direct kernel or the grids?  Estimated microseconds: the direct kernel takes 0.34 ps per pair and wavenumber with partial
         // derivatives (0.36 to 0.40 where it has few workgroups) and 0.24 without.  A pass over the sources (8 waves, K = 256, 1 x 1000 ... 8 x 2000 tokens, 4 to 12 terms) takes a round
         // of workgroups (two per compute unit) 22 us for its grids and products and 0.059 us per source, down to 0.026 for few workgroups.
-        float pairs = 0.f, nmax = 0.f, groups = 0.f;
-        for (int i = tid; i < Z; i += 256) {
-            const float n = (float)reinterpret_cast<const int*>(ws + L.counts)[i];
-            pairs += n * n; nmax = fmaxf(nmax, n); groups += __builtin_ceilf(n / WG_OBS);
-        }
-        float all[4] = {pairs, groups, nmax, wa_extent(reinterpret_cast<const WgBox*>(ws + L.boxes), Z, L.nbox)};
-        wg_block_reduce<2>(all);
-        pairs = all[0]; groups = all[1]; nmax = all[2];
-        const float extent = all[3] * (1.0f / WG_UNIT);
         const bool  one     = terms == 1;                                // (a single grid: no partial derivatives)
         const int   most    = one ? WgGrid<1>::CELLS : WgGrid<2>::CELLS;
         const float cells   = 0.7f * extent * inv_h;
@@ -146,7 +179,7 @@ void we_aniso_grid_tables_kernel(const float* __restrict__ cb_magnitudes, const 
         float direct = pairs * (float)K * (partials ? (few ? 3.7e-7f : 3.4e-7f) : 2.4e-7f);
         if (one) {
             // A single grid, 60 batches of 1 x 1000 ... 32 x 500 tokens, K = 64 to 256, extents of up to 16 windows.  Grids / direct, us:
-            // 1 x 2000 K = 64 1 window 45 / 172, 4 116 / 180, 7 212 / 179, 13 402 / 179; 1 x 4000 K = 64 5 234 / 350, 9 430 / 353; 1 x 4000 K = 256
+            // 1 x 2000 K = 64 1 window 43 / 172, 4 114 / 180, 7 212 / 179, 13 402 / 179; 1 x 4000 K = 64 5 234 / 350, 9 430 / 353; 1 x 4000 K = 256
             // 10 598 / 1074; 8 x 1000 K = 256 6 387 / 527, 11 742 / 529.  The direct kernel takes 0.086 us per source where its workgroups do not fill the chip.
             grid   = 12.0f + windows * (few ? 10.0f + 0.008f * nmax + 0.05f * (float)K
                                             : (6.0f + (0.5f + 0.5f * share) * (0.0118f * nmax + 0.18f * (float)K)) * fmaxf(1.0f, rounds));
@@ -154,19 +187,21 @@ void we_aniso_grid_tables_kernel(const float* __restrict__ cb_magnitudes, const 
         }
         if (!(grid < direct) || !(cells + fabsf(mid) * b * inv_h < (float)(most * WG_MAX_WINDOWS))) terms = 0;
     }
-    const int unit = (int)blockIdx.x * 4 + (tid >> 6);
-    if (unit == 0 && lane == 0) {
+    if (blockIdx.x == 0 && tid == 0) {
         WgParams* p = reinterpret_cast<WgParams*>(ws);
         p->inv_h = inv_h; p->h = (float)h; p->cb_mid = mid; p->b_max = b; p->terms = terms;
     }
     // A tile of 16 wavenumbers takes part in the terms that its own z asks for (at a tenth of the tail above, which only the worst
     // wavenumber of all comes near): 267 -> 251 us at 4 x 1000 tokens, 10 terms, partial derivatives.
-    if (blockIdx.x == 0)
-        for (int t = tid; t < L.nkt; t += 256) {
+    if (blockIdx.x == 0) {
+        for (int t = tid; terms > 1 && t < L.nkt; t += 256) {
             float zt = 0.f;
             for (int k = t * 16; k < min(t * 16 + 16, K); ++k) zt = fmaxf(zt, fabsf(wavenumbers[k] * (cb_magnitudes[k] - mid)));
             reinterpret_cast<int*>(ws + L.tiles)[t] = min(terms, wa_terms(zt * b, 3.0e-8f) + partials);
         }
+        return;
+    }
+    const int unit = ((int)blockIdx.x - 1) * 4 + (tid >> 6);
     const int rows = WG_GROUPS * L.nkt;
     if (unit < rows) { wg_fill_tables(wavenumbers, ws, L, K, h, unit); return; }
     // (2 - delta_p0) J_p and its derivative: four orders of 16 wavenumbers per wave, by the power series in double precision (|z| <= 10)
@@ -526,7 +561,7 @@ extern "C" int proteus_we_aniso_fwd_ws(const float* coordsA, const float* coords
     hipLaunchKernelGGL(we_aniso_grid_sources_kernel, dim3((unsigned)Z * (unsigned)L.blocks), dim3(256), 0, st, coordsA, coordsB, coords_layout, mask, ws, Z, N, K);
     const bool few = wa_few(Z, N, mask != nullptr);
     const unsigned units = (unsigned)((WG_GROUPS + (WG_MAX_TERMS + 3) / 4) * L.nkt);
-    hipLaunchKernelGGL(we_aniso_grid_tables_kernel, dim3((units + 3) / 4), dim3(256), 0, st, cb_magnitudes, wavenumbers, ws, Z, N, K, d_cb ? 1 : 0, few ? 1 : 0);
+    hipLaunchKernelGGL(we_aniso_grid_tables_kernel, dim3((units + 3) / 4 + 1), dim3(256), 0, st, cb_magnitudes, wavenumbers, ws, Z, N, K, d_cb ? 1 : 0, few ? 1 : 0);
     const dim3 grid((N + WG_OBS - 1) / WG_OBS, Z);
     const size_t lds = (size_t)WG_ROWS * WG_OBS * 4;
 #define WA_GO(G_, W_) hipLaunchKernelGGL((we_aniso_grid_kernel<G_, W_>), grid, dim3(W_ * 64), lds, st, (const char*)ws, cb_magnitudes, wavenumbers, out, d_cb, d_k, Z, N, K)

@@ -171,15 +171,20 @@ __device__ __forceinline__ void wg_block_reduce(float (&v)[COUNT])
     }
 }
 
-// Cells per unit of length, rounded to float once: h is its exact inverse from here on.  Wavenumbers beyond any use (wavelengths
-// below 0.11, where the coefficients of the spreading kernel would lose bits as denormals) give an infinite value, which sends
-// every workgroup to the direct sums.
-__device__ __forceinline__ float wg_cells_per_length(const float* __restrict__ wavenumbers, const int K)
+// Largest of a thread's share of the wavenumbers, for the 256 threads of a block; infinite if one of them is not finite.
+__device__ __forceinline__ float wg_largest(const float* __restrict__ wavenumbers, const int K)
 {
     float km = 0.f;
     bool bad = false;
     for (int k = threadIdx.x; k < K; k += 256) { const float w = fabsf(wavenumbers[k]); bad |= !(w < 3.0e38f); km = fmaxf(km, w); }
-    km = wg_block_max(bad ? __builtin_inff() : km);
+    return bad ? __builtin_inff() : km;
+}
+
+// Cells per unit of length for the largest wavenumber, rounded to float once: h is its exact inverse from here on.  Wavenumbers beyond
+// any use (wavelengths below 0.11, where the coefficients of the spreading kernel would lose bits as denormals) give an infinite
+// value, which sends every workgroup to the direct sums.
+__device__ __forceinline__ float wg_cells_per_length(const float km)
+{
     const float inv_h = fmaxf(km * (WG_OVERSAMPLING / 3.14159265f) * 1.000001f, 1.0e-6f);
     return inv_h < 64.0f ? inv_h : __builtin_inff();
 }

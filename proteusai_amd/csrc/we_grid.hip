@@ -41,7 +41,7 @@ void we_grid_prepare_kernel(const float* __restrict__ coords, const int layout, 
         wg_compact(coords, layout, mask, ws, L, N, blockIdx.x);
         return;
     }
-    const float inv_h = wg_cells_per_length(wavenumbers, K);
+    const float inv_h = wg_cells_per_length(wg_block_max(wg_largest(wavenumbers, K)));
     const double h = 1.0 / (double)inv_h;
     const int unit = ((int)blockIdx.x - blocks) * 4 + (threadIdx.x >> 6);
     if (unit == 0 && (threadIdx.x & 63) == 0) { WgParams* p = reinterpret_cast<WgParams*>(ws); p->inv_h = inv_h; p->h = (float)h; }

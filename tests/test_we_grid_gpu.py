@@ -157,6 +157,8 @@ ANISO = {                       # N, Z, K, scale of the chain, spread of the C-b
     "two grids in several windows": (2100, 2, 256, 3.0, 0.02, "scattered"),
     "many pairs too close for a cell": (1300, 3, 256, 0.3, 0.02, None),
     "more terms than pay": (200, 2, 64, 1.0, 1.5, None),
+    "more than 256 wavenumbers": (1500, 1, 300, 1.0, 0.02, None),
+    "more than 256 items of two boxes": (70, 300, 64, 1.0, 0.0, None),
     "equal scales, more than 256 workgroups": (4200, 1, 64, 1.0, 0.0, None),
     "at most 256 workgroups, flushes, tiles of few terms, a tile in part": (2100, 1, 250, 1.0, 0.1, None),
 }
