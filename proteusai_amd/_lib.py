@@ -7,6 +7,8 @@ import ctypes
 import functools
 import os
 
+import torch
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libproteus_hip.so")
 
@@ -225,7 +227,6 @@ def we_aniso_workspace_bytes(Z, N, K, partials, padded, tuning):
 
 def raw_stream(dev):
     """Handle of torch's current stream on `dev` for the `stream` argument of the entry points."""
-    import torch
     try:
         return torch._C._cuda_getCurrentRawStream(dev.index if dev.index is not None else torch.cuda.current_device())
     except AttributeError:       # (a torch without the short cut)
@@ -244,8 +245,7 @@ _NO_SWITCH = _NoSwitch()
 
 
 def on_device(dev):
-    """Context that makes `dev` the current device for the launch; free when it already is."""
-    import torch
-    if dev.index is None or torch.cuda.current_device() == dev.index:
+    """Context that makes `dev`, on which there are tensors, the current device for the launch; free when it already is."""
+    if dev.index is None or torch._C._cuda_getDevice() == dev.index:
         return _NO_SWITCH
     return torch.cuda.device(dev)

@@ -239,8 +239,6 @@ def geo_attn_backward(Q, K, V, O, L, dO, coords, sigma, key_padding_mask=None, b
     grad_dtype: None (fp32) or the operand type, in which dQ, dK, dV are then returned: the same sums, rounded once.
     """
     Z, H, N, _ = Q.shape
-    if not Q.is_cuda or not (Q.get_device() == K.get_device() == V.get_device() == O.get_device() == dO.get_device()):
-        raise _lib.ProteusError("geo_attn_backward needs tensors on the GPU, all on one (there is no CPU path)")
     if not (Q.shape == K.shape == V.shape == O.shape == dO.shape) or L.numel() != Z * H * N:
         raise AssertionError(f"Q, K, V, O and dO must have one shape and L an element per row, but got {Q.shape=}, {K.shape=}, {V.shape=}, "
                              f"{O.shape=}, {dO.shape=}, {L.shape=}")
@@ -248,8 +246,10 @@ def geo_attn_backward(Q, K, V, O, L, dO, coords, sigma, key_padding_mask=None, b
 
 
 def _backward(Q, K, V, O, L, dO, coords, sigma, key_padding_mask, betas, min_rbf, max_rbf, operand_dtype, grads=None, grad_dtype=None):
-    """geo_attn_backward on tensors that are known to go together (the forward's own, and a gradient from autograd)."""
+    """geo_attn_backward on tensors whose shapes are known to go together (the forward's own, and a gradient from autograd)."""
     Z, H, N, d = Q.shape
+    if not Q.is_cuda or not (Q.get_device() == K.get_device() == V.get_device() == O.get_device() == dO.get_device()):
+        raise _lib.ProteusError("geo_attn_backward needs tensors on the GPU, all on one (there is no CPU path)")
     lib = _lib.load()
     dev = Q.device
     op_dtype, op_type = _operand_type(operand_dtype, betas is not None)

@@ -23,9 +23,11 @@ def recording(*tensors):
     if not torch.is_grad_enabled() or torch.is_autocast_enabled("cuda"):
         return False
     needed = False
-    dev = tensors[0].device
+    dev = tensors[0].get_device()
+    if not tensors[0].is_cuda:
+        return False
     for t in tensors:
-        if type(t) not in _PLAIN_TYPES or t.dtype != torch.float32 or not t.is_cuda or t.device != dev or t.layout != torch.strided:
+        if type(t) not in _PLAIN_TYPES or t.dtype != torch.float32 or t.get_device() != dev or t.layout != torch.strided:
             return False
         needed = needed or t.requires_grad
     # (a dispatch mode, e.g. make_fx's, sees the torch operators only: a graph traced past a kernel would not hold what it writes)
@@ -56,6 +58,12 @@ def _call(fn, dev, *args):
     _lib.check(rc, fn)
 
 
+@functools.lru_cache(maxsize=1024)
+def _bytes(fn, *sizes):
+    """What the library answers for a workspace's size, kept per sizes."""
+    return getattr(_lib.load(), fn)(*sizes)
+
+
 def _workspace(nbytes, dev):
     return torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
 
@@ -73,12 +81,12 @@ def _by_expression(d):
             or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() > 0)
 
 
-def _saved(t, shape, dtype=torch.float32):
+def _saved(t, numel, dtype=torch.float32):
     """A saved tensor as a kernel may read it.  What saved-tensor hooks give back may lie differently (strides, alignment); another
-    type or shape is an error, as it would be in a torch operator."""
-    if t.dtype != dtype or tuple(t.shape) != tuple(shape):
-        raise RuntimeError(f"a tensor saved as {dtype} {tuple(shape)} came back as {t.dtype} {tuple(t.shape)}")
-    return _dense(t)
+    type, size or place is an error, as it would be in a torch operator."""
+    if t.dtype != dtype or t.numel() != numel or not t.is_cuda:
+        raise RuntimeError(f"a tensor of {numel} {dtype} that was saved on the GPU came back as {tuple(t.shape)} of {t.dtype} on {t.device}")
+    return t if t.is_contiguous() and t.data_ptr() % 16 == 0 else _dense(t)
 
 
 def _without_autocast(backward):
@@ -108,7 +116,7 @@ def column_sums(a, h=None):
     rows, C = a.shape
     sums = torch.empty(C, dtype=torch.float32, device=a.device)
     dh = None if h is None else torch.empty_like(h)
-    n = _lib.load().proteus_train_workspace_bytes(rows, C)
+    n = _bytes("proteus_train_workspace_bytes", rows, C)
     _call("proteus_colsum", a.device, a, h, dh, sums, _workspace(n, a.device), n, rows, C)
     return sums if h is None else (dh, sums)
 
@@ -142,13 +150,12 @@ class _AddLayerNorm(torch.autograd.Function):
         if _by_expression(d):
             dx, dw, db = _recorded(lambda y_, w_, b_: F.layer_norm(y_, (w.numel(),), w_, b_, ctx.eps), (ysum, w, b), (True, need[2], need[3]), d)
         else:
-            D = d.shape[-1]
+            d, D = _dense(d), d.shape[-1]
             rows = d.numel() // D
-            d, w = _dense(d), _saved(w, (D,))
-            ysum, stat = _saved(ysum, d.shape), _saved(stat, (rows, 2))
+            w, ysum, stat = _saved(w, D), _saved(ysum, rows * D), _saved(stat, 2 * rows)
             dx = torch.empty_like(ysum)
             dwb = torch.empty(2, D, dtype=torch.float32, device=d.device)
-            n = _lib.load().proteus_layernorm_bwd_workspace_bytes(rows, D)
+            n = _bytes("proteus_layernorm_bwd_workspace_bytes", rows, D)
             _call("proteus_layernorm_bwd", d.device, d, ysum, stat, w, dx, dwb, _workspace(n, d.device), n, rows, D)
             dw, db = dwb[0] if need[2] else None, dwb[1] if need[3] else None
         if dy is not None:
@@ -177,8 +184,8 @@ class _GeluMLP(torch.autograd.Function):
         h = torch.addmm(b1, x2, w1.t())
         a = F.gelu(h)
         ctx.save_for_backward(x, w1, b1, w2, b2, h, a)
-        # (not a view: what is changed in place behind the feed-forward must not be one)
-        return torch.ops.aten._unsafe_view(torch.addmm(b2, a, w2.t()), (*x.shape[:-1], w2.shape[0]))
+        # (resized, not viewed: autograd lets no view that a function returns be changed in place)
+        return torch.addmm(b2, a, w2.t()).resize_(*x.shape[:-1], w2.shape[0])
 
     @staticmethod
     @_without_autocast
@@ -194,7 +201,7 @@ class _GeluMLP(torch.autograd.Function):
         dx = dw1 = db1 = None
         if need[0] or need[1] or need[2]:
             da = d2.mm(w2)
-            dh, db1 = column_sums(da, _saved(h, da.shape))
+            dh, db1 = column_sums(da, _saved(h, da.numel()))
             dw1 = dh.t().mm(x2) if need[1] else None
             dx = dh.mm(w1).view(x.shape) if need[0] else None
         return dx, dw1, db1 if need[2] else None, dw2, db2
@@ -250,7 +257,7 @@ class _SelfAttention(torch.autograd.Function):
         W = torch.empty(dm, 3 * dm, dtype=torch.float32, device=dev)
         Wo = torch.empty(dm, dm, dtype=torch.float32, device=dev)
         b = torch.empty(3 * dm, dtype=torch.float32, device=dev)
-        sigma, spread = torch.empty(2, H, dtype=torch.float32, device=dev)
+        sigma, spread = torch.empty(H, dtype=torch.float32, device=dev), torch.empty(H, dtype=torch.float32, device=dev)
         _layout((qw, kw, vw, qb, kb, vb, spread, wo), W, b, Wo, sigma, spread_w, dm, H, dk, min_spread, 0)
         qkv = torch.addmm(b, _dense(x).view(Z * N, dm), W).to(operand_dtype or torch.bfloat16).view(Z, N, 3, H, dk)
         O, L = ga.geo_attn(*_heads(qkv), coords, sigma, mask, return_lse=True, check_sigma=False, token_major_out=True,
@@ -261,7 +268,7 @@ class _SelfAttention(torch.autograd.Function):
         ctx.params = (qw, kw, vw, qb, kb, vb, spread_w, wo)
         ctx.versions = [p._version for p in ctx.params]
         ctx.min_spread, ctx.operand_dtype = min_spread, operand_dtype
-        return torch.ops.aten._unsafe_view(O.permute(0, 2, 1, 3).reshape(Z * N, dm).mm(Wo.t()), (Z, N, dm))      # (not a view, as in the feed-forward)
+        return O.permute(0, 2, 1, 3).reshape(Z * N, dm).mm(Wo.t()).resize_(Z, N, dm)       # (as in the feed-forward)
 
     @staticmethod
     @_without_autocast
@@ -287,7 +294,7 @@ class _SelfAttention(torch.autograd.Function):
         dW = _dense(x).view(Z * N, dm).t().mm(g2) if any(need[3:6]) else g2
         db = column_sums(g2) if any(need[6:9]) else g2
         dWo = d2.t().mm(O.permute(0, 2, 1, 3).reshape(Z * N, dm)) if need[10] else g2
-        _layout(grads, dW, db, dWo, d_sigma, _saved(spread, (H,)), dm, H, dk, ctx.min_spread, 1)
+        _layout(grads, dW, db, dWo, d_sigma, _saved(spread, H), dm, H, dk, ctx.min_spread, 1)
         return (dx, None, None, *grads, None, None)
 
 
@@ -302,7 +309,7 @@ def self_attention(x, coords, mask, m):
             and params[6].shape == (H,) and params[7].shape == (dm, dm)):
         return None
     # (frozen projections keep the expression, which does not keep x: x may be changed in place behind it)
-    if (not any(p.requires_grad for p in params[:3]) or m.legacy_logits or dk not in (32, 64, 128) or dm > 16384 or x.numel() == 0 or not coords.is_cuda or coords.requires_grad or type(coords) not in _PLAIN_TYPES
+    if (not (params[0].requires_grad or params[1].requires_grad or params[2].requires_grad) or m.legacy_logits or dk not in (32, 64, 128) or dm > 16384 or x.numel() == 0 or not coords.is_cuda or coords.requires_grad or type(coords) not in _PLAIN_TYPES
             or (mask is not None and type(mask) is not torch.Tensor)
             or x.shape[1] * 3 * dm * 4 >= 2 ** 31 or m.operand_dtype not in (None, torch.bfloat16)
             or type(m).get_spreads is not ga.GeoAttention.get_spreads or "get_spreads" in m.__dict__ or not isinstance(m.min_spread, (int, float))
@@ -326,9 +333,9 @@ class _SmallEmbedding(torch.autograd.Function):
         if _by_expression(d):
             return (*_recorded(lambda w: F.embedding(tokens, w), (weight,), (True,), d), None)
         V, D = weight.shape
-        d, t = _dense(d), _saved(tokens, d.shape[:-1], torch.int64)
+        d, t = _dense(d), _saved(tokens, d.numel() // D, torch.int64)
         dW = torch.empty(V, D, dtype=torch.float32, device=d.device)
-        n = _lib.load().proteus_embedding_bwd_workspace_bytes(t.numel(), V, D)
+        n = _bytes("proteus_embedding_bwd_workspace_bytes", t.numel(), V, D)
         _call("proteus_embedding_bwd", d.device, d, t, dW, _workspace(n, d.device), n, t.numel(), V, D)
         return dW, None
 

@@ -282,10 +282,11 @@ def test_saved_tensors_of_another_type_are_refused(gpu):
     layer, emb, tokens, coords = _layer_and_inputs(gpu)
     x = torch.randn(1, 33, 64, device=gpu, requires_grad=True)
     for f in (lambda: train_ops.embedding(tokens, emb), lambda: layer.ffn(x), lambda: train_ops.add_layer_norm(x, x, layer.ffn_norm)):
-        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t.to(torch.int32 if t.dtype == torch.int64 else torch.bfloat16)):
-            out = f()
-        with pytest.raises(RuntimeError):
-            out.sum().backward()
+        for unpack in (lambda t: t.to(torch.int32 if t.dtype == torch.int64 else torch.bfloat16), lambda t: t.cpu()):
+            with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+                out = f()
+            with pytest.raises(RuntimeError):
+                out.sum().backward()
 
 
 def test_outputs_may_be_changed_in_place(gpu):
