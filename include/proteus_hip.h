@@ -66,7 +66,7 @@ extern "C" {
  * backward entry point take `int operand_type` before `tuning` / `stream`; a caller built against an older header
  * would pass its tuning selector there).  The Python binding checks for an exact match when it loads the library.
  */
-#define PROTEUS_VERSION 305
+#define PROTEUS_VERSION 306
 int proteus_version(void);
 
 /* Human-readable text for a return code of any entry point. */
@@ -547,6 +547,25 @@ int proteus_colsum(const float* a, const float* h, float* dh, float* sums, void*
 int proteus_heads_layout(float* const* tensors, float* W, float* b, float* Wo, float* sigma, const float* spread_w,
                          int d_model, int H, int d_head, float min_spread, int backward, void* stream);
 int proteus_embedding_bwd(const float* dout, const int64_t* tokens, float* dW, void* ws, size_t ws_bytes, long T, int V, int D, void* stream);
+
+/*
+ * C = op(A) op(B) (+ bias [N], added to every row) in fp32 for the encoder's training step: fp32 operands, fp32 sums (each operand as
+ * three bf16 pieces on the matrix cores; error at or below that of fp32 sums), the same bits on every call.
+ *   form      PROTEUS_GEMM_NN: A [M][K], B [K][N];  _NT: A [M][K], B [N][K];  _TN: A [K][M], B [K][N]; rows lda, ldb, ldc elements apart.
+ *             A matrix whose rows run along K (A in NN and NT, B in NT): K and its ld multiples of 4
+ *   epilogue  PROTEUS_GEMM_F32: C f32;  _BF16: C bf16, rounded once;  _GELU: H = the sums f32, C = gelu(H) f32;
+ *             _GELU_GRAD: C = sums * gelu'(h) f32 (exact GELU; H and h laid out as C)
+ *   A, B, C 16-byte aligned; bias, h, H may be NULL where not asked for.  One launch, no workspace.
+ */
+#define PROTEUS_GEMM_NN 0
+#define PROTEUS_GEMM_NT 1
+#define PROTEUS_GEMM_TN 2
+#define PROTEUS_GEMM_F32       0
+#define PROTEUS_GEMM_BF16      1
+#define PROTEUS_GEMM_GELU      2
+#define PROTEUS_GEMM_GELU_GRAD 3
+int proteus_gemm_f32(const float* A, const float* B, const float* bias, const float* h, void* C, float* H,
+                     int M, int N, int K, int lda, int ldb, int ldc, int form, int epilogue, void* stream);
 
 #ifdef __cplusplus
 }

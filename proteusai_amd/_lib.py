@@ -14,9 +14,11 @@ LIB_PATH = os.path.join(HERE, "libproteus_hip.so")
 
 COORDS_SOA = 0
 COORDS_AOS = 1
-ABI_VERSION = 305                    # PROTEUS_VERSION of the include/proteus_hip.h these argument lists were written from
+ABI_VERSION = 306                    # PROTEUS_VERSION of the include/proteus_hip.h these argument lists were written from
 OPERAND_BF16, OPERAND_F16 = 0, 1     # PROTEUS_OPERAND_* of include/proteus_hip.h
 GRAD_F32, GRAD_OPERAND = 0, 1        # PROTEUS_GRAD_*
+GEMM_NN, GEMM_NT, GEMM_TN = 0, 1, 2  # PROTEUS_GEMM_*: form
+GEMM_F32, GEMM_BF16, GEMM_GELU, GEMM_GELU_GRAD = 0, 1, 2, 3      # and epilogue
 DTYPE_F32, DTYPE_BF16, DTYPE_F16 = 0, 1, 2   # PROTEUS_DTYPE_*
 
 # every symbol include/proteus_hip.h declares
@@ -35,7 +37,7 @@ SYMBOLS = [
     "proteus_geo_attn_variant_name",
     "proteus_add_layernorm_fwd", "proteus_add_layernorm_fwd_check", "proteus_geo_attn_delta", "proteus_geo_attn_delta_check",
     "proteus_train_workspace_bytes", "proteus_layernorm_bwd_workspace_bytes", "proteus_embedding_bwd_workspace_bytes",
-    "proteus_add_layernorm_train_fwd", "proteus_layernorm_bwd", "proteus_colsum", "proteus_heads_layout", "proteus_embedding_bwd",
+    "proteus_add_layernorm_train_fwd", "proteus_layernorm_bwd", "proteus_colsum", "proteus_heads_layout", "proteus_embedding_bwd", "proteus_gemm_f32",
 ]
 
 _lib = None
@@ -169,6 +171,8 @@ def load():
     lib.proteus_heads_layout.argtypes = [ctypes.POINTER(vp)] + [vp] * 5 + [ci, ci, ci, cf, ci, vp]
     lib.proteus_embedding_bwd.restype = ci
     lib.proteus_embedding_bwd.argtypes = [vp] * 4 + [sz, cl, ci, ci, vp]
+    lib.proteus_gemm_f32.restype = ci
+    lib.proteus_gemm_f32.argtypes = [vp] * 6 + [ci] * 8 + [vp]
     _lib = lib
     return lib
 

@@ -1,0 +1,264 @@
+// Matrix products of the encoder's training step: fp32 in, fp32 sums, on the 16-bit matrix cores of gfx950.
+//
+// An fp32 number is the sum of three bf16 numbers (8 + 8 + 8 bits, each piece rounded to nearest: the third takes what is
+// left exactly).  Of the nine products of pieces the six largest are taken, x0 y0, x0 y1, x1 y0, x1 y1, x0 y2, x2 y0: what is left out
+// is below 2^-26 of |x y|, under the rounding of one fp32 addition.  Six v_mfma_f32_32x32x16_bf16 cost 192 clocks where the same
+// product on v_mfma_f32_32x32x2_f32 takes 512, and their fp32 accumulator rounds once per 16 products instead of once per 2.
+//
+// A workgroup makes one 64 x 64 tile of C.  Four waves (a group) hold 32 x 32 of it each and step through K by 16; where the tiles
+// are too few to fill the chip, 2 or 4 groups share a tile, each with its own steps and its own LDS stages, and add up at the end
+// in a fixed order (the same bits on every call).  A step: 8 floats per thread travel global -> registers two steps ahead, are
+// split (5.5 vector instructions each) and written to one of two stages as 16-byte fragments, eight consecutive k of one row; the
+// product reads them with ds_read_b128.  Odd groups split and then multiply, even ones the other way round, so that the matrix
+// cores of a SIMD have work while the other half of its waves split.  A bound of its own: a 64 x 64 x 16 step reads 24 KB
+// and writes 12 KB of LDS (288 clocks at 128 bytes a clock) beside 192 clocks of products and about 200 of splitting.
+//
+// Values that are not finite (or become so: bf16 ends half a step below fp32) do not split; an element of C that comes out not
+// finite is summed again in plain fp32.
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+#include "proteus_hip.h"
+
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float  f32x2  __attribute__((ext_vector_type(2)));
+typedef float  f32x16 __attribute__((ext_vector_type(16)));
+
+constexpr int GT        = 64;                       // rows and columns of a tile
+constexpr int GK        = 16;                       // k of a step
+constexpr int CHUNK     = GT * 16 + 64;             // bytes of 8 k of all rows of one piece (64 more: the two halves of a step in different banks)
+constexpr int PIECE     = 2 * CHUNK;
+constexpr int OPERAND   = 3 * PIECE;
+constexpr int STAGE     = 2 * OPERAND;              // of one group
+
+struct GemmArgs {
+    const float *A, *B, *bias, *h;
+    void  *C;
+    float *H;
+    int M, N, K, lda, ldb, ldc, tiles_n, tiles, per_xcd;
+};
+
+__device__ __forceinline__ uint32_t pack2(const float a, const float b) {
+    const f32x2 f = {a, b};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2));
+}
+__device__ __forceinline__ float low(const uint32_t w)  { return __builtin_bit_cast(float, w << 16); }
+__device__ __forceinline__ float high(const uint32_t w) { return __builtin_bit_cast(float, w & 0xffff0000u); }
+
+// Four consecutive k of one row into the three pieces' fragments.
+__device__ __forceinline__ void split_to_lds(char* at, const float4& v)
+{
+    uint2 p;
+    p.x = pack2(v.x, v.y); p.y = pack2(v.z, v.w);
+    *reinterpret_cast<uint2*>(at) = p;
+    const float a = v.x - low(p.x), b = v.y - high(p.x), c = v.z - low(p.y), d = v.w - high(p.y);
+    p.x = pack2(a, b); p.y = pack2(c, d);
+    *reinterpret_cast<uint2*>(at + PIECE) = p;
+    p.x = pack2(a - low(p.x), b - high(p.x)); p.y = pack2(c - low(p.y), d - high(p.y));
+    *reinterpret_cast<uint2*>(at + 2 * PIECE) = p;
+}
+
+// A thread's share of an operand: four consecutive k of one row (of A, or of B^T) per step.  KC: k is the contiguous dimension in memory,
+// else the row is.  Loads are unconditional (so that they stay in flight over the branches of the step): what lies outside the matrix
+// is out of the buffer's range and comes back as zero.
+template <bool KC> struct Source {
+    static constexpr uint32_t OUT = 0x80000000u;               // (matrices end below 2^31 bytes)
+    __amdgpu_buffer_rsrc_t rsrc;
+    uint32_t at;                                               // of the thread's row at k = 0
+    int k, K, pitch;
+    __device__ __forceinline__ Source(const float* X, const int ld, const int row, const int rows, const int k_, const int K_)
+        : rsrc(__builtin_amdgcn_make_buffer_rsrc((void*)X, 0, (uint32_t)((KC ? (size_t)(rows - 1) * ld + K_ : (size_t)(K_ - 1) * ld + rows) * 4), 0x00020000)),
+          at(row < rows ? (KC ? (uint32_t)row * (uint32_t)ld * 4u : (uint32_t)row * 4u) : OUT), k(k_), K(K_), pitch(ld * 4) {}
+    __device__ __forceinline__ float4 fetch(const int k0) const
+    {
+        if (KC) return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, k0 + k < K ? at + (uint32_t)(k0 + k) * 4u : OUT, 0, 0));     // (K is a multiple of 4)
+        const uint32_t o = at + (uint32_t)(k0 + k) * (uint32_t)pitch;          // (rows of k past K lie behind the end)
+        auto one = [&](const int i) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, at < OUT ? o + (uint32_t)(i * pitch) : OUT, 0, 0)); };
+        return make_float4(one(0), one(1), one(2), one(3));
+    }
+};
+
+// Barrier for LDS alone: loads from memory stay in flight.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); __builtin_amdgcn_s_barrier(); asm volatile("" ::: "memory"); }
+
+// One element of A B in plain fp32.
+template <bool AK, bool BK>
+__device__ __forceinline__ float plain_dot(const GemmArgs& g, const int m, const int n)
+{
+    float s = 0.f;
+    for (int k = 0; k < g.K; ++k)
+        s = __builtin_fmaf(AK ? g.A[(size_t)m * g.lda + k] : g.A[(size_t)k * g.lda + m], BK ? g.B[(size_t)n * g.ldb + k] : g.B[(size_t)k * g.ldb + n], s);
+    return s;
+}
+
+__device__ __forceinline__ float gelu(const float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
+__device__ __forceinline__ float gelu_grad(const float x) {
+    const float cdf = 0.5f * (1.0f + erff(x * 0.70710678118654752f));
+    return __builtin_fmaf(x, 0.39894228040143268f * expf(-0.5f * x * x), cdf);
+}
+
+// AK, BK: k contiguous in A [M][K] / B [N][K]; else A is [K][M] / B [K][N]
+template <bool AK, bool BK, int G, int EPI>
+__global__ __launch_bounds__(G * 256, 4)
+void gemm_f32_kernel(const GemmArgs g)
+{
+    extern __shared__ __align__(16) char lds[];               // [G][2 stages]; at the end [G][4 waves][16][64] sums
+    const int tile = (blockIdx.x & 7) * g.per_xcd + (blockIdx.x >> 3);      // consecutive tiles (of the same rows of A) on one XCD
+    if ((int)(blockIdx.x >> 3) >= g.per_xcd || tile >= g.tiles) return;
+    const int m0 = tile / g.tiles_n * GT, n0 = tile % g.tiles_n * GT;
+    const int t = threadIdx.x & 255, lane = t & 63;
+    const int group = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    char* const mine = lds + group * 2 * STAGE;
+
+    // what the thread fetches of a step: four k of one row of either operand
+    const int ra = AK ? t >> 2 : t & 63, ka = (AK ? t & 3 : t >> 6) * 4;
+    const int rb = BK ? t >> 2 : t & 63, kb = (BK ? t & 3 : t >> 6) * 4;
+    char* const wa = mine + (ka >> 3) * CHUNK + ra * 16 + (ka & 4) * 2;
+    char* const wb = mine + OPERAND + (kb >> 3) * CHUNK + rb * 16 + (kb & 4) * 2;
+    // and the fragments its wave reads
+    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+    const char* const fa = mine + (lane >> 5) * CHUNK + (wm + (lane & 31)) * 16;
+    const char* const fb = mine + OPERAND + (lane >> 5) * CHUNK + (wn + (lane & 31)) * 16;
+
+    const int rounds = ((g.K + GK - 1) / GK + 2 * G - 1) / (2 * G) * 2;       // (an even number; steps past the end are zeros)
+    const Source<AK> sa(g.A, g.lda, m0 + ra, g.M, ka, g.K);
+    const Source<BK> sb(g.B, g.ldb, n0 + rb, g.N, kb, g.K);
+    float4 va[2], vb[2];
+    auto load = [&](const int round, const int slot) {
+        const int k = (round * G + group) * GK;
+        va[slot] = sa.fetch(k);
+        vb[slot] = sb.fetch(k);
+    };
+    auto store = [&](const int slot) { split_to_lds(wa + slot * STAGE, va[slot]); split_to_lds(wb + slot * STAGE, vb[slot]); };
+    f32x16 acc = {};
+    auto multiply = [&](const int slot) {
+        bf16x8 a[3], b[3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+            a[p] = *reinterpret_cast<const bf16x8*>(fa + slot * STAGE + p * PIECE);
+            b[p] = *reinterpret_cast<const bf16x8*>(fb + slot * STAGE + p * PIECE);
+        }
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2], b[0], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[2], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[1], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[0], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[1], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[0], acc, 0, 0, 0);
+    };
+    load(0, 0);
+    load(1, 1);
+    store(0);
+    auto step = [&](const int round, const int s) {
+        // stage s of this round is written, stage 1 - s (of the round before) is read
+        lds_barrier();
+        load(round + 2, s);
+        if (group & 1) { store(1 - s); multiply(s); }
+        else           { multiply(s); store(1 - s); }
+    };
+    for (int r = 0; r < rounds; r += 2) {
+        step(r, 0);
+        step(r + 1, 1);
+    }
+
+    // ---- the groups' sums together: group i takes every G-th quad of accumulators of every wave ----
+    if (G > 1) {
+        float* const red = reinterpret_cast<float*>(lds);
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 16; ++i) red[((group * 4 + wave) * 16 + i) * 64 + lane] = acc[i];
+        __syncthreads();
+    }
+    const int n = n0 + wn + (lane & 31);
+    const float bias = g.bias && n < g.N ? g.bias[n] : 0.f;
+    auto finish = [&](const int m, float v) {
+        v += bias;
+        const size_t at = (size_t)m * g.ldc + n;
+        if (EPI == PROTEUS_GEMM_F32)        static_cast<float*>(g.C)[at] = v;
+        else if (EPI == PROTEUS_GEMM_BF16)  static_cast<__bf16*>(g.C)[at] = (__bf16)v;
+        else if (EPI == PROTEUS_GEMM_GELU)  { g.H[at] = v; static_cast<float*>(g.C)[at] = gelu(v); }
+        else                                static_cast<float*>(g.C)[at] = v * gelu_grad(g.h[at]);
+    };
+    uint32_t again = 0;                                        // of the lane's 16 elements those that are not finite
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        if (G > 1 && (q % G) != group) continue;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float v;
+            if (G == 1) v = acc[q * 4 + i];
+            else {
+                const float* red = reinterpret_cast<const float*>(lds) + (wave * 16 + q * 4 + i) * 64 + lane;
+                v = red[0];
+#pragma unroll
+                for (int o = 1; o < G; ++o) v += red[o * 4 * 16 * 64];
+            }
+            const int m = m0 + wm + 8 * q + 4 * (lane >> 5) + i;
+            if (m >= g.M || n >= g.N) continue;
+            if (fabsf(v) <= 3.4028234e38f) finish(m, v);
+            else again |= 1u << (q * 4 + i);
+        }
+    }
+    for (; again; again &= again - 1) {
+        const int e = __builtin_ctz(again), m = m0 + wm + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
+        finish(m, plain_dot<AK, BK>(g, m, n));
+    }
+}
+
+template <bool AK, bool BK, int EPI>
+int gemm_go(GemmArgs g, hipStream_t st)
+{
+    const int tm = (g.M + GT - 1) / GT;
+    g.tiles_n = (g.N + GT - 1) / GT;
+    g.tiles   = tm * g.tiles_n;
+    g.per_xcd = (g.tiles + 7) / 8;
+    const dim3 grid((unsigned)g.per_xcd * 8);
+    // Groups per tile: four waves per SIMD where the tiles allow.
+#define GO(G_) do { \
+        constexpr size_t sums = (G_) > 1 ? (size_t)(G_) * 4 * 16 * 64 * 4 : 0; \
+        hipLaunchKernelGGL((gemm_f32_kernel<AK, BK, G_, EPI>), grid, dim3(G_ * 256), G_ * 2 * STAGE > sums ? G_ * 2 * STAGE : sums, st, g); \
+    } while (0)
+    if (g.tiles > 640)      GO(1);
+    else if (g.tiles > 320) GO(2);
+    else                    GO(4);
+#undef GO
+    return (int)hipGetLastError();
+}
+
+bool off16(const void* p) { return ((uintptr_t)p & 15) != 0; }
+
+}  // namespace
+
+extern "C" int proteus_gemm_f32(const float* A, const float* B, const float* bias, const float* h, void* C, float* H,
+                                int M, int N, int K, int lda, int ldb, int ldc, int form, int epilogue, void* stream)
+{
+    if (!A || !B || !C || (epilogue == PROTEUS_GEMM_GELU && !H) || (epilogue == PROTEUS_GEMM_GELU_GRAD && !h)) return PROTEUS_ERR_NULL_POINTER;
+    if (form < 0 || form > PROTEUS_GEMM_TN || epilogue < 0 || epilogue > PROTEUS_GEMM_GELU_GRAD) return PROTEUS_ERR_UNSUPPORTED;
+    if (M <= 0 || N <= 0 || K <= 0 || ldc < N || lda < (form == PROTEUS_GEMM_TN ? M : K) || ldb < (form == PROTEUS_GEMM_NT ? K : N)) return PROTEUS_ERR_BAD_SHAPE;
+    // (tiles are numbered in 32 bits)
+    if ((int64_t)((M + (int64_t)GT - 1) / GT) * ((N + (int64_t)GT - 1) / GT) > (1 << 30)) return PROTEUS_ERR_TOO_LARGE;
+    // (buffer offsets, those of the steps past the end among them)
+    const int64_t bytes_a = ((int64_t)(form == PROTEUS_GEMM_TN ? K : M) + 512) * lda * 4, bytes_b = ((int64_t)(form == PROTEUS_GEMM_NT ? N : K) + 512) * ldb * 4;
+    if (bytes_a >= (1LL << 31) || bytes_b >= (1LL << 31)) return PROTEUS_ERR_TOO_LARGE;
+    // rows that are read 16 bytes at a time
+    if (off16(A) || off16(B) || off16(C)) return PROTEUS_ERR_BAD_ALIGNMENT;
+    if (form != PROTEUS_GEMM_TN && (K % 4 || lda % 4)) return PROTEUS_ERR_BAD_SHAPE;
+    if (form == PROTEUS_GEMM_NT && ldb % 4) return PROTEUS_ERR_BAD_SHAPE;
+    const GemmArgs g = {A, B, bias, h, C, H, M, N, K, lda, ldb, ldc, 0, 0, 0};
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+#define EPILOGUES(AK_, BK_) \
+    switch (epilogue) { \
+        case PROTEUS_GEMM_F32:  return gemm_go<AK_, BK_, PROTEUS_GEMM_F32>(g, st); \
+        case PROTEUS_GEMM_BF16: return gemm_go<AK_, BK_, PROTEUS_GEMM_BF16>(g, st); \
+        case PROTEUS_GEMM_GELU: return gemm_go<AK_, BK_, PROTEUS_GEMM_GELU>(g, st); \
+        default:                return gemm_go<AK_, BK_, PROTEUS_GEMM_GELU_GRAD>(g, st); \
+    }
+    switch (form) {
+        case PROTEUS_GEMM_NN: EPILOGUES(true, false)
+        case PROTEUS_GEMM_NT: EPILOGUES(true, true)
+        default:              EPILOGUES(false, false)
+    }
+#undef EPILOGUES
+}

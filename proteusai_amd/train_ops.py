@@ -111,14 +111,37 @@ def _recorded(expr, inputs, needs, grad):
     return tuple(next(got) if n else None for n in needs)
 
 
-def column_sums(a, h=None):
-    """Column sums of a [rows, C]; with h (dh, its column sums) of dh = a * gelu'(h)."""
+def column_sums(a):
+    """Column sums of a [rows, C]."""
     rows, C = a.shape
     sums = torch.empty(C, dtype=torch.float32, device=a.device)
-    dh = None if h is None else torch.empty_like(h)
     n = _bytes("proteus_train_workspace_bytes", rows, C)
-    _call("proteus_colsum", a.device, a, h, dh, sums, _workspace(n, a.device), n, rows, C)
-    return sums if h is None else (dh, sums)
+    _call("proteus_colsum", a.device, a, None, None, sums, _workspace(n, a.device), n, rows, C)
+    return sums
+
+
+# ---------------------------------------------------------------------------------------------------- matrix products
+
+NN, NT, TN = _lib.GEMM_NN, _lib.GEMM_NT, _lib.GEMM_TN
+
+
+def _product(form, A, B, bias=None, gelu=False, gelu_grad_of=None, dtype=torch.float32):
+    """A B (NN), A B^T (NT) or A^T B (TN) of dense fp32 matrices, plus `bias` per column: one launch of the library's product, which
+    issues in a fifth of the host time of torch's; torch's where rows are not multiples of 16 bytes or a matrix has 2 GiB.
+    gelu: returns (sums, gelu(sums)); gelu_grad_of: sums * gelu'(gelu_grad_of); dtype: of the result (bf16: the sums rounded once)."""
+    M, K = A.shape if form != TN else A.shape[::-1]
+    N = B.shape[0] if form == NT else B.shape[1]
+    if not ((form == TN or K % 4 == 0) and (A.shape[0] + 512) * A.shape[1] < 2 ** 29 and (B.shape[0] + 512) * B.shape[1] < 2 ** 29):
+        Am, Bm = A.t() if form == TN else A, B.t() if form == NT else B
+        C = Am.mm(Bm) if bias is None else torch.addmm(bias, Am, Bm)
+        if gelu:
+            return C, F.gelu(C)
+        return C.to(dtype) if gelu_grad_of is None else torch.ops.aten.gelu_backward(C, gelu_grad_of)
+    C = torch.empty(M, N, dtype=dtype, device=A.device)
+    H = torch.empty_like(C) if gelu else None
+    epilogue = _lib.GEMM_GELU if gelu else _lib.GEMM_GELU_GRAD if gelu_grad_of is not None else _lib.GEMM_BF16 if dtype == torch.bfloat16 else _lib.GEMM_F32
+    _call("proteus_gemm_f32", A.device, A, B, bias, gelu_grad_of, C, H, M, N, K, A.shape[1], B.shape[1], N, form, epilogue)
+    return (H, C) if gelu else C
 
 
 # ---------------------------------------------------------------------------------------------------- add + LayerNorm
@@ -181,11 +204,10 @@ class _GeluMLP(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w1, b1, w2, b2):
         x2 = _dense(x).view(-1, x.shape[-1])
-        h = torch.addmm(b1, x2, w1.t())
-        a = F.gelu(h)
+        h, a = _product(NT, x2, _dense(w1), _dense(b1), gelu=True)
         ctx.save_for_backward(x, w1, b1, w2, b2, h, a)
         # (resized, not viewed: autograd lets no view that a function returns be changed in place)
-        return torch.addmm(b2, a, w2.t()).resize_(*x.shape[:-1], w2.shape[0])
+        return _product(NT, a, _dense(w2), _dense(b2)).resize_(*x.shape[:-1], w2.shape[0])
 
     @staticmethod
     @_without_autocast
@@ -194,17 +216,19 @@ class _GeluMLP(torch.autograd.Function):
         need = ctx.needs_input_grad
         if _by_expression(d):
             return _recorded(lambda x_, w1_, b1_, w2_, b2_: F.linear(F.gelu(F.linear(x_, w1_, b1_)), w2_, b2_), (x, w1, b1, w2, b2), need, d)
-        d2 = _dense(d).view(-1, w2.shape[0])
-        x2 = _dense(x).view(-1, w1.shape[1])
-        dw2 = d2.t().mm(a) if need[3] else None
+        rows, (hidden, d_in), d_out = d.numel() // w2.shape[0], w1.shape, w2.shape[0]
+        d2 = _dense(d).view(-1, d_out)
+        x2, a = _saved(x, rows * d_in).view(rows, d_in), _saved(a, rows * hidden).view(rows, hidden)
+        w1, w2, h = _saved(w1, hidden * d_in).view(hidden, d_in), _saved(w2, d_out * hidden).view(d_out, hidden), _saved(h, rows * hidden)
+        dw2 = _product(TN, d2, a) if need[3] else None
         db2 = column_sums(d2) if need[4] else None
         dx = dw1 = db1 = None
         if need[0] or need[1] or need[2]:
-            da = d2.mm(w2)
-            dh, db1 = column_sums(da, _saved(h, da.numel()))
-            dw1 = dh.t().mm(x2) if need[1] else None
-            dx = dh.mm(w1).view(x.shape) if need[0] else None
-        return dx, dw1, db1 if need[2] else None, dw2, db2
+            dh = _product(NN, d2, w2, gelu_grad_of=h)
+            db1 = column_sums(dh) if need[2] else None
+            dw1 = _product(TN, dh, x2) if need[1] else None
+            dx = _product(NN, dh, w1).view(x.shape) if need[0] else None
+        return dx, dw1, db1, dw2, db2
 
 
 def gelu_mlp(x, lin1, lin2):
@@ -259,6 +283,7 @@ class _SelfAttention(torch.autograd.Function):
         b = torch.empty(3 * dm, dtype=torch.float32, device=dev)
         sigma, spread = torch.empty(H, dtype=torch.float32, device=dev), torch.empty(H, dtype=torch.float32, device=dev)
         _layout((qw, kw, vw, qb, kb, vb, spread, wo), W, b, Wo, sigma, spread_w, dm, H, dk, min_spread, 0)
+        # (torch's product: its sums are rounded to 16 bits next, and the expression's roundings are the ones to make)
         qkv = torch.addmm(b, _dense(x).view(Z * N, dm), W).to(operand_dtype or torch.bfloat16).view(Z, N, 3, H, dk)
         O, L = ga.geo_attn(*_heads(qkv), coords, sigma, mask, return_lse=True, check_sigma=False, token_major_out=True,
                            operand_dtype=operand_dtype)
@@ -268,7 +293,7 @@ class _SelfAttention(torch.autograd.Function):
         ctx.params = (qw, kw, vw, qb, kb, vb, spread_w, wo)
         ctx.versions = [p._version for p in ctx.params]
         ctx.min_spread, ctx.operand_dtype = min_spread, operand_dtype
-        return O.permute(0, 2, 1, 3).reshape(Z * N, dm).mm(Wo.t()).resize_(Z, N, dm)       # (as in the feed-forward)
+        return _product(NT, O.permute(0, 2, 1, 3).reshape(Z * N, dm), Wo).resize_(Z, N, dm)       # (as in the feed-forward)
 
     @staticmethod
     @_without_autocast
@@ -284,16 +309,17 @@ class _SelfAttention(torch.autograd.Function):
         Z, N, _, H, dk = qkv.shape
         dm = H * dk
         d2 = _dense(d).view(Z * N, dm)
-        dO = d2.mm(Wo).view(Z, N, H, dk).permute(0, 2, 1, 3)
+        W, Wo, x2 = _saved(W, 3 * dm * dm).view(dm, 3 * dm), _saved(Wo, dm * dm).view(dm, dm), _saved(x, Z * N * dm).view(Z * N, dm)
+        dO = _product(NN, d2, Wo).view(Z, N, H, dk).permute(0, 2, 1, 3)
         g = torch.empty(qkv.shape, dtype=torch.float32, device=d.device)
         _, _, _, d_sigma, _ = ga._backward(*_heads(qkv), O, L, dO, coords, sigma, mask, None, 0.0, 1.0, ctx.operand_dtype, grads=_heads(g))
         g2 = g.view(Z * N, 3 * dm)
-        dx = g2.mm(W.t()).view(x.shape) if need[0] else None
+        dx = _product(NT, g2, W).view(x.shape) if need[0] else None
         grads = [torch.empty_like(p, memory_format=torch.contiguous_format) if n else None for p, n in zip(params, need[3:11])]
         # (what a gradient is not asked of is not looked at: its place in the list is None)
-        dW = _dense(x).view(Z * N, dm).t().mm(g2) if any(need[3:6]) else g2
+        dW = _product(TN, x2, g2) if any(need[3:6]) else g2
         db = column_sums(g2) if any(need[6:9]) else g2
-        dWo = d2.t().mm(O.permute(0, 2, 1, 3).reshape(Z * N, dm)) if need[10] else g2
+        dWo = _product(TN, d2, _saved(O.permute(0, 2, 1, 3), Z * N * dm).view(Z * N, dm)) if need[10] else g2
         _layout(grads, dW, db, dWo, d_sigma, _saved(spread, H), dm, H, dk, ctx.min_spread, 1)
         return (dx, None, None, *grads, None, None)
 

@@ -1,0 +1,72 @@
+"""The fp32 product of the encoder's training step (proteus_gemm_f32) against float64, and what it refuses."""
+import ctypes
+
+import pytest
+import torch
+
+from proteusai_amd import _lib, train_ops
+
+NN, NT, TN = _lib.GEMM_NN, _lib.GEMM_NT, _lib.GEMM_TN
+
+
+def _operands(form, M, N, K, gpu):
+    g = torch.Generator(device=gpu).manual_seed(M * 7919 + N * 31 + K)
+    scale = torch.exp(3 * torch.randn(K, generator=g, device=gpu))             # terms of very different size
+    A, B = torch.randn(M, K, generator=g, device=gpu) * scale, torch.randn(K, N, generator=g, device=gpu) / scale.flip(0)[:, None]
+    return (A.t().contiguous() if form == TN else A), (B.t().contiguous() if form == NT else B), A.double() @ B.double(), A.double().abs() @ B.double().abs()
+
+
+# Edges of the 64 x 64 tiles, of the steps of 16 k and of what 1, 2 and 4 groups share out (more than 640 tiles, 321 to 640, fewer).
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", [NN, NT, TN])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 4), (63, 65, 16), (64, 64, 20), (65, 36, 68), (130, 512, 132), (1, 20, 512), (1100, 1200, 36), (1700, 1600, 52)])
+def test_product_against_float64(gpu, form, M, N, K):
+    if form == TN:
+        K -= 3                                                                  # (rows along K need no multiple of 4)
+    A, B, want, mass = _operands(form, M, N, K, gpu)
+    got = train_ops._product(form, A, B)
+    # six instructions per 16 k, each rounding a partial sum (at most the sum of magnitudes) once or, with its inner additions, twice;
+    # 16 more for the groups' sums and the dropped pieces (3 x 2^-26 of every term)
+    bound = (12 * ((K + 15) // 16) + 16) * 2.0 ** -24 * mass
+    assert bool(((got - want).abs() <= bound).all())
+    assert torch.equal(got, train_ops._product(form, A, B))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [5, 700])
+def test_epilogues(gpu, M):
+    A, B, want, mass = _operands(NT, M, 132, 72, gpu)
+    bias, h = torch.randn(132, device=gpu), torch.randn(M, 132, device=gpu)
+    bound = 76 * 2.0 ** -24 * mass + 2.0 ** -23 * bias.abs()
+    H, C = train_ops._product(NT, A, B, bias, gelu=True)
+    assert bool(((H - want - bias).abs() <= bound).all())
+    # (erff is good to 2 ulp; gelu of the kernel's own sums)
+    exact = torch.nn.functional.gelu(H.double())
+    assert bool(((C - exact).abs() <= 2.0 ** -21 * H.abs()).all())
+    hd = h.double().requires_grad_(True)
+    grad, = torch.autograd.grad(torch.nn.functional.gelu(hd).sum(), hd)
+    plain = train_ops._product(NT, A, B, bias)
+    assert bool(((train_ops._product(NT, A, B, bias, gelu_grad_of=h) - plain.double() * grad).abs() <= 2.0 ** -20 * plain.abs() * (1 + h.abs())).all())
+    assert torch.equal(train_ops._product(NT, A, B, bias, dtype=torch.bfloat16), plain.to(torch.bfloat16))
+
+
+@pytest.mark.gpu
+def test_values_that_do_not_split(gpu):
+    A, B, _, _ = _operands(NN, 70, 68, 36, gpu)
+    A[3, 5], A[7, 1], A[9, 2], A[11, 3] = float("inf"), float("nan"), 3.4e38, -3.39e38      # (bf16 ends at 3.39e38)
+    got, want = train_ops._product(NN, A, B), A.double() @ B.double()
+    want = want.where(want.abs() <= torch.finfo(torch.float32).max, want.sign() * float("inf")).where(~want.isnan(), want)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    assert torch.equal(got[got.isinf()].double(), want[want.isinf()])
+
+
+def test_what_it_refuses():
+    lib = _lib.load()
+    at = ctypes.c_void_p(4096)
+    def call(A=at, B=at, C=at, H=None, M=8, N=8, K=8, lda=8, ldb=8, ldc=8, form=NN, epilogue=0):
+        return lib.proteus_gemm_f32(A, B, None, None, C, H, M, N, K, lda, ldb, ldc, form, epilogue, None)
+    assert call(A=None) < 0 and call(C=None) < 0 and call(epilogue=_lib.GEMM_GELU) < 0 and call(epilogue=_lib.GEMM_GELU_GRAD) < 0
+    assert call(form=3) < 0 and call(epilogue=4) < 0
+    assert call(M=0) < 0 and call(K=6, lda=8) < 0 and call(lda=6) < 0 and call(ldc=4) < 0 and call(form=NT, ldb=10) < 0
+    assert call(A=ctypes.c_void_p(4100)) < 0
+    assert call(M=1 << 28, lda=8) < 0                                           # (2 GiB and more)
