@@ -554,7 +554,7 @@ int proteus_embedding_bwd(const float* dout, const int64_t* tokens, float* dW, v
  *   form      PROTEUS_GEMM_NN: A [M][K], B [K][N];  _NT: A [M][K], B [N][K];  _TN: A [K][M], B [K][N]; rows lda, ldb, ldc elements apart.
  *             A matrix whose rows run along K (A in NN and NT, B in NT): K and its ld multiples of 4
  *   epilogue  PROTEUS_GEMM_F32: C f32;  _BF16: C bf16, rounded once;  _GELU: H = the sums f32, C = gelu(H) f32;
- *             _GELU_GRAD: C = sums * gelu'(h) f32 (exact GELU; H and h laid out as C)
+ *             _GELU_GRAD: C = sums * gelu'(h) f32;  _ADD: C = sums + h f32 (exact GELU; H and h laid out as C)
  *   A, B, C 16-byte aligned; bias, h, H may be NULL where not asked for.  One launch, no workspace.
  */
 #define PROTEUS_GEMM_NN 0
@@ -564,8 +564,37 @@ int proteus_embedding_bwd(const float* dout, const int64_t* tokens, float* dW, v
 #define PROTEUS_GEMM_BF16      1
 #define PROTEUS_GEMM_GELU      2
 #define PROTEUS_GEMM_GELU_GRAD 3
+#define PROTEUS_GEMM_ADD       4
 int proteus_gemm_f32(const float* A, const float* B, const float* bias, const float* h, void* C, float* H,
                      int M, int N, int K, int lda, int ldb, int ldc, int form, int epilogue, void* stream);
+
+/*
+ * One post-LN encoder layer's training step on the kernels above, a call per direction (old/old_scripts/encoder.py:33-41 with the geometric
+ * attention branch on the README logits, exact GELU, no dropout):  x1 = LN(x + attn(x)), out = LN(x1 + ffn(x1)).  fp32 tensors; the
+ * attention's operands are bf16.
+ *   x, out, dout, dx   [Z*N][d_model];  coords [Z,N,3];  mask [Z,N] u8 or NULL (1 = padded)
+ *   params / grads     what proteus_encoder_layer_fwd reads / proteus_encoder_layer_bwd writes, in this order: q, k, v projections
+ *                      [H][d_model][d_head], their biases [H][d_head], spread weights [H], output projection [d_model][d_head][H], gamma and
+ *                      beta of the first LayerNorm [d_model], first [hidden][d_model] and second [d_model][hidden] linear layer's weight and
+ *                      bias (weight, bias, weight, bias), gamma and beta of the second LayerNorm: 16 pointers.  A gradient that is NULL
+ *                      (and dx) is left out, with the products that only it needs; those of a LayerNorm's gamma and beta are one array
+ *                      [2][d_model] in gamma's place, beta's place is not looked at.
+ *   kept               proteus_encoder_layer_kept_bytes: what the backward reads of the forward; the attention's parameters are among it
+ *                      as copies, those of the LayerNorms and the feed-forward are read again (params of the backward: the same 16, of
+ *                      which it reads 8, 10, 12 and 14)
+ *   ws                 workspace, proteus_encoder_layer_fwd_bytes / _bwd_bytes
+ *   d_model = H * d_head <= 2048, hidden a multiple of 4; every pointer 16-byte aligned, kept and ws 256-byte aligned
+ */
+#define PROTEUS_LAYER_PARAMS 16
+size_t proteus_encoder_layer_kept_bytes(int Z, int N, int H, int d_head, int hidden);
+size_t proteus_encoder_layer_fwd_bytes(int Z, int N, int H, int d_head, int hidden);
+size_t proteus_encoder_layer_bwd_bytes(int Z, int N, int H, int d_head, int hidden);
+int proteus_encoder_layer_fwd(const float* x, const float* coords, const uint8_t* mask, const float* const* params, float min_spread,
+                              float eps1, float eps2, float* out, void* kept, size_t kept_bytes, void* ws, size_t ws_bytes,
+                              int Z, int N, int H, int d_head, int hidden, void* stream);
+int proteus_encoder_layer_bwd(const float* x, const float* coords, const uint8_t* mask, const float* const* params, const float* dout,
+                              float* dx, float* const* grads, float min_spread, const void* kept, size_t kept_bytes, void* ws, size_t ws_bytes,
+                              int Z, int N, int H, int d_head, int hidden, void* stream);
 
 #ifdef __cplusplus
 }

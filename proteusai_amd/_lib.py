@@ -18,7 +18,7 @@ ABI_VERSION = 306                    # PROTEUS_VERSION of the include/proteus_hi
 OPERAND_BF16, OPERAND_F16 = 0, 1     # PROTEUS_OPERAND_* of include/proteus_hip.h
 GRAD_F32, GRAD_OPERAND = 0, 1        # PROTEUS_GRAD_*
 GEMM_NN, GEMM_NT, GEMM_TN = 0, 1, 2  # PROTEUS_GEMM_*: form
-GEMM_F32, GEMM_BF16, GEMM_GELU, GEMM_GELU_GRAD = 0, 1, 2, 3      # and epilogue
+GEMM_F32, GEMM_BF16, GEMM_GELU, GEMM_GELU_GRAD, GEMM_ADD = 0, 1, 2, 3, 4     # and epilogue
 DTYPE_F32, DTYPE_BF16, DTYPE_F16 = 0, 1, 2   # PROTEUS_DTYPE_*
 
 # every symbol include/proteus_hip.h declares
@@ -37,7 +37,8 @@ SYMBOLS = [
     "proteus_geo_attn_variant_name",
     "proteus_add_layernorm_fwd", "proteus_add_layernorm_fwd_check", "proteus_geo_attn_delta", "proteus_geo_attn_delta_check",
     "proteus_train_workspace_bytes", "proteus_layernorm_bwd_workspace_bytes", "proteus_embedding_bwd_workspace_bytes",
-    "proteus_add_layernorm_train_fwd", "proteus_layernorm_bwd", "proteus_colsum", "proteus_heads_layout", "proteus_embedding_bwd", "proteus_gemm_f32",
+    "proteus_add_layernorm_train_fwd", "proteus_layernorm_bwd", "proteus_colsum", "proteus_heads_layout", "proteus_embedding_bwd", "proteus_gemm_f32", "proteus_encoder_layer_kept_bytes", "proteus_encoder_layer_fwd_bytes",
+    "proteus_encoder_layer_bwd_bytes", "proteus_encoder_layer_fwd", "proteus_encoder_layer_bwd",
 ]
 
 _lib = None
@@ -173,6 +174,14 @@ def load():
     lib.proteus_embedding_bwd.argtypes = [vp] * 4 + [sz, cl, ci, ci, vp]
     lib.proteus_gemm_f32.restype = ci
     lib.proteus_gemm_f32.argtypes = [vp] * 6 + [ci] * 8 + [vp]
+    for name in ("kept", "fwd", "bwd"):
+        getattr(lib, f"proteus_encoder_layer_{name}_bytes").restype = sz
+        getattr(lib, f"proteus_encoder_layer_{name}_bytes").argtypes = [ci] * 5
+    vpp = ctypes.POINTER(vp)
+    lib.proteus_encoder_layer_fwd.restype = ci
+    lib.proteus_encoder_layer_fwd.argtypes = [vp, vp, vp, vpp, cf, cf, cf, vp, vp, sz, vp, sz, ci, ci, ci, ci, ci, vp]
+    lib.proteus_encoder_layer_bwd.restype = ci
+    lib.proteus_encoder_layer_bwd.argtypes = [vp, vp, vp, vpp, vp, vp, vpp, cf, vp, sz, vp, sz, ci, ci, ci, ci, ci, vp]
     _lib = lib
     return lib
 

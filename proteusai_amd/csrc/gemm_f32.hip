@@ -94,6 +94,17 @@ __device__ __forceinline__ float plain_dot(const GemmArgs& g, const int m, const
     return s;
 }
 
+// Does a row (of A, or of B^T) hold a NaN at k0 <= k < k1?
+template <bool KC>
+__device__ __forceinline__ bool any_nan(const float* __restrict__ X, const int ld, const int row, const int rows, const int k0, const int k1)
+{
+    if (row >= rows) return false;
+    bool found = false;
+#pragma unroll 8
+    for (int k = k0; k < k1; ++k) { const float v = KC ? X[(size_t)row * ld + k] : X[(size_t)k * ld + row]; found |= v != v; }
+    return found;
+}
+
 __device__ __forceinline__ float gelu(const float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
 __device__ __forceinline__ float gelu_grad(const float x) {
     const float cdf = 0.5f * (1.0f + erff(x * 0.70710678118654752f));
@@ -179,6 +190,7 @@ void gemm_f32_kernel(const GemmArgs g)
         if (EPI == PROTEUS_GEMM_F32)        static_cast<float*>(g.C)[at] = v;
         else if (EPI == PROTEUS_GEMM_BF16)  static_cast<__bf16*>(g.C)[at] = (__bf16)v;
         else if (EPI == PROTEUS_GEMM_GELU)  { g.H[at] = v; static_cast<float*>(g.C)[at] = gelu(v); }
+        else if (EPI == PROTEUS_GEMM_ADD)   static_cast<float*>(g.C)[at] = v + g.h[at];
         else                                static_cast<float*>(g.C)[at] = v * gelu_grad(g.h[at]);
     };
     uint32_t again = 0;                                        // of the lane's 16 elements those that are not finite
@@ -201,9 +213,15 @@ void gemm_f32_kernel(const GemmArgs g)
             else again |= 1u << (q * 4 + i);
         }
     }
+    if (__builtin_amdgcn_ballot_w64(again != 0) == 0) return;
+    // Where a row of A or a column of B holds a NaN so do their elements (a run that has diverged: all of them); the others are summed again.
+    const int half = (g.K / 2 + 3) / 4 * 4, k0 = lane >> 5 ? half : 0, k1 = lane >> 5 ? g.K : half;
+    const bool nan_a = any_nan<AK>(g.A, g.lda, m0 + wm + (lane & 31), g.M, k0, k1), nan_b = any_nan<BK>(g.B, g.ldb, n, g.N, k0, k1);
+    const uint64_t in_a = __builtin_amdgcn_ballot_w64(nan_a), in_b = __builtin_amdgcn_ballot_w64(nan_b);
+    const uint32_t rows_a = (uint32_t)in_a | (uint32_t)(in_a >> 32), cols_b = (uint32_t)in_b | (uint32_t)(in_b >> 32);
     for (; again; again &= again - 1) {
-        const int e = __builtin_ctz(again), m = m0 + wm + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
-        finish(m, plain_dot<AK, BK>(g, m, n));
+        const int e = __builtin_ctz(again), r = 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3), m = m0 + wm + r;
+        finish(m, (rows_a >> r | cols_b >> (lane & 31)) & 1 ? __builtin_nanf("") : plain_dot<AK, BK>(g, m, n));
     }
 }
 
@@ -234,8 +252,8 @@ bool off16(const void* p) { return ((uintptr_t)p & 15) != 0; }
 extern "C" int proteus_gemm_f32(const float* A, const float* B, const float* bias, const float* h, void* C, float* H,
                                 int M, int N, int K, int lda, int ldb, int ldc, int form, int epilogue, void* stream)
 {
-    if (!A || !B || !C || (epilogue == PROTEUS_GEMM_GELU && !H) || (epilogue == PROTEUS_GEMM_GELU_GRAD && !h)) return PROTEUS_ERR_NULL_POINTER;
-    if (form < 0 || form > PROTEUS_GEMM_TN || epilogue < 0 || epilogue > PROTEUS_GEMM_GELU_GRAD) return PROTEUS_ERR_UNSUPPORTED;
+    if (!A || !B || !C || (epilogue == PROTEUS_GEMM_GELU && !H) || ((epilogue == PROTEUS_GEMM_GELU_GRAD || epilogue == PROTEUS_GEMM_ADD) && !h)) return PROTEUS_ERR_NULL_POINTER;
+    if (form < 0 || form > PROTEUS_GEMM_TN || epilogue < 0 || epilogue > PROTEUS_GEMM_ADD) return PROTEUS_ERR_UNSUPPORTED;
     if (M <= 0 || N <= 0 || K <= 0 || ldc < N || lda < (form == PROTEUS_GEMM_TN ? M : K) || ldb < (form == PROTEUS_GEMM_NT ? K : N)) return PROTEUS_ERR_BAD_SHAPE;
     // (tiles are numbered in 32 bits)
     if ((int64_t)((M + (int64_t)GT - 1) / GT) * ((N + (int64_t)GT - 1) / GT) > (1 << 30)) return PROTEUS_ERR_TOO_LARGE;
@@ -253,6 +271,7 @@ extern "C" int proteus_gemm_f32(const float* A, const float* B, const float* bia
         case PROTEUS_GEMM_F32:  return gemm_go<AK_, BK_, PROTEUS_GEMM_F32>(g, st); \
         case PROTEUS_GEMM_BF16: return gemm_go<AK_, BK_, PROTEUS_GEMM_BF16>(g, st); \
         case PROTEUS_GEMM_GELU: return gemm_go<AK_, BK_, PROTEUS_GEMM_GELU>(g, st); \
+        case PROTEUS_GEMM_ADD:  return gemm_go<AK_, BK_, PROTEUS_GEMM_ADD>(g, st); \
         default:                return gemm_go<AK_, BK_, PROTEUS_GEMM_GELU_GRAD>(g, st); \
     }
     switch (form) {

@@ -344,6 +344,109 @@ def self_attention(x, coords, mask, m):
     return _SelfAttention.apply(x, coords, mask, *params, m.min_spread, m.operand_dtype)
 
 
+# ---------------------------------------------------------------------------------------------------- encoder layer
+
+def _layer_expression(x, coords, mask, qw, kw, vw, qb, kb, vb, spread_w, wo, g1, c1, w1, b1, w2, b2, g2, c2, min_spread, operand_dtype, eps1, eps2):
+    x = F.layer_norm(x + _self_attention_expression(x, coords, mask, qw, kw, vw, qb, kb, vb, spread_w, wo, min_spread, operand_dtype), g1.shape, g1, c1, eps1)
+    return F.layer_norm(x + F.linear(F.gelu(F.linear(x, w1, b1)), w2, b2), g2.shape, g2, c2, eps2)
+
+
+def _pointers(tensors):
+    return (ctypes.c_void_p * len(tensors))(*[None if t is None else t.data_ptr() for t in tensors])
+
+
+class _EncoderLayer(torch.autograd.Function):
+    """A whole post-LN layer: the launches of the functions above from one call of the library per direction."""
+
+    @staticmethod
+    def forward(ctx, x, coords, mask, *args):
+        params, (min_spread, operand_dtype, eps1, eps2) = args[:16], args[16:]
+        H, dm, dk = params[0].shape
+        Z, N, _ = x.shape
+        sizes = (Z, N, H, dk, params[10].shape[0])
+        dev = x.device
+        xc, c, m = _dense(x), ga._f32(coords, dev), None if mask is None else ga._mask_bytes(mask, dev)
+        kept = torch.empty(_bytes("proteus_encoder_layer_kept_bytes", *sizes), dtype=torch.uint8, device=dev)
+        n = _bytes("proteus_encoder_layer_fwd_bytes", *sizes)
+        out = torch.empty(Z, N, dm, dtype=torch.float32, device=dev)
+        _call("proteus_encoder_layer_fwd", dev, xc, c, m, _pointers(params), min_spread, eps1, eps2, out, kept, kept.numel(), _workspace(n, dev), n, *sizes)
+        # (the attention's parameters may change before the backward, as in its own function: what it reads of them is kept as copies)
+        ctx.save_for_backward(x, coords, mask, kept, *params[8:])
+        ctx.params = params[:8]
+        ctx.versions = [p._version for p in ctx.params]
+        ctx.args = args[16:]
+        return out
+
+    @staticmethod
+    @_without_autocast
+    def backward(ctx, d):
+        x, coords, mask, kept, *rest = ctx.saved_tensors
+        need, attn = ctx.needs_input_grad, ctx.params
+        min_spread, operand_dtype, eps1, eps2 = ctx.args
+        if _by_expression(d):
+            if any(p._version != v for p, v in zip(attn, ctx.versions)):
+                raise RuntimeError("a parameter of the self-attention was changed in place after the forward pass whose gradient is recorded")
+            gx, *gp = _recorded(lambda x_, *p: _layer_expression(x_, coords, mask, *p, *ctx.args), (x, *attn, *rest), (need[0], *need[3:19]), d)
+            return (gx, None, None, *gp, None, None, None, None)
+        Z, N, dm = x.shape
+        H, _, dk = attn[0].shape
+        hidden = rest[2].shape[0]
+        sizes = (Z, N, H, dk, hidden)
+        dev = d.device
+        g1, c1, w1, b1, w2, b2, g2, c2 = rest
+        g1, w1, w2, g2 = _saved(g1, dm), _saved(w1, hidden * dm), _saved(w2, dm * hidden), _saved(g2, dm)
+        x2, kept = _saved(x, Z * N * dm), _saved(kept, _bytes("proteus_encoder_layer_kept_bytes", *sizes), torch.uint8)
+        if kept.data_ptr() % 256:
+            kept = kept.clone()
+        c, m = ga._f32(coords, dev), None if mask is None else ga._mask_bytes(mask, dev)
+        wanted = need[3:19]
+        grads = [torch.empty_like(p, memory_format=torch.contiguous_format) if n and not 8 <= i <= 9 and i < 14 else None
+                 for i, (p, n) in enumerate(zip((*attn, *rest), wanted))]
+        for i in (8, 14):           # gamma's and beta's gradients are one array
+            if wanted[i] or wanted[i + 1]:
+                grads[i] = torch.empty(2, dm, dtype=torch.float32, device=dev)
+        dx = torch.empty(Z, N, dm, dtype=torch.float32, device=dev) if need[0] else None
+        n = _bytes("proteus_encoder_layer_bwd_bytes", *sizes)
+        _call("proteus_encoder_layer_bwd", dev, x2, c, m, _pointers((None,) * 8 + (g1, None, w1, None, w2, None, g2, None)), _dense(d), dx, _pointers(grads),
+              min_spread, kept, kept.numel(), _workspace(n, dev), n, *sizes)
+        for i in (8, 14):
+            both = grads[i]
+            if both is not None:
+                grads[i], grads[i + 1] = both[0] if wanted[i] else None, both[1] if wanted[i + 1] else None
+        return (dx, None, None, *grads, None, None, None, None)
+
+
+def encoder_layer(x, coords, mask, m, mlp_class):
+    """The output of the Encoder module `m` (self-attention, `mlp_class` its feed-forward) on x, or None where its parts go their own ways."""
+    if not torch.is_grad_enabled():
+        return None
+    a, n1, f, n2 = m.attn, m.attn_norm, m.ffn, m.ffn_norm
+    lin1, lin2 = getattr(f, "in_proj", None), getattr(f, "out_proj", None)
+    if not (plain_module(a, ga.GeoAttention) and plain_module(n1, nn.LayerNorm) and plain_module(n2, nn.LayerNorm) and inactive_dropout(m.dropout)
+            and plain_module(f, mlp_class) and f.act is F.gelu and not f.hidden_proj and inactive_dropout(f.in_dropout)
+            and plain_module(lin1, nn.Linear) and plain_module(lin2, nn.Linear) and plain_module(a.out_proj, nn.Linear) and "_residual_norm" not in m.__dict__):
+        return None
+    H, dk, dm = a.heads, a.d_k, a.d_model
+    params = (a.q_proj, a.k_proj, a.v_proj, a.q_bias, a.k_bias, a.v_bias, a.spread_weights, a.out_proj.weight,
+              n1.weight, n1.bias, lin1.weight, lin1.bias, lin2.weight, lin2.bias, n2.weight, n2.bias)
+    if any(p is None for p in params):
+        return None
+    hidden = lin1.weight.shape[0]
+    w, b = (H, dm, dk), (H, dk)
+    if tuple(p.shape for p in params) != (w, w, w, b, b, b, (H,), (dm, dm), (dm,), (dm,), (hidden, dm), (hidden,), (dm, hidden), (dm,), (dm,), (dm,)):
+        return None
+    # (frozen weights: the parts, which keep of the inputs only what they read again; spreads and what follows a product may be frozen)
+    if (not all(params[i].requires_grad for i in (0, 1, 2, 10, 12)) or a.legacy_logits or x.dim() != 3 or x.shape[2] != dm or x.numel() == 0
+            or type(coords) is not torch.Tensor or coords.device != x.device or tuple(coords.shape) != (*x.shape[:2], 3) or coords.requires_grad
+            or (mask is not None and (type(mask) is not torch.Tensor or tuple(mask.shape) != tuple(x.shape[:2])))
+            or a.operand_dtype not in (None, torch.bfloat16) or not isinstance(a.min_spread, (int, float)) or "get_spreads" in a.__dict__
+            or a.out_proj.bias is not None or not (n1.eps >= 0.0 and n2.eps >= 0.0)
+            or not recording(x, *params) or not aligned(*params)
+            or _bytes("proteus_encoder_layer_kept_bytes", *x.shape[:2], H, dk, hidden) == 0):
+        return None
+    return _EncoderLayer.apply(x, coords, mask, *params, a.min_spread, a.operand_dtype, float(n1.eps), float(n2.eps))
+
+
 # ---------------------------------------------------------------------------------------------------- token embedding
 
 class _SmallEmbedding(torch.autograd.Function):

@@ -51,6 +51,19 @@ def test_epilogues(gpu, M):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("form", [NN, NT, TN])
+def test_a_diverged_operand(gpu, form):
+    A, B, want, _ = _operands(form, 130, 132, 68, gpu)
+    clean = train_ops._product(form, A, B)
+    (A if form != TN else A.t())[66, 67] = float("nan")
+    (B if form == NT else B.t())[131, 0] = float("nan")
+    got = train_ops._product(form, A, B)
+    hit = torch.zeros_like(got, dtype=torch.bool)
+    hit[66], hit[:, 131] = True, True
+    assert torch.equal(got.isnan(), hit) and torch.equal(got[~hit], clean[~hit])
+
+
+@pytest.mark.gpu
 def test_values_that_do_not_split(gpu):
     A, B, _, _ = _operands(NN, 70, 68, 36, gpu)
     A[3, 5], A[7, 1], A[9, 2], A[11, 3] = float("inf"), float("nan"), 3.4e38, -3.39e38      # (bf16 ends at 3.39e38)
