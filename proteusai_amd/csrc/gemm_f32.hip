@@ -5,13 +5,22 @@
 // is below 2^-26 of |x y|, under the rounding of one fp32 addition.  Six v_mfma_f32_32x32x16_bf16 cost 192 clocks where the same
 // product on v_mfma_f32_32x32x2_f32 takes 512, and their fp32 accumulator rounds once per 16 products instead of once per 2.
 //
-// A workgroup makes one 64 x 64 tile of C.  Four waves (a group) hold 32 x 32 of it each and step through K by 16; where the tiles
-// are too few to fill the chip, 2 or 4 groups share a tile, each with its own steps and its own LDS stages, and add up at the end
-// in a fixed order (the same bits on every call).  A step: 8 floats per thread travel global -> registers two steps ahead, are
-// split (5.5 vector instructions each) and written to one of two stages as 16-byte fragments, eight consecutive k of one row; the
-// product reads them with ds_read_b128.  Odd groups split and then multiply, even ones the other way round, so that the matrix
-// cores of a SIMD have work while the other half of its waves split.  A bound of its own: a 64 x 64 x 16 step reads 24 KB
-// and writes 12 KB of LDS (288 clocks at 128 bytes a clock) beside 192 clocks of products and about 200 of splitting.
+// gemm_f32_kernel (rows of A along k): a workgroup makes one 64 x 64 tile of C.  Four waves (a group) hold 32 x 32 of it each and step through
+// K by 16; where the tiles are too few to fill the chip, 2 or 4 groups share a tile, each with its own steps and its own LDS stages, and
+// add up at the end in a fixed order (the same bits on every call).  A step: 8 floats per thread travel global -> registers two steps
+// ahead, are split (5.5 vector instructions each) and written to one of two stages as 16-byte fragments, eight consecutive k of one row; the
+// product reads them with ds_read_b128.  Odd groups split and then multiply, even ones the other way round.  What bounds it: a 64 x 64 x 16
+// step reads 24 KB and writes 12 KB of LDS (288 clocks at 128 bytes a clock), and splitting (200 clocks a wave) hardly overlaps with the
+// products (192).  Smaller where it counts than the traffic of operands split beforehand: 6 bytes an element through L2.
+//
+// gemm_f32_rows_kernel (rows of A and B across k: gradients of weights): there 32 lanes read 128 consecutive bytes of one k, so a wave loads what
+// its fragments hold straight into registers, no LDS and no barrier: 64 x 64 of C over the wave's share of the steps, the next step split
+// under the 24 products of this one, the one after it on its way; the waves of a workgroup add up in LDS at the end.  With rows along
+// k a lane would read 32 bytes of a row of its own: 38 and 43 us against 36 and 38 (2048 x 512 x 2048 and 2048 x 2048 x 512).
+//
+// us, 2048 tokens, this / the library's fp32 product: QKV 2048 x 1536 x 512 32 / 35, its output 12 / 12; feed-forward 2048 x 2048 x 512 38 / 39,
+// 2048 x 512 x 2048 36 / 37; gradients of weights 512 x 2048 x 2048 34 / 39 (through the first kernel 44), 2048 x 512 x 2048 30 / 39 (39),
+// 512 x 1536 x 2048 28 / 31 (35), 512 x 512 x 2048 23 / 16 (31).  Error against float64 at K = 2048 2.5e-7 to 3.5e-7, the library's 8.1e-7.
 //
 // Values that are not finite (or become so: bf16 ends half a step below fp32) do not split; an element of C that comes out not
 // finite is summed again in plain fp32.
@@ -111,6 +120,18 @@ __device__ __forceinline__ float gelu_grad(const float x) {
     return __builtin_fmaf(x, 0.39894228040143268f * expf(-0.5f * x * x), cdf);
 }
 
+template <int EPI>
+__device__ __forceinline__ void write(const GemmArgs& g, const int m, const int n, float v)
+{
+    if (g.bias) v += g.bias[n];
+    const size_t at = (size_t)m * g.ldc + n;
+    if (EPI == PROTEUS_GEMM_F32)        static_cast<float*>(g.C)[at] = v;
+    else if (EPI == PROTEUS_GEMM_BF16)  static_cast<__bf16*>(g.C)[at] = (__bf16)v;
+    else if (EPI == PROTEUS_GEMM_GELU)  { g.H[at] = v; static_cast<float*>(g.C)[at] = gelu(v); }
+    else if (EPI == PROTEUS_GEMM_ADD)   static_cast<float*>(g.C)[at] = v + g.h[at];
+    else                                static_cast<float*>(g.C)[at] = v * gelu_grad(g.h[at]);
+}
+
 // AK, BK: k contiguous in A [M][K] / B [N][K]; else A is [K][M] / B [K][N]
 template <bool AK, bool BK, int G, int EPI>
 __global__ __launch_bounds__(G * 256, 4)
@@ -183,16 +204,6 @@ void gemm_f32_kernel(const GemmArgs g)
         __syncthreads();
     }
     const int n = n0 + wn + (lane & 31);
-    const float bias = g.bias && n < g.N ? g.bias[n] : 0.f;
-    auto finish = [&](const int m, float v) {
-        v += bias;
-        const size_t at = (size_t)m * g.ldc + n;
-        if (EPI == PROTEUS_GEMM_F32)        static_cast<float*>(g.C)[at] = v;
-        else if (EPI == PROTEUS_GEMM_BF16)  static_cast<__bf16*>(g.C)[at] = (__bf16)v;
-        else if (EPI == PROTEUS_GEMM_GELU)  { g.H[at] = v; static_cast<float*>(g.C)[at] = gelu(v); }
-        else if (EPI == PROTEUS_GEMM_ADD)   static_cast<float*>(g.C)[at] = v + g.h[at];
-        else                                static_cast<float*>(g.C)[at] = v * gelu_grad(g.h[at]);
-    };
     uint32_t again = 0;                                        // of the lane's 16 elements those that are not finite
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -209,7 +220,7 @@ void gemm_f32_kernel(const GemmArgs g)
             }
             const int m = m0 + wm + 8 * q + 4 * (lane >> 5) + i;
             if (m >= g.M || n >= g.N) continue;
-            if (fabsf(v) <= 3.4028234e38f) finish(m, v);
+            if (fabsf(v) <= 3.4028234e38f) write<EPI>(g, m, n, v);
             else again |= 1u << (q * 4 + i);
         }
     }
@@ -221,7 +232,139 @@ void gemm_f32_kernel(const GemmArgs g)
     const uint32_t rows_a = (uint32_t)in_a | (uint32_t)(in_a >> 32), cols_b = (uint32_t)in_b | (uint32_t)(in_b >> 32);
     for (; again; again &= again - 1) {
         const int e = __builtin_ctz(again), r = 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3), m = m0 + wm + r;
-        finish(m, (rows_a >> r | cols_b >> (lane & 31)) & 1 ? __builtin_nanf("") : plain_dot<AK, BK>(g, m, n));
+        write<EPI>(g, m, n, (rows_a >> r | cols_b >> (lane & 31)) & 1 ? __builtin_nanf("") : plain_dot<AK, BK>(g, m, n));
+    }
+}
+
+// Eight consecutive k of one row, and the three pieces' fragments of them.
+struct Raw { float4 lo, hi; };
+struct Frags { bf16x8 x[3]; };
+__device__ __forceinline__ Frags split(const Raw& r)
+{
+    const float v[8] = {r.lo.x, r.lo.y, r.lo.z, r.lo.w, r.hi.x, r.hi.y, r.hi.z, r.hi.w};
+    uint32_t p[3][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        p[0][i] = pack2(v[2 * i], v[2 * i + 1]);
+        const float a = v[2 * i] - low(p[0][i]), b = v[2 * i + 1] - high(p[0][i]);
+        p[1][i] = pack2(a, b);
+        p[2][i] = pack2(a - low(p[1][i]), b - high(p[1][i]));
+    }
+    Frags f;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) f.x[i] = __builtin_bit_cast(bf16x8, make_uint4(p[i][0], p[i][1], p[i][2], p[i][3]));
+    return f;
+}
+
+// A lane's share of an operand whose rows run across k: columns lane % 32 and 32 further, k from 8 (lane / 32) on.
+struct RowSource {
+    __amdgpu_buffer_rsrc_t rsrc;
+    uint32_t at[2], pitch;                                     // of the lane's columns at its first k; bytes per k
+    __device__ __forceinline__ RowSource(const float* X, const int ld, const int col, const int cols, const int k, const int K)
+        : rsrc(__builtin_amdgcn_make_buffer_rsrc((void*)X, 0, (uint32_t)(((size_t)(K - 1) * ld + cols) * 4), 0x00020000)), pitch((uint32_t)ld * 4u)
+    {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) at[i] = col + 32 * i < cols ? (uint32_t)(col + 32 * i) * 4u + (uint32_t)k * pitch : 0x80000000u;
+    }
+    __device__ __forceinline__ void fetch(const int k0, Raw (&r)[2]) const
+    {
+        // (rows of k past K lie behind the end; so does what a column past the last reads)
+        const uint32_t o = (uint32_t)k0 * pitch;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            float v[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, at[i] + o + (uint32_t)j * pitch, 0, 0));
+            r[i].lo = make_float4(v[0], v[1], v[2], v[3]); r[i].hi = make_float4(v[4], v[5], v[6], v[7]);
+        }
+    }
+};
+
+template <int W, int EPI>
+__global__ __launch_bounds__(W * 64, 2)
+void gemm_f32_rows_kernel(const GemmArgs g)
+{
+    extern __shared__ __align__(16) float red[];              // [W][64 accumulators][64 lanes]
+    const int tile = (blockIdx.x & 7) * g.per_xcd + (blockIdx.x >> 3);      // consecutive tiles (of the same rows of A) on one XCD
+    if ((int)(blockIdx.x >> 3) >= g.per_xcd || tile >= g.tiles) return;
+    const int m0 = tile / g.tiles_n * GT, n0 = tile % g.tiles_n * GT;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r0 = lane & 31, half = lane >> 5;
+
+    const RowSource sa(g.A, g.lda, m0 + r0, g.M, 8 * half, g.K);
+    const RowSource sb(g.B, g.ldb, n0 + r0, g.N, 8 * half, g.K);
+    const int steps = (g.K + GK - 1) / GK, rounds = steps > wave ? (steps - wave + W - 1) / W : 0;         // this wave's
+    Raw ra[2][2], rb[2][2];
+    Frags a[2][2], b[2][2];
+    f32x16 acc[2][2] = {};
+    auto load = [&](const int round, const int s) { const int k0 = (round * W + wave) * GK; sa.fetch(k0, ra[s]); sb.fetch(k0, rb[s]); };      // (zeros past the end)
+    auto step = [&](const int round, const int s) {
+        // send for the step after the next; split the next under this step's products
+        load(round + 2, s);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) { a[1 - s][i] = split(ra[1 - s][i]); b[1 - s][i] = split(rb[1 - s][i]); }
+        constexpr int P[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};
+#pragma unroll
+        for (int p = 0; p < 6; ++p)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s][i].x[P[p][0]], b[s][j].x[P[p][1]], acc[i][j], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 24; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);        // a product,
+            __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);        // vector instructions
+        }
+    };
+    if (rounds > 0) {
+        load(0, 0);
+        load(1, 1);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) { a[0][i] = split(ra[0][i]); b[0][i] = split(rb[0][i]); }
+        for (int r = 0; r < rounds; r += 2) {
+            step(r, 0);
+            step(r + 1, 1);                                    // (past the last round: zeros)
+        }
+    }
+
+    // ---- the waves' sums together: wave w takes accumulators w (64 / W) to (w + 1) (64 / W) ----
+    float v[64 / W];
+#pragma unroll
+    for (int e = 0; e < 64; ++e) red[(wave * 64 + e) * 64 + lane] = acc[e >> 5][(e >> 4) & 1][e & 15];
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 64 / W; ++e) {
+        v[e] = red[(wave * (64 / W) + e) * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < W; ++w) v[e] += red[(w * 64 + wave * (64 / W) + e) * 64 + lane];
+    }
+    auto row = [&](const int e) { return 32 * (e >> 5) + 8 * ((e >> 2) & 3) + 4 * half + (e & 3); };       // of accumulator e, in the tile
+    auto column = [&](const int e) { return n0 + 32 * ((e >> 4) & 1) + r0; };
+    uint32_t again = 0;                                        // of the lane's elements those that are not finite
+#pragma unroll
+    for (int i = 0; i < 64 / W; ++i) {
+        const int e = wave * (64 / W) + i;
+        if (m0 + row(e) >= g.M || column(e) >= g.N) continue;
+        if (fabsf(v[i]) <= 3.4028234e38f) write<EPI>(g, m0 + row(e), column(e), v[i]);
+        else again |= 1u << i;
+    }
+    if (__builtin_amdgcn_ballot_w64(again != 0) == 0) return;
+    // (as above)
+    uint32_t rows_a[2], cols_b[2];
+    const int middle = (g.K / 2 + 3) / 4 * 4, k0 = half ? middle : 0, k1 = half ? g.K : middle;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uint64_t in_a = __builtin_amdgcn_ballot_w64(any_nan<false>(g.A, g.lda, m0 + 32 * i + r0, g.M, k0, k1));
+        const uint64_t in_b = __builtin_amdgcn_ballot_w64(any_nan<false>(g.B, g.ldb, n0 + 32 * i + r0, g.N, k0, k1));
+        rows_a[i] = (uint32_t)in_a | (uint32_t)(in_a >> 32);
+        cols_b[i] = (uint32_t)in_b | (uint32_t)(in_b >> 32);
+    }
+    for (; again; again &= again - 1) {
+        const int e = wave * (64 / W) + __builtin_ctz(again), j = (e >> 4) & 1;
+        const bool nan = ((e >> 5 ? rows_a[1] : rows_a[0]) >> (row(e) & 31) | (j ? cols_b[1] : cols_b[0]) >> r0) & 1;
+        write<EPI>(g, m0 + row(e), column(e), nan ? __builtin_nanf("") : plain_dot<false, false>(g, m0 + row(e), column(e)));
     }
 }
 
@@ -233,15 +376,24 @@ int gemm_go(GemmArgs g, hipStream_t st)
     g.tiles   = tm * g.tiles_n;
     g.per_xcd = (g.tiles + 7) / 8;
     const dim3 grid((unsigned)g.per_xcd * 8);
-    // Groups per tile: four waves per SIMD where the tiles allow.
-#define GO(G_) do { \
-        constexpr size_t sums = (G_) > 1 ? (size_t)(G_) * 4 * 16 * 64 * 4 : 0; \
-        hipLaunchKernelGGL((gemm_f32_kernel<AK, BK, G_, EPI>), grid, dim3(G_ * 256), G_ * 2 * STAGE > sums ? G_ * 2 * STAGE : sums, st, g); \
-    } while (0)
-    if (g.tiles > 640)      GO(1);
-    else if (g.tiles > 320) GO(2);
-    else                    GO(4);
+    if constexpr (!AK) {
+        // Waves per tile: two per SIMD where the steps allow.
+#define GO(W_) hipLaunchKernelGGL((gemm_f32_rows_kernel<W_, EPI>), grid, dim3(W_ * 64), (size_t)W_ * 64 * 64 * 4, st, g)
+        if (g.tiles > 512)      GO(2);
+        else if (g.tiles > 256) GO(4);
+        else                    GO(8);
 #undef GO
+    } else {
+        // Groups per tile: four waves per SIMD where the tiles allow.
+#define GO(G_) do { \
+            constexpr size_t sums = (G_) > 1 ? (size_t)(G_) * 4 * 16 * 64 * 4 : 0; \
+            hipLaunchKernelGGL((gemm_f32_kernel<AK, BK, G_, EPI>), grid, dim3(G_ * 256), G_ * 2 * STAGE > sums ? G_ * 2 * STAGE : sums, st, g); \
+        } while (0)
+        if (g.tiles > 640)      GO(1);
+        else if (g.tiles > 320) GO(2);
+        else                    GO(4);
+#undef GO
+    }
     return (int)hipGetLastError();
 }
 
