@@ -223,7 +223,7 @@ void we_aniso_grid_tables_kernel(const float* __restrict__ cb_magnitudes, const 
 // ---- main kernel ----
 
 // What decides whether a pair has a cell: n = rint((r - c A)/h) >= 1 and 2^floor(log2 n) h / r <= 2.
-struct Place { float A, r, inv, u, nf, x, c; uint32_t eb; };
+struct Place { float A, r, inv, u, um, x, c; uint32_t eb; };
 
 __device__ __forceinline__ Place wa_place(const float dx, const float dy, const float dz, const float4& b, const float mid, const float inv_h, const float magic, const uint32_t emask, float& r2)
 {
@@ -232,67 +232,38 @@ __device__ __forceinline__ Place wa_place(const float dx, const float dy, const 
     p.A = (b.x * dx + b.y * dy + b.z * dz) * p.inv;
     const float s = __builtin_fmaf(-mid, p.A, p.r);
     p.u  = __builtin_fmaf(s, inv_h, magic);
-    p.nf = __builtin_fmaxf(p.u, magic) - magic;               // (a value that is not a number becomes 0)
-    p.x  = __builtin_fmaf(s, inv_h, -p.nf);
-    p.eb = __builtin_bit_cast(uint32_t, p.nf) & emask;
+    p.um = __builtin_fmaxf(p.u, magic);                       // magic + n (a value that is not a number becomes 0)
+    const float nf = p.um - magic;
+    p.x  = __builtin_fmaf(s, inv_h, -nf);
+    p.eb = __builtin_bit_cast(uint32_t, nf) & emask;
     p.c  = p.inv * __builtin_bit_cast(float, p.eb);           // 2^e / r; 0 for n = 0
     return p;
 }
 
-// The pairs of one observer that have no cell, summed directly by one wave, a lane per wavenumber.
-template <bool GRADS>
-__device__ void wa_near(const float4* __restrict__ src, const float4* __restrict__ srcb, const int n, const float xi, const float yi, const float zi,
-                        const float mid, const float inv_h, const float climit,
-                        const float* __restrict__ cb_magnitudes, const float* __restrict__ wavenumbers,
-                        float* __restrict__ o, float* __restrict__ ob, float* __restrict__ ok, const int K, const int lane)
+// Source j's pair with an observer: has it no cell?
+__device__ __forceinline__ bool wa_no_cell(const float4& b, const float dx, const float dy, const float dz, const float mid, const float inv_h, WgPair& p)
 {
-    for (int kb = 0; kb < K; kb += 128) {
-        float kr[2], cb[2], s[2][GRADS ? 6 : 2];
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int k = kb + 64 * u + lane;
-            kr[u] = (float)((k < K ? (double)wavenumbers[k] : 0.0) * 0.15915494309189533577);
-            cb[u] = k < K ? cb_magnitudes[k] : 0.f;
-#pragma unroll
-            for (int i = 0; i < (GRADS ? 6 : 2); ++i) s[u][i] = 0.f;
-        }
-        for (int j0 = 0; j0 < n; j0 += 64) {
-            const float4 q = src[j0 + lane];
-            float r2;
-            const Place p = wa_place(xi - q.x, yi - q.y, zi - q.z, srcb[j0 + lane], mid * WG_UNIT, inv_h, WG_MAGIC, 0xff800000u, r2);
-            const bool near = !(p.u > WG_MAGIC) || p.c > climit;
-            uint64_t todo = __builtin_amdgcn_ballot_w64(j0 + lane < n && r2 != 0.0f && near);
-            const float r = p.r * (1.0f / WG_UNIT), m = p.inv * WG_UNIT;
-            while (todo) {
-                const int b = __builtin_ctzll(todo);
-                todo &= todo - 1;
-                const float rb = wg_lane(r, b), mb = wg_lane(m, b), Ab = wg_lane(p.A, b);
-#pragma unroll
-                for (int u = 0; u < 2; ++u) {
-                    const float ph = __builtin_amdgcn_fractf(__builtin_fmaf(-cb[u], Ab, rb) * kr[u]);
-                    const float cs = __builtin_amdgcn_cosf(ph), sn = __builtin_amdgcn_sinf(ph);
-                    s[u][0] = __builtin_fmaf(cs, mb, s[u][0]);
-                    s[u][1] = __builtin_fmaf(sn, mb, s[u][1]);
-                    if constexpr (GRADS) {
-                        s[u][2] += cs; s[u][3] += sn;
-                        s[u][4] = __builtin_fmaf(cs, mb * Ab, s[u][4]);
-                        s[u][5] = __builtin_fmaf(sn, mb * Ab, s[u][5]);
-                    }
-                }
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int k = kb + 64 * u + lane;
-            if (k >= K) continue;
-            auto put = [&](float* to, float re, float im) {
-                to[2 * k] += re; to[2 * k + 1] += im;
-            };
-            put(o, s[u][0], s[u][1]);
-            if constexpr (GRADS) {
-                put(ok, -s[u][3] + cb[u] * s[u][5], s[u][2] - cb[u] * s[u][4]);
-                put(ob, wavenumbers[k] * s[u][5], -wavenumbers[k] * s[u][4]);
-            }
+    float r2;
+    const Place w = wa_place(dx, dy, dz, b, mid * WG_UNIT, inv_h, WG_MAGIC, 0xff800000u, r2);
+    p.r = w.r * (1.0f / WG_UNIT); p.m = w.inv * WG_UNIT; p.A = w.A;
+    return r2 != 0.0f && (!(w.u > WG_MAGIC) || w.c > 2.0f * inv_h);
+}
+
+// add(pair) for the pairs of one observer that have no cell, more of them than the lists hold.
+template <class Add>
+__device__ __forceinline__ void wa_every_near(const float4* __restrict__ src, const float4* __restrict__ srcb, const int n, const float xi, const float yi, const float zi,
+                                              const float mid, const float inv_h, const int lane, Add add)
+{
+    for (int j0 = 0; j0 < n; j0 += 64) {
+        const float4 q = src[j0 + lane];
+        WgPair mine;
+        uint64_t todo = __builtin_amdgcn_ballot_w64(wa_no_cell(srcb[j0 + lane], xi - q.x, yi - q.y, zi - q.z, mid, inv_h, mine) && j0 + lane < n);
+        while (todo) {
+            const int b = __builtin_ctzll(todo);
+            todo &= todo - 1;
+            WgPair p;
+            p.r = wg_lane(mine.r, b); p.m = wg_lane(mine.m, b); p.A = wg_lane(mine.A, b);
+            add(p);
         }
     }
 }
@@ -353,16 +324,22 @@ __device__ __forceinline__ void wa_grids(uint32_t* s_grid, int* s_near, const in
             const int from = (lane >> 4) * quarter + wave * 2;
             const float4* p = src + from;
             const float4* pb = srcb + from;
-            auto spread = [&](const float4& q, const float4& qb) {
+            float ua, ca;
+            auto spread = [&](const float4& q, const float4& qb, auto second) {
                 float r2;
                 const Place w = wa_place(me.x - q.x, me.y - q.y, me.z - q.z, qb, midv, inv_hv, magic, emask, r2);
                 float wt[6];
                 kernel.template weights<GP == 1>(w.x, w.c, wt);
-                const uint32_t ub = __builtin_bit_cast(uint32_t, w.nf + magic);
+                const uint32_t ub = __builtin_bit_cast(uint32_t, w.um);
                 uint32_t at = (ub << 6) + base + (w.eb >> 14);
-                at = ub - first < (uint32_t)cells && !(w.c > climit) ? at : trash;
-                lowest  = __builtin_fminf(lowest, w.u);
-                largest = __builtin_fmaxf(largest, w.c);
+                // (both conditions looked at: with && the compiler branches on the first, twice a pair)
+                const bool in = (ub - first < (uint32_t)cells) & !(w.c > climit);
+                at = in ? at : trash;
+                // (the second of two pairs answers for both in instructions of three operands)
+                if (decltype(second)::value) {
+                    lowest  = __builtin_fminf(__builtin_fminf(ua, w.u), lowest);
+                    largest = __builtin_fmaxf(__builtin_fmaxf(ca, w.c), largest);
+                } else { ua = w.u; ca = w.c; }
                 wg_lds_u32* a = (wg_lds_u32*)(uintptr_t)at;
                 auto add = [&](const int row, const uint32_t v) { __hip_atomic_fetch_add(a + row * WG_OBS, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
                 if (GP == 1) {
@@ -385,9 +362,9 @@ __device__ __forceinline__ void wa_grids(uint32_t* s_grid, int* s_near, const in
             for (int it = 0;;) {
                 for (; it < until; ++it) {
                     p += STEP / 4; pb += STEP / 4;
-                    spread(qa, ba);
+                    spread(qa, ba, wg_false{});
                     qa = p[0]; ba = pb[0];
-                    spread(qb, bb);
+                    spread(qb, bb, wg_true{});
                     qb = p[1]; bb = pb[1];
                 }
                 if (!flushes) break;
@@ -482,6 +459,7 @@ void we_aniso_grid_kernel(const char* __restrict__ ws, const float* __restrict__
     __shared__ float s_red[WAVES];
     __shared__ int   s_near[WG_OBS];
     __shared__ int   s_tok[WG_OBS];
+    __shared__ int   s_cnt[WAVES];
 
     const WgLayout L = wg_layout(Z, N, K, true);
     const int tid = threadIdx.x, lane = tid & 63;
@@ -519,12 +497,52 @@ void we_aniso_grid_kernel(const char* __restrict__ ws, const float* __restrict__
     if (!GRADS && terms == 1) wa_grids<GRADS, 1, WAVES>(s_grid, s_near, s_tok, ws, L, cb_magnitudes, wavenumbers, out, d_cb, d_k, src, srcb, me, ok, n, slot0, ncell, zN, K);
     else                      wa_grids<GRADS, 2, WAVES>(s_grid, s_near, s_tok, ws, L, cb_magnitudes, wavenumbers, out, d_cb, d_k, src, srcb, me, ok, n, slot0, ncell, zN, K);
 
+    // ---- pairs without a cell ----
     __syncthreads();
-    for (int q = wave; q < WG_OBS; q += WAVES) {
-        if (slot0 + q >= n || !s_near[q]) continue;
+    const uint32_t near = (uint32_t)__builtin_amdgcn_ballot_w64(lane < WG_OBS && ok && s_near[obs]);
+    if (near == 0) return;
+    // They lie within |c A| + h / 2: without a cell r - c A <= h/2 or 2^floor(log2 n) h / r > 2, and 2^floor(log2 n) h <= r - c A + h/2.
+    const float closest = (fabsf(mid_cb) * WG_UNIT * params->b_max + 0.5f / inv_h) * 1.001f;
+    auto find = [&](int j, float dx, float dy, float dz, WgPair& p) {
+        return wa_no_cell(srcb[j], dx, dy, dz, mid_cb, inv_h, p);
+    };
+    // all observers' lists at once, or one observer's after the other where that is too much
+    bool listed = wg_collect<WAVES>(s_grid, s_cnt, near, src, n, me, closest * closest, find);
+    const bool together = listed;
+    int unit = 0;                                              // an observer and 64 wavenumbers for a wave
+    for (uint32_t left = near; left; left &= left - 1) {
+        const int q = __builtin_ctz(left);
+        if (!together) {
+            __syncthreads();                                   // the last observer's list is read
+            listed = wg_collect<WAVES>(s_grid, s_cnt, left & (0u - left), src, n, me, closest * closest, find);
+        }
         const size_t row = (zN + s_tok[q]) * 2 * K;
-        wa_near<GRADS>(src, srcb, n, wg_lane(me.x, q), wg_lane(me.y, q), wg_lane(me.z, q), mid_cb, inv_h, 2.0f * inv_h,
-                       cb_magnitudes, wavenumbers, out + row, GRADS ? d_cb + row : nullptr, GRADS ? d_k + row : nullptr, K, lane);
+        for (int kb = 0; kb < K; kb += 64) {
+            if ((unit++ & (WAVES - 1)) != wave) continue;
+            const int k = kb + lane;
+            const float kr = (float)((k < K ? (double)wavenumbers[k] : 0.0) * 0.15915494309189533577), cb = k < K ? cb_magnitudes[k] : 0.f;
+            float s[GRADS ? 6 : 2] = {};
+            auto add = [&](const WgPair& p) {
+                const float ph = __builtin_amdgcn_fractf(__builtin_fmaf(-cb, p.A, p.r) * kr);
+                const float cs = __builtin_amdgcn_cosf(ph), sn = __builtin_amdgcn_sinf(ph);
+                s[0] = __builtin_fmaf(cs, p.m, s[0]);
+                s[1] = __builtin_fmaf(sn, p.m, s[1]);
+                if constexpr (GRADS) {
+                    s[2] += cs; s[3] += sn;
+                    s[4] = __builtin_fmaf(cs, p.m * p.A, s[4]);
+                    s[5] = __builtin_fmaf(sn, p.m * p.A, s[5]);
+                }
+            };
+            if (listed) wg_listed<WAVES>(s_grid, s_cnt, q, add);
+            else wa_every_near(src, srcb, n, wg_lane(me.x, q), wg_lane(me.y, q), wg_lane(me.z, q), mid_cb, inv_h, lane, add);
+            if (k >= K) continue;
+            auto put = [&](float* to, float re, float im) { to[row + 2 * k] += re; to[row + 2 * k + 1] += im; };
+            put(out, s[0], s[1]);
+            if constexpr (GRADS) {
+                put(d_k, -s[3] + cb * s[5], s[2] - cb * s[4]);
+                put(d_cb, wavenumbers[k] * s[5], -wavenumbers[k] * s[4]);
+            }
+        }
     }
 }
 

@@ -313,6 +313,84 @@ __device__ __forceinline__ float wg_reach(const float4& me, const bool ok, const
     return (__builtin_sqrtf(far2) + __builtin_sqrtf(ex * ex + ey * ey + ez * ez)) * 1.00001f;
 }
 
+// Pairs of a workgroup's observers that no cell takes: a list per wave in the LDS that the grids no longer need.
+struct WgPair { float r, m, A; int obs; };                     // distance, 1/r, (anisotropic) A; in units of length
+
+// Every wave searches its share of the sources for them, 256 on their way while the 256 before are looked at: only what lies within
+// `reach2` (squared, scaled) of an observer in `near` is placed.  (One wave per observer, which waited for memory at every 64 sources and did
+// the sums as it met them, took as long as the spread where most workgroups have such an observer: compact chains, us before and now,
+// isotropic 1 x 16384 with the sums 476 / 384, 1 x 65536 5348 / 4608, 1 x 8192 anisotropic 249 / 155, 1 x 2000 58 / 51, extended 1 x 4000 95 / 71.)  find(j, dx, dy, dz, pair): does source j's pair have no cell?
+// Returns (to all threads) whether the lists hold all of them; a list is in the order of the sources.
+template <int WAVES, class Find>
+__device__ __forceinline__ bool wg_collect(uint32_t* s_grid, int* s_cnt, const uint32_t near, const float4* __restrict__ src, const int n, const float4& me,
+                                           const float reach2, Find find)
+{
+    constexpr int CAP = WG_ROWS * WG_OBS * 4 / 16 / WAVES, BATCH = 4;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    WgPair* const list = reinterpret_cast<WgPair*>(s_grid) + wave * CAP;
+    const int share = (n + WAVES * 64 * BATCH - 1) / (WAVES * 64 * BATCH) * (64 * BATCH);
+    const int end = min((wave + 1) * share, n);
+    int count = 0;
+    float4 next[BATCH];
+    if (wave * share < end)
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i) next[i] = src[wave * share + 64 * i + lane];
+    for (int j0 = wave * share; j0 < end; j0 += 64 * BATCH) {
+        float4 q[BATCH];
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i) q[i] = next[i];
+        if (j0 + 64 * BATCH < end)
+#pragma unroll
+            for (int i = 0; i < BATCH; ++i) next[i] = src[j0 + 64 * (BATCH + i) + lane];        // (less than 256 past n: inside the list's padding)
+        for (uint32_t left = near; left; left &= left - 1) {
+            const int o = __builtin_ctz(left);
+            const float xi = wg_lane(me.x, o), yi = wg_lane(me.y, o), zi = wg_lane(me.z, o);
+#pragma unroll
+            for (int i = 0; i < BATCH; ++i) {
+                const int j = j0 + 64 * i + lane;
+                const float dx = xi - q[i].x, dy = yi - q[i].y, dz = zi - q[i].z;
+                const bool close = j < n && dx * dx + dy * dy + dz * dz <= reach2;
+                if (__builtin_amdgcn_ballot_w64(close) == 0) continue;
+                WgPair p;
+                p.obs = o;
+                const uint64_t hits = __builtin_amdgcn_ballot_w64(find(j, dx, dy, dz, p) && close);
+                const int at = count + __builtin_popcountll(hits & ((1ull << lane) - 1ull));
+                if ((hits >> lane & 1) && at < CAP) list[at] = p;
+                count += __builtin_popcountll(hits);
+            }
+        }
+    }
+    if (lane == 0) s_cnt[wave] = count;
+    __syncthreads();
+    bool all = true;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) all &= s_cnt[w] <= CAP;
+    return all;
+}
+
+// add(pair) for the listed pairs of observer o, in the order of the sources.
+template <int WAVES, class Add>
+__device__ __forceinline__ void wg_listed(const uint32_t* s_grid, const int* s_cnt, const int o, Add add)
+{
+    constexpr int CAP = WG_ROWS * WG_OBS * 4 / 16 / WAVES;
+    for (int w = 0; w < WAVES; ++w) {
+        const WgPair* list = reinterpret_cast<const WgPair*>(s_grid) + w * CAP;
+        const int count = __builtin_amdgcn_readfirstlane(s_cnt[w]);
+        for (int i0 = 0; i0 < count; i0 += 64) {
+            const int lane = threadIdx.x & 63;
+            const WgPair mine = list[min(i0 + lane, count - 1)];
+            uint64_t todo = __builtin_amdgcn_ballot_w64(i0 + lane < count && mine.obs == o);
+            while (todo) {
+                const int b = __builtin_ctzll(todo);
+                todo &= todo - 1;
+                WgPair p;
+                p.r = wg_lane(mine.r, b); p.m = wg_lane(mine.m, b); p.A = wg_lane(mine.A, b);
+                add(p);
+            }
+        }
+    }
+}
+
 // The integers of GP grids in LDS, of which the first `used` rows hold anything.
 template <int GP, int THREADS>
 __device__ __forceinline__ void wg_clear(uint32_t* s_grid, const int used)

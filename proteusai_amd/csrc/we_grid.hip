@@ -48,46 +48,23 @@ void we_grid_prepare_kernel(const float* __restrict__ coords, const int layout, 
     if (unit < WG_GROUPS * L.nkt) wg_fill_tables(wavenumbers, ws, L, K, h, unit);
 }
 
-// The sources of `near` pairs of one observer, summed directly by one wave, a lane per wavenumber.
-template <bool SUMS>
-__device__ void wg_near(const float4* __restrict__ src, const int n, const float xi, const float yi, const float zi, const float inv_h,
-                        const float* __restrict__ wavenumbers, float* __restrict__ o, float* __restrict__ pc, float* __restrict__ ps, const int K, const int lane)
+// add(pair) for the pairs of one observer that are closer than h / 2, more of them than the lists hold (thousands of tokens in one place).
+template <class Add>
+__device__ __forceinline__ void wg_every_near(const float4* __restrict__ src, const int n, const float xi, const float yi, const float zi, const float inv_h,
+                                              const int lane, Add add)
 {
-    for (int kb = 0; kb < K; kb += 256) {
-        float kr[4], oc[4], os[4], c[4], s[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int k = kb + 64 * u + lane;
-            kr[u] = (float)((k < K ? (double)wavenumbers[k] : 0.0) * 0.15915494309189533577) * (1.0f / WG_UNIT);
-            oc[u] = os[u] = c[u] = s[u] = 0.f;
-        }
-        for (int j0 = 0; j0 < n; j0 += 64) {
-            const float4 q = src[j0 + lane];
-            float r2, inv, r;
-            wg_distance(xi - q.x, yi - q.y, zi - q.z, r2, inv, r);
-            const bool near = __builtin_bit_cast(int, __builtin_fmaf(r, inv_h, WG_MAGIC)) == __builtin_bit_cast(int, WG_MAGIC);
-            uint64_t todo = __builtin_amdgcn_ballot_w64(j0 + lane < n && r2 != 0.0f && near);
-            while (todo) {
-                const int b = __builtin_ctzll(todo);
-                todo &= todo - 1;
-                const float rb = wg_lane(r, b), mb = wg_lane(inv, b);
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    if (kb + 64 * u >= K) break;
-                    const float ph = __builtin_amdgcn_fractf(rb * kr[u]);
-                    const float cs = __builtin_amdgcn_cosf(ph), sn = __builtin_amdgcn_sinf(ph);
-                    oc[u] = __builtin_fmaf(cs, mb, oc[u]);
-                    os[u] = __builtin_fmaf(sn, mb, os[u]);
-                    if (SUMS) { c[u] += cs; s[u] += sn; }
-                }
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int k = kb + 64 * u + lane;
-            if (k >= K) continue;
-            o[2 * k] += oc[u] * WG_UNIT; o[2 * k + 1] += os[u] * WG_UNIT;
-            if (SUMS) { pc[k] += c[u]; ps[k] += s[u]; }
+    for (int j0 = 0; j0 < n; j0 += 64) {
+        const float4 q = src[j0 + lane];
+        float r2, inv, r;
+        wg_distance(xi - q.x, yi - q.y, zi - q.z, r2, inv, r);
+        const bool near = __builtin_bit_cast(int, __builtin_fmaf(r, inv_h, WG_MAGIC)) == __builtin_bit_cast(int, WG_MAGIC);
+        uint64_t todo = __builtin_amdgcn_ballot_w64(j0 + lane < n && r2 != 0.0f && near);
+        while (todo) {
+            const int b = __builtin_ctzll(todo);
+            todo &= todo - 1;
+            WgPair p;
+            p.r = wg_lane(r, b); p.m = wg_lane(inv, b);
+            add(p);
         }
     }
 }
@@ -206,6 +183,7 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
     __shared__ float s_red[WAVES];
     __shared__ int   s_near[WG_OBS];
     __shared__ int   s_tok[WG_OBS];
+    __shared__ int   s_cnt[WAVES];
 
     const WgLayout L = wg_layout(Z, N, K, false);
     const int tid = threadIdx.x, lane = tid & 63;
@@ -398,11 +376,46 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
 
     // ---- pairs closer than h / 2 ----
     __syncthreads();
-    for (int q = wave; q < WG_OBS; q += WAVES) {
-        if (slot0 + q >= n || !s_near[q]) continue;
+    const uint32_t near = (uint32_t)__builtin_amdgcn_ballot_w64(lane < WG_OBS && ok && s_near[obs]);
+    if (near == 0) return;
+    const float closest = 0.5005f / inv_h;
+    auto find = [&](int, float dx, float dy, float dz, WgPair& p) {
+        float r2, inv, r;
+        wg_distance(dx, dy, dz, r2, inv, r);
+        p.r = r; p.m = inv; p.A = 0.f;
+        return r2 != 0.0f && __builtin_bit_cast(int, __builtin_fmaf(r, inv_h, WG_MAGIC)) == __builtin_bit_cast(int, WG_MAGIC);
+    };
+    // all observers' lists at once, or one observer's after the other where that is too much
+    bool listed = wg_collect<WAVES>(s_grid, s_cnt, near, src, n, me, closest * closest, find);
+    const bool together = listed;
+    int unit = 0;                                              // an observer and 64 wavenumbers for a wave
+    for (uint32_t left = near; left; left &= left - 1) {
+        const int q = __builtin_ctz(left);
+        if (!together) {
+            __syncthreads();                                   // the last observer's list is read
+            listed = wg_collect<WAVES>(s_grid, s_cnt, left & (0u - left), src, n, me, closest * closest, find);
+        }
         const size_t row = zN + s_tok[q];
-        wg_near<SUMS>(src, n, wg_lane(me.x, q), wg_lane(me.y, q), wg_lane(me.z, q), inv_h, wavenumbers, out + row * 2 * K,
-                      SUMS ? cos_sums + row * K : nullptr, SUMS ? sin_sums + row * K : nullptr, K, lane);
+        for (int kb = 0; kb < K; kb += 64) {
+            if ((unit++ & (WAVES - 1)) != wave) continue;
+            const int k = kb + lane;
+            const float kr = (float)((k < K ? (double)wavenumbers[k] : 0.0) * 0.15915494309189533577) * (1.0f / WG_UNIT);
+            float oc = 0.f, os = 0.f, c = 0.f, s = 0.f;
+            auto add = [&](const WgPair& p) {
+                const float ph = __builtin_amdgcn_fractf(p.r * kr);
+                const float cs = __builtin_amdgcn_cosf(ph), sn = __builtin_amdgcn_sinf(ph);
+                oc = __builtin_fmaf(cs, p.m, oc);
+                os = __builtin_fmaf(sn, p.m, os);
+                if (SUMS) { c += cs; s += sn; }
+            };
+            if (listed) wg_listed<WAVES>(s_grid, s_cnt, q, add);
+            else wg_every_near(src, n, wg_lane(me.x, q), wg_lane(me.y, q), wg_lane(me.z, q), inv_h, lane, add);
+            if (k < K) {
+                float* o = out + row * 2 * K;
+                o[2 * k] += oc * WG_UNIT; o[2 * k + 1] += os * WG_UNIT;
+                if (SUMS) { cos_sums[row * K + k] += c; sin_sums[row * K + k] += s; }
+            }
+        }
     }
 }
 
