@@ -388,7 +388,7 @@ __device__ __forceinline__ void wa_grids(uint32_t* s_grid, int* s_near, const in
                 const int k = kp * 16 + obs;
                 // (a tile that takes part in the first of two terms only runs the product of the second for nothing, every other pass)
                 wg_f4 ec[GP][1], os[GP][1], oc[GP][1], es[GP][1];
-                wg_product<1, WAVES == 16 ? 4 : 2, GRADS, GP>(reinterpret_cast<const float*>(s_grid), WgGrid<GP>::ROWS * WG_OBS, mid, groups,
+                wg_product<1, WAVES == 16 ? 4 : 2, GRADS, GP>(reinterpret_cast<const float*>(s_grid), WgGrid<GP>::ROWS * WG_OBS, mid, 0, groups,
                                                               table + (size_t)kp * 64 + lane, (size_t)L.nkt * 64, 0, ec, os, oc, es);
                 // (what earlier terms and windows left, all loads in flight at once; with the two grids sharing the reads of the tables 251 -> 240 us
                 // at 4 x 1000 tokens, 10 terms, partial derivatives)

@@ -460,9 +460,9 @@ __device__ __forceinline__ void wg_combine(uint32_t* s_grid, wg_f4 (&acc)[CHUNKS
 
 // GR grids (`gs` floats apart) at KT tiles of 16 wavenumbers: rows j = 0 .. groups * 8 on both sides of the middle, E and O the sum
 // and difference of the two sides: ec += E cos, os += O sin and (MOMENT) oc += y O cos, es += y E sin with y = j + 1/2.  The tiles
-// share the grid values, the grids the tables, which come from L2, AHEAD groups of 8 rows ahead.
+// share the grid values, the grids the tables, which come from L2, AHEAD groups of 8 rows ahead.  Of the groups those from `begin` on.
 template <int KT, int AHEAD, bool MOMENT, int GR>
-__device__ __forceinline__ void wg_product(const float* g, const int gs, const int mid, const int groups, const float4* __restrict__ tb, const size_t ts, const int k2,
+__device__ __forceinline__ void wg_product(const float* g, const int gs, const int mid, const int begin, const int groups, const float4* __restrict__ tb, const size_t ts, const int k2,
                                            wg_f4 (&ec)[GR][KT], wg_f4 (&os)[GR][KT], wg_f4 (&oc)[GR][KT], wg_f4 (&es)[GR][KT])
 {
     const int lane = threadIdx.x & 63, obs = lane & 15, mm = lane >> 4;
@@ -479,9 +479,9 @@ __device__ __forceinline__ void wg_product(const float* g, const int gs, const i
         for (int t = 0; t < KT; ++t) bb[t] = at[t * k2];
     };
 #pragma unroll
-    for (int i = 0; i < AHEAD; ++i) fetch(i, b[i]);
-    float y = (float)mm + 0.5f;
-    for (int g0 = 0; g0 < groups; g0 += AHEAD) {
+    for (int i = 0; i < AHEAD; ++i) fetch(begin + i, b[i]);
+    float y = (float)(8 * begin + mm) + 0.5f;
+    for (int g0 = begin; g0 < groups; g0 += AHEAD) {
 #pragma unroll
         for (int i = 0; i < AHEAD; ++i) {
             const int gr = g0 + i;

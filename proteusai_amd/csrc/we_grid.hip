@@ -196,8 +196,8 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
     const float4* __restrict__ table = reinterpret_cast<const float4*>(ws + L.table);
     const float inv_h = reinterpret_cast<const WgParams*>(ws)->inv_h * (1.0f / WG_UNIT), h = reinterpret_cast<const WgParams*>(ws)->h;
 
-    // ---- the workgroup's slots: unpadded observers first, then padded tokens (zero rows), then nothing.  (Workgroups of a further
-    //      blockIdx.z have the same slots: they only take part in direct sums.) ----
+    // ---- the workgroup's slots: unpadded observers first, then padded tokens (zero rows), then nothing.  (Workgroups of every blockIdx.z
+    //      have the same slots and, of the tiles of 16 wavenumbers, every gridDim.z-th.) ----
     const int slot0 = blockIdx.x * WG_OBS;
     const int obs   = lane & 15;
     const float4 me = src[slot0 + obs];
@@ -236,7 +236,6 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
         else                 wg_direct<SUMS, WAVES, false>(s_grid, s_tok, src, n, slot0, me, wavenumbers, out, cos_sums, sin_sums, zN, K, blockIdx.z, gridDim.z);
         return;
     }
-    if (blockIdx.z) return;
     const int ncell = __builtin_amdgcn_readfirstlane((int)reach);
 
     {
@@ -247,6 +246,7 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
         // sources between two flushes stays below 2^32.
         const int nit = (n + STEP - 1) / STEP, quarter = nit * (STEP / 4);
         const bool flushes = nit * STEP > WG_FLUSH;
+        const int tiles = (L.nkt - (int)blockIdx.z + (int)gridDim.z - 1) / (int)gridDim.z;      // of this workgroup
         const float scale = flushes ? 1048000.0f : fminf(4190000.0f, 2147000000.0f / (float)(nit * STEP));
         const WgKernel kernel(scale * h * 0x1p-137f);
         const float magic = wg_vgpr(WG_MAGIC), inv_hv = wg_vgpr(inv_h);
@@ -331,43 +331,82 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
             const int groups = (mid + 7) / 8;
             const int vc     = n_lo - 3 + mid;                              // the middle lies at vc h
             const int mm     = lane >> 4;
-            for (int kp = KT * wave; kp < L.nkt; kp += KT * WAVES) {
-                wg_f4 ec_[1][KT], os_[1][KT], oc_[1][KT], es_[1][KT];
-                // (an odd number of tiles: the last one twice, written once)
-                wg_product<KT, AHEAD, SUMS, 1>(reinterpret_cast<const float*>(s_grid), 0, mid, groups, table + (size_t)kp * 64 + lane, (size_t)L.nkt * 64,
-                                               kp + 1 < L.nkt ? 64 : 0, ec_, os_, oc_, es_);
-                const auto &ec = ec_[0], &os = os_[0], &oc = oc_[0], &es = es_[0];
+            // rows `from` to `to` of a lane's four of a tile
+            auto finish = [&](const int kt, const int from, const int to, const wg_f4& ec, const wg_f4& os, const wg_f4& oc, const wg_f4& es) {
+                const int k = kt * 16 + obs;
+                if (k >= K) return;
+                const WgWave w = waves[k];
+                const double ph = w.rev * (double)vc;
+                const float f  = (float)(ph - __builtin_floor(ph));
+                const float rc = __builtin_amdgcn_cosf(f), rs = __builtin_amdgcn_sinf(f);
+                const float q1 = w.q / (scale * h), q0s = w.q / scale, dq = w.dq / scale;
 #pragma unroll
-                for (int t = 0; t < KT; ++t) {
-                    const int k = (kp + t) * 16 + obs;
-                    if (k >= K) continue;
-                    const WgWave w = waves[k];
-                    const double ph = w.rev * (double)vc;
-                    const float f  = (float)(ph - __builtin_floor(ph));
-                    const float rc = __builtin_amdgcn_cosf(f), rs = __builtin_amdgcn_sinf(f);
-                    const float q1 = w.q / (scale * h), q0s = w.q / scale, dq = w.dq / scale;
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const int  tok  = s_tok[mm * 4 + i];
-                        if (tok < 0) continue;
-                        const bool keep = slot0 + mm * 4 + i < n;
-                        const size_t row = zN + tok;
-                        float2 v = make_float2(q1 * (ec[t][i] * rc - os[t][i] * rs), q1 * (ec[t][i] * rs + os[t][i] * rc));
-                        float2* po = reinterpret_cast<float2*>(out + row * 2 * K) + k;
-                        if (n_lo > 1) { const float2 o = *po; v.x += o.x; v.y += o.y; }
-                        *po = keep ? v : make_float2(0.f, 0.f);
-                        if (SUMS) {
-                            // F0 = rot [ q h (vc G + Gy) - i q' h G ] with G = ec + i os, Gy = oc + i es
-                            const float gr_ = q0s * ((float)vc * ec[t][i] + oc[t][i]) + dq * os[t][i];
-                            const float gi_ = q0s * ((float)vc * os[t][i] + es[t][i]) - dq * ec[t][i];
-                            float c0 = gr_ * rc - gi_ * rs, s0 = gr_ * rs + gi_ * rc;
-                            float* pc = cos_sums + row * K + k;
-                            float* ps = sin_sums + row * K + k;
-                            if (n_lo > 1) { c0 += *pc; s0 += *ps; }
-                            *pc = keep ? c0 : 0.f;
-                            *ps = keep ? s0 : 0.f;
-                        }
+                for (int i = 0; i < 4; ++i) {
+                    if (i < from || i >= to) continue;
+                    const int  tok  = s_tok[mm * 4 + i];
+                    if (tok < 0) continue;
+                    const bool keep = slot0 + mm * 4 + i < n;
+                    const size_t row = zN + tok;
+                    float2 v = make_float2(q1 * (ec[i] * rc - os[i] * rs), q1 * (ec[i] * rs + os[i] * rc));
+                    float2* po = reinterpret_cast<float2*>(out + row * 2 * K) + k;
+                    if (n_lo > 1) { const float2 o = *po; v.x += o.x; v.y += o.y; }
+                    *po = keep ? v : make_float2(0.f, 0.f);
+                    if (SUMS) {
+                        // F0 = rot [ q h (vc G + Gy) - i q' h G ] with G = ec + i os, Gy = oc + i es
+                        const float gr_ = q0s * ((float)vc * ec[i] + oc[i]) + dq * os[i];
+                        const float gi_ = q0s * ((float)vc * os[i] + es[i]) - dq * ec[i];
+                        float c0 = gr_ * rc - gi_ * rs, s0 = gr_ * rs + gi_ * rc;
+                        float* pc = cos_sums + row * K + k;
+                        float* ps = sin_sums + row * K + k;
+                        if (n_lo > 1) { c0 += *pc; s0 += *ps; }
+                        *pc = keep ? c0 : 0.f;
+                        *ps = keep ? s0 : 0.f;
                     }
+                }
+            };
+            const float* grid = reinterpret_cast<const float*>(s_grid);
+            // Fewer tiles than waves: `parts` waves share a tile's rows, at least four groups of 8 each (a wave's reads of the tables are then in flight
+            // at once), and meet in LDS.  With the workgroups' shares, us, one workgroup and a wave a tile / so, with the sums and without: 1 x 700, K = 256
+            // 27.7 / 22.5 and 24.0 / 22.5, 1 x 1024 30.3 / 24.7 and 26.0 / 23.2, 1 x 2000 40.4 / 36.3 and 33.2 / 31.3, 1 x 1200, K = 512 46.8 / 31.8 and
+            // 36.0 / 28.1; with fewer rows than that the meeting costs what it saves (16 x 128, K = 256, without 20.9 / 22.1).
+            int parts = 1;
+            if (WAVES == 16) while (parts < 16 && tiles * parts * 2 <= 16 && groups >= 8 * parts) parts *= 2;
+            if (parts == 1) {
+                // (gridDim.z > 1 for one tile at a time only)
+                for (int kp = KT * wave; kp < tiles; kp += KT * WAVES) {
+                    const int kt = kp * (int)gridDim.z + (int)blockIdx.z;
+                    wg_f4 ec[1][KT], os[1][KT], oc[1][KT], es[1][KT];
+                    // (an odd number of tiles: the last one twice, written once)
+                    wg_product<KT, AHEAD, SUMS, 1>(grid, 0, mid, 0, groups, table + (size_t)kt * 64 + lane, (size_t)L.nkt * 64, kp + 1 < tiles ? 64 : 0, ec, os, oc, es);
+#pragma unroll
+                    for (int t = 0; t < KT; ++t) finish(kt + t, 0, 4, ec[0][t], os[0][t], oc[0][t], es[0][t]);
+                }
+            } else {
+                const int tile = wave / parts, part = wave % parts, kt = tile * (int)gridDim.z + (int)blockIdx.z;
+                constexpr int V = SUMS ? 4 : 2;
+                wg_f4* const red = reinterpret_cast<wg_f4*>(s_grid);              // [16 waves][V][64 lanes]
+                static_assert(16 * V * 64 * 16 <= WG_ROWS * WG_OBS * 4, "sums of the waves in LDS");
+                wg_f4 sum[V];
+                if (tile < tiles) {
+                    const int share = (groups + parts - 1) / parts, begin = min(part * share, groups);
+                    wg_f4 ec[1][1], os[1][1], oc[1][1], es[1][1];
+                    wg_product<1, AHEAD, SUMS, 1>(grid, 0, mid, begin, min(begin + share, groups), table + (size_t)kt * 64 + lane, (size_t)L.nkt * 64, 0, ec, os, oc, es);
+                    sum[0] = ec[0][0]; sum[1] = os[0][0];
+                    if (SUMS) { sum[V - 2] = oc[0][0]; sum[V - 1] = es[0][0]; }
+                }
+                __syncthreads();                                         // the grid is read
+                if (tile < tiles)
+#pragma unroll
+                    for (int v = 0; v < V; ++v) red[(wave * V + v) * 64 + lane] = sum[v];
+                __syncthreads();
+                const int each = parts == 2 ? 2 : 1;                     // of the four rows for a wave
+                if (tile < tiles && part * each < 4) {
+#pragma unroll
+                    for (int v = 0; v < V; ++v) {
+                        sum[v] = red[(tile * parts * V + v) * 64 + lane];
+                        for (int o = 1; o < parts; ++o) sum[v] += red[((tile * parts + o) * V + v) * 64 + lane];
+                    }
+                    finish(kt, part * each, part * each + each, sum[0], sum[1], sum[V - 2], sum[V - 1]);
                 }
             }
         }
@@ -410,7 +449,7 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
             };
             if (listed) wg_listed<WAVES>(s_grid, s_cnt, q, add);
             else wg_every_near(src, n, wg_lane(me.x, q), wg_lane(me.y, q), wg_lane(me.z, q), inv_h, lane, add);
-            if (k < K) {
+            if (k < K && (k >> 4) % (int)gridDim.z == (int)blockIdx.z) {       // (this workgroup's tiles)
                 float* o = out + row * 2 * K;
                 o[2 * k] += oc * WG_UNIT; o[2 * k + 1] += os * WG_UNIT;
                 if (SUMS) { cos_sums[row * K + k] += c; sin_sums[row * K + k] += s; }
@@ -454,7 +493,7 @@ extern "C" int proteus_we_fwd_ws(const float* coords, int coords_layout,
     dim3 grid((N + WG_OBS - 1) / WG_OBS, Z);
     const size_t lds = (size_t)WG_ROWS * WG_OBS * 4;
     const bool few = (long)grid.x * Z <= 256;
-    if (few) grid.z = min(L.nkt, 256 / (int)(grid.x * grid.y));        // (direct sums share the wavenumbers out over the idle compute units)
+    if (few) grid.z = min(L.nkt, 256 / (int)(grid.x * grid.y));        // (idle compute units spread the same pairs and share the wavenumbers out)
 #define WG_GO(S_, W_) hipLaunchKernelGGL((we_grid_kernel<S_, W_>), grid, dim3(W_ * 64), lds, st, (const char*)workspace, wavenumbers, out, cos_sums, sin_sums, Z, N, K)
     if (cos_sums) { if (few) WG_GO(true, 16); else WG_GO(true, 8); }
     else          { if (few) WG_GO(false, 16); else WG_GO(false, 8); }

@@ -1,0 +1,32 @@
+"""The distance grid in launches of at most 256 workgroups: the tiles of 16 wavenumbers are shared out over blockIdx.z, and waves without a tile of
+their own share the rows of one."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import c_oracle
+from proteusai_amd import synth
+from test_we_grid_gpu import rel_l2, run_grid
+
+pytestmark = pytest.mark.gpu
+
+
+# N, Z, K, scale: workgroups of a tile each and 2, 4, 8 and 16 waves on it (short chains have few rows); two and three tiles and four waves on each; 8
+# tiles, 2 waves; an odd number of tiles, a wave each; the last launch that is shared out and the first that is not; several windows
+@pytest.mark.parametrize("N,Z,K,scale", [
+    (40, 1, 33, 1.0), (100, 1, 80, 1.0), (520, 1, 80, 1.0), (2000, 1, 20, 1.0), (900, 1, 163, 1.0), (2000, 1, 250, 1.0), (1300, 1, 720, 1.0),
+    (2048, 1, 64, 1.0), (2049, 1, 64, 1.0), (333, 4, 250, 1.0), (700, 2, 163, 12.0)])
+def test_shared_tiles(gpu, N, Z, K, scale):
+    a, wn = synth.we_inputs(N, seed=N + K, batch=Z)[0] * scale, synth.wavenumbers(2 * K)
+    a[0, 20] = a[0, 30] + torch.tensor([0.01, -0.02, 0.015])          # a pair that no cell takes
+    mask = torch.rand(Z, N, generator=torch.Generator().manual_seed(K)) < 0.1
+    got = run_grid(gpu, a, wn, mask)
+    ref = c_oracle.we(a.numpy(), wn.numpy(), mask.numpy(), precision="f64")
+    # (four times the grid's aliasing and fixed point; a phase rounded to 2^-24 of itself, twice)
+    bar = 1.7e-6 + 2 * 2.0 ** -24 * float(wn.max()) * float((a.amax(1) - a.amin(1)).norm(dim=-1).max())
+    for x, r, what in zip(got, ref, ("out", "cos_sums", "sin_sums")):
+        assert (x[mask.numpy()] == 0).all(), what
+        assert rel_l2(x, r) <= bar, (what, rel_l2(x, r), bar)
+    assert all(np.array_equal(x, y) for x, y in zip(got, run_grid(gpu, a, wn, mask)))
+    lean = run_grid(gpu, a, wn, mask, sums=False)
+    assert np.array_equal(got[0], lean[0])
