@@ -112,7 +112,7 @@ struct WaBoxes {
 
 __global__ __launch_bounds__(256)
 void we_aniso_grid_tables_kernel(const float* __restrict__ cb_magnitudes, const float* __restrict__ wavenumbers,
-                                 char* __restrict__ ws, const int Z, const int N, const int K, const int partials, const int few)
+                                 char* __restrict__ ws, const int Z, const int N, const int K, const int partials, const int few)      // few: workgroups that share a batch's wavenumbers, 0 for the large launch
 {
     const WgLayout L = wg_layout(Z, N, K, true);
     const int tid = threadIdx.x, lane = tid & 63;
@@ -171,9 +171,10 @@ void we_aniso_grid_tables_kernel(const float* __restrict__ cb_magnitudes, const 
         const float windows = __builtin_ceilf(fmaxf(1.0f, cells / (float)most));
         const float rounds  = groups * (1.0f / 512.0f), share = fminf(1.0f, rounds);
         // (16 waves, 28 batches of 1 x 500 ... 2 x 2000 tokens, K = 128 and 256: a preparation of 37 to 53 us, and per pass 0.0128 us per source,
-        // 0.3 ns per cell and wavenumber, half of that without partial derivatives, and 10 us for the flushes of more than 1024 sources.)
+        // 0.3 ns per cell and wavenumber, half of that without partial derivatives, and 10 us for the flushes of more than 1024 sources.
+        // Of the cells' part four fifths are shared by `few` workgroups, which takes 5 us: 1 x 1000, K = 512 203 us with the grids and 198 without.)
         const float passes  = (float)((terms + 1) / 2) * windows;
-        float grid   = few ? (partials ? 53.0f : 37.0f) + passes * (0.0128f * nmax + (partials ? 3.0e-4f : 1.4e-4f) * (float)K * cells / windows
+        float grid   = few ? (partials ? 53.0f : 37.0f) + (few > 1 ? 5.0f : 0.0f) + passes * (0.0128f * nmax + (partials ? 3.0e-4f : 1.4e-4f) * (float)K * (0.2f + 0.8f / (float)few) * cells / windows
                                                                     + (nmax > (float)WA_FLUSH ? 10.0f : 0.0f))
                            : passes * (22.0f + (0.026f + 0.033f * share) * nmax) * fmaxf(1.0f, rounds);
         float direct = pairs * (float)K * (partials ? (few ? 3.7e-7f : 3.4e-7f) : 2.4e-7f);
@@ -270,13 +271,14 @@ __device__ __forceinline__ void wa_every_near(const float4* __restrict__ src, co
 
 // GP  grids per pass over the sources: 1 where the expansion has a single term (then its weights are those of the isotropic kernel,
 //     unsigned denormals), 2 otherwise (signed weights, through the low bits of a magic sum)
-template <bool GRADS, int GP, int WAVES>
+template <bool GRADS, int GP, int WAVES, bool SHARED>
 __device__ __forceinline__ void wa_grids(uint32_t* s_grid, int* s_near, const int* s_tok, const char* __restrict__ ws, const WgLayout& L,
                                          const float* __restrict__ cb_magnitudes, const float* __restrict__ wavenumbers,
                                          float* __restrict__ out, float* __restrict__ d_cb, float* __restrict__ d_k,
                                          const float4* __restrict__ src, const float4* __restrict__ srcb, const float4& me, const bool ok,
                                          const int n, const int slot0, const int ncell, const size_t zN, const int K)
 {
+    const int zk = SHARED ? blockIdx.z : 0, Zk = SHARED ? gridDim.z : 1;            // of the tiles of 16 wavenumbers, this workgroup's are zk, zk + Zk, ...
     constexpr int THREADS = WAVES * 64;
     constexpr int STEP   = WAVES * 8;                     // sources per iteration: a wave takes 16 observers x 4 sources, twice
     constexpr int CHUNKS = (WG_ROWS * WG_OBS / 4 + THREADS - 1) / THREADS;
@@ -382,7 +384,7 @@ __device__ __forceinline__ void wa_grids(uint32_t* s_grid, int* s_near, const in
             const int groups = (mid + 7) / 8;
             const int vc     = n_lo - 3 + mid;
             const bool more  = n_lo > 1 || p0 > 0;
-            for (int kp = wave; kp < L.nkt; kp += WAVES) {
+            for (int kp = wave * Zk + zk; kp < L.nkt; kp += WAVES * Zk) {
                 const int mine = GP == 1 ? 1 : __builtin_amdgcn_readfirstlane(reinterpret_cast<const int*>(ws + L.tiles)[kp]);
                 if (p0 >= mine) continue;
                 const int k = kp * 16 + obs;
@@ -449,7 +451,10 @@ __device__ __forceinline__ void wa_grids(uint32_t* s_grid, int* s_near, const in
 
 // WAVES  8: two workgroups share a compute unit; 16: twice the waves on the same observers, for launches whose workgroups with
 //        unpadded observers have a compute unit to themselves
-template <bool GRADS, int WAVES>
+// SHARED  workgroups of every blockIdx.z have the same slots and, of the tiles of 16 wavenumbers, every gridDim.z-th (of 16 waves, where compute
+//        units would be idle; us, before / so, partial derivatives: 1 x 2000, K = 256, scales spread by 0.2 398 / 270, compact 271 / 236, 1 x 1500, K = 512
+//        431 / 317, 2 x 1000, K = 256 206 / 198.  Launches of one share have kernels of their own: the two scalars cost registers, 4 x 1000 279 / 287)
+template <bool GRADS, int WAVES, bool SHARED>
 __global__ __launch_bounds__(WAVES * 64, 4)
 void we_aniso_grid_kernel(const char* __restrict__ ws, const float* __restrict__ cb_magnitudes, const float* __restrict__ wavenumbers,
                           float* __restrict__ out, float* __restrict__ d_cb, float* __restrict__ d_k, const int Z, const int N, const int K)
@@ -494,8 +499,8 @@ void we_aniso_grid_kernel(const char* __restrict__ ws, const float* __restrict__
     // the observers' own radius are at most twice that.)
     const int ncell = __builtin_amdgcn_readfirstlane((int)((wg_reach<WAVES>(me, ok, reinterpret_cast<const WgBox*>(ws + L.boxes) + (size_t)z * L.nbox, L.nbox, s_red)
                                                             + fabsf(mid_cb) * params->b_max * WG_UNIT) * inv_h + 2.0f));
-    if (!GRADS && terms == 1) wa_grids<GRADS, 1, WAVES>(s_grid, s_near, s_tok, ws, L, cb_magnitudes, wavenumbers, out, d_cb, d_k, src, srcb, me, ok, n, slot0, ncell, zN, K);
-    else                      wa_grids<GRADS, 2, WAVES>(s_grid, s_near, s_tok, ws, L, cb_magnitudes, wavenumbers, out, d_cb, d_k, src, srcb, me, ok, n, slot0, ncell, zN, K);
+    if (!GRADS && terms == 1) wa_grids<GRADS, 1, WAVES, SHARED>(s_grid, s_near, s_tok, ws, L, cb_magnitudes, wavenumbers, out, d_cb, d_k, src, srcb, me, ok, n, slot0, ncell, zN, K);
+    else                      wa_grids<GRADS, 2, WAVES, SHARED>(s_grid, s_near, s_tok, ws, L, cb_magnitudes, wavenumbers, out, d_cb, d_k, src, srcb, me, ok, n, slot0, ncell, zN, K);
 
     // ---- pairs without a cell ----
     __syncthreads();
@@ -535,7 +540,7 @@ void we_aniso_grid_kernel(const char* __restrict__ ws, const float* __restrict__
             };
             if (listed) wg_listed<WAVES>(s_grid, s_cnt, q, add);
             else wa_every_near(src, srcb, n, wg_lane(me.x, q), wg_lane(me.y, q), wg_lane(me.z, q), mid_cb, inv_h, lane, add);
-            if (k >= K) continue;
+            if (k >= K || (SHARED && (k >> 4) % (int)gridDim.z != (int)blockIdx.z)) continue;       // (this workgroup's tiles)
             auto put = [&](float* to, float re, float im) { to[row + 2 * k] += re; to[row + 2 * k + 1] += im; };
             put(out, s[0], s[1]);
             if constexpr (GRADS) {
@@ -549,7 +554,7 @@ void we_aniso_grid_kernel(const char* __restrict__ ws, const float* __restrict__
 // What the grids need beside the direct kernel, two launches of preparation and one that finds nothing to do, costs 13 us.  Without
 // partial derivatives the scales are likely to be equal, where the grid wins from about 1 x 512 tokens on (K = 256: 1 x 512 41 / 49 us,
 // 1 x 2000 79 / 272, 8 x 1000 67 / 486); with them they are likely to differ, and the grids win where the direct kernel takes 400 us or more
-// (4 x 1000 240 / 365, 1 x 2000 315 / 400, 8 x 1000 484 / 701, compact 1 x 8192 1.25 / 5.5 ms; below, 1 x 1500 305 / 238).  A batch with a padding mask is taken to hold 0.4 of its pairs.
+// (4 x 1000 240 / 365, 1 x 2000 268 / 398, 8 x 1000 484 / 701, compact 1 x 8192 1.25 / 5.5 ms; below, 1 x 1500 305 / 238).  A batch with a padding mask is taken to hold 0.4 of its pairs.
 bool we_aniso_grid_wanted(int Z, int N, int K, bool partials, bool padded, int tuning)
 {
     return tuning == 0 && K >= 64 && (padded ? 0.4 : 1.0) * Z * N * N * K >= (partials ? 1.0e9 : 2.0e8);
@@ -577,14 +582,16 @@ extern "C" int proteus_we_aniso_fwd_ws(const float* coordsA, const float* coords
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     char* ws = (char*)workspace;
     hipLaunchKernelGGL(we_aniso_grid_sources_kernel, dim3((unsigned)Z * (unsigned)L.blocks), dim3(256), 0, st, coordsA, coordsB, coords_layout, mask, ws, Z, N, K);
-    const bool few = wa_few(Z, N, mask != nullptr);
+    dim3 grid((N + WG_OBS - 1) / WG_OBS, Z);
+    // (idle compute units spread the same pairs and share the wavenumbers out)
+    const int few = wa_few(Z, N, mask != nullptr) ? max(1, min(L.nkt, 256 / (int)(grid.x * grid.y))) : 0;
+    if (few) grid.z = few;
     const unsigned units = (unsigned)((WG_GROUPS + (WG_MAX_TERMS + 3) / 4) * L.nkt);
-    hipLaunchKernelGGL(we_aniso_grid_tables_kernel, dim3((units + 3) / 4 + 1), dim3(256), 0, st, cb_magnitudes, wavenumbers, ws, Z, N, K, d_cb ? 1 : 0, few ? 1 : 0);
-    const dim3 grid((N + WG_OBS - 1) / WG_OBS, Z);
+    hipLaunchKernelGGL(we_aniso_grid_tables_kernel, dim3((units + 3) / 4 + 1), dim3(256), 0, st, cb_magnitudes, wavenumbers, ws, Z, N, K, d_cb ? 1 : 0, few);
     const size_t lds = (size_t)WG_ROWS * WG_OBS * 4;
-#define WA_GO(G_, W_) hipLaunchKernelGGL((we_aniso_grid_kernel<G_, W_>), grid, dim3(W_ * 64), lds, st, (const char*)ws, cb_magnitudes, wavenumbers, out, d_cb, d_k, Z, N, K)
-    if (d_cb) { if (few) WA_GO(true, 16); else WA_GO(true, 8); }
-    else      { if (few) WA_GO(false, 16); else WA_GO(false, 8); }
+#define WA_GO(G_, W_, S_) hipLaunchKernelGGL((we_aniso_grid_kernel<G_, W_, S_>), grid, dim3(W_ * 64), lds, st, (const char*)ws, cb_magnitudes, wavenumbers, out, d_cb, d_k, Z, N, K)
+    if (d_cb) { if (few > 1) WA_GO(true, 16, true); else if (few) WA_GO(true, 16, false); else WA_GO(true, 8, false); }
+    else      { if (few > 1) WA_GO(false, 16, true); else if (few) WA_GO(false, 16, false); else WA_GO(false, 8, false); }
 #undef WA_GO
     const int rl = (int)hipGetLastError();
     if (rl) return rl;

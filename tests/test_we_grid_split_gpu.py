@@ -6,7 +6,7 @@ import torch
 
 from oracle import c_oracle
 from proteusai_amd import synth
-from test_we_grid_gpu import rel_l2, run_grid
+from test_we_grid_gpu import rel_l2, run_aniso, run_grid
 
 pytestmark = pytest.mark.gpu
 
@@ -30,3 +30,26 @@ def test_shared_tiles(gpu, N, Z, K, scale):
     assert all(np.array_equal(x, y) for x, y in zip(got, run_grid(gpu, a, wn, mask)))
     lean = run_grid(gpu, a, wn, mask, sums=False)
     assert np.array_equal(got[0], lean[0])
+
+
+# one tile a workgroup; two and three; several windows; a single grid (equal scales); the last launch that is shared out and the first that is not
+@pytest.mark.parametrize("N,Z,K,scale,spread", [
+    (100, 1, 80, 1.0, 0.1), (520, 1, 80, 1.0, 0.1), (900, 1, 163, 1.0, 0.1), (333, 4, 250, 1.0, 0.05), (700, 2, 163, 6.0, 0.1), (1000, 1, 250, 1.0, 0.0),
+    (2048, 1, 64, 1.0, 0.1), (2049, 1, 64, 1.0, 0.1)])
+def test_shared_tiles_anisotropic(gpu, N, Z, K, scale, spread):
+    a, wn = synth.we_inputs(N, seed=N + K, batch=Z)[0] * scale, synth.wavenumbers(2 * K)
+    a[0, 20] = a[0, 30] + torch.tensor([0.01, -0.02, 0.015])
+    g = torch.Generator().manual_seed(K + N)
+    b = torch.randn(Z, N, 3, generator=g)
+    b = 1.5 * b / b.norm(dim=-1, keepdim=True)
+    cb = 1.0 + spread * torch.randn(K, generator=g).clamp(-2.0, 2.0)
+    mask = torch.rand(Z, N, generator=g) < 0.1
+    ref = c_oracle.we_aniso(a.numpy(), b.numpy(), cb.numpy(), wn.numpy(), mask.numpy())
+    # (the isotropic bar and 3e-7 for the terms left out of the expansion)
+    bar = 2e-6 + 2 * 2.0 ** -24 * float(wn.max()) * float((a.amax(1) - a.amin(1)).norm(dim=-1).max())
+    for partials in (True, False):
+        got = run_aniso(gpu, a, b, cb, wn, mask, partials=partials)
+        for x, r, what in zip(got, ref, ("out", "d_cb", "d_k")):
+            assert (x[mask.numpy()] == 0).all(), what
+            assert rel_l2(x, r) <= bar, (what, rel_l2(x, r), bar)
+        assert all(np.array_equal(x, y) for x, y in zip(got, run_aniso(gpu, a, b, cb, wn, mask, partials=partials)))
