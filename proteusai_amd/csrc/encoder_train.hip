@@ -5,8 +5,8 @@
 //
 // All of it is streaming work of a few MB per call, so a call's time is its launch and one trip through memory; what
 // these kernels remove is launches and trips.  A training step of 4 x 512 tokens (d_model 512, 3 layers) ran 178
-// launches, 2.14 ms on the device; with these it runs 108, 1.69 ms on the device.  In all it is issued by the host: 3.2 to 3.8 ms
-// before, 3.0 to 3.2 now.  At the kernels: device times of torch's kernels and of these at that size.
+// launches, 2.14 ms on the device; with these it ran 108, 1.69 ms on the device, and with a layer's launches issued by the library
+// (encoder_layer.hip) it takes 1.54 ms in all.  At the kernels: device times of torch's kernels and of these at that size.
 //
 // Sums over tokens are taken in a fixed order (partial sums per workgroup, then one pass over them): the same bits on
 // every call.
