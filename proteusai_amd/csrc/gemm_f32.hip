@@ -103,7 +103,7 @@ __device__ __forceinline__ float plain_dot(const GemmArgs& g, const int m, const
     return s;
 }
 
-// Does a row (of A, or of B^T) hold a NaN at k0 <= k < k1?
+// Does a row (of A, or of B^T) hold a NaN at k0 <= k < k1?  (Plain loads, which nothing keeps inside the matrix: k1 <= K.)
 template <bool KC>
 __device__ __forceinline__ bool any_nan(const float* __restrict__ X, const int ld, const int row, const int rows, const int k0, const int k1)
 {
@@ -226,7 +226,7 @@ void gemm_f32_kernel(const GemmArgs g)
     }
     if (__builtin_amdgcn_ballot_w64(again != 0) == 0) return;
     // Where a row of A or a column of B holds a NaN so do their elements (a run that has diverged: all of them); the others are summed again.
-    const int half = (g.K / 2 + 3) / 4 * 4, k0 = lane >> 5 ? half : 0, k1 = lane >> 5 ? g.K : half;
+    const int k0 = lane >> 5 ? g.K / 2 : 0, k1 = lane >> 5 ? g.K : g.K / 2;
     const bool nan_a = any_nan<AK>(g.A, g.lda, m0 + wm + (lane & 31), g.M, k0, k1), nan_b = any_nan<BK>(g.B, g.ldb, n, g.N, k0, k1);
     const uint64_t in_a = __builtin_amdgcn_ballot_w64(nan_a), in_b = __builtin_amdgcn_ballot_w64(nan_b);
     const uint32_t rows_a = (uint32_t)in_a | (uint32_t)(in_a >> 32), cols_b = (uint32_t)in_b | (uint32_t)(in_b >> 32);
@@ -353,7 +353,7 @@ void gemm_f32_rows_kernel(const GemmArgs g)
     if (__builtin_amdgcn_ballot_w64(again != 0) == 0) return;
     // (as above)
     uint32_t rows_a[2], cols_b[2];
-    const int middle = (g.K / 2 + 3) / 4 * 4, k0 = half ? middle : 0, k1 = half ? g.K : middle;
+    const int k0 = half ? g.K / 2 : 0, k1 = half ? g.K : g.K / 2;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const uint64_t in_a = __builtin_amdgcn_ballot_w64(any_nan<false>(g.A, g.lda, m0 + 32 * i + r0, g.M, k0, k1));

@@ -64,6 +64,25 @@ def test_a_diverged_operand(gpu, form):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("form,K", [(NN, 4), (NT, 4), (TN, 1), (TN, 2), (TN, 3), (TN, 5), (TN, 16)])
+def test_a_diverged_operand_is_read_to_its_end(gpu, form, K):
+    # NaN right behind either operand: an element that is infinite must not be taken for one whose row or column holds a NaN
+    M, N = 40, 36
+    def guarded(rows, cols, seed):
+        t = torch.rand(rows + 8, cols, generator=torch.Generator().manual_seed(seed)).to(gpu)
+        t[rows:] = float("nan")
+        return t[:rows]
+    A = guarded(K, M, 1) if form == TN else guarded(M, K, 1)
+    B = guarded(N, K, 2) if form == NT else guarded(K, N, 2)
+    clean = train_ops._product(form, A, B)
+    (A if form != TN else A.t())[7, K - 1] = float("inf")
+    got = train_ops._product(form, A, B)
+    assert bool((got[7] == float("inf")).all())
+    rest = torch.arange(M, device=gpu) != 7
+    assert torch.equal(got[rest], clean[rest])
+
+
+@pytest.mark.gpu
 def test_values_that_do_not_split(gpu):
     A, B, _, _ = _operands(NN, 70, 68, 36, gpu)
     A[3, 5], A[7, 1], A[9, 2], A[11, 3] = float("inf"), float("nan"), 3.4e38, -3.39e38      # (bf16 ends at 3.39e38)
