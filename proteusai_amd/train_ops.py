@@ -238,6 +238,9 @@ def gelu_mlp(x, lin1, lin2):
     if not (plain_module(lin1, nn.Linear) and plain_module(lin2, nn.Linear)) or lin1.bias is None or lin2.bias is None:
         return None
     w1, b1, w2, b2 = lin1.weight, lin1.bias, lin2.weight, lin2.bias
+    # (what does not have a linear layer's shapes is the expression's to broadcast or to refuse: the products read biases unseen)
+    if w1.dim() != 2 or w2.dim() != 2 or b1.shape != w1.shape[:1] or b2.shape != w2.shape[:1]:
+        return None
     # (a frozen first layer keeps the expression, which does not keep x: x may be changed in place behind it)
     if (not w1.requires_grad or x.dim() < 2 or x.shape[-1] != w1.shape[1] or w1.shape[0] != w2.shape[1] or x.numel() == 0 or w1.shape[0] % 4 or w2.shape[0] % 4
             or x.numel() // x.shape[-1] > 65535 * 2048        # (rows of a column sum)

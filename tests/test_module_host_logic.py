@@ -1,10 +1,15 @@
 """Host-side logic of the modules that needs no GPU: the constants GeoAttention keeps across inference calls, and the
-choice between writing the fused projection's gradient in place and through buffers of its own."""
+choice between writing the fused projection's gradient in place and through buffers of its own, and what the training functions
+hand to kernels."""
 import importlib
 
+import pytest
 import torch
+import torch.nn as nn
 
 import proteusai_amd as pa
+
+from proteusai_amd import train_ops
 
 ga = importlib.import_module("proteusai_amd.geometric_attn")
 
@@ -73,3 +78,19 @@ def test_fused_gradient_is_written_in_place_only_where_the_kernels_can_address_i
         g = torch.empty((1, N, 3, 8, 64), dtype=torch.float32, device="meta")
         grads = tuple(g[:, :, i].permute(0, 2, 1, 3) for i in range(3))
         assert ga._fused_grad_views_ok(grads) == ok, N
+
+
+@pytest.mark.parametrize("layer,name,shape", [
+    ("in_proj", "bias", (1,)), ("out_proj", "bias", (1,)), ("in_proj", "bias", (25,)), ("out_proj", "bias", (15,)), ("in_proj", "bias", (1, 24)),
+    ("in_proj", "weight", (24, 16, 1)), ("out_proj", "weight", (16, 24, 1))])
+def test_feed_forward_parameters_of_other_shapes_stay_with_the_expression(monkeypatch, layer, name, shape):
+    # (a bias that torch broadcasts or refuses would be read past its end)
+    taken = []
+    monkeypatch.setattr(train_ops, "recording", lambda *t: True)
+    monkeypatch.setattr(train_ops._GeluMLP, "apply", lambda *a: taken.append(a))
+    mlp = pa.MLP(d_in=16, d_out=16, d_hidden=24, dropout=0.0)
+    x = torch.randn(2, 3, 16, requires_grad=True)
+    train_ops.gelu_mlp(x, mlp.in_proj, mlp.out_proj)
+    assert len(taken) == 1
+    setattr(getattr(mlp, layer), name, nn.Parameter(torch.randn(shape)))
+    assert train_ops.gelu_mlp(x, mlp.in_proj, mlp.out_proj) is None and len(taken) == 1
