@@ -81,12 +81,19 @@ def _by_expression(d):
             or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() > 0)
 
 
-def _saved(t, numel, dtype=torch.float32):
-    """A saved tensor as a kernel may read it.  What saved-tensor hooks give back may lie differently (strides, alignment); another
-    type, size or place is an error, as it would be in a torch operator."""
-    if t.dtype != dtype or t.numel() != numel or not t.is_cuda:
-        raise RuntimeError(f"a tensor of {numel} {dtype} that was saved on the GPU came back as {tuple(t.shape)} of {t.dtype} on {t.device}")
+def _saved(t, numel, dev, dtype=torch.float32):
+    """A saved tensor as a kernel on `dev` may read it.  What saved-tensor hooks give back may lie differently (strides, alignment);
+    another type, size or place is an error, as it would be in a torch operator."""
+    if t.dtype != dtype or t.numel() != numel or t.device != dev:
+        raise RuntimeError(f"a tensor of {numel} {dtype} that was saved on {dev} came back as {tuple(t.shape)} of {t.dtype} on {t.device}")
     return t if t.is_contiguous() and t.data_ptr() % 16 == 0 else _dense(t)
+
+
+def _saved_sizes(*tensors_and_sizes):
+    """Saved tensors of the attention, which takes any type and place of them, hold what the forward saved."""
+    for t, numel in tensors_and_sizes:
+        if t is not None and t.numel() != numel:
+            raise RuntimeError(f"a tensor of {numel} elements that was saved came back as {tuple(t.shape)}")
 
 
 def _without_autocast(backward):
@@ -173,9 +180,9 @@ class _AddLayerNorm(torch.autograd.Function):
         if _by_expression(d):
             dx, dw, db = _recorded(lambda y_, w_, b_: F.layer_norm(y_, (w.numel(),), w_, b_, ctx.eps), (ysum, w, b), (True, need[2], need[3]), d)
         else:
-            d, D = _dense(d), d.shape[-1]
+            d, D, dev = _dense(d), d.shape[-1], d.device
             rows = d.numel() // D
-            w, ysum, stat = _saved(w, D), _saved(ysum, rows * D), _saved(stat, 2 * rows)
+            w, ysum, stat = _saved(w, D, dev), _saved(ysum, rows * D, dev), _saved(stat, 2 * rows, dev)
             dx = torch.empty_like(ysum)
             dwb = torch.empty(2, D, dtype=torch.float32, device=d.device)
             n = _bytes("proteus_layernorm_bwd_workspace_bytes", rows, D)
@@ -216,10 +223,11 @@ class _GeluMLP(torch.autograd.Function):
         need = ctx.needs_input_grad
         if _by_expression(d):
             return _recorded(lambda x_, w1_, b1_, w2_, b2_: F.linear(F.gelu(F.linear(x_, w1_, b1_)), w2_, b2_), (x, w1, b1, w2, b2), need, d)
-        rows, (hidden, d_in), d_out = d.numel() // w2.shape[0], w1.shape, w2.shape[0]
+        d_out, (hidden, d_in), dev = d.shape[-1], w1.shape, d.device
         d2 = _dense(d).view(-1, d_out)
-        x2, a = _saved(x, rows * d_in).view(rows, d_in), _saved(a, rows * hidden).view(rows, hidden)
-        w1, w2, h = _saved(w1, hidden * d_in).view(hidden, d_in), _saved(w2, d_out * hidden).view(d_out, hidden), _saved(h, rows * hidden)
+        rows = d2.shape[0]
+        x2, a = _saved(x, rows * d_in, dev).view(rows, d_in), _saved(a, rows * hidden, dev).view(rows, hidden)
+        w1, w2, h = _saved(w1, hidden * d_in, dev).view(hidden, d_in), _saved(w2, d_out * hidden, dev).view(d_out, hidden), _saved(h, rows * hidden, dev)
         dw2 = _product(TN, d2, a) if need[3] else None
         db2 = column_sums(d2) if need[4] else None
         dx = dw1 = db1 = None
@@ -309,12 +317,16 @@ class _SelfAttention(torch.autograd.Function):
             gx, *gp = _recorded(lambda x_, *p: _self_attention_expression(x_, coords, mask, *p, ctx.min_spread, ctx.operand_dtype),
                                 (x, *params), (need[0], *need[3:11]), d)
             return (gx, None, None, *gp, None, None)
-        Z, N, _, H, dk = qkv.shape
-        dm = H * dk
+        Z, N, dm = d.shape
+        H, _, dk = params[0].shape
+        dev = d.device
         d2 = _dense(d).view(Z * N, dm)
-        W, Wo, x2 = _saved(W, 3 * dm * dm).view(dm, 3 * dm), _saved(Wo, dm * dm).view(dm, dm), _saved(x, Z * N * dm).view(Z * N, dm)
+        W, Wo, x2 = _saved(W, 3 * dm * dm, dev).view(dm, 3 * dm), _saved(Wo, dm * dm, dev).view(dm, dm), _saved(x, Z * N * dm, dev).view(Z * N, dm)
+        _saved_sizes((coords, Z * N * 3), (mask, Z * N), (L, Z * H * N), (sigma, H))
+        if tuple(qkv.shape) != (Z, N, 3, H, dk) or tuple(O.shape) != (Z, H, N, dk):
+            raise RuntimeError(f"the projection and the output of {(Z, N, H, dk)} that were saved came back as {tuple(qkv.shape)} and {tuple(O.shape)}")
         dO = _product(NN, d2, Wo).view(Z, N, H, dk).permute(0, 2, 1, 3)
-        g = torch.empty(qkv.shape, dtype=torch.float32, device=d.device)
+        g = torch.empty(qkv.shape, dtype=torch.float32, device=dev)
         _, _, _, d_sigma, _ = ga._backward(*_heads(qkv), O, L, dO, coords, sigma, mask, None, 0.0, 1.0, ctx.operand_dtype, grads=_heads(g))
         g2 = g.view(Z * N, 3 * dm)
         dx = _product(NT, g2, W).view(x.shape) if need[0] else None
@@ -322,8 +334,8 @@ class _SelfAttention(torch.autograd.Function):
         # (what a gradient is not asked of is not looked at: its place in the list is None)
         dW = _product(TN, x2, g2) if any(need[3:6]) else g2
         db = column_sums(g2) if any(need[6:9]) else g2
-        dWo = _product(TN, d2, _saved(O.permute(0, 2, 1, 3), Z * N * dm).view(Z * N, dm)) if need[10] else g2
-        _layout(grads, dW, db, dWo, d_sigma, _saved(spread, H), dm, H, dk, ctx.min_spread, 1)
+        dWo = _product(TN, d2, _saved(O.permute(0, 2, 1, 3), Z * N * dm, dev).view(Z * N, dm)) if need[10] else g2
+        _layout(grads, dW, db, dWo, d_sigma, _saved(spread, H, dev), dm, H, dk, ctx.min_spread, 1)
         return (dx, None, None, *grads, None, None)
 
 
@@ -377,7 +389,7 @@ class _EncoderLayer(torch.autograd.Function):
         ctx.save_for_backward(x, coords, mask, kept, *params[8:])
         ctx.params = params[:8]
         ctx.versions = [p._version for p in ctx.params]
-        ctx.args = args[16:]
+        ctx.args, ctx.sizes = args[16:], sizes
         return out
 
     @staticmethod
@@ -391,16 +403,14 @@ class _EncoderLayer(torch.autograd.Function):
                 raise RuntimeError("a parameter of the self-attention was changed in place after the forward pass whose gradient is recorded")
             gx, *gp = _recorded(lambda x_, *p: _layer_expression(x_, coords, mask, *p, *ctx.args), (x, *attn, *rest), (need[0], *need[3:19]), d)
             return (gx, None, None, *gp, None, None, None, None)
-        Z, N, dm = x.shape
-        H, _, dk = attn[0].shape
-        hidden = rest[2].shape[0]
-        sizes = (Z, N, H, dk, hidden)
-        dev = d.device
+        sizes = Z, N, H, dk, hidden = ctx.sizes                 # (the forward's: what the hooks of saved tensors give back is held against them)
+        dm, dev = H * dk, d.device
         g1, c1, w1, b1, w2, b2, g2, c2 = rest
-        g1, w1, w2, g2 = _saved(g1, dm), _saved(w1, hidden * dm), _saved(w2, dm * hidden), _saved(g2, dm)
-        x2, kept = _saved(x, Z * N * dm), _saved(kept, _bytes("proteus_encoder_layer_kept_bytes", *sizes), torch.uint8)
+        g1, w1, w2, g2 = _saved(g1, dm, dev), _saved(w1, hidden * dm, dev), _saved(w2, dm * hidden, dev), _saved(g2, dm, dev)
+        x2, kept = _saved(x, Z * N * dm, dev), _saved(kept, _bytes("proteus_encoder_layer_kept_bytes", *sizes), dev, torch.uint8)
         if kept.data_ptr() % 256:
             kept = kept.clone()
+        _saved_sizes((coords, Z * N * 3), (mask, Z * N))
         c, m = ga._f32(coords, dev), None if mask is None else ga._mask_bytes(mask, dev)
         wanted = need[3:19]
         grads = [torch.empty_like(p, memory_format=torch.contiguous_format) if n and not 8 <= i <= 9 and i < 14 else None
@@ -465,7 +475,7 @@ class _SmallEmbedding(torch.autograd.Function):
         if _by_expression(d):
             return (*_recorded(lambda w: F.embedding(tokens, w), (weight,), (True,), d), None)
         V, D = weight.shape
-        d, t = _dense(d), _saved(tokens, d.numel() // D, torch.int64)
+        d, t = _dense(d), _saved(tokens, d.numel() // D, d.device, torch.int64)
         dW = torch.empty(V, D, dtype=torch.float32, device=d.device)
         n = _bytes("proteus_embedding_bwd_workspace_bytes", t.numel(), V, D)
         _call("proteus_embedding_bwd", d.device, d, t, dW, _workspace(n, d.device), n, t.numel(), V, D)

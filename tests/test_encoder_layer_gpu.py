@@ -149,6 +149,27 @@ def test_saved_tensors_and_outputs(gpu):
             out.sum().backward()
 
 
+@pytest.mark.parametrize("whole", [True, False])
+def test_saved_tensors_that_come_back_smaller(gpu, whole, monkeypatch):
+    # every tensor that the backward reads, one at a time, a row short: an error on the host, before any launch that reads it
+    layer, x, coords, mask, leaves = _layer(gpu)
+    if not whole:
+        monkeypatch.setattr(train_ops, "encoder_layer", lambda *a: None)
+    unread = [b.data_ptr() for n, b in layer.named_parameters() if n.endswith(".bias")]     # what is only added
+    saved = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: saved.append(t) or t, lambda t: t):
+        layer(x, x, x, coords, mask)
+    assert len(saved) >= 12
+    for i in range(len(saved)):
+        count = iter(range(len(saved)))
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: (next(count) == i, t), lambda p: p[1][:-1] if p[0] else p[1]):
+            out = layer(x, x, x, coords, mask)
+        if saved[i].data_ptr() in unread:
+            continue
+        with pytest.raises(RuntimeError):
+            torch.autograd.grad(out, leaves, torch.ones_like(out))
+
+
 def test_captured_training_step(gpu):
     layer, x, coords, mask, leaves = _layer(gpu)
     x, d = x.detach(), torch.randn_like(x)

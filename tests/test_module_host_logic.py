@@ -94,3 +94,15 @@ def test_feed_forward_parameters_of_other_shapes_stay_with_the_expression(monkey
     assert len(taken) == 1
     setattr(getattr(mlp, layer), name, nn.Parameter(torch.randn(shape)))
     assert train_ops.gelu_mlp(x, mlp.in_proj, mlp.out_proj) is None and len(taken) == 1
+
+
+def test_saved_tensors_of_another_size_type_or_device_are_refused():
+    # (another GPU cannot be had here: what is compared is the device)
+    t, other = torch.zeros(12), torch.zeros(12, device="meta")
+    assert train_ops._saved(t, 12, t.device) is t
+    for args in ((t, 11, t.device), (t, 12, t.device, torch.float64), (other, 12, t.device), (t, 12, torch.device("cuda", 1))):
+        with pytest.raises(RuntimeError, match="came back as"):
+            train_ops._saved(*args)
+    train_ops._saved_sizes((t, 12), (None, 5))
+    with pytest.raises(RuntimeError, match="came back as"):
+        train_ops._saved_sizes((t, 12), (t, 13))
