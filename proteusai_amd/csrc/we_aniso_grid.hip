@@ -255,10 +255,12 @@ template <class Add>
 __device__ __forceinline__ void wa_every_near(const float4* __restrict__ src, const float4* __restrict__ srcb, const int n, const float xi, const float yi, const float zi,
                                               const float mid, const float inv_h, const int lane, Add add)
 {
+    float4 next = src[lane], nextb = srcb[lane];
     for (int j0 = 0; j0 < n; j0 += 64) {
-        const float4 q = src[j0 + lane];
+        const float4 q = next, qb = nextb;
+        next = src[j0 + 64 + lane]; nextb = srcb[j0 + 64 + lane];       // (past the end: inside the lists' padding)
         WgPair mine;
-        uint64_t todo = __builtin_amdgcn_ballot_w64(wa_no_cell(srcb[j0 + lane], xi - q.x, yi - q.y, zi - q.z, mid, inv_h, mine) && j0 + lane < n);
+        uint64_t todo = __builtin_amdgcn_ballot_w64(wa_no_cell(qb, xi - q.x, yi - q.y, zi - q.z, mid, inv_h, mine) && j0 + lane < n);
         while (todo) {
             const int b = __builtin_ctzll(todo);
             todo &= todo - 1;
@@ -511,44 +513,49 @@ void we_aniso_grid_kernel(const char* __restrict__ ws, const float* __restrict__
     auto find = [&](int j, float dx, float dy, float dz, WgPair& p) {
         return wa_no_cell(srcb[j], dx, dy, dz, mid_cb, inv_h, p);
     };
-    // all observers' lists at once, or one observer's after the other where that is too much
-    bool listed = wg_collect<WAVES>(s_grid, s_cnt, near, src, n, me, closest * closest, find);
-    const bool together = listed;
-    int unit = 0;                                              // an observer and 64 wavenumbers for a wave
-    for (uint32_t left = near; left; left &= left - 1) {
-        const int q = __builtin_ctz(left);
-        if (!together) {
-            __syncthreads();                                   // the last observer's list is read
-            listed = wg_collect<WAVES>(s_grid, s_cnt, left & (0u - left), src, n, me, closest * closest, find);
+    int lengths;
+    const bool listed = wg_collect<WAVES>(s_grid, s_cnt, near, src, n, me, closest * closest, lengths, find);
+    const int zk = SHARED ? blockIdx.z : 0, Zk = SHARED ? gridDim.z : 1;
+    wg_near_units<WAVES, 2>(near, (L.nkt - zk + Zk - 1) / Zk, listed, [&](auto wide, const int q, const int first) {
+        constexpr int U = decltype(wide)::value;
+        int k[U];
+        float kr[U], cb[U], s[U][GRADS ? 6 : 2];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            k[u] = (zk + (first + 4 * u + (lane >> 4)) * Zk) * 16 + obs;             // a lane per wavenumber, of this workgroup's tiles
+            kr[u] = (float)((k[u] < K ? (double)wavenumbers[k[u]] : 0.0) * 0.15915494309189533577);
+            cb[u] = k[u] < K ? cb_magnitudes[k[u]] : 0.f;
+#pragma unroll
+            for (int i = 0; i < (GRADS ? 6 : 2); ++i) s[u][i] = 0.f;
         }
-        const size_t row = (zN + s_tok[q]) * 2 * K;
-        for (int kb = 0; kb < K; kb += 64) {
-            if ((unit++ & (WAVES - 1)) != wave) continue;
-            const int k = kb + lane;
-            const float kr = (float)((k < K ? (double)wavenumbers[k] : 0.0) * 0.15915494309189533577), cb = k < K ? cb_magnitudes[k] : 0.f;
-            float s[GRADS ? 6 : 2] = {};
-            auto add = [&](const WgPair& p) {
-                const float ph = __builtin_amdgcn_fractf(__builtin_fmaf(-cb, p.A, p.r) * kr);
+        auto add = [&](const WgPair& p) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const float ph = __builtin_amdgcn_fractf(__builtin_fmaf(-cb[u], p.A, p.r) * kr[u]);
                 const float cs = __builtin_amdgcn_cosf(ph), sn = __builtin_amdgcn_sinf(ph);
-                s[0] = __builtin_fmaf(cs, p.m, s[0]);
-                s[1] = __builtin_fmaf(sn, p.m, s[1]);
+                s[u][0] = __builtin_fmaf(cs, p.m, s[u][0]);
+                s[u][1] = __builtin_fmaf(sn, p.m, s[u][1]);
                 if constexpr (GRADS) {
-                    s[2] += cs; s[3] += sn;
-                    s[4] = __builtin_fmaf(cs, p.m * p.A, s[4]);
-                    s[5] = __builtin_fmaf(sn, p.m * p.A, s[5]);
+                    s[u][2] += cs; s[u][3] += sn;
+                    s[u][4] = __builtin_fmaf(cs, p.m * p.A, s[u][4]);
+                    s[u][5] = __builtin_fmaf(sn, p.m * p.A, s[u][5]);
                 }
-            };
-            if (listed) wg_listed<WAVES>(s_grid, s_cnt, q, add);
-            else wa_every_near(src, srcb, n, wg_lane(me.x, q), wg_lane(me.y, q), wg_lane(me.z, q), mid_cb, inv_h, lane, add);
-            if (k >= K || (SHARED && (k >> 4) % (int)gridDim.z != (int)blockIdx.z)) continue;       // (this workgroup's tiles)
-            auto put = [&](float* to, float re, float im) { to[row + 2 * k] += re; to[row + 2 * k + 1] += im; };
-            put(out, s[0], s[1]);
+            }
+        };
+        if (listed) wg_listed<WAVES>(s_grid, lengths, q, add);
+        else wa_every_near(src, srcb, n, wg_lane(me.x, q), wg_lane(me.y, q), wg_lane(me.z, q), mid_cb, inv_h, lane, add);
+        const size_t row = (zN + s_tok[q]) * 2 * K;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (k[u] >= K) continue;
+            auto put = [&](float* to, float re, float im) { to[row + 2 * k[u]] += re; to[row + 2 * k[u] + 1] += im; };
+            put(out, s[u][0], s[u][1]);
             if constexpr (GRADS) {
-                put(d_k, -s[3] + cb * s[5], s[2] - cb * s[4]);
-                put(d_cb, wavenumbers[k] * s[5], -wavenumbers[k] * s[4]);
+                put(d_k, -s[u][3] + cb[u] * s[u][5], s[u][2] - cb[u] * s[u][4]);
+                put(d_cb, wavenumbers[k[u]] * s[u][5], -wavenumbers[k[u]] * s[u][4]);
             }
         }
-    }
+    });
 }
 
 // What the grids need beside the direct kernel, two launches of preparation and one that finds nothing to do, costs 13 us.  Without

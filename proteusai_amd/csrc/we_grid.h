@@ -317,13 +317,13 @@ __device__ __forceinline__ float wg_reach(const float4& me, const bool ok, const
 struct WgPair { float r, m, A; int obs; };                     // distance, 1/r, (anisotropic) A; in units of length
 
 // Every wave searches its share of the sources for them, 256 on their way while the 256 before are looked at: only what lies within
-// `reach2` (squared, scaled) of an observer in `near` is placed.  (One wave per observer, which waited for memory at every 64 sources and did
-// the sums as it met them, took as long as the spread where most workgroups have such an observer: compact chains, us before and now,
-// isotropic 1 x 16384 with the sums 476 / 384, 1 x 65536 5348 / 4608, 1 x 8192 anisotropic 249 / 155, 1 x 2000 58 / 51, extended 1 x 4000 95 / 71.)  find(j, dx, dy, dz, pair): does source j's pair have no cell?
-// Returns (to all threads) whether the lists hold all of them; a list is in the order of the sources.
+// `reach2` (squared, scaled) of an observer in `near` is placed.  (One wave per observer, which waits for memory at every 64 sources and does
+// the sums as it meets them, took as long as the spread where most workgroups have such an observer: compact chains, us before and now,
+// isotropic 1 x 16384 with the sums 476 / 384, 1 x 65536 5348 / 4608, 1 x 8192 anisotropic 249 / 155.)  find(j, dx, dy, dz, pair): does source j's pair have no cell?
+// Returns (to all threads) whether the lists hold all of them, and the lists' lengths to the first lanes; a list is in the order of the sources.
 template <int WAVES, class Find>
 __device__ __forceinline__ bool wg_collect(uint32_t* s_grid, int* s_cnt, const uint32_t near, const float4* __restrict__ src, const int n, const float4& me,
-                                           const float reach2, Find find)
+                                           const float reach2, int& lengths, Find find)
 {
     constexpr int CAP = WG_ROWS * WG_OBS * 4 / 16 / WAVES, BATCH = 4;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -335,7 +335,7 @@ __device__ __forceinline__ bool wg_collect(uint32_t* s_grid, int* s_cnt, const u
     if (wave * share < end)
 #pragma unroll
         for (int i = 0; i < BATCH; ++i) next[i] = src[wave * share + 64 * i + lane];
-    for (int j0 = wave * share; j0 < end; j0 += 64 * BATCH) {
+    for (int j0 = wave * share; j0 < end && count <= CAP; j0 += 64 * BATCH) {
         float4 q[BATCH];
 #pragma unroll
         for (int i = 0; i < BATCH; ++i) q[i] = next[i];
@@ -362,20 +362,19 @@ __device__ __forceinline__ bool wg_collect(uint32_t* s_grid, int* s_cnt, const u
     }
     if (lane == 0) s_cnt[wave] = count;
     __syncthreads();
-    bool all = true;
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w) all &= s_cnt[w] <= CAP;
-    return all;
+    lengths = lane < WAVES ? s_cnt[lane] : 0;
+    return __builtin_amdgcn_ballot_w64(lengths > CAP) == 0;
 }
 
 // add(pair) for the listed pairs of observer o, in the order of the sources.
 template <int WAVES, class Add>
-__device__ __forceinline__ void wg_listed(const uint32_t* s_grid, const int* s_cnt, const int o, Add add)
+__device__ __forceinline__ void wg_listed(const uint32_t* s_grid, const int lengths, const int o, Add add)
 {
     constexpr int CAP = WG_ROWS * WG_OBS * 4 / 16 / WAVES;
-    for (int w = 0; w < WAVES; ++w) {
+    for (uint64_t some = __builtin_amdgcn_ballot_w64(lengths > 0); some; some &= some - 1) {
+        const int w = __builtin_ctzll(some);
         const WgPair* list = reinterpret_cast<const WgPair*>(s_grid) + w * CAP;
-        const int count = __builtin_amdgcn_readfirstlane(s_cnt[w]);
+        const int count = __builtin_amdgcn_readlane(lengths, w);
         for (int i0 = 0; i0 < count; i0 += 64) {
             const int lane = threadIdx.x & 63;
             const WgPair mine = list[min(i0 + lane, count - 1)];
@@ -387,6 +386,30 @@ __device__ __forceinline__ void wg_listed(const uint32_t* s_grid, const int* s_c
                 p.r = wg_lane(mine.r, b); p.m = wg_lane(mine.m, b); p.A = wg_lane(mine.A, b);
                 add(p);
             }
+        }
+    }
+}
+
+// The sums over these pairs, dealt out over the waves: sum(U, observer, first) does U times 64 wavenumbers, of the workgroup's `tiles` of 16 those from
+// `first` on.  U = 1 where the lists hold all pairs and larger units would leave waves idle; otherwise up to MAX_U: a pair is fetched once for
+// all of them.  Us, tokens in places of 20, 100 and 1000, 0.03 apart, 1 x 1100, K = 256, so / with 64 wavenumbers a unit always and over-full
+// lists an observer at a time: 30 / 39, 42 / 145, 177 / 941; 1 x 16384 in places of 1000 1380 / 4120.
+template <int U> struct WgWide { static constexpr int value = U; };
+template <int WAVES, int MAX_U, class Sum>
+__device__ __forceinline__ void wg_near_units(const uint32_t near, const int tiles, const bool listed, Sum sum)
+{
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const bool wide = !listed || __builtin_popcount(near) * ((tiles + 4 * MAX_U - 1) / (4 * MAX_U)) >= WAVES;
+    const int step = wide ? 4 * MAX_U : 4;
+    int unit = 0;
+    for (uint32_t left = near; left; left &= left - 1) {
+        const int o = __builtin_ctz(left);
+        for (int first = 0; first < tiles; first += step) {
+            if ((unit++ & (WAVES - 1)) != wave) continue;
+            const int some = min(tiles - first, step);
+            if (MAX_U > 2 && some > 8) sum(WgWide<MAX_U>{}, o, first);
+            else if (some > 4)         sum(WgWide<2>{}, o, first);
+            else                       sum(WgWide<1>{}, o, first);
         }
     }
 }

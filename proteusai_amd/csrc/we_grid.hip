@@ -53,8 +53,10 @@ template <class Add>
 __device__ __forceinline__ void wg_every_near(const float4* __restrict__ src, const int n, const float xi, const float yi, const float zi, const float inv_h,
                                               const int lane, Add add)
 {
+    float4 next = src[lane];
     for (int j0 = 0; j0 < n; j0 += 64) {
-        const float4 q = src[j0 + lane];
+        const float4 q = next;
+        next = src[j0 + 64 + lane];                            // (past the end: inside the list's padding)
         float r2, inv, r;
         wg_distance(xi - q.x, yi - q.y, zi - q.z, r2, inv, r);
         const bool near = __builtin_bit_cast(int, __builtin_fmaf(r, inv_h, WG_MAGIC)) == __builtin_bit_cast(int, WG_MAGIC);
@@ -424,38 +426,40 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
         p.r = r; p.m = inv; p.A = 0.f;
         return r2 != 0.0f && __builtin_bit_cast(int, __builtin_fmaf(r, inv_h, WG_MAGIC)) == __builtin_bit_cast(int, WG_MAGIC);
     };
-    // all observers' lists at once, or one observer's after the other where that is too much
-    bool listed = wg_collect<WAVES>(s_grid, s_cnt, near, src, n, me, closest * closest, find);
-    const bool together = listed;
-    int unit = 0;                                              // an observer and 64 wavenumbers for a wave
-    for (uint32_t left = near; left; left &= left - 1) {
-        const int q = __builtin_ctz(left);
-        if (!together) {
-            __syncthreads();                                   // the last observer's list is read
-            listed = wg_collect<WAVES>(s_grid, s_cnt, left & (0u - left), src, n, me, closest * closest, find);
+    int lengths;
+    const bool listed = wg_collect<WAVES>(s_grid, s_cnt, near, src, n, me, closest * closest, lengths, find);
+    const int zk = blockIdx.z, Zk = gridDim.z;
+    wg_near_units<WAVES, 4>(near, (L.nkt - zk + Zk - 1) / Zk, listed, [&](auto wide, const int q, const int first) {
+        constexpr int U = decltype(wide)::value;
+        int k[U];
+        float kr[U], oc[U], os[U], c[U], s[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            k[u] = (zk + (first + 4 * u + (lane >> 4)) * Zk) * 16 + obs;             // a lane per wavenumber, of this workgroup's tiles
+            kr[u] = (float)((k[u] < K ? (double)wavenumbers[k[u]] : 0.0) * 0.15915494309189533577) * (1.0f / WG_UNIT);
+            oc[u] = os[u] = c[u] = s[u] = 0.f;
         }
-        const size_t row = zN + s_tok[q];
-        for (int kb = 0; kb < K; kb += 64) {
-            if ((unit++ & (WAVES - 1)) != wave) continue;
-            const int k = kb + lane;
-            const float kr = (float)((k < K ? (double)wavenumbers[k] : 0.0) * 0.15915494309189533577) * (1.0f / WG_UNIT);
-            float oc = 0.f, os = 0.f, c = 0.f, s = 0.f;
-            auto add = [&](const WgPair& p) {
-                const float ph = __builtin_amdgcn_fractf(p.r * kr);
+        auto add = [&](const WgPair& p) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const float ph = __builtin_amdgcn_fractf(p.r * kr[u]);
                 const float cs = __builtin_amdgcn_cosf(ph), sn = __builtin_amdgcn_sinf(ph);
-                oc = __builtin_fmaf(cs, p.m, oc);
-                os = __builtin_fmaf(sn, p.m, os);
-                if (SUMS) { c += cs; s += sn; }
-            };
-            if (listed) wg_listed<WAVES>(s_grid, s_cnt, q, add);
-            else wg_every_near(src, n, wg_lane(me.x, q), wg_lane(me.y, q), wg_lane(me.z, q), inv_h, lane, add);
-            if (k < K && (k >> 4) % (int)gridDim.z == (int)blockIdx.z) {       // (this workgroup's tiles)
-                float* o = out + row * 2 * K;
-                o[2 * k] += oc * WG_UNIT; o[2 * k + 1] += os * WG_UNIT;
-                if (SUMS) { cos_sums[row * K + k] += c; sin_sums[row * K + k] += s; }
+                oc[u] = __builtin_fmaf(cs, p.m, oc[u]);
+                os[u] = __builtin_fmaf(sn, p.m, os[u]);
+                if (SUMS) { c[u] += cs; s[u] += sn; }
             }
+        };
+        if (listed) wg_listed<WAVES>(s_grid, lengths, q, add);
+        else wg_every_near(src, n, wg_lane(me.x, q), wg_lane(me.y, q), wg_lane(me.z, q), inv_h, lane, add);
+        const size_t row = zN + s_tok[q];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (k[u] >= K) continue;
+            float* o = out + row * 2 * K + 2 * k[u];
+            o[0] += oc[u] * WG_UNIT; o[1] += os[u] * WG_UNIT;
+            if (SUMS) { cos_sums[row * K + k[u]] += c[u]; sin_sums[row * K + k[u]] += s[u]; }
         }
-    }
+    });
 }
 
 }  // namespace
