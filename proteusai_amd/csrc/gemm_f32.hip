@@ -2,13 +2,13 @@
 //
 // An fp32 number is the sum of three bf16 numbers (8 + 8 + 8 bits, each piece rounded to nearest: the third takes what is
 // left exactly).  Of the nine products of pieces the six largest are taken, x0 y0, x0 y1, x1 y0, x1 y1, x0 y2, x2 y0: what is left out
-// is below 2^-26 of |x y|, under the rounding of one fp32 addition.  Six v_mfma_f32_32x32x16_bf16 cost 192 clocks where the same
+// is below 2^-26 of |x y|, at any magnitude (ENLARGED below), under the rounding of one fp32 addition.  Six v_mfma_f32_32x32x16_bf16 cost 192 clocks where the same
 // product on v_mfma_f32_32x32x2_f32 takes 512, and their fp32 accumulator rounds once per 16 products instead of once per 2.
 //
 // gemm_f32_kernel (rows of A along k): a workgroup makes one 64 x 64 tile of C.  Four waves (a group) hold 32 x 32 of it each and step through
 // K by 16; where the tiles are too few to fill the chip, 2 or 4 groups share a tile, each with its own steps and its own LDS stages, and
 // add up at the end in a fixed order (the same bits on every call).  A step: 8 floats per thread travel global -> registers two steps
-// ahead, are split (5.5 vector instructions each) and written to one of two stages as 16-byte fragments, eight consecutive k of one row; the
+// ahead, are split (6.5 vector instructions each) and written to one of two stages as 16-byte fragments, eight consecutive k of one row; the
 // product reads them with ds_read_b128.  Odd groups split and then multiply, even ones the other way round.  What bounds it: a 64 x 64 x 16
 // step reads 24 KB and writes 12 KB of LDS (288 clocks at 128 bytes a clock), and splitting (200 clocks a wave) hardly overlaps with the
 // products (192).  Smaller where it counts than the traffic of operands split beforehand: 6 bytes an element through L2.
@@ -54,12 +54,19 @@ __device__ __forceinline__ uint32_t pack2(const float a, const float b) {
     const f32x2 f = {a, b};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2));
 }
+// bf16 has fp32's range but not its smallest numbers: below 2^-109 the third piece, below 2^-117 the second would fall under 2^-133, where bf16
+// ends.  Operands are therefore split 2^16 times as large, which leaves nothing of an fp32 number out, subnormals among them, and sums are
+// 2^32 times the result.  (What overflows that way, operands from 2^112 and sums from 2^96 on, is not finite and summed again in plain fp32.)
+// Relative error (2-norm) against float64 of operands about 2^-113, 2^-120, 2^-126, as they are / so: 2.8e-7, 3.5e-5, 2.2e-3 / 5.5e-8 (the library 1.4e-7).
+// A multiplication per element: 2048 x 512 x 2048 31.7 -> 32.6 us, 512 x 2048 x 2048 28.3 -> 29.7.
+constexpr float ENLARGED = 0x1p16f, REDUCED = 0x1p-32f;
 __device__ __forceinline__ float low(const uint32_t w)  { return __builtin_bit_cast(float, w << 16); }
 __device__ __forceinline__ float high(const uint32_t w) { return __builtin_bit_cast(float, w & 0xffff0000u); }
 
 // Four consecutive k of one row into the three pieces' fragments.
-__device__ __forceinline__ void split_to_lds(char* at, const float4& v)
+__device__ __forceinline__ void split_to_lds(char* at, const float4& from)
 {
+    const float4 v = make_float4(from.x * ENLARGED, from.y * ENLARGED, from.z * ENLARGED, from.w * ENLARGED);
     uint2 p;
     p.x = pack2(v.x, v.y); p.y = pack2(v.z, v.w);
     *reinterpret_cast<uint2*>(at) = p;
@@ -220,7 +227,7 @@ void gemm_f32_kernel(const GemmArgs g)
             }
             const int m = m0 + wm + 8 * q + 4 * (lane >> 5) + i;
             if (m >= g.M || n >= g.N) continue;
-            if (fabsf(v) <= 3.4028234e38f) write<EPI>(g, m, n, v);
+            if (fabsf(v) <= 3.4028234e38f) write<EPI>(g, m, n, v * REDUCED);
             else again |= 1u << (q * 4 + i);
         }
     }
@@ -241,7 +248,9 @@ struct Raw { float4 lo, hi; };
 struct Frags { bf16x8 x[3]; };
 __device__ __forceinline__ Frags split(const Raw& r)
 {
-    const float v[8] = {r.lo.x, r.lo.y, r.lo.z, r.lo.w, r.hi.x, r.hi.y, r.hi.z, r.hi.w};
+    float v[8] = {r.lo.x, r.lo.y, r.lo.z, r.lo.w, r.hi.x, r.hi.y, r.hi.z, r.hi.w};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] *= ENLARGED;
     uint32_t p[3][4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -347,7 +356,7 @@ void gemm_f32_rows_kernel(const GemmArgs g)
     for (int i = 0; i < 64 / W; ++i) {
         const int e = wave * (64 / W) + i;
         if (m0 + row(e) >= g.M || column(e) >= g.N) continue;
-        if (fabsf(v[i]) <= 3.4028234e38f) write<EPI>(g, m0 + row(e), column(e), v[i]);
+        if (fabsf(v[i]) <= 3.4028234e38f) write<EPI>(g, m0 + row(e), column(e), v[i] * REDUCED);
         else again |= 1u << i;
     }
     if (__builtin_amdgcn_ballot_w64(again != 0) == 0) return;

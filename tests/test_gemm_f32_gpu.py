@@ -32,6 +32,21 @@ def test_product_against_float64(gpu, form, M, N, K):
     assert torch.equal(got, train_ops._product(form, A, B))
 
 
+# Operands and results near the ends of fp32's range: pieces that would be smaller than bf16's smallest numbers, subnormal operands, operands and
+# sums that leave the enlarged range (from 2^112 and 2^96 on)
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", [NN, NT, TN])
+@pytest.mark.parametrize("ea,eb", [(-112, 0), (-120, 0), (-126, 20), (-140, 60), (0, -120), (-60, -60), (115, -40), (40, 60), (111, -3)])
+def test_magnitudes(gpu, form, ea, eb):
+    M, N, K = 70, 68, 100
+    g = torch.Generator(device=gpu).manual_seed(ea * 1000 + eb + 200000)
+    A, B = (torch.randn(s, generator=g, device=gpu).clamp(-4, 4).mul(2.0 ** (e / 2)).mul(2.0 ** (e / 2)) for s, e in (((M, K), ea), ((K, N), eb)))
+    want, mass = A.double() @ B.double(), A.double().abs() @ B.double().abs()
+    got = train_ops._product(form, A.t().contiguous() if form == TN else A, B.t().contiguous() if form == NT else B)
+    # (as in test_product_against_float64; plain sums round once per term; a subnormal result is a multiple of 2^-149)
+    assert bool(((got - want).abs() <= (12 * 7 + 16) * 2.0 ** -24 * mass + 2.0 ** -149).all())
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M", [5, 700])
 def test_epilogues(gpu, M):
