@@ -66,7 +66,7 @@ extern "C" {
  * backward entry point take `int operand_type` before `tuning` / `stream`; a caller built against an older header
  * would pass its tuning selector there).  The Python binding checks for an exact match when it loads the library.
  */
-#define PROTEUS_VERSION 306
+#define PROTEUS_VERSION 307
 int proteus_version(void);
 
 /* Human-readable text for a return code of any entry point. */
@@ -555,7 +555,9 @@ int proteus_embedding_bwd(const float* dout, const int64_t* tokens, float* dW, v
  *             A matrix whose rows run along K (A in NN and NT, B in NT): K and its ld multiples of 4
  *   epilogue  PROTEUS_GEMM_F32: C f32;  _BF16: C bf16, rounded once;  _GELU: H = the sums f32, C = gelu(H) f32;
  *             _GELU_GRAD: C = sums * gelu'(h) f32;  _ADD: C = sums + h f32 (exact GELU; H and h laid out as C)
- *   A, B, C 16-byte aligned; bias, h, H may be NULL where not asked for.  One launch, no workspace.
+ *   A, B, C 16-byte aligned; bias, h, H may be NULL where not asked for.  One launch without a workspace.
+ *   ws        proteus_gemm_f32_workspace_bytes bytes, 16-byte aligned, or NULL: with it a TN product of few tiles and many rows (a gradient of a
+ *             weight over many tokens; else 0 bytes are asked for) is cut along K over the chip, and a second launch adds up
  */
 #define PROTEUS_GEMM_NN 0
 #define PROTEUS_GEMM_NT 1
@@ -567,6 +569,9 @@ int proteus_embedding_bwd(const float* dout, const int64_t* tokens, float* dW, v
 #define PROTEUS_GEMM_ADD       4
 int proteus_gemm_f32(const float* A, const float* B, const float* bias, const float* h, void* C, float* H,
                      int M, int N, int K, int lda, int ldb, int ldc, int form, int epilogue, void* stream);
+size_t proteus_gemm_f32_workspace_bytes(int M, int N, int K, int form);
+int proteus_gemm_f32_ws(const float* A, const float* B, const float* bias, const float* h, void* C, float* H,
+                        int M, int N, int K, int lda, int ldb, int ldc, int form, int epilogue, void* ws, size_t ws_bytes, void* stream);
 
 /*
  * One post-LN encoder layer's training step on the kernels above, a call per direction (old/old_scripts/encoder.py:33-41 with the geometric

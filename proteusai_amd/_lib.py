@@ -14,7 +14,7 @@ LIB_PATH = os.path.join(HERE, "libproteus_hip.so")
 
 COORDS_SOA = 0
 COORDS_AOS = 1
-ABI_VERSION = 306                    # PROTEUS_VERSION of the include/proteus_hip.h these argument lists were written from
+ABI_VERSION = 307                    # PROTEUS_VERSION of the include/proteus_hip.h these argument lists were written from
 OPERAND_BF16, OPERAND_F16 = 0, 1     # PROTEUS_OPERAND_* of include/proteus_hip.h
 GRAD_F32, GRAD_OPERAND = 0, 1        # PROTEUS_GRAD_*
 GEMM_NN, GEMM_NT, GEMM_TN = 0, 1, 2  # PROTEUS_GEMM_*: form
@@ -37,7 +37,8 @@ SYMBOLS = [
     "proteus_geo_attn_variant_name",
     "proteus_add_layernorm_fwd", "proteus_add_layernorm_fwd_check", "proteus_geo_attn_delta", "proteus_geo_attn_delta_check",
     "proteus_train_workspace_bytes", "proteus_layernorm_bwd_workspace_bytes", "proteus_embedding_bwd_workspace_bytes",
-    "proteus_add_layernorm_train_fwd", "proteus_layernorm_bwd", "proteus_colsum", "proteus_heads_layout", "proteus_embedding_bwd", "proteus_gemm_f32", "proteus_encoder_layer_kept_bytes", "proteus_encoder_layer_fwd_bytes",
+    "proteus_add_layernorm_train_fwd", "proteus_layernorm_bwd", "proteus_colsum", "proteus_heads_layout", "proteus_embedding_bwd", "proteus_gemm_f32", "proteus_gemm_f32_workspace_bytes", "proteus_gemm_f32_ws",
+    "proteus_encoder_layer_kept_bytes", "proteus_encoder_layer_fwd_bytes",
     "proteus_encoder_layer_bwd_bytes", "proteus_encoder_layer_fwd", "proteus_encoder_layer_bwd",
 ]
 
@@ -174,6 +175,10 @@ def load():
     lib.proteus_embedding_bwd.argtypes = [vp] * 4 + [sz, cl, ci, ci, vp]
     lib.proteus_gemm_f32.restype = ci
     lib.proteus_gemm_f32.argtypes = [vp] * 6 + [ci] * 8 + [vp]
+    lib.proteus_gemm_f32_workspace_bytes.restype = sz
+    lib.proteus_gemm_f32_workspace_bytes.argtypes = [ci] * 4
+    lib.proteus_gemm_f32_ws.restype = ci
+    lib.proteus_gemm_f32_ws.argtypes = [vp] * 6 + [ci] * 8 + [vp, sz, vp]
     for name in ("kept", "fwd", "bwd"):
         getattr(lib, f"proteus_encoder_layer_{name}_bytes").restype = sz
         getattr(lib, f"proteus_encoder_layer_{name}_bytes").argtypes = [ci] * 5

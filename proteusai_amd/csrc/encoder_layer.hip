@@ -1,6 +1,6 @@
 // A post-LN encoder layer's training step, one call per direction: the order in which the kernels of the layer are launched
 // and where in the two buffers their tensors lie.  Host code: launches cost 2 to 3 us each from here, 6 to 10 from Python and
-// 18 to 29 through torch's products, and a layer has 9 of them forward and 18 backward, of which most last less than that.
+// 18 to 29 through torch's products, and a layer has 9 of them forward and 18 to 22 backward, of which most last less than that.
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -69,8 +69,8 @@ struct Forward {
 struct Backward {
     float *dy2, *dh, *dx1, *dy1, *dO, *D, *g, *d_sigma, *dW, *db, *dWo, *ln;
     uint16_t* dO16;
-    void *lnws, *sums;
-    size_t ln_bytes, sums_bytes, bytes;
+    void *lnws, *sums, *shares;
+    size_t ln_bytes, sums_bytes, shares_bytes, bytes;
     Backward(const Sizes& s, void* base)
     {
         Carve c{static_cast<char*>(base)};
@@ -83,6 +83,14 @@ struct Backward {
         lnws = c.take<char>(ln_bytes);
         sums_bytes = proteus_train_workspace_bytes(s.rows, s.hidden > 3 * s.dm ? s.hidden : 3 * s.dm);
         sums = c.take<char>(sums_bytes);
+        // (one product after the other: the largest of the four gradients of weights)
+        shares_bytes = 0;
+        const int sizes[4][2] = {{s.dm, s.hidden}, {s.hidden, s.dm}, {s.dm, s.dm}, {s.dm, 3 * s.dm}};
+        for (const auto& z : sizes) {
+            const size_t n = proteus_gemm_f32_workspace_bytes(z[0], z[1], (int)s.rows, PROTEUS_GEMM_TN);
+            if (n > shares_bytes) shares_bytes = n;
+        }
+        shares = c.take<char>(shares_bytes);
         bytes = c.at;
     }
 };
@@ -162,7 +170,7 @@ extern "C" int proteus_encoder_layer_bwd(const float* x, const float* coords, co
     if (kept_bytes < k.bytes || ws_bytes < b.bytes) return PROTEUS_ERR_BAD_SHAPE;
     const int rows = (int)s.rows, dm = s.dm;
     auto product = [&](const float* A, const float* B, const float* h, float* C, int m, int n, int kk, int lda, int ldb, int form, int epilogue) {
-        return proteus_gemm_f32(A, B, nullptr, h, C, nullptr, m, n, kk, lda, ldb, n, form, epilogue, stream);
+        return proteus_gemm_f32_ws(A, B, nullptr, h, C, nullptr, m, n, kk, lda, ldb, n, form, epilogue, b.shares_bytes ? b.shares : nullptr, b.shares_bytes, stream);
     };
     auto column_sums = [&](const float* a, float* out, int C) { return proteus_colsum(a, nullptr, nullptr, out, b.sums, b.sums_bytes, s.rows, C, stream); };
     auto layernorm = [&](const float* d, const float* y, const float* stat, const float* gamma, float* dy, float* dgamma_dbeta) {

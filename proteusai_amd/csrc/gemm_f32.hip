@@ -18,9 +18,13 @@
 // under the 24 products of this one, the one after it on its way; the waves of a workgroup add up in LDS at the end.  With rows along
 // k a lane would read 32 bytes of a row of its own: 38 and 43 us against 36 and 38 (2048 x 512 x 2048 and 2048 x 2048 x 512).
 //
-// us, 2048 tokens, this / the library's fp32 product: QKV 2048 x 1536 x 512 32 / 35, its output 12 / 12; feed-forward 2048 x 2048 x 512 38 / 39,
-// 2048 x 512 x 2048 36 / 37; gradients of weights 512 x 2048 x 2048 34 / 39 (through the first kernel 44), 2048 x 512 x 2048 30 / 39 (39),
-// 512 x 1536 x 2048 28 / 31 (35), 512 x 512 x 2048 23 / 16 (31).  Error against float64 at K = 2048 2.5e-7 to 3.5e-7, the library's 8.1e-7.
+// Few tiles over many tokens leave compute units idle, each of the others a serial chain over K: there workgroups take shares of K (rows_shares), whose
+// sums a second launch adds up in their order.
+//
+// us, 2048 tokens, this / the library's fp32 product: QKV 2048 x 1536 x 512 28.3 / 30.8, its output 10.5 / 11.2; feed-forward 2048 x 2048 x 512 36.2 / 35.3
+// (with GELU's derivative EPILOGUE), 2048 x 512 x 2048 32.4 / 34.0; gradients of weights 512 x 2048 x 2048 and 2048 x 512 x 2048 28.6 / 34.6, 512 x 1536 x 2048 25.4 / 28.9,
+// 512 x 512 x 2048 14.5 / 14.5 (through the first kernel 44, 39, 35, 31); 8192 tokens 97 / 97, 35 / 35, 127 / 125, 129 / 120 and 98 / 121, 84 / 100, 32 / 55.
+// Error against float64 at K = 2048 2.5e-7 to 3.5e-7, the library's 8.1e-7.
 //
 // Values that are not finite (or become so: bf16 ends half a step below fp32) do not split; an element of C that comes out not
 // finite is summed again in plain fp32.
@@ -48,6 +52,8 @@ struct GemmArgs {
     void  *C;
     float *H;
     int M, N, K, lda, ldb, ldc, tiles_n, tiles, per_xcd;
+    float *part;                                    // sums of the shares of K, where a product is cut
+    int shares, steps;                              // their number, and the steps of each
 };
 
 __device__ __forceinline__ uint32_t pack2(const float a, const float b) {
@@ -289,24 +295,71 @@ struct RowSource {
     }
 };
 
+// Accumulators e0 to e0 + COUNT of a 64 x 64 tile at (m0, n0), a lane's sums of each.
+template <int COUNT, int EPI>
+__device__ __forceinline__ void finish_rows(const GemmArgs& g, const int m0, const int n0, const int e0, const float (&v)[COUNT])
+{
+    const int lane = threadIdx.x & 63, r0 = lane & 31, half = lane >> 5;
+    auto row = [&](const int e) { return 32 * (e >> 5) + 8 * ((e >> 2) & 3) + 4 * half + (e & 3); };       // of accumulator e, in the tile
+    auto column = [&](const int e) { return n0 + 32 * ((e >> 4) & 1) + r0; };
+    uint32_t again = 0;                                        // of the lane's elements those that are not finite
+#pragma unroll
+    for (int i = 0; i < COUNT; ++i) {
+        const int e = e0 + i;
+        if (m0 + row(e) >= g.M || column(e) >= g.N) continue;
+        if (fabsf(v[i]) <= 3.4028234e38f) write<EPI>(g, m0 + row(e), column(e), v[i] * REDUCED);
+        else again |= 1u << i;
+    }
+    if (__builtin_amdgcn_ballot_w64(again != 0) == 0) return;
+    // (as above)
+    uint32_t rows_a[2], cols_b[2];
+    const int k0 = half ? g.K / 2 : 0, k1 = half ? g.K : g.K / 2;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uint64_t in_a = __builtin_amdgcn_ballot_w64(any_nan<false>(g.A, g.lda, m0 + 32 * i + r0, g.M, k0, k1));
+        const uint64_t in_b = __builtin_amdgcn_ballot_w64(any_nan<false>(g.B, g.ldb, n0 + 32 * i + r0, g.N, k0, k1));
+        rows_a[i] = (uint32_t)in_a | (uint32_t)(in_a >> 32);
+        cols_b[i] = (uint32_t)in_b | (uint32_t)(in_b >> 32);
+    }
+    for (; again; again &= again - 1) {
+        const int e = e0 + __builtin_ctz(again), j = (e >> 4) & 1;
+        const bool nan = ((e >> 5 ? rows_a[1] : rows_a[0]) >> (row(e) & 31) | (j ? cols_b[1] : cols_b[0]) >> r0) & 1;
+        write<EPI>(g, m0 + row(e), column(e), nan ? __builtin_nanf("") : plain_dot<false, false>(g, m0 + row(e), column(e)));
+    }
+}
+
+// Where tile `tile` lies: consecutive ones are those of a line along the shorter side of the matrix, so that an XCD's share is as square as may be
+// (512 x 2048 of 2048 tokens 28.5 us, with lines along the longer side 36.5).
+__device__ __forceinline__ void tile_at(const GemmArgs& g, const int tile, int& m0, int& n0)
+{
+    const int tiles_m = g.tiles / g.tiles_n;
+    const bool wide = tiles_m < g.tiles_n;
+    m0 = (wide ? tile % tiles_m : tile / g.tiles_n) * GT;
+    n0 = (wide ? tile / tiles_m : tile % g.tiles_n) * GT;
+}
+
 template <int W, int EPI>
 __global__ __launch_bounds__(W * 64, 2)
 void gemm_f32_rows_kernel(const GemmArgs g)
 {
     extern __shared__ __align__(16) float red[];              // [W][64 accumulators][64 lanes]
-    const int tile = (blockIdx.x & 7) * g.per_xcd + (blockIdx.x >> 3);      // consecutive tiles (of the same rows of A) on one XCD
-    if ((int)(blockIdx.x >> 3) >= g.per_xcd || tile >= g.tiles) return;
-    const int m0 = tile / g.tiles_n * GT, n0 = tile % g.tiles_n * GT;
+    // consecutive tiles of one share of K on one XCD: 512 x 512 x 8192 in four shares, whose operands then come to one or two
+    // of the eight caches, 32 us, with the shares of a tile on one XCD 42
+    const int unit = (blockIdx.x & 7) * g.per_xcd + (blockIdx.x >> 3), share = unit / g.tiles, tile = unit % g.tiles;
+    if (share >= g.shares) return;
+    int m0, n0;
+    tile_at(g, tile, m0, n0);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r0 = lane & 31, half = lane >> 5;
 
     const RowSource sa(g.A, g.lda, m0 + r0, g.M, 8 * half, g.K);
     const RowSource sb(g.B, g.ldb, n0 + r0, g.N, 8 * half, g.K);
-    const int steps = (g.K + GK - 1) / GK, rounds = steps > wave ? (steps - wave + W - 1) / W : 0;         // this wave's
+    // (a share but the last is an even number of rounds: what is past its end, the next one's, is loaded but not multiplied)
+    const int begin = share * g.steps, steps = min((g.K + GK - 1) / GK - begin, g.steps), rounds = steps > wave ? (steps - wave + W - 1) / W : 0;         // this wave's
     Raw ra[2][2], rb[2][2];
     Frags a[2][2], b[2][2];
     f32x16 acc[2][2] = {};
-    auto load = [&](const int round, const int s) { const int k0 = (round * W + wave) * GK; sa.fetch(k0, ra[s]); sb.fetch(k0, rb[s]); };      // (zeros past the end)
+    auto load = [&](const int round, const int s) { const int k0 = (begin + round * W + wave) * GK; sa.fetch(k0, ra[s]); sb.fetch(k0, rb[s]); };      // (zeros past the end)
     auto step = [&](const int round, const int s) {
         // send for the step after the next; split the next under this step's products
         load(round + 2, s);
@@ -349,32 +402,31 @@ void gemm_f32_rows_kernel(const GemmArgs g)
 #pragma unroll
         for (int w = 1; w < W; ++w) v[e] += red[(w * 64 + wave * (64 / W) + e) * 64 + lane];
     }
-    auto row = [&](const int e) { return 32 * (e >> 5) + 8 * ((e >> 2) & 3) + 4 * half + (e & 3); };       // of accumulator e, in the tile
-    auto column = [&](const int e) { return n0 + 32 * ((e >> 4) & 1) + r0; };
-    uint32_t again = 0;                                        // of the lane's elements those that are not finite
+    if (g.shares > 1) {
+        float* to = g.part + ((size_t)share * g.tiles + tile) * (GT * GT) + wave * (64 / W) * 64 + lane;
 #pragma unroll
-    for (int i = 0; i < 64 / W; ++i) {
-        const int e = wave * (64 / W) + i;
-        if (m0 + row(e) >= g.M || column(e) >= g.N) continue;
-        if (fabsf(v[i]) <= 3.4028234e38f) write<EPI>(g, m0 + row(e), column(e), v[i] * REDUCED);
-        else again |= 1u << i;
+        for (int e = 0; e < 64 / W; ++e) to[e * 64] = v[e];
+        return;
     }
-    if (__builtin_amdgcn_ballot_w64(again != 0) == 0) return;
-    // (as above)
-    uint32_t rows_a[2], cols_b[2];
-    const int k0 = half ? g.K / 2 : 0, k1 = half ? g.K : g.K / 2;
+    finish_rows<64 / W, EPI>(g, m0, n0, wave * (64 / W), v);
+}
+
+// The shares' sums of a tile together, in their order: a quarter of a tile per workgroup, four accumulators per wave.
+template <int EPI>
+__global__ __launch_bounds__(256)
+void gemm_f32_rows_sum_kernel(const GemmArgs g)
+{
+    const int tile = blockIdx.x >> 2, e0 = (blockIdx.x & 3) * 16 + (threadIdx.x >> 6) * 4;
+    const float* from = g.part + (size_t)tile * (GT * GT) + e0 * 64 + (threadIdx.x & 63);
+    const size_t pitch = (size_t)g.tiles * (GT * GT);
+    float v[4] = {};
+#pragma unroll 4
+    for (int s = 0; s < g.shares; ++s)
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const uint64_t in_a = __builtin_amdgcn_ballot_w64(any_nan<false>(g.A, g.lda, m0 + 32 * i + r0, g.M, k0, k1));
-        const uint64_t in_b = __builtin_amdgcn_ballot_w64(any_nan<false>(g.B, g.ldb, n0 + 32 * i + r0, g.N, k0, k1));
-        rows_a[i] = (uint32_t)in_a | (uint32_t)(in_a >> 32);
-        cols_b[i] = (uint32_t)in_b | (uint32_t)(in_b >> 32);
-    }
-    for (; again; again &= again - 1) {
-        const int e = wave * (64 / W) + __builtin_ctz(again), j = (e >> 4) & 1;
-        const bool nan = ((e >> 5 ? rows_a[1] : rows_a[0]) >> (row(e) & 31) | (j ? cols_b[1] : cols_b[0]) >> r0) & 1;
-        write<EPI>(g, m0 + row(e), column(e), nan ? __builtin_nanf("") : plain_dot<false, false>(g, m0 + row(e), column(e)));
-    }
+        for (int i = 0; i < 4; ++i) v[i] += from[s * pitch + i * 64];
+    int m0, n0;
+    tile_at(g, tile, m0, n0);
+    finish_rows<4, EPI>(g, m0, n0, e0, v);
 }
 
 template <bool AK, bool BK, int EPI>
@@ -383,7 +435,7 @@ int gemm_go(GemmArgs g, hipStream_t st)
     const int tm = (g.M + GT - 1) / GT;
     g.tiles_n = (g.N + GT - 1) / GT;
     g.tiles   = tm * g.tiles_n;
-    g.per_xcd = (g.tiles + 7) / 8;
+    g.per_xcd = (g.tiles * g.shares + 7) / 8;
     const dim3 grid((unsigned)g.per_xcd * 8);
     if constexpr (!AK) {
         // Waves per tile: two per SIMD where the steps allow.
@@ -392,6 +444,7 @@ int gemm_go(GemmArgs g, hipStream_t st)
         else if (g.tiles > 256) GO(4);
         else                    GO(8);
 #undef GO
+        if (g.shares > 1) hipLaunchKernelGGL((gemm_f32_rows_sum_kernel<EPI>), dim3((unsigned)g.tiles * 4), dim3(256), 0, st, g);
     } else {
         // Groups per tile: four waves per SIMD where the tiles allow.
 #define GO(G_) do { \
@@ -406,12 +459,41 @@ int gemm_go(GemmArgs g, hipStream_t st)
     return (int)hipGetLastError();
 }
 
+// Gradients of weights: shares of K for workgroups of their own where the tiles leave compute units idle, so that at most 256 workgroups of 8 waves, one
+// per compute unit, are launched; at least 256 of K each (a round of 8 waves, two by two) and at most 32 of them, whose sums the second launch
+// adds up, and only where a workgroup is spared 768 of K, which is what that launch takes.  One, shares of 256, 512 and 1024, and the library, us:
+// 128 x 128 of 2048 tokens 23 / 9.9 / 11.8 / 16 / 14, of 8192 75 / 14 / 14 / 17 / 45; 512 x 512 of 2048 24 / 14.3 / 14.3 / 18 / 15, of 8192 77 / 33 / 33 / 33 / 55;
+// 256 x 1024 of 1024 15.2 / 12.5 / 13.6 / 15.1 / 9.7; 64 x 64 of 32768 283 with one, 44, 33 and 25 with 128, 64 and 32, library 117; 128 x 128 of 700 11.9 / 11.7 (two shares).
+struct Shares { int number, steps; };
+Shares rows_shares(int M, int N, int K)
+{
+    constexpr int UNIT = 2 * 8, MOST = 32;
+    const int64_t tiles = (int64_t)((M + (int64_t)GT - 1) / GT) * ((N + (int64_t)GT - 1) / GT);
+    const int steps = (K + GK - 1) / GK, units = (steps + UNIT - 1) / UNIT, most = tiles > 128 ? 1 : min((int)(256 / tiles), MOST);
+    const int per = (units + most - 1) / most * UNIT;
+    if (K - per * GK < 768) return {1, steps};
+    return {(steps + per - 1) / per, per};
+}
+
 bool off16(const void* p) { return ((uintptr_t)p & 15) != 0; }
 
 }  // namespace
 
+extern "C" size_t proteus_gemm_f32_workspace_bytes(int M, int N, int K, int form)
+{
+    if (form != PROTEUS_GEMM_TN || M <= 0 || N <= 0 || K <= 0 || K >= (1 << 29)) return 0;      // (2 GiB of a matrix are refused)
+    const Shares c = rows_shares(M, N, K);
+    return c.number > 1 ? (size_t)c.number * ((M + GT - 1) / GT) * ((N + GT - 1) / GT) * (GT * GT * 4) : 0;
+}
+
 extern "C" int proteus_gemm_f32(const float* A, const float* B, const float* bias, const float* h, void* C, float* H,
                                 int M, int N, int K, int lda, int ldb, int ldc, int form, int epilogue, void* stream)
+{
+    return proteus_gemm_f32_ws(A, B, bias, h, C, H, M, N, K, lda, ldb, ldc, form, epilogue, nullptr, 0, stream);
+}
+
+extern "C" int proteus_gemm_f32_ws(const float* A, const float* B, const float* bias, const float* h, void* C, float* H,
+                                   int M, int N, int K, int lda, int ldb, int ldc, int form, int epilogue, void* ws, size_t ws_bytes, void* stream)
 {
     if (!A || !B || !C || (epilogue == PROTEUS_GEMM_GELU && !H) || ((epilogue == PROTEUS_GEMM_GELU_GRAD || epilogue == PROTEUS_GEMM_ADD) && !h)) return PROTEUS_ERR_NULL_POINTER;
     if (form < 0 || form > PROTEUS_GEMM_TN || epilogue < 0 || epilogue > PROTEUS_GEMM_ADD) return PROTEUS_ERR_UNSUPPORTED;
@@ -425,7 +507,13 @@ extern "C" int proteus_gemm_f32(const float* A, const float* B, const float* bia
     if (off16(A) || off16(B) || off16(C)) return PROTEUS_ERR_BAD_ALIGNMENT;
     if (form != PROTEUS_GEMM_TN && (K % 4 || lda % 4)) return PROTEUS_ERR_BAD_SHAPE;
     if (form == PROTEUS_GEMM_NT && ldb % 4) return PROTEUS_ERR_BAD_SHAPE;
-    const GemmArgs g = {A, B, bias, h, C, H, M, N, K, lda, ldb, ldc, 0, 0, 0};
+    Shares cut = {1, (K + GK - 1) / GK};
+    if (ws && form == PROTEUS_GEMM_TN) {
+        if (off16(ws)) return PROTEUS_ERR_BAD_ALIGNMENT;
+        const size_t need = proteus_gemm_f32_workspace_bytes(M, N, K, form);
+        if (need && ws_bytes >= need) cut = rows_shares(M, N, K);
+    }
+    const GemmArgs g = {A, B, bias, h, C, H, M, N, K, lda, ldb, ldc, 0, 0, 0, static_cast<float*>(ws), cut.number, cut.steps};
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
 #define EPILOGUES(AK_, BK_) \
     switch (epilogue) { \

@@ -147,7 +147,8 @@ def _product(form, A, B, bias=None, gelu=False, gelu_grad_of=None, dtype=torch.f
     C = torch.empty(M, N, dtype=dtype, device=A.device)
     H = torch.empty_like(C) if gelu else None
     epilogue = _lib.GEMM_GELU if gelu else _lib.GEMM_GELU_GRAD if gelu_grad_of is not None else _lib.GEMM_BF16 if dtype == torch.bfloat16 else _lib.GEMM_F32
-    _call("proteus_gemm_f32", A.device, A, B, bias, gelu_grad_of, C, H, M, N, K, A.shape[1], B.shape[1], N, form, epilogue)
+    n = _bytes("proteus_gemm_f32_workspace_bytes", M, N, K, form) if form == TN else 0
+    _call("proteus_gemm_f32_ws", A.device, A, B, bias, gelu_grad_of, C, H, M, N, K, A.shape[1], B.shape[1], N, form, epilogue, _workspace(n, A.device), n)
     return (H, C) if gelu else C
 
 

@@ -32,6 +32,21 @@ def test_product_against_float64(gpu, form, M, N, K):
     assert torch.equal(got, train_ops._product(form, A, B))
 
 
+# Gradients of weights cut along K: a tile in 4 and in 32 shares, few tiles, 64 of them in four shares, the last in a remainder, 128 in two and the first
+# number of tiles that is not cut; below 1024 rows and where a share spares too little nothing is cut
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,shares", [(1, 4, 1024, 4), (64, 61, 8195, 17), (64, 64, 49150, 32), (64, 64, 50000, 28), (65, 130, 2050, 9), (512, 512, 2048, 4), (300, 320, 1033, 5), (500, 1000, 1536, 2),
+                                          (513, 1000, 2048, 1), (64, 64, 1000, 1), (500, 1000, 1535, 1)])
+def test_shares(gpu, M, N, K, shares):
+    tiles = ((M + 63) // 64) * ((N + 63) // 64)
+    assert _lib.load().proteus_gemm_f32_workspace_bytes(M, N, K, TN) == (tiles * shares * 16384 if shares > 1 else 0)
+    A, B, want, mass = _operands(TN, M, N, K, gpu)
+    got = train_ops._product(TN, A, B)
+    # (as above, a rounding more per share)
+    assert bool(((got - want).abs() <= (12 * ((K + 15) // 16) + 16 + shares) * 2.0 ** -24 * mass).all())
+    assert torch.equal(got, train_ops._product(TN, A, B))
+
+
 # Operands and results near the ends of fp32's range: pieces that would be smaller than bf16's smallest numbers, subnormal operands, operands and
 # sums that leave the enlarged range (from 2^112 and 2^96 on)
 @pytest.mark.gpu
@@ -66,9 +81,9 @@ def test_epilogues(gpu, M):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("form", [NN, NT, TN])
-def test_a_diverged_operand(gpu, form):
-    A, B, want, _ = _operands(form, 130, 132, 68, gpu)
+@pytest.mark.parametrize("form,K", [(NN, 68), (NT, 68), (TN, 68), (TN, 2100)])
+def test_a_diverged_operand(gpu, form, K):
+    A, B, want, _ = _operands(form, 130, 132, K, gpu)
     clean = train_ops._product(form, A, B)
     (A if form != TN else A.t())[66, 67] = float("nan")
     (B if form == NT else B.t())[131, 0] = float("nan")
@@ -97,14 +112,25 @@ def test_a_diverged_operand_is_read_to_its_end(gpu, form, K):
     assert torch.equal(got[rest], clean[rest])
 
 
+# (gradients of weights: 8, 4 and 2 waves per tile, and shares of K)
 @pytest.mark.gpu
-def test_values_that_do_not_split(gpu):
-    A, B, _, _ = _operands(NN, 70, 68, 36, gpu)
-    A[3, 5], A[7, 1], A[9, 2], A[11, 3] = float("inf"), float("nan"), 3.4e38, -3.39e38      # (bf16 ends at 3.39e38)
-    got, want = train_ops._product(NN, A, B), A.double() @ B.double()
-    want = want.where(want.abs() <= torch.finfo(torch.float32).max, want.sign() * float("inf")).where(~want.isnan(), want)
-    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
-    assert torch.equal(got[got.isinf()].double(), want[want.isinf()])
+@pytest.mark.parametrize("form,M,N,K", [(NN, 70, 68, 36), (NT, 70, 68, 36), (NN, 1700, 1600, 36), (NT, 1100, 1200, 36), (TN, 70, 68, 36), (TN, 70, 68, 2100), (TN, 1100, 1000, 37), (TN, 1700, 1600, 38)])
+def test_values_that_do_not_split(gpu, form, M, N, K):
+    A, B, _, _ = _operands(NN, M, N, K, gpu)
+    bad = [(3, 5, float("inf")), (7, 1, float("nan")), (9, 2, 3.4e38), (11, 3, -3.39e38)]      # (bf16 ends at 3.39e38)
+    bad += [(M - 1 - m, K - 1 - k, v) for m, k, v in bad] + [(M // 2 + m, K // 2 + k, -v) for m, k, v in bad]
+    for m, k, v in bad:
+        A[m, k] = v
+    got = train_ops._product(form, A.t().contiguous() if form == TN else A, B.t().contiguous() if form == NT else B)
+    want, mass = A.double() @ B.double(), A.double().abs() @ B.double().abs()
+    # (what fp32 cannot hold: an infinity, or what a plain sum makes of infinities of both signs on its way)
+    fits = mass <= torch.finfo(torch.float32).max
+    assert torch.equal(got.isnan() & fits, want.isnan() & fits) and bool((got[want.isnan()].isnan()).all())
+    infinite = want.isinf()
+    assert torch.equal(got[infinite].double(), want[infinite])
+    # (plain sums round once per term)
+    assert bool(((got - want).abs()[fits] <= (12 * ((K + 15) // 16) + 16 + K) * 2.0 ** -24 * mass[fits]).all())
+    assert not bool(got[fits].isinf().any())
 
 
 def test_what_it_refuses():
