@@ -470,7 +470,6 @@ void we_aniso_grid_kernel(const char* __restrict__ ws, const float* __restrict__
 
     const WgLayout L = wg_layout(Z, N, K, true);
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int z = blockIdx.y;
     const size_t zN = (size_t)z * N;
     const int n = reinterpret_cast<const int*>(ws + L.counts)[z];

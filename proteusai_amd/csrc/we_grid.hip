@@ -222,15 +222,17 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
     const float reach = wg_reach<WAVES>(me, ok, reinterpret_cast<const WgBox*>(ws + L.boxes) + (size_t)z * L.nbox, L.nbox, s_red) * inv_h + 2.0f;
     // Sums without the grid: where there is nothing to spread onto (values that are not finite, wavelengths below 0.11, more than 16
     // windows), where everything lies in a few cells and most pairs in none, and where the windows, each of which streams all sources
-    // again, cost more.  Per window 8 + 0.006 n us (16 waves; 8 waves, of which two workgroups share a compute unit, 16.6 + 0.0033 n per
-    // workgroup), its product 0.095 K, without the sums 0.055 K; all pairs directly 1.2e-3 n K and 1.0e-3 n K.  (Between the two, so that the
-    // choice and with it `out` do not depend on whether the sums are wanted.)  The direct kernel, the grid alone and this choice, us:
-    // K = 64, a structure 20 times as large 1 x 1024 40 / 168 / 31, 1 x 4096 352 / 499 / 342, 40 times 353 / 1225 / 334; 1 x 4096 at wavelengths from
-    // 1000 on, K = 64 321 / 1116 / 293, K = 256 1097 / 1122 / 1138; a token that is not finite, K = 64 339 / 1223 / 335, K = 256 1125 / 1225 / 1303.
+    // again, cost more.  Us with 16 waves: per window 7.5 + 0.005 n, its product 0.15 K, without the sums 0.085 K, all pairs directly 10 + 1.2e-3 n K and
+    // 10 + 1.0e-3 n K, K being the workgroup's share of the wavenumbers; 8 waves, of which two workgroups share a compute unit: 16.6 + 0.0033 n per window and
+    // workgroup, its product 0.095 K and 0.055 K, all pairs directly as before.  (Between the two, so that the choice and with it `out` do not
+    // depend on whether the sums are wanted.)  Wavelengths from 3.7 on, grid / pairs / this choice (without the sums): 1 x 1024 over 3 windows, K = 64 47 / 31 / 31,
+    // K = 128 51 / 50 / 50, K = 256 63 / 89 / 63, K = 512 89 / 168 / 89, over 5 windows 86 / 50 / 50, 109 / 89 / 89, 159 / 168 / 159; 1 x 2048, K = 64 3 windows 69 / 89 / 69, 6 133 / 89 / 89;
+    // 1 x 4096, K = 64 6 windows 225 / 325 / 225, 12 451 / 324 / 324, K = 256 12 785 / 1266 / 785.  (The direct kernel: 1 x 4096, K = 64 321, K = 256 1097.)
     const bool far = !(reach < (float)(CELLS * WG_MAX_WINDOWS));
     const float windows = __builtin_ceilf(reach * (1.0f / (float)CELLS));
-    const float by_grid = windows * ((WAVES == 16 ? 8.0f + 6.0e-3f * (float)n : 16.6f + 3.3e-3f * (float)n) + 0.075f * (float)K);
-    const float by_pair = 1.1e-3f * (float)n * (float)K / (float)gridDim.z;
+    const float mine    = (float)K / (float)gridDim.z;
+    const float by_grid = windows * (WAVES == 16 ? 7.5f + 5.0e-3f * (float)n + 0.115f * mine : 16.6f + 3.3e-3f * (float)n + 0.075f * mine);
+    const float by_pair = (WAVES == 16 ? 8.0f : 0.0f) + 1.1e-3f * (float)n * mine;
     const bool direct = __builtin_amdgcn_readfirstlane(far || reach < 4.0f || (windows > 1.0f && by_grid > by_pair)) != 0;
     if (direct) {
         // (a cell is at most pi / 3.5 of phase: 1750 of them are 250 revolutions)

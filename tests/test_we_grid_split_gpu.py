@@ -13,9 +13,10 @@ pytestmark = pytest.mark.gpu
 
 # N, Z, K, scale: workgroups of a tile each and 2, 4, 8 and 16 waves on it (short chains have few rows); two and three tiles and four waves on each; 8
 # tiles, 2 waves; an odd number of tiles, a wave each; the last launch that is shared out and the first that is not; several windows
+# (a chain so extended that the shared launch takes them, and one where it sums the pairs directly)
 @pytest.mark.parametrize("N,Z,K,scale", [
     (40, 1, 33, 1.0), (100, 1, 80, 1.0), (520, 1, 80, 1.0), (2000, 1, 20, 1.0), (900, 1, 163, 1.0), (2000, 1, 250, 1.0), (1300, 1, 720, 1.0),
-    (2048, 1, 64, 1.0), (2049, 1, 64, 1.0), (333, 4, 250, 1.0), (700, 2, 163, 12.0)])
+    (2048, 1, 64, 1.0), (2049, 1, 64, 1.0), (333, 4, 250, 1.0), (700, 2, 163, 12.0), (520, 1, 512, 8.0), (1024, 1, 64, 8.0)])
 def test_shared_tiles(gpu, N, Z, K, scale):
     a, wn = synth.we_inputs(N, seed=N + K, batch=Z)[0] * scale, synth.wavenumbers(2 * K)
     a[0, 20] = a[0, 30] + torch.tensor([0.01, -0.02, 0.015])          # a pair that no cell takes
