@@ -587,7 +587,7 @@ int proteus_gemm_f32_ws(const float* A, const float* B, const float* bias, const
  *   kept               proteus_encoder_layer_kept_bytes: what the backward reads of the forward; the attention's parameters are among it
  *                      as copies, those of the LayerNorms and the feed-forward are read again (params of the backward: the same 16, of
  *                      which it reads 8, 10, 12 and 14)
- *   ws                 workspace, proteus_encoder_layer_fwd_bytes / _bwd_bytes
+ *   ws                 workspace, proteus_encoder_layer_fwd_bytes / _bwd_bytes (backward: about Z*N * (3 d_model + max(hidden, 3 d_model)) floats)
  *   d_model = H * d_head <= 2048, hidden a multiple of 4; every pointer 16-byte aligned, kept and ws 256-byte aligned
  */
 #define PROTEUS_LAYER_PARAMS 16

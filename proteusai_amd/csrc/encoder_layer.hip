@@ -75,9 +75,12 @@ struct Backward {
     {
         Carve c{static_cast<char*>(base)};
         const size_t dm = s.dm, rows = s.rows;
-        dy2 = c.take<float>(rows * dm); dh = c.take<float>(rows * s.hidden); dx1 = c.take<float>(rows * dm); dy1 = c.take<float>(rows * dm);
-        dO = c.take<float>(rows * dm); dO16 = c.take<uint16_t>(rows * dm); D = c.take<float>(rows * s.H);
-        g = c.take<float>(rows * 3 * dm); d_sigma = c.take<float>(s.H);
+        // What the feed-forward's half leaves behind the attention's half takes over: dh is read for the last time by the product that gives dx1, as is
+        // dy2, and dx1 by the LayerNorm that gives dy1; g, dO and dO16 are written after that.
+        dh = g = c.take<float>(rows * (s.hidden > 3 * s.dm ? s.hidden : 3 * dm));
+        dy2 = dO = c.take<float>(rows * dm);
+        dx1 = c.take<float>(rows * dm); dO16 = reinterpret_cast<uint16_t*>(dx1);
+        dy1 = c.take<float>(rows * dm); D = c.take<float>(rows * s.H); d_sigma = c.take<float>(s.H);
         dW = c.take<float>(3 * dm * dm); db = c.take<float>(3 * dm); dWo = c.take<float>(dm * dm); ln = c.take<float>(2 * dm);
         ln_bytes = proteus_layernorm_bwd_workspace_bytes(s.rows, s.dm);
         lnws = c.take<char>(ln_bytes);

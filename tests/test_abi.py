@@ -395,3 +395,13 @@ def test_attention_delta_argument_validation():
     assert chk(strides=arr(*([-4, 100 * 64, 64] + plain))) == -4
     assert chk(strides=arr(*(plain + [4 * 100 * 64, 100 * 64, 66]))) == -5          # rows off the 4-element grid
     assert lib.proteus_geo_attn_delta(None, p, None, p, 2, 4, 100, 64, _lib.DTYPE_BF16, None) == -1
+
+
+@pytest.mark.parametrize("Z,N,H,dk,hidden", [(8, 1024, 8, 64, 2048), (8, 1024, 8, 64, 512), (32, 1024, 4, 32, 512), (2, 4096, 16, 128, 4096)])
+def test_encoder_layer_backward_workspace_holds_no_two_halves_at_once(Z, N, H, dk, hidden):
+    # a wide tensor and three of d_model per token, D, and what does not grow with the tokens: the attention's gradients of
+    # weights (4 d_model^2), partial sums and shares of products
+    rows, dm = Z * N, H * dk
+    got = _lib.load().proteus_encoder_layer_bwd_bytes(Z, N, H, dk, hidden)
+    wide = max(hidden, 3 * dm)
+    assert got <= 4 * (rows * (wide + 3 * dm + H) + 4 * dm * dm) + (8 << 20) + 4 * (rows // 128 + 2) * (wide + 2 * dm)
