@@ -434,9 +434,11 @@ def encoder_layer(x, coords, mask, m, mlp_class):
     """The output of the Encoder module `m` (self-attention, `mlp_class` its feed-forward) on x, or None where its parts go their own ways."""
     if not torch.is_grad_enabled() or x.dtype != torch.float32 or not x.is_cuda or torch.is_autocast_enabled("cuda"):
         return None                                                         # (what most other calls fail at, before the closer look)
+    if not inactive_dropout(m.dropout):
+        return None
     a, n1, f, n2 = m.attn, m.attn_norm, m.ffn, m.ffn_norm
     lin1, lin2 = getattr(f, "in_proj", None), getattr(f, "out_proj", None)
-    if not (plain_module(a, ga.GeoAttention) and plain_module(n1, nn.LayerNorm) and plain_module(n2, nn.LayerNorm) and inactive_dropout(m.dropout)
+    if not (plain_module(a, ga.GeoAttention) and plain_module(n1, nn.LayerNorm) and plain_module(n2, nn.LayerNorm)
             and plain_module(f, mlp_class) and f.act is F.gelu and not f.hidden_proj and inactive_dropout(f.in_dropout)
             and plain_module(lin1, nn.Linear) and plain_module(lin2, nn.Linear) and plain_module(a.out_proj, nn.Linear) and "_residual_norm" not in m.__dict__):
         return None

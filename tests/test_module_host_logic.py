@@ -2,6 +2,7 @@
 choice between writing the fused projection's gradient in place and through buffers of its own, and what the training functions
 hand to kernels."""
 import importlib
+import types
 
 import pytest
 import torch
@@ -106,3 +107,13 @@ def test_saved_tensors_of_another_size_type_or_device_are_refused():
     train_ops._saved_sizes((t, 12), (None, 5))
     with pytest.raises(RuntimeError, match="came back as"):
         train_ops._saved_sizes((t, 12), (t, 13))
+
+
+def test_a_layer_with_active_dropout_is_told_before_the_closer_look(monkeypatch):
+    looked = []
+    plain = train_ops.plain_module
+    monkeypatch.setattr(train_ops, "plain_module", lambda m, cls: looked.append(cls) or plain(m, cls))
+    layer = pa.Encoder(d_model=64, heads=2, d_hidden=64, dropout=0.1).train()
+    x = types.SimpleNamespace(dtype=torch.float32, is_cuda=True)
+    assert train_ops.encoder_layer(x, None, None, layer, pa.MLP) is None
+    assert looked == [nn.Dropout]
