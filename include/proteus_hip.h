@@ -526,8 +526,8 @@ int proteus_add_layernorm_fwd_check(const void* x, const void* res, const void* 
  * proteus_add_layernorm_train_fwd   ysum = x + res, out = LayerNorm(ysum) * gamma + beta, stat [rows][2] = (mean, 1 / sqrt(var + eps)).
  *                                   D a multiple of 4, at most 2048; all pointers 16-byte aligned.
  * proteus_layernorm_bwd             dx [rows][D] (the gradient of x and of res) and dgamma_dbeta [2][D] from what the forward kept.
- * proteus_colsum                    sums [C] = column sums of a [rows][C]; with h: of dh = a * gelu'(h) (exact GELU), written too.
- *                                   C a multiple of 4; dh is a buffer of its own.  Workspace: proteus_train_workspace_bytes (may be 0).
+ * proteus_colsum                    sums [C] = column sums of a [rows][C].
+ *                                   C a multiple of 4.  Workspace: proteus_train_workspace_bytes (may be 0).
  * proteus_heads_layout              tensors = {q, k, v projections [H][d_model][d_head], their biases [H][d_head], NULL or [H] (forward: a
  *                                   copy of spread_w; backward: its gradient), output projection [d_model][d_head][H]} and
  *                                   W [d_model][3][H][d_head], b [3][H][d_head], Wo [d_model][H][d_head], sigma [H]:
@@ -543,7 +543,7 @@ int proteus_add_layernorm_train_fwd(const float* x, const float* res, const floa
                                     float* ysum, float* stat, long rows, int D, float eps, void* stream);
 int proteus_layernorm_bwd(const float* dout, const float* ysum, const float* stat, const float* gamma, float* dx,
                           float* dgamma_dbeta, void* ws, size_t ws_bytes, long rows, int D, void* stream);
-int proteus_colsum(const float* a, const float* h, float* dh, float* sums, void* ws, size_t ws_bytes, long rows, int C, void* stream);
+int proteus_colsum(const float* a, float* sums, void* ws, size_t ws_bytes, long rows, int C, void* stream);
 int proteus_heads_layout(float* const* tensors, float* W, float* b, float* Wo, float* sigma, const float* spread_w,
                          int d_model, int H, int d_head, float min_spread, int backward, void* stream);
 int proteus_embedding_bwd(const float* dout, const int64_t* tokens, float* dW, void* ws, size_t ws_bytes, long T, int V, int D, void* stream);
@@ -554,7 +554,8 @@ int proteus_embedding_bwd(const float* dout, const int64_t* tokens, float* dW, v
  *   form      PROTEUS_GEMM_NN: A [M][K], B [K][N];  _NT: A [M][K], B [N][K];  _TN: A [K][M], B [K][N]; rows lda, ldb, ldc elements apart.
  *             A matrix whose rows run along K (A in NN and NT, B in NT): K and its ld multiples of 4
  *   epilogue  PROTEUS_GEMM_F32: C f32;  _BF16: C bf16, rounded once;  _GELU: H = the sums f32, C = gelu(H) f32;
- *             _GELU_GRAD: C = sums * gelu'(h) f32;  _ADD: C = sums + h f32 (exact GELU; H and h laid out as C)
+ *             _GELU_GRAD: C = sums * gelu'(h) f32;  _ADD: C = sums + h f32 (exact GELU; H and h laid out as C).  NN takes all but _GELU, NT
+ *             _F32, _GELU and _ADD, TN _F32 alone; the rest is PROTEUS_ERR_UNSUPPORTED
  *   A, B, C 16-byte aligned; bias, h, H may be NULL where not asked for.  One launch without a workspace.
  *   ws        proteus_gemm_f32_workspace_bytes bytes, 16-byte aligned, or NULL: with it a TN product of few tiles and many rows (a gradient of a
  *             weight over many tokens; else 0 bytes are asked for) is cut along K over the chip, and a second launch adds up

@@ -168,7 +168,7 @@ def load():
     lib.proteus_layernorm_bwd.restype = ci
     lib.proteus_layernorm_bwd.argtypes = [vp] * 7 + [sz, cl, ci, vp]
     lib.proteus_colsum.restype = ci
-    lib.proteus_colsum.argtypes = [vp] * 5 + [sz, cl, ci, vp]
+    lib.proteus_colsum.argtypes = [vp] * 3 + [sz, cl, ci, vp]
     lib.proteus_heads_layout.restype = ci
     lib.proteus_heads_layout.argtypes = [ctypes.POINTER(vp)] + [vp] * 5 + [ci, ci, ci, cf, ci, vp]
     lib.proteus_embedding_bwd.restype = ci

@@ -175,7 +175,7 @@ extern "C" int proteus_encoder_layer_bwd(const float* x, const float* coords, co
     auto product = [&](const float* A, const float* B, const float* h, float* C, int m, int n, int kk, int lda, int ldb, int form, int epilogue) {
         return proteus_gemm_f32_ws(A, B, nullptr, h, C, nullptr, m, n, kk, lda, ldb, n, form, epilogue, b.shares_bytes ? b.shares : nullptr, b.shares_bytes, stream);
     };
-    auto column_sums = [&](const float* a, float* out, int C) { return proteus_colsum(a, nullptr, nullptr, out, b.sums, b.sums_bytes, s.rows, C, stream); };
+    auto column_sums = [&](const float* a, float* out, int C) { return proteus_colsum(a, out, b.sums, b.sums_bytes, s.rows, C, stream); };
     auto layernorm = [&](const float* d, const float* y, const float* stat, const float* gamma, float* dy, float* dgamma_dbeta) {
         return proteus_layernorm_bwd(d, y, stat, gamma, dy, dgamma_dbeta ? dgamma_dbeta : b.ln, b.lnws, b.ln_bytes, s.rows, dm, stream);
     };

@@ -155,19 +155,9 @@ void layernorm_bwd_kernel(const float* __restrict__ dout, const float* __restric
     for (int i = threadIdx.x; i < D; i += LN_WAVES * 64) { p[i] = red[0][i]; p[D + i] = red[1][i]; }
 }
 
-// d/dx of x Phi(x)
-__device__ __forceinline__ float gelu_grad(const float x) {
-    const float cdf = 0.5f * (1.0f + erff(x * 0.70710678118654752f));
-    return __builtin_fmaf(x, 0.39894228040143268f * expf(-0.5f * x * x), cdf);
-}
-
-// sums[slab][c] = sum over the slab's rows of v[row][c]; with GELU v = da * gelu'(h), written to dh as well.  torch:
-// GELU's derivative 10.4 us and a reduction of 15.2 us with a clearing launch in front, this 20.0 (2048 columns); a bias
-// gradient alone 10.8 - 14.1, this 5.6 - 6.3.
-template <bool GELU>
+// sums[slab][c] = sum over the slab's rows of a[row][c].  torch's reduction 10.8 - 14.1 us with a clearing launch in front, this 5.6 - 6.3 (2048 columns).
 __global__ __launch_bounds__(CS_BLOCK)
-void colsum_kernel(const float* __restrict__ a, const float* __restrict__ h, float* __restrict__ dh, float* __restrict__ sums,
-                   const long rows, const int C, const long slab_rows)
+void colsum_kernel(const float* __restrict__ a, float* __restrict__ sums, const long rows, const int C, const long slab_rows)
 {
     __shared__ float red[CS_BLOCK / 64][CS_COLS];
     const int q = threadIdx.x & 3, r = threadIdx.x >> 2;
@@ -177,13 +167,7 @@ void colsum_kernel(const float* __restrict__ a, const float* __restrict__ h, flo
     if (col < C) {
 #pragma unroll 4
         for (long row = r0 + r; row < r1; row += CS_BLOCK / 4) {
-            const size_t i = (size_t)row * C + col;
-            float4 v = *reinterpret_cast<const float4*>(a + i);
-            if (GELU) {
-                const float4 x = *reinterpret_cast<const float4*>(h + i);
-                v = make_float4(v.x * gelu_grad(x.x), v.y * gelu_grad(x.y), v.z * gelu_grad(x.z), v.w * gelu_grad(x.w));
-                *reinterpret_cast<float4*>(dh + i) = v;
-            }
+            const float4 v = *reinterpret_cast<const float4*>(a + (size_t)row * C + col);
             s[0] += v.x; s[1] += v.y; s[2] += v.z; s[3] += v.w;
         }
     }
@@ -204,13 +188,12 @@ void colsum_kernel(const float* __restrict__ a, const float* __restrict__ h, flo
     }
 }
 
-template <bool GELU>
-int colsum(const float* a, const float* h, float* dh, float* out, float* ws, long rows, int C, hipStream_t st) {
+int colsum(const float* a, float* out, float* ws, long rows, int C, hipStream_t st) {
     const long slabs = (rows + CS_ROWS - 1) / CS_ROWS;
     const dim3 grid((unsigned)((C + CS_COLS - 1) / CS_COLS), (unsigned)slabs);
-    hipLaunchKernelGGL((colsum_kernel<GELU>), grid, dim3(CS_BLOCK), 0, st, a, h, dh, slabs > 1 ? ws : out, rows, C, (long)CS_ROWS);
+    hipLaunchKernelGGL(colsum_kernel, grid, dim3(CS_BLOCK), 0, st, a, slabs > 1 ? ws : out, rows, C, (long)CS_ROWS);
     if (slabs > 1)
-        hipLaunchKernelGGL((colsum_kernel<false>), dim3(grid.x), dim3(CS_BLOCK), 0, st, ws, nullptr, nullptr, out, slabs, C, slabs);
+        hipLaunchKernelGGL(colsum_kernel, dim3(grid.x), dim3(CS_BLOCK), 0, st, ws, out, slabs, C, slabs);
     return (int)hipGetLastError();
 }
 
@@ -362,19 +345,18 @@ extern "C" int proteus_layernorm_bwd(const float* dout, const float* ysum, const
         default: LN_GO(8); break;
     }
 #undef LN_GO
-    return colsum<false>((const float*)ws, nullptr, nullptr, dgamma_dbeta, nullptr, groups, 2 * D, st);      // (at most CS_ROWS groups)
+    return colsum((const float*)ws, dgamma_dbeta, nullptr, groups, 2 * D, st);      // (at most CS_ROWS groups)
 }
 
-extern "C" int proteus_colsum(const float* a, const float* h, float* dh, float* sums, void* ws, size_t ws_bytes, long rows, int C, void* stream)
+extern "C" int proteus_colsum(const float* a, float* sums, void* ws, size_t ws_bytes, long rows, int C, void* stream)
 {
-    if (!a || !sums || (h && !dh)) return PROTEUS_ERR_NULL_POINTER;
+    if (!a || !sums) return PROTEUS_ERR_NULL_POINTER;
     if (rows <= 0 || C <= 0 || C % 4 || rows > 65535L * CS_ROWS) return PROTEUS_ERR_BAD_SHAPE;
     const size_t need = proteus_train_workspace_bytes(rows, C);
     if (need && !ws) return PROTEUS_ERR_NULL_POINTER;
     if (ws_bytes < need) return PROTEUS_ERR_BAD_SHAPE;
-    if (misaligned(a) || misaligned(h) || misaligned(dh) || misaligned(sums) || misaligned(ws)) return PROTEUS_ERR_BAD_ALIGNMENT;
-    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    return h ? colsum<true>(a, h, dh, sums, (float*)ws, rows, C, st) : colsum<false>(a, nullptr, nullptr, sums, (float*)ws, rows, C, st);
+    if (misaligned(a) || misaligned(sums) || misaligned(ws)) return PROTEUS_ERR_BAD_ALIGNMENT;
+    return colsum(a, sums, (float*)ws, rows, C, reinterpret_cast<hipStream_t>(stream));
 }
 
 extern "C" int proteus_heads_layout(float* const* tensors, float* W, float* b, float* Wo, float* sigma, const float* spread_w,
@@ -407,5 +389,5 @@ extern "C" int proteus_embedding_bwd(const float* dout, const int64_t* tokens, f
     float* part = (float*)ws;
     hipLaunchKernelGGL(embedding_bwd_kernel, dim3((unsigned)((D + 63) / 64), (unsigned)slabs), dim3(256), (size_t)4 * V * 64 * 4, st,
                        dout, tokens, part, T, V, D);
-    return colsum<false>(part, nullptr, nullptr, dW, part + (size_t)slabs * V * D, slabs, V * D, st);
+    return colsum(part, dW, part + (size_t)slabs * V * D, slabs, V * D, st);
 }

@@ -296,7 +296,7 @@ struct RowSource {
 };
 
 // Accumulators e0 to e0 + COUNT of a 64 x 64 tile at (m0, n0), a lane's sums of each.
-template <int COUNT, int EPI>
+template <int COUNT>
 __device__ __forceinline__ void finish_rows(const GemmArgs& g, const int m0, const int n0, const int e0, const float (&v)[COUNT])
 {
     const int lane = threadIdx.x & 63, r0 = lane & 31, half = lane >> 5;
@@ -307,7 +307,7 @@ __device__ __forceinline__ void finish_rows(const GemmArgs& g, const int m0, con
     for (int i = 0; i < COUNT; ++i) {
         const int e = e0 + i;
         if (m0 + row(e) >= g.M || column(e) >= g.N) continue;
-        if (fabsf(v[i]) <= 3.4028234e38f) write<EPI>(g, m0 + row(e), column(e), v[i] * REDUCED);
+        if (fabsf(v[i]) <= 3.4028234e38f) write<PROTEUS_GEMM_F32>(g, m0 + row(e), column(e), v[i] * REDUCED);
         else again |= 1u << i;
     }
     if (__builtin_amdgcn_ballot_w64(again != 0) == 0) return;
@@ -324,7 +324,7 @@ __device__ __forceinline__ void finish_rows(const GemmArgs& g, const int m0, con
     for (; again; again &= again - 1) {
         const int e = e0 + __builtin_ctz(again), j = (e >> 4) & 1;
         const bool nan = ((e >> 5 ? rows_a[1] : rows_a[0]) >> (row(e) & 31) | (j ? cols_b[1] : cols_b[0]) >> r0) & 1;
-        write<EPI>(g, m0 + row(e), column(e), nan ? __builtin_nanf("") : plain_dot<false, false>(g, m0 + row(e), column(e)));
+        write<PROTEUS_GEMM_F32>(g, m0 + row(e), column(e), nan ? __builtin_nanf("") : plain_dot<false, false>(g, m0 + row(e), column(e)));
     }
 }
 
@@ -338,7 +338,7 @@ __device__ __forceinline__ void tile_at(const GemmArgs& g, const int tile, int& 
     n0 = (wide ? tile / tiles_m : tile % g.tiles_n) * GT;
 }
 
-template <int W, int EPI>
+template <int W>
 __global__ __launch_bounds__(W * 64, 2)
 void gemm_f32_rows_kernel(const GemmArgs g)
 {
@@ -408,11 +408,10 @@ void gemm_f32_rows_kernel(const GemmArgs g)
         for (int e = 0; e < 64 / W; ++e) to[e * 64] = v[e];
         return;
     }
-    finish_rows<64 / W, EPI>(g, m0, n0, wave * (64 / W), v);
+    finish_rows<64 / W>(g, m0, n0, wave * (64 / W), v);
 }
 
 // The shares' sums of a tile together, in their order: a quarter of a tile per workgroup, four accumulators per wave.
-template <int EPI>
 __global__ __launch_bounds__(256)
 void gemm_f32_rows_sum_kernel(const GemmArgs g)
 {
@@ -426,7 +425,7 @@ void gemm_f32_rows_sum_kernel(const GemmArgs g)
         for (int i = 0; i < 4; ++i) v[i] += from[s * pitch + i * 64];
     int m0, n0;
     tile_at(g, tile, m0, n0);
-    finish_rows<4, EPI>(g, m0, n0, e0, v);
+    finish_rows<4>(g, m0, n0, e0, v);
 }
 
 template <bool AK, bool BK, int EPI>
@@ -439,12 +438,12 @@ int gemm_go(GemmArgs g, hipStream_t st)
     const dim3 grid((unsigned)g.per_xcd * 8);
     if constexpr (!AK) {
         // Waves per tile: two per SIMD where the steps allow.
-#define GO(W_) hipLaunchKernelGGL((gemm_f32_rows_kernel<W_, EPI>), grid, dim3(W_ * 64), (size_t)W_ * 64 * 64 * 4, st, g)
+#define GO(W_) hipLaunchKernelGGL((gemm_f32_rows_kernel<W_>), grid, dim3(W_ * 64), (size_t)W_ * 64 * 64 * 4, st, g)
         if (g.tiles > 512)      GO(2);
         else if (g.tiles > 256) GO(4);
         else                    GO(8);
 #undef GO
-        if (g.shares > 1) hipLaunchKernelGGL((gemm_f32_rows_sum_kernel<EPI>), dim3((unsigned)g.tiles * 4), dim3(256), 0, st, g);
+        if (g.shares > 1) hipLaunchKernelGGL(gemm_f32_rows_sum_kernel, dim3((unsigned)g.tiles * 4), dim3(256), 0, st, g);
     } else {
         // Groups per tile: four waves per SIMD where the tiles allow.
 #define GO(G_) do { \
@@ -496,7 +495,9 @@ extern "C" int proteus_gemm_f32_ws(const float* A, const float* B, const float* 
                                    int M, int N, int K, int lda, int ldb, int ldc, int form, int epilogue, void* ws, size_t ws_bytes, void* stream)
 {
     if (!A || !B || !C || (epilogue == PROTEUS_GEMM_GELU && !H) || ((epilogue == PROTEUS_GEMM_GELU_GRAD || epilogue == PROTEUS_GEMM_ADD) && !h)) return PROTEUS_ERR_NULL_POINTER;
-    if (form < 0 || form > PROTEUS_GEMM_TN || epilogue < 0 || epilogue > PROTEUS_GEMM_ADD) return PROTEUS_ERR_UNSUPPORTED;
+    if (form < 0 || form > PROTEUS_GEMM_TN || epilogue < 0 || epilogue > PROTEUS_GEMM_ADD || (form == PROTEUS_GEMM_TN && epilogue != PROTEUS_GEMM_F32)
+        || (form == PROTEUS_GEMM_NN && epilogue == PROTEUS_GEMM_GELU) || (form == PROTEUS_GEMM_NT && (epilogue == PROTEUS_GEMM_BF16 || epilogue == PROTEUS_GEMM_GELU_GRAD)))
+        return PROTEUS_ERR_UNSUPPORTED;
     if (M <= 0 || N <= 0 || K <= 0 || ldc < N || lda < (form == PROTEUS_GEMM_TN ? M : K) || ldb < (form == PROTEUS_GEMM_NT ? K : N)) return PROTEUS_ERR_BAD_SHAPE;
     // (tiles are numbered in 32 bits)
     if ((int64_t)((M + (int64_t)GT - 1) / GT) * ((N + (int64_t)GT - 1) / GT) > (1 << 30)) return PROTEUS_ERR_TOO_LARGE;
@@ -515,18 +516,20 @@ extern "C" int proteus_gemm_f32_ws(const float* A, const float* B, const float* 
     }
     const GemmArgs g = {A, B, bias, h, C, H, M, N, K, lda, ldb, ldc, 0, 0, 0, static_cast<float*>(ws), cut.number, cut.steps};
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-#define EPILOGUES(AK_, BK_) \
-    switch (epilogue) { \
-        case PROTEUS_GEMM_F32:  return gemm_go<AK_, BK_, PROTEUS_GEMM_F32>(g, st); \
-        case PROTEUS_GEMM_BF16: return gemm_go<AK_, BK_, PROTEUS_GEMM_BF16>(g, st); \
-        case PROTEUS_GEMM_GELU: return gemm_go<AK_, BK_, PROTEUS_GEMM_GELU>(g, st); \
-        case PROTEUS_GEMM_ADD:  return gemm_go<AK_, BK_, PROTEUS_GEMM_ADD>(g, st); \
-        default:                return gemm_go<AK_, BK_, PROTEUS_GEMM_GELU_GRAD>(g, st); \
+    // (what the training step asks for; nothing else is built)
+#define GO(AK_, BK_, E_) case E_: return gemm_go<AK_, BK_, E_>(g, st)
+    if (form == PROTEUS_GEMM_NN) switch (epilogue) {
+        GO(true, false, PROTEUS_GEMM_F32);
+        GO(true, false, PROTEUS_GEMM_BF16);
+        GO(true, false, PROTEUS_GEMM_GELU_GRAD);
+        GO(true, false, PROTEUS_GEMM_ADD);
     }
-    switch (form) {
-        case PROTEUS_GEMM_NN: EPILOGUES(true, false)
-        case PROTEUS_GEMM_NT: EPILOGUES(true, true)
-        default:              EPILOGUES(false, false)
+    else if (form == PROTEUS_GEMM_NT) switch (epilogue) {
+        GO(true, true, PROTEUS_GEMM_F32);
+        GO(true, true, PROTEUS_GEMM_GELU);
+        GO(true, true, PROTEUS_GEMM_ADD);
     }
-#undef EPILOGUES
+    else return gemm_go<false, false, PROTEUS_GEMM_F32>(g, st);
+#undef GO
+    return PROTEUS_ERR_UNSUPPORTED;
 }

@@ -123,7 +123,7 @@ def column_sums(a):
     rows, C = a.shape
     sums = torch.empty(C, dtype=torch.float32, device=a.device)
     n = _bytes("proteus_train_workspace_bytes", rows, C)
-    _call("proteus_colsum", a.device, a, None, None, sums, _workspace(n, a.device), n, rows, C)
+    _call("proteus_colsum", a.device, a, sums, _workspace(n, a.device), n, rows, C)
     return sums
 
 
@@ -132,10 +132,10 @@ def column_sums(a):
 NN, NT, TN = _lib.GEMM_NN, _lib.GEMM_NT, _lib.GEMM_TN
 
 
-def _product(form, A, B, bias=None, gelu=False, gelu_grad_of=None, dtype=torch.float32):
+def _product(form, A, B, bias=None, gelu=False, gelu_grad_of=None):
     """A B (NN), A B^T (NT) or A^T B (TN) of dense fp32 matrices, plus `bias` per column: one launch of the library's product, which
     issues in a fifth of the host time of torch's; torch's where rows are not multiples of 16 bytes or a matrix has 2 GiB.
-    gelu: returns (sums, gelu(sums)); gelu_grad_of: sums * gelu'(gelu_grad_of); dtype: of the result (bf16: the sums rounded once)."""
+    gelu (NT): returns (sums, gelu(sums)); gelu_grad_of (NN): sums * gelu'(gelu_grad_of)."""
     M, K = A.shape if form != TN else A.shape[::-1]
     N = B.shape[0] if form == NT else B.shape[1]
     if not ((form == TN or K % 4 == 0) and (A.shape[0] + 512) * A.shape[1] < 2 ** 29 and (B.shape[0] + 512) * B.shape[1] < 2 ** 29):
@@ -143,10 +143,10 @@ def _product(form, A, B, bias=None, gelu=False, gelu_grad_of=None, dtype=torch.f
         C = Am.mm(Bm) if bias is None else torch.addmm(bias, Am, Bm)
         if gelu:
             return C, F.gelu(C)
-        return C.to(dtype) if gelu_grad_of is None else torch.ops.aten.gelu_backward(C, gelu_grad_of)
-    C = torch.empty(M, N, dtype=dtype, device=A.device)
+        return C if gelu_grad_of is None else torch.ops.aten.gelu_backward(C, gelu_grad_of)
+    C = torch.empty(M, N, dtype=torch.float32, device=A.device)
     H = torch.empty_like(C) if gelu else None
-    epilogue = _lib.GEMM_GELU if gelu else _lib.GEMM_GELU_GRAD if gelu_grad_of is not None else _lib.GEMM_BF16 if dtype == torch.bfloat16 else _lib.GEMM_F32
+    epilogue = _lib.GEMM_GELU if gelu else _lib.GEMM_GELU_GRAD if gelu_grad_of is not None else _lib.GEMM_F32
     n = _bytes("proteus_gemm_f32_workspace_bytes", M, N, K, form) if form == TN else 0
     _call("proteus_gemm_f32_ws", A.device, A, B, bias, gelu_grad_of, C, H, M, N, K, A.shape[1], B.shape[1], N, form, epilogue, _workspace(n, A.device), n)
     return (H, C) if gelu else C

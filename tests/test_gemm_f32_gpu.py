@@ -62,11 +62,20 @@ def test_magnitudes(gpu, form, ea, eb):
     assert bool(((got - want).abs() <= (12 * 7 + 16) * 2.0 ** -24 * mass + 2.0 ** -149).all())
 
 
+def _epilogue(form, epilogue, A, B, bias=None, h=None):
+    """The entry point itself, with the matrices' sizes as in _product."""
+    M, K = A.shape
+    N = B.shape[0] if form == NT else B.shape[1]
+    C = torch.empty(M, N, dtype=torch.bfloat16 if epilogue == _lib.GEMM_BF16 else torch.float32, device=A.device)
+    train_ops._call("proteus_gemm_f32", A.device, A, B, bias, h, C, None, M, N, K, A.shape[1], B.shape[1], N, form, epilogue)
+    return C
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M", [5, 700])
 def test_epilogues(gpu, M):
     A, B, want, mass = _operands(NT, M, 132, 72, gpu)
-    bias, h = torch.randn(132, device=gpu), torch.randn(M, 132, device=gpu)
+    Bt, bias, h = B.t().contiguous(), torch.randn(132, device=gpu), torch.randn(M, 132, device=gpu)
     bound = 76 * 2.0 ** -24 * mass + 2.0 ** -23 * bias.abs()
     H, C = train_ops._product(NT, A, B, bias, gelu=True)
     assert bool(((H - want - bias).abs() <= bound).all())
@@ -75,9 +84,12 @@ def test_epilogues(gpu, M):
     assert bool(((C - exact).abs() <= 2.0 ** -21 * H.abs()).all())
     hd = h.double().requires_grad_(True)
     grad, = torch.autograd.grad(torch.nn.functional.gelu(hd).sum(), hd)
-    plain = train_ops._product(NT, A, B, bias)
-    assert bool(((train_ops._product(NT, A, B, bias, gelu_grad_of=h) - plain.double() * grad).abs() <= 2.0 ** -20 * plain.abs() * (1 + h.abs())).all())
-    assert torch.equal(train_ops._product(NT, A, B, bias, dtype=torch.bfloat16), plain.to(torch.bfloat16))
+    plain = train_ops._product(NN, A, Bt, bias)
+    assert bool(((plain - want - bias).abs() <= bound).all())
+    assert bool(((train_ops._product(NN, A, Bt, bias, gelu_grad_of=h) - plain.double() * grad).abs() <= 2.0 ** -20 * plain.abs() * (1 + h.abs())).all())
+    assert torch.equal(_epilogue(NN, _lib.GEMM_BF16, A, Bt, bias), plain.to(torch.bfloat16))
+    assert torch.equal(_epilogue(NN, _lib.GEMM_ADD, A, Bt, None, h), train_ops._product(NN, A, Bt) + h)
+    assert torch.equal(_epilogue(NT, _lib.GEMM_ADD, A, B, bias, h), train_ops._product(NT, A, B, bias) + h)
 
 
 @pytest.mark.gpu
@@ -136,10 +148,19 @@ def test_values_that_do_not_split(gpu, form, M, N, K):
 def test_what_it_refuses():
     lib = _lib.load()
     at = ctypes.c_void_p(4096)
-    def call(A=at, B=at, C=at, H=None, M=8, N=8, K=8, lda=8, ldb=8, ldc=8, form=NN, epilogue=0):
-        return lib.proteus_gemm_f32(A, B, None, None, C, H, M, N, K, lda, ldb, ldc, form, epilogue, None)
-    assert call(A=None) < 0 and call(C=None) < 0 and call(epilogue=_lib.GEMM_GELU) < 0 and call(epilogue=_lib.GEMM_GELU_GRAD) < 0
-    assert call(form=3) < 0 and call(epilogue=4) < 0
+
+    def call(A=at, B=at, C=at, h=None, H=None, M=8, N=8, K=8, lda=8, ldb=8, ldc=8, form=NN, epilogue=0):
+        return lib.proteus_gemm_f32(A, B, None, h, C, H, M, N, K, lda, ldb, ldc, form, epilogue, None)
+    null, unsupported = call(A=None), call(form=3)
+    assert null < 0 and unsupported < 0 and null != unsupported
+    assert call(C=None) == call(form=NT, epilogue=_lib.GEMM_GELU) == call(epilogue=_lib.GEMM_GELU_GRAD) == call(epilogue=_lib.GEMM_ADD) == null
+    # unknown ones, and combinations that the training step does not ask for
+    assert call(epilogue=5, h=at, H=at) == call(epilogue=-1, h=at, H=at) == unsupported
+    for form, epilogue in ((NN, _lib.GEMM_GELU), (NT, _lib.GEMM_BF16), (NT, _lib.GEMM_GELU_GRAD), (TN, _lib.GEMM_BF16), (TN, _lib.GEMM_GELU), (TN, _lib.GEMM_GELU_GRAD), (TN, _lib.GEMM_ADD)):
+        assert call(form=form, epilogue=epilogue, h=at, H=at) == unsupported, (form, epilogue)
     assert call(M=0) < 0 and call(K=6, lda=8) < 0 and call(lda=6) < 0 and call(ldc=4) < 0 and call(form=NT, ldb=10) < 0
     assert call(A=ctypes.c_void_p(4100)) < 0
     assert call(M=1 << 28, lda=8) < 0                                           # (2 GiB and more)
+    assert lib.proteus_gemm_f32_ws(at, at, None, None, at, None, 8, 8, 4096, 8, 8, 8, TN, 0, ctypes.c_void_p(4100), 1 << 30, None) < 0      # (the workspace's alignment)
+    size = lib.proteus_gemm_f32_workspace_bytes
+    assert size(64, 64, 4096, TN) > 0 and size(64, 64, 4096, NN) == size(0, 64, 4096, TN) == size(64, 64, 1 << 30, TN) == 0
