@@ -437,21 +437,25 @@ int gemm_go(GemmArgs g, hipStream_t st)
     g.per_xcd = (g.tiles * g.shares + 7) / 8;
     const dim3 grid((unsigned)g.per_xcd * 8);
     if constexpr (!AK) {
-        // Waves per tile: two per SIMD where the steps allow.
+        // Waves per tile, of which a SIMD holds two: 8 while there is a tile at most per compute unit, 4 up to two or for several rounds, 2 for a single round of
+        // four.  Us with 2 / 4 / 8, 512 and 2048 tokens: 256 tiles 17.0 / 11.8 / 11.1 and 49 / 31 / 29, 288 25.0 / 16.7 / 19.7 and 79 / 47 / 51, 768 28.4 / 25.6 / 29.8 and 91 / 79 / 84,
+        // 896 29.9 / 31.3 / 38.2 and 95 / 98 / 105, 1024 31.6 / 32.7 / 38.9 and 103 / 104 / 111, 2048 64 / 61 / 76 and 209 / 203 / 221.
 #define GO(W_) hipLaunchKernelGGL((gemm_f32_rows_kernel<W_>), grid, dim3(W_ * 64), (size_t)W_ * 64 * 64 * 4, st, g)
-        if (g.tiles > 512)      GO(2);
-        else if (g.tiles > 256) GO(4);
-        else                    GO(8);
+        if (g.tiles <= 256)                        GO(8);
+        else if (g.tiles > 768 && g.tiles <= 1024) GO(2);
+        else                                       GO(4);
 #undef GO
         if (g.shares > 1) hipLaunchKernelGGL(gemm_f32_rows_sum_kernel, dim3((unsigned)g.tiles * 4), dim3(256), 0, st, g);
     } else {
-        // Groups per tile: four waves per SIMD where the tiles allow.
+        // Groups per tile, of which a compute unit holds four: as many as its tiles leave room for in one round.  Us with 1 / 2 / 4, K = 512 and 2048, X W^T: 256 tiles
+        // 16.2 / 13.1 / 10.8 and 51 / 40 / 33, 288 18.7 / 16.6 / 18.9 and 61 / 52 / 57, 512 20.8 / 19.0 / 19.8 and 70 / 63 / 64, 544 25.4 / 26.7 / 27.7 and 88 / 90 / 88, 1024 35.4 / 35.0 / 37.6 and
+        // 128 / 122 / 125, 2048 66 / 67 / 73 and 245 / 237 / 250; X W the same but for 1024 and 2048 tiles, K = 2048, 130 / 127 / 135 and 247 / 250 / 270.
 #define GO(G_) do { \
             constexpr size_t sums = (G_) > 1 ? (size_t)(G_) * 4 * 16 * 64 * 4 : 0; \
             hipLaunchKernelGGL((gemm_f32_kernel<AK, BK, G_, EPI>), grid, dim3(G_ * 256), G_ * 2 * STAGE > sums ? G_ * 2 * STAGE : sums, st, g); \
         } while (0)
-        if (g.tiles > 640)      GO(1);
-        else if (g.tiles > 320) GO(2);
+        if (g.tiles > 512)      GO(1);
+        else if (g.tiles > 256) GO(2);
         else                    GO(4);
 #undef GO
     }

@@ -16,10 +16,11 @@ def _operands(form, M, N, K, gpu):
     return (A.t().contiguous() if form == TN else A), (B.t().contiguous() if form == NT else B), A.double() @ B.double(), A.double().abs() @ B.double().abs()
 
 
-# Edges of the 64 x 64 tiles, of the steps of 16 k and of what 1, 2 and 4 groups share out (more than 640 tiles, 321 to 640, fewer).
+# Edges of the 64 x 64 tiles, of the steps of 16 k and of what 1, 2 and 4 groups share out (more than 512 tiles, 257 to 512, fewer);
+# gradients of weights: 4, 2 and 8 waves (928 tiles: 2).
 @pytest.mark.gpu
 @pytest.mark.parametrize("form", [NN, NT, TN])
-@pytest.mark.parametrize("M,N,K", [(1, 1, 4), (63, 65, 16), (64, 64, 20), (65, 36, 68), (130, 512, 132), (1, 20, 512), (1100, 1200, 36), (1700, 1600, 52)])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 4), (63, 65, 16), (64, 64, 20), (65, 36, 68), (130, 512, 132), (1, 20, 512), (1100, 1200, 36), (1700, 1600, 52), (2000, 1800, 20)])
 def test_product_against_float64(gpu, form, M, N, K):
     if form == TN:
         K -= 3                                                                  # (rows along K need no multiple of 4)
@@ -126,7 +127,7 @@ def test_a_diverged_operand_is_read_to_its_end(gpu, form, K):
 
 # (gradients of weights: 8, 4 and 2 waves per tile, and shares of K)
 @pytest.mark.gpu
-@pytest.mark.parametrize("form,M,N,K", [(NN, 70, 68, 36), (NT, 70, 68, 36), (NN, 1700, 1600, 36), (NT, 1100, 1200, 36), (TN, 70, 68, 36), (TN, 70, 68, 2100), (TN, 1100, 1000, 37), (TN, 1700, 1600, 38)])
+@pytest.mark.parametrize("form,M,N,K", [(NN, 70, 68, 36), (NT, 70, 68, 36), (NN, 1700, 1600, 36), (NT, 1100, 1200, 36), (TN, 70, 68, 36), (TN, 70, 68, 2100), (TN, 1100, 1000, 37), (TN, 2000, 1800, 38)])
 def test_values_that_do_not_split(gpu, form, M, N, K):
     A, B, _, _ = _operands(NN, M, N, K, gpu)
     bad = [(3, 5, float("inf")), (7, 1, float("nan")), (9, 2, 3.4e38), (11, 3, -3.39e38)]      # (bf16 ends at 3.39e38)
