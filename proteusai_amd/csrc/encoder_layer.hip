@@ -1,10 +1,10 @@
 // A post-LN encoder layer's training step, one call per direction: the order in which the kernels of the layer are launched
 // and where in the two buffers their tensors lie.  Host code: launches cost 2 to 3 us each from here, 6 to 10 from Python and
-// 18 to 29 through torch's products, and a layer has 9 of them forward and 18 to 22 backward, of which most last less than that.
+// 18 to 29 through torch's products, and a layer has 9 of them forward and 18 to 20 backward, of which most last less than that.
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
-#include "proteus_hip.h"
+#include "gemm_f32_internal.h"
 
 namespace {
 
@@ -69,8 +69,8 @@ struct Forward {
 struct Backward {
     float *dy2, *dh, *dx1, *dy1, *dO, *D, *g, *d_sigma, *dW, *db, *dWo, *ln;
     uint16_t* dO16;
-    void *lnws, *sums, *shares;
-    size_t ln_bytes, sums_bytes, shares_bytes, bytes;
+    void *lnws, *sums, *shares[4];                                               // of the gradients of weights: W2, W1, output projection, projections
+    size_t ln_bytes, sums_bytes, shares_bytes[4], bytes;
     Backward(const Sizes& s, void* base)
     {
         Carve c{static_cast<char*>(base)};
@@ -86,14 +86,11 @@ struct Backward {
         lnws = c.take<char>(ln_bytes);
         sums_bytes = proteus_train_workspace_bytes(s.rows, s.hidden > 3 * s.dm ? s.hidden : 3 * s.dm);
         sums = c.take<char>(sums_bytes);
-        // (one product after the other: the largest of the four gradients of weights)
-        shares_bytes = 0;
         const int sizes[4][2] = {{s.dm, s.hidden}, {s.hidden, s.dm}, {s.dm, s.dm}, {s.dm, 3 * s.dm}};
-        for (const auto& z : sizes) {
-            const size_t n = proteus_gemm_f32_workspace_bytes(z[0], z[1], (int)s.rows, PROTEUS_GEMM_TN);
-            if (n > shares_bytes) shares_bytes = n;
-        }
-        shares = c.take<char>(shares_bytes);
+        for (int i = 0; i < 4; ++i) shares_bytes[i] = proteus_gemm_f32_workspace_bytes(sizes[i][0], sizes[i][1], (int)s.rows, PROTEUS_GEMM_TN);
+        // (the last one's come when the others' are added up)
+        shares[0] = shares[3] = c.take<char>(shares_bytes[0] > shares_bytes[3] ? shares_bytes[0] : shares_bytes[3]);
+        shares[1] = c.take<char>(shares_bytes[1]); shares[2] = c.take<char>(shares_bytes[2]);
         bytes = c.at;
     }
 };
@@ -173,7 +170,12 @@ extern "C" int proteus_encoder_layer_bwd(const float* x, const float* coords, co
     if (kept_bytes < k.bytes || ws_bytes < b.bytes) return PROTEUS_ERR_BAD_SHAPE;
     const int rows = (int)s.rows, dm = s.dm;
     auto product = [&](const float* A, const float* B, const float* h, float* C, int m, int n, int kk, int lda, int ldb, int form, int epilogue) {
-        return proteus_gemm_f32_ws(A, B, nullptr, h, C, nullptr, m, n, kk, lda, ldb, n, form, epilogue, b.shares_bytes ? b.shares : nullptr, b.shares_bytes, stream);
+        return proteus_gemm_f32(A, B, nullptr, h, C, nullptr, m, n, kk, lda, ldb, n, form, epilogue, stream);
+    };
+    // (The shares of several in one launch, which must come before their operands are written over: it sums what is not finite again.)
+    proteus_gemm::PendingSums pending;
+    auto gradient = [&](const float* A, const float* B, float* C, int m, int n, int which) {
+        return proteus_gemm::gemm_begin(A, B, C, m, n, rows, m, n, n, b.shares_bytes[which] ? b.shares[which] : nullptr, b.shares_bytes[which], pending, stream);
     };
     auto column_sums = [&](const float* a, float* out, int C) { return proteus_colsum(a, out, b.sums, b.sums_bytes, s.rows, C, stream); };
     auto layernorm = [&](const float* d, const float* y, const float* stat, const float* gamma, float* dy, float* dgamma_dbeta) {
@@ -184,17 +186,18 @@ extern "C" int proteus_encoder_layer_bwd(const float* x, const float* coords, co
     const bool first_norm = attention || g[P_WO] || g[P_G1];
 
     TRY(layernorm(dout, k.y2, k.stat2, p[P_G2], b.dy2, g[P_G2]));
-    if (g[P_W2])    TRY(product(b.dy2, k.a, nullptr, g[P_W2], dm, hidden, rows, dm, hidden, PROTEUS_GEMM_TN, PROTEUS_GEMM_F32));
+    if (g[P_W2])    TRY(gradient(b.dy2, k.a, g[P_W2], dm, hidden, 0));
     if (g[P_BIAS2]) TRY(column_sums(b.dy2, g[P_BIAS2], dm));
-    if (!(first_norm || g[P_W1] || g[P_BIAS1])) return PROTEUS_OK;
+    if (!(first_norm || g[P_W1] || g[P_BIAS1])) return proteus_gemm::gemm_sums(pending, stream);
     TRY(product(b.dy2, p[P_W2], k.h, b.dh, rows, hidden, dm, dm, hidden, PROTEUS_GEMM_NN, PROTEUS_GEMM_GELU_GRAD));
-    if (g[P_W1])    TRY(product(b.dh, k.x1, nullptr, g[P_W1], hidden, dm, rows, hidden, dm, PROTEUS_GEMM_TN, PROTEUS_GEMM_F32));
+    if (g[P_W1])    TRY(gradient(b.dh, k.x1, g[P_W1], hidden, dm, 1));
     if (g[P_BIAS1]) TRY(column_sums(b.dh, g[P_BIAS1], hidden));
-    if (!first_norm) return PROTEUS_OK;
+    if (!first_norm) return proteus_gemm::gemm_sums(pending, stream);
     TRY(product(b.dh, p[P_W1], b.dy2, b.dx1, rows, dm, hidden, hidden, dm, PROTEUS_GEMM_NN, PROTEUS_GEMM_ADD));
     TRY(layernorm(b.dx1, k.y1, k.stat1, p[P_G1], b.dy1, g[P_G1]));
-    if (g[P_WO]) TRY(product(b.dy1, k.O, nullptr, b.dWo, dm, dm, rows, dm, dm, PROTEUS_GEMM_TN, PROTEUS_GEMM_F32));
+    if (g[P_WO]) TRY(gradient(b.dy1, k.O, b.dWo, dm, dm, 2));
     if (attention) {
+        TRY(proteus_gemm::gemm_sums(pending, stream));                          // dO takes dy2's place, g dh's
         TRY(product(b.dy1, k.Wo, nullptr, b.dO, rows, dm, dm, dm, dm, PROTEUS_GEMM_NN, PROTEUS_GEMM_F32));
         int64_t st[21];
         for (int i = 0; i < 3; ++i) head_strides(st + 3 * i, s, 1);          // O, dO, dO in bf16
@@ -202,10 +205,11 @@ extern "C" int proteus_encoder_layer_bwd(const float* x, const float* coords, co
         for (int i = 0; i < 7; ++i) head_strides(st + 3 * i, s, i == 3 ? 1 : 3);
         TRY(proteus_geo_attn_bwd_typed(k.qkv, k.qkv + dm, k.qkv + 2 * dm, b.dO16, st, coords, k.sigma, nullptr, mask, k.L, b.D, b.g, b.g + dm, b.g + 2 * dm,
                                        b.d_sigma, nullptr, Z, H, N, d_head, 0.0f, 1.0f, PROTEUS_OPERAND_BF16, PROTEUS_GRAD_F32, stream));
-        if (projections) TRY(product(x, b.g, nullptr, b.dW, dm, 3 * dm, rows, dm, 3 * dm, PROTEUS_GEMM_TN, PROTEUS_GEMM_F32));
+        if (projections) TRY(gradient(x, b.g, b.dW, dm, 3 * dm, 3));
         if (biases)      TRY(column_sums(b.g, b.db, 3 * dm));
         if (dx)          TRY(product(b.g, k.W, b.dy1, dx, rows, dm, 3 * dm, 3 * dm, 3 * dm, PROTEUS_GEMM_NT, PROTEUS_GEMM_ADD));
     }
+    TRY(proteus_gemm::gemm_sums(pending, stream));
     if (projections || biases || g[P_SPREAD] || g[P_WO])
         TRY(proteus_heads_layout(g, b.dW, b.db, b.dWo, b.d_sigma, k.spread, dm, H, d_head, min_spread, 1, stream));
     return PROTEUS_OK;

@@ -31,9 +31,11 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
-#include "proteus_hip.h"
+#include "gemm_f32_internal.h"
 
 namespace {
+
+using namespace proteus_gemm;
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -46,15 +48,6 @@ constexpr int CHUNK     = GT * 16 + 64;             // bytes of 8 k of all rows 
 constexpr int PIECE     = 2 * CHUNK;
 constexpr int OPERAND   = 3 * PIECE;
 constexpr int STAGE     = 2 * OPERAND;              // of one group
-
-struct GemmArgs {
-    const float *A, *B, *bias, *h;
-    void  *C;
-    float *H;
-    int M, N, K, lda, ldb, ldc, tiles_n, tiles, per_xcd;
-    float *part;                                    // sums of the shares of K, where a product is cut
-    int shares, steps;                              // their number, and the steps of each
-};
 
 __device__ __forceinline__ uint32_t pack2(const float a, const float b) {
     const f32x2 f = {a, b};
@@ -413,9 +406,12 @@ void gemm_f32_rows_kernel(const GemmArgs g)
 
 // The shares' sums of a tile together, in their order: a quarter of a tile per workgroup, four accumulators per wave.
 __global__ __launch_bounds__(256)
-void gemm_f32_rows_sum_kernel(const GemmArgs g)
+void gemm_f32_rows_sum_kernel(const PendingSums sums)
 {
-    const int tile = blockIdx.x >> 2, e0 = (blockIdx.x & 3) * 16 + (threadIdx.x >> 6) * 4;
+    int p = 0;
+    while ((int)blockIdx.x >= sums.first[p + 1]) ++p;
+    const GemmArgs& g = sums.product[p];
+    const int block = (int)blockIdx.x - sums.first[p], tile = block >> 2, e0 = (block & 3) * 16 + (threadIdx.x >> 6) * 4;
     const float* from = g.part + (size_t)tile * (GT * GT) + e0 * 64 + (threadIdx.x & 63);
     const size_t pitch = (size_t)g.tiles * (GT * GT);
     float v[4] = {};
@@ -429,7 +425,7 @@ void gemm_f32_rows_sum_kernel(const GemmArgs g)
 }
 
 template <bool AK, bool BK, int EPI>
-int gemm_go(GemmArgs g, hipStream_t st)
+int gemm_go(GemmArgs g, hipStream_t st, PendingSums* sums = nullptr)
 {
     const int tm = (g.M + GT - 1) / GT;
     g.tiles_n = (g.N + GT - 1) / GT;
@@ -445,7 +441,14 @@ int gemm_go(GemmArgs g, hipStream_t st)
         else if (g.tiles > 768 && g.tiles <= 1024) GO(2);
         else                                       GO(4);
 #undef GO
-        if (g.shares > 1) hipLaunchKernelGGL(gemm_f32_rows_sum_kernel, dim3((unsigned)g.tiles * 4), dim3(256), 0, st, g);
+        if (g.shares > 1) {
+            PendingSums own;
+            PendingSums& p = sums ? *sums : own;
+            p.product[p.count] = g;
+            p.first[p.count + 1] = p.first[p.count] + g.tiles * 4;
+            ++p.count;
+            if (!sums) return gemm_sums(own, st);
+        }
     } else {
         // Groups per tile, of which a compute unit holds four: as many as its tiles leave room for in one round.  Us with 1 / 2 / 4, K = 512 and 2048, X W^T: 256 tiles
         // 16.2 / 13.1 / 10.8 and 51 / 40 / 33, 288 18.7 / 16.6 / 18.9 and 61 / 52 / 57, 512 20.8 / 19.0 / 19.8 and 70 / 63 / 64, 544 25.4 / 26.7 / 27.7 and 88 / 90 / 88, 1024 35.4 / 35.0 / 37.6 and
@@ -464,7 +467,8 @@ int gemm_go(GemmArgs g, hipStream_t st)
 
 // Gradients of weights: shares of K for workgroups of their own where the tiles leave compute units idle, so that at most 256 workgroups of 8 waves, one
 // per compute unit, are launched; at least 256 of K each (a round of 8 waves, two by two) and at most 32 of them, whose sums the second launch
-// adds up, and only where a workgroup is spared 768 of K, which is what that launch takes.  One, shares of 256, 512 and 1024, and the library, us:
+// adds up, and only where a workgroup is spared 1536 of K: that launch takes 4 us of the device and 3 of the host, which is what bounds a training step of fewer
+// tokens (2 x 600, d_model 256, 3 layers 1025 us, from 768 spared on and a launch per product 1065).  One, shares of 256, 512 and 1024, and the library, us:
 // 128 x 128 of 2048 tokens 23 / 9.9 / 11.8 / 16 / 14, of 8192 75 / 14 / 14 / 17 / 45; 512 x 512 of 2048 24 / 14.3 / 14.3 / 18 / 15, of 8192 77 / 33 / 33 / 33 / 55;
 // 256 x 1024 of 1024 15.2 / 12.5 / 13.6 / 15.1 / 9.7; 64 x 64 of 32768 283 with one, 44, 33 and 25 with 128, 64 and 32, library 117; 128 x 128 of 700 11.9 / 11.7 (two shares).
 struct Shares { int number, steps; };
@@ -474,7 +478,7 @@ Shares rows_shares(int M, int N, int K)
     const int64_t tiles = (int64_t)((M + (int64_t)GT - 1) / GT) * ((N + (int64_t)GT - 1) / GT);
     const int steps = (K + GK - 1) / GK, units = (steps + UNIT - 1) / UNIT, most = tiles > 128 ? 1 : min((int)(256 / tiles), MOST);
     const int per = (units + most - 1) / most * UNIT;
-    if (K - per * GK < 768) return {1, steps};
+    if (K - per * GK < 1536) return {1, steps};
     return {(steps + per - 1) / per, per};
 }
 
@@ -495,8 +499,10 @@ extern "C" int proteus_gemm_f32(const float* A, const float* B, const float* bia
     return proteus_gemm_f32_ws(A, B, bias, h, C, H, M, N, K, lda, ldb, ldc, form, epilogue, nullptr, 0, stream);
 }
 
-extern "C" int proteus_gemm_f32_ws(const float* A, const float* B, const float* bias, const float* h, void* C, float* H,
-                                   int M, int N, int K, int lda, int ldb, int ldc, int form, int epilogue, void* ws, size_t ws_bytes, void* stream)
+namespace {
+
+int gemm(const float* A, const float* B, const float* bias, const float* h, void* C, float* H, int M, int N, int K, int lda, int ldb, int ldc,
+         int form, int epilogue, void* ws, size_t ws_bytes, PendingSums* sums, void* stream)
 {
     if (!A || !B || !C || (epilogue == PROTEUS_GEMM_GELU && !H) || ((epilogue == PROTEUS_GEMM_GELU_GRAD || epilogue == PROTEUS_GEMM_ADD) && !h)) return PROTEUS_ERR_NULL_POINTER;
     if (form < 0 || form > PROTEUS_GEMM_TN || epilogue < 0 || epilogue > PROTEUS_GEMM_ADD || (form == PROTEUS_GEMM_TN && epilogue != PROTEUS_GEMM_F32)
@@ -533,7 +539,28 @@ extern "C" int proteus_gemm_f32_ws(const float* A, const float* B, const float* 
         GO(true, true, PROTEUS_GEMM_GELU);
         GO(true, true, PROTEUS_GEMM_ADD);
     }
-    else return gemm_go<false, false, PROTEUS_GEMM_F32>(g, st);
+    else return gemm_go<false, false, PROTEUS_GEMM_F32>(g, st, sums);
 #undef GO
     return PROTEUS_ERR_UNSUPPORTED;
+}
+
+}  // namespace
+
+extern "C" int proteus_gemm_f32_ws(const float* A, const float* B, const float* bias, const float* h, void* C, float* H,
+                                   int M, int N, int K, int lda, int ldb, int ldc, int form, int epilogue, void* ws, size_t ws_bytes, void* stream)
+{
+    return gemm(A, B, bias, h, C, H, M, N, K, lda, ldb, ldc, form, epilogue, ws, ws_bytes, nullptr, stream);
+}
+
+int proteus_gemm::gemm_begin(const float* A, const float* B, float* C, int M, int N, int K, int lda, int ldb, int ldc, void* ws, size_t ws_bytes, PendingSums& sums, void* stream)
+{
+    return gemm(A, B, nullptr, nullptr, C, nullptr, M, N, K, lda, ldb, ldc, PROTEUS_GEMM_TN, PROTEUS_GEMM_F32, ws, ws_bytes, sums.count < PendingSums::MOST ? &sums : nullptr, stream);
+}
+
+int proteus_gemm::gemm_sums(PendingSums& sums, void* stream)
+{
+    if (sums.count == 0) return PROTEUS_OK;
+    hipLaunchKernelGGL(gemm_f32_rows_sum_kernel, dim3((unsigned)sums.first[sums.count]), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), sums);
+    sums.count = 0;
+    return (int)hipGetLastError();
 }

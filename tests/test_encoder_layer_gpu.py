@@ -61,6 +61,30 @@ def test_layer_is_as_near_to_float64_as_its_parts(gpu, Z, N, H, dk, hidden, monk
         assert N == 1 or float((p - w).norm()) <= 0.03 * float(w.norm()) + 1e-3 * d.numel() ** 0.5, tuple(w.shape)
 
 
+# Gradients of weights beyond 2^96, which the product sums again from its operands: of the second and of the first linear layer, whose operands' memory the
+# attention's half of the backward takes over, and with enough tokens for shares of them
+@pytest.mark.parametrize("which", ["out_proj", "in_proj"])
+@pytest.mark.parametrize("N", [70, 1500])
+def test_large_gradients_of_weights(gpu, N, which, monkeypatch):
+    layer, x, coords, mask, leaves = _layer(gpu, 2, N, 2, 64, 128)
+    with torch.no_grad():
+        if which == "out_proj":                                       # one hidden unit of 1e10 that nothing reads
+            layer.ffn.in_proj.bias[3], layer.ffn.out_proj.weight[:, 3] = 1e10, 0.0
+        else:                                                         # one feature of 1e10 that the feed-forward does not read
+            layer.attn_norm.bias[3], layer.ffn.in_proj.weight[:, 3] = 1e10, 0.0
+    d = torch.randn_like(x) * (1e20 if which == "out_proj" else 1e30)
+    weight = getattr(layer.ffn, which).weight
+    got, = torch.autograd.grad(layer(x, x, x, coords, mask), [weight], d, retain_graph=False)
+    every = torch.autograd.grad(layer(x, x, x, coords, mask), leaves, d)
+    assert torch.equal(every[[l is weight for l in leaves].index(True)], got)
+    monkeypatch.setattr(train_ops, "encoder_layer", lambda *a: None)
+    want, = torch.autograd.grad(layer(x, x, x, coords, mask), [weight], d)
+    big = want[:, 3]
+    assert float(big.abs().max()) > 2.0 ** 96 and bool(torch.isfinite(want).all())
+    # (operands rounded to bf16 elsewhere in the layer: some 1e-2)
+    assert rel(got[:, 3], big) <= 0.05 and bool(torch.isfinite(got).all())
+
+
 def test_any_subset_of_gradients(gpu):
     layer, x, coords, mask, leaves = _layer(gpu)
     d = torch.randn_like(x)

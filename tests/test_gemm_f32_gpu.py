@@ -33,11 +33,11 @@ def test_product_against_float64(gpu, form, M, N, K):
     assert torch.equal(got, train_ops._product(form, A, B))
 
 
-# Gradients of weights cut along K: a tile in 4 and in 32 shares, few tiles, 64 of them in four shares, the last in a remainder, 128 in two and the first
-# number of tiles that is not cut; below 1024 rows and where a share spares too little nothing is cut
+# Gradients of weights cut along K: a tile in 7 and in 32 shares, few tiles, 64 of them in four shares, the last in a remainder, 128 in two and the first
+# number of tiles that is not cut; nothing is cut where a share spares too little
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K,shares", [(1, 4, 1024, 4), (64, 61, 8195, 17), (64, 64, 49150, 32), (64, 64, 50000, 28), (65, 130, 2050, 9), (512, 512, 2048, 4), (300, 320, 1033, 5), (500, 1000, 1536, 2),
-                                          (513, 1000, 2048, 1), (64, 64, 1000, 1), (500, 1000, 1535, 1)])
+@pytest.mark.parametrize("M,N,K,shares", [(1, 4, 1792, 7), (64, 61, 8195, 17), (64, 64, 49150, 32), (64, 64, 50000, 28), (65, 130, 2050, 9), (512, 512, 2048, 4), (300, 320, 1801, 8), (500, 1000, 3072, 2),
+                                          (513, 1000, 4096, 1), (64, 64, 1791, 1), (500, 1000, 3071, 1)])
 def test_shares(gpu, M, N, K, shares):
     tiles = ((M + 63) // 64) * ((N + 63) // 64)
     assert _lib.load().proteus_gemm_f32_workspace_bytes(M, N, K, TN) == (tiles * shares * 16384 if shares > 1 else 0)
