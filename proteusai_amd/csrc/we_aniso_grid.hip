@@ -470,6 +470,7 @@ void we_aniso_grid_kernel(const char* __restrict__ ws, const float* __restrict__
 
     const WgLayout L = wg_layout(Z, N, K, true);
     const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int z = blockIdx.y;
     const size_t zN = (size_t)z * N;
     const int n = reinterpret_cast<const int*>(ws + L.counts)[z];
@@ -505,7 +506,9 @@ void we_aniso_grid_kernel(const char* __restrict__ ws, const float* __restrict__
 
     // ---- pairs without a cell ----
     __syncthreads();
-    const uint32_t near = (uint32_t)__builtin_amdgcn_ballot_w64(lane < WG_OBS && ok && s_near[obs]);
+    const int at = wg_lane_id(), token = at & 15;
+    const float4 own = src[slot0 + token];
+    const uint32_t near = (uint32_t)__builtin_amdgcn_ballot_w64(at < WG_OBS && slot0 + token < n && s_near[token]);
     if (near == 0) return;
     // They lie within |c A| + h / 2: without a cell r - c A <= h/2 or 2^floor(log2 n) h / r > 2, and 2^floor(log2 n) h <= r - c A + h/2.
     const float closest = (fabsf(mid_cb) * WG_UNIT * params->b_max + 0.5f / inv_h) * 1.001f;
@@ -513,15 +516,15 @@ void we_aniso_grid_kernel(const char* __restrict__ ws, const float* __restrict__
         return wa_no_cell(srcb[j], dx, dy, dz, mid_cb, inv_h, p);
     };
     int lengths;
-    const bool listed = wg_collect<WAVES>(s_grid, s_cnt, near, src, n, me, closest * closest, lengths, find);
+    const bool listed = wg_collect<WAVES>(s_grid, s_cnt, wave, near, src, n, own, closest * closest, lengths, find);
     const int zk = SHARED ? blockIdx.z : 0, Zk = SHARED ? gridDim.z : 1;
-    wg_near_units<WAVES, 2>(near, (L.nkt - zk + Zk - 1) / Zk, listed, [&](auto wide, const int q, const int first) {
+    wg_near_units<WAVES, 2>(wave, near, (L.nkt - zk + Zk - 1) / Zk, listed, [&](auto wide, const int q, const int first) {
         constexpr int U = decltype(wide)::value;
         int k[U];
         float kr[U], cb[U], s[U][GRADS ? 6 : 2];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            k[u] = (zk + (first + 4 * u + (lane >> 4)) * Zk) * 16 + obs;             // a lane per wavenumber, of this workgroup's tiles
+            k[u] = (zk + (first + 4 * u + (at >> 4)) * Zk) * 16 + token;             // a lane per wavenumber, of this workgroup's tiles
             kr[u] = (float)((k[u] < K ? (double)wavenumbers[k[u]] : 0.0) * 0.15915494309189533577);
             cb[u] = k[u] < K ? cb_magnitudes[k[u]] : 0.f;
 #pragma unroll
@@ -542,7 +545,7 @@ void we_aniso_grid_kernel(const char* __restrict__ ws, const float* __restrict__
             }
         };
         if (listed) wg_listed<WAVES>(s_grid, lengths, q, add);
-        else wa_every_near(src, srcb, n, wg_lane(me.x, q), wg_lane(me.y, q), wg_lane(me.z, q), mid_cb, inv_h, lane, add);
+        else wa_every_near(src, srcb, n, wg_lane(own.x, q), wg_lane(own.y, q), wg_lane(own.z, q), mid_cb, inv_h, at, add);
         const size_t row = (zN + s_tok[q]) * 2 * K;
 #pragma unroll
         for (int u = 0; u < U; ++u) {

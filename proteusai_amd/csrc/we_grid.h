@@ -314,6 +314,8 @@ __device__ __forceinline__ float wg_reach(const float4& me, const bool ok, const
 }
 
 // Pairs of a workgroup's observers that no cell takes: a list per wave in the LDS that the grids no longer need.
+// (What follows the grids finds its lane by itself: kept over the windows the thread's index costs the spread a register.)
+__device__ __forceinline__ int wg_lane_id() { return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
 struct WgPair { float r, m, A; int obs; };                     // distance, 1/r, (anisotropic) A; in units of length
 
 // Every wave searches its share of the sources for them, 256 on their way while the 256 before are looked at: only what lies within
@@ -322,11 +324,11 @@ struct WgPair { float r, m, A; int obs; };                     // distance, 1/r,
 // isotropic 1 x 16384 with the sums 476 / 384, 1 x 65536 5348 / 4608, 1 x 8192 anisotropic 249 / 155.)  find(j, dx, dy, dz, pair): does source j's pair have no cell?
 // Returns (to all threads) whether the lists hold all of them, and the lists' lengths to the first lanes; a list is in the order of the sources.
 template <int WAVES, class Find>
-__device__ __forceinline__ bool wg_collect(uint32_t* s_grid, int* s_cnt, const uint32_t near, const float4* __restrict__ src, const int n, const float4& me,
+__device__ __forceinline__ bool wg_collect(uint32_t* s_grid, int* s_cnt, const int wave, const uint32_t near, const float4* __restrict__ src, const int n, const float4& me,
                                            const float reach2, int& lengths, Find find)
 {
     constexpr int CAP = WG_ROWS * WG_OBS * 4 / 16 / WAVES, BATCH = 4;
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = wg_lane_id();
     WgPair* const list = reinterpret_cast<WgPair*>(s_grid) + wave * CAP;
     const int share = (n + WAVES * 64 * BATCH - 1) / (WAVES * 64 * BATCH) * (64 * BATCH);
     const int end = min((wave + 1) * share, n);
@@ -376,7 +378,7 @@ __device__ __forceinline__ void wg_listed(const uint32_t* s_grid, const int leng
         const WgPair* list = reinterpret_cast<const WgPair*>(s_grid) + w * CAP;
         const int count = __builtin_amdgcn_readlane(lengths, w);
         for (int i0 = 0; i0 < count; i0 += 64) {
-            const int lane = threadIdx.x & 63;
+            const int lane = wg_lane_id();
             const WgPair mine = list[min(i0 + lane, count - 1)];
             uint64_t todo = __builtin_amdgcn_ballot_w64(i0 + lane < count && mine.obs == o);
             while (todo) {
@@ -396,9 +398,8 @@ __device__ __forceinline__ void wg_listed(const uint32_t* s_grid, const int leng
 // lists an observer at a time: 30 / 39, 42 / 145, 177 / 941; 1 x 16384 in places of 1000 1380 / 4120.
 template <int U> struct WgWide { static constexpr int value = U; };
 template <int WAVES, int MAX_U, class Sum>
-__device__ __forceinline__ void wg_near_units(const uint32_t near, const int tiles, const bool listed, Sum sum)
+__device__ __forceinline__ void wg_near_units(const int wave, const uint32_t near, const int tiles, const bool listed, Sum sum)
 {
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const bool wide = !listed || __builtin_popcount(near) * ((tiles + 4 * MAX_U - 1) / (4 * MAX_U)) >= WAVES;
     const int step = wide ? 4 * MAX_U : 4;
     int unit = 0;

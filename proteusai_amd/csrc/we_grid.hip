@@ -419,7 +419,9 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
 
     // ---- pairs closer than h / 2 ----
     __syncthreads();
-    const uint32_t near = (uint32_t)__builtin_amdgcn_ballot_w64(lane < WG_OBS && ok && s_near[obs]);
+    const int at = wg_lane_id(), token = at & 15;
+    const float4 own = src[slot0 + token];
+    const uint32_t near = (uint32_t)__builtin_amdgcn_ballot_w64(at < WG_OBS && slot0 + token < n && s_near[token]);
     if (near == 0) return;
     const float closest = 0.5005f / inv_h;
     auto find = [&](int, float dx, float dy, float dz, WgPair& p) {
@@ -429,15 +431,15 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
         return r2 != 0.0f && __builtin_bit_cast(int, __builtin_fmaf(r, inv_h, WG_MAGIC)) == __builtin_bit_cast(int, WG_MAGIC);
     };
     int lengths;
-    const bool listed = wg_collect<WAVES>(s_grid, s_cnt, near, src, n, me, closest * closest, lengths, find);
+    const bool listed = wg_collect<WAVES>(s_grid, s_cnt, wave, near, src, n, own, closest * closest, lengths, find);
     const int zk = blockIdx.z, Zk = gridDim.z;
-    wg_near_units<WAVES, 4>(near, (L.nkt - zk + Zk - 1) / Zk, listed, [&](auto wide, const int q, const int first) {
+    wg_near_units<WAVES, 4>(wave, near, (L.nkt - zk + Zk - 1) / Zk, listed, [&](auto wide, const int q, const int first) {
         constexpr int U = decltype(wide)::value;
         int k[U];
         float kr[U], oc[U], os[U], c[U], s[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            k[u] = (zk + (first + 4 * u + (lane >> 4)) * Zk) * 16 + obs;             // a lane per wavenumber, of this workgroup's tiles
+            k[u] = (zk + (first + 4 * u + (at >> 4)) * Zk) * 16 + token;             // a lane per wavenumber, of this workgroup's tiles
             kr[u] = (float)((k[u] < K ? (double)wavenumbers[k[u]] : 0.0) * 0.15915494309189533577) * (1.0f / WG_UNIT);
             oc[u] = os[u] = c[u] = s[u] = 0.f;
         }
@@ -452,7 +454,7 @@ void we_grid_kernel(const char* __restrict__ ws, const float* __restrict__ waven
             }
         };
         if (listed) wg_listed<WAVES>(s_grid, lengths, q, add);
-        else wg_every_near(src, n, wg_lane(me.x, q), wg_lane(me.y, q), wg_lane(me.z, q), inv_h, lane, add);
+        else wg_every_near(src, n, wg_lane(own.x, q), wg_lane(own.y, q), wg_lane(own.z, q), inv_h, at, add);
         const size_t row = zN + s_tok[q];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
