@@ -21,9 +21,10 @@
 // Few tiles over many tokens leave compute units idle, each of the others a serial chain over K: there workgroups take shares of K (rows_shares), whose
 // sums a second launch adds up in their order.
 //
-// us, 2048 tokens, this / the library's fp32 product: QKV 2048 x 1536 x 512 28.3 / 30.8, its output 10.5 / 11.2; feed-forward 2048 x 2048 x 512 36.2 / 35.3
-// (with GELU's derivative EPILOGUE), 2048 x 512 x 2048 32.4 / 34.0; gradients of weights 512 x 2048 x 2048 and 2048 x 512 x 2048 28.6 / 34.6, 512 x 1536 x 2048 25.4 / 28.9,
-// 512 x 512 x 2048 14.5 / 14.5 (through the first kernel 44, 39, 35, 31); 8192 tokens 97 / 97, 35 / 35, 127 / 125, 129 / 120 and 98 / 121, 84 / 100, 32 / 55.
+// us, 2048 tokens, this / the library's fp32 product: QKV 2048 x 1536 x 512 28 / 31, its output 10.5 / 12; feed-forward 2048 x 2048 x 512 35.5 / 35.3 (with bias and
+// GELU 41, with GELU's derivative 45; the library and torch's elementwise kernels 44 and 45), 2048 x 512 x 2048 32 / 34; gradients of weights 512 x 2048 x 2048 and
+// 2048 x 512 x 2048 29 / 35, 512 x 1536 x 2048 25.4 / 29, 512 x 512 x 2048 14.7 / 14.5 (through the first kernel 44, 39, 35, 31); 8192 tokens 95 / 97, 35 / 35, 125 / 125
+// (149 / 146, 156 / 156), 126 / 119 and 99 / 120, 84 / 99, 32 / 54.
 // Error against float64 at K = 2048 2.5e-7 to 3.5e-7, the library's 8.1e-7.
 //
 // Values that are not finite (or become so: bf16 ends half a step below fp32) do not split; an element of C that comes out not

@@ -194,8 +194,10 @@ def test_saved_tensors_that_come_back_smaller(gpu, whole, monkeypatch):
             torch.autograd.grad(out, leaves, torch.ones_like(out))
 
 
-def test_captured_training_step(gpu):
-    layer, x, coords, mask, leaves = _layer(gpu)
+# (the larger one with shares of the gradients of weights)
+@pytest.mark.parametrize("Z,N,H,dk,hidden", [(2, 70, 2, 32, 100), (2, 1201, 2, 64, 132)])
+def test_captured_training_step(gpu, Z, N, H, dk, hidden):
+    layer, x, coords, mask, leaves = _layer(gpu, Z, N, H, dk, hidden)
     x, d = x.detach(), torch.randn_like(x)
     params = leaves[1:]
 

@@ -118,6 +118,8 @@ def test_a_diverged_operand_is_read_to_its_end(gpu, form, K):
     A = guarded(K, M, 1) if form == TN else guarded(M, K, 1)
     B = guarded(N, K, 2) if form == NT else guarded(K, N, 2)
     clean = train_ops._product(form, A, B)
+    want = (A.double() if form != TN else A.double().t()) @ (B.double() if form != NT else B.double().t())
+    assert bool(((clean - want).abs() <= 28 * 2.0 ** -24 * want).all())                       # (positive terms; as in test_product_against_float64)
     (A if form != TN else A.t())[7, K - 1] = float("inf")
     got = train_ops._product(form, A, B)
     assert bool((got[7] == float("inf")).all())
