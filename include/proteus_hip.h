@@ -64,9 +64,9 @@ extern "C" {
  * header describes; a caller built against it should refuse a library whose proteus_version() differs in
  * major*10000 + minor*100 (argument lists have changed between minors: since 210 the beta-weighted forward and every
  * backward entry point take `int operand_type` before `tuning` / `stream`; a caller built against an older header
- * would pass its tuning selector there).  The Python binding checks for an exact match when it loads the library.
+ * would pass its tuning selector there; since 400 proteus_colsum takes no h and dh, which it lost at 307).  The Python binding checks for an exact match when it loads the library.
  */
-#define PROTEUS_VERSION 307
+#define PROTEUS_VERSION 400
 int proteus_version(void);
 
 /* Human-readable text for a return code of any entry point. */
@@ -573,6 +573,29 @@ int proteus_gemm_f32(const float* A, const float* B, const float* bias, const fl
 size_t proteus_gemm_f32_workspace_bytes(int M, int N, int K, int form);
 int proteus_gemm_f32_ws(const float* A, const float* B, const float* bias, const float* h, void* C, float* H,
                         int M, int N, int K, int lda, int ldb, int ldc, int form, int epilogue, void* ws, size_t ws_bytes, void* stream);
+
+/*
+ * C = act(A B^T + bias) in bf16 for the encoder's inference: operands bf16 with k contiguous (A [M][K], B [N][K], rows lda, ldb elements apart), fp32 sums, C bf16
+ * [M][N], rounded once.  bias [N] bf16 or NULL; gelu: 0 none, else the exact GELU.  N, K, lda, ldb, ldc multiples of 8; A, B, C 16-byte aligned, bias 8.
+ */
+int proteus_gemm_bf16(const uint16_t* A, const uint16_t* B, const uint16_t* bias, uint16_t* C,
+                      int M, int N, int K, int lda, int ldb, int ldc, int gelu, void* stream);
+
+/* out = a + b, a f32, b and out bf16: summed in fp32, rounded once.  n elements, a multiple of 8; 16-byte aligned. */
+int proteus_add_to_bf16(const float* a, const uint16_t* b, uint16_t* out, long n, void* stream);
+
+/*
+ * One post-LN encoder layer's inference in bf16, one call (old/old_scripts/encoder.py:33-41, dropout inactive, the geometric attention branch on the README
+ * logits, exact GELU):  x1 = LN(x + attn(x)), out = LN(x1 + ffn(x1)).
+ *   x, out   [Z*N][d_model] bf16;  coords [Z,N,3] f32;  sigma [H] f32, positive;  mask [Z,N] u8 or NULL (1 = padded)
+ *   params   eleven pointers to bf16: the three projections side by side [3 H d_head][d_model] and their bias [3 H d_head], the output projection
+ *            [d_model][H d_head], gamma and beta of the first LayerNorm [d_model], first [hidden][d_model] and second [d_model][hidden] linear layer's weight and bias
+ *            (weight, bias, weight, bias), gamma and beta of the second LayerNorm; 16-byte aligned
+ *   ws       proteus_encoder_infer_bytes (0: shape not taken), 256-byte aligned
+ */
+size_t proteus_encoder_infer_bytes(int Z, int N, int H, int d_head, int hidden);
+int proteus_encoder_infer(const uint16_t* x, const float* coords, const float* sigma, const uint8_t* mask, const uint16_t* const* params,
+                          float eps1, float eps2, uint16_t* out, void* ws, size_t ws_bytes, int Z, int N, int H, int d_head, int hidden, void* stream);
 
 /*
  * One post-LN encoder layer's training step on the kernels above, a call per direction (old/old_scripts/encoder.py:33-41 with the geometric

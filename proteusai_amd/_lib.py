@@ -14,7 +14,7 @@ LIB_PATH = os.path.join(HERE, "libproteus_hip.so")
 
 COORDS_SOA = 0
 COORDS_AOS = 1
-ABI_VERSION = 307                    # PROTEUS_VERSION of the include/proteus_hip.h these argument lists were written from
+ABI_VERSION = 400                    # PROTEUS_VERSION of the include/proteus_hip.h these argument lists were written from
 OPERAND_BF16, OPERAND_F16 = 0, 1     # PROTEUS_OPERAND_* of include/proteus_hip.h
 GRAD_F32, GRAD_OPERAND = 0, 1        # PROTEUS_GRAD_*
 GEMM_NN, GEMM_NT, GEMM_TN = 0, 1, 2  # PROTEUS_GEMM_*: form
@@ -40,6 +40,7 @@ SYMBOLS = [
     "proteus_add_layernorm_train_fwd", "proteus_layernorm_bwd", "proteus_colsum", "proteus_heads_layout", "proteus_embedding_bwd", "proteus_gemm_f32", "proteus_gemm_f32_workspace_bytes", "proteus_gemm_f32_ws",
     "proteus_encoder_layer_kept_bytes", "proteus_encoder_layer_fwd_bytes",
     "proteus_encoder_layer_bwd_bytes", "proteus_encoder_layer_fwd", "proteus_encoder_layer_bwd",
+    "proteus_gemm_bf16", "proteus_add_to_bf16", "proteus_encoder_infer_bytes", "proteus_encoder_infer",
 ]
 
 _lib = None
@@ -187,6 +188,14 @@ def load():
     lib.proteus_encoder_layer_fwd.argtypes = [vp, vp, vp, vpp, cf, cf, cf, vp, vp, sz, vp, sz, ci, ci, ci, ci, ci, vp]
     lib.proteus_encoder_layer_bwd.restype = ci
     lib.proteus_encoder_layer_bwd.argtypes = [vp, vp, vp, vpp, vp, vp, vpp, cf, vp, sz, vp, sz, ci, ci, ci, ci, ci, vp]
+    lib.proteus_gemm_bf16.restype = ci
+    lib.proteus_gemm_bf16.argtypes = [vp] * 4 + [ci] * 7 + [vp]
+    lib.proteus_add_to_bf16.restype = ci
+    lib.proteus_add_to_bf16.argtypes = [vp, vp, vp, cl, vp]
+    lib.proteus_encoder_infer_bytes.restype = sz
+    lib.proteus_encoder_infer_bytes.argtypes = [ci] * 5
+    lib.proteus_encoder_infer.restype = ci
+    lib.proteus_encoder_infer.argtypes = [vp, vp, vp, vp, vpp, cf, cf, vp, vp, sz, ci, ci, ci, ci, ci, vp]
     _lib = lib
     return lib
 

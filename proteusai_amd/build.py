@@ -14,7 +14,7 @@ INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 LIB = os.path.join(HERE, "libproteus_hip.so")
 SOURCES = ["abi.hip", "we_fwd.hip", "we_grid.hip", "we_dropout_fwd.hip", "we_aniso_fwd.hip", "we_aniso_grid.hip", "we_bwd.hip", "geo_attn_fwd.hip", "geo_attn_fwd_d32.hip", "geo_attn_fwd_d128.hip",
            "geo_attn_bwd.hip", "geo_attn_bwd_d32.hip", "geo_attn_bwd_d128.hip", "geo_attn_delta.hip", "add_layernorm.hip", "encoder_train.hip",
-           "gemm_f32.hip", "encoder_layer.hip"]
+           "gemm_f32.hip", "gemm_bf16.hip", "encoder_layer.hip"]
 PROBE_LIB = os.path.join(HERE, "libproteus_probes.so")
 PROBE_SOURCES = ["probes.hip"]
 

@@ -1,10 +1,11 @@
-// A post-LN encoder layer's training step, one call per direction: the order in which the kernels of the layer are launched
+// A post-LN encoder layer's training step, one call per direction, and its inference in bf16, one call: the order in which the kernels of the layer are launched
 // and where in the two buffers their tensors lie.  Host code: launches cost 2 to 3 us each from here, 6 to 10 from Python and
 // 18 to 29 through torch's products, and a layer has 9 of them forward and 18 to 20 backward, of which most last less than that.
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include "gemm_f32_internal.h"
+#include "geo_attn_internal.h"
 
 namespace {
 
@@ -213,4 +214,65 @@ extern "C" int proteus_encoder_layer_bwd(const float* x, const float* coords, co
     if (projections || biases || g[P_SPREAD] || g[P_WO])
         TRY(proteus_heads_layout(g, b.dW, b.db, b.dWo, b.d_sigma, k.spread, dm, H, d_head, min_spread, 1, stream));
     return PROTEUS_OK;
+}
+
+// ---- inference in bf16 ----
+
+namespace {
+
+enum { I_QKV, I_QKVB, I_WO, I_G1, I_B1, I_W1, I_BIAS1, I_W2, I_BIAS2, I_G2, I_B2, I_PARAMS };
+
+struct Infer {
+    uint16_t *wide, *O, *branch, *x1;                          // wide: Q, K and V, then the feed-forward's hidden layer
+    char* attn;
+    size_t attn_bytes, bytes;
+    Infer(const Sizes& s, void* base)
+    {
+        Carve c{static_cast<char*>(base)};
+        const size_t dm = s.dm, rows = s.rows;
+        wide = c.take<uint16_t>(rows * (s.hidden > 3 * s.dm ? s.hidden : 3 * dm));
+        O = c.take<uint16_t>(rows * dm); branch = c.take<uint16_t>(rows * dm); x1 = c.take<uint16_t>(rows * dm);
+        attn_bytes = proteus_geo_attn_fwd_workspace_bytes(s.Z, s.H, s.N, s.dk, 0);
+        attn = c.take<char>(attn_bytes);
+        bytes = c.at;
+    }
+};
+
+bool infer_ok(const Sizes& s) { return s.ok && s.hidden % 8 == 0 && s.rows < (1L << 31); }
+
+}  // namespace
+
+extern "C" size_t proteus_encoder_infer_bytes(int Z, int N, int H, int d_head, int hidden)
+{
+    const Sizes s(Z, N, H, d_head, hidden);
+    return infer_ok(s) ? Infer(s, nullptr).bytes : 0;
+}
+
+extern "C" int proteus_encoder_infer(const uint16_t* x, const float* coords, const float* sigma, const uint8_t* mask, const uint16_t* const* p,
+                                     float eps1, float eps2, uint16_t* out, void* ws, size_t ws_bytes, int Z, int N, int H, int d_head, int hidden, void* stream)
+{
+    if (!x || !coords || !sigma || !p || !out || !ws) return PROTEUS_ERR_NULL_POINTER;
+    for (int i = 0; i < I_PARAMS; ++i) {
+        if (!p[i]) return PROTEUS_ERR_NULL_POINTER;
+        if (off(p[i], 16)) return PROTEUS_ERR_BAD_ALIGNMENT;
+    }
+    const Sizes s(Z, N, H, d_head, hidden);
+    if (!infer_ok(s)) return PROTEUS_ERR_BAD_SHAPE;
+    if (off(x, 16) || off(out, 16) || off(ws, 256)) return PROTEUS_ERR_BAD_ALIGNMENT;
+    const Infer f(s, ws);
+    if (ws_bytes < f.bytes) return PROTEUS_ERR_BAD_SHAPE;
+    const int rows = (int)s.rows, dm = s.dm;
+    auto product = [&](const uint16_t* A, int w, int b, uint16_t* C, int n, int k, int gelu) {
+        return proteus_gemm_bf16(A, p[w], b < 0 ? nullptr : p[b], C, rows, n, k, k, k, n, gelu, stream);
+    };
+    TRY(product(x, I_QKV, I_QKVB, f.wide, 3 * dm, dm, 0));
+    int64_t st[12];
+    for (int i = 0; i < 3; ++i) head_strides(st + 3 * i, s, 3);
+    head_strides(st + 9, s, 1);
+    TRY(proteus_internal::attn_fwd_bf16_out(f.wide, f.wide + dm, f.wide + 2 * dm, st, coords, sigma, mask, f.O, f.attn_bytes ? f.attn : nullptr, f.attn_bytes, Z, H, N, d_head, stream));
+    TRY(product(f.O, I_WO, -1, f.branch, dm, dm, 0));
+    TRY(proteus_add_layernorm_fwd(x, f.branch, p[I_G1], p[I_B1], f.x1, s.rows, dm, eps1, PROTEUS_DTYPE_BF16, stream));
+    TRY(product(f.x1, I_W1, I_BIAS1, f.wide, hidden, dm, 1));
+    TRY(product(f.wide, I_W2, I_BIAS2, f.branch, dm, hidden, 0));
+    return proteus_add_layernorm_fwd(f.x1, f.branch, p[I_G2], p[I_B2], out, s.rows, dm, eps2, PROTEUS_DTYPE_BF16, stream);
 }

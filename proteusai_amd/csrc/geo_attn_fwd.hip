@@ -166,7 +166,7 @@ __device__ __forceinline__ void gb_merge_parts(const SlotOf& slot_of, const int 
 {
     const int tid = (int)threadIdx.x;
     const int wave = tid >> 6, lane = tid & 63, half = lane >> 5, col = lane & 31;
-    float* Oh = O + (size_t)z * st.o[0] + (size_t)h * st.o[1];
+    const size_t o_at = (size_t)z * st.o[0] + (size_t)h * st.o[1];
     const uint8_t* mz = key_pad ? key_pad + (size_t)z * N : nullptr;
 #pragma unroll 1
     for (int bq = 0; bq < 2; ++bq) {
@@ -209,14 +209,14 @@ __device__ __forceinline__ void gb_merge_parts(const SlotOf& slot_of, const int 
         if (qi < N) {
             const bool row_ok = l > 0.f && !(mz && mz[qi]);
             const float inv_l = row_ok ? 1.0f / l : 0.f;
-            float* orow = Oh + (size_t)qi * (size_t)st.o[2];
+            const size_t orow = o_at + (size_t)qi * (size_t)st.o[2];
 #pragma unroll
             for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
                 for (int gq = 0; gq < 4; ++gq)
-                    *reinterpret_cast<float4*>(orow + dt * 32 + 8 * gq + 4 * half) =
-                        make_float4(acc[dt * 16 + 4 * gq] * inv_l, acc[dt * 16 + 4 * gq + 1] * inv_l,
-                                    acc[dt * 16 + 4 * gq + 2] * inv_l, acc[dt * 16 + 4 * gq + 3] * inv_l);
+                    ga_put(O, orow + dt * 32 + 8 * gq + 4 * half,
+                           make_float4(acc[dt * 16 + 4 * gq] * inv_l, acc[dt * 16 + 4 * gq + 1] * inv_l,
+                                       acc[dt * 16 + 4 * gq + 2] * inv_l, acc[dt * 16 + 4 * gq + 3] * inv_l), st.o16);
             if (L && half == 0) L[(size_t)zh * N + qi] = row_ok ? (M + __log2f(l)) * 0.69314718055994531f : -INFINITY;
         }
     }
@@ -316,12 +316,12 @@ void geo_attn_fwd_balanced_kernel(const uint16_t* __restrict__ Q, const uint16_t
         const int z = e / (H * nqt), rem = e - z * (H * nqt);
         const int h = rem / nqt, qt = rem - h * nqt;
         if (qt * GA_THREADS < bs.n_eff[z]) continue;
-        float* Oh = O + (size_t)z * st.o[0] + (size_t)h * st.o[1];
+        const size_t o_at = (size_t)z * st.o[0] + (size_t)h * st.o[1];
         const int chunk = tid & 15;
         for (int ql = tid >> 4; ql < GA_THREADS; ql += GA_THREADS / 16) {
             const int qi = qt * GA_THREADS + ql;
             if (qi >= N) break;
-            *reinterpret_cast<float4*>(Oh + (size_t)qi * (size_t)st.o[2] + 4 * chunk) = make_float4(0.f, 0.f, 0.f, 0.f);
+            ga_put(O, o_at + (size_t)qi * (size_t)st.o[2] + 4 * chunk, make_float4(0.f, 0.f, 0.f, 0.f), st.o16);
             if (L && chunk == 0) L[((size_t)z * H + h) * N + qi] = -INFINITY;
         }
     }
@@ -476,12 +476,12 @@ void geo_attn_fwd_split_kernel(const uint16_t* __restrict__ Q, const uint16_t* _
         const int z = e / (H * nqt), rem = e - z * (H * nqt);
         const int h = rem / nqt, qt = rem - h * nqt;
         if (qt * GA_THREADS < bs.n_eff[z]) continue;
-        float* Oh = O + (size_t)z * st.o[0] + (size_t)h * st.o[1];
+        const size_t o_at = (size_t)z * st.o[0] + (size_t)h * st.o[1];
         const int chunk = tid & 15;
         for (int ql = tid >> 4; ql < GA_THREADS; ql += GA_THREADS / 16) {
             const int qi = qt * GA_THREADS + ql;
             if (qi >= N) break;
-            *reinterpret_cast<float4*>(Oh + (size_t)qi * (size_t)st.o[2] + 4 * chunk) = make_float4(0.f, 0.f, 0.f, 0.f);
+            ga_put(O, o_at + (size_t)qi * (size_t)st.o[2] + 4 * chunk, make_float4(0.f, 0.f, 0.f, 0.f), st.o16);
             if (L && chunk == 0) L[((size_t)z * H + h) * N + qi] = -INFINITY;
         }
     }
@@ -794,6 +794,21 @@ extern "C" int proteus_geo_attn_fwd_ws(const uint16_t* Q, const uint16_t* K, con
         if (rc != PROTEUS_OK) return rc;
     }
     return launch_attn(false, false, d_head, Q, K, V, coords, sigma, key_pad_mask, O, L, Z, H, N, tuning, nullptr, 0.f, 1.f, gs,
+                       reinterpret_cast<hipStream_t>(stream), workspace, workspace_bytes);
+}
+
+// The forward into a bf16 O and without L, for the encoder's inference: self-attention on a fused projection.
+int proteus_internal::attn_fwd_bf16_out(const uint16_t* Q, const uint16_t* K, const uint16_t* V, const int64_t* strides, const float* coords, const float* sigma,
+                                        const uint8_t* key_pad_mask, uint16_t* O, void* workspace, size_t workspace_bytes, int Z, int H, int N, int d_head, void* stream)
+{
+    float* const out = reinterpret_cast<float*>(O);
+    int rc = proteus_geo_attn_fwd_check(Q, K, V, coords, sigma, key_pad_mask, out, nullptr, Z, H, N, d_head, 0);
+    if (rc != PROTEUS_OK) return rc;
+    GaStrides gs;
+    rc = strides_from(strides, Z, H, N, d_head, gs);
+    if (rc != PROTEUS_OK) return rc;
+    gs.o16 = 1;
+    return launch_attn(false, false, d_head, Q, K, V, coords, sigma, key_pad_mask, out, nullptr, Z, H, N, 0, nullptr, 0.f, 1.f, gs,
                        reinterpret_cast<hipStream_t>(stream), workspace, workspace_bytes);
 }
 

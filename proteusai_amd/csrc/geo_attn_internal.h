@@ -6,8 +6,9 @@
 
 namespace proteus_internal {
 
-// Element strides (batch, head, token) of Q, K, V (16-bit) and O (f32); the head dimension is contiguous.
-struct GaStrides { long q[3], k[3], v[3], o[3]; };
+// Element strides (batch, head, token) of Q, K, V (16-bit) and O; the head dimension is contiguous.  O is f32, or, where o16 is set, bf16,
+// rounded once from the fp32 sums (then the float* of the argument lists points to 16-bit elements).
+struct GaStrides { long q[3], k[3], v[3], o[3]; int o16 = 0; };
 // ... of Q, K, V, dO (16-bit) and dQ, dK, dV (f32, or of the operand type where grads16 is set: then the gradients' pointers,
 // float* in the argument lists, point to 16-bit elements)
 struct GbStrides { long q[3], k[3], v[3], g[3], dq[3], dk[3], dv[3]; int grads16; };
@@ -22,6 +23,9 @@ PROTEUS_HIDDEN int attn_fwd_d32(bool legacy, bool f16, const uint16_t* Q, const 
 PROTEUS_HIDDEN int attn_fwd_d128(bool legacy, bool f16, const uint16_t* Q, const uint16_t* K, const uint16_t* V, const float* coords,
                                  const float* sigma, const uint8_t* key_pad_mask, float* O, float* L, int Z, int H, int N, int tuning,
                                  const float* beta, float min_rbf, float max_rbf, const GaStrides& gs, hipStream_t st);
+
+PROTEUS_HIDDEN int attn_fwd_bf16_out(const uint16_t* Q, const uint16_t* K, const uint16_t* V, const int64_t* strides, const float* coords, const float* sigma,
+                                     const uint8_t* key_pad_mask, uint16_t* O, void* workspace, size_t workspace_bytes, int Z, int H, int N, int d_head, void* stream);
 
 // backward, head dimension 32 / 128
 PROTEUS_HIDDEN int attn_bwd_d32(bool legacy, bool f16, const uint16_t* Q, const uint16_t* K, const uint16_t* V, const uint16_t* dO,

@@ -1,4 +1,4 @@
-"""Encoder stack around the two kernels (inference forward).
+"""Encoder stack around the two kernels.
 
 Follows the legacy transformer architecture the reference's README describes
 (README.md:38,48) and its code:
@@ -14,7 +14,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _lib, train_ops
-from .geometric_attn import GeoAttention
+from .geometric_attn import GeoAttention, _f32, _mask_bytes
 from .wf_embedding import WaveFunctionEmbedding
 
 
@@ -94,6 +94,8 @@ class Encoder(nn.Module):
     def forward(self, q, k, v, coords, mask=None):
         if type(self) is Encoder and q is k and k is v:
             out = train_ops.encoder_layer(q, coords, mask, self, MLP)   # fp32 training
+            if out is None:
+                out = _infer_layer(q, coords, mask, self)               # bf16 inference
             if out is not None:
                 return out
         q = self._residual_norm(q, self.dropout(self.attn(q, k, v, coords, mask=mask)), self.attn_norm)
@@ -104,6 +106,62 @@ class Encoder(nn.Module):
     def _residual_norm(q, branch, norm):
         out = train_ops.add_layer_norm(q, branch, norm)
         return add_layer_norm(q, branch, norm) if out is None else out
+
+
+def _infer_layer(x, coords, mask, m):
+    """The output of the Encoder module `m` (self-attention) on a bf16 x where nothing needs a gradient, all launches of the layer from one call of the
+    library, or None where its parts go their own ways."""
+    if x.dtype != torch.bfloat16 or not x.is_cuda or type(x) is not torch.Tensor or torch.is_autocast_enabled("cuda"):
+        return None
+    a, n1, f, n2 = m.attn, m.attn_norm, m.ffn, m.ffn_norm
+    plain = train_ops.plain_module
+    if not (plain(a, GeoAttention) and plain(n1, nn.LayerNorm) and plain(n2, nn.LayerNorm) and plain(f, MLP) and f.act is F.gelu and not f.hidden_proj
+            and train_ops.inactive_dropout(m.dropout) and train_ops.inactive_dropout(f.in_dropout) and plain(f.in_proj, nn.Linear) and plain(f.out_proj, nn.Linear)
+            and plain(a.out_proj, nn.Linear) and "_residual_norm" not in m.__dict__ and a.out_proj.bias is None):
+        return None
+    H, dk, dm, l1, l2 = a.heads, a.d_k, a.d_model, f.in_proj, f.out_proj
+    rest = (n1.weight, n1.bias, l1.weight, l1.bias, l2.weight, l2.bias, n2.weight, n2.bias)
+    attn = (a.q_proj, a.k_proj, a.v_proj, a.q_bias, a.k_bias, a.v_bias, a.out_proj.weight)
+    if any(type(p) not in train_ops._PLAIN_TYPES or p.dtype != torch.bfloat16 or p.get_device() != x.get_device() for p in rest + attn):
+        return None
+    if torch.is_grad_enabled() and (x.requires_grad or a.spread_weights.requires_grad or any(p.requires_grad for p in rest + attn)):
+        return None
+    hidden = l1.weight.shape[0]
+    w, b = (H, dm, dk), (H, dk)
+    if (tuple(p.shape for p in rest + attn) != ((dm,), (dm,), (hidden, dm), (hidden,), (dm, hidden), (dm,), (dm,), (dm,), w, w, w, b, b, b, (dm, dm))
+            or a.legacy_logits or a.operand_dtype not in (None, torch.bfloat16) or x.dim() != 3 or x.shape[2] != dm or x.numel() == 0
+            or a.spread_weights.shape != (H,) or not (n1.eps >= 0.0 and n2.eps >= 0.0)
+            or tuple(coords.shape) != (*x.shape[:2], 3) or (mask is not None and tuple(mask.shape) != tuple(x.shape[:2]))
+            or not train_ops.unobserved() or not train_ops.aligned(*rest)):
+        return None
+    # Products beyond 512 features: the library's are the faster ones from about 2^33 rows x features^2 on.  Layers in parts / in one call, us: features 512, 8192 tokens
+    # (padded: 210 / 148 a layer), 65536 933 / 886; 768 12288 398 / 383, 32768 846 / 851; 1024 8192 339 / 326, 16384 581 / 625; 2048 2048 277 / 294
+    if dm > 512 and (dm > 1024 or x.shape[0] * x.shape[1] * dm * dm > 2 ** 33):
+        return None
+    sizes = (*x.shape[:2], H, dk, hidden)
+    nbytes = train_ops._bytes("proteus_encoder_infer_bytes", *sizes)
+    if nbytes == 0:
+        return None
+    dev = x.device
+    wqkv, bqkv = a._fused_qkv_rows()
+    params = (wqkv, bqkv, a._out_weight().contiguous(), *rest)
+    x, c, sigma = train_ops._dense(x), _f32(coords, dev), _f32(a._per_head("spread"), dev)
+    pad = None if mask is None else _mask_bytes(mask, dev)
+    out = torch.empty_like(x)
+    train_ops._call("proteus_encoder_infer", dev, x, c, sigma, pad, train_ops._pointers(params), float(n1.eps), float(n2.eps), out,
+                    train_ops._workspace(nbytes, dev), nbytes, *sizes)
+    return out
+
+
+def _add_to_bf16(a, b):
+    """(a + b.to(a.dtype)).to(torch.bfloat16) of an fp32 and a bf16 tensor in one pass, or None where a gradient is needed or the kernel does not take them."""
+    if not (type(a) is type(b) is torch.Tensor and a.is_cuda and a.dtype == torch.float32 and b.dtype == torch.bfloat16 and a.device == b.device
+            and a.shape == b.shape and a.numel() % 8 == 0 and a.numel() > 0 and not (torch.is_grad_enabled() and (a.requires_grad or b.requires_grad))
+            and train_ops.unobserved() and train_ops.aligned(a, b)):
+        return None
+    out = torch.empty_like(b)
+    train_ops._call("proteus_add_to_bf16", a.device, a, b, out, a.numel())
+    return out
 
 
 class ProteusEncoder(nn.Module):
@@ -135,8 +193,10 @@ class ProteusEncoder(nn.Module):
     def forward(self, coords, tokens, key_padding_mask=None):
         wf = self.wf_embedding(coords, None, key_padding_mask=key_padding_mask)           # fp32 [Z,N,d_model]
         aa = train_ops.embedding(tokens, self.aa_embedding)
-        x = wf + (self.aa_embedding(tokens) if aa is None else aa).to(wf.dtype)
-        x = x.to(self.head.weight.dtype)
+        aa = self.aa_embedding(tokens) if aa is None else aa
+        x = _add_to_bf16(wf, aa) if self.head.weight.dtype == torch.bfloat16 else None
+        if x is None:
+            x = (wf + aa.to(wf.dtype)).to(self.head.weight.dtype)
         for layer in self.layers:
             x = layer(x, x, x, coords, mask=key_padding_mask)
         return self.head(x)

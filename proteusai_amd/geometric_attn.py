@@ -507,6 +507,7 @@ class GeoAttention(nn.Module):
         self.__dict__.pop("_head_cache", None)
         self._wo_cache = None
         self._qkv_cache = None
+        self._qkv_rows_cache = None
 
     def train(self, mode: bool = True):
         self.invalidate_caches()
@@ -546,6 +547,19 @@ class GeoAttention(nn.Module):
         w_o = p.view(self.d_model, self.d_k, self.heads).permute(0, 2, 1).reshape(self.d_model, self.d_model)
         self._wo_cache = (key, w_o.detach()) if keep else None
         return w_o
+
+    def _fused_qkv_rows(self):
+        """The same fused projection with a row of d_model per output feature, [3*H*d_k, d_model], as proteus_gemm_bf16 reads it, and its bias."""
+        params = (self.q_proj, self.k_proj, self.v_proj, self.q_bias, self.k_bias, self.v_bias)
+        keep = self._may_keep(params)
+        key = tuple((p._version, p.data_ptr(), p.dtype) for p in params)
+        cache = getattr(self, "_qkv_rows_cache", None)
+        if keep and cache is not None and cache[0] == key:
+            return cache[1], cache[2]
+        w = torch.stack(params[:3]).permute(0, 1, 3, 2).reshape(3 * self.heads * self.d_k, self.d_model)
+        b = torch.stack(params[3:]).reshape(-1)
+        self._qkv_rows_cache = (key, w.detach(), b.detach()) if keep else None
+        return w, b
 
     def _fused_qkv(self):
         """[d_model, 3*H*d_k] weight and [3*H*d_k] bias of the fused self-attention projection, from the per-head

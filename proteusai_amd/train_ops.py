@@ -30,8 +30,13 @@ def recording(*tensors):
         if type(t) not in _PLAIN_TYPES or t.dtype != torch.float32 or t.get_device() != dev or t.layout != torch.strided:
             return False
         needed = needed or t.requires_grad
-    # (a dispatch mode, e.g. make_fx's, sees the torch operators only: a graph traced past a kernel would not hold what it writes)
-    return (needed and torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
+    return needed and unobserved()
+
+
+def unobserved():
+    """Does nothing look on that expects torch operators: no functional transform, forward-mode differentiation, tracing or dispatch mode?
+    (A dispatch mode, e.g. make_fx's, sees the torch operators only: a graph traced past a kernel would not hold what it writes.)"""
+    return (torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
             and torch._C._len_torch_dispatch_stack() == 0 and not torch.jit.is_tracing() and not torch.compiler.is_compiling())
 
 
