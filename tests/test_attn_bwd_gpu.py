@@ -177,6 +177,33 @@ def test_padded_batches_handed_out_longest_first(gpu, H):
     compare(gpu_grads(gpu, *a), reference_grads(*a), mask, "66 items")
 
 
+# Ranked batches against their sequences one by one (which nothing ranks): lengths off 16, whose pieces of 16 mask bytes lie in two sequences, a mask that is read
+# byte by byte, sequences without a token, with one, of equal length and with holes, as many as are ranked, and the first counts of workgroups that are not
+@pytest.mark.parametrize("Z,H,N,off", [(9, 2, 517, 0), (9, 2, 517, 3), (50, 1, 530, 0), (64, 1, 512, 0), (17, 2, 1507, 0), (2, 3, 1500, 0), (5, 8, 500, 0), (16, 8, 513, 0)])
+def test_ranked_batches_equal_their_sequences(gpu, Z, H, N, off):
+    g = torch.Generator(device=gpu).manual_seed(N + Z)
+    Q, K, V = (torch.randn(Z, H, N, 32, generator=g, device=gpu).bfloat16() for _ in range(3))
+    dO = torch.randn(Z, H, N, 32, generator=g, device=gpu)
+    coords = torch.cumsum(torch.randn(Z, N, 3, generator=g, device=gpu) * 2, 1)
+    sigma = torch.full((H,), 6.0, device=gpu)
+    lens = [(0, 1, N, N, N // 2, 15, 16, 17, N - 1)[z % 9] if z < 9 else (z * 97) % (N + 1) for z in range(Z)]
+    mask = torch.empty(Z * N + 16, dtype=torch.bool, device=gpu)[off:off + Z * N].view(Z, N)
+    mask.copy_(torch.arange(N, device=gpu)[None] >= torch.tensor(lens, device=gpu)[:, None])
+    mask[Z - 1, :N // 3] = True
+    one = lambda z: slice(z, z + 1)
+    O, L = pa.geo_attn(Q, K, V, coords, sigma, mask, return_lse=True)
+    from proteusai_amd.geometric_attn import geo_attn_backward as back
+    got = back(Q, K, V, O, L, dO, coords, sigma, mask)
+    d_sigma = torch.zeros(H, device=gpu)
+    for z in range(Z):
+        want = back(Q[one(z)], K[one(z)], V[one(z)], O[one(z)], L[one(z)], dO[one(z)], coords[one(z)], sigma, mask[one(z)].clone())
+        d_sigma += want[3]
+        for a, b in zip(got[:3], want[:3]):
+            # the same pairs and roundings; own tiles of 64 or 128 tokens add up in another order (2^-24 of some N terms)
+            assert bool(((a[z] - b[0]).abs() <= 1e-4 * b.abs().max() + 1e-6).all()), (z, lens[z])
+    assert float((got[3] - d_sigma).abs().max()) <= 1e-3 * float(d_sigma.abs().max()) + 1e-4
+
+
 def test_backward_after_a_forward_that_cut_its_items_into_parts(gpu):
     # N > 2048 and few items: the operator's forward splits every item along the keys (parts merged through a
     # workspace) and hands the backward its O and logsumexp; masked as well (the long items of a padded batch)
