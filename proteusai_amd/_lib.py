@@ -200,6 +200,26 @@ def load():
     return lib
 
 
+_ops = None
+
+
+def ops():
+    """The operators' host path in C++ (csrc/ops.cpp); raise if it has not been built."""
+    global _ops
+    if _ops is None:
+        try:
+            from . import _ops as built
+        except ImportError as e:
+            raise ProteusError(f"proteusai_amd/_ops.so is missing or does not load ({e}): build it with `python -m proteusai_amd.build`") from e
+        if built.version() != ABI_VERSION:
+            raise ProteusError(f"proteusai_amd/_ops.so goes with version {built.version()}, this binding with {ABI_VERSION}: rebuild with `python -m proteusai_amd.build`")
+        from .geometric_attn import _general_backward
+        from .wf_embedding import we_aniso_backward, we_backward
+        built.set_general(_general_backward, we_backward, we_aniso_backward)
+        _ops = built
+    return _ops
+
+
 def check(rc: int, what: str):
     """Turn a return code into an exception: argument errors -> ValueError,
     HIP errors -> ProteusError."""

@@ -310,12 +310,17 @@ class _geometric_attn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dO):
         Q, K, V, O, L, coords, spreads, betas, mask = ctx.saved_tensors
-        op_dtype = ctx.operand_dtype or torch.bfloat16
-        dQ, dK, dV, d_sigma, d_beta = _backward(Q, K, V, O, L, dO, coords, spreads, mask, betas,
-                                                ctx.min_rbf, ctx.max_rbf, ctx.operand_dtype,
-                                                grad_dtype=op_dtype if Q.dtype == K.dtype == V.dtype == op_dtype else None)
-        return (dQ.to(Q.dtype), dK.to(K.dtype), dV.to(V.dtype), None, d_sigma.to(spreads.dtype),
-                None if betas is None else d_beta.to(betas.dtype), None, None, None, None, None, None, None)
+        dQ, dK, dV, d_sigma, d_beta = _general_backward(Q, K, V, O, L, dO, coords, spreads, mask, betas, ctx.min_rbf, ctx.max_rbf,
+                                                        ctx.operand_dtype == torch.float16)
+        return dQ, dK, dV, None, d_sigma, d_beta, None, None, None, None, None, None, None
+
+
+def _general_backward(Q, K, V, O, L, dO, coords, spreads, mask, betas, min_rbf, max_rbf, f16):
+    """Gradients of Q, K, V, spreads and betas (None without), in their types, whatever form the tensors come in."""
+    operand_dtype = torch.float16 if f16 else torch.bfloat16
+    dQ, dK, dV, d_sigma, d_beta = _backward(Q, K, V, O, L, dO, coords, spreads, mask, betas, min_rbf, max_rbf, operand_dtype,
+                                            grad_dtype=operand_dtype if Q.dtype == K.dtype == V.dtype == operand_dtype else None)
+    return dQ.to(Q.dtype), dK.to(K.dtype), dV.to(V.dtype), d_sigma.to(spreads.dtype), None if betas is None else d_beta.to(betas.dtype)
 
 
 def _fused_grad_views_ok(grads):
@@ -394,6 +399,11 @@ def geometric_attn(Q, K, V, coords, spreads, betas=None, mask=None, min_rbf=0.00
     """
     if betas is None and (min_rbf > 0.0 or max_rbf < 1.0):
         raise NotImplementedError("the [min_rbf, max_rbf] pair mask belongs to the beta-weighted logits; pass betas")
+    if out_dtype in (None, torch.float32) and operand_dtype in (None, torch.bfloat16, torch.float16) and geo_attn is _forward:
+        O = _lib.ops().attention(Q, K, V, coords, spreads, betas, mask, float(min_rbf), float(max_rbf), bool(check_spreads), bool(token_major_out),
+                                 operand_dtype is torch.float16)
+        if O is not None:
+            return O
     if not (torch.is_grad_enabled() and (Q.requires_grad or K.requires_grad or V.requires_grad or spreads.requires_grad
                                          or (betas is not None and betas.requires_grad))):
         O = geo_attn(Q, K, V, coords, spreads, mask, betas=betas, min_rbf=min_rbf, max_rbf=max_rbf, check_sigma=check_spreads,
@@ -401,6 +411,9 @@ def geometric_attn(Q, K, V, coords, spreads, betas=None, mask=None, min_rbf=0.00
         return O if out_dtype is None or out_dtype == O.dtype else O.to(out_dtype)
     return _geometric_attn.apply(Q, K, V, coords, spreads, betas, mask, min_rbf, max_rbf, check_spreads,
                                  token_major_out, out_dtype, operand_dtype)
+
+
+_forward = geo_attn         # (where it has been replaced, that is called)
 
 
 class GeoAttention(nn.Module):

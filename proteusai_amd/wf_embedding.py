@@ -176,6 +176,10 @@ class _wf_embedding(torch.autograd.Function):
 def wf_embedding(coords, wavenumbers, magnitude_type=1, dropout_p=0.0, mask=None, rng_seed=None):
     """Same call as the reference's wf_embedding (isotropic/cuda/wf_embedding.py:18); rng_seed (not in the reference,
     which draws one per call) fixes the dropout mask."""
+    if type(magnitude_type) is int and magnitude_type == 1 and type(dropout_p) is float and dropout_p == 0.0 and we_forward is _forwards[0]:
+        out = _lib.ops().embedding(coords, wavenumbers, mask)
+        if out is not None:
+            return out
     return _wf_embedding.apply(coords, wavenumbers, magnitude_type, dropout_p, mask, torch.is_grad_enabled(), rng_seed)
 
 
@@ -261,7 +265,14 @@ class _wf_embedding_learnCB(torch.autograd.Function):
 def wf_embedding_learnCB(coordsA, coordsB, cb_magnitudes, wavenumbers, mask=None):
     """Same call as the reference's anisotropic wf_embedding
     (anisotropic/cb_scaling/learnable_wavenumbers/cuda/wf_embedding.py:16)."""
+    if we_aniso_forward is _forwards[1]:
+        out = _lib.ops().aniso(coordsA, coordsB, cb_magnitudes, wavenumbers, mask)
+        if out is not None:
+            return out
     return _wf_embedding_learnCB.apply(coordsA, coordsB, cb_magnitudes, wavenumbers, mask, torch.is_grad_enabled())
+
+
+_forwards = (we_forward, we_aniso_forward)         # (where one has been replaced, it is called)
 
 
 class WaveFunctionEmbedding(nn.Module):
