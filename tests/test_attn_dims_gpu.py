@@ -108,6 +108,30 @@ def test_forward_legacy_logits(gpu, d, dtype):
     check_forward(O, L, Q, K, V, coords, sigma, mask, betas, 0.0, 1.0, lse_tol, f"legacy d={d} {dtype}")
 
 
+@pytest.mark.parametrize("logits", ["readme", "readme_spread_out", "legacy_range", "legacy"])
+@pytest.mark.parametrize("d,N", [(32, 321), (32, 640), (32, 769), (64, 449), (64, 512), (64, 577), (64, 1025), (128, 513), (128, 544), (128, 768)])
+def test_forward_keys_shared_by_four_waves(gpu, d, N, logits):
+    """Launches of few workgroups: tiles of 128 keys, of which each of four waves takes a block of 32, one sequence whole, one with whole blocks and whole tiles
+    of padded keys (so that a wave's first keys, or all of them, are padded), one with a padded tail.  Coordinates forty times as far apart take the
+    direct distances, in the same workgroups."""
+    dtype = torch.float16 if logits == "legacy_range" else torch.bfloat16
+    Q, K, V, _, coords, sigma, _ = make(900 + N, 3, 2, N, d, dtype)
+    mask = torch.zeros(3, N, dtype=torch.bool)
+    mask[1, :32] = True
+    mask[1, 64:96] = True
+    mask[1, 128:256] = True
+    mask[1, N - 3:N - 1] = True
+    mask[2, N // 2 + 5:] = True
+    if logits == "readme_spread_out":
+        coords = coords * 40.0
+    betas = torch.tensor([0.7, 1.4]) if logits.startswith("legacy") else None
+    lo = 0.001 if logits == "legacy_range" else 0.0
+    opt = dict(operand_dtype=torch.float16) if dtype == torch.float16 else {}
+    O, L = pa.geo_attn(Q.to(gpu), K.to(gpu), V.to(gpu), coords.to(gpu), sigma.to(gpu), mask.to(gpu), return_lse=True,
+                       **({} if betas is None else dict(betas=betas.to(gpu), min_rbf=lo, max_rbf=1.0)), **opt)
+    check_forward(O, L, Q, K, V, coords, sigma, mask, betas, lo, 1.0, LSE_TOL_F16 if dtype == torch.float16 else LSE_TOL_BF16, f"{d} {N} {logits}")
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_large_logits_rebase_within_the_operand_range(gpu, dtype):
     # scores that run up by hundreds along the keys: the lazily re-based exponentials must stay below the largest
