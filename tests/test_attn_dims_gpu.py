@@ -203,6 +203,26 @@ def test_backward_legacy_logits(gpu, d, dtype):
         check_backward(gpu, *a, betas, lo, hi, dtype, 2.0 ** -9, f"legacy d={d} {dtype} [{lo},{hi}]")
 
 
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("d,N,Z,H,dtype,lo", [
+    (128, 100, 1, 2, torch.bfloat16, None), (128, 257, 2, 3, torch.bfloat16, None), (128, 401, 1, 3, torch.bfloat16, None), (128, 513, 2, 3, torch.bfloat16, None),
+    (128, 640, 3, 1, torch.bfloat16, None), (128, 129, 1, 2, torch.float16, 0.0), (128, 260, 2, 2, torch.bfloat16, 0.01), (64, 200, 2, 3, torch.bfloat16, 0.0),
+    (64, 512, 3, 2, torch.float16, 0.0), (64, 769, 1, 3, torch.float16, 0.001), (32, 255, 2, 2, torch.float16, 0.0), (32, 500, 2, 3, torch.bfloat16, 0.0), (32, 897, 1, 2, torch.float16, 0.001)])
+def test_backward_stream_shared_by_four_waves(gpu, d, N, Z, H, dtype, lo, masked):
+    """Launches of few workgroups at d = 128 and with the beta-weighted logits (`lo`): tiles of 128 streamed tokens, of which each of the four waves of an
+    own block takes 32.  Masks: whole blocks and a whole tile of padded tokens, a padded tail (batches from 500 tokens on are handed out by length)."""
+    Q, K, V, dO, coords, sigma, _ = make(950 + N + d, Z, H, N, d, dtype)
+    mask = None
+    if masked:
+        mask = torch.zeros(Z, N, dtype=torch.bool)
+        mask[0, :32] = True
+        mask[0, 64:96] = True
+        mask[0, 128:min(256, N - 30)] = True
+        mask[Z - 1, N - N // 3:] = True
+    betas = None if lo is None else torch.tensor([0.7, 1.3, 0.4])[:H]
+    check_backward(gpu, Q, K, V, dO, coords, sigma, mask, betas, lo or 0.0, 1.0, dtype, 2.0 ** -9, f"d={d} N={N} lo={lo}")
+
+
 def test_the_reference_test_shape_at_its_own_tolerance(gpu):
     """tests/attn/geo_attn.py: batch, nheads, N, d_k = 1, 4, 128, 32; coords = 50 N(0,1) on the line x = y = z;
     spreads 3, betas 1, min_rbf 0, max_rbf 1, no mask; fp32 Q, K, V ~ N(0,1) cast to fp16 by the operator; the dense
