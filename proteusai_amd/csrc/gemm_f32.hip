@@ -9,9 +9,9 @@
 // K by 16; where the tiles are too few to fill the chip, 2 or 4 groups share a tile, each with its own steps and its own LDS stages, and
 // add up at the end in a fixed order (the same bits on every call).  A step: 8 floats per thread travel global -> registers two steps
 // ahead, are split (6.5 vector instructions each) and written to one of two stages as 16-byte fragments, eight consecutive k of one row; the
-// product reads them with ds_read_b128.  Odd groups split and then multiply, even ones the other way round.  What bounds it: a 64 x 64 x 16
-// step reads 24 KB and writes 12 KB of LDS (288 clocks at 128 bytes a clock), and splitting (200 clocks a wave) hardly overlaps with the
-// products (192).  Smaller where it counts than the traffic of operands split beforehand: 6 bytes an element through L2.
+// product reads them with ds_read_b128.  The next step's split is laid between the products (one after the other, odd groups the other way round, 2048 x 512 x 2048
+// 34.2 us and with a matrix added 38.3, so 32.0 and 33.8; 4096 x 512 x 512 20.0 and 18.7, 8192 x 768 x 256 28.3 and 26.1).  What bounds it: a 64 x 64 x 16
+// step reads 24 KB and writes 12 KB of LDS (288 clocks at 128 bytes a clock) beside 192 of products.  Smaller where it counts than the traffic of operands split beforehand: 6 bytes an element through L2.
 //
 // gemm_f32_rows_kernel (rows of A and B across k: gradients of weights): there 32 lanes read 128 consecutive bytes of one k, so a wave loads what
 // its fragments hold straight into registers, no LDS and no barrier: 64 x 64 of C over the wave's share of the steps, the next step split
@@ -63,8 +63,8 @@ constexpr float ENLARGED = 0x1p16f, REDUCED = 0x1p-32f;
 __device__ __forceinline__ float low(const uint32_t w)  { return __builtin_bit_cast(float, w << 16); }
 __device__ __forceinline__ float high(const uint32_t w) { return __builtin_bit_cast(float, w & 0xffff0000u); }
 
-// Four consecutive k of one row into the three pieces' fragments.
-__device__ __forceinline__ void split_to_lds(char* at, const float4& from)
+// Four consecutive k of one row into the three pieces' fragments, `piece` bytes apart.
+__device__ __forceinline__ void split_to_lds(char* at, const float4& from, const int piece = PIECE)
 {
     const float4 v = make_float4(from.x * ENLARGED, from.y * ENLARGED, from.z * ENLARGED, from.w * ENLARGED);
     uint2 p;
@@ -72,9 +72,9 @@ __device__ __forceinline__ void split_to_lds(char* at, const float4& from)
     *reinterpret_cast<uint2*>(at) = p;
     const float a = v.x - low(p.x), b = v.y - high(p.x), c = v.z - low(p.y), d = v.w - high(p.y);
     p.x = pack2(a, b); p.y = pack2(c, d);
-    *reinterpret_cast<uint2*>(at + PIECE) = p;
+    *reinterpret_cast<uint2*>(at + piece) = p;
     p.x = pack2(a - low(p.x), b - high(p.x)); p.y = pack2(c - low(p.y), d - high(p.y));
-    *reinterpret_cast<uint2*>(at + 2 * PIECE) = p;
+    *reinterpret_cast<uint2*>(at + 2 * piece) = p;
 }
 
 // A thread's share of an operand: four consecutive k of one row (of A, or of B^T) per step.  KC: k is the contiguous dimension in memory,
@@ -194,8 +194,16 @@ void gemm_f32_kernel(const GemmArgs g)
         // stage s of this round is written, stage 1 - s (of the round before) is read
         lds_barrier();
         load(round + 2, s);
-        if (group & 1) { store(1 - s); multiply(s); }
-        else           { multiply(s); store(1 - s); }
+        multiply(s);
+        store(1 - s);
+        __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);            // the fragments; then, over and over,
+#pragma unroll
+        for (int i = 0; i < 6; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);        // a product,
+            __builtin_amdgcn_sched_group_barrier(0x002, 10, 0);       // vector instructions of the split,
+            __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);        // a piece to LDS
+        }
+        __builtin_amdgcn_sched_barrier(0);
     };
     for (int r = 0; r < rounds; r += 2) {
         step(r, 0);
@@ -240,6 +248,142 @@ void gemm_f32_kernel(const GemmArgs g)
     for (; again; again &= again - 1) {
         const int e = __builtin_ctz(again), r = 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3), m = m0 + wm + r;
         write<EPI>(g, m, n, (rows_a >> r | cols_b >> (lane & 31)) & 1 ? __builtin_nanf("") : plain_dot<AK, BK>(g, m, n));
+    }
+}
+
+// The same with tiles of 128 x 128, 64 x 64 of them a wave: two thirds of the LDS traffic per product (24 KB read and 12 KB written per 64 x 64 x 16 become 12 and 6) and half of the splitting, which is
+// laid between the products.  G groups of four waves share a tile, each with its own steps and stages.  What bounds it: the products (8192 x 2048 x 512 at 1060 TFLOP/s of bf16,
+// a library product of bf16 reaches 1300), at a tile per compute unit the fill and the epilogue.  Without the order below, split and then products, the odd group the other way
+// round: 2048 x 2048 x 512 31.3 us, so 28.8 (64 x 64 tiles 36.3), 8192 tokens with one group 108 and 97 (128).  Loads four steps ahead: 29.5.
+constexpr int WT       = 128;
+constexpr int WCHUNK   = WT * 16 + 64, WPIECE = 2 * WCHUNK, WOPERAND = 3 * WPIECE, WSTAGE = 2 * WOPERAND;
+template <bool AK, bool BK, int G, int EPI>
+__global__ __launch_bounds__(G * 256, 2)
+void gemm_f32_wide_kernel(const GemmArgs g)
+{
+    extern __shared__ __align__(16) char lds[];               // [G][2 stages]; at the end [2][4 waves][32][64] sums
+    const int tile = (blockIdx.x & 7) * g.per_xcd + (blockIdx.x >> 3);      // consecutive tiles (of the same rows of A) on one XCD
+    if ((int)(blockIdx.x >> 3) >= g.per_xcd || tile >= g.tiles) return;
+    const int m0 = tile / g.tiles_n * WT, n0 = tile % g.tiles_n * WT;
+    const int t = threadIdx.x & 255, lane = t & 63, half = lane >> 5, r0 = lane & 31;
+    const int group = G > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    char* const mine = lds + group * 2 * WSTAGE;
+
+    // what the thread fetches of a step: four k of two rows, 64 apart, of either operand
+    const int ra = AK ? t >> 2 : t & 63, ka = (AK ? t & 3 : t >> 6) * 4;
+    const int rb = BK ? t >> 2 : t & 63, kb = (BK ? t & 3 : t >> 6) * 4;
+    char* const wa = mine + (ka >> 3) * WCHUNK + ra * 16 + (ka & 4) * 2;
+    char* const wb = mine + WOPERAND + (kb >> 3) * WCHUNK + rb * 16 + (kb & 4) * 2;
+    // and the fragments its wave reads
+    const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
+    const char* const fa = mine + half * WCHUNK + (wm + r0) * 16;
+    const char* const fb = mine + WOPERAND + half * WCHUNK + (wn + r0) * 16;
+
+    const int rounds = ((g.K + GK - 1) / GK + 2 * G - 1) / (2 * G) * 2;       // (an even number; steps past the end are zeros)
+    const Source<AK> sa0(g.A, g.lda, m0 + ra, g.M, ka, g.K), sa1(g.A, g.lda, m0 + ra + 64, g.M, ka, g.K);
+    const Source<BK> sb0(g.B, g.ldb, n0 + rb, g.N, kb, g.K), sb1(g.B, g.ldb, n0 + rb + 64, g.N, kb, g.K);
+    float4 va[2][2], vb[2][2];
+    auto load = [&](const int round, const int slot) {
+        const int k = (round * G + group) * GK;
+        va[slot][0] = sa0.fetch(k); va[slot][1] = sa1.fetch(k);
+        vb[slot][0] = sb0.fetch(k); vb[slot][1] = sb1.fetch(k);
+    };
+    auto store = [&](const int slot) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            split_to_lds(wa + slot * WSTAGE + i * 64 * 16, va[slot][i], WPIECE);
+            split_to_lds(wb + slot * WSTAGE + i * 64 * 16, vb[slot][i], WPIECE);
+        }
+    };
+    f32x16 acc[2][2] = {};
+    auto multiply = [&](const int slot) {
+        bf16x8 a[2][3], b[2][3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                a[i][p] = *reinterpret_cast<const bf16x8*>(fa + slot * WSTAGE + p * WPIECE + i * 32 * 16);
+                b[i][p] = *reinterpret_cast<const bf16x8*>(fb + slot * WSTAGE + p * WPIECE + i * 32 * 16);
+            }
+        constexpr int P[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};
+#pragma unroll
+        for (int p = 0; p < 6; ++p)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][P[p][0]], b[j][P[p][1]], acc[i][j], 0, 0, 0);
+    };
+    load(0, 0);
+    load(1, 1);
+    store(0);
+    auto step = [&](const int round, const int s) {
+        // stage s of this round is written, stage 1 - s (of the round before) is read
+        lds_barrier();
+        load(round + 2, s);
+        multiply(s);
+        store(1 - s);
+        __builtin_amdgcn_sched_group_barrier(0x100, 12, 0);           // the fragments; then, over and over,
+#pragma unroll
+        for (int i = 0; i < 12; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);        // a product,
+            __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);        // vector instructions of the split,
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+            __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);        // and every second time a piece to LDS
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    for (int r = 0; r < rounds; r += 2) {
+        step(r, 0);
+        step(r + 1, 1);
+    }
+
+    // ---- the groups' sums together: group i takes the i-th 32 rows of every wave's 64, and hands on the others ----
+    if constexpr (G == 2) {
+        float* const red = reinterpret_cast<float*>(lds);
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) red[((group * 4 + wave) * 32 + j * 16 + e) * 64 + lane] = group ? acc[0][j][e] : acc[1][j][e];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const float other = red[(((1 - group) * 4 + wave) * 32 + j * 16 + e) * 64 + lane];
+                acc[0][j][e] = (group ? acc[1][j][e] : acc[0][j][e]) + other;
+            }
+    }
+#pragma unroll
+    for (int i = 0; i < 2 / G; ++i) {
+        const int mw = m0 + wm + 32 * (G == 2 ? group : i);
+        uint32_t again = 0;                                    // of the lane's 32 elements those that are not finite
+#pragma unroll
+        for (int e = 0; e < 32; ++e) {
+            const float v = acc[i][e >> 4][e & 15];
+            const int m = mw + 8 * ((e >> 2) & 3) + 4 * half + (e & 3), n = n0 + wn + 32 * (e >> 4) + r0;
+            if (m >= g.M || n >= g.N) continue;
+            if (fabsf(v) <= 3.4028234e38f) write<EPI>(g, m, n, v * REDUCED);
+            else again |= 1u << e;
+        }
+        if (__builtin_amdgcn_ballot_w64(again != 0) == 0) continue;
+        // (as above)
+        const int k0 = half ? g.K / 2 : 0, k1 = half ? g.K : g.K / 2;
+        const uint64_t in_a = __builtin_amdgcn_ballot_w64(any_nan<AK>(g.A, g.lda, mw + r0, g.M, k0, k1));
+        const uint32_t rows_a = (uint32_t)in_a | (uint32_t)(in_a >> 32);
+        uint32_t cols_b[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const uint64_t in_b = __builtin_amdgcn_ballot_w64(any_nan<BK>(g.B, g.ldb, n0 + wn + 32 * j + r0, g.N, k0, k1));
+            cols_b[j] = (uint32_t)in_b | (uint32_t)(in_b >> 32);
+        }
+        for (; again; again &= again - 1) {
+            const int e = __builtin_ctz(again), r = 8 * ((e >> 2) & 3) + 4 * half + (e & 3), n = n0 + wn + 32 * (e >> 4) + r0;
+            const bool nan = (rows_a >> r | (e >> 4 ? cols_b[1] : cols_b[0]) >> r0) & 1;
+            write<EPI>(g, mw + r, n, nan ? __builtin_nanf("") : plain_dot<AK, BK>(g, mw + r, n));
+        }
     }
 }
 
@@ -425,6 +569,21 @@ void gemm_f32_rows_sum_kernel(const PendingSums sums)
     finish_rows<4>(g, m0, n0, e0, v);
 }
 
+// Groups of gemm_f32_wide_kernel, 0: tiles of 64 x 64.  Two while its tiles leave a compute unit one each and few idle, one (three workgroups of which share a compute
+// unit) from where their rounds are full enough; not for a short K, and later where the epilogue is long, since nothing runs under that of a lone workgroup.  Us, 64 x 64 / 128 x 128
+// with two groups, M x N x K: 2048 x 2048 x 512 (256 tiles) with bias and GELU 41.3 / 36.0, with GELU's derivative 45.1 / 41.8; 2048 x 1536 x 512 (192) 28.0 / 25.7; 1536 x 1536 x 512 (144) 26.4 / 25.0;
+// 1536 x 2048 x 512 (192) 33.3 / 32.6 and 36.7 / 39.2 (the 64 x 64 ones before their steps were laid out: a twentieth slower than now); 5000 x 512 x 2048 (160) 91 / 74; 8192 x 512 x 2048 (256) 127 / 92, x 512 36.1 / 30.6, x 256 25.8 / 25.0; 4096 x 512 x 2048 (128) 63 / 71;
+// 2048 x 1024 x 1024 (128) 34 / 41; 4096 x 768 x 256 (192) 15.9 / 16.6.  With one group: 3072 x 1536 x 512 (288 tiles) 41 / 48, 4096 x 1536 (384) 51.0 / 50.2, 5000 x 1536 (480) 64 / 53, 4096 x 2048
+// (512) 77 / 69 and 80.2 / 80.7, 5000 x 2048 (640) 93 / 88 and 96 / 99, 6144 x 2048 (768) 108 / 92 and 115 / 105, 8192 x 2048 (1024) 146 / 120 and 156 / 146, 8192 x 1536 (768) 96 / 75,
+// 16384 x 1024 x 1024 244 / 184; 16384 x 512 x 256 (512) 44.1 / 45.5, 32768 x 512 x 128 (1024) 53 / 63.
+int wide_groups(int M, int N, int K, int epilogue)
+{
+    if (K < 512) return 0;
+    const int64_t tiles = ((M + (int64_t)WT - 1) / WT) * ((N + (int64_t)WT - 1) / WT);
+    if (tiles > 256) return tiles >= (epilogue == PROTEUS_GEMM_GELU_GRAD ? 704 : 448) ? 1 : 0;
+    return tiles >= (epilogue == PROTEUS_GEMM_GELU_GRAD || epilogue == PROTEUS_GEMM_GELU ? 240 : 160) ? 2 : 0;
+}
+
 template <bool AK, bool BK, int EPI>
 int gemm_go(GemmArgs g, hipStream_t st, PendingSums* sums = nullptr)
 {
@@ -458,6 +617,19 @@ int gemm_go(GemmArgs g, hipStream_t st, PendingSums* sums = nullptr)
             constexpr size_t sums = (G_) > 1 ? (size_t)(G_) * 4 * 16 * 64 * 4 : 0; \
             hipLaunchKernelGGL((gemm_f32_kernel<AK, BK, G_, EPI>), grid, dim3(G_ * 256), G_ * 2 * STAGE > sums ? G_ * 2 * STAGE : sums, st, g); \
         } while (0)
+        if (const int groups = wide_groups(g.M, g.N, g.K, EPI)) {
+            g.tiles_n = (g.N + WT - 1) / WT;
+            g.tiles   = (g.M + WT - 1) / WT * g.tiles_n;
+            g.per_xcd = (g.tiles + 7) / 8;
+            auto kern = groups == 2 ? gemm_f32_wide_kernel<AK, BK, 2, EPI> : gemm_f32_wide_kernel<AK, BK, 1, EPI>;
+            const size_t bytes = (size_t)groups * 2 * WSTAGE;
+            if (bytes > 64 * 1024) {      // (per device, cheap: set on every call)
+                const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+                if (attr != hipSuccess) return (int)attr;
+            }
+            hipLaunchKernelGGL(kern, dim3((unsigned)g.per_xcd * 8), dim3(groups * 256), bytes, st, g);
+            return (int)hipGetLastError();
+        }
         if (g.tiles > 512)      GO(1);
         else if (g.tiles > 256) GO(2);
         else                    GO(4);

@@ -33,6 +33,22 @@ def test_product_against_float64(gpu, form, M, N, K):
     assert torch.equal(got, train_ops._product(form, A, B))
 
 
+# Tiles of 128 x 128: from 160 of them and K = 512 on with two groups, from 448 on with one; edges of the tiles and of the steps that the groups share out
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", [NN, NT])
+@pytest.mark.parametrize("M,N,K", [(1920, 1280, 512), (2047, 1276, 516), (1921, 1284, 532), (129, 10244, 548), (20481, 4, 512), (2945, 2436, 512), (2817, 2492, 540)])
+def test_wide_tiles_against_float64(gpu, form, M, N, K):
+    A, B, want, mass = _operands(form, M, N, K, gpu)
+    got = train_ops._product(form, A, B)
+    # (as above)
+    assert bool(((got - want).abs() <= (12 * ((K + 15) // 16) + 16) * 2.0 ** -24 * mass).all())
+    assert torch.equal(got, train_ops._product(form, A, B))
+    # ... and not further off than sixty-four columns at a time, which tiles of 64 x 64 do
+    narrow = torch.cat([train_ops._product(form, A, (B[n:n + 64] if form == NT else B[:, n:n + 64]).contiguous()) for n in range(0, min(N, 256), 64)], 1)
+    near, far = (got[:, :256] - want[:, :256]).norm(), (narrow - want[:, :256]).norm()
+    assert float(near) <= 2.0 * float(far)          # (two chains over K for four: rounding errors that add up as sqrt(2), and some room)
+
+
 # Gradients of weights cut along K: a tile in 7 and in 32 shares, few tiles, 64 of them in four shares, the last in a remainder, 128 in two and the first
 # number of tiles that is not cut; nothing is cut where a share spares too little
 @pytest.mark.gpu
@@ -93,6 +109,32 @@ def test_epilogues(gpu, M):
     assert torch.equal(_epilogue(NT, _lib.GEMM_ADD, A, B, bias, h), train_ops._product(NT, A, B, bias) + h)
 
 
+# (tiles of 128 x 128, with two groups and with one)
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N", [(2049, 1804), (3457, 3204)])
+def test_epilogues_of_wide_tiles(gpu, M, N):
+    A, B, want, mass = _operands(NT, M, N, 524, gpu)
+    Bt, bias, h = B.t().contiguous(), torch.randn(N, device=gpu), torch.randn(M, N, device=gpu)
+    bound = (12 * 33 + 16) * 2.0 ** -24 * mass + 2.0 ** -23 * bias.abs()
+    H, C = train_ops._product(NT, A, B, bias, gelu=True)
+    assert bool(((H - want - bias).abs() <= bound).all())
+    assert bool(((C - torch.nn.functional.gelu(H.double())).abs() <= 2.0 ** -21 * H.abs()).all())
+    hd = h.double().requires_grad_(True)
+    grad, = torch.autograd.grad(torch.nn.functional.gelu(hd).sum(), hd)
+    plain = train_ops._product(NN, A, Bt, bias)
+    assert bool(((plain - want - bias).abs() <= bound).all())
+    assert bool(((train_ops._product(NN, A, Bt, bias, gelu_grad_of=h) - plain.double() * grad).abs() <= 2.0 ** -20 * plain.abs() * (1 + h.abs())).all())
+    assert torch.equal(_epilogue(NN, _lib.GEMM_BF16, A, Bt, bias), plain.to(torch.bfloat16))
+    assert torch.equal(_epilogue(NN, _lib.GEMM_ADD, A, Bt, None, h), train_ops._product(NN, A, Bt) + h)
+    assert torch.equal(_epilogue(NT, _lib.GEMM_ADD, A, B, bias, h), train_ops._product(NT, A, B, bias) + h)
+    A[M - 1, 523] = float("nan")
+    B[N - 1, 0] = float("nan")
+    hit = torch.zeros_like(plain, dtype=torch.bool)
+    hit[M - 1], hit[:, N - 1] = True, True
+    got, clean = train_ops._product(NT, A, B), train_ops._product(NN, A, Bt)
+    assert torch.equal(got.isnan(), hit) and bool(((got - want).abs()[~hit] <= bound[~hit]).all()) and torch.equal(clean[:M - 1].isnan(), torch.zeros_like(hit[:M - 1]))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("form,K", [(NN, 68), (NT, 68), (TN, 68), (TN, 2100)])
 def test_a_diverged_operand(gpu, form, K):
@@ -129,7 +171,7 @@ def test_a_diverged_operand_is_read_to_its_end(gpu, form, K):
 
 # (gradients of weights: 8, 4 and 2 waves per tile, and shares of K)
 @pytest.mark.gpu
-@pytest.mark.parametrize("form,M,N,K", [(NN, 70, 68, 36), (NT, 70, 68, 36), (NN, 1700, 1600, 36), (NT, 1100, 1200, 36), (TN, 70, 68, 36), (TN, 70, 68, 2100), (TN, 1100, 1000, 37), (TN, 2000, 1800, 38)])
+@pytest.mark.parametrize("form,M,N,K", [(NN, 70, 68, 36), (NT, 70, 68, 36), (NN, 1700, 1600, 36), (NT, 1100, 1200, 36), (NN, 2047, 1276, 516), (NT, 2945, 2436, 512), (TN, 70, 68, 36), (TN, 70, 68, 2100), (TN, 1100, 1000, 37), (TN, 2000, 1800, 38)])
 def test_values_that_do_not_split(gpu, form, M, N, K):
     A, B, _, _ = _operands(NN, M, N, K, gpu)
     bad = [(3, 5, float("inf")), (7, 1, float("nan")), (9, 2, 3.4e38), (11, 3, -3.39e38)]      # (bf16 ends at 3.39e38)
