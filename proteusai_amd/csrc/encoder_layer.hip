@@ -68,9 +68,9 @@ struct Forward {
 };
 
 struct Backward {
-    float *dy2, *dh, *dx1, *dy1, *dO, *D, *g, *d_sigma, *dW, *db, *dWo, *ln;
+    float *dy2, *dh, *dx1, *dy1, *dO, *D, *g, *d_sigma, *dW, *db, *dWo;
     uint16_t* dO16;
-    void *lnws, *sums, *shares[4];                                               // of the gradients of weights: W2, W1, output projection, projections
+    void *lnws[2], *sums, *shares[4];                                               // of the gradients of weights: W2, W1, output projection, projections
     size_t ln_bytes, sums_bytes, shares_bytes[4], bytes;
     Backward(const Sizes& s, void* base)
     {
@@ -82,9 +82,9 @@ struct Backward {
         dy2 = dO = c.take<float>(rows * dm);
         dx1 = c.take<float>(rows * dm); dO16 = reinterpret_cast<uint16_t*>(dx1);
         dy1 = c.take<float>(rows * dm); D = c.take<float>(rows * s.H); d_sigma = c.take<float>(s.H);
-        dW = c.take<float>(3 * dm * dm); db = c.take<float>(3 * dm); dWo = c.take<float>(dm * dm); ln = c.take<float>(2 * dm);
+        dW = c.take<float>(3 * dm * dm); db = c.take<float>(3 * dm); dWo = c.take<float>(dm * dm);
         ln_bytes = proteus_layernorm_bwd_workspace_bytes(s.rows, s.dm);
-        lnws = c.take<char>(ln_bytes);
+        lnws[0] = c.take<char>(ln_bytes); lnws[1] = c.take<char>(ln_bytes);
         sums_bytes = proteus_train_workspace_bytes(s.rows, s.hidden > 3 * s.dm ? s.hidden : 3 * s.dm);
         sums = c.take<char>(sums_bytes);
         const int sizes[4][2] = {{s.dm, s.hidden}, {s.hidden, s.dm}, {s.dm, s.dm}, {s.dm, 3 * s.dm}};
@@ -173,20 +173,26 @@ extern "C" int proteus_encoder_layer_bwd(const float* x, const float* coords, co
     auto product = [&](const float* A, const float* B, const float* h, float* C, int m, int n, int kk, int lda, int ldb, int form, int epilogue) {
         return proteus_gemm_f32(A, B, nullptr, h, C, nullptr, m, n, kk, lda, ldb, n, form, epilogue, stream);
     };
-    // (The shares of several in one launch, which must come before their operands are written over: it sums what is not finite again.)
+    // (The shares of several products, the last sums of the LayerNorms and the biases' in one launch, which must come before what they are of is written over.  Each of the
+    // sums in a launch of its own, five per layer, took 5.3 us.)
     proteus_gemm::PendingSums pending;
     auto gradient = [&](const float* A, const float* B, float* C, int m, int n, int which) {
         return proteus_gemm::gemm_begin(A, B, C, m, n, rows, m, n, n, b.shares_bytes[which] ? b.shares[which] : nullptr, b.shares_bytes[which], pending, stream);
     };
-    auto column_sums = [&](const float* a, float* out, int C) { return proteus_colsum(a, out, b.sums, b.sums_bytes, s.rows, C, stream); };
-    auto layernorm = [&](const float* d, const float* y, const float* stat, const float* gamma, float* dy, float* dgamma_dbeta) {
-        return proteus_layernorm_bwd(d, y, stat, gamma, dy, dgamma_dbeta ? dgamma_dbeta : b.ln, b.lnws, b.ln_bytes, s.rows, dm, stream);
+    auto column_sums = [&](const float* a, float* out, int C) {
+        return pending.add({a, out, rows, C}) ? (int)PROTEUS_OK : proteus_colsum(a, out, b.sums, b.sums_bytes, s.rows, C, stream);
+    };
+    auto layernorm = [&](const float* d, const float* y, const float* stat, const float* gamma, float* dy, float* dgamma_dbeta, int which) {
+        proteus_train::ColumnSums sums;
+        const int rc = proteus_train::layernorm_bwd_begin(d, y, stat, gamma, dy, dgamma_dbeta, b.lnws[which], b.ln_bytes, s.rows, dm, sums, stream);
+        if (rc != PROTEUS_OK || !dgamma_dbeta || pending.add(sums)) return rc;
+        return proteus_colsum(sums.a, sums.out, nullptr, 0, sums.rows, sums.cols, stream);
     };
     const bool projections = g[P_QW] || g[P_KW] || g[P_VW], biases = g[P_QB] || g[P_KB] || g[P_VB];
     const bool attention = dx || projections || biases || g[P_SPREAD];
     const bool first_norm = attention || g[P_WO] || g[P_G1];
 
-    TRY(layernorm(dout, k.y2, k.stat2, p[P_G2], b.dy2, g[P_G2]));
+    TRY(layernorm(dout, k.y2, k.stat2, p[P_G2], b.dy2, g[P_G2], 1));
     if (g[P_W2])    TRY(gradient(b.dy2, k.a, g[P_W2], dm, hidden, 0));
     if (g[P_BIAS2]) TRY(column_sums(b.dy2, g[P_BIAS2], dm));
     if (!(first_norm || g[P_W1] || g[P_BIAS1])) return proteus_gemm::gemm_sums(pending, stream);
@@ -195,7 +201,7 @@ extern "C" int proteus_encoder_layer_bwd(const float* x, const float* coords, co
     if (g[P_BIAS1]) TRY(column_sums(b.dh, g[P_BIAS1], hidden));
     if (!first_norm) return proteus_gemm::gemm_sums(pending, stream);
     TRY(product(b.dh, p[P_W1], b.dy2, b.dx1, rows, dm, hidden, hidden, dm, PROTEUS_GEMM_NN, PROTEUS_GEMM_ADD));
-    TRY(layernorm(b.dx1, k.y1, k.stat1, p[P_G1], b.dy1, g[P_G1]));
+    TRY(layernorm(b.dx1, k.y1, k.stat1, p[P_G1], b.dy1, g[P_G1], 0));
     if (g[P_WO]) TRY(gradient(b.dy1, k.O, b.dWo, dm, dm, 2));
     if (attention) {
         TRY(proteus_gemm::gemm_sums(pending, stream));                          // dO takes dy2's place, g dh's

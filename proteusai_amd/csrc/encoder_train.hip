@@ -14,14 +14,13 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include "proteus_hip.h"
+#include "train_internal.h"
 
 namespace {
 
 constexpr int LN_WAVES  = 4;
 constexpr int LN_MAX_D  = 2048;
-constexpr int CS_COLS   = 16;           // columns of a column-sum workgroup: 64 bytes of a row
-constexpr int CS_BLOCK  = 512;          // 4 threads of 16 bytes x 128 rows
-constexpr int CS_ROWS   = 2048;         // rows a column-sum workgroup takes before the rows are cut into slabs
+using namespace proteus_train;
 constexpr int EB_TOKENS = 128;          // tokens of an embedding-gradient workgroup
 constexpr int EB_MAX_V  = 64;
 
@@ -155,37 +154,13 @@ void layernorm_bwd_kernel(const float* __restrict__ dout, const float* __restric
     for (int i = threadIdx.x; i < D; i += LN_WAVES * 64) { p[i] = red[0][i]; p[D + i] = red[1][i]; }
 }
 
-// sums[slab][c] = sum over the slab's rows of a[row][c].  torch's reduction 10.8 - 14.1 us with a clearing launch in front, this 5.6 - 6.3 (2048 columns).
+// sums[slab][c] = sum over the slab's rows of a[row][c].
 __global__ __launch_bounds__(CS_BLOCK)
 void colsum_kernel(const float* __restrict__ a, float* __restrict__ sums, const long rows, const int C, const long slab_rows)
 {
     __shared__ float red[CS_BLOCK / 64][CS_COLS];
-    const int q = threadIdx.x & 3, r = threadIdx.x >> 2;
-    const int col = blockIdx.x * CS_COLS + q * 4;
     const long r0 = (long)blockIdx.y * slab_rows, r1 = r0 + slab_rows < rows ? r0 + slab_rows : rows;
-    float s[4] = {0.f, 0.f, 0.f, 0.f};
-    if (col < C) {
-#pragma unroll 4
-        for (long row = r0 + r; row < r1; row += CS_BLOCK / 4) {
-            const float4 v = *reinterpret_cast<const float4*>(a + (size_t)row * C + col);
-            s[0] += v.x; s[1] += v.y; s[2] += v.z; s[3] += v.w;
-        }
-    }
-#pragma unroll
-    for (int o = 4; o < 64; o <<= 1)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) s[e] += __shfl_xor(s[e], o);
-    if ((threadIdx.x & 63) < 4)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) red[threadIdx.x >> 6][q * 4 + e] = s[e];
-    __syncthreads();
-    const int c = blockIdx.x * CS_COLS + threadIdx.x;
-    if (threadIdx.x < CS_COLS && c < C) {
-        float t = 0.f;
-#pragma unroll
-        for (int w = 0; w < CS_BLOCK / 64; ++w) t += red[w][threadIdx.x];
-        sums[(size_t)blockIdx.y * C + c] = t;
-    }
+    column_sums(a, sums + (size_t)blockIdx.y * C, r0, r1, C, blockIdx.x, red);
 }
 
 int colsum(const float* a, float* out, float* ws, long rows, int C, hipStream_t st) {
@@ -327,10 +302,10 @@ extern "C" int proteus_add_layernorm_train_fwd(const float* x, const float* res,
     return (int)hipGetLastError();
 }
 
-extern "C" int proteus_layernorm_bwd(const float* dout, const float* ysum, const float* stat, const float* gamma, float* dx,
-                                     float* dgamma_dbeta, void* ws, size_t ws_bytes, long rows, int D, void* stream)
+int proteus_train::layernorm_bwd_begin(const float* dout, const float* ysum, const float* stat, const float* gamma, float* dx, float* dgamma_dbeta, void* ws, size_t ws_bytes,
+                                       long rows, int D, ColumnSums& sums, void* stream)
 {
-    if (!dout || !ysum || !stat || !gamma || !dx || !dgamma_dbeta || !ws) return PROTEUS_ERR_NULL_POINTER;
+    if (!dout || !ysum || !stat || !gamma || !dx || !ws) return PROTEUS_ERR_NULL_POINTER;
     if (rows <= 0 || D <= 0 || D % 4 || D > LN_MAX_D || ws_bytes < proteus_layernorm_bwd_workspace_bytes(rows, D)) return PROTEUS_ERR_BAD_SHAPE;
     if (misaligned(dout) || misaligned(ysum) || misaligned(stat) || misaligned(gamma) || misaligned(dx) || misaligned(dgamma_dbeta) || misaligned(ws))
         return PROTEUS_ERR_BAD_ALIGNMENT;
@@ -345,7 +320,18 @@ extern "C" int proteus_layernorm_bwd(const float* dout, const float* ysum, const
         default: LN_GO(8); break;
     }
 #undef LN_GO
-    return colsum((const float*)ws, dgamma_dbeta, nullptr, groups, 2 * D, st);      // (at most CS_ROWS groups)
+    sums = {(const float*)ws, dgamma_dbeta, groups, 2 * D};      // (at most CS_ROWS groups)
+    return (int)hipGetLastError();
+}
+
+extern "C" int proteus_layernorm_bwd(const float* dout, const float* ysum, const float* stat, const float* gamma, float* dx,
+                                     float* dgamma_dbeta, void* ws, size_t ws_bytes, long rows, int D, void* stream)
+{
+    if (!dgamma_dbeta) return PROTEUS_ERR_NULL_POINTER;
+    ColumnSums sums;
+    const int rc = layernorm_bwd_begin(dout, ysum, stat, gamma, dx, dgamma_dbeta, ws, ws_bytes, rows, D, sums, stream);
+    if (rc != PROTEUS_OK) return rc;
+    return colsum(sums.a, sums.out, nullptr, sums.rows, sums.cols, reinterpret_cast<hipStream_t>(stream));
 }
 
 extern "C" int proteus_colsum(const float* a, float* sums, void* ws, size_t ws_bytes, long rows, int C, void* stream)

@@ -21,10 +21,10 @@
 // Few tiles over many tokens leave compute units idle, each of the others a serial chain over K: there workgroups take shares of K (rows_shares), whose
 // sums a second launch adds up in their order.
 //
-// us, 2048 tokens, this / the library's fp32 product: QKV 2048 x 1536 x 512 28 / 31, its output 10.5 / 12; feed-forward 2048 x 2048 x 512 35.5 / 35.3 (with bias and
-// GELU 41, with GELU's derivative 45; the library and torch's elementwise kernels 44 and 45), 2048 x 512 x 2048 32 / 34; gradients of weights 512 x 2048 x 2048 and
-// 2048 x 512 x 2048 29 / 35, 512 x 1536 x 2048 25.4 / 29, 512 x 512 x 2048 14.7 / 14.5 (through the first kernel 44, 39, 35, 31); 8192 tokens 95 / 97, 35 / 35, 125 / 125
-// (149 / 146, 156 / 156), 126 / 119 and 99 / 120, 84 / 99, 32 / 54.
+// us, 2048 tokens, this / the library's fp32 product: QKV 2048 x 1536 x 512 25 / 31, its output 10.5 / 12; feed-forward 2048 x 2048 x 512 27 / 35 (with bias and
+// GELU 31, with GELU's derivative 37; the library and torch's elementwise kernels 44 and 45), 2048 x 512 x 2048 32 / 34; gradients of weights 512 x 2048 x 2048 and
+// 2048 x 512 x 2048 29 / 35, 512 x 1536 x 2048 25.4 / 29, 512 x 512 x 2048 14.7 / 14.5 (through the first kernel 44, 39, 35, 31); 8192 tokens 77 / 97, 31 / 35, 97 / 125
+// (108 / 146, 134 / 156), 92 / 119 and 99 / 120, 84 / 99, 32 / 54.
 // Error against float64 at K = 2048 2.5e-7 to 3.5e-7, the library's 8.1e-7.
 //
 // Values that are not finite (or become so: bf16 ends half a step below fp32) do not split; an element of C that comes out not
@@ -91,8 +91,8 @@ template <bool KC> struct Source {
     __device__ __forceinline__ float4 fetch(const int k0) const
     {
         if (KC) return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, k0 + k < K ? at + (uint32_t)(k0 + k) * 4u : OUT, 0, 0));     // (K is a multiple of 4)
-        const uint32_t o = at + (uint32_t)(k0 + k) * (uint32_t)pitch;          // (rows of k past K lie behind the end)
-        auto one = [&](const int i) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, at < OUT ? o + (uint32_t)(i * pitch) : OUT, 0, 0)); };
+        const uint32_t o = at + (uint32_t)(k0 + k) * (uint32_t)pitch;          // (rows of k past K lie behind the end, and so does all of a row outside: below 2^32)
+        auto one = [&](const int i) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, o + (uint32_t)(i * pitch), 0, 0)); };
         return make_float4(one(0), one(1), one(2), one(3));
     }
 };
@@ -127,16 +127,18 @@ __device__ __forceinline__ float gelu_grad(const float x) {
     return __builtin_fmaf(x, 0.39894228040143268f * expf(-0.5f * x * x), cdf);
 }
 
+// Element (m, n); `h` is that of g.h where the epilogue reads it.
+template <int EPI> constexpr bool reads_h() { return EPI == PROTEUS_GEMM_ADD || EPI == PROTEUS_GEMM_GELU_GRAD; }
 template <int EPI>
-__device__ __forceinline__ void write(const GemmArgs& g, const int m, const int n, float v)
+__device__ __forceinline__ void write(const GemmArgs& g, const int m, const int n, float v, const float h = 0.f)
 {
     if (g.bias) v += g.bias[n];
     const size_t at = (size_t)m * g.ldc + n;
     if (EPI == PROTEUS_GEMM_F32)        static_cast<float*>(g.C)[at] = v;
     else if (EPI == PROTEUS_GEMM_BF16)  static_cast<__bf16*>(g.C)[at] = (__bf16)v;
     else if (EPI == PROTEUS_GEMM_GELU)  { g.H[at] = v; static_cast<float*>(g.C)[at] = gelu(v); }
-    else if (EPI == PROTEUS_GEMM_ADD)   static_cast<float*>(g.C)[at] = v + g.h[at];
-    else                                static_cast<float*>(g.C)[at] = v * gelu_grad(g.h[at]);
+    else if (EPI == PROTEUS_GEMM_ADD)   static_cast<float*>(g.C)[at] = v + h;
+    else                                static_cast<float*>(g.C)[at] = v * gelu_grad(h);
 }
 
 // AK, BK: k contiguous in A [M][K] / B [N][K]; else A is [K][M] / B [K][N]
@@ -210,6 +212,14 @@ void gemm_f32_kernel(const GemmArgs g)
         step(r + 1, 1);
     }
 
+    // what the epilogue reads, sent for under the groups' exchange (the last row and column in the place of what lies outside; one by one,
+    // us: 2048 x 2048 x 512 with a matrix added 38.4, so 32.1, with GELU's derivative 42.4 and 36.9, 3000 x 2048 x 512 60.9 and 56.6, 8192 x 512 x 256 30.1 and 26.4)
+    const int n = n0 + wn + (lane & 31);
+    auto row = [&](const int q, const int i) { return m0 + wm + 8 * q + 4 * (lane >> 5) + i; };
+    float hv[16 / G];
+    if constexpr (reads_h<EPI>())
+#pragma unroll
+        for (int e = 0; e < 16 / G; ++e) hv[e] = g.h[(size_t)min(row((e >> 2) * G + group, e & 3), g.M - 1) * g.ldc + min(n, g.N - 1)];
     // ---- the groups' sums together: group i takes every G-th quad of accumulators of every wave ----
     if (G > 1) {
         float* const red = reinterpret_cast<float*>(lds);
@@ -218,26 +228,21 @@ void gemm_f32_kernel(const GemmArgs g)
         for (int i = 0; i < 16; ++i) red[((group * 4 + wave) * 16 + i) * 64 + lane] = acc[i];
         __syncthreads();
     }
-    const int n = n0 + wn + (lane & 31);
     uint32_t again = 0;                                        // of the lane's 16 elements those that are not finite
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        if (G > 1 && (q % G) != group) continue;
+    for (int e = 0; e < 16 / G; ++e) {
+        const int q = (e >> 2) * G + group, i = e & 3, m = row(q, i);
+        float v;
+        if (G == 1) v = acc[e];
+        else {
+            const float* red = reinterpret_cast<const float*>(lds) + (wave * 16 + q * 4 + i) * 64 + lane;
+            v = red[0];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            float v;
-            if (G == 1) v = acc[q * 4 + i];
-            else {
-                const float* red = reinterpret_cast<const float*>(lds) + (wave * 16 + q * 4 + i) * 64 + lane;
-                v = red[0];
-#pragma unroll
-                for (int o = 1; o < G; ++o) v += red[o * 4 * 16 * 64];
-            }
-            const int m = m0 + wm + 8 * q + 4 * (lane >> 5) + i;
-            if (m >= g.M || n >= g.N) continue;
-            if (fabsf(v) <= 3.4028234e38f) write<EPI>(g, m, n, v * REDUCED);
-            else again |= 1u << (q * 4 + i);
+            for (int o = 1; o < G; ++o) v += red[o * 4 * 16 * 64];
         }
+        if (m >= g.M || n >= g.N) continue;
+        if (fabsf(v) <= 3.4028234e38f) write<EPI>(g, m, n, v * REDUCED, reads_h<EPI>() ? hv[e] : 0.f);
+        else again |= 1u << (q * 4 + i);
     }
     if (__builtin_amdgcn_ballot_w64(again != 0) == 0) return;
     // Where a row of A or a column of B holds a NaN so do their elements (a run that has diverged: all of them); the others are summed again.
@@ -247,7 +252,7 @@ void gemm_f32_kernel(const GemmArgs g)
     const uint32_t rows_a = (uint32_t)in_a | (uint32_t)(in_a >> 32), cols_b = (uint32_t)in_b | (uint32_t)(in_b >> 32);
     for (; again; again &= again - 1) {
         const int e = __builtin_ctz(again), r = 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3), m = m0 + wm + r;
-        write<EPI>(g, m, n, (rows_a >> r | cols_b >> (lane & 31)) & 1 ? __builtin_nanf("") : plain_dot<AK, BK>(g, m, n));
+        write<EPI>(g, m, n, (rows_a >> r | cols_b >> (lane & 31)) & 1 ? __builtin_nanf("") : plain_dot<AK, BK>(g, m, n), reads_h<EPI>() ? g.h[(size_t)m * g.ldc + n] : 0.f);
     }
 }
 
@@ -339,6 +344,17 @@ void gemm_f32_wide_kernel(const GemmArgs g)
         step(r + 1, 1);
     }
 
+    // (as above)
+    float hv[2 / G][32];
+    if constexpr (reads_h<EPI>())
+#pragma unroll
+        for (int i = 0; i < 2 / G; ++i)
+#pragma unroll
+            for (int e = 0; e < 32; ++e) {
+                const int m = m0 + wm + 32 * (G == 2 ? group : i) + 8 * ((e >> 2) & 3) + 4 * half + (e & 3), n = n0 + wn + 32 * (e >> 4) + r0;
+                hv[i][e] = g.h[(size_t)min(m, g.M - 1) * g.ldc + min(n, g.N - 1)];
+            }
+
     // ---- the groups' sums together: group i takes the i-th 32 rows of every wave's 64, and hands on the others ----
     if constexpr (G == 2) {
         float* const red = reinterpret_cast<float*>(lds);
@@ -365,7 +381,7 @@ void gemm_f32_wide_kernel(const GemmArgs g)
             const float v = acc[i][e >> 4][e & 15];
             const int m = mw + 8 * ((e >> 2) & 3) + 4 * half + (e & 3), n = n0 + wn + 32 * (e >> 4) + r0;
             if (m >= g.M || n >= g.N) continue;
-            if (fabsf(v) <= 3.4028234e38f) write<EPI>(g, m, n, v * REDUCED);
+            if (fabsf(v) <= 3.4028234e38f) write<EPI>(g, m, n, v * REDUCED, reads_h<EPI>() ? hv[i][e] : 0.f);
             else again |= 1u << e;
         }
         if (__builtin_amdgcn_ballot_w64(again != 0) == 0) continue;
@@ -382,7 +398,7 @@ void gemm_f32_wide_kernel(const GemmArgs g)
         for (; again; again &= again - 1) {
             const int e = __builtin_ctz(again), r = 8 * ((e >> 2) & 3) + 4 * half + (e & 3), n = n0 + wn + 32 * (e >> 4) + r0;
             const bool nan = (rows_a >> r | (e >> 4 ? cols_b[1] : cols_b[0]) >> r0) & 1;
-            write<EPI>(g, mw + r, n, nan ? __builtin_nanf("") : plain_dot<AK, BK>(g, mw + r, n));
+            write<EPI>(g, mw + r, n, nan ? __builtin_nanf("") : plain_dot<AK, BK>(g, mw + r, n), reads_h<EPI>() ? g.h[(size_t)(mw + r) * g.ldc + n] : 0.f);
         }
     }
 }
@@ -549,14 +565,24 @@ void gemm_f32_rows_kernel(const GemmArgs g)
     finish_rows<64 / W>(g, m0, n0, wave * (64 / W), v);
 }
 
-// The shares' sums of a tile together, in their order: a quarter of a tile per workgroup, four accumulators per wave.
-__global__ __launch_bounds__(256)
+// The shares' sums of a tile together, in their order: half of a tile per workgroup, four accumulators per wave.  The workgroups behind those make column sums.
+__global__ __launch_bounds__(proteus_train::CS_BLOCK)
 void gemm_f32_rows_sum_kernel(const PendingSums sums)
 {
+    static_assert(proteus_train::CS_BLOCK == 512, "eight waves");
+    __shared__ float red[proteus_train::CS_BLOCK / 64][proteus_train::CS_COLS];
+    const int behind = (int)blockIdx.x - sums.first[sums.count];
+    if (behind >= 0) {
+        int c = 0;
+        while (behind >= sums.first_column[c + 1]) ++c;
+        const proteus_train::ColumnSums& of = sums.columns[c];
+        proteus_train::column_sums(of.a, of.out, 0, of.rows, of.cols, behind - sums.first_column[c], red);
+        return;
+    }
     int p = 0;
     while ((int)blockIdx.x >= sums.first[p + 1]) ++p;
     const GemmArgs& g = sums.product[p];
-    const int block = (int)blockIdx.x - sums.first[p], tile = block >> 2, e0 = (block & 3) * 16 + (threadIdx.x >> 6) * 4;
+    const int block = (int)blockIdx.x - sums.first[p], tile = block >> 1, e0 = (block & 1) * 32 + (threadIdx.x >> 6) * 4;
     const float* from = g.part + (size_t)tile * (GT * GT) + e0 * 64 + (threadIdx.x & 63);
     const size_t pitch = (size_t)g.tiles * (GT * GT);
     float v[4] = {};
@@ -572,7 +598,7 @@ void gemm_f32_rows_sum_kernel(const PendingSums sums)
 // Groups of gemm_f32_wide_kernel, 0: tiles of 64 x 64.  Two while its tiles leave a compute unit one each and few idle, one (three workgroups of which share a compute
 // unit) from where their rounds are full enough; not for a short K, and later where the epilogue is long, since nothing runs under that of a lone workgroup.  Us, 64 x 64 / 128 x 128
 // with two groups, M x N x K: 2048 x 2048 x 512 (256 tiles) with bias and GELU 41.3 / 36.0, with GELU's derivative 45.1 / 41.8; 2048 x 1536 x 512 (192) 28.0 / 25.7; 1536 x 1536 x 512 (144) 26.4 / 25.0;
-// 1536 x 2048 x 512 (192) 33.3 / 32.6 and 36.7 / 39.2 (the 64 x 64 ones before their steps were laid out: a twentieth slower than now); 5000 x 512 x 2048 (160) 91 / 74; 8192 x 512 x 2048 (256) 127 / 92, x 512 36.1 / 30.6, x 256 25.8 / 25.0; 4096 x 512 x 2048 (128) 63 / 71;
+// 1536 x 2048 x 512 (192) 33.3 / 32.6 and 36.7 / 39.2 (all before the epilogues' reads were sent off early, the 64 x 64 ones before their steps were laid out: up to a tenth slower than now); 5000 x 512 x 2048 (160) 91 / 74; 8192 x 512 x 2048 (256) 127 / 92, x 512 36.1 / 30.6, x 256 25.8 / 25.0; 4096 x 512 x 2048 (128) 63 / 71;
 // 2048 x 1024 x 1024 (128) 34 / 41; 4096 x 768 x 256 (192) 15.9 / 16.6.  With one group: 3072 x 1536 x 512 (288 tiles) 41 / 48, 4096 x 1536 (384) 51.0 / 50.2, 5000 x 1536 (480) 64 / 53, 4096 x 2048
 // (512) 77 / 69 and 80.2 / 80.7, 5000 x 2048 (640) 93 / 88 and 96 / 99, 6144 x 2048 (768) 108 / 92 and 115 / 105, 8192 x 2048 (1024) 146 / 120 and 156 / 146, 8192 x 1536 (768) 96 / 75,
 // 16384 x 1024 x 1024 244 / 184; 16384 x 512 x 256 (512) 44.1 / 45.5, 32768 x 512 x 128 (1024) 53 / 63.
@@ -605,7 +631,7 @@ int gemm_go(GemmArgs g, hipStream_t st, PendingSums* sums = nullptr)
             PendingSums own;
             PendingSums& p = sums ? *sums : own;
             p.product[p.count] = g;
-            p.first[p.count + 1] = p.first[p.count] + g.tiles * 4;
+            p.first[p.count + 1] = p.first[p.count] + g.tiles * 2;
             ++p.count;
             if (!sums) return gemm_sums(own, st);
         }
@@ -732,8 +758,9 @@ int proteus_gemm::gemm_begin(const float* A, const float* B, float* C, int M, in
 
 int proteus_gemm::gemm_sums(PendingSums& sums, void* stream)
 {
-    if (sums.count == 0) return PROTEUS_OK;
-    hipLaunchKernelGGL(gemm_f32_rows_sum_kernel, dim3((unsigned)sums.first[sums.count]), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), sums);
-    sums.count = 0;
+    const int blocks = sums.first[sums.count] + sums.first_column[sums.column_count];
+    if (blocks == 0) return PROTEUS_OK;
+    hipLaunchKernelGGL(gemm_f32_rows_sum_kernel, dim3((unsigned)blocks), dim3(proteus_train::CS_BLOCK), 0, reinterpret_cast<hipStream_t>(stream), sums);
+    sums.count = sums.column_count = 0;
     return (int)hipGetLastError();
 }
