@@ -5,9 +5,9 @@
 // (so that the compiler sees that a read of one does not wait for loads into another).  Bias and GELU are added to the fp32 sums, which are then rounded once.
 //
 // What bounds it: LDS at 64 x 64 of C per wave (16 KB read per 128 clocks of matrix instructions and compute unit, its whole rate), a quarter less at 128 x 64; and the
-// rounds of workgroups (one to three of them on a compute unit).  8192 tokens, d_model 512, us, the library's product and torch's GELU / this: QKV 24 / 20, output 13 / 9, feed-forward
-// 25 + 15 / 28 and 23 / 21; a call costs the host 3, the library's 18 to 21.
-// From about 16384 x 1024 of d_model 1024 on the library is ahead (32768 x 3072 x 1024 155 / 218).
+// rounds of workgroups (one to three of them on a compute unit).  8192 tokens, d_model 512, us, the library's product and torch's GELU / this: QKV 24 / 18, output 13 / 9, feed-forward
+// 25 + 15 / 27 and 23 / 21; a call costs the host 3, the library's 18 to 21.
+// From about 16384 x 1024 of d_model 1024 on the library is ahead (32768 x 3072 x 1024 155 / 194).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include "proteus_hip.h"
@@ -131,7 +131,26 @@ void gemm_bf16_kernel(const Args g)
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         issue(step + STAGES - 1, next);                                        // (past the end: zeros)
+        // Two stages: the loads leave before the products, not behind them, where the compiler puts them and where the next step waits for all of
+        // their way; the fragments of 16 k are read under the products of the 16 before.  Us, left alone / so: 8192 x 2048 x 512 (GELU) 29.6 / 27.3, 8192 x 1536 x 512 19.0 / 18.0, 6000 x 1536 x
+        // 512 16.1 / 15.3, 12288 x 2304 x 768 50 / 45, 65536 x 2048 x 512 228 / 207.  (Three steps ahead there is no hurry, and the reads come first: 2048 x 512 x 2048 8.4 / 9.5.)
+        if constexpr (STAGES == 2) __builtin_amdgcn_sched_barrier(0);
         multiply(mine);
+        if constexpr (STAGES == 2) {
+            constexpr int READS = TM + TN, PRODUCTS = TM * TN, PAIRS = READS < PRODUCTS ? READS : PRODUCTS;
+            __builtin_amdgcn_sched_group_barrier(0x100, READS, 0);
+#pragma unroll
+            for (int ks = 1; ks < HK / 16; ++ks) {
+#pragma unroll
+                for (int i = 0; i < PAIRS; ++i) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);         // a product,
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);         // a fragment
+                }
+                if (READS > PAIRS)    __builtin_amdgcn_sched_group_barrier(0x100, READS - PAIRS, 0);
+                if (PRODUCTS > PAIRS) __builtin_amdgcn_sched_group_barrier(0x008, PRODUCTS - PAIRS, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x008, PRODUCTS, 0);
+        }
     };
     issue(0, s0);
     if (STAGES > 2) issue(1, s1);
