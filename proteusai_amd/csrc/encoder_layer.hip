@@ -82,9 +82,11 @@ struct Backward {
         dy2 = dO = c.take<float>(rows * dm);
         dx1 = c.take<float>(rows * dm); dO16 = reinterpret_cast<uint16_t*>(dx1);
         dy1 = c.take<float>(rows * dm); D = c.take<float>(rows * s.H); d_sigma = c.take<float>(s.H);
-        dW = c.take<float>(3 * dm * dm); db = c.take<float>(3 * dm); dWo = c.take<float>(dm * dm);
+        // (the second LayerNorm's partial sums are added up before the projections' gradient takes their place)
         ln_bytes = proteus_layernorm_bwd_workspace_bytes(s.rows, s.dm);
-        lnws[0] = c.take<char>(ln_bytes); lnws[1] = c.take<char>(ln_bytes);
+        dW = c.take<float>(3 * dm * dm > ln_bytes / 4 ? 3 * dm * dm : ln_bytes / 4); lnws[1] = dW;
+        db = c.take<float>(3 * dm); dWo = c.take<float>(dm * dm);
+        lnws[0] = c.take<char>(ln_bytes);
         sums_bytes = proteus_train_workspace_bytes(s.rows, s.hidden > 3 * s.dm ? s.hidden : 3 * s.dm);
         sums = c.take<char>(sums_bytes);
         const int sizes[4][2] = {{s.dm, s.hidden}, {s.hidden, s.dm}, {s.dm, s.dm}, {s.dm, 3 * s.dm}};

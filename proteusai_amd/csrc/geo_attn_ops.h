@@ -87,4 +87,88 @@ template <> __device__ __forceinline__ int tile_swizzle<32>(int r)  { return (r 
 template <> __device__ __forceinline__ int tile_swizzle<64>(int r)  { return (((r >> 1) & 1) << 2) | ((r >> 2) & 3); }
 template <> __device__ __forceinline__ int tile_swizzle<128>(int r) { return ((r & 3) << 2) | ((r >> 2) & 3); }
 
+// ---- padded batches handed out longest sequence first ----
+constexpr int ATTN_LPT_MAX_Z = 64;
+
+// Is a batch's mask read 16 bytes at a time?  (A piece then lies in at most two sequences.)
+__device__ __forceinline__ bool mask_in_pieces(const uint8_t* mask, const int N) { return N >= 16 && ((uintptr_t)mask & 15) == 0; }
+
+// lens[z], zero before: 1 + index of the last unpadded token of sequence z of Z.  Called by all threads of a workgroup.
+template <int THREADS>
+__device__ __forceinline__ void sequence_lengths(const uint8_t* __restrict__ mask, const int Z, const int N, int* lens)
+{
+    const int total = Z * N;
+    int from = 0;
+    if (mask_in_pieces(mask, N)) {
+        const int pieces = total >> 4;
+        from = pieces << 4;
+#pragma unroll 4
+        for (int p = (int)threadIdx.x; p < pieces; p += THREADS) {
+            const uint4 m16 = *reinterpret_cast<const uint4*>(mask + (size_t)p * 16);
+            const unsigned w[4] = {m16.x, m16.y, m16.z, m16.w};
+            unsigned usable = 0;                                  // bit e: byte e is zero
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const unsigned zero = ~(((w[e] & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w[e]) & 0x80808080u;       // (bit 7 of a byte that is zero)
+                usable |= (((zero >> 7) & 1u) | ((zero >> 14) & 2u) | ((zero >> 21) & 4u) | (zero >> 28)) << (4 * e);
+            }
+            const int z = 16 * p / N, here = (z + 1) * N - 16 * p;                   // bytes of the piece in sequence z, the others in z + 1
+            const unsigned low = here >= 16 ? usable : usable & ((1u << here) - 1u), high = usable ^ low;
+            if (low)  atomicMax(&lens[z], 16 * p - z * N + 32 - __builtin_clz(low));
+            if (high) atomicMax(&lens[z + 1], 32 - __builtin_clz(high) - here);
+        }
+    }
+    for (int j = from + (int)threadIdx.x; j < total; j += THREADS) if (!mask[j]) atomicMax(&lens[j / N], j % N + 1);
+}
+
+// Workgroup `block_id` of n_tiles * Z * H takes the block_id-th item of the list "live tiles (of OWN tokens) of the longest sequence, tile-major, the heads of a tile
+// side by side, those of the next one, ..., then the dead tiles"; tile and zh = (sequence, head) of it.  lens: LDS, left with 1 + index of the last unpadded
+// token of every sequence.  Called by all threads of a workgroup.
+template <int THREADS>
+__device__ __forceinline__ void by_length(const uint8_t* __restrict__ key_pad, const int Z, const int N, const int H, const int n_tiles, const int own, const int block_id,
+                                          int* lens, int& tile, int& zh)
+{
+    const int tid = threadIdx.x, lane = tid & 63;
+    if (tid < Z) lens[tid] = 0;
+    __syncthreads();
+    sequence_lengths<THREADS>(key_pad, Z, N, lens);
+    __syncthreads();
+    const int mine = lane < Z ? lens[lane] : 0;
+    int rank = lane < Z ? 0 : lane;
+    for (int u = 0; u < Z; ++u) {
+        const int o = __builtin_amdgcn_readlane(mine, u);
+        if (lane < Z) rank += (o > mine || (o == mine && u < lane)) ? 1 : 0;
+    }
+    // lane r: the sequence of rank r, its live tiles, and the workgroups of all up to it
+    const int item = __builtin_amdgcn_ds_permute(rank << 2, lane);
+    const int tiles = (__builtin_amdgcn_ds_permute(rank << 2, mine) + own - 1) / own;
+    auto up_to = [&](int n) {
+        for (int o = 1; o < 64; o *= 2) { const int below = __shfl_up(n, o); if (lane >= o) n += below; }
+        return n;
+    };
+    // (the list laid over the launch as a snake, every second row of 256 workgroups reversed: workgroups b and
+    // b + 256 share a compute unit while the launch fills the chip, and get a long and a short item)
+    int rem = block_id;
+    {
+        const int total = n_tiles * Z * H, row0 = block_id - block_id % 256;
+        const int rowlen = min(total - row0, 256);
+        if ((block_id / 256) & 1) rem = row0 + (rowlen - 1 - (block_id - row0));
+    }
+    int cnt = lane < Z ? tiles * H : 0, sum = up_to(cnt), first = 0;
+    const int live = __builtin_amdgcn_readlane(sum, 63);
+    const bool dead = rem >= live;
+    if (dead) {
+        rem -= live;
+        cnt = lane < Z ? (n_tiles - tiles) * H : 0;
+        sum = up_to(cnt);
+    }
+    const int sel = __builtin_ctzll(__builtin_amdgcn_ballot_w64(rem < sum));        // (the list has a place for every workgroup)
+    if (dead) first = __builtin_amdgcn_readlane(tiles, sel);
+    rem -= __builtin_amdgcn_readlane(sum, sel) - __builtin_amdgcn_readlane(cnt, sel);
+    const int zsel = __builtin_amdgcn_readlane(item, sel);
+    rem = __builtin_amdgcn_readfirstlane(rem);
+    tile = __builtin_amdgcn_readfirstlane(first) + rem / H;
+    zh = zsel * H + rem % H;
+}
+
 }  // namespace proteus_ops
