@@ -123,16 +123,18 @@ __device__ __forceinline__ void sequence_lengths(const uint8_t* __restrict__ mas
 
 // Workgroup `block_id` of n_tiles * Z * H takes the block_id-th item of the list "live tiles (of OWN tokens) of the longest sequence, tile-major, the heads of a tile
 // side by side, those of the next one, ..., then the dead tiles"; tile and zh = (sequence, head) of it.  lens: LDS, left with 1 + index of the last unpadded
-// token of every sequence.  Called by all threads of a workgroup.
-template <int THREADS>
+// token of every sequence (KNOWN: they are there).  Called by all threads of a workgroup.
+template <int THREADS, bool KNOWN = false>
 __device__ __forceinline__ void by_length(const uint8_t* __restrict__ key_pad, const int Z, const int N, const int H, const int n_tiles, const int own, const int block_id,
                                           int* lens, int& tile, int& zh)
 {
     const int tid = threadIdx.x, lane = tid & 63;
-    if (tid < Z) lens[tid] = 0;
-    __syncthreads();
-    sequence_lengths<THREADS>(key_pad, Z, N, lens);
-    __syncthreads();
+    if (!KNOWN) {
+        if (tid < Z) lens[tid] = 0;
+        __syncthreads();
+        sequence_lengths<THREADS>(key_pad, Z, N, lens);
+        __syncthreads();
+    }
     const int mine = lane < Z ? lens[lane] : 0;
     int rank = lane < Z ? 0 : lane;
     for (int u = 0; u < Z; ++u) {
