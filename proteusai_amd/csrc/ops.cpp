@@ -114,8 +114,12 @@ std::pair<Tensor, Tensor> attention_forward(const Tensor& q, const Tensor& k, co
         launched(proteus_geo_attn_fwd_ws(halves(q), halves(k), halves(v), st.get(), floats(coords), floats(sigma), bytes(mask), out_floats(O), out_floats(L),
                                          need ? ws.mutable_data_ptr() : nullptr, need, Z, H, N, d, 0, stream), "proteus_geo_attn_fwd");
     } else {
-        launched(proteus_geo_attn_legacy_fwd_strided(halves(q), halves(k), halves(v), st.v, floats(coords), floats(sigma), floats(betas), bytes(mask), out_floats(O), out_floats(L),
-                                                     Z, H, N, d, how.min_rbf, how.max_rbf, how.f16 ? PROTEUS_OPERAND_F16 : PROTEUS_OPERAND_BF16, 0, stream), "proteus_geo_attn_fwd");
+        // (contiguous tensors may have any stride along a dimension of size one, which the strided entry point would hold against them)
+        const int type = how.f16 ? PROTEUS_OPERAND_F16 : PROTEUS_OPERAND_BF16;
+        launched(st.get() ? proteus_geo_attn_legacy_fwd_strided(halves(q), halves(k), halves(v), st.get(), floats(coords), floats(sigma), floats(betas), bytes(mask), out_floats(O), out_floats(L),
+                                                                Z, H, N, d, how.min_rbf, how.max_rbf, type, 0, stream)
+                          : proteus_geo_attn_legacy_fwd(halves(q), halves(k), halves(v), floats(coords), floats(sigma), floats(betas), bytes(mask), out_floats(O), out_floats(L),
+                                                        Z, H, N, d, how.min_rbf, how.max_rbf, type, 0, stream), "proteus_geo_attn_fwd");
     }
     return {O, L};
 }

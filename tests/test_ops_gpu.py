@@ -79,6 +79,30 @@ def test_attention_equals_the_python_path(gpu, general, legacy, d, form):
         assert torch.equal(pa.geometric_attn(*qkv, coords, spreads, mask=mask, **kw), want[0])
 
 
+# Contiguous operands with strides of their own along a dimension of size one: a single token (transposed), a single sequence, a single head
+@pytest.mark.gpu
+@pytest.mark.parametrize("legacy", [False, True])
+@pytest.mark.parametrize("token_major", [False, True])
+@pytest.mark.parametrize("one", ["token", "sequence", "head"])
+@pytest.mark.parametrize("which", [(0, 1, 2), (1,)])
+def test_dimensions_of_size_one(gpu, general, legacy, token_major, one, which):
+    Z, H, N, d = {"token": (2, 4, 1, 32), "sequence": (1, 4, 40, 32), "head": (2, 1, 40, 32)}[one]
+    qkv, coords, spreads, _, kw, dO = _attention(gpu, legacy, d, Z=Z, N=N, H=H)
+    strides = {"token": (H * d, d, 1, 1), "sequence": (9, N * d, d, 1), "head": (N * d, 9, d, 1)}[one]
+    qkv = [torch.as_strided(t.detach(), t.shape, strides).requires_grad_() if i in which else t for i, t in enumerate(qkv)]
+    assert all(t.is_contiguous() for t in qkv) and any(t.stride() == strides for t in qkv)
+    kw["token_major_out"] = token_major
+    with general():
+        try:
+            want = _run(qkv, coords, spreads, None, kw, dO)
+        except ValueError:
+            want = None             # (an odd stride beside O in token order)
+    if want is not None:
+        got = _run(qkv, coords, spreads, None, kw, dO)
+        assert "Attention" in got[0].grad_fn.name()
+        _same(got, want)
+
+
 # What has to be converted or refused is the Python functions': not taken, and the same result or error
 @pytest.mark.gpu
 def test_attention_that_is_not_plain(gpu, general):
