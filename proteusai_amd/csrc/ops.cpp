@@ -70,7 +70,9 @@ bool current(const int dev)
 
 void* stream_of(const int dev) { return c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(dev)).stream(); }
 
-void launched(const int rc, const char* what) { TORCH_CHECK(rc == 0, what, ": ", proteus_strerror(rc), " (code ", rc, ")"); }
+// What the library does not take, or could not launch, goes the general way, which says what is wrong with it (as a ValueError or a ProteusError).
+struct Refused {};
+void launched(const int rc) { if (rc != 0) throw Refused(); }
 
 at::TensorOptions on(const Tensor& t, const at::ScalarType type) { return t.options().dtype(type).requires_grad(false); }
 
@@ -112,14 +114,14 @@ std::pair<Tensor, Tensor> attention_forward(const Tensor& q, const Tensor& k, co
         Tensor ws;
         if (need) ws = at::empty({static_cast<int64_t>(need)}, on(q, at::kByte));
         launched(proteus_geo_attn_fwd_ws(halves(q), halves(k), halves(v), st.get(), floats(coords), floats(sigma), bytes(mask), out_floats(O), out_floats(L),
-                                         need ? ws.mutable_data_ptr() : nullptr, need, Z, H, N, d, 0, stream), "proteus_geo_attn_fwd");
+                                         need ? ws.mutable_data_ptr() : nullptr, need, Z, H, N, d, 0, stream));
     } else {
         // (contiguous tensors may have any stride along a dimension of size one, which the strided entry point would hold against them)
         const int type = how.f16 ? PROTEUS_OPERAND_F16 : PROTEUS_OPERAND_BF16;
         launched(st.get() ? proteus_geo_attn_legacy_fwd_strided(halves(q), halves(k), halves(v), st.get(), floats(coords), floats(sigma), floats(betas), bytes(mask), out_floats(O), out_floats(L),
                                                                 Z, H, N, d, how.min_rbf, how.max_rbf, type, 0, stream)
                           : proteus_geo_attn_legacy_fwd(halves(q), halves(k), halves(v), floats(coords), floats(sigma), floats(betas), bytes(mask), out_floats(O), out_floats(L),
-                                                        Z, H, N, d, how.min_rbf, how.max_rbf, type, 0, stream), "proteus_geo_attn_fwd");
+                                                        Z, H, N, d, how.min_rbf, how.max_rbf, type, 0, stream));
     }
     return {O, L};
 }
@@ -137,7 +139,7 @@ variable_list attention_backward_general(const variable_list& s, const Tensor& d
     return out;                                  // dQ, dK, dV, d_sigma, d_betas
 }
 
-variable_list attention_backward(const variable_list& s, const Tensor& dO, const Logits& how)
+variable_list attention_backward_plain(const variable_list& s, const Tensor& dO, const Logits& how)
 {
     const Tensor &q = s[0], &k = s[1], &v = s[2], &O = s[3], &L = s[4], &coords = s[5], &sigma = s[6], &betas = s[7], &mask = s[8];
     const auto op = how.f16 ? at::kHalf : at::kBFloat16;
@@ -172,8 +174,7 @@ variable_list attention_backward(const variable_list& s, const Tensor& dO, const
     Strides prep;
     for (const Tensor* t : {&O, &dO, static_cast<const Tensor*>(&cast)}) prep.add(*t);
     launched(proteus_geo_attn_prepare_bwd(floats(O), dO.const_data_ptr(), prep.get(), out_floats(D), type != op ? static_cast<uint16_t*>(cast.mutable_data_ptr()) : nullptr, out_floats(d_sigma),
-                                          to_beta, Z, H, N, d, type == at::kFloat ? PROTEUS_DTYPE_F32 : type == at::kHalf ? PROTEUS_DTYPE_F16 : PROTEUS_DTYPE_BF16, operand, stream),
-             "proteus_geo_attn_prepare_bwd");
+                                          to_beta, Z, H, N, d, type == at::kFloat ? PROTEUS_DTYPE_F32 : type == at::kHalf ? PROTEUS_DTYPE_F16 : PROTEUS_DTYPE_BF16, operand, stream));
     // gradients in the memory order of their operands (dense) and in their type
     auto like = [&](const Tensor& t) {
         const Tensor g = at::empty_like(t, on(t, op));
@@ -184,8 +185,17 @@ variable_list attention_backward(const variable_list& s, const Tensor& dO, const
     for (const Tensor* t : {&q, &k, &v, static_cast<const Tensor*>(&cast), &dq, &dk, &dv}) st.add(*t);
     launched(proteus_geo_attn_bwd_typed(halves(q), halves(k), halves(v), halves(cast), st.get(), floats(coords), floats(sigma), betas.defined() ? floats(betas) : nullptr, bytes(mask),
                                         floats(L), floats(D), dq.mutable_data_ptr(), dk.mutable_data_ptr(), dv.mutable_data_ptr(), out_floats(d_sigma), to_beta, Z, H, N, d,
-                                        how.legacy ? how.min_rbf : 0.0, how.legacy ? how.max_rbf : 1.0, operand, PROTEUS_GRAD_OPERAND, stream), "proteus_geo_attn_bwd");
+                                        how.legacy ? how.min_rbf : 0.0, how.legacy ? how.max_rbf : 1.0, operand, PROTEUS_GRAD_OPERAND, stream));
     return {dq, dk, dv, d_sigma, d_beta};
+}
+
+variable_list attention_backward(const variable_list& s, const Tensor& dO, const Logits& how)
+{
+    try {
+        return attention_backward_plain(s, dO, how);
+    } catch (const Refused&) {
+        return attention_backward_general(s, dO, how);
+    }
 }
 
 struct Attention : torch::autograd::Function<Attention> {
@@ -260,7 +270,7 @@ py::object attention(const py::object& Q, const py::object& K, const py::object&
     const bool recording = at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad() || spreads.requires_grad() || (legacy && betas.requires_grad()));
     Tensor O;
     bool good = true;
-    {
+    try {
         py::gil_scoped_release no_gil;
         const std::optional<Tensor> b = legacy ? std::optional<Tensor>(betas) : std::nullopt, m = mask.defined() ? std::optional<Tensor>(mask) : std::nullopt;
         if (recording) O = Attention::apply(q, k, v, coords, spreads, b, m, legacy, f16, min_rbf, max_rbf, token_major);
@@ -269,6 +279,8 @@ py::object attention(const py::object& Q, const py::object& K, const py::object&
             O = attention_forward(q, k, v, coords, spreads, betas, mask, Logits{legacy, f16, min_rbf, max_rbf}, token_major).first;
         }
         if (arriving) good = arriving->positive();
+    } catch (const Refused&) {
+        return py::none();
     }
     return good ? py::cast(O) : py::none();                   // (what is wrong with the spreads is said by the general path)
 }
@@ -302,7 +314,7 @@ std::array<Tensor, 3> embedding_forward(const Tensor& coords, const Tensor& wn, 
     Tensor ws;
     if (need) ws = at::empty({static_cast<int64_t>(need)}, on(coords, at::kByte));
     launched(proteus_we_fwd_ws(floats(coords), PROTEUS_COORDS_AOS, floats(wn), bytes(mask), out_floats(out), sums ? out_floats(cs) : nullptr, sums ? out_floats(sn) : nullptr,
-                               need ? ws.mutable_data_ptr() : nullptr, need, Z, N, K, 0, stream_of(coords.get_device())), "proteus_we_fwd");
+                               need ? ws.mutable_data_ptr() : nullptr, need, Z, N, K, 0, stream_of(coords.get_device())));
     return {out, cs, sn};
 }
 
@@ -317,14 +329,18 @@ struct Embedding : torch::autograd::Function<Embedding> {
     {
         const variable_list s = ctx->get_saved_variables();
         const Tensor& dO = grads[0];
-        if (!backward_ok(dO, s, 2)) {
-            py::gil_scoped_acquire gil;
-            return {Tensor(), py::reinterpret_borrow<py::object>(g_embedding_backward)(dO, s[0], s[1]).cast<Tensor>(), Tensor()};
-        }
+        if (backward_ok(dO, s, 2)) try {
+            return {Tensor(), reduced(dO, s), Tensor()};
+        } catch (const Refused&) {}
+        py::gil_scoped_acquire gil;
+        return {Tensor(), py::reinterpret_borrow<py::object>(g_embedding_backward)(dO, s[0], s[1]).cast<Tensor>(), Tensor()};
+    }
+    static Tensor reduced(const Tensor& dO, const variable_list& s)
+    {
         const int64_t K = dO.size(2) / 2;
         const Tensor ws = bwd_workspace(dO, K), dk = at::empty({K}, on(dO, at::kFloat));
-        launched(proteus_we_bwd(floats(dO), floats(s[0]), floats(s[1]), out_floats(dk), out_floats(ws), ws.numel(), dO.size(0), dO.size(1), K, stream_of(dO.get_device())), "proteus_we_bwd");
-        return {Tensor(), dk, Tensor()};
+        launched(proteus_we_bwd(floats(dO), floats(s[0]), floats(s[1]), out_floats(dk), out_floats(ws), ws.numel(), dO.size(0), dO.size(1), K, stream_of(dO.get_device())));
+        return dk;
     }
 };
 
@@ -338,7 +354,7 @@ std::array<Tensor, 3> aniso_forward(const Tensor& a, const Tensor& b, const Tens
     Tensor ws;
     if (need) ws = at::empty({static_cast<int64_t>(need)}, on(a, at::kByte));
     launched(proteus_we_aniso_fwd_ws(floats(a), floats(b), PROTEUS_COORDS_AOS, floats(cb), floats(wn), bytes(mask), out_floats(out), partials ? out_floats(d_cb) : nullptr,
-                                     partials ? out_floats(d_k) : nullptr, need ? ws.mutable_data_ptr() : nullptr, need, Z, N, K, 0, stream_of(a.get_device())), "proteus_we_aniso_fwd");
+                                     partials ? out_floats(d_k) : nullptr, need ? ws.mutable_data_ptr() : nullptr, need, Z, N, K, 0, stream_of(a.get_device())));
     return {out, d_cb, d_k};
 }
 
@@ -355,19 +371,23 @@ struct Aniso : torch::autograd::Function<Aniso> {
         const Tensor& dO = grads[0];
         for (int i = 0; i < 2; ++i) if (!ctx->needs_input_grad(2 + i)) s[i] = Tensor();
         if (!s[0].defined() && !s[1].defined()) return {Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
-        if (!backward_ok(dO, s, 1)) {
-            py::gil_scoped_acquire gil;
-            auto opt = [](const Tensor& t) -> py::object { return t.defined() ? py::cast(t) : py::none(); };
-            const py::tuple got = py::reinterpret_borrow<py::object>(g_aniso_backward)(dO, opt(s[0]), opt(s[1]));
-            auto back = [&](const int i) { const py::object o = got[i]; return o.is_none() ? Tensor() : o.cast<Tensor>(); };
-            return {Tensor(), Tensor(), back(0), back(1), Tensor()};
-        }
+        if (backward_ok(dO, s, 1)) try {
+            return reduced(dO, s);
+        } catch (const Refused&) {}
+        py::gil_scoped_acquire gil;
+        auto opt = [](const Tensor& t) -> py::object { return t.defined() ? py::cast(t) : py::none(); };
+        const py::tuple got = py::reinterpret_borrow<py::object>(g_aniso_backward)(dO, opt(s[0]), opt(s[1]));
+        auto back = [&](const int i) { const py::object o = got[i]; return o.is_none() ? Tensor() : o.cast<Tensor>(); };
+        return {Tensor(), Tensor(), back(0), back(1), Tensor()};
+    }
+    static variable_list reduced(const Tensor& dO, const variable_list& s)
+    {
         const int64_t K = dO.size(2) / 2;
         const Tensor ws = bwd_workspace(dO, K);
         Tensor g[2];
         for (int i = 0; i < 2; ++i) if (s[i].defined()) g[i] = at::empty({K}, on(dO, at::kFloat));
         launched(proteus_we_aniso_bwd(floats(dO), s[0].defined() ? floats(s[0]) : nullptr, s[1].defined() ? floats(s[1]) : nullptr, g[0].defined() ? out_floats(g[0]) : nullptr,
-                                      g[1].defined() ? out_floats(g[1]) : nullptr, out_floats(ws), ws.numel(), dO.size(0), dO.size(1), K, stream_of(dO.get_device())), "proteus_we_aniso_bwd");
+                                      g[1].defined() ? out_floats(g[1]) : nullptr, out_floats(ws), ws.numel(), dO.size(0), dO.size(1), K, stream_of(dO.get_device())));
         return {Tensor(), Tensor(), g[0], g[1], Tensor()};
     }
 };
@@ -385,10 +405,12 @@ py::object embedding(const py::object& coords_, const py::object& wn_, const py:
     if (!unobserved() || !get(coords_, coords) || !current(coords.get_device()) || !get(wn_, wn, coords.get_device()) || !sizes_ok(coords, wn)
         || !get_mask(mask_, mask, coords.get_device(), coords.size(0), coords.size(1)) || coords.requires_grad()) return py::none();
     Tensor out;
-    {
+    try {
         py::gil_scoped_release no_gil;
         if (at::GradMode::is_enabled() && wn.requires_grad()) out = Embedding::apply(coords, wn, mask.defined() ? std::optional<Tensor>(mask) : std::nullopt);
         else { at::NoGradGuard no_grad; out = embedding_forward(coords, wn, mask, false)[0]; }
+    } catch (const Refused&) {
+        return py::none();
     }
     return py::cast(out);
 }
@@ -402,10 +424,12 @@ py::object aniso(const py::object& a_, const py::object& b_, const py::object& c
     if (!get(b_, b, dev) || !get(cb_, cb, dev) || !get(wn_, wn, dev) || !sizes_ok(a, wn) || !f32(b) || b.sizes() != a.sizes() || !f32(cb) || cb.sizes() != wn.sizes()
         || !get_mask(mask_, mask, dev, a.size(0), a.size(1)) || a.requires_grad() || b.requires_grad()) return py::none();
     Tensor out;
-    {
+    try {
         py::gil_scoped_release no_gil;
         if (at::GradMode::is_enabled() && (cb.requires_grad() || wn.requires_grad())) out = Aniso::apply(a, b, cb, wn, mask.defined() ? std::optional<Tensor>(mask) : std::nullopt);
         else { at::NoGradGuard no_grad; out = aniso_forward(a, b, cb, wn, mask, false)[0]; }
+    } catch (const Refused&) {
+        return py::none();
     }
     return py::cast(out);
 }

@@ -92,15 +92,20 @@ def test_dimensions_of_size_one(gpu, general, legacy, token_major, one, which):
     qkv = [torch.as_strided(t.detach(), t.shape, strides).requires_grad_() if i in which else t for i, t in enumerate(qkv)]
     assert all(t.is_contiguous() for t in qkv) and any(t.stride() == strides for t in qkv)
     kw["token_major_out"] = token_major
-    with general():
-        try:
-            want = _run(qkv, coords, spreads, None, kw, dO)
-        except ValueError:
-            want = None             # (an odd stride beside O in token order)
-    if want is not None:
-        got = _run(qkv, coords, spreads, None, kw, dO)
-        assert "Attention" in got[0].grad_fn.name()
-        _same(got, want)
+    # (what the library holds against an odd stride, beside O in token order or a gradient that is not dense, is refused alike)
+    for d_out in (dO, dO.transpose(1, 2).contiguous().transpose(1, 2)):
+        with general():
+            try:
+                want = _run(qkv, coords, spreads, None, kw, d_out)
+            except ValueError:
+                want = None
+        if want is None:
+            with pytest.raises(ValueError, match="code -"):
+                _run(qkv, coords, spreads, None, kw, d_out)
+        else:
+            got = _run(qkv, coords, spreads, None, kw, d_out)
+            assert "Attention" in got[0].grad_fn.name()
+            _same(got, want)
 
 
 # What has to be converted or refused is the Python functions': not taken, and the same result or error
@@ -134,6 +139,7 @@ def test_attention_that_is_not_plain(gpu, general):
             pa.geometric_attn(q, k, v, coords, s.to(gpu))
     both(q, k, v, coords, spreads, operand_dtype=torch.float16)
     both(q, k, v, coords, spreads, out_dtype=torch.bfloat16)
+    both(q, k, v, coords, spreads, betas=torch.ones_like(spreads), min_rbf=0.5, max_rbf=0.5 + 1e-12)       # (a range that is empty in fp32)
 
 
 @pytest.mark.gpu
