@@ -143,9 +143,9 @@ def _infer_layer(x, coords, mask, m):
     if nbytes == 0:
         return None
     dev = x.device
-    wqkv, bqkv = a._fused_qkv_rows()
-    params = (wqkv, bqkv, a._out_weight().contiguous(), *rest)
-    x, c, sigma = train_ops._dense(x), _f32(coords, dev), _f32(a._per_head("spread"), dev)
+    wqkv, bqkv, wo, sigma = a._infer_constants()
+    params = (wqkv, bqkv, wo, *rest)
+    x, c = train_ops._dense(x), _f32(coords, dev)
     pad = None if mask is None else _mask_bytes(mask, dev)
     out = torch.empty_like(x)
     train_ops._call("proteus_encoder_infer", dev, x, c, sigma, pad, train_ops._pointers(params), float(n1.eps), float(n2.eps), out,

@@ -513,14 +513,12 @@ class GeoAttention(nn.Module):
     # the weights: train() / eval(), .to() / .half() / .cuda() (through _apply), load_state_dict, and
     # invalidate_caches().  A write through `p.data` (e.g. `p.data.copy_(ema)`) bumps no version counter and cannot be
     # seen from here: after such a write in eval() mode call invalidate_caches() (or eval() again).
+    # They may be used on any stream (_Kept).  What a captured graph makes is not kept: it is there once the graph has run.
 
     def invalidate_caches(self):
         """Drop the constants kept from earlier inference calls.  Needed only after the parameters were changed
         behind autograd's back (writes through `.data`) while the module stayed in eval() mode."""
-        self.__dict__.pop("_head_cache", None)
-        self._wo_cache = None
-        self._qkv_cache = None
-        self._qkv_rows_cache = None
+        self.__dict__.pop("_constants", None)
 
     def train(self, mode: bool = True):
         self.invalidate_caches()
@@ -534,59 +532,80 @@ class GeoAttention(nn.Module):
         self.invalidate_caches()
         return super()._load_from_state_dict(*args, **kwargs)
 
-    def _may_keep(self, params):
-        return (not self.training) and not (torch.is_grad_enabled() and any(p.requires_grad for p in params))
+    def _kept(self, name, params, make, *more):
+        """make(), tensors that depend on `params` and `more` alone, kept across calls where they may be."""
+        if self.training or (torch.is_grad_enabled() and any(p.requires_grad for p in params)):
+            return make()
+        key = (more, tuple((p._version, p.data_ptr(), p.dtype) for p in params))
+        kept = self.__dict__.setdefault("_constants", {}).get(name)
+        if kept is not None and kept.key == key:
+            return kept.tensors_here()
+        tensors = tuple(t.detach() for t in make())
+        if not (params[0].is_cuda and torch.cuda.is_current_stream_capturing()):
+            self.__dict__.setdefault("_constants", {})[name] = _Kept(key, tensors)
+        return tensors
 
     def _per_head(self, which):
         """sigma (`spread`) or beta of the heads, as the fp32 tensor the kernel reads (kept across inference calls:
         three small launches per layer otherwise)."""
         p = self.spread_weights if which == "spread" else self.beta_weights
         fn = self.get_spreads if which == "spread" else self.get_betas
-        if not self._may_keep((p,)):
+        if self.training or torch.is_grad_enabled() and p.requires_grad:
             return fn()
-        key = (p._version, p.data_ptr(), p.dtype, self.min_spread)
-        cache = self.__dict__.setdefault("_head_cache", {})
-        if which not in cache or cache[which][0] != key:
-            cache[which] = (key, fn().detach().float().contiguous())
-        return cache[which][1]
+        return self._kept(which, (p,), lambda: (fn().float().contiguous(),), self.min_spread)[0]
+
+    def _make_out_weight(self):
+        return self.out_proj.weight.view(self.d_model, self.d_k, self.heads).permute(0, 2, 1).reshape(self.d_model, self.d_model)
 
     def _out_weight(self):
         """The output projection's weight with its input columns in (heads x d_k) order."""
-        p = self.out_proj.weight
-        keep = self._may_keep((p,))
-        key = (p._version, p.data_ptr(), p.dtype)
-        if keep and getattr(self, "_wo_cache", None) is not None and self._wo_cache[0] == key:
-            return self._wo_cache[1]
-        w_o = p.view(self.d_model, self.d_k, self.heads).permute(0, 2, 1).reshape(self.d_model, self.d_model)
-        self._wo_cache = (key, w_o.detach()) if keep else None
-        return w_o
+        return self._kept("out", (self.out_proj.weight,), lambda: (self._make_out_weight(),))[0]
 
-    def _fused_qkv_rows(self):
-        """The same fused projection with a row of d_model per output feature, [3*H*d_k, d_model], as proteus_gemm_bf16 reads it, and its bias."""
-        params = (self.q_proj, self.k_proj, self.v_proj, self.q_bias, self.k_bias, self.v_bias)
-        keep = self._may_keep(params)
-        key = tuple((p._version, p.data_ptr(), p.dtype) for p in params)
-        cache = getattr(self, "_qkv_rows_cache", None)
-        if keep and cache is not None and cache[0] == key:
-            return cache[1], cache[2]
-        w = torch.stack(params[:3]).permute(0, 1, 3, 2).reshape(3 * self.heads * self.d_k, self.d_model)
-        b = torch.stack(params[3:]).reshape(-1)
-        self._qkv_rows_cache = (key, w.detach(), b.detach()) if keep else None
-        return w, b
+    def _infer_constants(self):
+        """What a layer's inference in one call reads of this module: the fused projection with a row of d_model per output feature, [3*H*d_k, d_model], and its
+        bias, the output projection with its input columns in (heads x d_k) order, and sigma of the heads in fp32."""
+        params = (self.q_proj, self.k_proj, self.v_proj, self.q_bias, self.k_bias, self.v_bias, self.out_proj.weight, self.spread_weights)
+
+        def make():
+            w = torch.stack(params[:3]).permute(0, 1, 3, 2).reshape(3 * self.heads * self.d_k, self.d_model)
+            return w, torch.stack(params[3:6]).reshape(-1), self._make_out_weight().contiguous(), self.get_spreads().float().contiguous()
+        return self._kept("infer", params, make, self.min_spread)
 
     def _fused_qkv(self):
         """[d_model, 3*H*d_k] weight and [3*H*d_k] bias of the fused self-attention projection, from the per-head
         parameters."""
         params = (self.q_proj, self.k_proj, self.v_proj, self.q_bias, self.k_bias, self.v_bias)
-        keep = self._may_keep(params)
-        key = tuple((p._version, p.data_ptr(), p.dtype) for p in params)
-        if keep and getattr(self, "_qkv_cache", None) is not None and self._qkv_cache[0] == key:
-            return self._qkv_cache[1], self._qkv_cache[2]
-        H, dk = self.heads, self.d_k
-        w = torch.stack((self.q_proj, self.k_proj, self.v_proj)).permute(2, 0, 1, 3).reshape(self.d_model, 3 * H * dk)
-        b = torch.stack((self.q_bias, self.k_bias, self.v_bias)).reshape(-1)
-        self._qkv_cache = (key, w.detach(), b.detach()) if keep else None
-        return w, b
+
+        def make():
+            w = torch.stack(params[:3]).permute(2, 0, 1, 3).reshape(self.d_model, 3 * self.heads * self.d_k)
+            return w, torch.stack(params[3:]).reshape(-1)
+        return self._kept("qkv", params, make)
+
+
+class _Kept:
+    """Tensors made on one stream for use on any: a stream that has not used them yet waits until they are made, and the allocator hears of it, so that
+    their memory goes back only once its reads are over.  (Under capture they have been made: capturing begins on an idle device.)"""
+
+    def __init__(self, key, tensors):
+        self.key, self.tensors, self.event = key, tensors, None
+        if tensors[0].is_cuda:
+            self.device = tensors[0].device
+            self.streams = {_lib.raw_stream(self.device)}
+            self.event = torch.cuda.current_stream(self.device).record_event()
+
+    def tensors_here(self):
+        if self.event is not None:
+            stream = _lib.raw_stream(self.device)
+            if stream not in self.streams and not torch.cuda.is_current_stream_capturing():
+                current = torch.cuda.current_stream(self.device)
+                current.wait_event(self.event)
+                for t in self.tensors:
+                    t.record_stream(current)
+                self.streams.add(stream)
+        return self.tensors
+
+    def __reduce__(self):                    # (a copied or stored module makes its own)
+        return type(None), ()
 
 
 from . import train_ops  # noqa: E402  (it uses the operators above)

@@ -140,6 +140,47 @@ def test_layer_follows_its_weights(gpu):
         assert torch.equal(layer(x, x, x, coords, mask), other(x, x, x, coords, mask)) and torch.equal(x, keep)
 
 
+# What the module keeps between calls, made on one stream and read on another: the other waits until it is there, and it stays until that read is over; what a capture
+# makes is not kept
+@pytest.mark.gpu
+@pytest.mark.parametrize("one_call", [True, False])
+def test_kept_constants_on_other_streams(gpu, monkeypatch, one_call):
+    layer, x, coords, mask = _layer(gpu, 2, 70, 2, 32, 104)
+    if not one_call:
+        monkeypatch.setattr(encoder, "_infer_layer", lambda *a: None)
+    run = lambda m: m(x, x, x, coords, mask)
+    with torch.no_grad():
+        want = run(copy.deepcopy(layer))
+        a, b = torch.cuda.Stream(), torch.cuda.Stream()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(a):
+            torch.cuda._sleep(20_000_000)
+            first = run(layer)
+        kept = [t for k in layer.attn._constants.values() for t in k.tensors]
+        with torch.cuda.stream(b):
+            second = run(layer)                              # (waits for the sleep of the other stream)
+            torch.cuda._sleep(20_000_000)
+            third = run(layer)
+        at = {t.data_ptr() for t in kept}
+        shapes = [(t.shape, t.dtype) for t in kept]
+        del kept
+        layer.attn.invalidate_caches()
+        with torch.cuda.stream(a):                           # (whatever is given back to this stream's memory is written over)
+            over = [torch.full(s, float("nan"), dtype=d, device=gpu) for s, d in shapes for _ in range(4)]
+        assert not any(t.data_ptr() in at for t in over)
+        torch.cuda.synchronize()
+        assert torch.equal(first, want) and torch.equal(second, want) and torch.equal(third, want)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            captured = run(layer)
+        assert not layer.attn._constants
+        for _ in range(3):
+            captured.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(captured, want) and torch.equal(run(layer), want)
+
+
 @pytest.mark.gpu
 def test_sum_in_front_of_the_layers(gpu):
     a, b = torch.randn(3, 67, 40, device=gpu), torch.randn(3, 67, 40, device=gpu).bfloat16()

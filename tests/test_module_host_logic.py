@@ -1,7 +1,9 @@
 """Host-side logic of the modules that needs no GPU: the constants GeoAttention keeps across inference calls, and the
 choice between writing the fused projection's gradient in place and through buffers of its own, and what the training functions
 hand to kernels."""
+import copy
 import importlib
+import pickle
 import types
 
 import pytest
@@ -42,6 +44,9 @@ def test_kept_constants_follow_every_way_the_weights_are_known_to_change():
         m.double()
         assert m._fused_qkv()[0].dtype == torch.float64 and m._out_weight().dtype == torch.float64
         m.float()
+        # a copy makes its own
+        kept, other = m._out_weight(), copy.deepcopy(m)
+        assert not same(other._out_weight(), kept) and torch.equal(other._out_weight(), kept) and pickle.loads(pickle.dumps(m))._constants == {"out": None}
 
 
 def test_writes_through_data_need_invalidate_caches_only_in_eval_mode():
