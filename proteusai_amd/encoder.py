@@ -117,7 +117,8 @@ def _infer_layer(x, coords, mask, m):
     plain = train_ops.plain_module
     if not (plain(a, GeoAttention) and plain(n1, nn.LayerNorm) and plain(n2, nn.LayerNorm) and plain(f, MLP) and f.act is F.gelu and not f.hidden_proj
             and train_ops.inactive_dropout(m.dropout) and train_ops.inactive_dropout(f.in_dropout) and plain(f.in_proj, nn.Linear) and plain(f.out_proj, nn.Linear)
-            and plain(a.out_proj, nn.Linear) and "_residual_norm" not in m.__dict__ and a.out_proj.bias is None):
+            and plain(a.out_proj, nn.Linear) and "_residual_norm" not in m.__dict__ and a.out_proj.bias is None
+            and "get_spreads" not in a.__dict__ and isinstance(a.min_spread, (int, float))):       # (a sigma of another shape is the operator's to refuse)
         return None
     H, dk, dm, l1, l2 = a.heads, a.d_k, a.d_model, f.in_proj, f.out_proj
     rest = (n1.weight, n1.bias, l1.weight, l1.bias, l2.weight, l2.bias, n2.weight, n2.bias)
@@ -130,7 +131,7 @@ def _infer_layer(x, coords, mask, m):
     w, b = (H, dm, dk), (H, dk)
     if (tuple(p.shape for p in rest + attn) != ((dm,), (dm,), (hidden, dm), (hidden,), (dm, hidden), (dm,), (dm,), (dm,), w, w, w, b, b, b, (dm, dm))
             or a.legacy_logits or a.operand_dtype not in (None, torch.bfloat16) or x.dim() != 3 or x.shape[2] != dm or x.numel() == 0
-            or a.spread_weights.shape != (H,) or not (n1.eps >= 0.0 and n2.eps >= 0.0)
+            or type(a.spread_weights) not in train_ops._PLAIN_TYPES or a.spread_weights.shape != (H,) or a.spread_weights.device != x.device or not (n1.eps >= 0.0 and n2.eps >= 0.0)
             or tuple(coords.shape) != (*x.shape[:2], 3) or (mask is not None and tuple(mask.shape) != tuple(x.shape[:2]))
             or not train_ops.unobserved() or not train_ops.aligned(*rest)):
         return None

@@ -550,7 +550,7 @@ class GeoAttention(nn.Module):
         three small launches per layer otherwise)."""
         p = self.spread_weights if which == "spread" else self.beta_weights
         fn = self.get_spreads if which == "spread" else self.get_betas
-        if self.training or torch.is_grad_enabled() and p.requires_grad:
+        if self.training or (torch.is_grad_enabled() and p.requires_grad) or not isinstance(self.min_spread, (int, float)):
             return fn()
         return self._kept(which, (p,), lambda: (fn().float().contiguous(),), self.min_spread)[0]
 

@@ -118,6 +118,16 @@ def test_what_the_call_does_not_take(gpu):
         layer.eval()
         layer.ffn.in_proj.bias = None
         assert not take()
+    with torch.no_grad(), pytest.MonkeyPatch.context() as mp:                                             # sigma that the kernel would read past its end, or on the host
+        for name, value in (("get_spreads", lambda: torch.full((1,), 5.0, device=gpu)), ("get_spreads", lambda: torch.full((2,), 5.0)), ("min_spread", torch.full((2, 1), 2.0, device=gpu))):
+            layer, x, coords, mask = _layer(gpu, 2, 70, 2, 32, 104)
+            mp.setattr(layer.attn, name, value)
+            assert not take()
+            if name == "get_spreads" and value().numel() == 2:
+                assert bool(layer(x, x, x, coords, mask)[~mask].isfinite().all())
+            else:
+                with pytest.raises(AssertionError, match="spreads"):
+                    layer(x, x, x, coords, mask)
     wide, y, at, _ = _layer(gpu, 1, 8200, 32, 32, 64)
     with torch.no_grad():                                                                                # products that the library does faster
         assert encoder._infer_layer(y, at, None, wide) is None and encoder._infer_layer(y[:, :8192], at[:, :8192], None, wide) is not None
