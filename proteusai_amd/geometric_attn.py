@@ -568,7 +568,7 @@ class GeoAttention(nn.Module):
 
         def make():
             w = torch.stack(params[:3]).permute(0, 1, 3, 2).reshape(3 * self.heads * self.d_k, self.d_model)
-            return w, torch.stack(params[3:6]).reshape(-1), self._make_out_weight().contiguous(), self.get_spreads().float().contiguous()
+            return w, torch.stack(params[3:6]).reshape(-1), train_ops._dense(self._make_out_weight()), self.get_spreads().float().contiguous()
         return self._kept("infer", params, make, self.min_spread)
 
     def _fused_qkv(self):

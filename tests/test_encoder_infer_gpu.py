@@ -135,6 +135,18 @@ def test_what_the_call_does_not_take(gpu):
         layer(x, x, x, coords[:, :69], mask)                                                             # refused as before
 
 
+# One head: its output projection is read where it lies, which need not be on 16 bytes (a parameter cut out of a flat buffer)
+@pytest.mark.gpu
+def test_one_head_with_an_output_projection_off_16_bytes(gpu):
+    layer, x, coords, mask = _layer(gpu, 2, 70, 1, 64, 104)
+    with torch.no_grad():
+        want = layer(x, x, x, coords, mask)
+        flat = torch.empty(64 * 64 + 8, dtype=torch.bfloat16, device=gpu)
+        w = flat[1:64 * 64 + 1].view(64, 64).copy_(layer.attn.out_proj.weight)
+        layer.attn.out_proj.weight = torch.nn.Parameter(w)
+        assert layer.attn.out_proj.weight.data_ptr() % 16 == 2 and torch.equal(layer(x, x, x, coords, mask), want)
+
+
 # new weights, in place and by a state dict, are seen; x as it was
 @pytest.mark.gpu
 def test_layer_follows_its_weights(gpu):
