@@ -113,6 +113,8 @@ def _infer_layer(x, coords, mask, m):
     library, or None where its parts go their own ways."""
     if x.dtype != torch.bfloat16 or not x.is_cuda or type(x) is not torch.Tensor or torch.is_autocast_enabled("cuda"):
         return None
+    if torch.is_grad_enabled() and (x.requires_grad or getattr(getattr(m.attn_norm, "weight", None), "requires_grad", False)):
+        return None                                                         # (training, before the closer look, which takes 15 us of host time)
     a, n1, f, n2 = m.attn, m.attn_norm, m.ffn, m.ffn_norm
     plain = train_ops.plain_module
     if not (plain(a, GeoAttention) and plain(n1, nn.LayerNorm) and plain(n2, nn.LayerNorm) and plain(f, MLP) and f.act is F.gelu and not f.hidden_proj

@@ -104,7 +104,14 @@ def test_layer_is_as_near_to_its_weights_as_its_parts(gpu, Z, N, H, dk, hidden, 
 def test_what_the_call_does_not_take(gpu):
     layer, x, coords, mask = _layer(gpu, 2, 70, 2, 32, 104)
     take = lambda **k: encoder._infer_layer(k.get("x", x), k.get("coords", coords), k.get("mask", mask), layer) is not None
-    assert not take()                                                                                    # gradients are recorded
+    with pytest.MonkeyPatch.context() as mp:                                                             # gradients are recorded: told before the closer look
+        looked = []
+        mp.setattr(train_ops, "plain_module", lambda *a: looked.append(a))
+        assert not take() and not take(x=x.clone().requires_grad_()) and not looked
+        layer.attn_norm.weight.requires_grad_(False)
+        assert not take() and looked
+    assert not take()
+    layer.attn_norm.weight.requires_grad_(True)
     with torch.no_grad():
         assert take() and take(mask=None) and take(x=x.transpose(0, 1).contiguous().transpose(0, 1))
         assert not take(x=x.float()) and not take(mask=mask[:1]) and not take(coords=coords[:, :69]) and not take(x=x[:, :0], coords=coords[:, :0], mask=None)
