@@ -90,35 +90,33 @@ template <> __device__ __forceinline__ int tile_swizzle<128>(int r) { return ((r
 // ---- padded batches handed out longest sequence first ----
 constexpr int ATTN_LPT_MAX_Z = 64;
 
-// Is a batch's mask read 16 bytes at a time?  (A piece then lies in at most two sequences.)
-__device__ __forceinline__ bool mask_in_pieces(const uint8_t* mask, const int N) { return N >= 16 && ((uintptr_t)mask & 15) == 0; }
-
-// lens[z], zero before: 1 + index of the last unpadded token of sequence z of Z.  Called by all threads of a workgroup.
+// lens[z], zero before: 1 + index of the last unpadded token of sequence z of Z.  Called by all threads of a workgroup.  From 16 tokens on the mask is read 16 bytes at a time
+// wherever it lies (a piece is then in at most two sequences), and byte by byte in front of the first multiple of 16 and behind the last: what a launch makes of the lengths
+// does not depend on the mask's address.
 template <int THREADS>
 __device__ __forceinline__ void sequence_lengths(const uint8_t* __restrict__ mask, const int Z, const int N, int* lens)
 {
-    const int total = Z * N;
-    int from = 0;
-    if (mask_in_pieces(mask, N)) {
-        const int pieces = total >> 4;
-        from = pieces << 4;
+    const int total = Z * N, lead = min((int)(-(uintptr_t)mask & 15), total), pieces = N >= 16 ? (total - lead) >> 4 : 0;
 #pragma unroll 4
-        for (int p = (int)threadIdx.x; p < pieces; p += THREADS) {
-            const uint4 m16 = *reinterpret_cast<const uint4*>(mask + (size_t)p * 16);
-            const unsigned w[4] = {m16.x, m16.y, m16.z, m16.w};
-            unsigned usable = 0;                                  // bit e: byte e is zero
+    for (int p = (int)threadIdx.x; p < pieces; p += THREADS) {
+        const int at = lead + 16 * p;
+        const uint4 m16 = *reinterpret_cast<const uint4*>(mask + at);
+        const unsigned w[4] = {m16.x, m16.y, m16.z, m16.w};
+        unsigned usable = 0;                                  // bit e: byte e is zero
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const unsigned zero = ~(((w[e] & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w[e]) & 0x80808080u;       // (bit 7 of a byte that is zero)
-                usable |= (((zero >> 7) & 1u) | ((zero >> 14) & 2u) | ((zero >> 21) & 4u) | (zero >> 28)) << (4 * e);
-            }
-            const int z = 16 * p / N, here = (z + 1) * N - 16 * p;                   // bytes of the piece in sequence z, the others in z + 1
-            const unsigned low = here >= 16 ? usable : usable & ((1u << here) - 1u), high = usable ^ low;
-            if (low)  atomicMax(&lens[z], 16 * p - z * N + 32 - __builtin_clz(low));
-            if (high) atomicMax(&lens[z + 1], 32 - __builtin_clz(high) - here);
+        for (int e = 0; e < 4; ++e) {
+            const unsigned zero = ~(((w[e] & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w[e]) & 0x80808080u;       // (bit 7 of a byte that is zero)
+            usable |= (((zero >> 7) & 1u) | ((zero >> 14) & 2u) | ((zero >> 21) & 4u) | (zero >> 28)) << (4 * e);
         }
+        const int z = at / N, here = (z + 1) * N - at;                               // bytes of the piece in sequence z, the others in z + 1
+        const unsigned low = here >= 16 ? usable : usable & ((1u << here) - 1u), high = usable ^ low;
+        if (low)  atomicMax(&lens[z], at - z * N + 32 - __builtin_clz(low));
+        if (high) atomicMax(&lens[z + 1], 32 - __builtin_clz(high) - here);
     }
-    for (int j = from + (int)threadIdx.x; j < total; j += THREADS) if (!mask[j]) atomicMax(&lens[j / N], j % N + 1);
+    for (int i = (int)threadIdx.x; i < total - 16 * pieces; i += THREADS) {
+        const int j = i < lead ? i : i + 16 * pieces;
+        if (!mask[j]) atomicMax(&lens[j / N], j % N + 1);
+    }
 }
 
 // Workgroup `block_id` of n_tiles * Z * H takes the block_id-th item of the list "live tiles (of OWN tokens) of the longest sequence, tile-major, the heads of a tile

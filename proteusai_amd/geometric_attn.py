@@ -85,6 +85,9 @@ def geo_attn(Q, K, V, coords, sigma, key_padding_mask=None, return_lse: bool = F
     token_major_out=True returns O as a [Z,H,N,d] view of memory laid out [Z,N,H,d] (what a following
     projection over the concatenated heads reads without a copy).
 
+    The same call gives the same bits.  The order in which a row is summed up follows from the shape and, in a padded
+    batch, from the lengths of all its sequences: beside others a sequence may be rounded differently.
+
     With `betas` [H] the logits are those of the reference's kernel instead,
     S + beta_h*(2(rbf-min_rbf)/(max_rbf-min_rbf)-1)*|S| with pairs whose rbf lies outside
     [min_rbf, max_rbf] masked (old/old_scripts/attn/geometric_attn.py:193-201).

@@ -177,8 +177,8 @@ def test_padded_batches_handed_out_longest_first(gpu, H):
     compare(gpu_grads(gpu, *a), reference_grads(*a), mask, "66 items")
 
 
-# Ranked batches against their sequences one by one (which nothing ranks): lengths off 16, whose pieces of 16 mask bytes lie in two sequences, a mask that is read
-# byte by byte, sequences without a token, with one, of equal length and with holes, as many as are ranked, and the first counts of workgroups that are not
+# Ranked batches against their sequences one by one (which nothing ranks): lengths off 16, whose pieces of 16 mask bytes lie in two sequences, a mask off 16
+# bytes, sequences without a token, with one, of equal length and with holes, as many as are ranked, and the first counts of workgroups that are not
 @pytest.mark.parametrize("Z,H,N,off", [(9, 2, 517, 0), (9, 2, 517, 3), (50, 1, 530, 0), (64, 1, 512, 0), (17, 2, 1507, 0), (2, 3, 1500, 0), (5, 8, 500, 0), (16, 8, 513, 0)])
 def test_ranked_batches_equal_their_sequences(gpu, Z, H, N, off):
     g = torch.Generator(device=gpu).manual_seed(N + Z)
