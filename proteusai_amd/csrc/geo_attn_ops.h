@@ -119,6 +119,13 @@ __device__ __forceinline__ void sequence_lengths(const uint8_t* __restrict__ mas
     }
 }
 
+// Is token `at` of some sequence padded?  (At most 64 sequences; the same for every wave.)
+__device__ __forceinline__ bool some_padded_at(const uint8_t* __restrict__ mask, const int Z, const int N, const int at)
+{
+    const int lane = threadIdx.x & 63;
+    return __builtin_amdgcn_ballot_w64(lane < Z && mask[(size_t)min(lane, Z - 1) * N + at] != 0) != 0;
+}
+
 // Workgroup `block_id` of n_tiles * Z * H takes the block_id-th item of the list "live tiles (of OWN tokens) of the longest sequence, tile-major, the heads of a tile
 // side by side, those of the next one, ..., then the dead tiles"; tile and zh = (sequence, head) of it.  lens: LDS, left with 1 + index of the last unpadded
 // token of every sequence (KNOWN: they are there).  Called by all threads of a workgroup.

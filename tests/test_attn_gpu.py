@@ -400,8 +400,9 @@ def test_legacy_logits(gpu):
 # Ranked padded batches (more than 512 workgroups of 128 queries, at most 24 sequences) against the sequences by themselves, and to the bit against the same mask off 16 bytes, of which
 # neither the order nor the split may make anything: sequences without a token, with one, of equal length, with holes, as many as are ranked and one more, lengths whose
 # pieces of 16 mask bytes lie in two sequences
-# (8 x 8 x 1023 and 16 x 4 x 960: at most a round of 128-query workgroups, live ones of 64 queries few enough for two waves to a query block; 4 x 16 x 1000: not)
-@pytest.mark.parametrize("Z,H,N,d", [(9, 16, 517, 64), (24, 8, 400, 64), (24, 10, 400, 32), (25, 8, 400, 64), (17, 8, 515, 32), (3, 45, 513, 32), (8, 8, 1023, 64), (16, 4, 960, 32), (4, 16, 1000, 64), (13, 5, 901, 64)])
+# (8 x 8 x 1023 and 16 x 4 x 960: at most a round of 128-query workgroups, live ones of 64 queries few enough for two waves to a query block; 7 x 9 x 1000: not;
+# 4 x 16 x 1000: lengths that are nearly alike)
+@pytest.mark.parametrize("Z,H,N,d", [(9, 16, 517, 64), (24, 8, 400, 64), (24, 10, 400, 32), (25, 8, 400, 64), (17, 8, 515, 32), (3, 45, 513, 32), (8, 8, 1023, 64), (16, 4, 960, 32), (4, 16, 1000, 64), (7, 9, 1000, 64), (13, 5, 901, 64)])
 def test_ranked_batches_equal_their_sequences_wherever_the_mask_lies(gpu, Z, H, N, d):
     g = torch.Generator(device=gpu).manual_seed(N + Z)
     Q, K, V = (torch.randn(Z, H, N, d, generator=g, device=gpu).bfloat16() for _ in range(3))
@@ -412,6 +413,8 @@ def test_ranked_batches_equal_their_sequences_wherever_the_mask_lies(gpu, Z, H, 
         lens = [N - 1, 0, N]
     if Z == 4:
         lens = [N, N - 1, N - 70, N]
+    if Z == 7:
+        lens = [N, N - 1, N - 170, N, N - 168, N, N]
     buf = torch.zeros(Z * N + 3, dtype=torch.bool, device=gpu)
     apart = buf[3:].view(Z, N)
     for z, n in enumerate(lens):
