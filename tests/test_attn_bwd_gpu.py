@@ -178,8 +178,10 @@ def test_padded_batches_handed_out_longest_first(gpu, H):
 
 
 # Ranked batches against their sequences one by one (which nothing ranks): lengths off 16, whose pieces of 16 mask bytes lie in two sequences, a mask off 16
-# bytes, sequences without a token, with one, of equal length and with holes, as many as are ranked, and the first counts of workgroups that are not
-@pytest.mark.parametrize("Z,H,N,off", [(9, 2, 517, 0), (9, 2, 517, 3), (50, 1, 530, 0), (64, 1, 512, 0), (17, 2, 1507, 0), (2, 3, 1500, 0), (5, 8, 500, 0), (16, 8, 513, 0)])
+# bytes, sequences without a token, with one, of equal length and with holes, as many as are ranked; the second row: too many workgroups of too short sequences, more sequences
+# than a single round is ranked for, which are not
+@pytest.mark.parametrize("Z,H,N,off", [(9, 2, 517, 0), (9, 2, 517, 3), (50, 6, 530, 0), (64, 1, 1504, 0), (64, 1, 1501, 9), (17, 2, 1507, 0), (2, 3, 1500, 0), (5, 8, 500, 0), (12, 7, 513, 0), (64, 1, 512, 0),
+                                         (16, 8, 513, 0), (50, 1, 530, 0)])
 def test_ranked_batches_equal_their_sequences(gpu, Z, H, N, off):
     g = torch.Generator(device=gpu).manual_seed(N + Z)
     Q, K, V = (torch.randn(Z, H, N, 32, generator=g, device=gpu).bfloat16() for _ in range(3))
