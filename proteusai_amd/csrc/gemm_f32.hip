@@ -605,7 +605,8 @@ void gemm_f32_rows_sum_kernel(const PendingSums sums)
 int wide_groups(int M, int N, int K, int epilogue)
 {
     if (K < 512) return 0;
-    const int64_t tiles = ((M + (int64_t)WT - 1) / WT) * ((N + (int64_t)WT - 1) / WT);
+    const int64_t tiles = ((M + (int64_t)WT - 1) / WT) * ((N + (int64_t)WT - 1) / WT), small = ((M + (int64_t)GT - 1) / GT) * ((N + (int64_t)GT - 1) / GT);
+    if (5 * small < 16 * tiles) return 0;
     if (tiles > 256) return tiles >= (epilogue == PROTEUS_GEMM_GELU_GRAD ? 704 : 448) ? 1 : 0;
     return tiles >= (epilogue == PROTEUS_GEMM_GELU_GRAD || epilogue == PROTEUS_GEMM_GELU ? 240 : 160) ? 2 : 0;
 }

@@ -33,10 +33,10 @@ def test_product_against_float64(gpu, form, M, N, K):
     assert torch.equal(got, train_ops._product(form, A, B))
 
 
-# Tiles of 128 x 128: from 160 of them and K = 512 on with two groups, from 448 on with one; edges of the tiles and of the steps that the groups share out
+# Tiles of 128 x 128: from 160 of them and K = 512 on with two groups, from 448 on with one; edges of the tiles and of the steps that the groups share out (the last two: half empty, tiles of 64 x 64)
 @pytest.mark.gpu
 @pytest.mark.parametrize("form", [NN, NT])
-@pytest.mark.parametrize("M,N,K", [(1920, 1280, 512), (2047, 1276, 516), (1921, 1284, 532), (129, 10244, 548), (20481, 4, 512), (2945, 2436, 512), (2817, 2492, 540)])
+@pytest.mark.parametrize("M,N,K", [(1920, 1280, 512), (2047, 1276, 516), (1921, 1284, 532), (257, 10244, 548), (20481, 116, 512), (2945, 2436, 512), (2817, 2492, 540), (129, 10244, 548), (20481, 4, 512)])
 def test_wide_tiles_against_float64(gpu, form, M, N, K):
     A, B, want, mass = _operands(form, M, N, K, gpu)
     got = train_ops._product(form, A, B)
