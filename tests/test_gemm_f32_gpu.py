@@ -109,9 +109,9 @@ def test_epilogues(gpu, M):
     assert torch.equal(_epilogue(NT, _lib.GEMM_ADD, A, B, bias, h), train_ops._product(NT, A, B, bias) + h)
 
 
-# (tiles of 128 x 128, with two groups and with one)
+# (tiles of 128 x 128, with two groups; with one where the epilogue reads no matrix; with one)
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N", [(2049, 1804), (3457, 3204)])
+@pytest.mark.parametrize("M,N", [(2049, 1804), (3457, 3204), (3457, 4228)])
 def test_epilogues_of_wide_tiles(gpu, M, N):
     A, B, want, mass = _operands(NT, M, N, 524, gpu)
     Bt, bias, h = B.t().contiguous(), torch.randn(N, device=gpu), torch.randn(M, N, device=gpu)
