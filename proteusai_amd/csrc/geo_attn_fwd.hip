@@ -210,13 +210,15 @@ __device__ __forceinline__ void gb_merge_parts(const SlotOf& slot_of, const int 
             const bool row_ok = l > 0.f && !(mz && mz[qi]);
             const float inv_l = row_ok ? 1.0f / l : 0.f;
             const size_t orow = o_at + (size_t)qi * (size_t)st.o[2];
+            ga_rows(st.o16, [&](auto type) {
 #pragma unroll
-            for (int dt = 0; dt < 2; ++dt)
+                for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
-                for (int gq = 0; gq < 4; ++gq)
-                    ga_put(O, orow + dt * 32 + 8 * gq + 4 * half,
-                           make_float4(acc[dt * 16 + 4 * gq] * inv_l, acc[dt * 16 + 4 * gq + 1] * inv_l,
-                                       acc[dt * 16 + 4 * gq + 2] * inv_l, acc[dt * 16 + 4 * gq + 3] * inv_l), st.o16);
+                    for (int gq = 0; gq < 4; ++gq)
+                        ga_put<decltype(type)::value>(O, orow + dt * 32 + 8 * gq + 4 * half,
+                                                      make_float4(acc[dt * 16 + 4 * gq] * inv_l, acc[dt * 16 + 4 * gq + 1] * inv_l,
+                                                                  acc[dt * 16 + 4 * gq + 2] * inv_l, acc[dt * 16 + 4 * gq + 3] * inv_l));
+            });
             if (L && half == 0) L[(size_t)zh * N + qi] = row_ok ? (M + __log2f(l)) * 0.69314718055994531f : -INFINITY;
         }
     }
@@ -321,7 +323,7 @@ void geo_attn_fwd_balanced_kernel(const uint16_t* __restrict__ Q, const uint16_t
         for (int ql = tid >> 4; ql < GA_THREADS; ql += GA_THREADS / 16) {
             const int qi = qt * GA_THREADS + ql;
             if (qi >= N) break;
-            ga_put(O, o_at + (size_t)qi * (size_t)st.o[2] + 4 * chunk, make_float4(0.f, 0.f, 0.f, 0.f), st.o16);
+            ga_rows(st.o16, [&](auto type) { ga_put<decltype(type)::value>(O, o_at + (size_t)qi * (size_t)st.o[2] + 4 * chunk, make_float4(0.f, 0.f, 0.f, 0.f)); });
             if (L && chunk == 0) L[((size_t)z * H + h) * N + qi] = -INFINITY;
         }
     }
@@ -481,7 +483,7 @@ void geo_attn_fwd_split_kernel(const uint16_t* __restrict__ Q, const uint16_t* _
         for (int ql = tid >> 4; ql < GA_THREADS; ql += GA_THREADS / 16) {
             const int qi = qt * GA_THREADS + ql;
             if (qi >= N) break;
-            ga_put(O, o_at + (size_t)qi * (size_t)st.o[2] + 4 * chunk, make_float4(0.f, 0.f, 0.f, 0.f), st.o16);
+            ga_rows(st.o16, [&](auto type) { ga_put<decltype(type)::value>(O, o_at + (size_t)qi * (size_t)st.o[2] + 4 * chunk, make_float4(0.f, 0.f, 0.f, 0.f)); });
             if (L && chunk == 0) L[((size_t)z * H + h) * N + qi] = -INFINITY;
         }
     }
