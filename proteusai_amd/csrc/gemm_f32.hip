@@ -595,27 +595,29 @@ void gemm_f32_rows_sum_kernel(const PendingSums sums)
     finish_rows<4>(g, m0, n0, e0, v);
 }
 
-// Groups of gemm_f32_wide_kernel, 0: tiles of 64 x 64.  Two while its tiles leave a compute unit one each and few idle, one from where the rounds of its workgroups are full enough: three share a compute
-// unit, two where the epilogue keeps a matrix in registers (just over a round of 512 those lose).  Not for a short K; later where the epilogue is long, since nothing runs under that of a lone workgroup.
-// Us, M x N x K (tiles), 64 x 64 / 128 x 128.  Two groups: 1536 x 1536 x 512 (144) 25.2 / 25.7, 2048 x 1280 x 512 (160) 25.8 / 26.0, 5000 x 512 x 2048 (160) 88 / 72, 4096 x 768 x 768 (192) 39 / 35, 6400 x 512 x 512
-// (200) 31.8 / 27.7, 4096 x 1024 x 1024 (256) 64 / 50, 8192 x 512 x 2048 (256) 123 / 90; 4096 x 512 x 2048 (128) 59 / 70; with GELU and with its derivative 1536 x 2048 x 512 (192) 32.0 / 32.0 and 31.9 / 33.3, 1792 x
-// 2048 (224) 37.3 / 33.5 and 38.0 / 34.5, 2048 x 2048 (256) 39.1 / 35.2 and 39.6 / 36.3; x 256 before 4096 x 768 (192) 15.9 / 16.6.  One group: 3072 x 1536 x 512 (288) 41 / 50, 4096 x 1536 (384) 50 / 53,
-// 5000 x 1536 (480) 62 / 56, 18000 x 512 x 512 (564) 70.5 / 69.5, 8192 x 1536 (768) 92 / 77, 16384 x 512 x 2048 (512) 234 / 182; GELU 3584 x 2048 x 512 (448) 64.3 / 64.3, 4600 x 2048 (576) 81.0 / 82.8, 5632 x 2048 (704) 97 / 88,
-// 8192 x 2048 (1024) 138 / 119; a matrix added 14400 x 512 x 2048 (452) 219 / 183, 16384 x 512 x 2048 (512) 230 / 191, 18000 x 512 x 512 (564) 70 / 85, 20000 x 512 x 2048 (628) 286 / 290, 24000 x 512 x 512 (752) 90 / 89,
-// x 2048 344 / 309; GELU's derivative 4096 x 2048 x 512 (512) 72 / 72, 5632 x 2048 (704) 98 / 107, 6700 x 2048 (848) 119 / 128, 7200 x 2048 (912) 128 / 132, 3600 x 4096 x 1024 (928) 229 / 213, 8192 x 2048 x 512 (1024)
-// 138 / 133, 9000 x 2048 (1136) 154 / 163, 10000 x 2048 (1264) 169 / 166, 16384 x 2048 (2048) 279 / 272.
-// And only where a fifth of the tiles' area at most lies outside (counted in tiles of 64): 20480 x 64 x 512 17 / 24, 30000 x 64 x 2048 60 / 77, 65536 x 64 x 512 37 / 53, 129 x 10244 x 512 19 / 27, 40000 x 192 x 512
-// 63 / 66 and with a matrix added 61 / 79, 30000 x 320 x 512 76 / 71.
+// Groups of gemm_f32_wide_kernel, 0: tiles of 64 x 64.  Us, M x N x K (tiles of 128 x 128), 64 x 64 / 128 x 128.
+// Two groups while the tiles leave a compute unit one each and few idle, later where the epilogue is long, since nothing runs under that of a lone workgroup: 1536 x 1536 x 512 (144) 25.2 / 25.7, 2048 x 1280
+// x 512 (160) 25.8 / 26.0, 5000 x 512 x 2048 (160) 88 / 72, 4096 x 768 x 768 (192) 39 / 35, 6400 x 512 x 512 (200) 31.8 / 27.7, 4096 x 1024 x 1024 (256) 64 / 50, 8192 x 512 x 2048 (256) 123 / 90; 4096 x 512 x 2048 (128)
+// 59 / 70; with GELU and with its derivative 1536 x 2048 x 512 (192) 32.0 / 32.0 and 31.9 / 33.3, 1792 x 2048 (224) 37.3 / 33.5 and 38.0 / 34.5, 2048 x 2048 (256) 39.1 / 35.2 and 39.6 / 36.3.
+// One group where there are more tiles of 64 x 64 than the chip holds at once (six per compute unit): 4096 x 1536 x 512 (384) 50 / 53, 4480 x 1536 (420) 57 / 55, 7000 x 876 x 884 (385) 103 / 79, 16384 x 512 x 2048 (512)
+// 234 / 182, 8192 x 1536 x 512 (768) 92 / 77; GELU 3584 x 2048 x 512 (448) 64.3 / 64.3, 4600 x 2048 (576) 81.0 / 82.8, 5632 x 2048 (704) 97 / 88, 8192 x 2048 (1024) 138 / 119.
+// Where the epilogue reads a matrix, which it keeps in registers, only two workgroups instead of three share a compute unit, and rounds of 512 that end nearly empty lose: a matrix added 14400 x 512 x 2048 (452)
+// 219 / 183, 18000 x 512 x 512 (564) 70 / 85, 20000 x 512 x 2048 (628) 286 / 290, 24000 x 512 x 512 (752) 90 / 89, x 2048 344 / 309, 16000 x 768 x 768 (750) 130 / 121, 32768 x 512 x 512 (1024) 120 / 116, 11000 x 1536 x 512
+// (1032) 10 % more; GELU's derivative 4096 x 2048 x 512 (512) 72 / 72, 2048 x 4096 x 1024 (512) 131 / 120, 5632 x 2048 x 512 (704) 98 / 107, 7200 x 2048 (912) 128 / 132, 3600 x 4096 x 1024 (928) 229 / 213, 8192 x 2048 x 512
+// (1024) 138 / 133, 9000 x 2048 (1136) 154 / 163, 10000 x 2048 (1264) 169 / 166, 16384 x 2048 (2048) 279 / 272.
+// Not for a short K: 13000 x 512 x 256 and 4992 x 1536 x 256 3 to 9 % more.  And only where a fifth of the tiles' area at most lies outside (counted in tiles of 64): 20480 x 64 x 512 17 / 24, 30000 x 64 x 2048 60 / 77, 65536 x
+// 64 x 512 37 / 53, 129 x 10244 x 512 19 / 27, 40000 x 192 x 512 63 / 66 and with a matrix added 61 / 79, 30000 x 320 x 512 76 / 71.
 int wide_groups(int M, int N, int K, int epilogue)
 {
     if (K < 512) return 0;
     const int64_t tiles = ((M + (int64_t)WT - 1) / WT) * ((N + (int64_t)WT - 1) / WT), small = ((M + (int64_t)GT - 1) / GT) * ((N + (int64_t)GT - 1) / GT);
     if (5 * small < 16 * tiles) return 0;
-    if (tiles > 256) {
-        if (epilogue == PROTEUS_GEMM_ADD && tiles > 512 && tiles < 730) return 0;
-        return tiles >= (epilogue == PROTEUS_GEMM_GELU_GRAD ? 900 : 448) ? 1 : 0;
-    }
-    return tiles >= (epilogue == PROTEUS_GEMM_GELU_GRAD || epilogue == PROTEUS_GEMM_GELU ? 216 : 160) ? 2 : 0;
+    const bool grad = epilogue == PROTEUS_GEMM_GELU_GRAD, add = epilogue == PROTEUS_GEMM_ADD;
+    if (tiles <= 256) return tiles >= (grad || epilogue == PROTEUS_GEMM_GELU ? 216 : 160) ? 2 : 0;
+    if (small <= 6 * 256) return 0;
+    if (!grad && !add) return 1;
+    const double filled = (double)tiles / (double)((tiles + 511) / 512 * 512);
+    return filled >= (add ? 0.9 : 0.95) || (K >= (add ? 768 : 1024) && filled >= 0.7) || (tiles > 1200 && filled >= 0.8) ? 1 : 0;
 }
 
 template <bool AK, bool BK, int EPI>

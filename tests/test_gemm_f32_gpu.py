@@ -33,7 +33,7 @@ def test_product_against_float64(gpu, form, M, N, K):
     assert torch.equal(got, train_ops._product(form, A, B))
 
 
-# Tiles of 128 x 128: from 160 of them and K = 512 on with two groups, from 448 on with one; edges of the tiles and of the steps that the groups share out (the last two: half empty, tiles of 64 x 64)
+# Tiles of 128 x 128: from 160 of them and K = 512 on with two groups, with one from where those of 64 x 64 are more than 1536; edges of the tiles and of the steps that the groups share out (the last two: half empty, tiles of 64 x 64)
 @pytest.mark.gpu
 @pytest.mark.parametrize("form", [NN, NT])
 @pytest.mark.parametrize("M,N,K", [(1920, 1280, 512), (2047, 1276, 516), (1921, 1284, 532), (257, 10244, 548), (20481, 116, 512), (2945, 2436, 512), (2817, 2492, 540), (129, 10244, 548), (20481, 4, 512)])
@@ -109,9 +109,9 @@ def test_epilogues(gpu, M):
     assert torch.equal(_epilogue(NT, _lib.GEMM_ADD, A, B, bias, h), train_ops._product(NT, A, B, bias) + h)
 
 
-# (tiles of 128 x 128, with two groups; with one where the epilogue reads no matrix; with one)
+# (tiles of 128 x 128, with two groups; with one where the epilogue reads no matrix; but with GELU's derivative; with one)
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N", [(2049, 1804), (3457, 3204), (3457, 4228)])
+@pytest.mark.parametrize("M,N", [(2049, 1804), (3457, 3204), (3457, 4228), (3969, 4092)])
 def test_epilogues_of_wide_tiles(gpu, M, N):
     A, B, want, mass = _operands(NT, M, N, 524, gpu)
     Bt, bias, h = B.t().contiguous(), torch.randn(N, device=gpu), torch.randn(M, N, device=gpu)
