@@ -565,24 +565,30 @@ void gemm_f32_rows_kernel(const GemmArgs g)
     finish_rows<64 / W>(g, m0, n0, wave * (64 / W), v);
 }
 
-// The shares' sums of a tile together, in their order: half of a tile per workgroup, four accumulators per wave.  The workgroups behind those make column sums.
-__global__ __launch_bounds__(proteus_train::CS_BLOCK)
+// The shares' sums of a tile together, in their order: W sixteenths of a tile per workgroup, four accumulators per wave.  With eight waves the workgroups behind those make column sums; without any,
+// four waves are the faster ones (shares of 88 x 48 x 7834 in all 13.5 us with eight, 12.8 with four).
+template <int W>
+__global__ __launch_bounds__(W * 64)
 void gemm_f32_rows_sum_kernel(const PendingSums sums)
 {
     static_assert(proteus_train::CS_BLOCK == 512, "eight waves");
-    __shared__ float red[proteus_train::CS_BLOCK / 64][proteus_train::CS_COLS];
-    const int behind = (int)blockIdx.x - sums.first[sums.count];
-    if (behind >= 0) {
-        int c = 0;
-        while (behind >= sums.first_column[c + 1]) ++c;
-        const proteus_train::ColumnSums& of = sums.columns[c];
-        proteus_train::column_sums(of.a, of.out, 0, of.rows, of.cols, behind - sums.first_column[c], red);
-        return;
+    constexpr int PER = 16 / W;                                    // workgroups per tile
+    const int id = (int)blockIdx.x;
+    if constexpr (W * 64 == proteus_train::CS_BLOCK) {
+        __shared__ float red[proteus_train::CS_BLOCK / 64][proteus_train::CS_COLS];
+        const int behind = id - sums.first[sums.count] * PER;
+        if (behind >= 0) {
+            int c = 0;
+            while (behind >= sums.first_column[c + 1]) ++c;
+            const proteus_train::ColumnSums& of = sums.columns[c];
+            proteus_train::column_sums(of.a, of.out, 0, of.rows, of.cols, behind - sums.first_column[c], red);
+            return;
+        }
     }
     int p = 0;
-    while ((int)blockIdx.x >= sums.first[p + 1]) ++p;
+    while (id / PER >= sums.first[p + 1]) ++p;
     const GemmArgs& g = sums.product[p];
-    const int block = (int)blockIdx.x - sums.first[p], tile = block >> 1, e0 = (block & 1) * 32 + (threadIdx.x >> 6) * 4;
+    const int tile = id / PER - sums.first[p], e0 = (id % PER) * (W * 4) + (threadIdx.x >> 6) * 4;
     const float* from = g.part + (size_t)tile * (GT * GT) + e0 * 64 + (threadIdx.x & 63);
     const size_t pitch = (size_t)g.tiles * (GT * GT);
     float v[4] = {};
@@ -641,7 +647,7 @@ int gemm_go(GemmArgs g, hipStream_t st, PendingSums* sums = nullptr)
             PendingSums own;
             PendingSums& p = sums ? *sums : own;
             p.product[p.count] = g;
-            p.first[p.count + 1] = p.first[p.count] + g.tiles * 2;
+            p.first[p.count + 1] = p.first[p.count] + g.tiles;
             ++p.count;
             if (!sums) return gemm_sums(own, st);
         }
@@ -768,9 +774,10 @@ int proteus_gemm::gemm_begin(const float* A, const float* B, float* C, int M, in
 
 int proteus_gemm::gemm_sums(PendingSums& sums, void* stream)
 {
-    const int blocks = sums.first[sums.count] + sums.first_column[sums.column_count];
-    if (blocks == 0) return PROTEUS_OK;
-    hipLaunchKernelGGL(gemm_f32_rows_sum_kernel, dim3((unsigned)blocks), dim3(proteus_train::CS_BLOCK), 0, reinterpret_cast<hipStream_t>(stream), sums);
+    const int tiles = sums.first[sums.count], columns = sums.first_column[sums.column_count];
+    if (tiles + columns == 0) return PROTEUS_OK;
+    if (columns) hipLaunchKernelGGL(gemm_f32_rows_sum_kernel<8>, dim3((unsigned)(tiles * 2 + columns)), dim3(512), 0, reinterpret_cast<hipStream_t>(stream), sums);
+    else         hipLaunchKernelGGL(gemm_f32_rows_sum_kernel<4>, dim3((unsigned)(tiles * 4)), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), sums);
     sums.count = sums.column_count = 0;
     return (int)hipGetLastError();
 }

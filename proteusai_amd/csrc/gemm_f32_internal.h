@@ -16,8 +16,8 @@ struct GemmArgs {
     int shares, steps;                              // their number, and the steps of each
 };
 
-// Products whose shares are not added up yet and column sums that are yet to be made, and the workgroups of the launch that does it: first[i] to first[i + 1] for
-// product i, behind them first_column[i] to first_column[i + 1] for column sum i.
+// Products whose shares are not added up yet and column sums that are yet to be made, for the launch that does it: tiles first[i] to first[i + 1] are product i's,
+// workgroups first_column[i] to first_column[i + 1] behind those of the tiles column sum i's.
 struct PendingSums {
     static constexpr int MOST = 4;
     GemmArgs product[MOST];
