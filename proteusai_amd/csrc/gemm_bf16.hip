@@ -5,9 +5,10 @@
 // (so that the compiler sees that a read of one does not wait for loads into another).  Bias and GELU are added to the fp32 sums, which are then rounded once.
 //
 // What bounds it: LDS at 64 x 64 of C per wave (16 KB read per 128 clocks of matrix instructions and compute unit, its whole rate), a quarter less at 128 x 64; and the
-// rounds of workgroups (one to three of them on a compute unit).  8192 tokens, d_model 512, us, the library's product and torch's GELU / this: QKV 24 / 18, output 13 / 9, feed-forward
-// 25 + 15 / 27 and 23 / 21; a call costs the host 3, the library's 18 to 21.
-// From about 16384 x 1024 of d_model 1024 on the library is ahead (32768 x 3072 x 1024 155 / 194).
+// rounds of workgroups (one to three of them on a compute unit).  8192 tokens, d_model 512, us, the library's product and torch's GELU / this: QKV 24 to 27 / 18.9, output 13 / 8.4, feed-forward
+// 39.5 / 27.7 and 21.7 / 20.8; a call costs the host 3, the library's 18 to 21.
+// Where K is long and there are many rows the library is ahead (10000 x 512 x 2048 24.4 / 29.7, 32768 49 / 59, 65536 99 / 132; 4096 x 2304 x 768 19.5 / 23.7, 8192 x 3072 x 1024 53 / 59), by less than
+// the layer's other launches gain up to the sizes that encoder.py names.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include "proteus_hip.h"
@@ -232,10 +233,11 @@ extern "C" int proteus_gemm_bf16(const uint16_t* A, const uint16_t* B, const uin
     // Small tiles until there is one for every compute unit, since a workgroup is a chain over K; its loads then run three steps ahead, as there is no other workgroup to
     // wait under.  From there on larger tiles, which read less LDS per product, unless their last round is mostly empty.  Us, 64 x 64 / 128 x 64, both four stages /
     // 128 x 64 two stages / 128 x 128 four stages / 128 x 128 two / 256 x 256 two, for M x N x K:
-    //   2048 x 512 x 512 4.6 / 5.7 / 6.2 / 7.7 / 8.2 / 15.1, of 2048 8.8 / 11.9 / 15.6 / 17.8 / 22 / 43;  4096 x 512 x 512 6.3 / 6.1 / 6.9 / 8.1 / 8.5 / 15.3, of 2048 14.3 / 13.0 / 19 / 18.7 / 26 / 49
-    //   8192 x 512 x 512 10.9 / 10.8 / 8.9 / 9.0 / 9.7 / 15.9, of 2048 27.6 / 25.9 / 26.5 / 22.0 / 31.7 / 52.7;  4096 x 2048 x 512 (GELU) 21 / 23 / 18.6 / 20.4 / 17.3 / 24.9
-    //   6000 x 1536 x 512 20.7 / 23.6 / 17.5 / 22 / 20 / 18.6;  8192 x 1536 x 512 26.8 / 27.8 / 21.5 / 22.9 / 21.3 / 19.7;  8192 x 2048 x 512 (GELU) 40 / 44 / 32 / 39 / 30.6 / 28.9
-    //   12288 x 1536 x 512 37 / 39 / 28.4 / 33.5 / 29.7 / 36.5;  16384 x 1536 x 512 48 / 50 / 36 / 40 / 32 / 36;  65536 x 2048 x 512 (GELU) 373 / 421 / 286 / 320 / 264 / 228
+    //   2048 x 512 x 512 4.5 / 5.6 / 6.1 / 7.7 / 7.5 / 14.7, of 2048 8.7 / 11.7 / 14.5 / 17.6 / 18.5 / 42;  4096 x 512 x 512 6.2 / 6.1 / 6.5 / 8.0 / 7.9 / 15.0, of 2048 14.6 / 13.5 / 17.7 / 18.4 / 20.1 / 43
+    //   8192 x 512 x 512 10.5 / 10.5 / 8.3 / 8.8 / 8.6 / 15.5, of 2048 26.8 / 25.5 / 22.8 / 21.2 / 24.3 / 44;  4096 x 2048 x 512 (GELU) 21.6 / 22.8 / 17.5 / 20.4 / 16.5 / 24.7
+    //   6000 x 1536 x 512 20.7 / 22.9 / 16.0 / 21.9 / 19.1 / 17.7;  8192 x 1536 x 512 26.8 / 27.0 / 21.7 / 22.6 / 20.6 / 18.9;  6000 x 2048 x 512 (GELU) 30.0 / 33.0 / 23.8 / 29.1 / 24.0 / 26.1;  8192 x 2048 x 512
+    //   (GELU) 40 / 43 / 30.0 / 37.8 / 29.0 / 27.8;  12288 x 1536 x 512 40.5 / 39.8 / 28.2 / 35.6 / 28.6 / 33.1;  16384 x 1536 x 512 54 / 53 / 36.7 / 44 / 35.3 / 36.6;  65536 x 2048 x 512 (GELU) 374 / 419 / 279 / 318 / 256 / 216
+    //   half-empty tiles are not told apart: 200000 x 64 x 64 21.6 / 24.0 / 14.3 / 33.7 / 18.1 / 28.1 (the library 31.6), 70000 x 256 x 256 30.7 / 31.1 / 19.8 / 26.9 / 24.6 / 23.5 (34.5)
     if (tiles(64, 64) <= 256)   return go<64, 64, 2, 2, 4>(g, gelu != 0, st);
     if (tiles(128, 64) <= 256)  return go<128, 64, 2, 2, 4>(g, gelu != 0, st);
     if (tiles(128, 128) <= 256) return K >= 1024 ? go<128, 128, 2, 2, 4>(g, gelu != 0, st) : go<128, 64, 2, 2, 2>(g, gelu != 0, st);

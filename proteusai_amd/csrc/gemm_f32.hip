@@ -21,10 +21,10 @@
 // Few tiles over many tokens leave compute units idle, each of the others a serial chain over K: there workgroups take shares of K (rows_shares), whose
 // sums a second launch adds up in their order.
 //
-// us, 2048 tokens, this / the library's fp32 product: QKV 2048 x 1536 x 512 25 / 31, its output 10.5 / 12; feed-forward 2048 x 2048 x 512 27 / 35 (with bias and
-// GELU 31, with GELU's derivative 37; the library and torch's elementwise kernels 44 and 45), 2048 x 512 x 2048 32 / 34; gradients of weights 512 x 2048 x 2048 and
-// 2048 x 512 x 2048 29 / 35, 512 x 1536 x 2048 25.4 / 29, 512 x 512 x 2048 14.7 / 14.5 (through the first kernel 44, 39, 35, 31); 8192 tokens 77 / 97, 31 / 35, 97 / 125
-// (108 / 146, 134 / 156), 92 / 119 and 99 / 120, 84 / 99, 32 / 54.
+// us, 2048 tokens, this / the library's fp32 product and torch's elementwise kernels (calls one behind the other; up to a tenth between boxes): QKV 2048 x 1536 x 512 26.5 to 28.7 / 33.5, its
+// output 10.8 / 18; feed-forward 2048 x 2048 x 512 31.7 / 36.0 (with bias and GELU 36.0 / 45.4, with GELU's derivative 36.7 / 45.4), 2048 x 512 x 2048 31.7 / 34.1 (with a matrix added 32.0 / 41.0);
+// gradients of weights 512 x 2048 x 2048 and 2048 x 512 x 2048 30.3 / 38, 512 x 1536 x 2048 26.0 / 29.4, 512 x 512 x 2048 14.9 / 18.2 (through the first kernel 44, 39, 35, 31); 8192 tokens 79 / 97, 31 / 36,
+// 103 / 126 (119 / 147, 133 / 156), 93 / 119 (95 / 128) and 103 / 121, 85 / 98, 33 / 54.
 // Error against float64 at K = 2048 2.5e-7 to 3.5e-7, the library's 8.1e-7.
 //
 // Values that are not finite (or become so: bf16 ends half a step below fp32) do not split; an element of C that comes out not
@@ -257,7 +257,7 @@ void gemm_f32_kernel(const GemmArgs g)
 }
 
 // The same with tiles of 128 x 128, 64 x 64 of them a wave: two thirds of the LDS traffic per product (24 KB read and 12 KB written per 64 x 64 x 16 become 12 and 6) and half of the splitting, which is
-// laid between the products.  G groups of four waves share a tile, each with its own steps and stages.  What bounds it: the products (8192 x 2048 x 512 at 1060 TFLOP/s of bf16,
+// laid between the products.  G groups of four waves share a tile, each with its own steps and stages.  What bounds it: the products (8192 x 2048 x 512 at 1000 to 1060 TFLOP/s of bf16,
 // a library product of bf16 reaches 1300), at a tile per compute unit the fill and the epilogue.  Without the order below, split and then products, the odd group the other way
 // round: 2048 x 2048 x 512 31.3 us, so 28.8 (64 x 64 tiles 36.3), 8192 tokens with one group 108 and 97 (128).  Loads four steps ahead: 29.5.
 constexpr int WT       = 128;

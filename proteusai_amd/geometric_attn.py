@@ -539,11 +539,11 @@ class GeoAttention(nn.Module):
         """make(), tensors that depend on `params` and `more` alone, kept across calls where they may be."""
         if self.training or (torch.is_grad_enabled() and any(p.requires_grad for p in params)):
             return make()
-        key = (more, tuple((p._version, p.data_ptr(), p.dtype) for p in params))
+        key = (more, tuple([(p._version, p.data_ptr(), p.dtype) for p in params]))
         kept = self.__dict__.setdefault("_constants", {}).get(name)
         if kept is not None and kept.key == key:
             return kept.tensors_here()
-        tensors = tuple(t.detach() for t in make())
+        tensors = tuple([t.detach() if t.requires_grad else t for t in make()])
         if not (params[0].is_cuda and torch.cuda.is_current_stream_capturing()):
             self.__dict__.setdefault("_constants", {})[name] = _Kept(key, tensors)
         return tensors
@@ -586,25 +586,26 @@ class GeoAttention(nn.Module):
 
 
 class _Kept:
-    """Tensors made on one stream for use on any: a stream that has not used them yet waits until they are made, and the allocator hears of it, so that
-    their memory goes back only once its reads are over.  (Under capture they have been made: capturing begins on an idle device.)"""
+    """Tensors made on one stream for use on any: a stream that has not used them yet waits for the one they were made on, and the allocator hears of it, so
+    that their memory goes back only once its reads are over.  (Under capture they have been made: capturing begins on an idle device.)"""
 
     def __init__(self, key, tensors):
-        self.key, self.tensors, self.event = key, tensors, None
-        if tensors[0].is_cuda:
-            self.device = tensors[0].device
-            self.streams = {_lib.raw_stream(self.device)}
-            self.event = torch.cuda.current_stream(self.device).record_event()
+        self.key, self.tensors, self.device = key, tensors, tensors[0].device
+        # (no event of their own: making one took 11 us of a layer's first pass)
+        self.streams = [_lib.raw_stream(self.device)] if tensors[0].is_cuda else None
 
     def tensors_here(self):
-        if self.event is not None:
+        if self.streams is not None:
             stream = _lib.raw_stream(self.device)
             if stream not in self.streams and not torch.cuda.is_current_stream_capturing():
-                current = torch.cuda.current_stream(self.device)
-                current.wait_event(self.event)
+                current, made_on = torch.cuda.current_stream(self.device), torch.cuda.ExternalStream(self.streams[0], self.device)
+                with torch.cuda.stream(made_on):
+                    made = torch.cuda.is_current_stream_capturing()
+                if not made:
+                    current.wait_event(made_on.record_event())
                 for t in self.tensors:
                     t.record_stream(current)
-                self.streams.add(stream)
+                self.streams.append(stream)
         return self.tensors
 
     def __reduce__(self):                    # (a copied or stored module makes its own)
